@@ -132,6 +132,25 @@ int sga_masked_norm_sq(const float* grad, const uint8_t* mask, int64_t n,
 int sga_scale_masked(float* grad, const uint8_t* mask, int64_t n, float coeff,
                      void* stream);
 
+/* The clip service over MANY tensors in one launch per pass (the per-record
+ * loops of engine.py:1075-1130, 1172-1216).  recs: DEVICE table ordered by
+ * first_span; a tensor of n elements covers ceil(n / 4096) spans, total_spans
+ * is their sum; mask may be NULL per record.
+ * sga_norm_sq_multi: total[0] = sum of g^2 over the (masked) coordinates of all
+ *   records, fixed order.  partials: total_spans floats of workspace.
+ * sga_scale_multi:   g *= coeff on the (masked) coordinates of all records. */
+typedef struct sga_span_record {
+  float* g;
+  const uint8_t* mask;
+  int64_t n;
+  int64_t first_span;
+} sga_span_record;
+int sga_norm_sq_multi(const sga_span_record* recs, int n_recs,
+                      int64_t total_spans, float* partials, float* total,
+                      void* stream);
+int sga_scale_multi(const sga_span_record* recs, int n_recs,
+                    int64_t total_spans, float coeff, void* stream);
+
 /* block gather / scatter  -- gather_selected_blocks / scatter_selected_blocks,
  * kernels.py:190-249 */
 int sga_gather_selected_blocks(const float* grad, const uint8_t* mask,

@@ -83,6 +83,8 @@ SIGNATURES = {
     "sga_hist_topbits": (I32, [P, I64, I32, I32, I32, P, I32, P, P]),
     "sga_mask_topbits_ge": (I32, [P, I64, I32, I32, P, P]),
     "sga_scale_masked": (I32, [P, P, I64, F, P]),
+    "sga_norm_sq_multi": (I32, [P, I32, I64, P, P, P]),
+    "sga_scale_multi": (I32, [P, I32, I64, F, P]),
     "sga_mask_abs_ge": (I32, [P, I64, F, P, P, P]),
     "sga_cand_extract_count": (I32, [P, I64, I32, P, P, P]),
     "sga_cand_extract_fill": (I32, [P, I64, I32, P, P, I64, P]),
@@ -187,6 +189,35 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host side of the plugin steps (``csrc/host_ext.cpp``), bound to
+    the entry points of libsga_hip.so; raises loudly when it is not built."""
+    global _host
+    if _host is None:
+        lib = load()
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise RuntimeError("sga_amd/_host.so is missing or does not load: run "
+                               f"`python -m sga_amd.build` ({e})") from e
+        from .adamw import ParamRecord
+        mod.bind(ParamRecord, *(C.cast(getattr(lib, n), P).value for n in (
+            "sga_adamw_grad_correct_multi", "sga_adamw_grad_correct_compact_multi",
+            "sga_norm_sq_multi", "sga_scale_multi")))
+        _host = mod
+    return _host
+
+
+def check(rc, name):
+    """Raise with the library's text when an entry point reported an error."""
+    if rc != 0:
+        raise RuntimeError(f"{name} failed ({rc}): "
+                           f"{load().sga_last_error().decode(errors='replace')}")
 
 
 def call(name, *args):

@@ -3,8 +3,9 @@
 Usage: ``python -m sga_amd.build`` -- compiles every product source of
 ``csrc/`` into ``sga_amd/libsga_hip.so`` (the C ABI of include/sga_hip.h and
 nothing else) and ``csrc/bench_hooks.hip`` into ``sga_amd/libsga_hip_bench.so``
-(timing observer + calibration kernels, loaded by bench.py only), both
-in-tree.  -ffp-contract=off keeps every fp32 operation separately rounded (the
+(timing observer + calibration kernels, loaded by bench.py only), and the
+CPython extension ``csrc/host_ext.cpp`` (host side of the plugin steps, plain
+C++ against torch's headers) into ``sga_amd/_host.so``, all in-tree.  -ffp-contract=off keeps every fp32 operation separately rounded (the
 kernels place FMAs explicitly where the arithmetic recipe has one).
 """
 import os
@@ -16,6 +17,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libsga_hip.so")
 BENCH_LIB = os.path.join(HERE, "libsga_hip_bench.so")
+HOST_EXT = os.path.join(HERE, "_host.so")
 SOURCES = ["fused_step.hip", "replay_group.hip", "select.hip", "elementwise.hip", "adamw.hip",
            "replay.hip", "runtime.hip", "scan.hip"]
 BENCH_SOURCES = ["bench_hooks.hip"]
@@ -42,8 +44,28 @@ def _stale(src, obj):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def build_host_ext(incremental=False):
+    """The CPython extension; the torch libraries it names are the ones the
+    importing process has loaded already."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    src = os.path.join(CSRC, "host_ext.cpp")
+    if incremental and not _stale(src, HOST_EXT):
+        return
+    import torch
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+           "-I" + sysconfig.get_paths()["include"], src, "-o", HOST_EXT,
+           *(f"-L{p}" for p in cpp_extension.library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed on host_ext.cpp:\n{r.stdout}\n{r.stderr}")
+
+
 def build(verbose=True, jobs=8, extra=(), incremental=False):
-    """Compile and link both libraries.  ``incremental`` (a convenience while
+    """Compile and link both libraries and the host extension.  ``incremental`` (a convenience while
     editing) skips sources whose object file is newer than the source and all
     headers; the default compiles everything."""
     hipcc = _hipcc()
@@ -68,7 +90,9 @@ def build(verbose=True, jobs=8, extra=(), incremental=False):
         return obj
 
     with ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(build_host_ext, incremental)
         objs = list(ex.map(one, SOURCES + BENCH_SOURCES))
+        host.result()
     for lib, group in ((LIB, objs[:len(SOURCES)]), (BENCH_LIB, objs[len(SOURCES):])):
         cmd = [hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *group, "-o", lib]
         r = subprocess.run(cmd, capture_output=True, text=True)
@@ -76,6 +100,8 @@ def build(verbose=True, jobs=8, extra=(), incremental=False):
             raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
         if verbose:
             print(f"built {lib} from {len(group)} sources")
+    if verbose:
+        print(f"built {HOST_EXT}")
     return LIB
 
 

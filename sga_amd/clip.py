@@ -28,6 +28,32 @@ def scale_masked_(grad, mask, coeff):
            g.numel(), L.f32(coeff), L.stream())
 
 
+def _clip_one_launch(records, clip_grad, was_full, trace_dumps):
+    """The clip over every record's gradient with one launch per pass
+    (``csrc/host_ext.cpp`` walks the records); None when a record is not the
+    ordinary ``ParamRecord`` over flat fp32 device tensors."""
+    host = L.host()
+    table = host.norm_table(records, was_full)
+    if not table:                        # False: not ordinary; None: nothing to clip
+        return None
+    rows, any_maskless, st = table[:3], table[3], L.stream()
+    # a sparse step's mask-less records are scaled on their own: the general route does that
+    if any_maskless and not was_full:
+        return None
+    grad_norm = host.norm(*rows, st)
+    if isinstance(grad_norm, int):
+        L.check(grad_norm, "sga_norm_sq_multi")
+    sparse_coeff = 1.0
+    if clip_grad > 0.0:
+        coeff = clip_grad / (grad_norm + 1.0e-6)
+        if coeff < 1.0:
+            if was_full or trace_dumps:
+                L.check(host.scale(*rows, coeff, st), "sga_scale_multi")
+            else:
+                sparse_coeff = float(coeff)
+    return grad_norm, sparse_coeff
+
+
 def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
                           trace_dumps=False):
     """Returns ``(grad_norm, sparse_coeff)``.
@@ -38,6 +64,10 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
     mask-less records; otherwise it is returned for the commit kernel's
     in-register multiply (``engine.py:1172-1217``).
     """
+    if not compact_values or was_full:
+        done = _clip_one_launch(records, clip_grad, was_full, trace_dumps)
+        if done is not None:
+            return done
     live = [r for r in records if r.grad is not None]
     if not live:
         return 0.0, 1.0

@@ -89,6 +89,119 @@ __global__ __launch_bounds__(kBlock) void k_norm_stage2(
   }
 }
 
+// ------------------------------------------- clip service over many records
+// One workgroup per 4096-element span of one record (sga_span_record): the
+// norm and the scale of a step are one launch each, whatever the number of
+// parameter tensors (45 tensors of a 1.15 M-element bucket: 90 + 45 launches,
+// 0.5 ms of host time, for 4 us of traffic).  A masked record loads its mask
+// bytes first and then only the quads that hold a selected coordinate: at 1 %
+// three of four 128-byte lines of the gradient are never touched.
+struct SpanWork {
+  float* g;
+  const uint8_t* mask;
+  int64_t n, base;
+  bool vec, full;
+};
+__device__ __forceinline__ SpanWork span_work(const sga_span_record* __restrict__ recs, int n_recs) {
+  const int64_t span = blockIdx.x;
+  const sga_span_record r = recs[find_record(recs, n_recs, span)];
+  SpanWork w;
+  w.g = r.g; w.mask = r.mask; w.n = r.n;
+  w.base = (span - r.first_span) * kBlockSpan;
+  w.vec = aligned4(r.g, 4) && aligned4(r.mask, 1);
+  w.full = w.vec && w.base + kBlockSpan <= r.n;
+  return w;
+}
+constexpr int kSpanIters = kBlockSpan / (kBlock * kVec);   // 4 quads per lane
+
+// the lane's quads of the span; quads without a selected coordinate are not read
+template <bool FULL>
+__device__ __forceinline__ void span_quads(const SpanWork& w, float v[kSpanIters][4],
+                                           uint32_t mk[kSpanIters][4]) {
+#pragma unroll
+  for (int it = 0; it < kSpanIters; ++it) {
+    const int64_t i = w.base + ((int64_t)it * kBlock + threadIdx.x) * kVec;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mk[it][e] = 1u;
+    if (w.mask) ld_u8<FULL>(w.mask, i, w.n, mk[it], w.vec);
+    else if (!FULL) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mk[it][e] = i + e < w.n;
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < kSpanIters; ++it) {
+    const int64_t i = w.base + ((int64_t)it * kBlock + threadIdx.x) * kVec;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[it][e] = 0.0f;
+    if (mk[it][0] | mk[it][1] | mk[it][2] | mk[it][3]) {
+      if (FULL) {
+        const F4 q = ld4(w.g + i);
+        v[it][0] = q.x; v[it][1] = q.y; v[it][2] = q.z; v[it][3] = q.w;
+      } else {
+        load4_f32(w.g, i, w.n, v[it], w.vec);
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_norm_multi(const sga_span_record* __restrict__ recs,
+                                                       int n_recs, float* __restrict__ partials) {
+  __shared__ float s_w[kChunksPerBlock];
+  const SpanWork w = span_work(recs, n_recs);
+  float v[kSpanIters][4];
+  uint32_t mk[kSpanIters][4];
+  if (w.full) span_quads<true>(w, v, mk);
+  else span_quads<false>(w, v, mk);
+  float acc = 0.0f;
+#pragma unroll
+  for (int it = 0; it < kSpanIters; ++it)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float x = mk[it][e] ? v[it][e] : 0.0f;
+      acc += x * x;
+    }
+  acc = wave_sum(acc);
+  if (lane_id() == 0) s_w[wave_id()] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) partials[blockIdx.x] = (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
+}
+
+// One workgroup folds the spans' partials in a fixed order, in double.
+constexpr int kFoldBlock = 1024;
+__global__ __launch_bounds__(kFoldBlock) void k_norm_multi_fold(const float* __restrict__ partials,
+                                                                int64_t np, float* __restrict__ total) {
+  __shared__ double s_w[kFoldBlock / kWave];
+  double acc = 0.0;
+  for (int64_t i = threadIdx.x; i < np; i += kFoldBlock) acc += (double)partials[i];
+  acc = wave_sum(acc);
+  if (lane_id() == 0) s_w[wave_id()] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double t = 0.0;
+    for (int w = 0; w < kFoldBlock / kWave; ++w) t += s_w[w];
+    total[0] = (float)t;
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_scale_multi(const sga_span_record* __restrict__ recs,
+                                                        int n_recs, float coeff) {
+  const SpanWork w = span_work(recs, n_recs);
+  float v[kSpanIters][4];
+  uint32_t mk[kSpanIters][4];
+  if (w.full) span_quads<true>(w, v, mk);
+  else span_quads<false>(w, v, mk);
+#pragma unroll
+  for (int it = 0; it < kSpanIters; ++it) {
+    const int64_t i = w.base + ((int64_t)it * kBlock + threadIdx.x) * kVec;
+    if (!(mk[it][0] | mk[it][1] | mk[it][2] | mk[it][3])) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[it][e] = mk[it][e] ? v[it][e] * coeff : v[it][e];
+    if (w.full) st4(w.g + i, F4{v[it][0], v[it][1], v[it][2], v[it][3]});
+    else store4_f32(w.g, i, w.n, v[it], w.vec);
+  }
+}
+
 // --------------------------------------------------------- block gather
 template <bool SCALE>
 __global__ __launch_bounds__(kBlock) void k_gather_blocks(
@@ -461,6 +574,30 @@ extern "C" int sga_scale_masked(float* grad, const uint8_t* mask, int64_t n, flo
   else
     hipLaunchKernelGGL((k_scale_masked<false>), grid, block, 0, (hipStream_t)stream, grad, mask, n, coeff, vec);
   return check_launch("sga_scale_masked");
+}
+
+static int span_args(const char* who, const sga_span_record* recs, int n_recs, int64_t total_spans) {
+  if (recs && n_recs > 0 && total_spans > 0 && total_spans < (1ll << 31)) return SGA_OK;
+  set_error("%s: bad argument (n_recs=%d spans=%lld)", who, n_recs, (long long)total_spans);
+  return SGA_ERR_ARG;
+}
+
+extern "C" int sga_norm_sq_multi(const sga_span_record* recs, int n_recs, int64_t total_spans,
+                                 float* partials, float* total, void* stream) {
+  if (int rc = span_args("sga_norm_sq_multi", recs, n_recs, total_spans)) return rc;
+  if (!partials || !total) { set_error("sga_norm_sq_multi: bad argument"); return SGA_ERR_ARG; }
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL(k_norm_multi, dim3((unsigned)total_spans), dim3(kBlock), 0, st, recs, n_recs, partials);
+  hipLaunchKernelGGL(k_norm_multi_fold, dim3(1), dim3(kFoldBlock), 0, st, partials, total_spans, total);
+  return check_launch("sga_norm_sq_multi");
+}
+
+extern "C" int sga_scale_multi(const sga_span_record* recs, int n_recs, int64_t total_spans,
+                               float coeff, void* stream) {
+  if (int rc = span_args("sga_scale_multi", recs, n_recs, total_spans)) return rc;
+  hipLaunchKernelGGL(k_scale_multi, dim3((unsigned)total_spans), dim3(kBlock), 0, (hipStream_t)stream, recs,
+                     n_recs, coeff);
+  return check_launch("sga_scale_multi");
 }
 
 static int xlog_of(int x) {

@@ -1,0 +1,86 @@
+"""The table-driven launches of the plugin steps (clip norm, clip scale, commits)
+against the per-tensor entry points and float64, at the edges of their
+4096-element spans and of the 64-record rounds of the table search."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 3, 4095, 4096, 4097, 8192, 12_289]
+
+
+def _records(dev, sizes, seed, with_mask):
+    from sga_amd.adamw import ParamRecord
+    gen = torch.Generator().manual_seed(seed)
+    n = sum(sizes)
+    t = {k: (torch.randn(n, generator=gen) * s).to(dev) for k, s in
+         (("p", 0.02), ("g", 1e-2), ("m", 1e-3))}
+    t["v"] = (torch.rand(n, generator=gen) * 1e-4).to(dev)
+    mask = (torch.rand(n, generator=gen) < 0.03).to(torch.uint8).to(dev) if with_mask else None
+    bucket = SimpleNamespace(active_mask_u8=mask, grad_data=t["g"], extra_main_grads=[], support_index=0)
+    recs, off = [], 0
+    for i, s in enumerate(sizes):
+        e = slice(off, off + s)
+        recs.append(ParamRecord(None, SimpleNamespace(data=t["p"][e], grad=t["g"][e]), bucket, off, off + s,
+                                1e-3, 0.9, 0.95, 1e-8, 0.1 * (i % 2), 7,
+                                _state={"exp_avg": t["m"][e], "exp_avg_sq": t["v"][e]}))
+        off += s
+    return recs, t, mask
+
+
+# 63 / 64 / 65 records: one and two rounds of the search; odd sizes shift every later record off
+# 16-byte alignment, so both the vector and the scalar forms run
+@pytest.mark.parametrize("count", [1, 7, 63, 64, 65, 200])
+@pytest.mark.parametrize("with_mask", [True, False])
+def test_clip_tables(dev, count, with_mask):
+    from sga_amd.clip import masked_clip_grad_norm
+    sizes = [EDGES[i % len(EDGES)] for i in range(count)]
+    recs, t, mask = _records(dev, sizes, count, with_mask)
+    before = t["g"].clone()
+    on = before if mask is None else before * mask
+    exact = float(on.double().square().sum().sqrt())
+    norm, coeff = masked_clip_grad_norm(recs, 0.5 * exact, was_full=False, trace_dumps=with_mask)
+    # fp32 partials of 4096 squares each, folded in double: below 4096 * 2^-24 relative
+    assert abs(norm - exact) <= 2.5e-4 * exact
+    if with_mask:                                # dump steps scale in place
+        c32 = torch.tensor(0.5 * exact / (norm + 1e-6), device=dev)
+        assert coeff == 1.0 and torch.equal(t["g"], torch.where(mask > 0, before * c32, before))
+
+
+@pytest.mark.parametrize("count", [1, 7, 64, 65, 200])
+@pytest.mark.parametrize("phase", ["full", "sparse", "sparse_fold", "compact"])
+def test_commit_tables(dev, count, phase):
+    from sga_amd import config
+    from sga_amd.adamw import (OptContext, SgaAdamW, adamw_grad_correct, adamw_grad_correct_compact,
+                               build_dir_table)
+    from sga_amd.support import compact_mask_u8
+    config.set_args(SimpleNamespace(sga_score="update", sga_optimizer_residual_mean=True,
+                                    sga_optimizer_compact_search="table",
+                                    sga_optimizer_full_sync_inactive_lr_scale=1.0))
+    sizes = [EDGES[i % len(EDGES)] for i in range(count)]
+    recs, t, mask = _records(dev, sizes, 100 + count, phase != "full")
+    ref_recs, ref, _ = _records(dev, sizes, 100 + count, phase != "full")
+    opt, kw = SgaAdamW(), {}
+    if phase == "compact":
+        idx = compact_mask_u8(mask)
+        vals = t["g"][idx.long()].contiguous()
+        table = build_dir_table(idx, sum(sizes))
+        kw = dict(compact_values={id(recs[0].bucket_state): vals},
+                  support=SimpleNamespace(buckets=[SimpleNamespace(idx=idx, dir_table=table)]))
+    ctx = OptContext(recs, phase, bucket_states=[recs[0].bucket_state], apply_coeff=0.5, fold_window=4,
+                     next_step_is_full=phase == "sparse_fold", **kw)
+    (opt.full_step if phase == "full" else opt.sparse_step)(ctx)
+    for r in ref_recs:
+        a = (r.main_param.data, r.grad, r.m, r.v)
+        h = (r.lr, r.beta1, r.beta2, r.eps, r.weight_decay, r.step)
+        if phase == "full":
+            adamw_grad_correct(*a, *h, emit_score="update")
+        elif phase == "compact":
+            adamw_grad_correct_compact(*a, idx, vals, r.start, *h, coeff=0.5, dir_table=table)
+        else:
+            adamw_grad_correct(*a, *h, mask=r.mask_u8(), coeff=0.5, clear=True,
+                               fold=phase == "sparse_fold", interval=4.0)
+    for k in t:
+        assert torch.equal(t[k], ref[k]), k
