@@ -31,11 +31,17 @@ __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict_
   const bool adams = flags & SGA_GC_ADAMS;   // v basis = pre-commit m*m, h.bc1 = h.bc2 = 1
   float pp[4], gg[4], mm[4], vv[4];
   uint32_t mk[4] = {1, 1, 1, 1};
+  if (has_mask) ld_u8<FULL>(mask, i, n, mk, vec);
   ld_f32<FULL>(p, i, n, pp, vec);
-  ld_f32<FULL>(g, i, n, gg, vec);
   ld_f32<FULL>(m, i, n, mm, vec);
   if (!adams) ld_f32<FULL>(v, i, n, vv, vec);
-  if (has_mask) ld_u8<FULL>(mask, i, n, mk, vec);
+  // A sparse commit without the fold takes a zero gradient off the support and leaves the buffer
+  // there as it is: quads without a selected coordinate are neither read nor written (at 1 % three
+  // of four 128-byte lines of g: 33 -> about 27 bytes per element).
+  const bool touch_g = EMIT >= 0 || !has_mask || fold || (mk[0] | mk[1] | mk[2] | mk[3]) != 0u;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) gg[e] = 0.0f;
+  if (touch_g) ld_f32<FULL>(g, i, n, gg, vec);
   if (adams) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) vv[e] = mm[e] * mm[e];
@@ -65,7 +71,7 @@ __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict_
   }
   st_f32<FULL>(m, i, n, mm, vec);
   st_f32<FULL>(v, i, n, vv, vec);
-  if (EMIT >= 0 || clear || fold) st_f32<FULL>(g, i, n, gout, vec);
+  if (EMIT >= 0 || fold || (clear && touch_g)) st_f32<FULL>(g, i, n, gout, vec);
   st_f32<FULL>(p, i, n, pp, vec);
 }
 
@@ -100,12 +106,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct_multi(const GcRecord* _
                                                                int n_recs, float coeff,
                                                                float interval) {
   const int64_t span = blockIdx.x;
-  int a = 0, b = n_recs - 1;
-  while (a < b) {                       // last record whose first span is <= this one
-    const int mid = (a + b + 1) >> 1;
-    if (recs[mid].first_span <= span) a = mid; else b = mid - 1;
-  }
-  const GcRecord r = recs[a];
+  const GcRecord r = recs[find_record(recs, n_recs, span)];
   Hyper h;
   h.lr = r.lr; h.b1 = r.b1; h.om1 = r.om1; h.b2 = r.b2; h.om2 = r.om2; h.eps = r.eps;
   h.wd = r.wd; h.bc1 = r.bc1; h.bc2 = r.bc2;
@@ -171,7 +172,22 @@ __device__ __forceinline__ void compact_span(
   const int64_t c0 = rec_start + off0;
   int64_t c1 = c0 + kBlockSpan;
   if (c1 > rec_start + n) c1 = rec_start + n;
-  for (int t = threadIdx.x; t < kBlockSpan; t += kBlock) s_val[t] = 0.0f;
+  // A whole, aligned span requests its p / m / v up front (12 quads per lane): the search and the
+  // staging of the gradient below are two chains of dependent loads, and without this nothing of
+  // the span's 24 bytes per element is in flight while they run.
+  const bool full = vec && off0 + kBlockSpan <= n;
+  F4 rp[kChunkIters], rm[kChunkIters], rv[kChunkIters];
+  if (full) {
+#pragma unroll
+    for (int it = 0; it < kChunkIters; ++it) {
+      const int64_t i = off0 + it * (kBlock * kVec) + threadIdx.x * kVec;
+      rp[it] = ld4_nt(p + i);
+      rm[it] = ld4_nt(m + i);
+      if (!adams) rv[it] = ld4_nt(v + i);
+    }
+  }
+  for (int t = threadIdx.x * kVec; t < kBlockSpan; t += kBlock * kVec)
+    *reinterpret_cast<F4*>(s_val + t) = F4{0.0f, 0.0f, 0.0f, 0.0f};
   if (threadIdx.x < kBlockSpan / 32) s_found[threadIdx.x] = 0u;
   if (wave_id() < 2) {
     const int64_t key = wave_id() == 0 ? c0 : c1;
@@ -206,13 +222,18 @@ __device__ __forceinline__ void compact_span(
     const int64_t i = off0 + t0;
     if (i < n) {
       float pp[4], mm[4], vv[4], raw[4] = {0, 0, 0, 0};
-      load4_f32(p, i, n, pp, vec);
-      load4_f32(m, i, n, mm, vec);
+      if (full) {
+        unpack_f32(rp[it], pp);
+        unpack_f32(rm[it], mm);
+        if (!adams) unpack_f32(rv[it], vv);
+      } else {
+        load4_f32(p, i, n, pp, vec);
+        load4_f32(m, i, n, mm, vec);
+        if (!adams) load4_f32(v, i, n, vv, vec);
+      }
       if (adams) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) vv[e] = mm[e] * mm[e];
-      } else {
-        load4_f32(v, i, n, vv, vec);
       }
       if (fold) load4_f32(g, i, n, raw, vec);
       const uint32_t fw = s_found[t0 >> 5] >> (t0 & 31);
@@ -227,10 +248,16 @@ __device__ __forceinline__ void compact_span(
         vv[e] = c.v_new;
         if (fold && !found) raw[e] = __fdiv_rn(raw[e], interval);
       }
-      store4_f32(m, i, n, mm, vec);
-      store4_f32(v, i, n, vv, vec);
+      if (full) {
+        st4_nt(m + i, F4{mm[0], mm[1], mm[2], mm[3]});
+        st4_nt(v + i, F4{vv[0], vv[1], vv[2], vv[3]});
+        st4_nt(p + i, F4{pp[0], pp[1], pp[2], pp[3]});
+      } else {
+        store4_f32(m, i, n, mm, vec);
+        store4_f32(v, i, n, vv, vec);
+        store4_f32(p, i, n, pp, vec);
+      }
       if (fold) store4_f32(g, i, n, raw, vec);
-      store4_f32(p, i, n, pp, vec);
     }
   }
   __syncthreads();
@@ -243,7 +270,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct_compact(
     const void* __restrict__ values, int64_t rec_start, int64_t n,
     int64_t k_total, Hyper h, float coeff, float interval, int flags,
     const int32_t* __restrict__ table, int64_t n_table, bool vec) {
-  __shared__ float s_val[kBlockSpan];
+  __shared__ __align__(16) float s_val[kBlockSpan];
   __shared__ uint32_t s_found[kBlockSpan / 32];
   __shared__ int64_t s_bounds[2];
   const int64_t n_spans = cdiv64(n, kBlockSpan);
@@ -264,16 +291,11 @@ struct GccRecord {          // sga_gcc_record, see the header
 template <bool BF16>
 __global__ __launch_bounds__(kBlock) void k_grad_correct_compact_multi(
     const GccRecord* __restrict__ recs, int n_recs, float coeff, float interval) {
-  __shared__ float s_val[kBlockSpan];
+  __shared__ __align__(16) float s_val[kBlockSpan];
   __shared__ uint32_t s_found[kBlockSpan / 32];
   __shared__ int64_t s_bounds[2];
   const int64_t span = blockIdx.x;
-  int a = 0, b = n_recs - 1;
-  while (a < b) {
-    const int mid = (a + b + 1) >> 1;
-    if (recs[mid].first_span <= span) a = mid; else b = mid - 1;
-  }
-  const GccRecord r = recs[a];
+  const GccRecord r = recs[find_record(recs, n_recs, span)];
   Hyper h;
   h.lr = r.lr; h.b1 = r.b1; h.om1 = r.om1; h.b2 = r.b2; h.om2 = r.om2; h.eps = r.eps;
   h.wd = r.wd; h.bc1 = r.bc1; h.bc2 = r.bc2;
