@@ -140,19 +140,21 @@ struct SegCursor {
   }
 };
 
-// Builds the directory of a segment table: dir[b] = last segment with start <= b << kSegDirLog.
+// Entry b of the directory of a segment table: the last segment with start <= b << kSegDirLog.
+__device__ __forceinline__ int seg_dir_entry(const sga_segment* __restrict__ segs, int n_segs, int64_t b) {
+  const int64_t i = b << kSegDirLog;
+  int lo = 0, hi = n_segs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (segs[mid].start <= i) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
 __device__ __forceinline__ void seg_dir_body(const sga_segment* __restrict__ segs, int n_segs,
                                              int64_t n, int32_t* __restrict__ dir) {
   const int64_t nb = (n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
-  for (int64_t b = (int64_t)blockIdx.x * kBlock + threadIdx.x; b < nb; b += (int64_t)gridDim.x * kBlock) {
-    const int64_t i = b << kSegDirLog;
-    int lo = 0, hi = n_segs - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (segs[mid].start <= i) lo = mid; else hi = mid - 1;
-    }
-    dir[b] = lo;
-  }
+  for (int64_t b = (int64_t)blockIdx.x * kBlock + threadIdx.x; b < nb; b += (int64_t)gridDim.x * kBlock)
+    dir[b] = seg_dir_entry(segs, n_segs, b);
 }
 static __global__ __launch_bounds__(kBlock) void k_seg_dir(const sga_segment* __restrict__ segs,
                                                            int n_segs, int64_t n,

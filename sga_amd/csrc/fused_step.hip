@@ -7,7 +7,7 @@
 // (6 B each); the final sweep reads g, resid, p, m, v (18 B) and writes
 // resid, p, m, v (16 B) plus the rho*(4+2) B pack.
 #include "adam_math.hpp"
-#include "select_impl.hpp"
+#include "small_select.hpp"
 
 namespace sga {
 
@@ -160,7 +160,7 @@ struct FinalArgs {
 // the keys are not formed again; SCORE is then irrelevant.
 template <bool BF16G, bool BF16V, int SCORE, bool FULL, int IT0, int NIT, bool PLANES>
 __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, ChunkCursor& cur,
-                                            SegCursor& sc, SegCursor& lc) {
+                                            SegCursor& sc) {
   const int64_t n = a.n;
   const int64_t sh = pack_shift<true>(c << 10, a.pack_extra);     // c is wave-uniform
   const float* const R = a.r + sh;
@@ -244,7 +244,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
       pos = cur.sel_run + below;
       cur.sel_run += total;
     } else {
-      uint32_t key[4];
+      uint32_t key[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         valid[e] = FULL || i + e < n;
@@ -252,13 +252,15 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
         if (SCORE == SGA_SCORE_ABS_G) key[e] = abs_key(q[e]);
         else if (SCORE == SGA_SCORE_ABS_G_BLIND) key[e] = abs_key(gg[it][e]);
         else if (SCORE == SGA_SCORE_ABS_M) key[e] = abs_key(mm[it][e]);
-        else {
-          // only when the one-sweep select is off or failed: a per-lane cursor
-          if (valid[e]) lc.seek(i + e);
-          Hyper hk = lc.h;
-          float ve = vv[it][e];
-          if (a.adams) { ve = mm[it][e] * mm[it][e]; hk.bc1 = 1.0f; hk.bc2 = 1.0f; }
-          key[e] = valid[e] ? score_key<SCORE>(q[e], pp[it][e], mm[it][e], ve, hk) : 0u;
+      }
+      if (SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI || SCORE == SGA_SCORE_GR_OVER_SQRT_V) {
+        const int64_t s0 = uniform_i64(c) * kChunk + it * (kWave * kVec);
+        if (FULL || s0 < n) {
+          float vk[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) vk[e] = a.adams ? mm[it][e] * mm[it][e] : vv[it][e];
+          if (s0 < sc.lo || s0 >= sc.hi) sc.seek_uniform(s0);
+          slab_score_keys<SCORE, FULL>(sc, a.adams ? 1 : 0, i, n, q, pp[it], mm[it], vk, key);
         }
       }
       slab_select(key, valid, a.T, a.need, cur, sel, pos);
@@ -351,9 +353,8 @@ void k_fused_final(
   a.need = st->need;
   const int64_t n_chunks = cdiv64(a.n, kChunk);
   const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  SegCursor sc, lc;              // sc: wave-uniform (scalar unit); lc: per lane, key forming only
+  SegCursor sc;                  // wave-uniform (scalar unit)
   sc.init(segs, n_segs, seg_dir);
-  lc.init(segs, n_segs, seg_dir);
   const bool can_full = a.vec && (a.mask_out == nullptr || a.mvec);
   const unsigned blk = a.pack_extra != 0 ? xcd_contiguous_block(blockIdx.x, gridDim.x) : blockIdx.x;
   for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks;
@@ -364,17 +365,17 @@ void k_fused_final(
     if (can_full && (c + 1) * kChunk <= a.n) {
       // one 256-element slab at a time (5 loads in flight per lane): measured
       // as fast as batching all four slabs, at twice the occupancy
-      final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, true, 1, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, true, 2, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, true, 3, 1, PLANES>(a, c, cur, sc, lc);
+      final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, true, 1, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, true, 2, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, true, 3, 1, PLANES>(a, c, cur, sc);
     } else {
       // the ragged path too: holding four slabs at once would set the register count (and so
       // the occupancy) of the whole kernel
-      final_chunk<BF16G, BF16V, SCORE, false, 0, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, false, 1, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, false, 2, 1, PLANES>(a, c, cur, sc, lc);
-      final_chunk<BF16G, BF16V, SCORE, false, 3, 1, PLANES>(a, c, cur, sc, lc);
+      final_chunk<BF16G, BF16V, SCORE, false, 0, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, false, 1, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, false, 2, 1, PLANES>(a, c, cur, sc);
+      final_chunk<BF16G, BF16V, SCORE, false, 3, 1, PLANES>(a, c, cur, sc);
     }
   }
 }
@@ -415,8 +416,12 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   // evaluating the score chain a second time; if the bracket fails on the device, the key-forming
   // final sweep runs instead.  For |g + r| and |m| the key is one instruction and re-forming it is
   // cheaper than writing and reading the planes (measured: 0.3 ms per step at 1.2e9 elements).
-  bool use_fast = fast != 0;
-  for (int b = 0; b < count; ++b) use_fast = use_fast && SelBatch::fast_ok(fj[b].w, fj[b].n);
+  bool use_fast = fast != 0, small = fast != 0;
+  for (int b = 0; b < count; ++b) {
+    small = small && SelBatch::small_ok(fj[b].n);
+    use_fast = use_fast && SelBatch::fast_ok(fj[b].w, fj[b].n);
+  }
+  if (small) use_fast = false;       // three launches do the whole select (small_select.hpp)
   const bool planes = Src::kHyper && use_fast;
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
@@ -432,8 +437,12 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     J.planes = planes ? f.w.pbits : nullptr;
     J.result = f.result;
   }
-  hipLaunchKernelGGL(k_seg_dir_batch, B.grid(stream_grid(max_dir, kBlock, 128)), dim3(kBlock), 0, s, dj);
-  run_select_batch(srcs, B, use_fast, planes ? 1 : 0, s);
+  if (small) {
+    run_small_select(srcs, B, dj, s);
+  } else {
+    hipLaunchKernelGGL(k_seg_dir_batch, B.grid(stream_grid(max_dir, kBlock, 128)), dim3(kBlock), 0, s, dj);
+    run_select_batch(srcs, B, use_fast, planes ? 1 : 0, s);
+  }
   if (planes) hipLaunchKernelGGL(k_cand_bits, B.grid(256), dim3(kBlock), 0, s, B.jobs);
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
@@ -465,7 +474,7 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     }
     prof_end(pp, s);
   }
-  launch_result(B, s);
+  if (!small) launch_result(B, s);
   return check_launch(who);
 }
 
@@ -1375,9 +1384,9 @@ extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int 
   }
   hipStream_t s = (hipStream_t)stream;
   const bool bg = g_dtype == SGA_BF16, bv = values_dtype == SGA_BF16;
-  // buckets that take the sampled-bracket path and buckets too small for it go through the
-  // chain in separate batches of up to kMaxJobs
-  for (int pass = 0; pass < 2; ++pass) {
+  // the buckets of a batch (up to kMaxJobs) take the same path: the sampled bracket, the
+  // one-workgroup path of the small buckets, or the radix passes
+  for (int pass = 0; pass < 3; ++pass) {
     FusedJob jobs[kMaxJobs];
     int cnt = 0;
     for (int b = 0; b <= n_buckets; ++b) {
@@ -1395,14 +1404,14 @@ extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int 
                     "sga_fused_workspace_bytes(n)=%zu", who, b, sel_ws_bytes(u.n));
           return SGA_ERR_WORKSPACE;
         }
-        const bool is_fast = fast != 0 && SelBatch::fast_ok(w, u.n);
-        if (is_fast != (pass == 0)) continue;
+        const int path = fast != 0 && SelBatch::small_ok(u.n) ? 1 : fast != 0 && SelBatch::fast_ok(w, u.n) ? 0 : 2;
+        if (path != pass) continue;
         jobs[cnt++] = FusedJob{u.g, u.resid, u.p, u.m, u.v, u.n, u.k, u.segs, u.n_segs, u.idx_out,
                                u.values_out, u.mask_out, u.result, w, {nullptr, nullptr, nullptr, nullptr}};
       }
       if (cnt == kMaxJobs || (b == n_buckets && cnt > 0)) {
         int rc;
-#define SGA_RUNM(BG, BV, SC) rc = run_fused<BG, BV, SC>(jobs, cnt, factor, coeff, pass == 0, flags, interval, s, 0, who); break
+#define SGA_RUNM(BG, BV, SC) rc = run_fused<BG, BV, SC>(jobs, cnt, factor, coeff, pass != 2, flags, interval, s, 0, who); break
 #define SGA_RUNM_SC(BG, BV)                    \
         switch (score_id) {                    \
           case 0: SGA_RUNM(BG, BV, 0);         \

@@ -14,7 +14,7 @@
 // configs, bf16 g: non-boundary 34 + 4/G (sel 1 | sel 1 + res 8 + m,v,w 24),
 // boundary 36 + 4/G.
 #include "adam_math.hpp"
-#include "select_impl.hpp"
+#include "small_select.hpp"
 
 namespace sga {
 
@@ -743,7 +743,8 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     any_hyper = any_hyper || score[b] == SGA_SCORE_UPDATE || score[b] == SGA_SCORE_COI ||
                 score[b] == SGA_SCORE_GR_OVER_SQRT_V;
   }
-  if (any_hyper) {                     // only the Adam-normalised scores ever look a tensor up
+  const bool small = SelBatch::small_ok(n);
+  if (any_hyper && !small) {           // only the Adam-normalised scores ever look a tensor up
     const int64_t nb = (n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
     hipLaunchKernelGGL(k_seg_dir_batch, B.grid(stream_grid(nb, kBlock, 128)), dim3(kBlock), 0, s, dj);
   }
@@ -774,6 +775,19 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
       });
     }
   };
+  if (small) {
+    per_score([&](auto& srcs, const SelBatch& sub) {
+      using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
+      SegDirJobs dirs = {};
+      for (int b = 0; Src::kHyper && b < sub.count; ++b) {
+        dirs.j[b].segs = segs; dirs.j[b].dir = sub.w[b].seg_dir; dirs.j[b].n = n; dirs.j[b].n_segs = n_segs;
+      }
+      run_small_select(srcs, sub, dirs, s);
+      hipLaunchKernelGGL((k_write_bits<Src>), sub.grid((unsigned)cdiv64(sub.max_tiles, kChunksPerBlock)),
+                         dim3(kBlock), 0, s, srcs, sub.jobs);
+    });
+    return check_launch(who);
+  }
   chain_begin(B, fast, s);
   if (fast) {
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sample(srcs, sub, s); });

@@ -1,6 +1,6 @@
 // Exact top-k selection entry points over fp32 score arrays, plus the
 // histogram / candidate / compare building blocks of the replay select.
-#include "select_impl.hpp"
+#include "small_select.hpp"
 
 namespace sga {
 int exclusive_scan_u32(uint32_t* data, int64_t n, int64_t* total, hipStream_t st);
@@ -356,6 +356,12 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   ChainJob& J = B.add(w, n, k, tie_mode == SGA_TIE_ALL);
   J.mask = mask_out;
   J.result = result;
+  if (SelBatch::small_ok(n)) {
+    run_small_select(srcs, B, SegDirJobs{}, s);
+    hipLaunchKernelGGL((k_write_mask<SrcF32>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)),
+                       dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0, 0, (uint8_t*)nullptr);
+    return check_launch("sga_select_topk");
+  }
   const bool fast = SelBatch::fast_ok(w, n);
   // the select sweep writes the keys above the bracket straight into mask_out
   run_select_batch(srcs, B, fast, 2, s);

@@ -68,13 +68,21 @@ struct SelWorkspace {
   uint32_t* cand_idx;  // dense candidates
   uint32_t* cand_key;
   uint32_t* pbits;     // 32 words per chunk: bit planes of "key above the bracket"
+  // one-workgroup path (small_select.hpp): list of the bracket's keys, shares the memory of the
+  // segments above
+  uint32_t* small_idx;
+  uint32_t* small_key;
   int64_t sample_cap;
   int64_t seg_cap;     // per-wave candidate capacity
 };
 
 constexpr int kSegWaves = 8192;            // candidate segments the sweep's chunks hash to
 constexpr int kSweepParts = 256;            // partial counters of the sweep's two totals
-constexpr int64_t kFastMinN = 1 << 20;     // below this the radix passes are cheap enough
+constexpr int64_t kFastMinN = 1 << 20;     // the sampled bracket of the large buckets begins here
+constexpr int kSmallTiles = 8192;          // up to this many chunks a bucket takes small_select.hpp
+constexpr int kSmallSegs = 16;             // list segments there (one per wave of its finishing workgroup)
+// Margin of a bracket that has a way back when it misses, in standard deviations of the sample rank.
+constexpr double kBracketSigmas = 5.0;
 
 static inline int64_t fast_sample_vecs(int64_t n) {
   int64_t v = n / 1024;
@@ -110,6 +118,8 @@ struct ChainJob {
   uint32_t* cand_idx;
   uint32_t* cand_key;
   uint32_t* seg_fail;          // single-sweep step: per-segment first failed reservation
+  uint32_t* small_idx;         // small_select.hpp: list of the bracket's keys
+  uint32_t* small_key;
   const F4* seg_rec;           // single-sweep step: records beside the segments' keys
   F4* cand_rec;
   uint32_t* planes;            // where the settlement writes the selection (bit planes) ...
@@ -134,12 +144,23 @@ constexpr int kSelDirEntries = 1 << 15;                        // n < 2^31 in bl
 constexpr size_t kSelFixedBytes =
     512 + (size_t)kHistStride * 2 * 4 + (size_t)kMaxTileBlocks * 4 * 2 + (size_t)kSelDirEntries * 4;
 
+// List entries of the small path: its kSmallSegs segments hold every coordinate of their
+// workgroups, and the last one may fall a segment's share short of full.
+static inline size_t small_list_entries(int64_t nt) {
+  const int64_t t = nt < kSmallTiles + 8 ? nt : kSmallTiles + 8;
+  return (size_t)(t + t / kSmallSegs + 4 * kChunksPerBlock) * kChunk;
+}
+// Bytes the candidate segments (four arrays) and the small path's list (two) share.  Above
+// kSmallTiles the list's share stays what it was there, so that the layout grows with nt.
+static inline size_t list_bytes_for_tiles(int64_t nt) {
+  const size_t segs = nt * kChunk < kFastMinN ? 0 : (size_t)kSegWaves * fast_seg_cap(nt * kChunk) * 16;
+  const size_t small = small_list_entries(nt) * 8;
+  return segs > small ? segs : small;
+}
 static inline size_t fast_bytes_for_tiles(int64_t nt) {
   const int64_t n = nt * kChunk;
-  if (n < kFastMinN) return 0;
-  const int64_t sc = fast_seg_cap(n);
-  return (size_t)fast_sample_vecs(n) * 16 + (size_t)(kSegWaves + 64) * 4 +
-         (size_t)kSegWaves * sc * 4 * 4 + (size_t)nt * 128 + 256;
+  const size_t always = (size_t)(kSegWaves + 64) * 4 + list_bytes_for_tiles(nt) + 256;
+  return n < kFastMinN ? always : always + (size_t)fast_sample_vecs(n) * 16 + (size_t)nt * 128;
 }
 
 static inline size_t sel_ws_bytes(int64_t n) {
@@ -179,24 +200,28 @@ static inline bool sel_ws_carve(void* ws, size_t bytes, int64_t n_tiles_needed,
   p += (size_t)nt * 4;
   out->n_tiles_cap = nt;
   out->sample = nullptr;
-  out->seg_cnt = out->seg_idx = out->seg_key = out->cand_idx = out->cand_key = nullptr;
+  out->seg_idx = out->seg_key = out->cand_idx = out->cand_key = nullptr;
   out->pbits = nullptr;
   out->sample_cap = 0;
   out->seg_cap = 0;
-  if (fast_bytes_for_tiles(nt) > 0) {
+  p = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
+  out->seg_cnt = reinterpret_cast<uint32_t*>(p);
+  p += (size_t)(kSegWaves + 64) * 4;
+  out->small_idx = reinterpret_cast<uint32_t*>(p);
+  out->small_key = out->small_idx + small_list_entries(nt);
+  if (nt * kChunk >= kFastMinN) {
     const int64_t n = nt * kChunk;
-    p = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~(uintptr_t)255);
-    out->sample_cap = fast_sample_vecs(n) * 4;
+    char* q = p;
     out->seg_cap = fast_seg_cap(n);
+    const size_t seg_bytes = (size_t)kSegWaves * out->seg_cap * 4;
+    out->seg_idx = reinterpret_cast<uint32_t*>(q); q += seg_bytes;
+    out->seg_key = reinterpret_cast<uint32_t*>(q); q += seg_bytes;
+    out->cand_idx = reinterpret_cast<uint32_t*>(q); q += seg_bytes;
+    out->cand_key = reinterpret_cast<uint32_t*>(q);
+    p += list_bytes_for_tiles(nt);
+    out->sample_cap = fast_sample_vecs(n) * 4;
     out->sample = reinterpret_cast<uint32_t*>(p);
     p += (size_t)out->sample_cap * 4;
-    out->seg_cnt = reinterpret_cast<uint32_t*>(p);
-    p += (size_t)(kSegWaves + 64) * 4;
-    const size_t seg_bytes = (size_t)kSegWaves * out->seg_cap * 4;
-    out->seg_idx = reinterpret_cast<uint32_t*>(p); p += seg_bytes;
-    out->seg_key = reinterpret_cast<uint32_t*>(p); p += seg_bytes;
-    out->cand_idx = reinterpret_cast<uint32_t*>(p); p += seg_bytes;
-    out->cand_key = reinterpret_cast<uint32_t*>(p); p += seg_bytes;
     out->pbits = reinterpret_cast<uint32_t*>(p);
   }
   return true;
@@ -793,6 +818,8 @@ struct SelBatch {
   ChainJobs jobs;
   SelWorkspace w[kMaxJobs];
   int64_t max_n = 0, max_tiles = 0, max_nsv = 0;
+  // true when the job takes the one-workgroup path of small_select.hpp
+  static bool small_ok(int64_t n) { return cdiv64(n, kChunk) <= kSmallTiles; }
   // true when the job takes the sampled-bracket path (all jobs of one batch must agree)
   static bool fast_ok(const SelWorkspace& ws, int64_t n) {
     return n >= kFastMinN && ws.sample != nullptr && n < (1ll << 32);
@@ -805,6 +832,7 @@ struct SelBatch {
     J.tile_gt = ws.tile_gt; J.tile_eq = ws.tile_eq; J.blk_gt = ws.blk_gt; J.blk_eq = ws.blk_eq;
     J.sample = ws.sample; J.seg_cnt = ws.seg_cnt; J.seg_idx = ws.seg_idx; J.seg_key = ws.seg_key;
     J.cand_idx = ws.cand_idx; J.cand_key = ws.cand_key;
+    J.small_idx = ws.small_idx; J.small_key = ws.small_key;
     J.n = n; J.n_tiles = cdiv64(n, kChunk);
     J.n_vec = n / 4;
     J.n_sv = ws.sample_cap / 4 < J.n_vec ? ws.sample_cap / 4 : J.n_vec;
@@ -1444,7 +1472,7 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 // not form keys: chain_begin, chain_sample_levels, chain_candidates, launch_tile_scan (and the
 // settlement) take the whole batch; chain_sample, chain_sweeps and chain_fallback are templates
 // of the key source and take the jobs of one kind (a sub-batch over the same workspaces).
-static inline void chain_begin(const SelBatch& B, bool fast, hipStream_t s, double sigmas = 5.0) {
+static inline void chain_begin(const SelBatch& B, bool fast, hipStream_t s, double sigmas = kBracketSigmas) {
   hipLaunchKernelGGL(k_chain_begin, B.grid(1), dim3(kBlock), 0, s, B.jobs, fast ? 1 : 0, sigmas);
 }
 template <class Src>
@@ -1502,7 +1530,7 @@ static inline void chain_fallback(const SrcPack<Src>& srcs, const SelBatch& B, h
 
 template <class Src>
 static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, bool fast, int pm,
-                                    hipStream_t s, double sigmas = 5.0) {
+                                    hipStream_t s, double sigmas = kBracketSigmas) {
   chain_begin(B, fast, s, sigmas);
   if (fast) {
     chain_sample(srcs, B, s);

@@ -1,0 +1,79 @@
+"""Exact top-k of buckets up to 8,388,608 coordinates (csrc/small_select.hpp) at
+the edges of its tiles, its lists and its sample, against the oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import select as SEL
+from tests.util import student_t
+
+pytestmark = pytest.mark.gpu
+
+LIMIT = 8192 * 1024
+
+
+def _check(dev, sc, k, what, path=None):
+    from sga_amd import _lib as L
+    from sga_amd.selection import read_result, select_exact_device
+    m_ref, t_ref = SEL.select_topk_flat(sc, k)
+    sd = sc.to(dev)
+    mask = torch.full((sc.numel(),), 7, dtype=torch.uint8, device=dev)
+    r = read_result(select_exact_device([sd], k, L.TIE_LOWEST_INDEX, masks=[mask])[0])
+    eq = int((sc == t_ref).sum())
+    assert (r.status, r.n_selected, r.thresh, r.n_eq) == (0, k, t_ref, eq), (what, vars(r))
+    assert r.n_gt == int((sc > t_ref).sum()) and r.need == k - r.n_gt, (what, vars(r))
+    assert torch.equal(mask.cpu(), m_ref.to(torch.uint8)), what
+    assert path is None or r.path == path, (what, vars(r))
+    _, (m2,) = select_exact_device([sd], k, L.TIE_ALL)
+    assert torch.equal(m2.cpu().bool(), sc >= t_ref), what
+
+
+# below one quad, around a chunk / a workgroup's span / the smallest sample, and the last size of
+# this path and the first of the large buckets'
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1025, 4095, 4097, 8191, 8193, 65_537, 1 << 20,
+                               (1 << 20) + 3, 2_097_153, LIMIT, LIMIT + 1])
+def test_sizes(dev, n):
+    sc = student_t(n, n % 97).abs()
+    for k in sorted({1, max(1, n // 100), max(1, n // 3), n}):
+        _check(dev, sc, k, (n, k))
+
+
+@pytest.mark.parametrize("n", [200_003, 1_500_001, 4_194_304])
+def test_plateaus_and_crowded_chunks(dev, n):
+    base = student_t(n, 5).abs()
+    zeros = torch.where(base > base.kthvalue(n - n // 50)[0], base, torch.zeros(()))   # 2 % not zero
+    for k in (n // 100, n // 50 - 1, n // 50, n // 50 + 1, n // 50 + n // 2000, n // 10):
+        _check(dev, zeros, k, ("zeros", n, k))                    # ends inside, at and past the zeros
+    grid = base.to(torch.bfloat16).float()                        # ties everywhere
+    hot = base * 1e-6
+    hot[n // 2:n // 2 + n // 40] += 1.0                           # the top keys crowd into a few chunks
+    steep = 1.0 + base * 1e-4                                     # all keys in one sixteenth of an octave
+    for name, sc in (("grid", grid), ("hot", hot), ("steep", steep)):
+        for k in (n // 1000, n // 100, n // 41, n // 10):
+            _check(dev, sc, k, (name, n, k))
+
+
+def _mix32(x):
+    x = x.astype(np.uint32)
+    x ^= x >> np.uint32(16)
+    x *= np.uint32(0x7FEB352D)
+    x ^= x >> np.uint32(15)
+    x *= np.uint32(0x846CA68B)
+    return x ^ (x >> np.uint32(16))
+
+
+@pytest.mark.parametrize("n", [50_001, 2_000_003])
+@pytest.mark.parametrize("side", ["low", "high"])
+def test_a_missed_bracket_is_redone_over_the_data(dev, n, side):
+    """Keys planted at the restated sample positions put the bracket far below
+    (above) the k-th key: the finishing workgroup selects over the data itself."""
+    n_vec = n // 4
+    n_sv = min(n_vec, min(max(n // 512, 2048), 4096))
+    j = np.arange(n_sv, dtype=np.int64)
+    w0, w1 = j * n_vec // n_sv, (j + 1) * n_vec // n_sv
+    vec = w0 + _mix32(j.astype(np.uint32)).astype(np.int64) % (w1 - w0)
+    pos = torch.from_numpy((vec[:, None] * 4 + np.arange(4)).reshape(-1))
+    sc = student_t(n, 3).abs() + 1.0
+    sc[pos] = sc[pos] * (1e-9 if side == "low" else 1e9)
+    for k in (n // 100, n // 2):
+        _check(dev, sc, k, (side, n, k), path=0 if side == "low" else None)
