@@ -550,6 +550,14 @@ typedef struct sga_replay_segment {
   float beta1, om1, beta2, om2, eps, bc1, bc2, wdf;
 } sga_replay_segment;
 
+/* What changes in a segment table from step to step -- learning rates and bias
+ * corrections -- written into the DEVICE tables segs and / or rsegs (either may
+ * be NULL) of the same n_segs tensors.  lr, bc1, bc2: HOST arrays of n_segs;
+ * they travel in the kernel arguments, so the call neither stages nor waits. */
+int sga_segments_refresh(sga_segment* segs, sga_replay_segment* rsegs,
+                         int n_segs, const double* lr, const float* bc1,
+                         const float* bc2, void* stream);
+
 /* pass 1 (replay_fused.py:1682-1743): qn2[c] = sum q_pre^2 over the shard
  * (fp32 products, double accumulation, fixed order), coef[c] in double and
  * fp32.  partials: sga_replay_partials() doubles.  cfgs is a HOST array. */

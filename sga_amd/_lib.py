@@ -91,6 +91,7 @@ SIGNATURES = {
     "sga_gt_eq": (I32, [P, I64, F, P, P, P, P]),
     "sga_score_formula": (I32, [I32, P, P, P, P, P, I64] + [F] * 8 + [I32, I32, P]),
     "sga_opt_step_inplace": (I32, [P, P, P, P, P, P, I64] + [F] * 13 + [I32, P]),
+    "sga_segments_refresh": (I32, [P, P, I32, P, P, P, P]),
     "sga_replay_partials": (I64, []),
     "sga_replay_pass1": (I32, [P, I32, I64, F, C.c_double, P, I32, P, P, P, P, P]),
     "sga_replay_reselect": (I32, [P, I32, P, P, P, P, I64, I64, P, I32, I32, P, F, I32, I32, I32,
@@ -222,7 +223,7 @@ def check(rc, name):
 
 def call(name, *args):
     """Invoke an int-returning entry point; raise with the library's text."""
-    lib = load()
+    lib = _lib or load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         raise RuntimeError(f"{name} failed ({rc}): "
@@ -233,9 +234,12 @@ def raw(name, *args):
     return getattr(load(), name)(*args)
 
 
+_F32 = struct.Struct("f")
+
+
 def f32(x):
     """Round a Python float to fp32 (nearest-even), back as a Python float."""
-    return struct.unpack("f", struct.pack("f", float(x)))[0]
+    return _F32.unpack(_F32.pack(x))[0]
 
 
 def require_dev(*tensors):
@@ -253,7 +257,9 @@ def require_contig(**named):
 
 
 def ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    """Device address for a ``P`` argument (a plain int: wrapping it in a
+    ``c_void_p`` costs more than reading it)."""
+    return None if t is None else t.data_ptr()
 
 
 def stream():

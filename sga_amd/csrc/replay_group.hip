@@ -633,6 +633,46 @@ static void launch_pass1(int n_b, unsigned nb, hipStream_t s, const void* g, int
 #undef SGA_P1
 }
 
+// The changing columns of a segment table, by value in the kernel arguments: a launch writes up to N
+// rows.  (Rebuilding and copying the whole table per step took 11 us of host time for the staging
+// copy and its event, and as much again per 20 tensors to fill the rows in Python.)
+namespace sga {
+template <int N>
+struct SegCols { double lr[N]; float bc1[N], bc2[N]; };
+template <int N>
+__global__ __launch_bounds__(N) void k_segments_refresh(sga_segment* __restrict__ segs,
+                                                        sga_replay_segment* __restrict__ rsegs, int base,
+                                                        int count, SegCols<N> c) {
+  const int i = threadIdx.x;
+  if (i >= count) return;
+  if (segs) { segs[base + i].lr = (float)c.lr[i]; segs[base + i].bc1 = c.bc1[i]; segs[base + i].bc2 = c.bc2[i]; }
+  if (rsegs) { rsegs[base + i].lr = c.lr[i]; rsegs[base + i].bc1 = c.bc1[i]; rsegs[base + i].bc2 = c.bc2[i]; }
+}
+template <int N>
+static void launch_refresh(sga_segment* segs, sga_replay_segment* rsegs, int base, int count, const double* lr,
+                           const float* bc1, const float* bc2, hipStream_t s) {
+  SegCols<N> c;
+  for (int i = 0; i < count; ++i) { c.lr[i] = lr[base + i]; c.bc1[i] = bc1[base + i]; c.bc2[i] = bc2[base + i]; }
+  hipLaunchKernelGGL((k_segments_refresh<N>), dim3(1), dim3(N), 0, s, segs, rsegs, base, count, c);
+}
+}  // namespace sga
+
+extern "C" int sga_segments_refresh(sga_segment* segs, sga_replay_segment* rsegs, int n_segs, const double* lr,
+                                    const float* bc1, const float* bc2, void* stream) {
+  if ((!segs && !rsegs) || n_segs < 1 || !lr || !bc1 || !bc2) {
+    set_error("sga_segments_refresh: bad argument (n_segs=%d)", n_segs);
+    return SGA_ERR_ARG;
+  }
+  // 240 rows fill the 4 KiB of kernel arguments; a small table takes the 64-row form (1 KiB less to
+  // copy per launch)
+  for (int base = 0; base < n_segs; base += 240) {
+    const int count = n_segs - base < 240 ? n_segs - base : 240;
+    if (count <= 64) launch_refresh<64>(segs, rsegs, base, count, lr, bc1, bc2, (hipStream_t)stream);
+    else launch_refresh<240>(segs, rsegs, base, count, lr, bc1, bc2, (hipStream_t)stream);
+  }
+  return check_launch("sga_segments_refresh");
+}
+
 extern "C" int64_t sga_replay_partials(void) { return (int64_t)kReplayBlocks * kMaxCfg; }
 
 extern "C" int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coef_dense, double clip,

@@ -1,12 +1,11 @@
 """Fused per-rank sparse step over a flat bucket (engine order of
 ``sga/engine.py:416-604``): score -> exact top-k -> index pack -> residual
 update -> residual-aware AdamW, as two kinds of sweeps over HBM."""
-import ctypes as C
-
 import torch
 
 from . import _lib as L
 from .scores import STEP_SCORE_MAP as SCORE_MAP
+from .segments import SegmentTable
 from .selection import read_result
 
 
@@ -50,16 +49,10 @@ class FusedSparseStep:
         self.values = torch.empty(self.max_k, dtype=values_dtype, device=device)
         self.mask = (torch.empty(n, dtype=torch.uint8, device=device)
                      if want_mask else None)
-        self._seg_host = (L.Segment * len(segments))()
-        for e, s in zip(self._seg_host, segments):
-            e.start, e.n = s["start"], s["n"]
-            e.lr = L.f32(s["lr"])
-            e.beta1, e.om1 = L.f32(s["b1"]), L.f32(1.0 - s["b1"])
-            e.beta2, e.om2 = L.f32(s["b2"]), L.f32(1.0 - s["b2"])
-            e.eps, e.wd = L.f32(s["eps"]), L.f32(s["wd"])
-        self._seg_up = L.TableUploader(C.sizeof(self._seg_host), device)
-        self._seg_dev = self._seg_up.dev
+        self._seg_table = SegmentTable(segments, device)
+        self._seg_dev = self._seg_table.segs
         self._seg_step = None
+        self._views = (None, None, None)
         self._ws2 = None          # second workspace of the single-sweep step, on first use
         self._calls = 0
 
@@ -73,14 +66,8 @@ class FusedSparseStep:
     def _upload_segments(self, step):
         if self._seg_step == step:
             return
-        bc = {}
-        for e, s in zip(self._seg_host, self.segments):
-            key = (s["b1"], s["b2"])
-            if key not in bc:
-                bc[key] = (L.f32(1.0 - s["b1"] ** step), L.f32(1.0 - s["b2"] ** step))
-            e.lr = L.f32(s["lr"])                      # callers may retune lr between steps
-            e.bc1, e.bc2 = bc[key]
-        self._seg_up.upload(self._seg_host)
+        # callers may retune lr between steps
+        self._seg_table.refresh([s["lr"] for s in self.segments], step)
         self._seg_step = step
 
     @staticmethod
@@ -137,7 +124,13 @@ class FusedSparseStep:
         else:
             L.call(name, *head, 1 if fast else 0, flags, L.f32(interval), L.ptr(result),
                    L.ptr(self.ws), self.ws_bytes, L.stream())
-        return self.idx[:k], self.values[:k]
+        return self._pack_views(k)
+
+    def _pack_views(self, k):
+        """(idx[:k], values[:k]); the views of the last k are kept (1 us each to make)."""
+        if self._views[0] != k:
+            self._views = (k, self.idx[:k], self.values[:k])
+        return self._views[1:]
 
     def step(self, g, resid, p, m, v, step, k=None, ratio_percent=None,
              score="abs_g", factor=1.0, coeff=1.0, fast=True, optimizer="adamw", fold=False,
@@ -275,7 +268,7 @@ def fused_step_multi(steppers, grads, resids, ps, ms, vs, step, ks=None, ratio_p
         e.ws, e.ws_bytes = fs.ws.data_ptr(), fs.ws_bytes
     L.call("sga_fused_sparse_step_multi", table, nb, gd, SCORE_MAP[score], vd, L.f32(factor),
            L.f32(coeff), 1 if fast else 0, flags, L.f32(interval), L.stream())
-    return [(fs.idx[:k], fs.values[:k]) for fs, k in zip(steppers, ks)]
+    return [fs._pack_views(k) for fs, k in zip(steppers, ks)]
 
 
 class PackedState:

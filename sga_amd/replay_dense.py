@@ -8,14 +8,13 @@ State is flat over the shard (one launch per recorded step, per-tensor
 hyper-parameters through a segment table) and the snapshots stay resident on
 the device, where the sparse arms compare against them.
 """
-import ctypes as C
 import math
 
 import torch
 
 from . import _lib as L
-from .replay import _bc_pair, coef_dense_for
-from .replay_group import ReplaySegment
+from .replay import coef_dense_for
+from .segments import SegmentTable
 from .trace_io import lr_for_step
 
 
@@ -26,6 +25,12 @@ def lr_max_abs_diff(gmeta):
         return 0.0
     mean = sum(lrs) / len(lrs)
     return max(abs(x - mean) for x in lrs)
+
+
+def lr_by_group(gmeta, entries):
+    """``lr_for_step`` of every entry, each group looked up once."""
+    of = {g: float(lr_for_step(gmeta, g)) for g in {e.get("group") for e in entries}}
+    return [of[e.get("group")] for e in entries]
 
 
 class DenseReplay:
@@ -46,9 +51,8 @@ class DenseReplay:
                                      device=dev)
         self._recon2 = torch.zeros(1, dtype=torch.float64, device=dev)
         self._dist = torch.zeros(1, dtype=torch.float64, device=dev)
-        self._seg_host = (ReplaySegment * len(entries))()
-        self._seg_up = L.TableUploader(C.sizeof(self._seg_host), dev)
-        self._seg_dev = self._seg_up.dev
+        self._seg_table = SegmentTable(entries, dev, start="a", segs=False, rsegs=True)
+        self._seg_dev = self._seg_table.rsegs
         self.si = 0
         self.den_at, self.snapshots, self.recon_steps = {}, {}, []
 
@@ -61,15 +65,7 @@ class DenseReplay:
             raise ValueError("gradient length does not match the shard")
         coef_dense, flag = coef_dense_for(gmeta)
         count = self.t0 + self.si + 1
-        for i, e in enumerate(self.entries):
-            r = self._seg_host[i]
-            bc1, bc2 = _bc_pair(self.optimizer, count, e["b1"], e["b2"])
-            r.start, r.n = e["a"], e["n"]
-            r.lr, r.wd = float(lr_for_step(gmeta, e.get("group"))), float(e["wd"])
-            r.beta1, r.om1 = L.f32(e["b1"]), L.f32(1.0 - e["b1"])
-            r.beta2, r.om2 = L.f32(e["b2"]), L.f32(1.0 - e["b2"])
-            r.eps, r.wdf, r.bc1, r.bc2 = L.f32(e["eps"]), L.f32(e["wd"]), L.f32(bc1), L.f32(bc2)
-        self._seg_up.upload(self._seg_host)
+        self._seg_table.refresh(lr_by_group(gmeta, self.entries), count, self.optimizer == "adamw")
         st = L.stream()
         L.call("sga_dense_replay_step", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),
                L.ptr(self.v), L.ptr(self.label), self.N, L.ptr(self._seg_dev),

@@ -12,6 +12,7 @@ import torch
 
 from . import _lib as L
 from .scores import STEP_SCORE_MAP as SCORE_MAP
+from .segments import ReplaySegment, SegmentTable  # noqa: F401 (the table's row type)
 from .selection import read_result
 
 MAX_CONFIGS = 16
@@ -27,14 +28,6 @@ class ReplayCfg(C.Structure):
                 ("sel", C.c_void_p), ("out_sel", C.c_void_p), ("lr_scale", C.c_double),
                 ("boundary", C.c_int), ("adams", C.c_int), ("split", C.c_int), ("packed", C.c_int),
                 ("res_zero", C.c_int), ("pad_", C.c_int)]
-
-
-class ReplaySegment(C.Structure):
-    """struct sga_replay_segment"""
-    _fields_ = [("start", C.c_int64), ("n", C.c_int64), ("lr", C.c_double), ("wd", C.c_double),
-                ("beta1", C.c_float), ("om1", C.c_float), ("beta2", C.c_float),
-                ("om2", C.c_float), ("eps", C.c_float), ("bc1", C.c_float), ("bc2", C.c_float),
-                ("wdf", C.c_float)]
 
 
 class Config:
@@ -153,12 +146,8 @@ class ReplayGroup:
             self._bal_hist = torch.zeros(int(L.raw("sga_balanced_hist_words")),
                                          dtype=torch.int32, device=dev)
         self._cfg_host = (ReplayCfg * G)()
-        self._rseg_host = (ReplaySegment * len(entries))()
-        self._rseg_up = L.TableUploader(C.sizeof(self._rseg_host), dev)
-        self._rseg_dev = self._rseg_up.dev
-        self._seg_host = (L.Segment * len(entries))()
-        self._seg_up = L.TableUploader(C.sizeof(self._seg_host), dev)
-        self._seg_dev = self._seg_up.dev
+        self._seg_table = SegmentTable(entries, dev, start="a", segs=True, rsegs=True)
+        self._seg_dev, self._rseg_dev = self._seg_table.segs, self._seg_table.rsegs
         self.dist_at = [dict() for _ in configs]
         # res is all zeros at the start and again after every boundary commit;
         # the kernels then skip its traffic (same values either way)
@@ -171,23 +160,6 @@ class ReplayGroup:
         return self._ws[j]
 
     # -- per-step tables ----------------------------------------------------
-    def _fill_segments(self, count, lr_of):
-        for i, e in enumerate(self.entries):
-            r = self._rseg_host[i]
-            r.start, r.n = e["a"], e["n"]
-            r.lr, r.wd = float(lr_of(e)), float(e["wd"])
-            r.beta1, r.om1 = L.f32(e["b1"]), L.f32(1.0 - e["b1"])
-            r.beta2, r.om2 = L.f32(e["b2"]), L.f32(1.0 - e["b2"])
-            r.eps, r.wdf = L.f32(e["eps"]), L.f32(e["wd"])
-            r.bc1 = L.f32(1.0 - e["b1"] ** count)
-            r.bc2 = L.f32(1.0 - e["b2"] ** count)
-            s = self._seg_host[i]
-            s.start, s.n, s.lr = e["a"], e["n"], L.f32(lr_of(e))
-            s.beta1, s.om1, s.beta2, s.om2 = r.beta1, r.om1, r.beta2, r.om2
-            s.eps, s.wd, s.bc1, s.bc2 = r.eps, r.wdf, r.bc1, r.bc2
-        self._rseg_up.upload(self._rseg_host)
-        self._seg_up.upload(self._seg_host)
-
     def _fill_cfgs(self, bnd, out_sel):
         for ci, c in enumerate(self.configs):
             s, h = self.state[ci], self._cfg_host[ci]
@@ -210,7 +182,6 @@ class ReplayGroup:
         clip = float(meta.get("clip_grad", 0.0))
         coef_dense = coef_dense_for(clip, float(meta.get("grad_norm", float("nan"))))
         lr = meta["lr"]
-        lr_of = lr if callable(lr) else (lambda e: lr)
         count = self.t0 + si + 1
         bnd = [si % c.T == 0 for c in self.configs]
         st = L.stream()
@@ -219,7 +190,7 @@ class ReplayGroup:
                 if bnd[ci] and c.fold and not self.res_zero[ci]:
                     L.call("sga_div_inplace", C.c_void_p(self.state[ci].base("res")), N,
                            L.f32(float(c.T)), 1, st)
-        self._fill_segments(count, lr_of)
+        self._seg_table.refresh([float(lr(e)) for e in self.entries] if callable(lr) else float(lr), count)
         self._fill_cfgs(bnd, {})
         gd = L.dtype_code(g)
         L.call("sga_replay_pass1", L.ptr(g), gd, N, L.f32(coef_dense), clip, self._cfg_host, G,

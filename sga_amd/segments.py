@@ -1,0 +1,65 @@
+"""Device tables of per-tensor hyper-parameters, laid out once per bucket or
+shard; a step only rewrites the learning rates and the bias corrections
+(``sga_segments_refresh``: the values travel in the kernel arguments, nothing
+is staged or waited for)."""
+import ctypes as C
+
+import numpy as np
+import torch
+
+from . import _lib as L
+
+
+class ReplaySegment(C.Structure):
+    """struct sga_replay_segment"""
+    _fields_ = [("start", C.c_int64), ("n", C.c_int64), ("lr", C.c_double), ("wd", C.c_double),
+                ("beta1", C.c_float), ("om1", C.c_float), ("beta2", C.c_float),
+                ("om2", C.c_float), ("eps", C.c_float), ("bc1", C.c_float), ("bc2", C.c_float),
+                ("wdf", C.c_float)]
+
+
+_SEGMENT, _REPLAY_SEGMENT = np.dtype(L.Segment), np.dtype(ReplaySegment)
+
+
+def _device_table(dtype, rows, start, device):
+    t = np.zeros(len(rows), dtype=dtype)
+    t["start"], t["n"] = [r[start] for r in rows], [r["n"] for r in rows]
+    # numpy rounds a Python float to nearest fp32, like a store into a C float
+    for name, values in (("beta1", [r["b1"] for r in rows]), ("om1", [1.0 - r["b1"] for r in rows]),
+                         ("beta2", [r["b2"] for r in rows]), ("om2", [1.0 - r["b2"] for r in rows]),
+                         ("eps", [r["eps"] for r in rows]), ("wd", [r["wd"] for r in rows])):
+        t[name] = values
+    if dtype is _REPLAY_SEGMENT:
+        t["wdf"] = [r["wd"] for r in rows]
+    return torch.from_numpy(t.view(np.uint8)).to(device)
+
+
+class SegmentTable:
+    """``rows``: dicts with ``n, b1, b2, eps, wd`` and the first coordinate under
+    ``start``.  ``segs`` / ``rsegs`` are the device tables (``sga_segment`` /
+    ``sga_replay_segment``) that were asked for."""
+
+    def __init__(self, rows, device, start="start", segs=True, rsegs=False):
+        self.count = len(rows)
+        self.segs = _device_table(_SEGMENT, rows, start, device) if segs else None
+        self.rsegs = _device_table(_REPLAY_SEGMENT, rows, start, device) if rsegs else None
+        self._lr, self._bc1, self._bc2 = (np.zeros(self.count, dtype=d) for d in ("f8", "f4", "f4"))
+        self._args = (None if self.segs is None else self.segs.data_ptr(),
+                      None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
+                      self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
+        groups = {}
+        for i, r in enumerate(rows):
+            groups.setdefault((r["b1"], r["b2"]), []).append(i)
+        self._groups = [(b, slice(None) if len(groups) == 1 else np.array(at)) for b, at in groups.items()]
+        self._last_lr = None
+
+    def refresh(self, lr, count, bias_correction=True):
+        """Learning rates (one float, or one per row) and the bias corrections of
+        step ``count``, on the current stream."""
+        if lr != self._last_lr:
+            self._lr[:] = lr
+            self._last_lr = lr
+        for (b1, b2), at in self._groups:
+            self._bc1[at] = 1.0 - b1 ** count if bias_correction else 1.0
+            self._bc2[at] = 1.0 - b2 ** count if bias_correction else 1.0
+        L.call("sga_segments_refresh", *self._args, L.stream())

@@ -8,6 +8,7 @@ gather); ``balanced`` / ``fast`` keep the reference's stride-8 subsample
 histogram and crossing-bin rule so the masks are identical to its.
 """
 import ctypes as C
+import struct
 from types import SimpleNamespace
 
 import torch
@@ -27,19 +28,23 @@ class SelectResult(C.Structure):
                  "status", "path")]
 
 
+def _f32_of(bits):
+    """The fp32 value with these bits (given as a signed or unsigned int32)."""
+    return struct.unpack("<f", struct.pack("<I", bits & 0xFFFFFFFF))[0]
+
+
 def read_result(res_t):
     """Decode a device uint32[8] result block (one host sync)."""
     r = res_t.cpu().tolist()
     out = SimpleNamespace(thresh_bits=r[0], need=r[1], n_gt=r[2], n_eq=r[3],
                           n_selected=r[4], nonfinite=r[5], status=r[6], path=r[7] & 0xFF,
                           negative=bool(r[7] & 0x100), redone=bool(r[7] & 0x200))
-    out.thresh = torch.tensor([r[0]], dtype=torch.int32).view(torch.float32).item()
+    out.thresh = _f32_of(r[0])
     return out
 
 
 def _bin_edge_float(b, shift):
-    bits = (b << shift) & 0x7FFFFFFF
-    return torch.tensor([bits], dtype=torch.int32).view(torch.float32).item()
+    return _f32_of((b << shift) & 0x7FFFFFFF)
 
 
 def _sampled_count(n, stride, phase=0):

@@ -84,3 +84,27 @@ def test_commit_tables(dev, count, phase):
                                fold=phase == "sparse_fold", interval=4.0)
     for k in t:
         assert torch.equal(t[k], ref[k]), k
+
+
+# a launch writes 64 or 240 rows: one short of, at and past both, and several launches
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 239, 240, 241, 500])
+def test_segment_table_refresh(dev, count):
+    import ctypes
+    from sga_amd import _lib as L
+    from sga_amd.segments import ReplaySegment, SegmentTable
+    rows = [dict(start=17 * i, n=17, b1=(0.9, 0.8)[i % 2], b2=0.95 + 0.01 * (i % 3), eps=1e-8, wd=0.1 * (i % 2))
+            for i in range(count)]
+    table = SegmentTable(rows, dev, segs=True, rsegs=True)
+    for step, lr in ((1, 1e-4), (7, [1e-3 * (1 + i) for i in range(count)]), (8, 2e-4)):
+        table.refresh(lr, step)
+        got = (L.Segment * count).from_buffer_copy(bytes(table.segs.cpu().numpy()))
+        rgot = (ReplaySegment * count).from_buffer_copy(bytes(table.rsegs.cpu().numpy()))
+        for i, r in enumerate(rows):
+            x = lr if isinstance(lr, float) else lr[i]
+            want = [r["start"], r["n"]] + [L.f32(v) for v in (
+                x, r["b1"], 1.0 - r["b1"], r["b2"], 1.0 - r["b2"], r["eps"], r["wd"], 1.0 - r["b1"] ** step,
+                1.0 - r["b2"] ** step)]
+            assert [getattr(got[i], f[0]) for f in got[i]._fields_][:-1] == want, (step, i)
+            assert (rgot[i].lr, rgot[i].wd, rgot[i].bc1, rgot[i].bc2, rgot[i].om2) == \
+                (x, r["wd"], want[-2], want[-1], want[6]), (step, i)
+    assert ctypes.sizeof(L.Segment) * count == table.segs.numel()
