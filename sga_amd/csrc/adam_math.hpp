@@ -161,14 +161,10 @@ static __global__ __launch_bounds__(kBlock) void k_seg_dir(const sga_segment* __
                                                            int32_t* __restrict__ dir) {
   seg_dir_body(segs, n_segs, n, dir);
 }
-// The directories of up to 8 tables in one launch (blockIdx.y = table).
+// The tables of up to 8 jobs whose directories a batched kernel builds on the way.
 struct SegDirJobs {
   struct { const sga_segment* segs; int32_t* dir; int64_t n; int n_segs; } j[8];
 };
-static __global__ __launch_bounds__(kBlock) void k_seg_dir_batch(SegDirJobs jobs) {
-  const auto& J = jobs.j[blockIdx.y];
-  seg_dir_body(J.segs, J.n_segs, J.n, J.dir);
-}
 static inline void launch_seg_dir(const sga_segment* segs, int n_segs, int64_t n, int32_t* dir,
                                   hipStream_t s) {
   const int64_t nb = (n + (1ll << kSegDirLog) - 1) >> kSegDirLog;

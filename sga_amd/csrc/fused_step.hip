@@ -410,7 +410,6 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   SegDirJobs dj = {};
   SelBatch B;
   bool vec[kMaxJobs];
-  int64_t max_dir = 0;
   // Adam-normalised scores with the one-sweep select armed: the sweep leaves the selection as bit
   // planes (settled by the candidates) and the final sweep reads one bit per coordinate instead of
   // evaluating the score chain a second time; if the bracket fails on the device, the key-forming
@@ -431,8 +430,6 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     srcs.s[b] = Src{f.g, f.resid, f.p, f.m, f.v, vec[b], {}, pack_extra, adams};
     srcs.s[b].sc.init(f.segs, f.n_segs, f.w.seg_dir);
     dj.j[b].segs = f.segs; dj.j[b].dir = f.w.seg_dir; dj.j[b].n = f.n; dj.j[b].n_segs = f.n_segs;
-    const int64_t nb = (f.n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
-    if (nb > max_dir) max_dir = nb;
     ChainJob& J = B.add(f.w, f.n, f.k, 0);
     J.planes = planes ? f.w.pbits : nullptr;
     J.result = f.result;
@@ -440,10 +437,8 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   if (small) {
     run_small_select(srcs, B, dj, s);
   } else {
-    hipLaunchKernelGGL(k_seg_dir_batch, B.grid(stream_grid(max_dir, kBlock, 128)), dim3(kBlock), 0, s, dj);
-    run_select_batch(srcs, B, use_fast, planes ? 1 : 0, s);
+    run_select_batch(srcs, B, dj, use_fast, planes ? 1 : 0, s);
   }
-  if (planes) hipLaunchKernelGGL(k_cand_bits, B.grid(256), dim3(kBlock), 0, s, B.jobs);
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
     const SelWorkspace& w = f.w;
@@ -702,19 +697,16 @@ __device__ __forceinline__ void spec_slab(const FinalArgs& a, const SpecArgs& sa
 template <bool BF16G, bool BF16V, int SCORE>
 __global__ __launch_bounds__(kBlock) void k_fused_spec(
     FinalArgs a, SpecArgs sa, const sga_segment* __restrict__ segs, int n_segs,
-    SelState* __restrict__ st, const SelState* __restrict__ aux,
-    const int32_t* __restrict__ seg_dir) {
+    SelState* __restrict__ st, const int32_t* __restrict__ seg_dir) {
   __shared__ uint32_t s_hi[kChunksPerBlock], s_nf[kChunksPerBlock];
   __shared__ SpecLds s_lds[kChunksPerBlock];
   // the sample's own count of keys inside the bracket predicts the records
-  const SelState hi = aux[0], lo = aux[1];
-  if (lo.skip) return;                                   // open below: nothing bounds the records
-  const double in_bracket = (double)(lo.k - lo.need + lo.n_eq) - (hi.skip ? 0.0 : (double)(hi.k - hi.need));
-  if (in_bracket * sa.n_over_ns > sa.est_limit) return;  // plateau inside the bracket: stand back
-  const uint32_t T_HI = hi.skip ? 0x80000000u : hi.thresh_bits + 1u;
-  const uint32_t T_LO = lo.thresh_bits;
+  const uint32_t in_sample = st->in_sample;
+  if (in_sample == ~0u) return;                          // open below: nothing bounds the records
+  if ((double)in_sample * sa.n_over_ns > sa.est_limit) return;  // plateau inside the bracket: stand back
+  const uint32_t T_HI = st->t_hi, T_LO = st->t_lo;
   const uint32_t T_MID = spec_mid(T_LO, T_HI);
-  if (blockIdx.x == 0 && threadIdx.x == 0) { st->t_lo = T_LO; st->t_hi = T_HI; st->spec = 1u; }
+  if (blockIdx.x == 0 && threadIdx.x == 0) st->spec = 1u;
   const int64_t n_chunks = cdiv64(a.n, kChunk);
   const unsigned blk = a.pack_extra != 0 ? xcd_contiguous_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const int64_t c = (int64_t)blk * kChunksPerBlock + wave_id();
@@ -1173,7 +1165,8 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
                              aligned4(out[3], 4)));
   const int adams = (flags & SGA_GC_ADAMS) ? 1 : 0;
   SrcFused<BF16G, SCORE> src{g, resid, p, m, v, vec, {}, pack_extra, adams};
-  launch_seg_dir(segs, n_segs, n, w.seg_dir, s);
+  SegDirJobs dirs = {};
+  dirs.j[0].segs = segs; dirs.j[0].dir = w.seg_dir; dirs.j[0].n = n; dirs.j[0].n_segs = n_segs;
   src.sc.init(segs, n_segs, w.seg_dir);
   const int64_t n_tiles = cdiv64(n, kChunk);
   FinalArgs fa;
@@ -1195,11 +1188,7 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   J.seed = seed; J.spec = out ? 2 : 1; J.ovf_cap = (uint32_t)x.ovf_cap; J.seg_fail = x.seg_fail;
   J.seg_rec = x.seg_rec; J.cand_rec = x.cand_rec; J.result = result;
   const int64_t ns = J.n_sv * 4;
-  hipLaunchKernelGGL(k_chain_begin, B.grid(1), dim3(kBlock), 0, s, B.jobs, 1,
-                     out ? kSpecSigmasOut : kSpecSigmas);
-  hipLaunchKernelGGL((k_sample<SrcFused<BF16G, SCORE>>), B.grid(stream_grid(B.max_nsv, kBlock)),
-                     dim3(kBlock), 0, s, srcs, B.jobs);
-  for (int level = 0; level < 3; ++level) launch_level_raw<false>(B, level, s, kRawKeyBlocks);
+  chain_bracket(srcs, B, dirs, out ? kSpecSigmasOut : kSpecSigmas, s);
   // the sweep
   SpecArgs sa;
   sa.splane = w.pbits; sa.fplane = x.dplane; sa.stage = x.stage;
@@ -1214,14 +1203,14 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   const dim3 one_shot((unsigned)cdiv64(n_tiles, kChunksPerBlock));
   ProfPair* pp = prof_begin(SGA_PROF_FUSED_FINAL, s);
   hipLaunchKernelGGL((k_fused_spec<BF16G, BF16V, SCORE>), one_shot, dim3(kBlock), 0, s, fa, sa, segs,
-                     n_segs, w.st, w.aux, w.seg_dir);
+                     n_segs, w.st, w.seg_dir);
   prof_end(pp, s);
   hipLaunchKernelGGL(k_bracket_check, B.grid(1), dim3(kBlock), 0, s, B.jobs);
   hipLaunchKernelGGL(k_cand_compact, B.grid(kSegWaves / kChunksPerBlock), dim3(kBlock), 0, s, B.jobs);
   hipLaunchKernelGGL(k_spec_ovf_compact, dim3(64), dim3(kBlock), 0, s, w.aux, w.seg_cnt, x.ovf_idx,
                      x.ovf_key, x.ovf_rec, (uint32_t)x.ovf_cap, w.cand_idx, w.cand_key, x.cand_rec,
                      x.tie_cnt);
-  for (int level = 0; level < 3; ++level) launch_level_raw<true>(B, level, s, 3 * kRawKeyBlocks);
+  for (int level = 0; level < 3; ++level) launch_level_raw(B, level, s, 3 * kRawKeyBlocks);
   hipLaunchKernelGGL(k_cand_tiles, B.grid(512), dim3(kBlock), 0, s, B.jobs);
   // only when the sweep stood back: the radix passes over the untouched data
   for (int level = 0; level < 3; ++level)

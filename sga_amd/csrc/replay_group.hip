@@ -778,16 +778,13 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     dj.j[b].segs = segs; dj.j[b].dir = r.ws.seg_dir; dj.j[b].n = n; dj.j[b].n_segs = n_segs;
     ChainJob& J = B.add(r.ws, n, r.k, 0);
     J.planes = r.sel_out;
+    J.mask_only = 1;
     J.result = r.result;
     fast = fast && SelBatch::fast_ok(r.ws, n);
     any_hyper = any_hyper || score[b] == SGA_SCORE_UPDATE || score[b] == SGA_SCORE_COI ||
                 score[b] == SGA_SCORE_GR_OVER_SQRT_V;
   }
   const bool small = SelBatch::small_ok(n);
-  if (any_hyper && !small) {           // only the Adam-normalised scores ever look a tensor up
-    const int64_t nb = (n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
-    hipLaunchKernelGGL(k_seg_dir_batch, B.grid(stream_grid(nb, kBlock, 128)), dim3(kBlock), 0, s, dj);
-  }
   // the jobs of one score, as a sub-batch over the same workspaces, and their key sources
   auto per_score = [&](auto&& phase) {
     bool seen[SGA_SCORE_GR_OVER_SQRT_V + 1] = {};
@@ -828,16 +825,19 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     });
     return check_launch(who);
   }
-  chain_begin(B, fast, s);
+  if (!any_hyper) dj = {};               // only the Adam-normalised scores ever look a tensor up
+  chain_begin(B, dj, fast, s);
   if (fast) {
-    per_score([&](auto& srcs, const SelBatch& sub) { chain_sample(srcs, sub, s); });
-    chain_sample_levels(B, s);
+    per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_coarse(srcs, sub, SegDirJobs{}, true, s); });
+    chain_pick_coarse(B, kBracketSigmas, s);
+    per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, s); });
+    chain_pick_fine(B, kBracketSigmas, s);
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, 1, s); });
-    chain_candidates(B, s);
+    chain_settle(B, s);
   }
   per_score([&](auto& srcs, const SelBatch& sub) { chain_fallback(srcs, sub, s); });
   launch_tile_scan(B, s);
-  if (fast) hipLaunchKernelGGL(k_cand_bits, B.grid(256), dim3(kBlock), 0, s, B.jobs);
+  if (fast) chain_settle_ties(B, s);
   per_score([&](auto& srcs, const SelBatch& sub) {
     using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
     hipLaunchKernelGGL((k_write_bits<Src>), sub.grid(stream_grid(sub.max_tiles, kChunksPerBlock, 1 << 14)),

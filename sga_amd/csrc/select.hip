@@ -253,7 +253,7 @@ extern "C" int sga_sel_begin(int64_t k, void* ws, size_t ws_bytes, void* stream)
   }
   SelBatch B;
   B.add(w, 1, k, 0);
-  hipLaunchKernelGGL(k_chain_begin, B.grid(1), dim3(kBlock), 0, (hipStream_t)stream, B.jobs, 0, 0.0);
+  chain_begin(B, SegDirJobs{}, false, (hipStream_t)stream);
   return check_launch("sga_sel_begin");
 }
 
@@ -364,7 +364,8 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   }
   const bool fast = SelBatch::fast_ok(w, n);
   // the select sweep writes the keys above the bracket straight into mask_out
-  run_select_batch(srcs, B, fast, 2, s);
+  J.mask_only = 1;
+  run_select_batch(srcs, B, SegDirJobs{}, fast, 2, s);
   finish_mask_batch(srcs, B, fast, s);
   launch_result(B, s);
   return check_launch("sga_select_topk");

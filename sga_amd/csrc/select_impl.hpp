@@ -8,7 +8,8 @@
 #pragma once
 #include <atomic>
 #include <type_traits>
-#include "common.hpp"
+#include "adam_math.hpp"
+#include "wide_scan.hpp"
 
 namespace sga {
 
@@ -46,9 +47,15 @@ struct SelState {
   uint32_t spec;        // 1: the single-sweep step committed on the sampled bracket (no way back)
   uint32_t negative;    // 1: an fp32 score array held a value below zero (magnitudes were ranked)
   uint32_t redone;      // 1: an out-of-place single-sweep step missed its bracket and was redone
-  uint32_t pad_[5];
+  uint32_t in_sample;   // sample keys inside the bracket (~0: open below, nothing bounds them)
+  uint32_t ticket;      // k_settle: workgroups that are done
+  uint32_t edge_cnt;    // k_settle: entries of the edge list
+  uint32_t edge_inv;    // k_settle: ~(smallest key of the edge list), and ...
+  uint32_t edge_max;    // ... the largest, by atomic maxima (0: none)
+  uint32_t ties_left;   // k_settle_ties has the ties to place
+  uint32_t pad_[31];
 };
-static_assert(sizeof(SelState) == 128, "SelState layout");
+static_assert(sizeof(SelState) == 256, "SelState layout");
 
 struct SelWorkspace {
   SelState* st;        // main state (result, bracket)
@@ -61,7 +68,8 @@ struct SelWorkspace {
   int32_t* seg_dir;    // kSelDirEntries: tensor directory of segment-keyed sources (adam_math.hpp)
   int64_t n_tiles_cap;
   // sampled-bracket path (null / 0 when the workspace has no room for it)
-  uint32_t* sample;    // sample_cap keys
+  uint32_t* sample;    // keys of the coarse sample
+  uint32_t* rel;       // kRelWords
   uint32_t* seg_cnt;   // kSegWaves (+1) counts -> offsets
   uint32_t* seg_idx;   // kSegWaves * seg_cap
   uint32_t* seg_key;
@@ -72,7 +80,7 @@ struct SelWorkspace {
   // segments above
   uint32_t* small_idx;
   uint32_t* small_key;
-  int64_t sample_cap;
+  int64_t sample_cap;  // keys of the sample the bracket comes from
   int64_t seg_cap;     // per-wave candidate capacity
 };
 
@@ -81,8 +89,27 @@ constexpr int kSweepParts = 256;            // partial counters of the sweep's t
 constexpr int64_t kFastMinN = 1 << 20;     // the sampled bracket of the large buckets begins here
 constexpr int kSmallTiles = 8192;          // up to this many chunks a bucket takes small_select.hpp
 constexpr int kSmallSegs = 16;             // list segments there (one per wave of its finishing workgroup)
+constexpr int kSmallSegStride = 64;        // their counters lie 256 bytes apart (see small_geom)
+// Histograms of keys relative to a bracket (large buckets): kRelCopies copies of kRelBins bins that the
+// sweep's workgroups add to by turns (equal keys would otherwise queue on one word, 11 ns each), and
+// one of kWideBins bins with kRelSpread spread counters for the sample.
+constexpr int kRelBins = 1024, kRelCopies = 32, kRelSpread = 16;
+constexpr int kRelSample = kRelBins * kRelCopies;
+constexpr int kRelAbove = kRelSample + kWideBins;
+constexpr int kRelWords = kRelAbove + kRelSpread * 64;
 // Margin of a bracket that has a way back when it misses, in standard deviations of the sample rank.
 constexpr double kBracketSigmas = 5.0;
+
+// Sample: one quad of keys in 512 coordinates, 8 K to 16 K keys (or all).  A thousand more keys cost
+// the picking workgroup 0.25 us and a thousand more list entries the finishing one 0.12: at 4 M
+// coordinates and 1 % (35 K entries from 16 K keys) the two sum to a flat minimum near these sizes.
+constexpr int64_t kSmallSampleMin = 2048, kSmallSampleMax = 4096;
+__host__ __device__ static inline int64_t small_sample_vecs(int64_t n) {
+  int64_t v = n / 512;
+  if (v < kSmallSampleMin) v = kSmallSampleMin;
+  if (v > kSmallSampleMax) v = kSmallSampleMax;
+  return v < n / 4 ? v : n / 4;
+}
 
 static inline int64_t fast_sample_vecs(int64_t n) {
   int64_t v = n / 1024;
@@ -112,6 +139,7 @@ struct ChainJob {
   uint32_t* blk_gt;
   uint32_t* blk_eq;
   uint32_t* sample;
+  uint32_t* rel;
   uint32_t* seg_cnt;
   uint32_t* seg_idx;
   uint32_t* seg_key;
@@ -128,6 +156,7 @@ struct ChainJob {
   int64_t n, n_tiles, n_sv, n_vec;
   uint32_t k, seg_cap, seed, ovf_cap;
   int tie_all, spec;
+  int mask_only;               // no pack: a settled bracket needs no chunk scan
 };
 struct ChainJobs { ChainJob j[kMaxJobs]; };
 template <class Src>
@@ -142,7 +171,7 @@ constexpr int kHistEntries = 2 * kBinsBig + kBinsSmall;      // 8320
 constexpr int kHistStride = kHistEntries + 64;               // per-state stride
 constexpr int kSelDirEntries = 1 << 15;                        // n < 2^31 in blocks of 2^16
 constexpr size_t kSelFixedBytes =
-    512 + (size_t)kHistStride * 2 * 4 + (size_t)kMaxTileBlocks * 4 * 2 + (size_t)kSelDirEntries * 4;
+    3 * sizeof(SelState) + (size_t)kHistStride * 2 * 4 + (size_t)kMaxTileBlocks * 4 * 2 + (size_t)kSelDirEntries * 4;
 
 // List entries of the small path: its kSmallSegs segments hold every coordinate of their
 // workgroups, and the last one may fall a segment's share short of full.
@@ -160,7 +189,7 @@ static inline size_t list_bytes_for_tiles(int64_t nt) {
 static inline size_t fast_bytes_for_tiles(int64_t nt) {
   const int64_t n = nt * kChunk;
   const size_t always = (size_t)(kSegWaves + 64) * 4 + list_bytes_for_tiles(nt) + 256;
-  return n < kFastMinN ? always : always + (size_t)fast_sample_vecs(n) * 16 + (size_t)nt * 128;
+  return n < kFastMinN ? always : always + (size_t)kSmallSampleMax * 16 + (size_t)kRelWords * 4 + (size_t)nt * 128;
 }
 
 static inline size_t sel_ws_bytes(int64_t n) {
@@ -184,8 +213,8 @@ static inline bool sel_ws_carve(void* ws, size_t bytes, int64_t n_tiles_needed,
   if (nt < n_tiles_needed) return false;
   char* p = reinterpret_cast<char*>(ws);
   out->st = reinterpret_cast<SelState*>(p);
-  out->aux = reinterpret_cast<SelState*>(p + 128);
-  p += 512;
+  out->aux = out->st + 1;
+  p += 3 * sizeof(SelState);
   out->hist = reinterpret_cast<uint32_t*>(p);
   p += (size_t)kHistStride * 2 * 4;
   out->blk_gt = reinterpret_cast<uint32_t*>(p);
@@ -199,7 +228,7 @@ static inline bool sel_ws_carve(void* ws, size_t bytes, int64_t n_tiles_needed,
   out->tile_eq = reinterpret_cast<uint32_t*>(p);
   p += (size_t)nt * 4;
   out->n_tiles_cap = nt;
-  out->sample = nullptr;
+  out->sample = out->rel = nullptr;
   out->seg_idx = out->seg_key = out->cand_idx = out->cand_key = nullptr;
   out->pbits = nullptr;
   out->sample_cap = 0;
@@ -221,7 +250,9 @@ static inline bool sel_ws_carve(void* ws, size_t bytes, int64_t n_tiles_needed,
     p += list_bytes_for_tiles(nt);
     out->sample_cap = fast_sample_vecs(n) * 4;
     out->sample = reinterpret_cast<uint32_t*>(p);
-    p += (size_t)out->sample_cap * 4;
+    p += (size_t)kSmallSampleMax * 16;
+    out->rel = reinterpret_cast<uint32_t*>(p);
+    p += (size_t)kRelWords * 4;
     out->pbits = reinterpret_cast<uint32_t*>(p);
   }
   return true;
@@ -501,17 +532,13 @@ __global__ __launch_bounds__(kBlock) void k_level_hist(SrcPack<Src> srcs, ChainJ
   Src src = srcs.s[blockIdx.y];
   level_hist_body<Src, LEVEL, 1, MERGE>(src, J.n, nullptr, J.st, J.hist);
 }
-// over a raw key buffer of the job: the sample (both bracket ends descend together, states
-// aux[0], aux[1]) or the candidates (their count lives on the device; state aux[0])
-template <int LEVEL, bool CAND>
+// over the dense candidate keys of the job (the single-sweep step's records; their count lives on the
+// device, state aux[0])
+template <int LEVEL>
 __global__ __launch_bounds__(kBlock) void k_level_hist_raw(ChainJobs jobs) {
   const ChainJob& J = jobs.j[blockIdx.y];
-  SrcU32 src{CAND ? J.cand_key : J.sample};
-  if (CAND)
-    level_hist_body<SrcU32, LEVEL, 1, true>(src, (int64_t)kSegWaves * J.seg_cap, &J.st->cand_count,
-                                            J.aux, J.hist);
-  else
-    level_hist_body<SrcU32, LEVEL, 2, true>(src, J.n_sv * 4, nullptr, J.aux, J.hist);
+  SrcU32 src{J.cand_key};
+  level_hist_body<SrcU32, LEVEL, 1, true>(src, (int64_t)kSegWaves * J.seg_cap, &J.st->cand_count, J.aux, J.hist);
 }
 
 // Stand-alone scan (used when one level's histogram is built by several
@@ -581,6 +608,7 @@ static __global__ __launch_bounds__(kBlock) void k_tile_sums(ChainJobs jobs) {
   const ChainJob& J = jobs.j[blockIdx.y];
   const int64_t n_tiles = J.n_tiles;
   if ((int64_t)blockIdx.x * kTileScanSpan >= n_tiles) return;     // a job with fewer tiles
+  if (J.mask_only && J.st->bracket_ok && !J.st->ties_left) return;
   const uint32_t* __restrict__ tile_gt = J.tile_gt;
   const uint32_t* __restrict__ tile_eq = J.tile_eq;
   uint32_t* __restrict__ blk_gt = J.blk_gt;
@@ -627,6 +655,7 @@ static __global__ __launch_bounds__(kBlock) void k_tile_apply(ChainJobs jobs) {
   const int64_t n_tiles = J.n_tiles;
   const int n_blocks = (int)cdiv64(n_tiles, kTileScanSpan);
   if ((int)blockIdx.x >= n_blocks) return;                        // a job with fewer tiles
+  if (J.mask_only && J.st->bracket_ok && !J.st->ties_left) return;
   uint32_t* __restrict__ tile_gt = J.tile_gt;
   uint32_t* __restrict__ tile_eq = J.tile_eq;
   const uint32_t* __restrict__ blk_gt = J.blk_gt;
@@ -698,7 +727,9 @@ static __global__ __launch_bounds__(kBlock) void k_tile_apply(ChainJobs jobs) {
     }
     sr += scount[j];
   }
-  if ((int)blockIdx.x == n_blocks - 1 && threadIdx.x == 0) st->n_selected = S0 + blk_tot_s;
+  // (a settlement that placed a mask has stored the number and kept no selected counts)
+  if ((int)blockIdx.x == n_blocks - 1 && threadIdx.x == 0 && !(J.mask_only && st->bracket_ok))
+    st->n_selected = S0 + blk_tot_s;
 }
 
 // Ordered flags for one 256-element slab of a wave's chunk: `sel[e]` says
@@ -830,7 +861,7 @@ struct SelBatch {
     J = ChainJob{};
     J.st = ws.st; J.aux = ws.aux; J.hist = ws.hist;
     J.tile_gt = ws.tile_gt; J.tile_eq = ws.tile_eq; J.blk_gt = ws.blk_gt; J.blk_eq = ws.blk_eq;
-    J.sample = ws.sample; J.seg_cnt = ws.seg_cnt; J.seg_idx = ws.seg_idx; J.seg_key = ws.seg_key;
+    J.sample = ws.sample ? ws.sample : ws.small_idx; J.rel = ws.rel; J.seg_cnt = ws.seg_cnt; J.seg_idx = ws.seg_idx; J.seg_key = ws.seg_key;
     J.cand_idx = ws.cand_idx; J.cand_key = ws.cand_key;
     J.small_idx = ws.small_idx; J.small_key = ws.small_key;
     J.n = n; J.n_tiles = cdiv64(n, kChunk);
@@ -854,19 +885,12 @@ static inline void launch_level_data(const SrcPack<Src>& srcs, const SelBatch& B
   else if (level == 1) hipLaunchKernelGGL((k_level_hist<Src, 1, MERGE>), grid, block, 0, s, srcs, B.jobs);
   else hipLaunchKernelGGL((k_level_hist<Src, 2, MERGE>), grid, block, 0, s, srcs, B.jobs);
 }
-// the same over the jobs' sample keys (CAND false) or candidate keys (CAND true)
-template <bool CAND>
+// the same over the jobs' dense candidate keys
 static inline void launch_level_raw(const SelBatch& B, int level, hipStream_t s, unsigned blocks) {
-  // the fixed cost per workgroup is paid by every job of the batch at once: with 8 jobs, 16
-  // workgroups per job take 86 us for the sample's three levels where 64 take 141
-  if (B.count > 1) {
-    blocks /= (unsigned)B.count;
-    if (blocks < 16) blocks = 16;
-  }
   const dim3 grid = B.grid(blocks), block(kBlock);
-  if (level == 0) hipLaunchKernelGGL((k_level_hist_raw<0, CAND>), grid, block, 0, s, B.jobs);
-  else if (level == 1) hipLaunchKernelGGL((k_level_hist_raw<1, CAND>), grid, block, 0, s, B.jobs);
-  else hipLaunchKernelGGL((k_level_hist_raw<2, CAND>), grid, block, 0, s, B.jobs);
+  if (level == 0) hipLaunchKernelGGL((k_level_hist_raw<0>), grid, block, 0, s, B.jobs);
+  else if (level == 1) hipLaunchKernelGGL((k_level_hist_raw<1>), grid, block, 0, s, B.jobs);
+  else hipLaunchKernelGGL((k_level_hist_raw<2>), grid, block, 0, s, B.jobs);
 }
 static inline void launch_level_scan(int level, const SelBatch& B, hipStream_t s) {
   if (level == 0) hipLaunchKernelGGL((k_level_scan<0>), B.grid(1), dim3(kBlock), 0, s, B.jobs);
@@ -905,57 +929,274 @@ __device__ __forceinline__ uint32_t mix32(uint32_t x) {
   return x;
 }
 
-// One 4-element vector per window, at a hashed offset; the n_sv windows tile
-// ALL n_vec vectors (window j = [j n_vec / n_sv, (j + 1) n_vec / n_sv)): a tail
-// that no window covered would bias the sample whenever the last tensors score
-// differently from the rest.  `seed` moves the offsets (0: the fixed pattern);
-// the select is exact for any of them.
-template <class Src>
-__global__ __launch_bounds__(kBlock) void k_sample(SrcPack<Src> srcs, ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  Src src = srcs.s[blockIdx.y];
-  const int64_t n = J.n, n_sv = J.n_sv, n_vec = J.n_vec;
-  uint32_t* __restrict__ keys = J.sample;
-  const uint32_t seed = J.seed;
-  for (int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x; j < n_sv;
-       j += (int64_t)gridDim.x * kBlock) {
-    const int64_t w0 = j * n_vec / n_sv, w1 = (j + 1) * n_vec / n_sv;
-    const int64_t vec = w0 + (int64_t)(mix32((uint32_t)j + seed * 0x9E3779B9u) % (uint32_t)(w1 - w0));
-    uint32_t key[4];
-    src.template load<false>(vec * 4, n, key);
-    U4 o{key[0], key[1], key[2], key[3]};
-    *reinterpret_cast<U4*>(keys + j * 4) = o;
-  }
+// Quad j of a sample: one 4-element vector per window, at a hashed offset; the n_sv windows tile ALL
+// n_vec vectors (window j = [j n_vec / n_sv, (j + 1) n_vec / n_sv)): a tail that no window covered
+// would bias the sample whenever the last tensors score differently from the rest.  `seed` moves the
+// offsets (0: the fixed pattern); the select is exact for any of them.
+__device__ __forceinline__ int64_t quad_of_window(int64_t j, int64_t n_vec, int64_t n_sv, uint32_t seed) {
+  const int64_t w0 = j * n_vec / n_sv, w1 = (j + 1) * n_vec / n_sv;
+  return w0 + (int64_t)(mix32((uint32_t)j + seed * 0x9E3779B9u) % (uint32_t)(w1 - w0));
 }
 
-// First kernel of a select, one workgroup per job: zeroes both histogram sets and the sweep's
-// counters, resets the main state to rank k and, on the sampled-bracket path (`fast`), places
-// the two ends of the bracket inside the sample at ranks r = k*ns/n -/+ (sigmas * sigma + 8):
-// aux[0] descends to the upper end (smaller rank = larger key), aux[1] to the lower end.
-static __global__ __launch_bounds__(kBlock) void k_chain_begin(ChainJobs jobs, int fast, double sigmas) {
+// Shift that maps the offsets of [lo, hi) onto at most `bins` (a power of two) bins.
+__device__ __forceinline__ int rel_shift(uint32_t lo, uint32_t hi, int bins) {
+  const int w = 32 - __clz((int)(hi - 1u - lo)), b = 31 - __clz(bins);     // hi - lo == 1: w = 0
+  return w > b ? w - b : 0;
+}
+
+// First kernel of a select of the large buckets: clears the histograms and counters, resets the state to
+// rank k, builds the directories of the segment tables (dirs.j[job].dir null: none wanted).
+static __global__ __launch_bounds__(kBlock) void k_chain_begin(ChainJobs jobs, SegDirJobs dirs, int fast) {
   const ChainJob& J = jobs.j[blockIdx.y];
-  for (int i = threadIdx.x; i < kHistStride * 2; i += blockDim.x) J.hist[i] = 0u;
+  const int t0 = blockIdx.x * kBlock + threadIdx.x, step = gridDim.x * kBlock;
+  for (int i = t0; i < kHistStride * 2; i += step) J.hist[i] = 0u;
   if (fast) {
-    for (int i = threadIdx.x; i <= kSegWaves + 1; i += blockDim.x) J.seg_cnt[i] = 0u;   // + overflow count
-    for (int i = threadIdx.x; i < kSweepParts; i += blockDim.x) { J.blk_gt[i] = 0u; J.blk_eq[i] = 0u; }
+    for (int i = t0; i <= kSegWaves + 1; i += step) J.seg_cnt[i] = 0u;   // + overflow count
+    for (int i = t0; i < kSweepParts; i += step) { J.blk_gt[i] = 0u; J.blk_eq[i] = 0u; }
+    for (int i = t0; i < kRelWords; i += step) J.rel[i] = 0u;
     if (J.seg_fail)
-      for (int i = threadIdx.x; i < kSegWaves; i += blockDim.x) J.seg_fail[i] = 0u;
+      for (int i = t0; i < kSegWaves; i += step) J.seg_fail[i] = 0u;
   }
-  if (threadIdx.x != 0) return;
+  const auto& D = dirs.j[blockIdx.y];
+  if (D.dir) {
+    const int nb = (int)((D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog);
+    for (int b = t0; b < nb; b += step) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
+  }
+  if (t0 != 0) return;
   SelState z = {};
   z.k = J.k;
   *J.st = z;
-  if (!fast) return;
-  const double n = (double)J.n, ns = (double)(J.n_sv * 4);
-  const double frac = (double)J.k / n;
-  const double r = frac * ns;
+}
+
+constexpr int kSmallPick = (int)(kSmallSampleMax / kWide);   // quads per thread of the picking workgroup
+
+// A key source that looks tensors up: without the directory (it is being built while the sample is
+// taken) the lookup bisects the table.
+template <class S>
+__device__ __forceinline__ auto drop_dir(S& s, int) -> decltype(s.sc.dir, void()) { s.sc.dir = nullptr; }
+template <class S>
+__device__ __forceinline__ void drop_dir(S&, long) {}
+
+// Sample keys (one quad per window at a hashed offset; the windows tile all quads, see k_sample),
+// the list counters, and, in a job's last workgroup, the directory of its segment table
+// (dirs.j[job].dir null: none wanted).  Gathering from one workgroup would be bound by one CU's
+// translation misses (4096 quads of two arrays: 25 us; 64 workgroups: 4).
+template <class Src>
+__global__ __launch_bounds__(kBlock) void k_sample_coarse(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
+                                                          int of_fine) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x < kSmallSegs) J.seg_cnt[threadIdx.x * kSmallSegStride] = 0u;
+    const auto& D = dirs.j[blockIdx.y];
+    if (D.dir) {
+      const int64_t nb = (D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
+      for (int64_t b = threadIdx.x; b < nb; b += kBlock) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
+    }
+    return;
+  }
+  Src src = srcs.s[blockIdx.y];
+  drop_dir(src, 0);
+  const int64_t n_sv = small_sample_vecs(J.n);
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (j >= n_sv) return;
+  // of_fine: a subset of the windows of the large buckets' fine sample, which it then agrees with
+  const int64_t all = of_fine ? J.n_sv : n_sv;
+  uint32_t key[4];
+  src.template load<false>(quad_of_window(j * all / n_sv, J.n / 4, all, J.seed) * 4, J.n, key);
+  reinterpret_cast<U4*>(J.sample)[j] = U4{key[0], key[1], key[2], key[3]};
+}
+
+// Ranks in a sample of ns keys (1-based from the top) between which the k-th of n lies.
+struct RankEnds { double hi, lo; };
+__device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns, double sigmas) {
+  const double frac = k / n, r = frac * ns;
   const double d = sigmas * sqrt(r * (1.0 - frac) + 1.0) + 8.0;
-  SelState hi = {}, lo = {};
-  const double rh = floor(r - d), rl = ceil(r + d);
-  if (rh < 1.0) hi.skip = 1; else hi.k = (uint32_t)rh;
-  if (rl > ns) lo.skip = 1; else lo.k = (uint32_t)rl;
-  J.aux[0] = hi;
-  J.aux[1] = lo;
+  return RankEnds{floor(r - d), ceil(r + d)};
+}
+
+// One workgroup per job: state reset, the two ends of the bracket from the sample.  The top 12 bits of
+// all keys go into one LDS histogram, the next 12 of the keys in the two bins the ends fall into into
+// one each; what is left in a bin then is ranked by counting (or split by the last 7 bits, on plateaus).
+//
+// The small buckets bracket the k-th key of the data this way (sigmas: kBracketSigmas).  The large ones
+// (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with four
+// sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.
+template <bool COARSE>
+__global__ __launch_bounds__(kWide) void k_pick_coarse(ChainJobs jobs, double sigmas) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
+  __shared__ __align__(16) uint32_t s_list[2][kWideList];
+  __shared__ uint32_t s_cnt[2], s_out[2][3];
+  __shared__ WideScratch s_scan;
+  const int64_t n = J.n;
+  const int64_t n_sv = small_sample_vecs(n);
+  U4 key[kSmallPick];
+#pragma unroll
+  for (int u = 0; u < kSmallPick; ++u) {
+    const int64_t j = (int64_t)u * kWide + threadIdx.x;
+    if (u * (int64_t)kWide < n_sv && j < n_sv) key[u] = reinterpret_cast<const U4*>(J.sample)[j];
+  }
+  const U4 zero{0u, 0u, 0u, 0u};
+  reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
+  if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
+  __syncthreads();
+  const uint32_t ns = (uint32_t)(n_sv * 4);
+  double rh, rl;
+  if (COARSE) {
+    const double nf = (double)(J.n_sv * 4), to = (double)ns / nf;
+    const RankEnds f = bracket_ranks((double)J.k, (double)n, nf, sigmas);
+    const double ah = f.hi * to, al = f.lo * to;
+    rh = floor(ah - (4.0 * sqrt(fmax(ah, 0.0) + 1.0) + 4.0));
+    rl = ceil(al + (4.0 * sqrt(al + 1.0) + 4.0));
+  } else {
+    const RankEnds f = bracket_ranks((double)J.k, (double)n, (double)ns, sigmas);
+    rh = f.hi;
+    rl = f.lo;
+  }
+  const bool open_hi = rh < 1.0 || ns == 0, open_lo = rl > (double)ns || ns == 0;
+  const uint32_t rank[2] = {open_hi ? 1u : (uint32_t)rh, open_lo ? 1u : (uint32_t)rl};
+  uint32_t t_hi = 0x80000000u, t_lo = 0u;
+  if (ns) {
+    auto each = [&](auto&& f) {
+#pragma unroll
+      for (int u = 0; u < kSmallPick; ++u) {
+        if (u * (int64_t)kWide >= n_sv) break;                  // uniform
+        const bool live = (int64_t)u * kWide + threadIdx.x < n_sv;
+        f(key[u].x, live); f(key[u].y, live); f(key[u].z, live); f(key[u].w, live);
+      }
+    };
+    each([&](uint32_t kk, bool live) { if (live) atomicAdd(&s_h[0][kk >> kL0Shift], 1u); });
+    __syncthreads();
+    RankHit hit[2];
+    wide_find_rank<2>(s_h[0], rank, s_scan, 0, hit);
+    uint32_t bin[2] = {hit[0].bin, hit[1].bin};
+    uint32_t rk[2] = {rank[0] - hit[0].above, rank[1] - hit[1].above};
+    uint32_t cnt[2] = {hit[0].count, hit[1].count};
+    int w = kL0Shift, turn = 1;                        // bits of a key below the bins found so far
+    while (w > 0 && (cnt[0] > (uint32_t)kWideList || cnt[1] > (uint32_t)kWideList)) {
+      const int sh = w > 12 ? w - 12 : 0, bits = w - sh;
+      reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
+      reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
+      __syncthreads();
+      each([&](uint32_t kk, bool live) {
+        const uint32_t top = kk >> w;
+        if (!live || (top != bin[0] && top != bin[1])) return;
+        const uint32_t low = (kk >> sh) & ((1u << bits) - 1u);
+        if (top == bin[0]) atomicAdd(&s_h[0][low], 1u);
+        if (top == bin[1]) atomicAdd(&s_h[1][low], 1u);
+      });
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint32_t want[1] = {rk[q]};
+        RankHit h[1];
+        wide_find_rank<1>(s_h[q], want, s_scan, turn, h);
+        turn ^= 1;
+        bin[q] = (bin[q] << bits) | h[0].bin;
+        rk[q] -= h[0].above;
+        cnt[q] = h[0].count;
+      }
+      w = sh;
+    }
+    if (w > 0) {
+      each([&](uint32_t kk, bool live) {
+        const uint32_t top = kk >> w;
+        if (!live || (top != bin[0] && top != bin[1])) return;
+        if (top == bin[0]) s_list[0][atomicAdd(&s_cnt[0], 1u)] = kk;
+        if (top == bin[1]) s_list[1][atomicAdd(&s_cnt[1], 1u)] = kk;
+      });
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < 2; ++q) wide_list_rank(s_list[q], cnt[q], rk[q], s_out[q]);
+      __syncthreads();
+    }
+    // keys equal to the upper sample key stay inside the bracket
+    if (!open_hi) t_hi = (w > 0 ? s_out[0][0] : bin[0]) + 1u;
+    if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
+  }
+  if (threadIdx.x == 0) {
+    SelState z = {};
+    z.k = J.k;
+    z.t_hi = t_hi;
+    z.t_lo = t_lo;
+    *J.st = z;
+  }
+}
+
+// The fine sample of a large bucket: only how its keys fall relative to the coarse bracket is kept --
+// counts above it, and a histogram of the few inside.
+template <class Src>
+__global__ __launch_bounds__(kBlock) void k_sample_fine(SrcPack<Src> srcs, ChainJobs jobs) {
+  __shared__ uint32_t s_w[kChunksPerBlock];
+  const ChainJob& J = jobs.j[blockIdx.y];
+  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if ((int64_t)blockIdx.x * kBlock >= J.n_sv) return;                 // a smaller job of the batch
+  Src src = srcs.s[blockIdx.y];
+  const uint32_t c_lo = J.st->t_lo, c_hi = J.st->t_hi;
+  const int sh = rel_shift(c_lo, c_hi, kWideBins);
+  uint32_t* __restrict__ bins = J.rel + kRelSample;
+  uint32_t key[4] = {0u, 0u, 0u, 0u};
+  const bool live = j < J.n_sv;
+  if (live) src.template load<false>(quad_of_window(j, J.n_vec, J.n_sv, J.seed) * 4, J.n, key);
+  uint32_t above = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    above += (uint32_t)__popcll(ballot64(live && key[e] >= c_hi));
+    const bool in = live && key[e] >= c_lo && key[e] < c_hi;
+    const uint32_t bin = (key[e] - c_lo) >> sh;
+    const uint64_t act = ballot64(in);
+    if (act == 0) continue;
+    // many lanes on one bin (a plateau) add once
+    const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane((int)bin, __ffsll((unsigned long long)act) - 1);
+    const uint64_t same = ballot64(in && bin == lead);
+    const bool fold = __popcll(same) >= 8;
+    if (fold && lane_id() == 0) atomicAdd(&bins[lead], (uint32_t)__popcll(same));
+    if (in && !(fold && bin == lead)) atomicAdd(&bins[bin], 1u);
+  }
+  if (lane_id() == 0) s_w[wave_id()] = above;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const uint32_t all = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+    if (all) atomicAdd(&J.rel[kRelAbove + (blockIdx.x % kRelSpread) * 64], all);
+  }
+}
+
+// The bracket from the fine sample, at the edges of its histogram's bins (rounded outwards: a few sample
+// keys wide).  An end the coarse bracket missed is left open.
+static __global__ __launch_bounds__(kWide) void k_pick_fine(ChainJobs jobs, double sigmas) {
+  __shared__ WideScratch s_scan;
+  const ChainJob& J = jobs.j[blockIdx.y];
+  const uint32_t c_lo = J.st->t_lo, c_hi = J.st->t_hi;
+  const int sh = rel_shift(c_lo, c_hi, kWideBins);
+  const uint32_t* bins = J.rel + kRelSample;
+  uint32_t above = 0;
+  for (int i = 0; i < kRelSpread; ++i) above += J.rel[kRelAbove + i * 64];
+  const U4 q = reinterpret_cast<const U4*>(bins)[threadIdx.x];
+  uint32_t inside;
+  wide_prefix(q.x + q.y + q.z + q.w, s_scan, 1, inside);
+  const double ns = (double)(J.n_sv * 4);
+  const RankEnds f = bracket_ranks((double)J.k, (double)J.n, ns, sigmas);
+  const bool in_hi = f.hi >= 1.0 && f.hi > (double)above && f.hi <= (double)above + (double)inside;
+  const bool in_lo = f.lo <= ns && f.lo > (double)above && f.lo <= (double)above + (double)inside;
+  const uint32_t rank[2] = {in_hi ? (uint32_t)f.hi - above : 1u, in_lo ? (uint32_t)f.lo - above : 1u};
+  RankHit hit[2] = {};
+  if (inside) wide_find_rank<2>(bins, rank, s_scan, 0, hit);
+  if (threadIdx.x != 0) return;
+  uint32_t t_hi = 0x80000000u, t_lo = 0u, in_sample = ~0u;
+  if (in_hi) {
+    t_hi = c_lo + ((hit[0].bin + 1u) << sh);
+    if (t_hi > c_hi) t_hi = c_hi;
+  }
+  if (in_lo) {
+    t_lo = c_lo + (hit[1].bin << sh);
+    in_sample = above + hit[1].above + hit[1].count - (in_hi ? above + hit[0].above : 0u);
+  }
+  SelState z = {};
+  z.k = J.k;
+  z.t_hi = t_hi;
+  z.t_lo = t_lo;
+  z.in_sample = in_sample;
+  *J.st = z;
 }
 
 // The one sweep over the data: a one-shot grid, one 1024-element chunk per
@@ -1093,62 +1334,394 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
   }
 }
 
+// A wave's candidates beyond its LDS buffer: a second look at the chunk, slab by slab.
+template <class Src, class F>
+__device__ __forceinline__ void recollect(Src& src, int64_t n, int64_t c, uint32_t T_LO, uint32_t T_HI, F&& put) {
+  src.chunk_hyper(c);
+  uint32_t run = 0;
+  for (int it = 0; it < kChunkIters; ++it) {
+    const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
+    uint32_t key[4] = {0u, 0u, 0u, 0u};
+    if (i < n) src.template load<false>(i, n, key);
+    Ballot4 in;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) in.m[e] = ballot64(i + e < n && key[e] >= T_LO && key[e] < T_HI);
+    ballot_append(in, run, [&](uint32_t pos, int e) { put(pos, (uint32_t)(i + e), key[e]); });
+  }
+}
+
+// A bracket of a single key (a plateau of equal keys holds the k-th one) collects nothing: its members
+// are ties, counted per chunk (tile_eq) and in bin 0 of the relative histogram.
 template <class Src, int PM>
 __global__ __launch_bounds__(kBlock) void k_bracket_sweep(
-    Src src, int64_t n, SelState* __restrict__ st, const SelState* __restrict__ aux,
+    Src src, int64_t n, SelState* __restrict__ st, uint32_t* __restrict__ rel,
     uint32_t* __restrict__ tile_gt, uint32_t* __restrict__ tile_eq, uint32_t* __restrict__ seg_idx,
     uint32_t* __restrict__ seg_key, uint32_t* __restrict__ seg_cnt, uint32_t seg_cap,
     uint32_t* __restrict__ pbits, uint32_t* __restrict__ hi_part, uint32_t* __restrict__ nf_part,
     uint8_t* __restrict__ mask_bytes = nullptr, bool mvec = false) {
   const bool m16 = PM == 2 && (reinterpret_cast<uintptr_t>(mask_bytes) & 15) == 0;
-  __shared__ uint32_t s_hi[kChunksPerBlock], s_nf[kChunksPerBlock];
+  __shared__ uint32_t s_hi[kChunksPerBlock], s_nf[kChunksPerBlock], s_eq[kChunksPerBlock];
   __shared__ SweepLds s_lds[kChunksPerBlock];
-  // keys equal to the upper sample key stay candidates; a skipped end means
-  // the bracket is open on that side
-  const uint32_t T_HI = aux[0].skip ? 0x80000000u : aux[0].thresh_bits + 1u;
-  const uint32_t T_LO = aux[1].skip ? 0u : aux[1].thresh_bits;
-  if (blockIdx.x == 0 && threadIdx.x == 0) { st->t_lo = T_LO; st->t_hi = T_HI; }
+  const uint32_t T_HI = st->t_hi, T_LO = st->t_lo;
+  const bool single = T_HI - T_LO == 1u;
   const int64_t n_chunks = cdiv64(n, kChunk);
   const int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id();
-  uint32_t chi = 0, tot_nf = 0;
+  uint32_t chi = 0, tot_nf = 0, ties = 0;
+  uint32_t* __restrict__ const bins = rel + (blockIdx.x % kRelCopies) * kRelBins;
   if (c < n_chunks) {
     uint32_t mycnt = 0;
     SweepLds& lds = s_lds[wave_id()];
-    uint32_t* const my_idx = lds.idx;
-    uint32_t* const my_key = lds.key;
     const typename Src::Chunk ck = src.chunk_begin(c);
     if (src.vec && (c + 1) * kChunk <= n)
       bracket_chunk<Src, true, PM>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec, m16);
     else
       bracket_chunk<Src, false, PM>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec);
-    if (lane_id() == 0) { tile_gt[c] = chi; tile_eq[c] = 0u; }     // chi / tot_nf are wave totals
+    if (single) { ties = mycnt; mycnt = 0; }
+    if (lane_id() == 0) { tile_gt[c] = chi; tile_eq[c] = ties; }   // chi / tot_nf are wave totals
     if (mycnt) {                                        // wave-uniform
       const uint32_t seg = (uint32_t)c & (uint32_t)(kSegWaves - 1);
       uint32_t base = 0;
-      if (lane_id() == 0) base = atomicAdd(&seg_cnt[seg], mycnt);   // a segment over its capacity is seen by the check
+      if (lane_id() == 0) base = atomicAdd(&seg_cnt[seg], mycnt);
       base = __shfl(base, 0, kWave);
-      if (mycnt > (uint32_t)kWaveCandCap) {
+      if (base + mycnt > seg_cap) {
         if (lane_id() == 0) atomicOr(&st->overflow, 1u);
       } else {
-        __builtin_amdgcn_wave_barrier();                // the wave's LDS stores above are read below
-        uint32_t* const g_idx = seg_idx + (int64_t)seg * seg_cap;
-        uint32_t* const g_key = seg_key + (int64_t)seg * seg_cap;
-        for (uint32_t j = lane_id(); j < mycnt; j += kWave)
-          if (base + j < seg_cap) { g_idx[base + j] = my_idx[j]; g_key[base + j] = my_key[j]; }
+        const int sh = rel_shift(T_LO, T_HI, kRelBins);
+        uint32_t* const g_idx = seg_idx + (int64_t)seg * seg_cap + base;
+        uint32_t* const g_key = seg_key + (int64_t)seg * seg_cap + base;
+        if (mycnt <= (uint32_t)kWaveCandCap) {
+          __builtin_amdgcn_wave_barrier();              // the wave's LDS stores above are read below
+          for (uint32_t j = lane_id(); j < mycnt; j += kWave) {
+            const uint32_t key = lds.key[j];
+            g_idx[j] = lds.idx[j];
+            g_key[j] = key;
+            atomicAdd(&bins[(key - T_LO) >> sh], 1u);
+          }
+        } else {
+          recollect(src, n, c, T_LO, T_HI, [&](uint32_t pos, uint32_t idx, uint32_t key) {
+            g_idx[pos] = idx;
+            g_key[pos] = key;
+            atomicAdd(&bins[(key - T_LO) >> sh], 1u);
+          });
+        }
       }
     }
   }
   const bool neg = ballot64(src_negative(src) != 0u) != 0ull;
-  if (lane_id() == 0) { s_hi[wave_id()] = chi; s_nf[wave_id()] = tot_nf | (neg ? 0x80000000u : 0u); }
+  if (lane_id() == 0) {
+    s_hi[wave_id()] = chi;
+    s_eq[wave_id()] = ties;
+    s_nf[wave_id()] = tot_nf | (neg ? 0x80000000u : 0u);
+  }
   __syncthreads();
   if (threadIdx.x == 0) {
     const uint32_t h = s_hi[0] + s_hi[1] + s_hi[2] + s_hi[3];
+    const uint32_t t = s_eq[0] + s_eq[1] + s_eq[2] + s_eq[3];
     const uint32_t any_neg = (s_nf[0] | s_nf[1] | s_nf[2] | s_nf[3]) & 0x80000000u;
     const uint32_t f = (s_nf[0] + s_nf[1] + s_nf[2] + s_nf[3]) & 0x7FFFFFFFu;
     if (h) atomicAdd(&hi_part[blockIdx.x & (kSweepParts - 1)], h);
+    if (t) atomicAdd(&bins[0], t);
     if (f) atomicAdd(&nf_part[blockIdx.x & (kSweepParts - 1)], f);
     if (any_neg) raise_negative(st);
   }
+}
+
+// Settlement of a bracket, one launch for all that lies between the sweep and the chunk scan: exact
+// threshold, per-chunk corrections, and the candidates' places in the mask or the planes.
+//   1. Every workgroup sums the copies of the sweep's relative histogram and finds the bin where the
+//      count from the top reaches k -- each for itself, so nothing has to wait for anything.
+//   2. It then walks its share of the candidate segments: keys above the bin are selected, the bin's
+//      own go to the edge list (about C / kRelBins of C candidates) and are counted as ties for now.
+//   3. The last workgroup to finish ranks the edge list (threshold, ties, which of them are granted:
+//      lowest index first) and corrects the counts.  An edge list of one key value needs no ranking
+//      whatever its length (gradients on the bf16 grid: a hundred thousand equal keys); the ties of
+//      one too long for LDS are placed by k_settle_ties, behind the chunk scan.
+// What step 3 reads of the others' is written by device-scope atomics and atomic stores, each wave
+// waits for its own (vmcnt) before the workgroup takes its ticket, and the last one reads with atomic
+// loads: no cache-wide fence, which costs 65 ns a workgroup here.
+// The chain of one-level launches this replaces (check, compaction, three histogram levels, chunk
+// counts, mask) took 75 to 150 us.  Now 16 us at 40 M coordinates (48 K candidates), 53 us at 1e9
+// (1.25 M candidates: their random mask bytes), 20 us over the bf16 ties of a replayed step.
+constexpr int kEdgeCap = 4096;              // edge entries the last workgroup holds in LDS
+struct EdgeList {                           // LDS, or global memory when there are more
+  const uint32_t* key;
+  const uint32_t* idx;
+  uint32_t cnt;
+  bool lds;
+  __device__ __forceinline__ uint32_t key_at(uint32_t j) const {
+    return lds ? key[j] : __hip_atomic_load(key + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __device__ __forceinline__ uint32_t idx_at(uint32_t j) const {
+    return lds ? idx[j] : __hip_atomic_load(idx + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+};
+// `rank`-th (1-based) largest of the w-bit offsets value(j) - lo, by 12-bit levels.  `lo`, `rank`, `eq`
+// end as the value, its rank among the equal ones, and their number.
+template <class V>
+__device__ __forceinline__ void edge_descend(uint32_t cnt, V&& value, uint32_t& lo, int w, uint32_t& rank,
+                                             uint32_t& eq, uint32_t* s_hist, WideScratch& s_scan) {
+  int turn = 0;
+  while (w > 0) {
+    const int sh = w > 12 ? w - 12 : 0;
+    reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
+    __syncthreads();
+    constexpr int U = 4;                                 // global lists: loads in flight per thread
+    for (uint32_t j0 = 0; j0 < cnt; j0 += U * kWide) {
+      uint32_t v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t j = j0 + u * kWide + threadIdx.x;
+        v[u] = j < cnt ? value(j) : ~0u;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t off = v[u] - lo;
+        wide_hist_add(s_hist, off >> sh, off >> w == 0u);
+      }
+    }
+    __syncthreads();
+    const uint32_t want[1] = {rank};
+    RankHit h[1];
+    wide_find_rank<1>(s_hist, want, s_scan, turn, h);
+    turn ^= 1;
+    lo += h[0].bin << sh;
+    rank -= h[0].above;
+    eq = h[0].count;
+    w = sh;
+  }
+  __syncthreads();
+}
+// The place of a settled coordinate in the job's mask bytes or bit planes (neither: the writing pass
+// forms the keys again).
+__device__ __forceinline__ void place_selected(const ChainJob& J, uint32_t idx) {
+  if (J.mask) {
+    J.mask[idx] = 1;
+  } else if (J.planes) {
+    const uint32_t lane = (idx >> 2) & 63u, e = idx & 3u;
+    atomicOr(&J.planes[(idx >> 8) * 8 + 2 * e + (lane >> 5)], 1u << (lane & 31));
+  }
+}
+// The calling wave's share of the candidate segments: f(valid, key, idx, position), by whole waves.  Eight
+// segments at a time: their counts in one load, their entries as one run, so that short segments still
+// fill the wave and several loads are in flight.
+template <class F>
+__device__ __forceinline__ void walk_segments(const ChainJob& J, int wave, int waves, F&& f) {
+  constexpr int kRun = 8, U = 4;
+  for (int w0 = wave * kRun; w0 < kSegWaves; w0 += waves * kRun) {
+    const uint32_t cl = lane_id() < kRun ? J.seg_cnt[w0 + lane_id()] : 0u;
+    uint32_t off[kRun + 1];
+    off[0] = 0;
+#pragma unroll
+    for (int r = 0; r < kRun; ++r) off[r + 1] = off[r] + (uint32_t)__builtin_amdgcn_readlane((int)cl, r);
+    for (uint32_t q0 = 0; q0 < off[kRun]; q0 += U * kWave) {
+      uint32_t key[U], idx[U], pos[U];
+      bool valid[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t q = q0 + u * kWave + lane_id();
+        valid[u] = q < off[kRun];
+        uint32_t at = q;                                 // entry q is entry q - off[r] of segment w0 + r
+#pragma unroll
+        for (int r = 0; r < kRun - 1; ++r) at = q >= off[r + 1] ? q - off[r + 1] + (uint32_t)(r + 1) * J.seg_cap : at;
+        pos[u] = (uint32_t)w0 * J.seg_cap + at;          // kSegWaves * seg_cap <= n / 32 rounded up: 27 bits
+        key[u] = valid[u] ? J.seg_key[pos[u]] : 0u;
+        idx[u] = valid[u] ? J.seg_idx[pos[u]] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (q0 + u * kWave >= off[kRun]) break;          // wave-uniform
+        f(valid[u], key[u], idx[u], pos[u]);
+      }
+    }
+  }
+}
+// Adds the wave's flagged entries to their chunks' counters.  A chunk's candidates follow one another
+// in the list, so equal neighbours are counted together: one atomic per chunk and 64 entries.
+__device__ __forceinline__ void count_by_chunk(uint32_t* __restrict__ tiles, bool flag, uint32_t idx) {
+  const uint64_t on = ballot64(flag);
+  if (on == 0) return;
+  const uint32_t c = idx >> 10;
+  const uint32_t left = __shfl_up(c, 1, kWave);
+  const uint64_t heads = ballot64(lane_id() == 0 || c != left);       // first lane of every run of one chunk
+  if ((heads >> lane_id()) & 1ull) {
+    const uint64_t behind = lane_id() == 63 ? 0ull : heads >> (lane_id() + 1) << (lane_id() + 1);
+    const uint64_t run = (behind ? (1ull << (__ffsll((unsigned long long)behind) - 1)) - 1ull : ~0ull) &
+                         (~0ull << lane_id());
+    const uint32_t cnt = (uint32_t)__popcll(on & run);
+    if (cnt) atomicAdd(&tiles[c], cnt);
+  }
+}
+static __global__ __launch_bounds__(kWide) void k_settle(ChainJobs jobs) {
+  __shared__ __align__(16) uint32_t s_hist[kWideBins];
+  __shared__ uint32_t s_key[kEdgeCap], s_idx[kEdgeCap];
+  __shared__ uint32_t s_n, s_inv, s_max, s_base, s_last;
+  __shared__ WideScratch s_scan;
+  const ChainJob& J = jobs.j[blockIdx.y];
+  SelState* __restrict__ st = J.st;
+  const uint32_t T_LO = st->t_lo, T_HI = st->t_hi, k = J.k;
+  const bool single = T_HI - T_LO == 1u;
+  const int sh = rel_shift(T_LO, T_HI, kRelBins);
+  // ---- 1
+  uint32_t mine = 0;
+#pragma unroll
+  for (int r = 0; r < kRelCopies; ++r) mine += J.rel[r * kRelBins + threadIdx.x];
+  static_assert(kRelBins == kWide && kSweepParts <= kWide, "a bin and a partial counter per thread");
+  const uint32_t part = threadIdx.x < kSweepParts ? J.blk_gt[threadIdx.x] : 0u;
+  if (threadIdx.x == 0) s_n = s_inv = s_max = 0u;
+  uint32_t n_hi, n_in;
+  wide_prefix(part, s_scan, 0, n_hi);
+  const uint32_t before = wide_prefix(mine, s_scan, 1, n_in);
+  const bool ok = !st->overflow && n_hi < k && k <= n_hi + n_in;
+  const uint32_t above_me = n_in - before - mine, rank0 = k - n_hi;
+  if (ok && above_me < rank0 && rank0 <= above_me + mine) {
+    s_scan.hit[0][0][0] = threadIdx.x;
+    s_scan.hit[0][0][1] = above_me;
+    s_scan.hit[0][0][2] = mine;
+  }
+  __syncthreads();
+  const bool first = blockIdx.x == 0;
+  if (first) {
+    uint32_t n_nf;
+    wide_prefix(threadIdx.x < kSweepParts ? J.blk_eq[threadIdx.x] : 0u, s_scan, 0, n_nf);
+    if (threadIdx.x == 0) {
+      st->n_hi = n_hi;
+      st->cand_count = n_in;
+      st->bracket_ok = ok && !single ? 1u : 0u;     // a plateau's selection is written by an ordered pass
+      st->skip = ok ? 1u : 0u;                      // the radix passes run only when the bracket failed
+      st->path = ok && !single ? 1u : 0u;
+      st->nonfinite = ok ? n_nf : 0u;               // recounted by the radix passes otherwise
+      if (ok && single) {
+        st->thresh_bits = T_LO;
+        st->need = rank0;
+        st->n_eq = n_in;
+        st->n_gt = n_hi;
+      }
+    }
+  }
+  if (!ok || single) return;
+  const uint32_t bin = s_scan.hit[0][0][0], above = s_scan.hit[0][0][1];
+  // ---- 2
+  const uint32_t e_lo = T_LO + (bin << sh);
+  uint32_t e_inv = 0, e_max = 0;
+  walk_segments(J, (int)blockIdx.x * kWideWaves + wave_id(), (int)gridDim.x * kWideWaves,
+                [&](bool valid, uint32_t key, uint32_t idx, uint32_t) {
+    const uint32_t off = key - e_lo;
+    const bool sel = valid && (int32_t)off >= 0 && off >> sh != 0u;
+    const bool edge = valid && (int32_t)off >= 0 && off >> sh == 0u;
+    if (!J.mask_only) count_by_chunk(J.tile_gt, sel, idx);
+    if (sel) place_selected(J, idx);
+    if (ballot64(edge) == 0) return;
+    count_by_chunk(J.tile_eq, edge, idx);
+    if (!edge) return;
+    e_inv = e_inv > ~key ? e_inv : ~key;
+    e_max = e_max > key ? e_max : key;
+    const uint32_t at = atomicAdd(&s_n, 1u);
+    if (at < (uint32_t)kEdgeCap) {
+      s_key[at] = key;
+      s_idx[at] = idx;
+    } else {                                            // more than a workgroup's share of any but a plateau
+      const uint32_t g = atomicAdd(&st->edge_cnt, 1u);
+      __hip_atomic_store(&J.cand_key[g], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(&J.cand_idx[g], idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  });
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) {
+    const uint32_t a = __shfl_xor(e_inv, o, kWave), b = __shfl_xor(e_max, o, kWave);
+    e_inv = e_inv > a ? e_inv : a;
+    e_max = e_max > b ? e_max : b;
+  }
+  if (lane_id() == 0 && e_inv) { atomicMax(&s_inv, e_inv); atomicMax(&s_max, e_max); }
+  __syncthreads();
+  const uint32_t held = s_n < (uint32_t)kEdgeCap ? s_n : (uint32_t)kEdgeCap;
+  if (threadIdx.x == 0 && held) {
+    s_base = atomicAdd(&st->edge_cnt, held);
+    atomicMax(&st->edge_inv, s_inv);
+    atomicMax(&st->edge_max, s_max);
+  }
+  __syncthreads();
+  for (uint32_t j = threadIdx.x; j < held; j += kWide) {
+    __hip_atomic_store(&J.cand_key[s_base + j], s_key[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&J.cand_idx[s_base + j], s_idx[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  // ---- 3
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // this wave's atomics and stores have landed
+  __syncthreads();
+  if (threadIdx.x == 0)
+    s_last = __hip_atomic_fetch_add(&st->ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+  __syncthreads();
+  if (!s_last) return;
+  const uint32_t cnt = __hip_atomic_load(&st->edge_cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t inv = __hip_atomic_load(&st->edge_inv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const uint32_t top = __hip_atomic_load(&st->edge_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const bool one_key = top == ~inv, short_list = cnt <= (uint32_t)kEdgeCap;
+  EdgeList L{J.cand_key, J.cand_idx, cnt, false};
+  if (short_list) {
+    for (uint32_t j = threadIdx.x; j < cnt; j += kWide) { s_key[j] = L.key_at(j); s_idx[j] = L.idx_at(j); }
+    L = EdgeList{s_key, s_idx, cnt, true};
+    __syncthreads();
+  }
+  uint32_t T = one_key ? top : e_lo, need = rank0 - above, n_eq = cnt;
+  if (!one_key)
+    edge_descend(cnt, [&](uint32_t j) { return L.key_at(j); }, T, sh, need, n_eq, s_hist, s_scan);
+  const bool places = J.mask || J.planes;
+  // of the ties the `need` lowest indices are granted: the last granted one is the need-th from below
+  const bool all = J.tie_all || need == n_eq;
+  uint32_t last_idx = 0xFFFFFFFFu;
+  if (short_list && places && !all) {
+    uint32_t lo = 0, r = n_eq - need + 1, eq = 0;         // rank from the top among the ties
+    edge_descend(cnt, [&](uint32_t j) { return L.key_at(j) == T ? L.idx_at(j) : ~0u; }, lo, 31, r, eq, s_hist, s_scan);
+    last_idx = lo;
+  }
+  if (!one_key || (short_list && places)) {
+    for (uint32_t j = threadIdx.x; j < cnt; j += kWide) {
+      const uint32_t key = L.key_at(j), idx = L.idx_at(j);
+      if (key != T) {
+        atomicSub(&J.tile_eq[idx >> 10], 1u);
+        if (key < T) continue;
+        atomicAdd(&J.tile_gt[idx >> 10], 1u);
+      }
+      if (key > T || (short_list && idx <= last_idx)) place_selected(J, idx);
+    }
+  }
+  if (threadIdx.x == 0) {
+    st->thresh_bits = T;
+    st->need = need;
+    st->n_eq = n_eq;
+    st->n_gt = k - need;
+    st->n_selected = J.tie_all ? k - need + n_eq : k;     // the chunk scan says the same where it runs
+    st->ties_left = places && !short_list ? 1u : 0u;
+  }
+}
+
+// Ties of an edge list that did not fit the last workgroup's LDS, in index order: the chunk scan has
+// left the ties before every chunk in tile_eq, so only the one chunk where the quota runs out has to
+// rank its ties (a chunk's candidates are contiguous and index-ordered in its segment).
+static __global__ __launch_bounds__(kBlock) void k_settle_ties(ChainJobs jobs) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  const SelState* __restrict__ st = J.st;
+  if (!st->ties_left) return;
+  const uint32_t T = st->thresh_bits, n_eq = st->n_eq;
+  const uint32_t need = J.tie_all ? 0xFFFFFFFFu : st->need;
+  walk_segments(J, (int)blockIdx.x * kChunksPerBlock + wave_id(), (int)gridDim.x * kChunksPerBlock,
+                [&](bool valid, uint32_t key, uint32_t idx, uint32_t pos) {
+    if (!valid || key != T) return;
+    bool on = true;
+    if (need < n_eq) {
+      const uint32_t c = idx >> 10;
+      const uint32_t before = J.tile_eq[c];
+      const uint32_t upto = (int64_t)c + 1 < J.n_tiles ? J.tile_eq[c + 1] : n_eq;
+      if (before >= need) {
+        on = false;
+      } else if (upto > need) {                           // the quota ends inside this chunk
+        uint32_t rank = before;
+        const uint32_t begin = pos / J.seg_cap * J.seg_cap;
+        for (uint32_t q = pos; q > begin && (J.seg_idx[q - 1] >> 10) == c; --q) rank += J.seg_key[q - 1] == T;
+        on = rank < need;
+      }
+    }
+    if (on) place_selected(J, idx);
+  });
 }
 
 // Single workgroup: segment counts -> offsets, validate the bracket, arm the
@@ -1320,85 +1893,8 @@ static __global__ __launch_bounds__(kBlock) void k_expand_mask(
   }
 }
 
-// Settles the bracket's candidates in the expanded mask: keys above the
-// threshold are selected; of the ties, the first `need` by index.  After the
-// tile scan tile_eq[c] counts the ties before chunk c, so only the one chunk
-// where the quota runs out has to rank its ties (a chunk's candidates are
-// contiguous and index-ordered in the list).
-static __global__ __launch_bounds__(kBlock) void k_cand_mask(ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const SelState* __restrict__ st = J.st;
-  if (!st->bracket_ok) return;
-  const uint32_t* __restrict__ cand_idx = J.cand_idx;
-  const uint32_t* __restrict__ cand_key = J.cand_key;
-  const uint32_t* __restrict__ tile_eq = J.tile_eq;
-  const int64_t n_tiles = J.n_tiles;
-  const int tie_all = J.tie_all;
-  uint8_t* __restrict__ mask = J.mask;
-  const uint32_t T = st->thresh_bits, nc = st->cand_count, n_eq = st->n_eq;
-  const uint32_t need = tie_all ? 0xFFFFFFFFu : st->need;
-  for (uint32_t j = blockIdx.x * kBlock + threadIdx.x; j < nc; j += gridDim.x * kBlock) {
-    const uint32_t key = cand_key[j];
-    if (key < T) continue;
-    const uint32_t idx = cand_idx[j];
-    bool on = true;
-    if (key == T && need < n_eq) {
-      const uint32_t c = idx >> 10;
-      const uint32_t before = tile_eq[c];
-      const uint32_t upto = (int64_t)c + 1 < n_tiles ? tile_eq[c + 1] : n_eq;
-      if (before >= need) {
-        on = false;
-      } else if (upto > need) {            // the quota ends inside this chunk
-        uint32_t rank = before;
-        for (uint32_t q = j; q > 0 && (cand_idx[q - 1] >> 10) == c; --q)
-          rank += cand_key[q - 1] == T;
-        on = rank < need;
-      }
-    }
-    if (on) mask[idx] = 1;
-  }
-}
-
-// The same settlement when the mask itself is kept as bit planes.
-static __global__ __launch_bounds__(kBlock) void k_cand_bits(ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const SelState* __restrict__ st = J.st;
-  if (!st->bracket_ok) return;
-  const uint32_t* __restrict__ cand_idx = J.cand_idx;
-  const uint32_t* __restrict__ cand_key = J.cand_key;
-  const uint32_t* __restrict__ tile_eq = J.tile_eq;
-  const int64_t n_tiles = J.n_tiles;
-  const int tie_all = J.tie_all;
-  uint32_t* __restrict__ planes = J.planes;
-  const uint32_t T = st->thresh_bits, nc = st->cand_count, n_eq = st->n_eq;
-  const uint32_t need = tie_all ? 0xFFFFFFFFu : st->need;
-  for (uint32_t j = blockIdx.x * kBlock + threadIdx.x; j < nc; j += gridDim.x * kBlock) {
-    const uint32_t key = cand_key[j];
-    if (key < T) continue;
-    const uint32_t idx = cand_idx[j];
-    bool on = true;
-    if (key == T && need < n_eq) {
-      const uint32_t c = idx >> 10;
-      const uint32_t before = tile_eq[c];
-      const uint32_t upto = (int64_t)c + 1 < n_tiles ? tile_eq[c + 1] : n_eq;
-      if (before >= need) {
-        on = false;
-      } else if (upto > need) {
-        uint32_t rank = before;
-        for (uint32_t q = j; q > 0 && (cand_idx[q - 1] >> 10) == c; --q)
-          rank += cand_key[q - 1] == T;
-        on = rank < need;
-      }
-    }
-    if (on) {
-      const uint32_t lane = (idx >> 2) & 63u, e = idx & 3u;
-      atomicOr(&planes[(idx >> 8) * 8 + 2 * e + (lane >> 5)], 1u << (lane & 31));
-    }
-  }
-}
-
-// Ordered full pass that writes the mask as bit planes (the fallback of
-// k_cand_bits when the sampled bracket failed or was never tried).
+// Ordered full pass that writes the mask as bit planes: where no bracket was settled (k_settle), or
+// none was tried.
 template <class Src>
 __global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJobs jobs) {
   const ChainJob& J = jobs.j[blockIdx.y];
@@ -1458,32 +1954,54 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
   }
 }
 
-// The select of every job of a batch: begin -> (sampled-bracket path: sample, dual-rank descent,
-// ONE data sweep per job, check, candidate compaction and descent, per-chunk counts) -> the radix
-// passes (no-ops unless a job's bracket failed) -> chunk scan.  The short kernels run once for
-// the whole batch; only the data sweeps are launched per job.
+// The select of every job of a batch: begin -> (sampled-bracket path: coarse sample and pick, fine sample
+// and pick, ONE data sweep per job, settlement) -> the radix passes (no-ops unless a job's bracket
+// failed) -> chunk scan.  The short kernels run once for the whole batch; only the data sweeps are
+// launched per job.
 // PM: what the sweep leaves behind for a mask-only caller -- 0 nothing, 1 the keys above the
-// bracket as bit planes (job.planes), 2 as mask bytes (job.mask) -- to be finished by
-// finish_planes / finish_mask from those bits and the candidates instead of re-reading the data.
+// bracket as bit planes (job.planes), 2 as mask bytes (job.mask) -- where the settlement adds the
+// candidates; a writing pass over the data (finish_planes / finish_mask) is then a no-op.
 // All jobs of a batch take the same path (`fast`: SelBatch::fast_ok for every one of them).
 //
 // The chain comes in phases so that a batch whose jobs form their keys differently (the
 // re-selections of a replay step rank by different scores) still shares every kernel that does
-// not form keys: chain_begin, chain_sample_levels, chain_candidates, launch_tile_scan (and the
-// settlement) take the whole batch; chain_sample, chain_sweeps and chain_fallback are templates
-// of the key source and take the jobs of one kind (a sub-batch over the same workspaces).
-static inline void chain_begin(const SelBatch& B, bool fast, hipStream_t s, double sigmas = kBracketSigmas) {
-  hipLaunchKernelGGL(k_chain_begin, B.grid(1), dim3(kBlock), 0, s, B.jobs, fast ? 1 : 0, sigmas);
+// not form keys: chain_begin, chain_pick_*, chain_settle and launch_tile_scan take the whole batch;
+// chain_sample_*, chain_sweeps and chain_fallback are templates of the key source and take the jobs of
+// one kind (a sub-batch over the same workspaces).
+static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, bool fast, hipStream_t s) {
+  static_assert(sizeof(ChainJobs) + sizeof(SegDirJobs) + 64 <= 4096, "operands travel in the kernel arguments");
+  hipLaunchKernelGGL(k_chain_begin, B.grid(fast ? 32 : 4), dim3(kBlock), 0, s, B.jobs, dirs, fast ? 1 : 0);
 }
 template <class Src>
-static inline void chain_sample(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
-  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + 64 <= 4096,
+static inline void launch_sample_coarse(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
+                                        bool of_fine, hipStream_t s) {
+  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + 64 <= 4096,
                 "the operands of a batched chain kernel travel in its 4 KiB of kernel arguments");
-  hipLaunchKernelGGL((k_sample<Src>), B.grid(stream_grid(B.max_nsv, kBlock)), dim3(kBlock), 0, s,
-                     srcs, B.jobs);
+  int64_t n_sv = 0;
+  for (int b = 0; b < B.count; ++b) n_sv = n_sv > small_sample_vecs(B.jobs.j[b].n) ? n_sv : small_sample_vecs(B.jobs.j[b].n);
+  hipLaunchKernelGGL((k_sample_coarse<Src>), B.grid((unsigned)cdiv64(n_sv, kBlock) + 1), dim3(kBlock), 0, s, srcs,
+                     B.jobs, dirs, of_fine ? 1 : 0);
 }
-static inline void chain_sample_levels(const SelBatch& B, hipStream_t s) {
-  for (int level = 0; level < 3; ++level) launch_level_raw<false>(B, level, s, kRawKeyBlocks);
+template <class Src>
+static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
+  hipLaunchKernelGGL((k_sample_fine<Src>), B.grid((unsigned)cdiv64(B.max_nsv, kBlock)), dim3(kBlock), 0, s, srcs,
+                     B.jobs);
+}
+static inline void chain_pick_coarse(const SelBatch& B, double sigmas, hipStream_t s) {
+  hipLaunchKernelGGL((k_pick_coarse<true>), B.grid(1), dim3(kWide), 0, s, B.jobs, sigmas);
+}
+static inline void chain_pick_fine(const SelBatch& B, double sigmas, hipStream_t s) {
+  hipLaunchKernelGGL(k_pick_fine, B.grid(1), dim3(kWide), 0, s, B.jobs, sigmas);
+}
+// begin ... bracket, for a batch of one key source
+template <class Src>
+static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
+                                 hipStream_t s) {
+  chain_begin(B, dirs, true, s);
+  launch_sample_coarse(srcs, B, SegDirJobs{}, true, s);
+  chain_pick_coarse(B, sigmas, s);
+  launch_sample_fine(srcs, B, s);
+  chain_pick_fine(B, sigmas, s);
 }
 template <class Src>
 static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int pm, hipStream_t s) {
@@ -1493,35 +2011,36 @@ static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int
     const unsigned sweep_blocks = (unsigned)cdiv64(J.n_tiles, kChunksPerBlock);
     ProfPair* pp = prof_begin(SGA_PROF_SELECT_SWEEP, s);
     // the sweep's two totals go through 256 partial counters (blk_gt / blk_eq are free until
-    // the tile scan, which runs after the check has read them)
+    // the tile scan, which runs after the settlement has read them)
     if (pm == 2)
       hipLaunchKernelGGL((k_bracket_sweep<Src, 2>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.aux, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
+                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
                          w.seg_cnt, (uint32_t)w.seg_cap, (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
                          J.mask, (reinterpret_cast<uintptr_t>(J.mask) & 3) == 0);
     else if (pm == 1)
       hipLaunchKernelGGL((k_bracket_sweep<Src, 1>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.aux, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
+                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
                          w.seg_cnt, (uint32_t)w.seg_cap, J.planes, w.blk_gt, w.blk_eq);
     else
       hipLaunchKernelGGL((k_bracket_sweep<Src, 0>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.aux, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
+                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
                          w.seg_cnt, (uint32_t)w.seg_cap, (uint32_t*)nullptr, w.blk_gt, w.blk_eq);
     prof_end(pp, s);
   }
 }
-static inline void chain_candidates(const SelBatch& B, hipStream_t s) {
-  hipLaunchKernelGGL(k_bracket_check, B.grid(1), dim3(kBlock), 0, s, B.jobs);
-  hipLaunchKernelGGL(k_cand_compact, B.grid(256), dim3(kBlock), 0, s, B.jobs);
-  // a batch's candidate lists are as long as a single select's (millions of keys each at large
-  // sizes and ratios): 256 workgroups for the batch, where the sample's short passes take 64
-  // (four re-selections of the 596 M-element replay set: 97 us for the three levels, 203 with 64)
-  for (int level = 0; level < 3; ++level)
-    launch_level_raw<true>(B, level, s, B.count > 1 ? 4 * kRawKeyBlocks : kRawKeyBlocks);
-  hipLaunchKernelGGL(k_cand_tiles, B.grid(256), dim3(kBlock), 0, s, B.jobs);
+static inline void chain_settle(const SelBatch& B, hipStream_t s) {
+  // The work is the random atomics and stores of about n / 800 candidates: a workgroup per 4 M coordinates,
+  // no fewer than hold every segment at once (64; a batch shares them), no more than the chip has CUs.
+  const int64_t want = B.max_n >> 22, least = B.count > 1 ? 32 : 64;
+  const unsigned wgs = (unsigned)(want < least ? least : want > 256 ? 256 : want);
+  hipLaunchKernelGGL(k_settle, B.grid(wgs), dim3(kWide), 0, s, B.jobs);
+}
+// behind the chunk scan, for callers whose mask or planes the settlement fills
+static inline void chain_settle_ties(const SelBatch& B, hipStream_t s) {
+  hipLaunchKernelGGL(k_settle_ties, B.grid(256), dim3(kBlock), 0, s, B.jobs);
 }
 // The radix passes and the per-chunk counts over the data: no-ops unless a job's bracket failed
-// (st->skip == 0; k_bracket_check left the histograms zeroed for them) or was never tried.
+// (st->skip == 0) or was never tried.
 template <class Src>
 static inline void chain_fallback(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
   for (int level = 0; level < 3; ++level) launch_level_data<Src, true>(srcs, B, level, s);
@@ -1529,36 +2048,25 @@ static inline void chain_fallback(const SrcPack<Src>& srcs, const SelBatch& B, h
 }
 
 template <class Src>
-static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, bool fast, int pm,
-                                    hipStream_t s, double sigmas = kBracketSigmas) {
-  chain_begin(B, fast, s, sigmas);
+static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, bool fast,
+                                    int pm, hipStream_t s) {
   if (fast) {
-    chain_sample(srcs, B, s);
-    chain_sample_levels(B, s);
+    chain_bracket(srcs, B, dirs, kBracketSigmas, s);
     chain_sweeps(srcs, B, pm, s);
-    chain_candidates(B, s);
+    chain_settle(B, s);
+  } else {
+    chain_begin(B, dirs, false, s);
   }
   chain_fallback(srcs, B, s);
   launch_tile_scan(B, s);
+  if (fast && pm != 0) chain_settle_ties(B, s);
 }
 
-// Bit-plane masks of the selections after run_select_batch(..., pm = 1): the candidates settle
-// the sweep's planes when the bracket held, else the ordered full pass writes them.
-template <class Src>
-static inline void finish_planes_batch(const SrcPack<Src>& srcs, const SelBatch& B, bool fast,
-                                       hipStream_t s) {
-  if (fast) hipLaunchKernelGGL(k_cand_bits, B.grid(256), dim3(kBlock), 0, s, B.jobs);
-  hipLaunchKernelGGL((k_write_bits<Src>), B.grid(stream_grid(B.max_tiles, kChunksPerBlock, 1 << 14)),
-                     dim3(kBlock), 0, s, srcs, B.jobs);
-}
-
-// Byte masks after run_select_batch(..., pm = 2) (the sweep wrote the provisional selection
-// straight into the caller's mask): the candidates settle it when the bracket held, else the
-// ordered full pass writes it.
+// Byte masks after run_select_batch(..., pm = 2): the sweep and the settlement wrote them when the bracket
+// held, else the ordered full pass does.
 template <class Src>
 static inline void finish_mask_batch(const SrcPack<Src>& srcs, const SelBatch& B, bool fast,
                                      hipStream_t s) {
-  if (fast) hipLaunchKernelGGL(k_cand_mask, B.grid(256), dim3(kBlock), 0, s, B.jobs);
   hipLaunchKernelGGL((k_write_mask<Src>), B.grid(stream_grid(B.max_tiles, kChunksPerBlock, 1 << 14)),
                      dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0, fast ? 1 : 0, (uint8_t*)nullptr);
 }

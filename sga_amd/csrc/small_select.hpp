@@ -1,6 +1,6 @@
 // Exact top-k of a bucket of up to kSmallTiles chunks (8.4 M coordinates) in four launches:
-//   k_small_sample    8 K to 16 K sample keys (and the directory of the segment table)
-//   k_small_pick      one workgroup brackets the k-th key between two sample keys
+//   k_sample_coarse   8 K to 16 K sample keys (and the directory of the segment table)
+//   k_pick_coarse     one workgroup brackets the k-th key between two sample keys
 //   k_small_sweep     the one sweep over the data: per-chunk counts above the bracket, and a list
 //                     of the few keys inside it
 //   k_small_finish    one workgroup: exact threshold from the list, ties to grant, and the
@@ -21,127 +21,16 @@
 // The result is exact for any sample: a bracket that misses the k-th key is redone by the finishing
 // workgroup over the data itself.
 #pragma once
-#include "adam_math.hpp"
 #include "select_impl.hpp"
 
 namespace sga {
 
 #ifdef __HIPCC__
 
-constexpr int kWide = 1024;                       // threads of the one-workgroup kernels
-constexpr int kWideWaves = kWide / kWave;         // 16
-// Sample: one quad of keys in 512 coordinates, 8 K to 16 K keys (or all).  A thousand more keys cost
-// the picking workgroup 0.25 us and a thousand more list entries the finishing one 0.12: at 4 M
-// coordinates and 1 % (35 K entries from 16 K keys) the two sum to a flat minimum near these sizes.
-constexpr int64_t kSmallSampleMin = 2048, kSmallSampleMax = 4096;
-__host__ __device__ static inline int64_t small_sample_vecs(int64_t n) {
-  int64_t v = n / 512;
-  if (v < kSmallSampleMin) v = kSmallSampleMin;
-  if (v > kSmallSampleMax) v = kSmallSampleMax;
-  return v < n / 4 ? v : n / 4;
-}
-constexpr int kSmallPick = (int)(kSmallSampleMax / kWide);   // quads per thread of the picking workgroup
-
-// A key source that looks tensors up: without the directory (it is being built while the sample is
-// taken) the lookup bisects the table.
-template <class S>
-__device__ __forceinline__ auto drop_dir(S& s, int) -> decltype(s.sc.dir, void()) { s.sc.dir = nullptr; }
-template <class S>
-__device__ __forceinline__ void drop_dir(S&, long) {}
-
-// LDS scratch of the workgroup-wide scans.  Consecutive scans alternate between the two halves
-// (`turn`), so one scan's last reads and the next one's first writes need no barrier between them.
-struct WideScratch {
-  uint32_t tot[2][kWideWaves];
-  uint32_t hit[2][2][3];
-};
-
-// Exclusive prefix sum over the workgroup, and the total.  One barrier.
-__device__ __forceinline__ uint32_t wide_prefix(uint32_t mine, WideScratch& s, int turn, uint32_t& total) {
-  const uint32_t incl = wave_incl_scan(mine);
-  if (lane_id() == kWave - 1) s.tot[turn][wave_id()] = incl;
-  __syncthreads();
-  uint32_t before = incl - mine, all = 0;
-#pragma unroll
-  for (int w = 0; w < kWideWaves; ++w) {
-    const uint32_t t = s.tot[turn][w];
-    before += w < wave_id() ? t : 0u;
-    all += t;
-  }
-  total = all;
-  return before;
-}
-
-struct RankHit { uint32_t bin, above, count; };
-// The bins of a 4096-bin LDS histogram where the count from the top reaches each of NR ranks
-// (1-based).  All threads get the answers.  Two barriers, after the one that completes the histogram.
-template <int NR>
-__device__ __forceinline__ void wide_find_rank(const uint32_t* s_hist, const uint32_t (&rank)[NR],
-                                               WideScratch& s, int turn, RankHit (&hit)[NR]) {
-  constexpr int PER = kBinsBig / kWide;           // 4
-  const U4 q = reinterpret_cast<const U4*>(s_hist)[threadIdx.x];
-  const uint32_t h[PER] = {q.x, q.y, q.z, q.w};
-  const uint32_t mine = h[0] + h[1] + h[2] + h[3];
-  uint32_t total;
-  const uint32_t before = wide_prefix(mine, s, turn, total);
-#pragma unroll
-  for (int r = 0; r < NR; ++r) {
-    uint32_t above = total - before - mine;
-    if (above < rank[r] && rank[r] <= above + mine) {
-#pragma unroll
-      for (int j = PER - 1; j >= 0; --j) {
-        if (above < rank[r] && rank[r] <= above + h[j]) {
-          s.hit[turn][r][0] = (uint32_t)(threadIdx.x * PER + j);
-          s.hit[turn][r][1] = above;
-          s.hit[turn][r][2] = h[j];
-        }
-        above += h[j];
-      }
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NR; ++r) hit[r] = RankHit{s.hit[turn][r][0], s.hit[turn][r][1], s.hit[turn][r][2]};
-}
-
-// Short list of keys in LDS (what one histogram bin holds): `rank` (1-based, from the top) by counting.
-// The thread that owns an entry compares it with all of them; the one whose key it is leaves (key,
-// keys above, equal keys) in out.  128 entries cost 32 LDS reads of two waves; with 1024 the one LDS
-// of the workgroup was busy for 20 us.
-constexpr int kWideList = 128;
-__device__ __forceinline__ void wide_list_rank(const uint32_t* s_key, uint32_t cnt, uint32_t rank, uint32_t* out) {
-  if (threadIdx.x >= cnt) return;
-  const uint32_t me = s_key[threadIdx.x];
-  uint32_t gt = 0, eq = 0;
-  for (uint32_t j = 0; j < cnt; j += kVec) {
-    const U4 o = *reinterpret_cast<const U4*>(s_key + j);
-    const uint32_t left = cnt - j;
-    gt += (o.x > me) + (left > 1 && o.y > me) + (left > 2 && o.z > me) + (left > 3 && o.w > me);
-    eq += (o.x == me) + (left > 1 && o.y == me) + (left > 2 && o.z == me) + (left > 3 && o.w == me);
-  }
-  if (gt < rank && rank <= gt + eq) { out[0] = me; out[1] = gt; out[2] = eq; }   // equal keys write the same
-}
-
-// One LDS increment per participating lane; a wave whose lanes all hit one bin (a plateau of equal
-// keys) adds once.  For loops of unbounded length only: the 16 to 20 keys per thread of the usual
-// passes add plainly (one workgroup's instruction issue is the bound there -- 0.2 us for every
-// instruction per key of 24 K keys -- and 64 lanes on one bin cost no more than this test).
-__device__ __forceinline__ void wide_hist_add(uint32_t* s_hist, uint32_t bin, bool part) {
-  const uint64_t act = ballot64(part);
-  if (act == 0) return;
-  const uint32_t lead = (uint32_t)__builtin_amdgcn_readlane((int)bin, __ffsll((unsigned long long)act) - 1);
-  if (ballot64(part && bin != lead) == 0) {
-    if (lane_id() == 0) atomicAdd(&s_hist[lead], (uint32_t)__popcll(act));
-  } else if (part) {
-    atomicAdd(&s_hist[bin], 1u);
-  }
-}
-
 // Candidate lists of the small path: WGs of the sweep share kSmallSegs counters (the segments of
 // the list); a segment has room for every coordinate of its workgroups, so it never overflows.
 // The counters lie 256 bytes apart: atomics on one cache line queue like those on one address (11 ns
 // each; 1024 workgroups on 16 adjacent words: the sweep of 4 M elements took 19 us, 8.6 with this).
-constexpr int kSmallSegStride = 64;
 struct SmallGeom { uint32_t n_wg, segs, cap; };    // cap: list entries per segment
 __host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles) {
   SmallGeom s;
@@ -150,130 +39,6 @@ __host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles) {
   s.segs = (uint32_t)cdiv64(s.n_wg, per);
   s.cap = per * (uint32_t)kBlockSpan;
   return s;
-}
-
-// Sample keys (one quad per window at a hashed offset; the windows tile all quads, see k_sample),
-// the list counters, and, in a job's last workgroup, the directory of its segment table
-// (dirs.j[job].dir null: none wanted).  Gathering from one workgroup would be bound by one CU's
-// translation misses (4096 quads of two arrays: 25 us; 64 workgroups: 4).
-template <class Src>
-__global__ __launch_bounds__(kBlock) void k_small_sample(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  if (blockIdx.x == gridDim.x - 1) {
-    if (threadIdx.x < kSmallSegs) J.seg_cnt[threadIdx.x * kSmallSegStride] = 0u;
-    const auto& D = dirs.j[blockIdx.y];
-    if (D.dir) {
-      const int64_t nb = (D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
-      for (int64_t b = threadIdx.x; b < nb; b += kBlock) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
-    }
-    return;
-  }
-  Src src = srcs.s[blockIdx.y];
-  drop_dir(src, 0);
-  const int64_t n_vec = J.n / 4, n_sv = small_sample_vecs(J.n);
-  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (j >= n_sv) return;
-  const int64_t w0 = j * n_vec / n_sv, w1 = (j + 1) * n_vec / n_sv;
-  const int64_t vec = w0 + (int64_t)(mix32((uint32_t)j + J.seed * 0x9E3779B9u) % (uint32_t)(w1 - w0));
-  uint32_t key[4];
-  src.template load<false>(vec * 4, J.n, key);
-  // the list is written by the sweep, after the sample has been read: its memory holds the sample
-  reinterpret_cast<U4*>(J.small_idx)[j] = U4{key[0], key[1], key[2], key[3]};
-}
-
-// One workgroup per job: state reset, the two ends of the bracket from the sample.  The top 12 bits of
-// all keys go into one LDS histogram, the next 12 of the keys in the two bins the ends fall into into
-// one each; what is left in a bin then is ranked by counting (or split by the last 7 bits, on plateaus).
-static __global__ __launch_bounds__(kWide) void k_small_pick(ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
-  __shared__ __align__(16) uint32_t s_list[2][kWideList];
-  __shared__ uint32_t s_cnt[2], s_out[2][3];
-  __shared__ WideScratch s_scan;
-  const int64_t n = J.n;
-  const int64_t n_sv = small_sample_vecs(n);
-  U4 key[kSmallPick];
-#pragma unroll
-  for (int u = 0; u < kSmallPick; ++u) {
-    const int64_t j = (int64_t)u * kWide + threadIdx.x;
-    if (u * (int64_t)kWide < n_sv && j < n_sv) key[u] = reinterpret_cast<const U4*>(J.small_idx)[j];
-  }
-  const U4 zero{0u, 0u, 0u, 0u};
-  reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
-  if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
-  __syncthreads();
-  const uint32_t ns = (uint32_t)(n_sv * 4);
-  const double frac = (double)J.k / (double)n, r = frac * (double)ns;
-  const double d = kBracketSigmas * sqrt(r * (1.0 - frac) + 1.0) + 8.0;
-  const double rh = floor(r - d), rl = ceil(r + d);
-  const bool open_hi = rh < 1.0 || ns == 0, open_lo = rl > (double)ns || ns == 0;
-  const uint32_t rank[2] = {open_hi ? 1u : (uint32_t)rh, open_lo ? 1u : (uint32_t)rl};
-  uint32_t t_hi = 0x80000000u, t_lo = 0u;
-  if (ns) {
-    auto each = [&](auto&& f) {
-#pragma unroll
-      for (int u = 0; u < kSmallPick; ++u) {
-        if (u * (int64_t)kWide >= n_sv) break;                  // uniform
-        const bool live = (int64_t)u * kWide + threadIdx.x < n_sv;
-        f(key[u].x, live); f(key[u].y, live); f(key[u].z, live); f(key[u].w, live);
-      }
-    };
-    each([&](uint32_t kk, bool live) { if (live) atomicAdd(&s_h[0][kk >> kL0Shift], 1u); });
-    __syncthreads();
-    RankHit hit[2];
-    wide_find_rank<2>(s_h[0], rank, s_scan, 0, hit);
-    uint32_t bin[2] = {hit[0].bin, hit[1].bin};
-    uint32_t rk[2] = {rank[0] - hit[0].above, rank[1] - hit[1].above};
-    uint32_t cnt[2] = {hit[0].count, hit[1].count};
-    int w = kL0Shift, turn = 1;                        // bits of a key below the bins found so far
-    while (w > 0 && (cnt[0] > (uint32_t)kWideList || cnt[1] > (uint32_t)kWideList)) {
-      const int sh = w > 12 ? w - 12 : 0, bits = w - sh;
-      reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
-      reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
-      __syncthreads();
-      each([&](uint32_t kk, bool live) {
-        const uint32_t top = kk >> w;
-        if (!live || (top != bin[0] && top != bin[1])) return;
-        const uint32_t low = (kk >> sh) & ((1u << bits) - 1u);
-        if (top == bin[0]) atomicAdd(&s_h[0][low], 1u);
-        if (top == bin[1]) atomicAdd(&s_h[1][low], 1u);
-      });
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint32_t want[1] = {rk[q]};
-        RankHit h[1];
-        wide_find_rank<1>(s_h[q], want, s_scan, turn, h);
-        turn ^= 1;
-        bin[q] = (bin[q] << bits) | h[0].bin;
-        rk[q] -= h[0].above;
-        cnt[q] = h[0].count;
-      }
-      w = sh;
-    }
-    if (w > 0) {
-      each([&](uint32_t kk, bool live) {
-        const uint32_t top = kk >> w;
-        if (!live || (top != bin[0] && top != bin[1])) return;
-        if (top == bin[0]) s_list[0][atomicAdd(&s_cnt[0], 1u)] = kk;
-        if (top == bin[1]) s_list[1][atomicAdd(&s_cnt[1], 1u)] = kk;
-      });
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < 2; ++q) wide_list_rank(s_list[q], cnt[q], rk[q], s_out[q]);
-      __syncthreads();
-    }
-    // keys equal to the upper sample key stay inside the bracket
-    if (!open_hi) t_hi = (w > 0 ? s_out[0][0] : bin[0]) + 1u;
-    if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
-  }
-  if (threadIdx.x == 0) {
-    SelState z = {};
-    z.k = J.k;
-    z.t_hi = t_hi;
-    z.t_lo = t_lo;
-    *J.st = z;
-  }
 }
 
 // The sweep: one chunk per wave, counts above the bracket, keys inside it to the list (one
@@ -323,22 +88,11 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
     }
     return;
   }
-  // more keys than the wave's LDS holds (the bracket's keys crowd into few chunks): form them again
-  src.chunk_hyper(c);
-  for (int it = 0; it < kChunkIters; ++it) {
-    const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
-    uint32_t key[4] = {0u, 0u, 0u, 0u};
-    if (i < n) src.template load<false>(i, n, key);
-    Ballot4 in;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) in.m[e] = ballot64(i + e < n && key[e] >= T_LO && key[e] < T_HI);
-    uint32_t run = 0;
-    ballot_append(in, run, [&](uint32_t pos, int e) {
-      J.small_idx[base + pos] = (uint32_t)(i + e);
-      J.small_key[base + pos] = key[e];
-    });
-    base += run;
-  }
+  // more keys than the wave's LDS holds: the bracket's keys crowd into few chunks
+  recollect(src, n, c, T_LO, T_HI, [&](uint32_t pos, uint32_t idx, uint32_t key) {
+    J.small_idx[base + pos] = idx;
+    J.small_key[base + pos] = key;
+  });
 }
 
 // The candidate list as the finishing workgroup sees it: wave w owns segment w (kSmallSegs ==
@@ -603,13 +357,8 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
 template <class Src>
 static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
                                     hipStream_t s) {
-  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + 64 <= 4096,
-                "the operands travel in the 4 KiB of kernel arguments");
-  int64_t n_sv = 0;
-  for (int b = 0; b < B.count; ++b) n_sv = n_sv > small_sample_vecs(B.jobs.j[b].n) ? n_sv : small_sample_vecs(B.jobs.j[b].n);
-  hipLaunchKernelGGL((k_small_sample<Src>), B.grid((unsigned)cdiv64(n_sv, kBlock) + 1), dim3(kBlock), 0, s, srcs,
-                     B.jobs, dirs);
-  hipLaunchKernelGGL(k_small_pick, B.grid(1), dim3(kWide), 0, s, B.jobs);
+  launch_sample_coarse(srcs, B, dirs, false, s);
+  hipLaunchKernelGGL((k_pick_coarse<false>), B.grid(1), dim3(kWide), 0, s, B.jobs, kBracketSigmas);
   hipLaunchKernelGGL((k_small_sweep<Src>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)), dim3(kBlock),
                      0, s, srcs, B.jobs);
   hipLaunchKernelGGL((k_small_finish<Src>), B.grid(1), dim3(kWide), 0, s, srcs, B.jobs);

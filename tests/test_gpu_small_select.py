@@ -1,5 +1,6 @@
 """Exact top-k of buckets up to 8,388,608 coordinates (csrc/small_select.hpp) at
-the edges of its tiles, its lists and its sample, against the oracle."""
+the edges of its tiles, its lists and its sample, and of larger ones where the
+settlement of the bracket takes another way (k_settle), against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -51,6 +52,27 @@ def test_plateaus_and_crowded_chunks(dev, n):
     for name, sc in (("grid", grid), ("hot", hot), ("steep", steep)):
         for k in (n // 1000, n // 100, n // 41, n // 10):
             _check(dev, sc, k, (name, n, k))
+
+
+@pytest.mark.parametrize("n", [LIMIT + 5, 20_000_003])
+@pytest.mark.parametrize("name", ["plain", "grid", "zeros", "crowd", "hot"])
+def test_settlement_of_large_buckets(dev, n, name):
+    sc = student_t(n, 5).abs()
+    k = n // 100
+    if name == "grid":                              # one key value in the threshold's bin, more than LDS holds
+        sc = sc.to(torch.bfloat16).float()
+    elif name == "zeros":                           # a plateau: nothing is collected
+        sc = torch.where(sc > sc.kthvalue(n - n // 200)[0], sc, torch.zeros(()))
+    elif name == "crowd":                           # many keys in the threshold's bin, more than LDS holds
+        top = sc > sc.kthvalue(n - k - n // 8)[0]
+        near = 4.0 + torch.arange(n, dtype=torch.float32) % 251 * 2.0 ** -20
+        sc = torch.where(top, torch.where(sc > sc.kthvalue(n - k + k // 64)[0], sc + 8.0, near), sc * 0.01)
+    elif name == "hot":                             # more than a wave's list holds, and in few segments
+        sc *= 1e-6
+        sc[n // 2:n // 2 + n // 400] += 1.0
+        k = n // 450
+    for kk in (k, k + 1) if name != "plain" else (1, k, n - 3):
+        _check(dev, sc, kk, (name, n, kk))
 
 
 def _mix32(x):
