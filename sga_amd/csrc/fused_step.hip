@@ -437,7 +437,7 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   if (small) {
     run_small_select(srcs, B, dj, s);
   } else {
-    run_select_batch(srcs, B, dj, use_fast, planes ? 1 : 0, s);
+    run_select_batch<0>(srcs, B, dj, use_fast, planes ? 1 : 0, s);
   }
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
@@ -469,7 +469,6 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     }
     prof_end(pp, s);
   }
-  if (!small) launch_result(B, s);
   return check_launch(who);
 }
 
@@ -1212,11 +1211,8 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
                      x.tie_cnt);
   for (int level = 0; level < 3; ++level) launch_level_raw(B, level, s, 3 * kRawKeyBlocks);
   hipLaunchKernelGGL(k_cand_tiles, B.grid(512), dim3(kBlock), 0, s, B.jobs);
-  // only when the sweep stood back: the radix passes over the untouched data
-  for (int level = 0; level < 3; ++level)
-    launch_level_data<SrcFused<BF16G, SCORE>, true>(srcs, B, level, s);
-  launch_tile_count(srcs, B, 0, s);
-  launch_tile_scan(B, s);
+  // the chunk scan; before it, only when the sweep stood back, the radix passes over the untouched data
+  chain_tail<0>(srcs, B, s);
   hipLaunchKernelGGL(k_spec_ties, dim3(512), dim3(kBlock), 0, s, w.st, w.cand_idx, w.cand_key,
                      w.tile_eq, n_tiles, x.tie_cnt, x.tie_idx);
   hipLaunchKernelGGL(k_spec_settle, dim3(512), dim3(kBlock), 0, s, w.st, w.cand_idx, w.cand_key,
@@ -1239,7 +1235,6 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>),
                      dim3(stream_grid(n_tiles, kChunksPerBlock, 2048)), dim3(kBlock), 0, s, fa,
                      segs, n_segs, w.st, w.tile_gt, w.tile_eq, 3, w.seg_dir);
-  launch_result(B, s);
   return check_launch("sga_fused_sparse_step_single_sweep");
 }
 

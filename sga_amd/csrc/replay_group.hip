@@ -835,15 +835,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, 1, s); });
     chain_settle(B, s);
   }
-  per_score([&](auto& srcs, const SelBatch& sub) { chain_fallback(srcs, sub, s); });
-  launch_tile_scan(B, s);
-  if (fast) chain_settle_ties(B, s);
-  per_score([&](auto& srcs, const SelBatch& sub) {
-    using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
-    hipLaunchKernelGGL((k_write_bits<Src>), sub.grid(stream_grid(sub.max_tiles, kChunksPerBlock, 1 << 14)),
-                       dim3(kBlock), 0, s, srcs, sub.jobs);
-  });
-  launch_result(B, s);
+  per_score([&](auto& srcs, const SelBatch& sub) { chain_tail<1>(srcs, sub, s); });
   return check_launch(who);
 }
 

@@ -271,7 +271,7 @@ extern "C" int sga_sel_hist(const float* score, int64_t n, int level, void* ws,
   srcs.s[0] = SrcF32{score, aligned4(score, 4)};
   SelBatch B;
   B.add(w, n, 1, 0);
-  launch_level_data<SrcF32, false>(srcs, B, level, (hipStream_t)stream);
+  launch_level_data<SrcF32>(srcs, B, level, (hipStream_t)stream);
   return check_launch("sga_sel_hist");
 }
 
@@ -324,8 +324,7 @@ extern "C" int sga_sel_mask(const float* score, int64_t n, int64_t tile_base, in
   SelBatch B;
   B.add(w, n, 1, tie_mode == SGA_TIE_ALL).mask = mask_out;
   hipLaunchKernelGGL((k_write_mask<SrcF32>), B.grid(stream_grid(B.max_tiles, kChunksPerBlock, 1 << 22)),
-                     dim3(kBlock), 0, (hipStream_t)stream, srcs, B.jobs, tile_base, 0,
-                     (uint8_t*)nullptr);
+                     dim3(kBlock), 0, (hipStream_t)stream, srcs, B.jobs, tile_base);
   return check_launch("sga_sel_mask");
 }
 
@@ -359,15 +358,13 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   if (SelBatch::small_ok(n)) {
     run_small_select(srcs, B, SegDirJobs{}, s);
     hipLaunchKernelGGL((k_write_mask<SrcF32>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)),
-                       dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0, 0, (uint8_t*)nullptr);
+                       dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0);
     return check_launch("sga_select_topk");
   }
   const bool fast = SelBatch::fast_ok(w, n);
   // the select sweep writes the keys above the bracket straight into mask_out
   J.mask_only = 1;
-  run_select_batch(srcs, B, SegDirJobs{}, fast, 2, s);
-  finish_mask_batch(srcs, B, fast, s);
-  launch_result(B, s);
+  run_select_batch<2>(srcs, B, SegDirJobs{}, fast, 2, s);
   return check_launch("sga_select_topk");
 }
 

@@ -52,8 +52,10 @@ struct SelState {
   uint32_t edge_cnt;    // k_settle: entries of the edge list
   uint32_t edge_inv;    // k_settle: ~(smallest key of the edge list), and ...
   uint32_t edge_max;    // ... the largest, by atomic maxima (0: none)
-  uint32_t ties_left;   // k_settle_ties has the ties to place
-  uint32_t pad_[31];
+  uint32_t ties_left;   // the settlement has left the ties to k_tail
+  uint32_t tail_ticket; // k_tail: items handed out, and ...
+  uint32_t tail_done;   // ... finished
+  uint32_t pad_[29];
 };
 static_assert(sizeof(SelState) == 256, "SelState layout");
 
@@ -353,6 +355,19 @@ __device__ __forceinline__ void level_bin(uint32_t key, uint32_t prefix, bool va
   else { bin = key & (kBinsSmall - 1); part = valid && (key >> kL1Shift) == prefix; }
 }
 
+// State that other workgroups of the same launch write or read: past the caches of this CU and XCD.
+__device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Every such store and atomic of the workgroup has landed when this returns.
+__device__ __forceinline__ void wait_landed() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
 // One level of the descent for one state, run by a single workgroup: find
 // the bin where the descending cumulative count crosses the remaining rank.
 template <int LEVEL>
@@ -365,8 +380,8 @@ __device__ __forceinline__ void level_scan_body(SelState* __restrict__ st,
   const int t = threadIdx.x;
   // read the incoming rank before any barrier: the one thread that descends
   // overwrites st->krem after the barriers below
-  const uint32_t krem = (LEVEL == 0) ? st->k : st->krem;
-  const uint32_t pre_in = (LEVEL == 0) ? 0u : st->prefix;
+  const uint32_t krem = (LEVEL == 0) ? st->k : ld_agent(&st->krem);
+  const uint32_t pre_in = (LEVEL == 0) ? 0u : ld_agent(&st->prefix);
   uint32_t loc[PER];
   uint32_t mine = 0;
 #pragma unroll
@@ -423,46 +438,22 @@ __device__ __forceinline__ uint32_t* level_hist_of(uint32_t* hist_set) {
   return hist_set + (LEVEL == 0 ? 0 : LEVEL == 1 ? kBinsBig : 2 * kBinsBig);
 }
 
-// Histogram sweep of one radix level for NS states at once (NS = 2 lets the
-// two ends of the sample bracket descend together).  n_dev (optional) caps n
-// with a count produced on the device; a state whose `skip` flag is set does
-// not take part.  MERGE: the last workgroup to finish also runs the level's
-// scan, so hist + scan is one launch.
-template <class Src, int LEVEL, int NS, bool MERGE>
-__device__ __forceinline__ void level_hist_body(Src& src, int64_t n,
-                                                const uint32_t* __restrict__ n_dev,
-                                                SelState* __restrict__ st,
-                                                uint32_t* __restrict__ hist) {
+// Histogram of one radix level, by workgroup blk of n_blk: LDS bins, flushed to global ones.
+template <class Src, int LEVEL>
+__device__ __forceinline__ void level_hist_body(Src& src, int64_t n, uint32_t prefix,
+                                                uint32_t* __restrict__ gh, uint32_t* s_h /* kBinsBig */,
+                                                uint32_t blk, uint32_t n_blk) {
   constexpr int NB = LEVEL == 2 ? kBinsSmall : kBinsBig;
-  // Level 0 has no prefix: every state sees the same histogram of all keys, so it is built and
-  // flushed once (set 0) and every state's scan reads that one.
-  constexpr int NH = LEVEL == 0 ? 1 : NS;
-  __shared__ uint32_t s_h[NH][NB];
-  __shared__ uint32_t s_suf[kBlock + 1];
-  __shared__ uint32_t s_last;
-  bool on[NS];
-  uint32_t prefix[NS];
-  bool any = false;
-#pragma unroll
-  for (int q = 0; q < NS; ++q) {
-    on[q] = st[q].skip == 0;
-    prefix[q] = st[q].prefix;
-    any = any || on[q];
-  }
-  if (!any) return;
-  if (n_dev && (int64_t)*n_dev < n) n = (int64_t)*n_dev;
-#pragma unroll
-  for (int q = 0; q < NH; ++q)
-    for (int b = threadIdx.x; b < NB; b += kBlock) s_h[q][b] = 0u;
+  for (int b = threadIdx.x; b < NB; b += kBlock) s_h[b] = 0u;
   __syncthreads();
   // Raw key buffers (sample, candidates) are short and sit in L2: what their passes cost is load
-  // latency, so each lane keeps kQuads 16-byte loads in flight per trip.  Key sources that compute
-  // (the radix passes over the data itself) go one quad at a time.
-  constexpr int kQuads = std::is_same<Src, SrcU32>::value ? 4 : 1;
+  // latency, so each lane keeps kQuads 16-byte loads in flight per trip; the passes over the data
+  // itself run on a small grid and need them too.
+  constexpr int kQuads = 4;
   constexpr int64_t kSlabKeys = (int64_t)kBlock * kVec;
-  const int64_t stride = (int64_t)gridDim.x * kSlabKeys * kQuads;
+  const int64_t stride = (int64_t)n_blk * kSlabKeys * kQuads;
   // uniform trip count so the wave-level ballots inside lds_hist_add are safe
-  const int64_t first = (int64_t)blockIdx.x * kSlabKeys * kQuads;
+  const int64_t first = (int64_t)blk * kSlabKeys * kQuads;
   for (int64_t base = first; base < n; base += stride) {
     uint32_t key[kQuads][4];
     bool full[kQuads];
@@ -480,65 +471,59 @@ __device__ __forceinline__ void level_hist_body(Src& src, int64_t n,
       const int64_t i = base + u * kSlabKeys + (int64_t)threadIdx.x * kVec;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-#pragma unroll
-        for (int q = 0; q < NH; ++q) {
-          uint32_t bin; bool part;
-          level_bin<LEVEL>(key[u][e], prefix[q], full[u] || i + e < n, bin, part);
-          const bool live = NH == NS ? on[q] : any;
-          // Raw key buffers are at most a few million keys for 64 workgroups of one wave per
-          // SIMD: what a pass costs there is the latency of each key's chain, and the folding of
-          // equal bins (two ballots, a cross-lane read and two scalar branches per key) is most of
-          // it.  A plain LDS atomic per lane is shorter; on a plateau (every lane on one bin) it
-          // serialises 64-fold, which for these few keys is a couple of microseconds.
-          if (std::is_same<Src, SrcU32>::value) {
-            if (part && live) atomicAdd(&s_h[q][bin], 1u);
-          } else {
-            lds_hist_add(s_h[q], bin, part && live);
-          }
+        uint32_t bin; bool part;
+        level_bin<LEVEL>(key[u][e], prefix, full[u] || i + e < n, bin, part);
+        // Raw key buffers are at most a few million keys for 64 workgroups of one wave per
+        // SIMD: what a pass costs there is the latency of each key's chain, and the folding of
+        // equal bins (two ballots, a cross-lane read and two scalar branches per key) is most of
+        // it.  A plain LDS atomic per lane is shorter; on a plateau (every lane on one bin) it
+        // serialises 64-fold, which for these few keys is a couple of microseconds.
+        if (std::is_same<Src, SrcU32>::value) {
+          if (part) atomicAdd(&s_h[bin], 1u);
+        } else {
+          lds_hist_add(s_h, bin, part);
         }
       }
     }
   }
   __syncthreads();
-#pragma unroll
-  for (int q = 0; q < NH; ++q) {
-    if (NH == NS && !on[q]) continue;
-    uint32_t* gh = level_hist_of<LEVEL>(hist + q * kHistStride);
-    for (int b = threadIdx.x; b < NB; b += kBlock) {
-      const uint32_t c = s_h[q][b];
-      if (c) atomicAdd(&gh[b], c);
-    }
+  for (int b = threadIdx.x; b < NB; b += kBlock) {
+    const uint32_t c = s_h[b];
+    if (c) atomicAdd(&gh[b], c);
   }
-  if (!MERGE) return;
-  __threadfence();
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const uint32_t ticket = atomicAdd(&st[0].done[LEVEL], 1u);
-    s_last = (ticket == gridDim.x - 1) ? 1u : 0u;
-  }
-  __syncthreads();
-  if (!s_last) return;
-  __threadfence();
-#pragma unroll
-  for (int q = 0; q < NS; ++q)
-    if (on[q])
-      level_scan_body<LEVEL>(&st[q], level_hist_of<LEVEL>(hist + (NH == NS ? q : 0) * kHistStride), s_suf);
-  if (threadIdx.x == 0) st[0].done[LEVEL] = 0u;
 }
-// over the data itself (a key source per job): the radix passes, state = st
-template <class Src, int LEVEL, bool MERGE>
+// True in the last of a level's n_blk workgroups.  The bins are device-scope atomics and are read by
+// atomic loads (level_scan_body): waiting for one's own is enough, no fence.
+__device__ __forceinline__ bool level_last(uint32_t* done, uint32_t n_blk, uint32_t* s_last) {
+  wait_landed();
+  if (threadIdx.x == 0) *s_last = atomicAdd(done, 1u) == n_blk - 1 ? 1u : 0u;
+  __syncthreads();
+  return *s_last != 0;
+}
+// Histogram only: several views of a staged select feed one level before its scan.
+template <class Src, int LEVEL>
 __global__ __launch_bounds__(kBlock) void k_level_hist(SrcPack<Src> srcs, ChainJobs jobs) {
+  __shared__ uint32_t s_h[kBinsBig];
   const ChainJob& J = jobs.j[blockIdx.y];
+  if (J.st->skip) return;
   Src src = srcs.s[blockIdx.y];
-  level_hist_body<Src, LEVEL, 1, MERGE>(src, J.n, nullptr, J.st, J.hist);
+  level_hist_body<Src, LEVEL>(src, J.n, J.st->prefix, level_hist_of<LEVEL>(J.hist), s_h, blockIdx.x, gridDim.x);
 }
 // over the dense candidate keys of the job (the single-sweep step's records; their count lives on the
-// device, state aux[0])
+// device, state aux[0]).  The last workgroup to finish also runs the level's scan.
 template <int LEVEL>
 __global__ __launch_bounds__(kBlock) void k_level_hist_raw(ChainJobs jobs) {
+  __shared__ uint32_t s_h[kBinsBig], s_suf[kBlock + 1], s_last;
   const ChainJob& J = jobs.j[blockIdx.y];
+  SelState* st = J.aux;
+  if (st->skip) return;
+  const int64_t cap = (int64_t)kSegWaves * J.seg_cap;
+  const int64_t n = J.st->cand_count < cap ? J.st->cand_count : cap;
   SrcU32 src{J.cand_key};
-  level_hist_body<SrcU32, LEVEL, 1, true>(src, (int64_t)kSegWaves * J.seg_cap, &J.st->cand_count, J.aux, J.hist);
+  uint32_t* gh = level_hist_of<LEVEL>(J.hist);
+  level_hist_body<SrcU32, LEVEL>(src, n, st->prefix, gh, s_h, blockIdx.x, gridDim.x);
+  if (!level_last(&st->done[LEVEL], gridDim.x, &s_last)) return;
+  level_scan_body<LEVEL>(st, gh, s_suf);
 }
 
 // Stand-alone scan (used when one level's histogram is built by several
@@ -554,19 +539,14 @@ __global__ __launch_bounds__(kBlock) void k_level_scan(ChainJobs jobs) {
 // Per-chunk (1024 elements, one wave) counts of keys above / equal to the
 // threshold.
 template <class Src>
-__global__ __launch_bounds__(kBlock) void k_tile_count(SrcPack<Src> srcs, ChainJobs jobs,
-                                                       int64_t tile_base) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  SelState* __restrict__ st = J.st;
-  if (st->skip) return;
-  Src src = srcs.s[blockIdx.y];
+__device__ __forceinline__ void tile_count_body(Src& src, const ChainJob& J, uint32_t T, int64_t tile_base,
+                                                uint32_t blk, uint32_t n_blk) {
   const int64_t n = J.n;
-  uint32_t* __restrict__ tile_gt = J.tile_gt;
-  uint32_t* __restrict__ tile_eq = J.tile_eq;
-  const uint32_t T = st->thresh_bits;
+  uint32_t* tile_gt = J.tile_gt;
+  uint32_t* tile_eq = J.tile_eq;
   const int64_t n_chunks = cdiv64(n, kChunk);
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  for (int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id(); c < n_chunks;
+  const int64_t wstride = (int64_t)n_blk * kChunksPerBlock;
+  for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks;
        c += wstride) {
     uint32_t cg = 0, ce = 0;
     if (src.vec && (c + 1) * kChunk <= n) {
@@ -595,20 +575,26 @@ __global__ __launch_bounds__(kBlock) void k_tile_count(SrcPack<Src> srcs, ChainJ
     cg = wave_sum(cg);
     ce = wave_sum(ce);
     if (lane_id() == 0) {
-      tile_gt[tile_base + c] = cg;
-      tile_eq[tile_base + c] = ce;
+      st_agent(&tile_gt[tile_base + c], cg);
+      st_agent(&tile_eq[tile_base + c], ce);
     }
   }
-  note_negative(src, st);
+  note_negative(src, J.st);
+}
+template <class Src>
+__global__ __launch_bounds__(kBlock) void k_tile_count(SrcPack<Src> srcs, ChainJobs jobs, int64_t tile_base) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  if (J.st->skip) return;
+  Src src = srcs.s[blockIdx.y];
+  tile_count_body(src, J, J.st->thresh_bits, tile_base, blockIdx.x, gridDim.x);
 }
 
-// Tile scan, kernel 1: per-workgroup totals of (gt, eq).
+// Tile scan of a staged select, kernel 1: per-workgroup totals of (gt, eq).
 static __global__ __launch_bounds__(kBlock) void k_tile_sums(ChainJobs jobs) {
   __shared__ uint32_t s_g[kChunksPerBlock], s_e[kChunksPerBlock];
   const ChainJob& J = jobs.j[blockIdx.y];
   const int64_t n_tiles = J.n_tiles;
   if ((int64_t)blockIdx.x * kTileScanSpan >= n_tiles) return;     // a job with fewer tiles
-  if (J.mask_only && J.st->bracket_ok && !J.st->ties_left) return;
   const uint32_t* __restrict__ tile_gt = J.tile_gt;
   const uint32_t* __restrict__ tile_eq = J.tile_eq;
   uint32_t* __restrict__ blk_gt = J.blk_gt;
@@ -655,7 +641,6 @@ static __global__ __launch_bounds__(kBlock) void k_tile_apply(ChainJobs jobs) {
   const int64_t n_tiles = J.n_tiles;
   const int n_blocks = (int)cdiv64(n_tiles, kTileScanSpan);
   if ((int)blockIdx.x >= n_blocks) return;                        // a job with fewer tiles
-  if (J.mask_only && J.st->bracket_ok && !J.st->ties_left) return;
   uint32_t* __restrict__ tile_gt = J.tile_gt;
   uint32_t* __restrict__ tile_eq = J.tile_eq;
   const uint32_t* __restrict__ blk_gt = J.blk_gt;
@@ -727,8 +712,7 @@ static __global__ __launch_bounds__(kBlock) void k_tile_apply(ChainJobs jobs) {
     }
     sr += scount[j];
   }
-  // (a settlement that placed a mask has stored the number and kept no selected counts)
-  if ((int)blockIdx.x == n_blocks - 1 && threadIdx.x == 0 && !(J.mask_only && st->bracket_ok))
+  if ((int)blockIdx.x == n_blocks - 1 && threadIdx.x == 0)
     st->n_selected = S0 + blk_tot_s;
 }
 
@@ -771,28 +755,18 @@ __device__ __forceinline__ void slab_select(const uint32_t key[4], const bool va
 }
 
 template <class Src>
-__global__ __launch_bounds__(kBlock) void k_write_mask(SrcPack<Src> srcs, ChainJobs jobs,
-                                                       int64_t tile_base, int unless_settled,
-                                                       uint8_t* __restrict__ mask_override) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const SelState* __restrict__ st = J.st;
-  if (unless_settled && st->bracket_ok) return;
-  Src src = srcs.s[blockIdx.y];
-  const int64_t n = J.n;
-  const int tie_all = J.tie_all;
-  const uint32_t* __restrict__ tile_sel = J.tile_gt;
-  const uint32_t* __restrict__ tile_eq = J.tile_eq;
-  uint8_t* __restrict__ mask = mask_override ? mask_override : J.mask;
+__device__ __forceinline__ void write_mask_body(Src& src, const ChainJob& J, uint32_t T, uint32_t need,
+                                                int64_t tile_base, uint8_t* __restrict__ mask, uint32_t blk,
+                                                uint32_t n_blk) {
   const bool mvec = aligned4(mask, 1);
-  const uint32_t T = st->thresh_bits;
-  const uint32_t need = tie_all ? 0xFFFFFFFFu : st->need;
+  const int64_t n = J.n;
   const int64_t n_chunks = cdiv64(n, kChunk);
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  for (int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id(); c < n_chunks;
+  const int64_t wstride = (int64_t)n_blk * kChunksPerBlock;
+  for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks;
        c += wstride) {
     ChunkCursor cur;
-    cur.sel_run = tile_sel[tile_base + c];
-    cur.eq_run = tile_eq[tile_base + c];
+    cur.sel_run = (uint32_t)uniform_i32((int)ld_agent(&J.tile_gt[tile_base + c]));
+    cur.eq_run = (uint32_t)uniform_i32((int)ld_agent(&J.tile_eq[tile_base + c]));
     const bool full = src.vec && mvec && (c + 1) * kChunk <= n;
     uint32_t key[kChunkIters][4];
 #pragma unroll
@@ -818,19 +792,28 @@ __global__ __launch_bounds__(kBlock) void k_write_mask(SrcPack<Src> srcs, ChainJ
   }
 }
 
-static __global__ void k_sel_result(ChainJobs jobs) {
-  const SelState* st = jobs.j[blockIdx.y].st;
-  sga_select_result* out = jobs.j[blockIdx.y].result;
-  if (!out) return;
-  out->thresh_bits = st->thresh_bits;
-  out->need = st->need;
-  out->n_gt = st->n_gt;
-  out->n_eq = st->n_eq;
-  out->n_selected = st->n_selected;
-  out->nonfinite = st->nonfinite;
-  out->status = st->status;
-  out->path = st->path | (st->negative ? 0x100u : 0u) | (st->redone ? 0x200u : 0u);
+template <class Src>
+__global__ __launch_bounds__(kBlock) void k_write_mask(SrcPack<Src> srcs, ChainJobs jobs, int64_t tile_base) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  Src src = srcs.s[blockIdx.y];
+  write_mask_body(src, J, J.st->thresh_bits, J.tie_all ? 0xFFFFFFFFu : J.st->need, tile_base, J.mask, blockIdx.x,
+                  gridDim.x);
 }
+
+__device__ __forceinline__ void write_result(const ChainJob& J) {
+  const SelState* st = J.st;
+  sga_select_result* out = J.result;
+  if (!out) return;
+  out->thresh_bits = ld_agent(&st->thresh_bits);
+  out->need = ld_agent(&st->need);
+  out->n_gt = ld_agent(&st->n_gt);
+  out->n_eq = ld_agent(&st->n_eq);
+  out->n_selected = ld_agent(&st->n_selected);
+  out->nonfinite = ld_agent(&st->nonfinite);
+  out->status = ld_agent(&st->status);
+  out->path = st->path | (ld_agent(&st->negative) ? 0x100u : 0u) | (st->redone ? 0x200u : 0u);
+}
+static __global__ void k_sel_result(ChainJobs jobs) { write_result(jobs.j[blockIdx.y]); }
 
 // -------------------------------------------------------------- host drivers
 // Grid of the histogram passes over raw key buffers (<= 1M sample keys, ~1e6 candidates whose
@@ -876,14 +859,14 @@ struct SelBatch {
   dim3 grid(unsigned gx) const { return dim3(gx, (unsigned)count); }
 };
 
-// hist (+ merged scan) of one radix level over the data, for every job of the batch
-template <class Src, bool MERGE>
+// histogram of one radix level over the data, for every job of the batch (staged selects)
+template <class Src>
 static inline void launch_level_data(const SrcPack<Src>& srcs, const SelBatch& B, int level,
                                      hipStream_t s) {
   const dim3 grid = B.grid(hist_grid(B.max_n).x), block(kBlock);
-  if (level == 0) hipLaunchKernelGGL((k_level_hist<Src, 0, MERGE>), grid, block, 0, s, srcs, B.jobs);
-  else if (level == 1) hipLaunchKernelGGL((k_level_hist<Src, 1, MERGE>), grid, block, 0, s, srcs, B.jobs);
-  else hipLaunchKernelGGL((k_level_hist<Src, 2, MERGE>), grid, block, 0, s, srcs, B.jobs);
+  if (level == 0) hipLaunchKernelGGL((k_level_hist<Src, 0>), grid, block, 0, s, srcs, B.jobs);
+  else if (level == 1) hipLaunchKernelGGL((k_level_hist<Src, 1>), grid, block, 0, s, srcs, B.jobs);
+  else hipLaunchKernelGGL((k_level_hist<Src, 2>), grid, block, 0, s, srcs, B.jobs);
 }
 // the same over the jobs' dense candidate keys
 static inline void launch_level_raw(const SelBatch& B, int level, hipStream_t s, unsigned blocks) {
@@ -1435,7 +1418,7 @@ __global__ __launch_bounds__(kBlock) void k_bracket_sweep(
 //   3. The last workgroup to finish ranks the edge list (threshold, ties, which of them are granted:
 //      lowest index first) and corrects the counts.  An edge list of one key value needs no ranking
 //      whatever its length (gradients on the bf16 grid: a hundred thousand equal keys); the ties of
-//      one too long for LDS are placed by k_settle_ties, behind the chunk scan.
+//      one too long for LDS are placed by k_tail, behind the chunk scan.
 // What step 3 reads of the others' is written by device-scope atomics and atomic stores, each wave
 // waits for its own (vmcnt) before the workgroup takes its ticket, and the last one reads with atomic
 // loads: no cache-wide fence, which costs 65 ns a workgroup here.
@@ -1697,13 +1680,11 @@ static __global__ __launch_bounds__(kWide) void k_settle(ChainJobs jobs) {
 // Ties of an edge list that did not fit the last workgroup's LDS, in index order: the chunk scan has
 // left the ties before every chunk in tile_eq, so only the one chunk where the quota runs out has to
 // rank its ties (a chunk's candidates are contiguous and index-ordered in its segment).
-static __global__ __launch_bounds__(kBlock) void k_settle_ties(ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const SelState* __restrict__ st = J.st;
-  if (!st->ties_left) return;
+__device__ __forceinline__ void settle_ties_body(const ChainJob& J, uint32_t blk, uint32_t n_blk) {
+  const SelState* st = J.st;
   const uint32_t T = st->thresh_bits, n_eq = st->n_eq;
   const uint32_t need = J.tie_all ? 0xFFFFFFFFu : st->need;
-  walk_segments(J, (int)blockIdx.x * kChunksPerBlock + wave_id(), (int)gridDim.x * kChunksPerBlock,
+  walk_segments(J, (int)blk * kChunksPerBlock + wave_id(), (int)n_blk * kChunksPerBlock,
                 [&](bool valid, uint32_t key, uint32_t idx, uint32_t pos) {
     if (!valid || key != T) return;
     bool on = true;
@@ -1896,24 +1877,16 @@ static __global__ __launch_bounds__(kBlock) void k_expand_mask(
 // Ordered full pass that writes the mask as bit planes: where no bracket was settled (k_settle), or
 // none was tried.
 template <class Src>
-__global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const SelState* __restrict__ st = J.st;
-  if (st->bracket_ok) return;
-  Src src = srcs.s[blockIdx.y];
+__device__ __forceinline__ void write_bits_body(Src& src, const ChainJob& J, uint32_t T, uint32_t need, uint32_t blk,
+                                                uint32_t n_blk) {
   const int64_t n = J.n;
-  const int tie_all = J.tie_all;
-  const uint32_t* __restrict__ tile_sel = J.tile_gt;
-  const uint32_t* __restrict__ tile_eq = J.tile_eq;
   uint32_t* __restrict__ planes = J.planes;
-  const uint32_t T = st->thresh_bits;
-  const uint32_t need = tie_all ? 0xFFFFFFFFu : st->need;
   const int64_t n_chunks = cdiv64(n, kChunk);
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  for (int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id(); c < n_chunks; c += wstride) {
+  const int64_t wstride = (int64_t)n_blk * kChunksPerBlock;
+  for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks; c += wstride) {
     ChunkCursor cur;
-    cur.sel_run = tile_sel[c];
-    cur.eq_run = tile_eq[c];
+    cur.sel_run = (uint32_t)uniform_i32((int)ld_agent(&J.tile_gt[c]));
+    cur.eq_run = (uint32_t)uniform_i32((int)ld_agent(&J.tile_eq[c]));
     const bool full = src.vec && (c + 1) * kChunk <= n;
     uint32_t word = 0u;
 #pragma unroll
@@ -1931,6 +1904,151 @@ __global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJ
       plane_collect(flag, it, word);
     }
     if (lane_id() < 32) planes[c * kPlaneWordsPerChunk + lane_id()] = word;
+  }
+}
+template <class Src>
+__global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJobs jobs) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  Src src = srcs.s[blockIdx.y];
+  write_bits_body(src, J, J.st->thresh_bits, J.tie_all ? 0xFFFFFFFFu : J.st->need, blockIdx.x, gridDim.x);
+}
+
+// All that can be left to do behind a settlement, in one launch: the radix passes over the data and the
+// chunk counts (a bracket that failed or was never tried), the chunk scan (callers that pack, plateaus),
+// the ties of an edge list too long for LDS, the ordered pass that writes the mask or the planes (OUT:
+// 1 planes, 2 mask bytes, 0 the caller forms the keys again), the result.  Usually that is the chunk scan
+// or nothing at all, and what a select paid for was nine launches that returned at once, 4.7 us each.
+// With them -> in one launch: step of 40 M coordinates 450 -> 424 us, select of 1e9 1097 -> 1034, eight
+// buckets of 596 M 4584 -> 4407; the radix passes themselves (sorted scores) 711 -> 324 at 20 M, 994 -> 668
+// at 63 M.
+//
+// The steps are items of one queue: a workgroup takes the next item by its ticket, waits until every
+// item of the steps before is finished, and does it.  Whoever waits holds a later ticket than those it
+// waits for, which running workgroups hold, so the queue drains with any number of workgroups resident.
+// The items of the scan wait for one another's totals the same way (in ticket order), through 64-bit
+// words that carry the totals themselves.  Nearly all else that crosses workgroups goes by device-scope
+// atomics, waited for before an item counts as finished: a cache-wide fence on both sides of 1024 items,
+// with all waiting workgroups looking at the counter that they add to, took 240 ns an item.  The waiting
+// ones look at a word of its own, away from that counter.
+constexpr int kTailBlocks = 512;
+constexpr int kTailStep = kHistStride + 2 * kMaxTileBlocks + 256;    // that word, in the second histogram set
+struct TailLds {
+  uint32_t h[kBinsBig];
+  uint32_t suf[kBlock + 1], w4[kChunksPerBlock], last, ticket;
+};
+__device__ __forceinline__ void tail_scan(const ChainJob& J, uint32_t b, uint32_t n_blk, TailLds& s) {
+  const int64_t n_tiles = J.n_tiles;
+  unsigned long long* words = reinterpret_cast<unsigned long long*>(J.hist + kHistStride);
+  static_assert(kTailStep < 2 * kHistStride && kHistStride % 2 == 0, "a word per workgroup of the scan");
+  static_assert((int64_t)kTileScanSpan * kChunk < (1 << 23), "two totals and a flag in 64 bits");
+  const int64_t base = (int64_t)b * kTileScanSpan + (int64_t)threadIdx.x * kTileScanPer;
+  uint32_t g[kTileScanPer], e[kTileScanPer], my_g = 0, my_e = 0;
+#pragma unroll
+  for (int j = 0; j < kTileScanPer; ++j) {
+    const bool ok = base + j < n_tiles;
+    g[j] = ok ? J.tile_gt[base + j] : 0u;
+    e[j] = ok ? J.tile_eq[base + j] : 0u;
+    my_g += g[j];
+    my_e += e[j];
+  }
+  uint32_t tot_g, tot_e;
+  uint32_t gr = block_excl_scan(my_g, s.w4, tot_g);
+  uint32_t er = block_excl_scan(my_e, s.w4, tot_e);
+  if (threadIdx.x == 0)
+    __hip_atomic_store(&words[b], (1ull << 63) | ((unsigned long long)tot_g << 32) | tot_e, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  uint32_t pg = 0, pe = 0;
+  for (uint32_t j = threadIdx.x; j < b; j += kBlock) {
+    unsigned long long w;
+    while ((w = __hip_atomic_load(&words[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0ull)
+      __builtin_amdgcn_s_sleep(1);
+    pg += (uint32_t)(w >> 32) & 0x7FFFFFFFu;
+    pe += (uint32_t)w;
+  }
+  uint32_t G0, E0;
+  block_excl_scan(pg, s.w4, G0);
+  block_excl_scan(pe, s.w4, E0);
+  gr += G0;
+  er += E0;
+  // ties are granted in index order until `need` is used up: min(need, ties before) of them lie before a chunk
+  const uint32_t need = J.tie_all ? 0xFFFFFFFFu : ld_agent(&J.st->need);
+#pragma unroll
+  for (int j = 0; j < kTileScanPer; ++j) {
+    if (base + j < n_tiles) {
+      J.tile_gt[base + j] = gr + (er < need ? er : need);
+      J.tile_eq[base + j] = er;
+    }
+    gr += g[j];
+    er += e[j];
+  }
+  // (a settlement that placed a mask has stored the number and kept no selected counts)
+  if (b == n_blk - 1 && threadIdx.x == 0 && !(J.mask_only && J.st->bracket_ok)) {
+    const uint32_t E = E0 + tot_e;
+    st_agent(&J.st->n_selected, G0 + tot_g + (E < need ? E : need));
+  }
+}
+template <class Src, int LEVEL>
+__device__ __forceinline__ void tail_level(Src& src, const ChainJob& J, uint32_t blk, uint32_t n_blk, TailLds& s) {
+  uint32_t* gh = level_hist_of<LEVEL>(J.hist);
+  level_hist_body<Src, LEVEL>(src, J.n, LEVEL == 0 ? 0u : ld_agent(&J.st->prefix), gh, s.h, blk, n_blk);
+  if (!level_last(&J.st->done[LEVEL], n_blk, &s.last)) return;
+  level_scan_body<LEVEL>(J.st, gh, s.suf);
+  __threadfence();
+}
+template <class Src, int OUT>
+__global__ __launch_bounds__(kBlock) void k_tail(SrcPack<Src> srcs, ChainJobs jobs) {
+  __shared__ TailLds s;
+  const ChainJob& J = jobs.j[blockIdx.y];
+  SelState* st = J.st;
+  // none of these changes while the queue is worked off
+  const bool armed = st->skip == 0, ties = st->ties_left != 0, write = OUT != 0 && !st->bracket_ok;
+  const uint32_t G = gridDim.x;
+  const uint32_t n_pass = armed ? G : 0u, n_ties = ties ? (G < 256u ? G : 256u) : 0u, n_write = write ? G : 0u;
+  const uint32_t n_scan = J.mask_only && st->bracket_ok && !ties ? 0u : (uint32_t)cdiv64(J.n_tiles, kTileScanSpan);
+  const uint32_t at_scan = 4u * n_pass, at_ties = at_scan + n_scan, at_write = at_ties + n_ties;
+  const uint32_t total = at_write + n_write;
+  if (total == 0) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) write_result(J);
+    return;
+  }
+  if (!armed && !write && !ties && blockIdx.x >= n_scan) return;      // a workgroup per item is enough
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) s.ticket = atomicAdd(&st->tail_ticket, 1u);
+    __syncthreads();
+    const uint32_t t = s.ticket;
+    if (t >= total) return;
+    const uint32_t first = t >= at_ties ? at_ties : t >= at_scan ? at_scan : t / G * G;
+    if (first) {
+      if (threadIdx.x == 0)
+        while (ld_agent(&J.hist[kTailStep]) < first) __builtin_amdgcn_s_sleep(16);
+      __syncthreads();
+      if (t >= at_scan && t < at_write) __threadfence();              // chunk counters and prefixes, read as they lie
+    }
+    Src src = srcs.s[blockIdx.y];
+    if (t < at_scan) {
+      const uint32_t step = t / G, blk = t - first;
+      if (step == 0) tail_level<Src, 0>(src, J, blk, G, s);
+      else if (step == 1) tail_level<Src, 1>(src, J, blk, G, s);
+      else if (step == 2) tail_level<Src, 2>(src, J, blk, G, s);
+      else tile_count_body(src, J, ld_agent(&st->thresh_bits), 0, blk, G);
+    } else if (t < at_ties) {
+      tail_scan(J, t - first, n_scan, s);
+    } else if (t < at_write) {
+      settle_ties_body(J, t - first, n_ties);
+    } else if (OUT != 0) {
+      const uint32_t T = ld_agent(&st->thresh_bits), need = J.tie_all ? 0xFFFFFFFFu : ld_agent(&st->need);
+      if (OUT == 1) write_bits_body(src, J, T, need, t - first, n_write);
+      else write_mask_body(src, J, T, need, 0, J.mask, t - first, n_write);
+    }
+    if (t >= at_ties) continue;                                       // nothing in this launch reads what these wrote
+    if (t >= at_scan && at_ties != total) __threadfence();            // the prefixes are read below
+    wait_landed();
+    if (threadIdx.x == 0) {
+      const uint32_t done = atomicAdd(&st->tail_done, 1u) + 1u;
+      if (done == at_ties) write_result(J);                           // settled with the scan's last item
+      if (done == at_ties || (done <= at_scan && done % G == 0)) st_agent(&J.hist[kTailStep], done);
+    }
   }
 }
 
@@ -1955,19 +2073,18 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 }
 
 // The select of every job of a batch: begin -> (sampled-bracket path: coarse sample and pick, fine sample
-// and pick, ONE data sweep per job, settlement) -> the radix passes (no-ops unless a job's bracket
-// failed) -> chunk scan.  The short kernels run once for the whole batch; only the data sweeps are
-// launched per job.
+// and pick, ONE data sweep per job, settlement) -> k_tail.  The short kernels run once for the whole
+// batch; only the data sweeps are launched per job.
 // PM: what the sweep leaves behind for a mask-only caller -- 0 nothing, 1 the keys above the
 // bracket as bit planes (job.planes), 2 as mask bytes (job.mask) -- where the settlement adds the
-// candidates; a writing pass over the data (finish_planes / finish_mask) is then a no-op.
+// candidates; the tail's writing pass over the data then has nothing to do.
 // All jobs of a batch take the same path (`fast`: SelBatch::fast_ok for every one of them).
 //
 // The chain comes in phases so that a batch whose jobs form their keys differently (the
 // re-selections of a replay step rank by different scores) still shares every kernel that does
-// not form keys: chain_begin, chain_pick_*, chain_settle and launch_tile_scan take the whole batch;
-// chain_sample_*, chain_sweeps and chain_fallback are templates of the key source and take the jobs of
-// one kind (a sub-batch over the same workspaces).
+// not form keys: chain_begin, chain_pick_* and chain_settle take the whole batch; chain_sample_*,
+// chain_sweeps and chain_tail are templates of the key source and take the jobs of one kind (a sub-batch
+// over the same workspaces).
 static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, bool fast, hipStream_t s) {
   static_assert(sizeof(ChainJobs) + sizeof(SegDirJobs) + 64 <= 4096, "operands travel in the kernel arguments");
   hipLaunchKernelGGL(k_chain_begin, B.grid(fast ? 32 : 4), dim3(kBlock), 0, s, B.jobs, dirs, fast ? 1 : 0);
@@ -2035,19 +2152,14 @@ static inline void chain_settle(const SelBatch& B, hipStream_t s) {
   const unsigned wgs = (unsigned)(want < least ? least : want > 256 ? 256 : want);
   hipLaunchKernelGGL(k_settle, B.grid(wgs), dim3(kWide), 0, s, B.jobs);
 }
-// behind the chunk scan, for callers whose mask or planes the settlement fills
-static inline void chain_settle_ties(const SelBatch& B, hipStream_t s) {
-  hipLaunchKernelGGL(k_settle_ties, B.grid(256), dim3(kBlock), 0, s, B.jobs);
-}
-// The radix passes and the per-chunk counts over the data: no-ops unless a job's bracket failed
-// (st->skip == 0) or was never tried.
-template <class Src>
-static inline void chain_fallback(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
-  for (int level = 0; level < 3; ++level) launch_level_data<Src, true>(srcs, B, level, s);
-  launch_tile_count(srcs, B, 0, s);
+// OUT: what the ordered pass over the data writes where no bracket settled it (k_tail)
+template <int OUT, class Src>
+static inline void chain_tail(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
+  const unsigned wgs = stream_grid(B.max_n, kTileScanSpan, kTailBlocks);
+  hipLaunchKernelGGL((k_tail<Src, OUT>), B.grid(wgs), dim3(kBlock), 0, s, srcs, B.jobs);
 }
 
-template <class Src>
+template <int OUT, class Src>
 static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, bool fast,
                                     int pm, hipStream_t s) {
   if (fast) {
@@ -2057,18 +2169,7 @@ static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B,
   } else {
     chain_begin(B, dirs, false, s);
   }
-  chain_fallback(srcs, B, s);
-  launch_tile_scan(B, s);
-  if (fast && pm != 0) chain_settle_ties(B, s);
-}
-
-// Byte masks after run_select_batch(..., pm = 2): the sweep and the settlement wrote them when the bracket
-// held, else the ordered full pass does.
-template <class Src>
-static inline void finish_mask_batch(const SrcPack<Src>& srcs, const SelBatch& B, bool fast,
-                                     hipStream_t s) {
-  hipLaunchKernelGGL((k_write_mask<Src>), B.grid(stream_grid(B.max_tiles, kChunksPerBlock, 1 << 14)),
-                     dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0, fast ? 1 : 0, (uint8_t*)nullptr);
+  chain_tail<OUT>(srcs, B, s);
 }
 
 #endif  // __HIPCC__

@@ -75,6 +75,18 @@ def test_settlement_of_large_buckets(dev, n, name):
         _check(dev, sc, kk, (name, n, kk))
 
 
+# the candidates of sorted scores lie side by side and overrun their segments: the radix passes, the chunk
+# scan and the ordered mask pass all run, as items of one queue
+@pytest.mark.parametrize("n", [LIMIT + 1, 12_345_679, 16_777_216])
+@pytest.mark.parametrize("grid", [False, True])
+def test_radix_passes_of_large_buckets(dev, n, grid):
+    sc = torch.rand(n, generator=torch.Generator().manual_seed(n % 89)).sort()[0]
+    if grid:                                        # runs of equal keys across chunk boundaries
+        sc = (sc * 3000.0).floor()
+    for k in (n // 100, n // 3):
+        _check(dev, sc, k, (grid, n, k), path=None if grid else 0)
+
+
 def _mix32(x):
     x = x.astype(np.uint32)
     x ^= x >> np.uint32(16)
