@@ -15,7 +15,7 @@ namespace sga {
 
 // One 4-element vector of the masked / full-step commit.
 // EMIT: -1 sparse step; 0 update, 1 |g|, 2 |m|, 3 coi -> written into g.
-// FULL: the whole workgroup span is in range and every array vector-aligned,
+// FULL: the whole workgroup span is in range and every array element-aligned,
 // so all loads are unconditional and in flight together.
 template <int EMIT, bool FULL>
 __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict__ g,
@@ -110,8 +110,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct_multi(const GcRecord* _
   Hyper h;
   h.lr = r.lr; h.b1 = r.b1; h.om1 = r.om1; h.b2 = r.b2; h.om2 = r.om2; h.eps = r.eps;
   h.wd = r.wd; h.bc1 = r.bc1; h.bc2 = r.bc2;
-  const bool vec = aligned4(r.p, 4) && aligned4(r.g, 4) && aligned4(r.m, 4) && aligned4(r.v, 4) &&
-                   aligned4(r.mask, 1);
+  const bool vec = quads_ok(r.p, 4) && quads_ok(r.g, 4) && quads_ok(r.m, 4) && quads_ok(r.v, 4) &&
+                   quads_ok(r.mask, 1);
   const int64_t base = (span - r.first_span) * kBlockSpan;
   const bool full = vec && base + kBlockSpan <= r.n;
 #pragma unroll
@@ -299,7 +299,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct_compact_multi(
   Hyper h;
   h.lr = r.lr; h.b1 = r.b1; h.om1 = r.om1; h.b2 = r.b2; h.om2 = r.om2; h.eps = r.eps;
   h.wd = r.wd; h.bc1 = r.bc1; h.bc2 = r.bc2;
-  const bool vec = aligned4(r.p, 4) && aligned4(r.g, 4) && aligned4(r.m, 4) && aligned4(r.v, 4);
+  const bool vec = quads_ok(r.p, 4) && quads_ok(r.g, 4) && quads_ok(r.m, 4) && quads_ok(r.v, 4);
   compact_span<BF16>(r.p, r.g, r.m, r.v, r.idx, r.values, r.rec_start, r.n, r.k_total, h, coeff,
                      interval, r.flags, r.table, r.n_table, vec, span - r.first_span, s_val,
                      s_found, s_bounds);
@@ -352,8 +352,8 @@ extern "C" int sga_adamw_grad_correct(float* p, float* g, float* m, float* v,
   }
   if (flags & SGA_GC_ADAMS) { bc1 = 1.0f; bc2 = 1.0f; }
   const Hyper h = mk_hyper(lr, beta1, om1, beta2, om2, eps, wd, bc1, bc2);
-  const bool vec = aligned4(p, 4) && aligned4(g, 4) && aligned4(m, 4) &&
-                   aligned4(v, 4) && aligned4(mask, 1);
+  const bool vec = quads_ok(p, 4) && quads_ok(g, 4) && quads_ok(m, 4) &&
+                   quads_ok(v, 4) && quads_ok(mask, 1);
   dim3 grid(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
 #define SGA_GC_LAUNCH(E)                                                       \
@@ -424,7 +424,7 @@ extern "C" int sga_adamw_grad_correct_compact(
   }
   if (flags & SGA_GC_ADAMS) { bc1 = 1.0f; bc2 = 1.0f; }
   const Hyper h = mk_hyper(lr, beta1, om1, beta2, om2, eps, wd, bc1, bc2);
-  const bool vec = aligned4(p, 4) && aligned4(g, 4) && aligned4(m, 4) && aligned4(v, 4);
+  const bool vec = quads_ok(p, 4) && quads_ok(g, 4) && quads_ok(m, 4) && quads_ok(v, 4);
   dim3 grid(stream_grid(n, kBlockSpan, 1 << 22)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
   if (values_dtype == SGA_BF16)

@@ -76,6 +76,12 @@ __host__ __device__ static inline bool aligned4(const void* p, int elem) {
   return p == nullptr || (reinterpret_cast<uintptr_t>(p) % (4 * (size_t)elem)) == 0;
 }
 
+// True when the elements at p lie on multiples of their size: quads of them then go as one access each
+// (ld4 and the like take quads at any element's address).
+__host__ __device__ static inline bool quads_ok(const void* p, int elem) {
+  return p == nullptr || (reinterpret_cast<uintptr_t>(p) % (size_t)elem) == 0;
+}
+
 #ifdef __HIPCC__
 
 __device__ __forceinline__ uint32_t f2u(float x) { return __float_as_uint(x); }
@@ -173,19 +179,34 @@ struct alignas(8) H4 { uint16_t x, y, z, w; };
 struct alignas(16) U4 { uint32_t x, y, z, w; };
 struct alignas(4) B4 { uint8_t x, y, z, w; };
 
-typedef float f4v __attribute__((ext_vector_type(4)));
+// Quads in global memory: one 64/128-bit (32-bit for bytes) access at any address an element may have.
+// gfx950 takes them unaligned under HSA and the types say so.  Views of a flat buffer begin wherever a
+// tensor does, and with four accesses per quad such a view cost up to 1.7 times an aligned one.  Eight
+// buckets behind an embedding of odd length, 200 M coordinates: 2820 -> 1910 us bf16, 2672 -> 2029 fp32
+// (aligned 1630, 1740: what is left is the lines that two waves share); plugin steps on 63 M coordinates
+// full 1103 -> 932, index layout 565 -> 444, mask layout 718 -> 605.
+typedef float f4v __attribute__((ext_vector_type(4), aligned(4)));
+typedef unsigned char b4v __attribute__((ext_vector_type(4), aligned(1)));
 __device__ __forceinline__ F4 ld4(const float* p) {
-  return *reinterpret_cast<const F4*>(p);
+  const f4v t = *reinterpret_cast<const f4v*>(p);
+  return F4{t.x, t.y, t.z, t.w};
 }
 __device__ __forceinline__ void st4(float* p, const F4& v) {
-  *reinterpret_cast<F4*>(p) = v;
+  *reinterpret_cast<f4v*>(p) = f4v{v.x, v.y, v.z, v.w};
+}
+__device__ __forceinline__ B4 ldb4(const uint8_t* p) {
+  const b4v t = *reinterpret_cast<const b4v*>(p);
+  return B4{t.x, t.y, t.z, t.w};
+}
+__device__ __forceinline__ void stb4(uint8_t* p, const B4& v) {
+  *reinterpret_cast<b4v*>(p) = b4v{v.x, v.y, v.z, v.w};
 }
 // Streaming (non-temporal) 128-bit accesses for data touched once per sweep.
 __device__ __forceinline__ F4 ld4_nt(const float* p) {
   const f4v t = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(p));
   return F4{t.x, t.y, t.z, t.w};
 }
-typedef unsigned short h4v __attribute__((ext_vector_type(4)));
+typedef unsigned short h4v __attribute__((ext_vector_type(4), aligned(2)));
 __device__ __forceinline__ H4 ldh4_nt(const uint16_t* p) {
   const h4v t = __builtin_nontemporal_load(reinterpret_cast<const h4v*>(p));
   return H4{t.x, t.y, t.z, t.w};
@@ -195,8 +216,8 @@ __device__ __forceinline__ void st4_nt(float* p, const F4& v) {
   __builtin_nontemporal_store(t, reinterpret_cast<f4v*>(p));
 }
 
-// Load 4 consecutive elements starting at i (i % 4 == 0 relative to a
-// 16-byte aligned base) with a scalar tail when fewer than 4 remain.
+// Load 4 consecutive elements starting at i with a scalar tail when fewer
+// than 4 remain.
 __device__ __forceinline__ void load4_f32(const float* base, int64_t i,
                                           int64_t n, float out[4],
                                           bool vec = true) {
@@ -212,7 +233,7 @@ __device__ __forceinline__ void load4_bf16(const uint16_t* base, int64_t i,
                                            int64_t n, float out[4],
                                            bool vec = true) {
   if (vec && i + 4 <= n) {
-    H4 v = *reinterpret_cast<const H4*>(base + i);
+    const h4v v = *reinterpret_cast<const h4v*>(base + i);
     out[0] = bf16_to_f32(v.x); out[1] = bf16_to_f32(v.y);
     out[2] = bf16_to_f32(v.z); out[3] = bf16_to_f32(v.w);
   } else {
@@ -225,7 +246,7 @@ __device__ __forceinline__ void load4_u8(const uint8_t* base, int64_t i,
                                          int64_t n, uint32_t out[4],
                                          bool vec = true) {
   if (vec && i + 4 <= n) {
-    B4 v = *reinterpret_cast<const B4*>(base + i);
+    const B4 v = ldb4(base + i);
     out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
   } else {
 #pragma unroll
@@ -247,7 +268,7 @@ __device__ __forceinline__ void store4_u8(uint8_t* base, int64_t i, int64_t n,
                                           const uint32_t v[4], bool vec = true) {
   if (vec && i + 4 <= n) {
     B4 t{(uint8_t)v[0], (uint8_t)v[1], (uint8_t)v[2], (uint8_t)v[3]};
-    *reinterpret_cast<B4*>(base + i) = t;
+    stb4(base + i, t);
   } else {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -256,7 +277,7 @@ __device__ __forceinline__ void store4_u8(uint8_t* base, int64_t i, int64_t n,
 }
 
 // FULL variants: when the caller has established (wave-uniformly) that the
-// whole span is in range and vector-aligned, the access is a single
+// whole span is in range and element-aligned, the access is a single
 // unconditional 64/128-bit instruction -- no per-lane branch, so the compiler
 // can keep many loads in flight before the first wait.
 template <bool FULL>
@@ -316,7 +337,7 @@ __device__ __forceinline__ void unpack_g(const RawG& r, float out[4]) {
 template <bool FULL>
 __device__ __forceinline__ void ld_u8(const uint8_t* base, int64_t i, int64_t n, uint32_t out[4], bool vec) {
   if (FULL) {
-    const B4 v = *reinterpret_cast<const B4*>(base + i);
+    const B4 v = ldb4(base + i);
     out[0] = v.x; out[1] = v.y; out[2] = v.z; out[3] = v.w;
   } else {
     load4_u8(base, i, n, out, vec);
@@ -335,7 +356,7 @@ template <bool FULL>
 __device__ __forceinline__ void st_u8(uint8_t* base, int64_t i, int64_t n, const uint32_t v[4], bool vec) {
   if (FULL) {
     B4 t{(uint8_t)v[0], (uint8_t)v[1], (uint8_t)v[2], (uint8_t)v[3]};
-    *reinterpret_cast<B4*>(base + i) = t;
+    stb4(base + i, t);
   } else {
     store4_u8(base, i, n, v, vec);
   }

@@ -108,7 +108,7 @@ __device__ __forceinline__ SpanWork span_work(const sga_span_record* __restrict_
   SpanWork w;
   w.g = r.g; w.mask = r.mask; w.n = r.n;
   w.base = (span - r.first_span) * kBlockSpan;
-  w.vec = aligned4(r.g, 4) && aligned4(r.mask, 1);
+  w.vec = quads_ok(r.g, 4) && quads_ok(r.mask, 1);
   w.full = w.vec && w.base + kBlockSpan <= r.n;
   return w;
 }
@@ -460,7 +460,7 @@ extern "C" int sga_compact_norm_sq(const float* values, int64_t k,
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL((k_norm_stage1<false>), dim3(nb), dim3(kBlock), 0, st,
                      values, (const uint8_t*)nullptr, k, partials,
-                     aligned4(values, 4));
+                     quads_ok(values, 4));
   hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials,
                      (int64_t)nb, total);
   return check_launch("sga_compact_norm_sq");
@@ -520,7 +520,7 @@ extern "C" int sga_compact_norm_sq_noalloc(const float* values, int64_t k, float
   const unsigned nb = (unsigned)sga_norm_partials(k);
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL((k_norm_stage1<false>), dim3(nb), dim3(kBlock), 0, st, values,
-                     (const uint8_t*)nullptr, k, partials, aligned4(values, 4));
+                     (const uint8_t*)nullptr, k, partials, quads_ok(values, 4));
   hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials, (int64_t)nb, total);
   return check_launch("sga_compact_norm_sq_noalloc");
 }
@@ -536,7 +536,7 @@ extern "C" int sga_masked_norm_sq(const float* grad, const uint8_t* mask,
   const unsigned nb = (unsigned)sga_norm_partials(n);
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL((k_norm_stage1<true>), dim3(nb), dim3(kBlock), 0, st, grad,
-                     mask, n, partials, aligned4(grad, 4) && aligned4(mask, 1));
+                     mask, n, partials, quads_ok(grad, 4) && quads_ok(mask, 1));
   hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials,
                      (int64_t)nb, total);
   return check_launch("sga_masked_norm_sq");
@@ -568,7 +568,7 @@ extern "C" int sga_scale_masked(float* grad, const uint8_t* mask, int64_t n, flo
   if (n == 0) return SGA_OK;
   if (!grad || n < 0) { set_error("sga_scale_masked: bad argument"); return SGA_ERR_ARG; }
   dim3 grid(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), block(kBlock);
-  const bool vec = aligned4(grad, 4) && aligned4(mask, 1);
+  const bool vec = quads_ok(grad, 4) && quads_ok(mask, 1);
   if (mask)
     hipLaunchKernelGGL((k_scale_masked<true>), grid, block, 0, (hipStream_t)stream, grad, mask, n, coeff, vec);
   else
@@ -666,7 +666,7 @@ extern "C" int sga_mask_count(const uint8_t* mask, int64_t n,
   if (nc > 0)
     hipLaunchKernelGGL(k_mask_count, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)),
                        dim3(kBlock), 0, st, mask, n, chunk_counts, nc,
-                       aligned4(mask, 1));
+                       quads_ok(mask, 1));
   int rc = exclusive_scan_u32(chunk_counts, nc, total, st);
   if (rc) return rc;
   return check_launch("sga_mask_count");
@@ -685,6 +685,6 @@ extern "C" int sga_mask_fill(const uint8_t* mask, int64_t n,
   hipLaunchKernelGGL(k_mask_fill, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)),
                      dim3(kBlock), 0, (hipStream_t)stream, mask, n,
                      chunk_offsets, idx_out, idx_capacity, nc,
-                     aligned4(mask, 1));
+                     quads_ok(mask, 1));
   return check_launch("sga_mask_fill");
 }

@@ -151,7 +151,7 @@ struct FinalArgs {
 };
 
 // One 1024-element chunk of the final sweep, owned by one wave.  FULL: the
-// chunk is entirely in range and every array is vector-aligned, so all 20
+// chunk is entirely in range and every array is element-aligned, so all 20
 // loads are unconditional and issued before the first use.
 // IT0 / NIT: the slabs [IT0, IT0+NIT) of the chunk are handled by this call;
 // `cur` carries the running selected / tie counts across calls.
@@ -424,9 +424,9 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   const bool planes = Src::kHyper && use_fast;
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
-    vec[b] = aligned4(f.g, BF16G ? 2 : 4) && aligned4(f.resid, 4) && aligned4(f.p, 4) &&
-             aligned4(f.m, 4) && aligned4(f.v, 4) && aligned4(f.out[0], 4) &&
-             aligned4(f.out[1], 4) && aligned4(f.out[2], 4) && aligned4(f.out[3], 4);
+    vec[b] = quads_ok(f.g, BF16G ? 2 : 4) && quads_ok(f.resid, 4) && quads_ok(f.p, 4) &&
+             quads_ok(f.m, 4) && quads_ok(f.v, 4) && quads_ok(f.out[0], 4) &&
+             quads_ok(f.out[1], 4) && quads_ok(f.out[2], 4) && quads_ok(f.out[3], 4);
     srcs.s[b] = Src{f.g, f.resid, f.p, f.m, f.v, vec[b], {}, pack_extra, adams};
     srcs.s[b].sc.init(f.segs, f.n_segs, f.w.seg_dir);
     dj.j[b].segs = f.segs; dj.j[b].dir = f.w.seg_dir; dj.j[b].n = f.n; dj.j[b].n_segs = f.n_segs;
@@ -450,7 +450,7 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     fa.mo = f.out[0] ? f.out[2] : f.m; fa.vo = f.out[0] ? f.out[3] : f.v;
     fa.idx_out = f.idx_out; fa.values_out = f.values_out; fa.mask_out = f.mask_out;
     fa.factor = factor; fa.coeff = coeff; fa.T = 0; fa.need = 0;
-    fa.vec = vec[b]; fa.mvec = aligned4(f.mask_out, 1);
+    fa.vec = vec[b]; fa.mvec = quads_ok(f.mask_out, 1);
     fa.scale = factor != 1.0f; fa.apply_coeff = coeff != 1.0f;
     fa.pack_extra = pack_extra;
     fa.adams = adams != 0; fa.fold = (flags & SGA_GC_FOLD) != 0; fa.interval = interval;
@@ -1158,10 +1158,10 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   // out: resid / p / m / v of the NEW state when the step runs out of place (the inputs stay
   // untouched, so a bracket that missed is redone by the radix passes and the key-forming final
   // sweep like a sweep that stood back); null: in place
-  const bool vec = aligned4(g, BF16G ? 2 : 4) && aligned4(resid, 4) && aligned4(p, 4) &&
-                   aligned4(m, 4) && aligned4(v, 4) &&
-                   (!out || (aligned4(out[0], 4) && aligned4(out[1], 4) && aligned4(out[2], 4) &&
-                             aligned4(out[3], 4)));
+  const bool vec = quads_ok(g, BF16G ? 2 : 4) && quads_ok(resid, 4) && quads_ok(p, 4) &&
+                   quads_ok(m, 4) && quads_ok(v, 4) &&
+                   (!out || (quads_ok(out[0], 4) && quads_ok(out[1], 4) && quads_ok(out[2], 4) &&
+                             quads_ok(out[3], 4)));
   const int adams = (flags & SGA_GC_ADAMS) ? 1 : 0;
   SrcFused<BF16G, SCORE> src{g, resid, p, m, v, vec, {}, pack_extra, adams};
   SegDirJobs dirs = {};
@@ -1174,7 +1174,7 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   fa.mo = out ? out[2] : m; fa.vo = out ? out[3] : v;
   fa.idx_out = idx_out; fa.values_out = values_out; fa.mask_out = mask_out;
   fa.factor = factor; fa.coeff = coeff; fa.T = 0; fa.need = 0;
-  fa.vec = vec; fa.mvec = aligned4(mask_out, 1);
+  fa.vec = vec; fa.mvec = quads_ok(mask_out, 1);
   fa.scale = factor != 1.0f; fa.apply_coeff = coeff != 1.0f;
   fa.pack_extra = pack_extra;
   fa.adams = adams != 0; fa.fold = (flags & SGA_GC_FOLD) != 0; fa.interval = interval;

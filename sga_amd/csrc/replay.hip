@@ -181,8 +181,8 @@ extern "C" int sga_score_formula(int score_id, const float* w, const float* m, c
   }
   if (adams) { bc1 = 1.0f; bc2 = 1.0f; }
   const Hyper h = mk_hyper(0.0f, beta1, om1, beta2, om2, eps, wd, bc1, bc2);
-  const bool vec = aligned4(w, 4) && aligned4(m, 4) && aligned4(v, 4) && aligned4(g, 4) &&
-                   aligned4(out, 4);
+  const bool vec = quads_ok(w, 4) && quads_ok(m, 4) && quads_ok(v, 4) && quads_ok(g, 4) &&
+                   quads_ok(out, 4);
   dim3 grid(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
 #define SGA_SF(S) hipLaunchKernelGGL((k_score_formula<S>), grid, block, 0, st, w, m, v, g, out, n, h, absolute != 0, adams != 0, no_wd, vec)
@@ -213,8 +213,8 @@ extern "C" int sga_branch_score_f64(int score_id, const float* w, const float* m
   }
   if (adams) { bc1 = 1.0; bc2 = 1.0; }
   const BranchK c{beta1, 1.0 - beta1, beta2, 1.0 - beta2, eps, wd, bc1, bc2};
-  const bool vec = aligned4(w, 4) && aligned4(m, 4) && aligned4(v, 4) && aligned4(g, 4) &&
-                   aligned4(out, 4);
+  const bool vec = quads_ok(w, 4) && quads_ok(m, 4) && quads_ok(v, 4) && quads_ok(g, 4) &&
+                   quads_ok(out, 4);
   dim3 grid(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
 #define SGA_BS(S) hipLaunchKernelGGL((k_branch_score<S>), grid, block, 0, st, w, m, v, g, out, n, c, adams != 0, include_wd != 0, vec)
@@ -241,8 +241,8 @@ extern "C" int sga_opt_step_inplace(const float* q, float* m, float* v, float* w
     return SGA_ERR_ARG;
   }
   StepK c{beta1, om1, beta2, om2, bc1, bc2, eps, omlwd, neglr, lr2, lr, lr_inactive, wd};
-  const bool vec = aligned4(q, 4) && aligned4(m, 4) && aligned4(v, 4) && aligned4(w, 4) &&
-                   aligned4(lab, 4) && aligned4(inactive, 1);
+  const bool vec = quads_ok(q, 4) && quads_ok(m, 4) && quads_ok(v, 4) && quads_ok(w, 4) &&
+                   quads_ok(lab, 4) && quads_ok(inactive, 1);
   dim3 grid(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
 #define SGA_OS(A, S, L) hipLaunchKernelGGL((k_opt_step<A, S, L>), grid, block, 0, st, q, m, v, w, lab, inactive, n, c, vec)

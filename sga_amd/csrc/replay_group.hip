@@ -601,7 +601,7 @@ static bool fill_group(RGroup* grp, const sga_replay_cfg* cfgs, int G) {
 static bool group_aligned(const RGroup& grp) {
   for (int c = 0; c < grp.G; ++c) {
     const RCfg& d = grp.c[c];
-    if (!aligned4(d.w, 4) || !aligned4(d.m, 4) || !aligned4(d.v, 4) || !aligned4(d.res, 4) ||
+    if (!quads_ok(d.w, 4) || !quads_ok(d.m, 4) || !quads_ok(d.v, 4) || !quads_ok(d.res, 4) ||
         !aligned4(d.sel, 1) || !aligned4(d.out_sel, 1))   // 4-byte words
       return false;
   }
@@ -685,7 +685,7 @@ extern "C" int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coe
     return SGA_ERR_ARG;
   }
   const bool bg = g_dtype == SGA_BF16;
-  const bool vec = aligned4(g, bg ? 2 : 4) && group_aligned(grp);
+  const bool vec = quads_ok(g, bg ? 2 : 4) && group_aligned(grp);
   const unsigned nb = stream_grid(cdiv64(n, kChunk), kChunksPerBlock, kReplayBlocks);
   hipStream_t s = (hipStream_t)stream;
   P1List lst = {};
@@ -723,7 +723,7 @@ extern "C" int sga_replay_pass3(const void* g, int g_dtype, int64_t n, float coe
     return SGA_ERR_ARG;
   }
   const bool bg = g_dtype == SGA_BF16;
-  const bool vec = aligned4(g, bg ? 2 : 4) && group_aligned(grp);
+  const bool vec = quads_ok(g, bg ? 2 : 4) && group_aligned(grp);
   const unsigned nb = stream_grid(n, (int64_t)kBlock * kVec, 1 << 22);   // one-shot: nothing to reduce
   hipStream_t s = (hipStream_t)stream;
   const RSeg* rs = reinterpret_cast<const RSeg*>(segs);
@@ -799,8 +799,8 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
         for (int b = a; b < count; ++b) {
           if (score[b] != score[a]) continue;
           const ReselJob& r = rj[b];
-          const bool vec = aligned4(g, BF16G ? 2 : 4) && aligned4(r.res, 4) && aligned4(r.w, 4) &&
-                           aligned4(r.m, 4) && aligned4(r.v, 4);
+          const bool vec = quads_ok(g, BF16G ? 2 : 4) && quads_ok(r.res, 4) && quads_ok(r.w, 4) &&
+                           quads_ok(r.m, 4) && quads_ok(r.v, 4);
           Src& src = srcs.s[sub.count];
           src = Src{g, r.res, r.w, r.m, r.v, r.coef_f, coef_dense, r.adams, vec, {},
                     packed ? kPackExtra : 0, r.res_zero};
@@ -1096,8 +1096,8 @@ static int run_reselect_balanced(const void* g, const float* res, const float* w
                                  float coef_dense, int adams, int packed, int res_zero,
                                  uint32_t* sel_out, sga_select_result* result, uint32_t* hist,
                                  const SelWorkspace& ws, hipStream_t s) {
-  const bool vec = aligned4(g, BF16G ? 2 : 4) && aligned4(res, 4) && aligned4(w, 4) &&
-                   aligned4(m, 4) && aligned4(v, 4);
+  const bool vec = quads_ok(g, BF16G ? 2 : 4) && quads_ok(res, 4) && quads_ok(w, 4) &&
+                   quads_ok(m, 4) && quads_ok(v, 4);
   SrcReplay<BF16G, SCORE> src{g, res, w, m, v, coef_f, coef_dense, adams, vec, {},
                               packed ? kPackExtra : 0, res_zero};
   launch_seg_dir(segs, n_segs, n, ws.seg_dir, s);
@@ -1160,8 +1160,8 @@ extern "C" int sga_dense_replay_step(const void* g, int g_dtype, float* w, float
     return SGA_ERR_ARG;
   }
   const bool bg = g_dtype == SGA_BF16;
-  const bool vec = aligned4(g, bg ? 2 : 4) && aligned4(w, 4) && aligned4(m, 4) && aligned4(v, 4) &&
-                   aligned4(lab, 4);
+  const bool vec = quads_ok(g, bg ? 2 : 4) && quads_ok(w, 4) && quads_ok(m, 4) && quads_ok(v, 4) &&
+                   quads_ok(lab, 4);
   // as close to one 1024-element slab per workgroup as the partials workspace allows (a capped
   // grid-stride loop leaves a quarter of the bandwidth unused); the fold stays in a fixed order
   const unsigned nb = stream_grid(n, (int64_t)kBlock * kVec, kReplayBlocks * kMaxCfg);
@@ -1182,7 +1182,7 @@ extern "C" int sga_mask_to_planes(const uint8_t* mask, int64_t n, uint32_t* plan
   if (n == 0) return SGA_OK;
   if (!mask || !planes || n < 0) { set_error("sga_mask_to_planes: bad argument"); return SGA_ERR_ARG; }
   hipLaunchKernelGGL(k_mask_to_planes, dim3(stream_grid(cdiv64(n, kChunk), kChunksPerBlock, 1 << 22)),
-                     dim3(kBlock), 0, (hipStream_t)stream, mask, n, planes, aligned4(mask, 1));
+                     dim3(kBlock), 0, (hipStream_t)stream, mask, n, planes, quads_ok(mask, 1));
   return check_launch("sga_mask_to_planes");
 }
 
@@ -1199,7 +1199,7 @@ extern "C" int sga_div_inplace(float* x, int64_t n, float d, int packed, void* s
   if (n == 0) return SGA_OK;
   if (!x || n < 0) { set_error("sga_div_inplace: bad argument"); return SGA_ERR_ARG; }
   hipLaunchKernelGGL(k_div_inplace, dim3(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), dim3(kBlock), 0,
-                     (hipStream_t)stream, x, n, d, aligned4(x, 4), packed ? kPackExtra : 0);
+                     (hipStream_t)stream, x, n, d, quads_ok(x, 4), packed ? kPackExtra : 0);
   return check_launch("sga_div_inplace");
 }
 
@@ -1209,7 +1209,7 @@ extern "C" int sga_sq_dist(const float* a, int a_packed, const float* b, int64_t
   const unsigned nb = stream_grid(n, (int64_t)kBlock * kVec, 1024);
   hipStream_t s = (hipStream_t)stream;
   hipLaunchKernelGGL(k_sqdist_stage1, dim3(nb), dim3(kBlock), 0, s, a, b, n, partials,
-                     aligned4(a, 4) && aligned4(b, 4), a_packed ? kPackExtra : 0);
+                     quads_ok(a, 4) && quads_ok(b, 4), a_packed ? kPackExtra : 0);
   hipLaunchKernelGGL(k_sqdist_stage2, dim3(1), dim3(kWave), 0, s, partials, (int)nb, out);
   return check_launch("sga_sq_dist");
 }

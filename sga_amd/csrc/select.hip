@@ -268,7 +268,7 @@ extern "C" int sga_sel_hist(const float* score, int64_t n, int level, void* ws,
   }
   // histogram only: several views feed one level before its scan
   SrcPack<SrcF32> srcs = {};
-  srcs.s[0] = SrcF32{score, aligned4(score, 4)};
+  srcs.s[0] = SrcF32{score, quads_ok(score, 4)};
   SelBatch B;
   B.add(w, n, 1, 0);
   launch_level_data<SrcF32>(srcs, B, level, (hipStream_t)stream);
@@ -292,7 +292,7 @@ extern "C" int sga_sel_count(const float* score, int64_t n, int64_t tile_base, v
   if (int rc = carve(ws, ws_bytes, tile_base + cdiv64(n, kChunk), &w, "sga_sel_count")) return rc;
   if (!score || n < 0 || tile_base < 0) { set_error("sga_sel_count: bad argument"); return SGA_ERR_ARG; }
   SrcPack<SrcF32> srcs = {};
-  srcs.s[0] = SrcF32{score, aligned4(score, 4)};
+  srcs.s[0] = SrcF32{score, quads_ok(score, 4)};
   SelBatch B;
   B.add(w, n, 1, 0);
   launch_tile_count(srcs, B, tile_base, (hipStream_t)stream);
@@ -320,7 +320,7 @@ extern "C" int sga_sel_mask(const float* score, int64_t n, int64_t tile_base, in
   if (int rc = carve(ws, ws_bytes, tile_base + cdiv64(n, kChunk), &w, "sga_sel_mask")) return rc;
   if (!score || !mask_out || n < 0 || tile_base < 0) { set_error("sga_sel_mask: bad argument"); return SGA_ERR_ARG; }
   SrcPack<SrcF32> srcs = {};
-  srcs.s[0] = SrcF32{score, aligned4(score, 4)};
+  srcs.s[0] = SrcF32{score, quads_ok(score, 4)};
   SelBatch B;
   B.add(w, n, 1, tie_mode == SGA_TIE_ALL).mask = mask_out;
   hipLaunchKernelGGL((k_write_mask<SrcF32>), B.grid(stream_grid(B.max_tiles, kChunksPerBlock, 1 << 22)),
@@ -350,7 +350,7 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   if (int rc = carve(ws, ws_bytes, cdiv64(n, kChunk), &w, "sga_select_topk")) return rc;
   hipStream_t s = (hipStream_t)stream;
   SrcPack<SrcF32> srcs = {};
-  srcs.s[0] = SrcF32{score, aligned4(score, 4)};
+  srcs.s[0] = SrcF32{score, quads_ok(score, 4)};
   SelBatch B;
   ChainJob& J = B.add(w, n, k, tie_mode == SGA_TIE_ALL);
   J.mask = mask_out;
@@ -400,7 +400,7 @@ extern "C" int sga_mask_topbits_ge(const float* score, int64_t n, int shift, int
   }
   hipLaunchKernelGGL(k_mask_topbits_ge, dim3(stream_grid(n, (int64_t)kBlock * kVec, 1 << 22)), dim3(kBlock),
                      0, (hipStream_t)stream, score, n, shift, (uint32_t)bin, mask_out,
-                     aligned4(score, 4) && aligned4(mask_out, 1));
+                     quads_ok(score, 4) && quads_ok(mask_out, 1));
   return check_launch("sga_mask_topbits_ge");
 }
 
@@ -411,7 +411,7 @@ extern "C" int sga_mask_abs_ge(const float* score, int64_t n, float tau, uint8_t
   hipLaunchKernelGGL(k_mask_abs_ge, dim3(stream_grid(n, (int64_t)kBlock * kVec * 4, 256 * 16)),
                      dim3(kBlock), 0, (hipStream_t)stream, score, n, tau, mask_out,
                      reinterpret_cast<unsigned long long*>(count),
-                     aligned4(score, 4) && aligned4(mask_out, 1));
+                     quads_ok(score, 4) && quads_ok(mask_out, 1));
   return check_launch("sga_mask_abs_ge");
 }
 
@@ -425,7 +425,7 @@ extern "C" int sga_cand_extract_count(const float* score, int64_t n, int32_t bin
   hipStream_t st = (hipStream_t)stream;
   if (nc > 0)
     hipLaunchKernelGGL(k_cand_count, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)), dim3(kBlock), 0, st,
-                       score, n, (uint32_t)bin, chunk_counts, nc, aligned4(score, 4));
+                       score, n, (uint32_t)bin, chunk_counts, nc, quads_ok(score, 4));
   if (int rc = exclusive_scan_u32(chunk_counts, nc, total, st)) return rc;
   return check_launch("sga_cand_extract_count");
 }
@@ -441,7 +441,7 @@ extern "C" int sga_cand_extract_fill(const float* score, int64_t n, int32_t bin,
   const int64_t nc = cdiv64(n, kChunk);
   hipLaunchKernelGGL(k_cand_fill, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)), dim3(kBlock), 0,
                      (hipStream_t)stream, score, n, (uint32_t)bin, chunk_offsets, cand,
-                     cand_capacity, nc, aligned4(score, 4));
+                     cand_capacity, nc, quads_ok(score, 4));
   return check_launch("sga_cand_extract_fill");
 }
 
@@ -456,6 +456,6 @@ extern "C" int sga_gt_eq(const float* score, int64_t n, float thresh, uint8_t* g
   if (n > 0)
     hipLaunchKernelGGL(k_gt_eq, dim3(stream_grid(n, (int64_t)kBlock * kVec * 4, 256 * 16)),
                        dim3(kBlock), 0, st, score, n, thresh, gt, eq, counts2,
-                       aligned4(score, 4) && aligned4(gt, 1) && aligned4(eq, 1));
+                       quads_ok(score, 4) && quads_ok(gt, 1) && quads_ok(eq, 1));
   return check_launch("sga_gt_eq");
 }

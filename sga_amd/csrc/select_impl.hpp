@@ -758,7 +758,7 @@ template <class Src>
 __device__ __forceinline__ void write_mask_body(Src& src, const ChainJob& J, uint32_t T, uint32_t need,
                                                 int64_t tile_base, uint8_t* __restrict__ mask, uint32_t blk,
                                                 uint32_t n_blk) {
-  const bool mvec = aligned4(mask, 1);
+  const bool mvec = quads_ok(mask, 1);
   const int64_t n = J.n;
   const int64_t n_chunks = cdiv64(n, kChunk);
   const int64_t wstride = (int64_t)n_blk * kChunksPerBlock;
@@ -1254,7 +1254,7 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
   // The loads of kAhead slabs (256 elements each) are issued together, then
   // their keys are formed slab by slab: expensive key sources (Adam-normalised
   // scores) look fewer slabs ahead to stay within their register budget.  The
-  // ragged path (last chunk, unaligned views) goes one slab at a time through
+  // ragged path (the last chunk) goes one slab at a time through
   // a rolled loop: it only has to be small.
   constexpr int kAhead = FULL ? Src::kAhead : 1;
   static_assert(kChunkIters % kAhead == 0, "look-ahead divides the slabs of a chunk");
@@ -2133,7 +2133,7 @@ static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int
       hipLaunchKernelGGL((k_bracket_sweep<Src, 2>), dim3(sweep_blocks), dim3(kBlock), 0, s,
                          srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
                          w.seg_cnt, (uint32_t)w.seg_cap, (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
-                         J.mask, (reinterpret_cast<uintptr_t>(J.mask) & 3) == 0);
+                         J.mask, true);
     else if (pm == 1)
       hipLaunchKernelGGL((k_bracket_sweep<Src, 1>), dim3(sweep_blocks), dim3(kBlock), 0, s,
                          srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
