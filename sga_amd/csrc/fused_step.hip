@@ -154,13 +154,13 @@ struct FinalArgs {
 // chunk is entirely in range and every array is element-aligned, so all 20
 // loads are unconditional and issued before the first use.
 // IT0 / NIT: the slabs [IT0, IT0+NIT) of the chunk are handled by this call;
-// `cur` carries the running selected / tie counts across calls.
+// `cur` carries the running selected / tie counts across calls.  slab: added to the slab numbers.
 // PLANES: the selection was already settled as bit planes (bracket sweep +
 // candidates): the slab's four 64-bit ballots are read on the scalar unit and
 // the keys are not formed again; SCORE is then irrelevant.
 template <bool BF16G, bool BF16V, int SCORE, bool FULL, int IT0, int NIT, bool PLANES>
 __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, ChunkCursor& cur,
-                                            SegCursor& sc) {
+                                            SegCursor& sc, int slab = 0) {
   const int64_t n = a.n;
   const int64_t sh = pack_shift<true>(c << 10, a.pack_extra);     // c is wave-uniform
   const float* const R = a.r + sh;
@@ -182,7 +182,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
         vraw[kChunkIters];
 #pragma unroll
     for (int it = IT0; it < IT0 + NIT; ++it) {
-      const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
+      const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
       if (BF16G) graw_h[it] = ldh4_nt(reinterpret_cast<const uint16_t*>(a.g) + i);
       else if (has_g) graw_f[it] = ld4_nt(reinterpret_cast<const float*>(a.g) + i);
       else graw_f[it] = F4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -192,6 +192,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
       vraw[it] = ld4_nt(V + i);
     }
     __builtin_amdgcn_sched_barrier(0);
+    if (NIT > 1) sc.seek_uniform(uniform_i64(c) * kChunk);   // its chain of scalar loads runs beside the data's
 #pragma unroll
     for (int it = IT0; it < IT0 + NIT; ++it) {
       if (BF16G) {
@@ -208,7 +209,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
   } else {
 #pragma unroll
     for (int it = IT0; it < IT0 + NIT; ++it) {
-      const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
+      const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
 #pragma unroll
       for (int e = 0; e < 4; ++e) gg[it][e] = rr[it][e] = pp[it][e] = mm[it][e] = vv[it][e] = 0.0f;
       if (i < n) {
@@ -222,7 +223,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
   }
 #pragma unroll
   for (int it = IT0; it < IT0 + NIT; ++it) {
-    const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
+    const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
     float q[4];
     bool valid[4], sel[4];
     uint32_t pos;
@@ -230,7 +231,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
       // words 2e, 2e + 1 of the slab are the ballot of element e over the 64 lanes; lanes are in
       // index order, so the selected coordinates before (lane, e) are the mask bits below the
       // lane over all four ballots plus the lane's own earlier elements
-      const uint64_t* pw = reinterpret_cast<const uint64_t*>(a.planes) + (uniform_i64(c) * kChunkIters + it) * 4;
+      const uint64_t* pw = reinterpret_cast<const uint64_t*>(a.planes) + (uniform_i64(c) * kChunkIters + it + slab) * 4;
       uint32_t below = 0, total = 0;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -254,7 +255,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
         else if (SCORE == SGA_SCORE_ABS_M) key[e] = abs_key(mm[it][e]);
       }
       if (SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI || SCORE == SGA_SCORE_GR_OVER_SQRT_V) {
-        const int64_t s0 = uniform_i64(c) * kChunk + it * (kWave * kVec);
+        const int64_t s0 = uniform_i64(c) * kChunk + (it + slab) * (kWave * kVec);
         if (FULL || s0 < n) {
           float vk[4];
 #pragma unroll
@@ -294,7 +295,7 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
       }
       // The commit takes its hyper-parameters from the scalar unit: the slab lies inside one
       // tensor but for the few that hold a boundary, which are committed once per tensor piece.
-      const int64_t s0 = uniform_i64(c) * kChunk + it * (kWave * kVec);
+      const int64_t s0 = uniform_i64(c) * kChunk + (it + slab) * (kWave * kVec);
       int64_t s1 = s0 + kWave * kVec;
       if (!FULL && s1 > n) s1 = n;
       if (s0 < sc.lo || s0 >= sc.hi) sc.seek_uniform(s0);
@@ -340,8 +341,9 @@ __device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, Chunk
 // keys are formed again here); 3 like 2, and only if the single-sweep step
 // stood back before it touched anything.
 // (five waves per SIMD wherever the key is not an Adam-normalised chain formed in this kernel)
-template <bool BF16G, bool BF16V, int SCORE, bool PLANES>
-__global__ __launch_bounds__(kBlock, (PLANES || SCORE == SGA_SCORE_ABS_G || SCORE == SGA_SCORE_ABS_M ||
+// AHEAD: slabs of a chunk whose loads are issued together.
+template <bool BF16G, bool BF16V, int SCORE, bool PLANES, int AHEAD = 1>
+__global__ __launch_bounds__(kBlock, AHEAD > 1 ? 1 : (PLANES || SCORE == SGA_SCORE_ABS_G || SCORE == SGA_SCORE_ABS_M ||
                                       SCORE == SGA_SCORE_ABS_G_BLIND) ? 5 : 1)
 void k_fused_final(
     FinalArgs a, const sga_segment* __restrict__ segs, int n_segs,
@@ -363,6 +365,10 @@ void k_fused_final(
     cur.sel_run = tile_sel[c];
     cur.eq_run = PLANES ? 0u : tile_eq[c];
     if (can_full && (c + 1) * kChunk <= a.n) {
+      if (AHEAD == kChunkIters) {
+        final_chunk<BF16G, BF16V, SCORE, true, 0, kChunkIters, PLANES>(a, c, cur, sc);
+        continue;
+      }
       // one 256-element slab at a time (5 loads in flight per lane): measured
       // as fast as batching all four slabs, at twice the occupancy
       final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc);
@@ -370,15 +376,24 @@ void k_fused_final(
       final_chunk<BF16G, BF16V, SCORE, true, 2, 1, PLANES>(a, c, cur, sc);
       final_chunk<BF16G, BF16V, SCORE, true, 3, 1, PLANES>(a, c, cur, sc);
     } else {
-      // the ragged path too: holding four slabs at once would set the register count (and so
-      // the occupancy) of the whole kernel
-      final_chunk<BF16G, BF16V, SCORE, false, 0, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, false, 1, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, false, 2, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, false, 3, 1, PLANES>(a, c, cur, sc);
+      // A ragged chunk slab by slab (four at once would set the register count, and so the occupancy, of
+      // the whole kernel), its whole slabs by the unconditional accesses: the wave that owns it is the last
+      // to finish, which a small bucket waits for.
+#pragma unroll 1
+      for (int sl = 0; sl < kChunkIters; ++sl) {
+        const int64_t s0 = c * kChunk + sl * (kWave * kVec);
+        if (can_full && s0 + kWave * kVec <= a.n) final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc, sl);
+        else if (s0 < a.n) final_chunk<BF16G, BF16V, SCORE, false, 0, 1, PLANES>(a, c, cur, sc, sl);
+      }
     }
   }
 }
+
+// Up to this many chunks (four waves per SIMD) every wave of the final sweep is resident at once, so that
+// nothing hides the latency of its four slabs but having all their loads in flight.  Step, one slab at a
+// time -> four, with the same in k_small_sweep: 2 M coordinates 64.8 -> 61.3 us, 4 M 88.3 -> 84.1, eight
+// buckets of 1 M 199 -> 183.  Large buckets have waves enough to hide it (k_fused_final).
+constexpr int64_t kBatchedTiles = 4096;
 
 // One bucket of a (possibly batched) fused step.
 struct FusedJob {
@@ -463,6 +478,9 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
       hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>),
                          dim3(stream_grid(n_tiles, kChunksPerBlock, 2048)), dim3(kBlock), 0, s, fa,
                          f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 2, w.seg_dir);
+    } else if (n_tiles <= kBatchedTiles && !Src::kHyper) {
+      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, Src::kHyper ? SGA_SCORE_ABS_G : SCORE, false, kChunkIters>),
+                         one_shot, dim3(kBlock), 0, s, fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 0, w.seg_dir);
     } else {
       hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>), one_shot, dim3(kBlock), 0, s, fa,
                          f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 0, w.seg_dir);

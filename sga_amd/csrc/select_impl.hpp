@@ -960,7 +960,7 @@ __device__ __forceinline__ auto drop_dir(S& s, int) -> decltype(s.sc.dir, void()
 template <class S>
 __device__ __forceinline__ void drop_dir(S&, long) {}
 
-// Sample keys (one quad per window at a hashed offset; the windows tile all quads, see k_sample),
+// Sample keys (one quad per window at a hashed offset; the windows tile all quads, see quad_of_window),
 // the list counters, and, in a job's last workgroup, the directory of its segment table
 // (dirs.j[job].dir null: none wanted).  Gathering from one workgroup would be bound by one CU's
 // translation misses (4096 quads of two arrays: 25 us; 64 workgroups: 4).
@@ -1243,7 +1243,7 @@ __device__ __forceinline__ void plane_put(const Ballot4& a, int it, uint32_t* ld
 // PM: 0 counts only; 1 the provisional selection (keys above the bracket) also goes out as bit
 // planes; 2 as mask bytes, straight into the caller's mask (a mask-only select then needs no
 // expansion pass: the candidates are settled in the bytes).
-template <class Src, bool FULL, int PM>
+template <class Src, bool FULL, int PM, int AHEAD = Src::kAhead>
 __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chunk& ck, int64_t n,
                                               int64_t c, uint32_t T_LO,
                                               uint32_t T_HI, uint32_t& chi, uint32_t& tot_nf,
@@ -1256,7 +1256,7 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
   // scores) look fewer slabs ahead to stay within their register budget.  The
   // ragged path (the last chunk) goes one slab at a time through
   // a rolled loop: it only has to be small.
-  constexpr int kAhead = FULL ? Src::kAhead : 1;
+  constexpr int kAhead = FULL ? AHEAD : 1;
   static_assert(kChunkIters % kAhead == 0, "look-ahead divides the slabs of a chunk");
   constexpr int kGroupUnroll = kAhead == kChunkIters ? kChunkIters : 1;
   src.chunk_hyper(c);        // measured: looking the tensor up behind the first loads instead is slower

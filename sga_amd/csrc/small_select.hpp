@@ -8,8 +8,8 @@
 // followed by the caller's writing pass (final sweep, k_write_mask, k_write_bits), which forms the
 // keys again: the whole bucket sits in L2 / Infinity Cache then.
 //
-// Why not the chain of the large buckets (select_impl.hpp): that is about twenty dependent
-// launches, 150 us of launch latency, device-scope fences and half-empty grids whatever the size,
+// Why not the chain of the large buckets (select_impl.hpp): that is seven dependent
+// launches beside the sweeps (twenty, 150 us, when this path was written) and half-empty grids,
 // where the data of a 4 M-element bucket takes 24 us.  One workgroup is enough for what lies
 // between the sweeps as long as the chunk counts fit its LDS, which draws the line at kSmallTiles
 // (8 M coordinates at 1 %: 30 us in k_small_finish, as much as the sweep and a half).
@@ -61,7 +61,8 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
   uint32_t chi = 0, nf = 0, cnt = 0;
   if (c < n_chunks) {
     const typename Src::Chunk ck = src.chunk_begin(c);
-    if (full) bracket_chunk<Src, true, 0>(src, ck, n, c, T_LO, T_HI, chi, nf, cnt, lds, nullptr);
+    // small grids: the latency of a chunk's four slabs counts, not how many waves are resident
+    if (full) bracket_chunk<Src, true, 0, kChunkIters>(src, ck, n, c, T_LO, T_HI, chi, nf, cnt, lds, nullptr);
     else bracket_chunk<Src, false, 0>(src, ck, n, c, T_LO, T_HI, chi, nf, cnt, lds, nullptr);
     if (lane_id() == 0) { J.tile_gt[c] = chi; J.tile_eq[c] = single ? cnt : 0u; }
   }
