@@ -1243,14 +1243,16 @@ __device__ __forceinline__ void plane_put(const Ballot4& a, int it, uint32_t* ld
 // PM: 0 counts only; 1 the provisional selection (keys above the bracket) also goes out as bit
 // planes; 2 as mask bytes, straight into the caller's mask (a mask-only select then needs no
 // expansion pass: the candidates are settled in the bytes).
-template <class Src, bool FULL, int PM, int AHEAD = Src::kAhead>
+// BELOW: `below` also counts the keys right below the range, T_LO - 1.
+template <class Src, bool FULL, int PM, int AHEAD = Src::kAhead, bool BELOW = false>
 __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chunk& ck, int64_t n,
                                               int64_t c, uint32_t T_LO,
                                               uint32_t T_HI, uint32_t& chi, uint32_t& tot_nf,
                                               uint32_t& mycnt, SweepLds& lds,
                                               uint32_t* __restrict__ pbits,
                                               uint8_t* __restrict__ mask_bytes = nullptr,
-                                              bool mvec = false, bool m16 = false) {
+                                              bool mvec = false, bool m16 = false,
+                                              uint32_t* below = nullptr) {
   // The loads of kAhead slabs (256 elements each) are issued together, then
   // their keys are formed slab by slab: expensive key sources (Adam-normalised
   // scores) look fewer slabs ahead to stay within their register budget.  The
@@ -1282,6 +1284,7 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
         above.m[e] = ballot64(key[e] >= T_HI) & valid;
         cand.m[e] = ballot64(key[e] >= T_LO) & valid & ~above.m[e];
         nf |= ballot64(key[e] >= 0x7F800000u) & valid;
+        if (BELOW) *below += (uint32_t)__popcll(ballot64(key[e] == T_LO - 1u) & valid);
       }
       chi += above.count();
       if (nf) {                                  // rare: count them properly

@@ -42,8 +42,10 @@ __host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles) {
 }
 
 // The sweep: one chunk per wave, counts above the bracket, keys inside it to the list (one
-// reservation per workgroup).  A bracket of a single key (the sample says a plateau of equal keys
-// holds the k-th one) needs no list: its members are ties, counted per chunk.
+// reservation per workgroup).  Keys equal to the bracket's lower end are counted per chunk and not
+// listed: a plateau of equal keys (zeros, momenta that have decayed to the last denormal) puts the
+// lower end on itself, and the one workgroup behind the sweep would walk a list as long as the bucket
+// (|m| after a thousand sparse steps, 1.7 M coordinates: 889 us, 86 like this).
 template <class Src>
 __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, ChainJobs jobs) {
   const ChainJob& J = jobs.j[blockIdx.y];
@@ -54,20 +56,23 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
   SelState* __restrict__ st = J.st;
   Src src = srcs.s[blockIdx.y];
   const uint32_t T_LO = st->t_lo, T_HI = st->t_hi;
-  const bool single = T_HI - T_LO == 1u;
   const int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id();
   const bool full = src.vec && (c + 1) * kChunk <= n;
   SweepLds& lds = s_lds[wave_id()];
-  uint32_t chi = 0, nf = 0, cnt = 0;
+  uint32_t chi = 0, nf = 0, cnt = 0, eq = 0;
   if (c < n_chunks) {
     const typename Src::Chunk ck = src.chunk_begin(c);
     // small grids: the latency of a chunk's four slabs counts, not how many waves are resident
-    if (full) bracket_chunk<Src, true, 0, kChunkIters>(src, ck, n, c, T_LO, T_HI, chi, nf, cnt, lds, nullptr);
-    else bracket_chunk<Src, false, 0>(src, ck, n, c, T_LO, T_HI, chi, nf, cnt, lds, nullptr);
-    if (lane_id() == 0) { J.tile_gt[c] = chi; J.tile_eq[c] = single ? cnt : 0u; }
+    if (full)
+      bracket_chunk<Src, true, 0, kChunkIters, true>(src, ck, n, c, T_LO + 1u, T_HI, chi, nf, cnt, lds, nullptr,
+                                                     nullptr, false, false, &eq);
+    else
+      bracket_chunk<Src, false, 0, 1, true>(src, ck, n, c, T_LO + 1u, T_HI, chi, nf, cnt, lds, nullptr, nullptr, false,
+                                            false, &eq);
+    if (lane_id() == 0) { J.tile_gt[c] = chi; J.tile_eq[c] = eq; }
   }
   const bool neg = ballot64(src_negative(src) != 0u) != 0ull;
-  if (lane_id() == 0) { s_cnt[wave_id()] = single ? 0u : cnt; s_nf[wave_id()] = nf | (neg ? 0x80000000u : 0u); }
+  if (lane_id() == 0) { s_cnt[wave_id()] = cnt; s_nf[wave_id()] = nf | (neg ? 0x80000000u : 0u); }
   __syncthreads();
   const SmallGeom geo = small_geom(n_chunks);
   const uint32_t seg = blockIdx.x % geo.segs;
@@ -79,7 +84,7 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
     if ((s_nf[0] | s_nf[1] | s_nf[2] | s_nf[3]) & 0x80000000u) raise_negative(st);
   }
   __syncthreads();
-  if (single || cnt == 0) return;
+  if (cnt == 0) return;
   uint32_t base = seg * geo.cap + s_base;
   for (int w = 0; w < wave_id(); ++w) base += s_cnt[w];
   if (cnt <= (uint32_t)kWaveCandCap) {
@@ -90,7 +95,7 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
     return;
   }
   // more keys than the wave's LDS holds: the bracket's keys crowd into few chunks
-  recollect(src, n, c, T_LO, T_HI, [&](uint32_t pos, uint32_t idx, uint32_t key) {
+  recollect(src, n, c, T_LO + 1u, T_HI, [&](uint32_t pos, uint32_t idx, uint32_t key) {
     J.small_idx[base + pos] = idx;
     J.small_key[base + pos] = key;
   });
@@ -177,7 +182,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   for (int j = 0; j < PER; ++j) {
     const int t = j * kWide + threadIdx.x;
     g8[j] = t < nt ? J.tile_gt[t] : 0u;
-    e8[j] = t < nt && single ? J.tile_eq[t] : 0u;
+    e8[j] = t < nt ? J.tile_eq[t] : 0u;
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -189,22 +194,29 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   if (threadIdx.x < kWideWaves)
     s_seg[threadIdx.x] = threadIdx.x < geo.segs ? J.seg_cnt[threadIdx.x * kSmallSegStride] : 0u;
   if (threadIdx.x == 0) s_cnt = 0u;
-  uint32_t n_hi, n_in;
+  uint32_t n_hi, n_low, n_list = 0;
   wide_prefix(hi, s_scan, 0, n_hi);
-  wide_prefix(eqs, s_scan, 1, n_in);
+  wide_prefix(eqs, s_scan, 1, n_low);
   list.counted(s_seg[wave_id()]);
-  if (!single) {
-    n_in = 0;
-    for (int w = 0; w < kWideWaves; ++w) n_in += s_seg[w];
-  }
-  const bool ok = n_hi < k && k <= n_hi + n_in;
-  uint32_t T = T_LO, need = k - n_hi, n_eq = n_in;
+  for (int w = 0; w < kWideWaves; ++w) n_list += s_seg[w];
+  const bool ok = n_hi < k && k <= n_hi + n_list + n_low;
+  const bool low = ok && k > n_hi + n_list;           // the lower end is the threshold
+  uint32_t T = T_LO, need = k - n_hi - n_list, n_eq = n_low;
   int turn = 0;
-  if (ok && !single) {
-    // descent over the list inside [T_LO, T_HI): 4096 bins per level, until one bin is left whose
+  if (low) {
+    auto above = [&](uint32_t key, uint32_t idx) {
+      if (key != ~0u) atomicAdd(&s_tile[idx >> 10], 1u);
+    };
+    list.visit(above, above);
+    __syncthreads();
+  } else if (ok) {
+    // the lower end is below the threshold: its members are no ties
+#pragma unroll
+    for (int j = 0; j < PER; ++j) s_tile[j * kWide + threadIdx.x] = g8[j];
+    // descent over the list inside (T_LO, T_HI): 4096 bins per level, until one bin is left whose
     // keys fit the short list (nearly always after the first level) or are all equal
-    uint32_t lo = T_LO, rank = k - n_hi;
-    int w = 32 - __clz((int)(T_HI - 1u - T_LO));       // bits of the offset (T_HI - T_LO >= 2)
+    uint32_t lo = T_LO + 1u, rank = k - n_hi;
+    int w = 32 - __clz((int)(T_HI - 1u - lo));         // bits of the offset (the list is not empty)
     for (;;) {
       const int sh = w > 12 ? w - 12 : 0;
       list.visit(

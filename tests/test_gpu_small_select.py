@@ -54,6 +54,17 @@ def test_plateaus_and_crowded_chunks(dev, n):
             _check(dev, sc, k, (name, n, k))
 
 
+# momenta decayed to the last denormals: the lower end of the bracket is a value that nearly all share
+@pytest.mark.parametrize("n", [4097, 1_671_561, LIMIT])
+def test_plateau_at_the_lower_end(dev, n):
+    base = student_t(n, 8).abs() + 1e-6
+    few = max(2, n // 40)
+    tiny = torch.where(torch.arange(n) % 977 == 0, 3.0, 4.0) * 2.0 ** -149
+    sc = torch.where(base >= base.kthvalue(n - few + 1)[0], base, tiny)
+    for k in (few - 1, few, few + 1, few + n // 1000, n // 4, n - 1):
+        _check(dev, sc, k, (n, k))
+
+
 @pytest.mark.parametrize("n", [LIMIT + 5, 20_000_003])
 @pytest.mark.parametrize("name", ["plain", "grid", "zeros", "crowd", "hot"])
 def test_settlement_of_large_buckets(dev, n, name):
