@@ -51,6 +51,16 @@ struct Ref {                       // owned reference
   operator PyObject*() const { return o; }
 };
 
+// The interpreter lock is released while one of these lives: also where what runs under it throws
+// (a device error surfaces at the next read from the device) the handler holds the lock again.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  Unlocked() = default;
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 bool number(PyObject* obj, PyObject* name, double* out) {
   Ref v(PyObject_GetAttr(obj, name));
   if (!v.o) return false;
@@ -338,10 +348,10 @@ PyObject* norm(PyObject*, PyObject* args) {
   const int rc = f_norm_multi(static_cast<const sga_span_record*>(table.data_ptr()), n_rows, spans, partials,
                               partials + spans, (void*)stream);
   if (rc != 0) return PyLong_FromLong(rc);
-  double total;
-  Py_BEGIN_ALLOW_THREADS
-  total = buf[spans].item<float>();
-  Py_END_ALLOW_THREADS
+  const double total = [&] {
+    Unlocked released;
+    return buf[spans].item<float>();
+  }();
   return PyFloat_FromDouble((double)(float)std::sqrt(total));
   END_HANDLE_TH_ERRORS
 }

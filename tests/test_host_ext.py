@@ -1,0 +1,39 @@
+"""The native host side of the plugin steps (csrc/host_ext.cpp) where it can be
+driven without a device."""
+import subprocess
+import sys
+import textwrap
+
+from sga_amd import build as B
+
+
+def _run(body):
+    """``body`` in a process of its own (what it binds must not reach the other
+    tests, and a crash must end nothing but it), with the extension as ``host``."""
+    head = f"""
+        import ctypes as C, importlib.util, sys
+        import torch
+        spec = importlib.util.spec_from_file_location("_host", {B.HOST_EXT!r})
+        host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(host)
+        nop = C.CFUNCTYPE(C.c_int)(lambda: 0)
+        addr = C.cast(nop, C.c_void_p).value
+        """
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(head) + textwrap.dedent(body)],
+                       capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and r.stdout.endswith("done\n"), (r.returncode, r.stdout, r.stderr)
+
+
+def test_an_error_while_the_norm_is_read_raises():
+    """The read of the norm is where an earlier device error surfaces: it has to
+    arrive as an exception in a thread that holds the interpreter again.  A meta
+    tensor stands for the device whose read fails."""
+    _run("""
+        host.bind(object, addr, addr, addr, addr)
+        try:
+            host.norm(torch.empty(64, dtype=torch.uint8, device="meta"), 1, 1, 0)
+            raise SystemExit("no error")
+        except RuntimeError as e:
+            assert "meta" in str(e), e
+        print("done")
+        """)
