@@ -121,13 +121,13 @@ at::Tensor to_device(const std::vector<T>& rows, c10::Device dev) {
   return out;
 }
 
-struct Walk {                      // iterates a list / tuple of records
-  Ref seq;
+struct Walk {                      // a list / tuple of records; n < 0: anything else, left untouched
+  PyObject* seq;
   Py_ssize_t n;
-  explicit Walk(PyObject* records) : seq(PySequence_Fast(records, "records")) {
-    n = seq.o ? PySequence_Fast_GET_SIZE(seq.o) : -1;
+  explicit Walk(PyObject* records) : seq(records) {
+    n = PyList_Check(records) || PyTuple_Check(records) ? PySequence_Fast_GET_SIZE(records) : -1;
   }
-  PyObject* at(Py_ssize_t i) { return PySequence_Fast_GET_ITEM(seq.o, i); }
+  PyObject* at(Py_ssize_t i) { return PySequence_Fast_GET_ITEM(seq, i); }
 };
 
 PyObject* not_ordinary() {
@@ -181,7 +181,7 @@ PyObject* commit(PyObject*, PyObject* args) {
                         &inactive, &adams, &stream))
     return nullptr;
   Walk w(records);
-  if (w.n < 0) return nullptr;
+  if (w.n < 0) return not_ordinary();
   std::vector<sga_gc_record> rows;
   rows.reserve((size_t)w.n);
   int64_t spans = 0;
@@ -225,7 +225,7 @@ PyObject* commit_compact(PyObject*, PyObject* args) {
                         &adams, &stream))
     return nullptr;
   Walk w(records);
-  if (w.n < 0) return nullptr;
+  if (w.n < 0) return not_ordinary();
   if (!PyDict_Check(values_of)) return not_ordinary();
   std::vector<sga_gcc_record> rows;
   rows.reserve((size_t)w.n);
@@ -303,7 +303,7 @@ PyObject* norm_table(PyObject*, PyObject* args) {
   int was_full;
   if (!PyArg_ParseTuple(args, "Op", &records, &was_full)) return nullptr;
   Walk w(records);
-  if (w.n < 0) return nullptr;
+  if (w.n < 0) return not_ordinary();
   std::vector<sga_span_record> rows;
   rows.reserve((size_t)w.n);
   int64_t spans = 0;

@@ -37,3 +37,18 @@ def test_an_error_while_the_norm_is_read_raises():
             assert "meta" in str(e), e
         print("done")
         """)
+
+
+def test_an_iterator_of_records_is_left_for_the_general_route():
+    """What is not a list or a tuple is walked once, by the general route: had the
+    native walk used it up, that route would see a step without records."""
+    _run("""
+        host.bind(object, addr, addr, addr, addr)
+        for call in (lambda r: host.commit(r, False, -1, 1.0, False, False, 1.0, 1.0, False, 0),
+                     lambda r: host.commit_compact(r, {}, None, True, 1.0, False, 1.0, False, 0),
+                     lambda r: host.norm_table(r, True)):
+            records = iter([object(), object()])
+            assert call(records) is False
+            assert len(list(records)) == 2
+        print("done")
+        """)
