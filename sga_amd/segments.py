@@ -51,14 +51,11 @@ class SegmentTable:
         for i, r in enumerate(rows):
             groups.setdefault((r["b1"], r["b2"]), []).append(i)
         self._groups = [(b, slice(None) if len(groups) == 1 else np.array(at)) for b, at in groups.items()]
-        self._last_lr = None
 
     def refresh(self, lr, count, bias_correction=True):
         """Learning rates (one float, or one per row) and the bias corrections of
         step ``count``, on the current stream."""
-        if lr != self._last_lr:
-            self._lr[:] = lr
-            self._last_lr = lr
+        self._lr[:] = lr
         for (b1, b2), at in self._groups:
             self._bc1[at] = 1.0 - b1 ** count if bias_correction else 1.0
             self._bc2[at] = 1.0 - b2 ** count if bias_correction else 1.0
