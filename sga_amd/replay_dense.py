@@ -65,6 +65,7 @@ class DenseReplay:
             raise ValueError("gradient length does not match the shard")
         coef_dense, flag = coef_dense_for(gmeta)
         count = self.t0 + self.si + 1
+        self._seg_table.follow(self.entries)          # callers may change them between steps
         self._seg_table.refresh(lr_by_group(gmeta, self.entries), count, self.optimizer == "adamw")
         st = L.stream()
         L.call("sga_dense_replay_step", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),

@@ -190,6 +190,7 @@ class ReplayGroup:
                 if bnd[ci] and c.fold and not self.res_zero[ci]:
                     L.call("sga_div_inplace", C.c_void_p(self.state[ci].base("res")), N,
                            L.f32(float(c.T)), 1, st)
+        self._seg_table.follow(self.entries)         # callers may change them between steps
         self._seg_table.refresh([float(lr(e)) for e in self.entries] if callable(lr) else float(lr), count)
         self._fill_cfgs(bnd, {})
         gd = L.dtype_code(g)

@@ -1,8 +1,9 @@
 """Device tables of per-tensor hyper-parameters, laid out once per bucket or
-shard; a step only rewrites the learning rates and the bias corrections
+shard; a step rewrites the learning rates and the bias corrections
 (``sga_segments_refresh``: the values travel in the kernel arguments, nothing
-is staged or waited for)."""
+is staged or waited for), and the whole table only where its rows changed."""
 import ctypes as C
+from operator import itemgetter
 
 import numpy as np
 import torch
@@ -18,10 +19,11 @@ class ReplaySegment(C.Structure):
                 ("wdf", C.c_float)]
 
 
+_HYPER = itemgetter("b1", "b2", "eps", "wd")
 _SEGMENT, _REPLAY_SEGMENT = np.dtype(L.Segment), np.dtype(ReplaySegment)
 
 
-def _device_table(dtype, rows, start, device):
+def _host_table(dtype, rows, start):
     t = np.zeros(len(rows), dtype=dtype)
     t["start"], t["n"] = [r[start] for r in rows], [r["n"] for r in rows]
     # numpy rounds a Python float to nearest fp32, like a store into a C float
@@ -31,7 +33,7 @@ def _device_table(dtype, rows, start, device):
         t[name] = values
     if dtype is _REPLAY_SEGMENT:
         t["wdf"] = [r["wd"] for r in rows]
-    return torch.from_numpy(t.view(np.uint8)).to(device)
+    return torch.from_numpy(t.view(np.uint8))
 
 
 class SegmentTable:
@@ -41,16 +43,34 @@ class SegmentTable:
 
     def __init__(self, rows, device, start="start", segs=True, rsegs=False):
         self.count = len(rows)
-        self.segs = _device_table(_SEGMENT, rows, start, device) if segs else None
-        self.rsegs = _device_table(_REPLAY_SEGMENT, rows, start, device) if rsegs else None
+        self._start = start
+        self.segs = _host_table(_SEGMENT, rows, start).to(device) if segs else None
+        self.rsegs = _host_table(_REPLAY_SEGMENT, rows, start).to(device) if rsegs else None
         self._lr, self._bc1, self._bc2 = (np.zeros(self.count, dtype=d) for d in ("f8", "f4", "f4"))
         self._args = (None if self.segs is None else self.segs.data_ptr(),
                       None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
                       self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
+        self._hyper = list(map(_HYPER, rows))
+        self._group(self._hyper)
+
+    def _group(self, betas):
+        """Rows of equal betas share their bias corrections."""
         groups = {}
-        for i, r in enumerate(rows):
-            groups.setdefault((r["b1"], r["b2"]), []).append(i)
+        for i, b in enumerate(betas):
+            groups.setdefault(b[:2], []).append(i)
         self._groups = [(b, slice(None) if len(groups) == 1 else np.array(at)) for b, at in groups.items()]
+
+    def follow(self, rows):
+        """Takes over the betas, eps and weight decay that ``rows`` hold now (4 us
+        for 50 rows that did not change; the copy of changed ones waits)."""
+        hyper = list(map(_HYPER, rows))
+        if hyper == self._hyper:
+            return
+        for t, dtype in ((self.segs, _SEGMENT), (self.rsegs, _REPLAY_SEGMENT)):
+            if t is not None:
+                t.copy_(_host_table(dtype, rows, self._start))
+        self._hyper = hyper
+        self._group(hyper)
 
     def refresh(self, lr, count, bias_correction=True):
         """Learning rates (one float, or one per row) and the bias corrections of

@@ -41,3 +41,34 @@ def test_a_list_of_learning_rates_changed_in_place(dev):
     lr[1] = 5e-4
     table.refresh(lr, 2)
     assert [r.lr for r in _table(table.segs, L.Segment)] == [L.f32(1e-3), L.f32(5e-4)]
+
+
+@pytest.mark.parametrize("kind", ["group", "dense"])
+def test_replay_follows_its_entries(dev, kind):
+    from sga_amd import _lib as L
+    from sga_amd.replay_dense import DenseReplay
+    from sga_amd.replay_group import Config, ReplayGroup
+    from sga_amd.segments import ReplaySegment
+    rows, (w, m, v) = _rows("a"), _state(dev)
+    meta = {"clip_grad": 1.0, "grad_norm": float("nan"), "lr": 1e-4 if kind == "group" else [1e-4]}
+    if kind == "group":
+        rep = ReplayGroup(rows, w, m, v, [torch.ones(N, dtype=torch.uint8, device=dev)],
+                          [Config("abs_g", 10.0, 4)], 3, 4)
+        step = lambda i: rep.step(_flat(dev, i, 1e-2), meta)                  # noqa: E731
+    else:
+        rep = DenseReplay(rows, w, m, v, 3)
+        step = lambda i: rep.step(i, _flat(dev, i, 1e-2), meta)               # noqa: E731
+    step(0)
+    rows[0].update(wd=0.3, eps=1e-6)
+    rows[1].update(b1=0.8, b2=0.99)
+    step(1)
+    for t, row_type in ((rep._seg_table.rsegs, ReplaySegment), (rep._seg_table.segs, L.Segment)):
+        if t is None:
+            continue
+        for got, r in zip(_table(t, row_type), rows):
+            assert (got.start, got.n) == (r["a"], r["n"])
+            want = (r["b1"], 1 - r["b1"], r["b2"], 1 - r["b2"], r["eps"], 1 - r["b1"] ** 5, 1 - r["b2"] ** 5)
+            assert (got.beta1, got.om1, got.beta2, got.om2, got.eps, got.bc1, got.bc2) == \
+                tuple(L.f32(x) for x in want)
+            assert got.wd == (r["wd"] if row_type is ReplaySegment else L.f32(r["wd"]))
+            assert row_type is L.Segment or got.wdf == L.f32(r["wd"])
