@@ -66,7 +66,8 @@ class FusedSparseStep:
     def _upload_segments(self, step):
         if self._seg_step == step:
             return
-        # callers may retune lr between steps
+        # callers may retune lr between steps; of the betas only the bias corrections follow
+        self._seg_table.follow_betas(self.segments)
         self._seg_table.refresh([s["lr"] for s in self.segments], step)
         self._seg_step = step
 

@@ -20,6 +20,7 @@ class ReplaySegment(C.Structure):
 
 
 _HYPER = itemgetter("b1", "b2", "eps", "wd")
+_BETAS = itemgetter("b1", "b2")
 _SEGMENT, _REPLAY_SEGMENT = np.dtype(L.Segment), np.dtype(ReplaySegment)
 
 
@@ -51,13 +52,18 @@ class SegmentTable:
                       None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
                       self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
         self._hyper = list(map(_HYPER, rows))
-        self._group(self._hyper)
+        self._betas = None
+        self.follow_betas(rows)
 
-    def _group(self, betas):
-        """Rows of equal betas share their bias corrections."""
-        groups = {}
+    def follow_betas(self, rows):
+        """Bias corrections are those of the betas that ``rows`` hold now; rows of equal
+        betas share them."""
+        betas = list(map(_BETAS, rows))
+        if betas == self._betas:
+            return
+        self._betas, groups = betas, {}
         for i, b in enumerate(betas):
-            groups.setdefault(b[:2], []).append(i)
+            groups.setdefault(b, []).append(i)
         self._groups = [(b, slice(None) if len(groups) == 1 else np.array(at)) for b, at in groups.items()]
 
     def follow(self, rows):
@@ -70,7 +76,7 @@ class SegmentTable:
             if t is not None:
                 t.copy_(_host_table(dtype, rows, self._start))
         self._hyper = hyper
-        self._group(hyper)
+        self.follow_betas(rows)
 
     def refresh(self, lr, count, bias_correction=True):
         """Learning rates (one float, or one per row) and the bias corrections of

@@ -72,3 +72,17 @@ def test_replay_follows_its_entries(dev, kind):
                 tuple(L.f32(x) for x in want)
             assert got.wd == (r["wd"] if row_type is ReplaySegment else L.f32(r["wd"]))
             assert row_type is L.Segment or got.wdf == L.f32(r["wd"])
+
+
+def test_fused_step_takes_the_bias_corrections_of_its_segments(dev):
+    """Learning rates and bias corrections follow the segments; betas, eps and weight
+    decay are those the stepper was made with."""
+    from sga_amd import _lib as L
+    rows = _rows("start")
+    fs, step = _stepper(dev, rows)
+    step(1)
+    rows[1].update(lr=5e-4, b1=0.8, b2=0.99, wd=0.7)
+    step(2)
+    got = _table(fs._seg_dev, L.Segment)[1]
+    assert (got.lr, got.bc1, got.bc2) == (L.f32(5e-4), L.f32(1 - 0.8 ** 2), L.f32(1 - 0.99 ** 2))
+    assert (got.beta1, got.beta2, got.wd) == (L.f32(0.9), L.f32(0.95), 0.0)
