@@ -52,7 +52,6 @@ class FusedSparseStep:
         self._seg_table = SegmentTable(segments, device)
         self._seg_dev = self._seg_table.segs
         self._seg_step = None
-        self._views = (None, None, None)
         self._ws2 = None          # second workspace of the single-sweep step, on first use
         self._calls = 0
 
@@ -125,13 +124,7 @@ class FusedSparseStep:
         else:
             L.call(name, *head, 1 if fast else 0, flags, L.f32(interval), L.ptr(result),
                    L.ptr(self.ws), self.ws_bytes, L.stream())
-        return self._pack_views(k)
-
-    def _pack_views(self, k):
-        """(idx[:k], values[:k]); the views of the last k are kept (1 us each to make)."""
-        if self._views[0] != k:
-            self._views = (k, self.idx[:k], self.values[:k])
-        return self._views[1:]
+        return self.idx[:k], self.values[:k]
 
     def step(self, g, resid, p, m, v, step, k=None, ratio_percent=None,
              score="abs_g", factor=1.0, coeff=1.0, fast=True, optimizer="adamw", fold=False,
@@ -269,7 +262,7 @@ def fused_step_multi(steppers, grads, resids, ps, ms, vs, step, ks=None, ratio_p
         e.ws, e.ws_bytes = fs.ws.data_ptr(), fs.ws_bytes
     L.call("sga_fused_sparse_step_multi", table, nb, gd, SCORE_MAP[score], vd, L.f32(factor),
            L.f32(coeff), 1 if fast else 0, flags, L.f32(interval), L.stream())
-    return [fs._pack_views(k) for fs, k in zip(steppers, ks)]
+    return [(fs.idx[:k], fs.values[:k]) for fs, k in zip(steppers, ks)]
 
 
 class PackedState:

@@ -86,3 +86,14 @@ def test_fused_step_takes_the_bias_corrections_of_its_segments(dev):
     got = _table(fs._seg_dev, L.Segment)[1]
     assert (got.lr, got.bc1, got.bc2) == (L.f32(5e-4), L.f32(1 - 0.8 ** 2), L.f32(1 - 0.99 ** 2))
     assert (got.beta1, got.beta2, got.wd) == (L.f32(0.9), L.f32(0.95), 0.0)
+
+
+def test_the_returned_pack_is_of_the_present_buffers(dev):
+    fs, step = _stepper(dev, _rows("start"))
+    idx, val = step(1)
+    idx.resize_(10)                                     # the caller's own view, done with as it likes
+    assert step(2)[0].shape == (50,)
+    fs.idx, fs.values = torch.empty_like(fs.idx), torch.empty_like(fs.values)
+    idx, val = step(3)
+    assert (idx.data_ptr(), val.data_ptr()) == (fs.idx.data_ptr(), fs.values.data_ptr())
+    assert idx.shape == val.shape == (50,) and bool((idx[1:] > idx[:-1]).all())
