@@ -239,7 +239,7 @@ _F32 = struct.Struct("f")
 
 def f32(x):
     """Round a Python float to fp32 (nearest-even), back as a Python float."""
-    return _F32.unpack(_F32.pack(x))[0]
+    return _F32.unpack(_F32.pack(float(x)))[0]
 
 
 def require_dev(*tensors):

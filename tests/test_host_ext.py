@@ -52,3 +52,11 @@ def test_an_iterator_of_records_is_left_for_the_general_route():
             assert len(list(records)) == 2
         print("done")
         """)
+
+
+def test_scalars_are_taken_in_every_form_that_float_takes():
+    import numpy as np
+    import torch
+    from sga_amd import _lib as L
+    for x in ("0.1", 0.1, np.float64(0.1), np.float32(0.1), torch.tensor(0.1), torch.tensor([0.1])):
+        assert L.f32(x) == float(np.float32(0.1))
