@@ -233,7 +233,7 @@ PyObject* commit_compact(PyObject*, PyObject* args) {
   PyObject* last = nullptr;                            // the bucket looked up last (borrowed)
   const int32_t *idx = nullptr, *table = nullptr;
   const void* vals = nullptr;
-  int64_t k_total = 0, n_table = 0;
+  int64_t k_total = 0, n_table = -1;                   // n_table < 0: no table to search by
   int dtype = -1;
   for (Py_ssize_t i = 0; i < w.n; ++i) {
     PyObject* rec = w.at(i);
@@ -262,7 +262,7 @@ PyObject* commit_compact(PyObject*, PyObject* args) {
       vals = tv.data_ptr();
       k_total = ti.numel();
       table = nullptr;
-      n_table = 0;
+      n_table = -1;
       if (use_table && dt.o && dt.o != Py_None) {
         if (!THPVariable_Check(dt.o)) return not_ordinary();
         const at::Tensor& tt = THPVariable_Unpack(dt.o);
@@ -277,12 +277,12 @@ PyObject* commit_compact(PyObject*, PyObject* args) {
     }
     if (c.n == 0) continue;
     const int64_t lim = (int64_t)1 << 31;
-    if (k_total + 1024 >= lim || start + c.n + 1024 >= lim || (table && n_table < ((start + c.n - 1) >> 10) + 2))
+    if (k_total + 1024 >= lim || start + c.n + 1024 >= lim || (n_table >= 0 && n_table < ((start + c.n - 1) >> 10) + 2))
       return not_ordinary();
     sga_gcc_record e = {};
     e.p = c.p; e.g = c.g; e.m = c.m; e.v = c.v;
     e.idx = idx; e.values = vals; e.table = table;
-    e.rec_start = start; e.n = c.n; e.k_total = k_total; e.n_table = n_table; e.first_span = spans;
+    e.rec_start = start; e.n = c.n; e.k_total = k_total; e.n_table = table ? n_table : 0; e.first_span = spans;
     hyper_into(e, c, adams);
     e.flags = (coeff != 1.0 ? SGA_GC_APPLY_COEFF : 0) | (fold ? SGA_GC_FOLD : 0) | (adams ? SGA_GC_ADAMS : 0);
     rows.push_back(e);

@@ -86,6 +86,26 @@ def test_commit_tables(dev, count, phase):
         assert torch.equal(t[k], ref[k]), k
 
 
+@pytest.mark.parametrize("entries", [0, 1])
+def test_a_directory_table_too_short_is_refused(dev, entries):
+    from sga_amd import config
+    from sga_amd.adamw import OptContext, SgaAdamW
+    from sga_amd.support import compact_mask_u8
+    config.set_args(SimpleNamespace(sga_score="update", sga_optimizer_residual_mean=False,
+                                    sga_optimizer_compact_search="table",
+                                    sga_optimizer_full_sync_inactive_lr_scale=1.0))
+    recs, t, mask = _records(dev, [4097], 3, True)
+    idx = compact_mask_u8(mask)
+    bucket = SimpleNamespace(idx=idx, dir_table=torch.zeros(entries, dtype=torch.int32, device=dev))
+    ctx = OptContext(recs, "sparse", bucket_states=[recs[0].bucket_state],
+                     compact_values={id(recs[0].bucket_state): t["g"][idx.long()].contiguous()},
+                     support=SimpleNamespace(buckets=[bucket]))
+    before = t["p"].clone()
+    with pytest.raises(AssertionError, match="dir_table"):
+        SgaAdamW().sparse_step(ctx)
+    assert torch.equal(t["p"], before)
+
+
 # a launch writes 64 or 240 rows: one short of, at and past both, and several launches
 @pytest.mark.parametrize("count", [1, 63, 64, 65, 239, 240, 241, 500])
 def test_segment_table_refresh(dev, count):
