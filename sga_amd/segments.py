@@ -3,7 +3,7 @@ shard; a step rewrites the learning rates and the bias corrections
 (``sga_segments_refresh``: the values travel in the kernel arguments, nothing
 is staged or waited for), and the whole table only where its rows changed."""
 import ctypes as C
-from operator import itemgetter
+from operator import index, itemgetter
 
 import numpy as np
 import torch
@@ -26,14 +26,16 @@ _SEGMENT, _REPLAY_SEGMENT = np.dtype(L.Segment), np.dtype(ReplaySegment)
 
 def _host_table(dtype, rows, start):
     t = np.zeros(len(rows), dtype=dtype)
-    t["start"], t["n"] = [r[start] for r in rows], [r["n"] for r in rows]
-    # numpy rounds a Python float to nearest fp32, like a store into a C float
+    t["start"], t["n"] = [index(r[start]) for r in rows], [index(r["n"]) for r in rows]
     for name, values in (("beta1", [r["b1"] for r in rows]), ("om1", [1.0 - r["b1"] for r in rows]),
                          ("beta2", [r["b2"] for r in rows]), ("om2", [1.0 - r["b2"] for r in rows]),
-                         ("eps", [r["eps"] for r in rows]), ("wd", [r["wd"] for r in rows])):
-        t[name] = values
+                         ("eps", [r["eps"] for r in rows])):
+        t[name] = list(map(L.f32, values))
     if dtype is _REPLAY_SEGMENT:
-        t["wdf"] = [r["wd"] for r in rows]
+        t["wd"] = [float(r["wd"]) for r in rows]
+        t["wdf"] = [L.f32(r["wd"]) for r in rows]
+    else:
+        t["wd"] = [L.f32(r["wd"]) for r in rows]
     return torch.from_numpy(t.view(np.uint8))
 
 
@@ -79,10 +81,10 @@ class SegmentTable:
         self.follow_betas(rows)
 
     def refresh(self, lr, count, bias_correction=True):
-        """Learning rates (one float, or one per row) and the bias corrections of
+        """Learning rates (one number, or one per row) and the bias corrections of
         step ``count``, on the current stream."""
-        self._lr[:] = lr
+        self._lr[:] = list(map(float, lr)) if isinstance(lr, list) else float(lr)
         for (b1, b2), at in self._groups:
-            self._bc1[at] = 1.0 - b1 ** count if bias_correction else 1.0
-            self._bc2[at] = 1.0 - b2 ** count if bias_correction else 1.0
+            self._bc1[at] = L.f32(1.0 - b1 ** count) if bias_correction else 1.0
+            self._bc2[at] = L.f32(1.0 - b2 ** count) if bias_correction else 1.0
         L.call("sga_segments_refresh", *self._args, L.stream())

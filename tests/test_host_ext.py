@@ -4,6 +4,8 @@ import subprocess
 import sys
 import textwrap
 
+import pytest
+
 from sga_amd import build as B
 
 
@@ -60,3 +62,31 @@ def test_scalars_are_taken_in_every_form_that_float_takes():
     from sga_amd import _lib as L
     for x in ("0.1", 0.1, np.float64(0.1), np.float32(0.1), torch.tensor(0.1), torch.tensor([0.1])):
         assert L.f32(x) == float(np.float32(0.1))
+
+
+@pytest.mark.parametrize("replay", [False, True])
+def test_segment_tables_take_and_refuse_what_struct_fields_do(monkeypatch, replay):
+    """Text that holds a number (learning rates and eps of a configuration file), numpy
+    scalars and one-element tensors are numbers; a fractional offset is no offset, and
+    a number beyond fp32 no fp32."""
+    import numpy as np
+    import torch
+    from sga_amd import _lib as L
+    from sga_amd.segments import ReplaySegment, SegmentTable
+    monkeypatch.setattr(L, "call", lambda *a: None)
+    monkeypatch.setattr(L, "stream", lambda: 0)
+    kw = dict(segs=not replay, rsegs=replay)
+    rows = [dict(start=0, n=np.int64(5), b1=np.float64(0.9), b2=torch.tensor(0.95, dtype=torch.float64),
+                 eps="1e-8", wd="0.1"),
+            dict(start=5, n=7, b1=0.9, b2=0.95, eps=1e-8, wd=0.1)]
+    t = SegmentTable(rows, "cpu", **kw)
+    row_type = ReplaySegment if replay else L.Segment
+    a, b = (row_type * 2).from_buffer_copy(bytes((t.rsegs if replay else t.segs).numpy()))
+    assert (a.start, a.n, b.start, b.n) == (0, 5, 5, 7)
+    for name in [f[0] for f in row_type._fields_][2:]:
+        assert getattr(a, name) == getattr(b, name), name
+    t.refresh(["1e-3", torch.tensor(2e-3, dtype=torch.float64)], 3)
+    assert t._lr.tolist() == [1e-3, 2e-3] and t._bc2[0] == t._bc2[1] == np.float32(1 - 0.95 ** 3)
+    for key, value, error in (("start", 0.5, TypeError), ("n", 7.0, TypeError), ("eps", 1e39, OverflowError)):
+        with pytest.raises(error):
+            SegmentTable([dict(rows[1], **{key: value})], "cpu", **kw)
