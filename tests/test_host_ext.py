@@ -67,8 +67,7 @@ def test_scalars_are_taken_in_every_form_that_float_takes():
 @pytest.mark.parametrize("replay", [False, True])
 def test_segment_tables_take_and_refuse_what_struct_fields_do(monkeypatch, replay):
     """Text that holds a number (learning rates and eps of a configuration file), numpy
-    scalars and one-element tensors are numbers; a fractional offset is no offset, and
-    a number beyond fp32 no fp32."""
+    scalars and one-element tensors are numbers; a fractional offset is no offset."""
     import numpy as np
     import torch
     from sga_amd import _lib as L
@@ -87,6 +86,6 @@ def test_segment_tables_take_and_refuse_what_struct_fields_do(monkeypatch, repla
         assert getattr(a, name) == getattr(b, name), name
     t.refresh(["1e-3", torch.tensor(2e-3, dtype=torch.float64)], 3)
     assert t._lr.tolist() == [1e-3, 2e-3] and t._bc2[0] == t._bc2[1] == np.float32(1 - 0.95 ** 3)
-    for key, value, error in (("start", 0.5, TypeError), ("n", 7.0, TypeError), ("eps", 1e39, OverflowError)):
-        with pytest.raises(error):
+    for key, value in (("start", 0.5), ("n", 7.0)):
+        with pytest.raises(TypeError):
             SegmentTable([dict(rows[1], **{key: value})], "cpu", **kw)
