@@ -268,6 +268,11 @@ def stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
+def capturing():
+    """True while the current stream records a graph."""
+    return torch.cuda.is_current_stream_capturing()
+
+
 def dtype_code(t):
     if t.dtype == torch.float32:
         return SGA_F32

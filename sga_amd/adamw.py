@@ -377,9 +377,12 @@ class SgaAdamW:
         # every record of the step in ONE launch (the reference issues one kernel
         # per record, adamw.py:869-905); per-record knobs as in that loop.  The
         # records are walked in native code; anything out of the ordinary takes
-        # the general loop below, which also raises the refusals.
-        rc = L.host().commit(ctx.records, use_mask, SCORE_MAP[emit_score] if emit_score else -1,
-                             coeff, clear, fold, interval, inactive_lr_scale, self._adams, L.stream())
+        # the general loop below, which also raises the refusals.  So does a
+        # graph capture: a replay reads the staged table again, and the native
+        # walk gives its staging block back when the call is over.
+        rc = not L.capturing() and L.host().commit(
+            ctx.records, use_mask, SCORE_MAP[emit_score] if emit_score else -1,
+            coeff, clear, fold, interval, inactive_lr_scale, self._adams, L.stream())
         if rc is not False:
             L.check(rc, "sga_adamw_grad_correct_multi")
             return
@@ -400,9 +403,9 @@ class SgaAdamW:
     def _records_pass_compact(self, ctx, coeff=1.0, fold=False, interval=1.0):
         # records of buckets with communicated values: one merge-join launch;
         # the others (no support in their bucket): one plain-commit launch
-        rc = L.host().commit_compact(ctx.records, ctx.compact_values, ctx.support,
-                                     self.compact_search == "table", coeff, fold, interval,
-                                     self._adams, L.stream())
+        rc = not L.capturing() and L.host().commit_compact(
+            ctx.records, ctx.compact_values, ctx.support, self.compact_search == "table", coeff,
+            fold, interval, self._adams, L.stream())
         if rc is not False:
             L.check(rc, "sga_adamw_grad_correct_compact_multi")
             return

@@ -64,7 +64,7 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
     mask-less records; otherwise it is returned for the commit kernel's
     in-register multiply (``engine.py:1172-1217``).
     """
-    if not compact_values or was_full:
+    if (not compact_values or was_full) and not L.capturing():
         done = _clip_one_launch(records, clip_grad, was_full, trace_dumps)
         if done is not None:
             return done

@@ -14,7 +14,8 @@
 // Tables travel through torch's caching allocators: a pinned block and a device
 // block per call, both returned when the call is over, ordered on the current
 // stream by torch itself -- nothing here outlives a call or is shared between
-// threads or streams.
+// threads or streams.  A captured graph would read the pinned block again at its
+// replay: the callers keep captures away from here.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 

@@ -86,6 +86,50 @@ def test_commit_tables(dev, count, phase):
         assert torch.equal(t[k], ref[k]), k
 
 
+@pytest.mark.parametrize("phase", ["sparse", "compact"])
+def test_a_captured_commit_keeps_its_table(dev, phase):
+    """Replays read the staged table again: nothing that the program stages between them may get there."""
+    from sga_amd import config
+    from sga_amd import adamw as A
+    from sga_amd.support import compact_mask_u8
+    config.set_args(SimpleNamespace(sga_score="update", sga_optimizer_residual_mean=False,
+                                    sga_optimizer_compact_search="table",
+                                    sga_optimizer_full_sync_inactive_lr_scale=1.0))
+    sizes = [4097, 12_289, 3]
+    recs, t, mask = _records(dev, sizes, 9, True)
+    refs, ref, _ = _records(dev, sizes, 9, True)
+    kw = {}
+    if phase == "compact":
+        idx = compact_mask_u8(mask)
+        vals = t["g"][idx.long()].contiguous()
+        table = A.build_dir_table(idx, sum(sizes))
+        kw = dict(support=SimpleNamespace(buckets=[SimpleNamespace(idx=idx, dir_table=table)]))
+    opt = A.SgaAdamW()
+
+    def step(rs):
+        if kw:
+            kw["compact_values"] = {id(rs[0].bucket_state): vals}
+        opt.sparse_step(A.OptContext(rs, "sparse", bucket_states=[rs[0].bucket_state], apply_coeff=0.5, **kw))
+    warm, _, _ = _records(dev, sizes, 10, True)         # the general route lays its staging out once
+    walk, A.L.capturing = A.L.capturing, lambda: True
+    try:
+        step(warm)
+    finally:
+        A.L.capturing = walk
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(recs)
+    for turn in range(3):
+        staged = [torch.full((1 << b,), 0, dtype=torch.uint8, pin_memory=True) for b in range(7, 14)]
+        graph.replay()
+        torch.cuda.synchronize()
+        step(refs)
+        for k in t:
+            assert torch.equal(t[k], ref[k]), (k, turn)
+        del staged
+
+
 @pytest.mark.parametrize("entries", [0, 1])
 def test_a_directory_table_too_short_is_refused(dev, entries):
     from sga_amd import config
