@@ -55,7 +55,10 @@ struct SelState {
   uint32_t ties_left;   // the settlement has left the ties to k_tail
   uint32_t tail_ticket; // k_tail: items handed out, and ...
   uint32_t tail_done;   // ... finished
-  uint32_t pad_[29];
+  uint32_t finish_ticket; // k_small_finish: workgroups that have begun; the first one judges the bracket ...
+  uint32_t verdict;     // ... 1: it holds the k-th key, 2: all of them go over the data again
+  uint32_t redo_step;   // passes of that which are done
+  uint32_t pad_[26];
 };
 static_assert(sizeof(SelState) == 256, "SelState layout");
 
@@ -537,17 +540,15 @@ __global__ __launch_bounds__(kBlock) void k_level_scan(ChainJobs jobs) {
 }
 
 // Per-chunk (1024 elements, one wave) counts of keys above / equal to the
-// threshold.
+// threshold, by wave `wave` of `wstride`.
 template <class Src>
 __device__ __forceinline__ void tile_count_body(Src& src, const ChainJob& J, uint32_t T, int64_t tile_base,
-                                                uint32_t blk, uint32_t n_blk) {
+                                                int64_t wave, int64_t wstride) {
   const int64_t n = J.n;
   uint32_t* tile_gt = J.tile_gt;
   uint32_t* tile_eq = J.tile_eq;
   const int64_t n_chunks = cdiv64(n, kChunk);
-  const int64_t wstride = (int64_t)n_blk * kChunksPerBlock;
-  for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks;
-       c += wstride) {
+  for (int64_t c = wave; c < n_chunks; c += wstride) {
     uint32_t cg = 0, ce = 0;
     if (src.vec && (c + 1) * kChunk <= n) {
       uint32_t key[kChunkIters][4];
@@ -586,7 +587,8 @@ __global__ __launch_bounds__(kBlock) void k_tile_count(SrcPack<Src> srcs, ChainJ
   const ChainJob& J = jobs.j[blockIdx.y];
   if (J.st->skip) return;
   Src src = srcs.s[blockIdx.y];
-  tile_count_body(src, J, J.st->thresh_bits, tile_base, blockIdx.x, gridDim.x);
+  tile_count_body(src, J, J.st->thresh_bits, tile_base, (int64_t)blockIdx.x * kChunksPerBlock + wave_id(),
+                  (int64_t)gridDim.x * kChunksPerBlock);
 }
 
 // Tile scan of a staged select, kernel 1: per-workgroup totals of (gt, eq).
@@ -2034,7 +2036,8 @@ __global__ __launch_bounds__(kBlock) void k_tail(SrcPack<Src> srcs, ChainJobs jo
       if (step == 0) tail_level<Src, 0>(src, J, blk, G, s);
       else if (step == 1) tail_level<Src, 1>(src, J, blk, G, s);
       else if (step == 2) tail_level<Src, 2>(src, J, blk, G, s);
-      else tile_count_body(src, J, ld_agent(&st->thresh_bits), 0, blk, G);
+      else tile_count_body(src, J, ld_agent(&st->thresh_bits), 0, (int64_t)blk * kChunksPerBlock + wave_id(),
+                           (int64_t)G * kChunksPerBlock);
     } else if (t < at_ties) {
       tail_scan(J, t - first, n_scan, s);
     } else if (t < at_write) {

@@ -18,8 +18,8 @@
 //   select_topk_flat, 3 M scores, 1 %              168 -> 69
 // (4.2 M: sample 2.5, pick 8, sweep 6, finish 19, final sweep 30 us).
 //
-// The result is exact for any sample: a bracket that misses the k-th key is redone by the finishing
-// workgroup over the data itself.
+// The result is exact for any sample: where the bracket misses the k-th key the finishing launch goes
+// over the data itself, with all of its workgroups (small_redo).
 #pragma once
 #include "select_impl.hpp"
 
@@ -159,16 +159,96 @@ struct SmallList {
 };
 static_assert(kSmallHead * kWave * kVec <= kBlockSpan, "the head never reaches past a segment");
 
+// A bracket that missed: the radix descent and the chunk counts over the data itself, as items of one
+// queue that every workgroup of the launch works on (the way of k_tail: whoever waits holds a later
+// ticket than those it waits for, so any number of resident workgroups will do).  True in the workgroup
+// that finished the last item: it finds the threshold in the state and the counts per chunk in tile_gt /
+// tile_eq.
+// The margin is five sigma of independent keys, but the sample is drawn by quads: scores that neighbours
+// share miss about once in a hundred times.  One workgroup alone took 5.9 ms for such a select of 8.4 M
+// coordinates, the launch takes 0.21 (a bracket that holds: 0.10).
+constexpr int kRedoGroups = 64;                       // at most; one per kRedoTiles chunks
+constexpr int kRedoTiles = 32;
+template <class Src>
+__device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t* s_hist, WideScratch& s_scan,
+                                           uint32_t* s_word) {
+  SelState* st = J.st;
+  const int64_t n = J.n;
+  const uint32_t G = gridDim.x;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) *s_word = atomicAdd(&st->tail_ticket, 1u);
+    __syncthreads();
+    const uint32_t t = *s_word, step = t / G, blk = t % G;
+    if (step > 3) return false;
+    if (step) {
+      if (threadIdx.x == 0)
+        while (ld_agent(&st->redo_step) < step) __builtin_amdgcn_s_sleep(16);
+      __syncthreads();
+    }
+    const uint32_t prefix = step ? ld_agent(&st->prefix) : 0u;
+    const int shift = step == 0 ? kL0Shift : step == 1 ? kL1Shift : 0;
+    const int above = step == 0 ? 31 : step == 1 ? kL0Shift : kL1Shift, bits = above - shift;
+    uint32_t* gh = J.hist + (step == 0 ? 0 : step == 1 ? kBinsBig : 2 * kBinsBig);
+    if (step == 3) {
+      tile_count_body(src, J, prefix, 0, (int64_t)blk * kWideWaves + wave_id(), (int64_t)G * kWideWaves);
+    } else {
+      reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
+      __syncthreads();
+      constexpr int U = 4;                            // quads in flight per thread
+      constexpr int64_t kSlab = (int64_t)kWide * kVec;
+      for (int64_t base = (int64_t)blk * kSlab * U; base < n; base += (int64_t)G * kSlab * U) {
+        uint32_t key[U][4];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t b = base + u * kSlab, i = b + (int64_t)threadIdx.x * kVec;
+          key[u][0] = key[u][1] = key[u][2] = key[u][3] = 0u;
+          if (src.vec && b + kSlab <= n) src.template load<true>(i, n, key[u]);
+          else if (i < n) src.template load<false>(i, n, key[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t i = base + u * kSlab + (int64_t)threadIdx.x * kVec;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            wide_hist_add(s_hist, (key[u][e] >> shift) & ((1u << bits) - 1u),
+                          i + e < n && (key[u][e] >> above) == prefix);
+        }
+      }
+      __syncthreads();
+      for (int b = threadIdx.x; b < (1 << bits); b += kWide)
+        if (const uint32_t c = s_hist[b]) atomicAdd(&gh[b], c);
+    }
+    wait_landed();
+    if (threadIdx.x == 0) *s_word = atomicAdd(&st->tail_done, 1u) + 1u;
+    __syncthreads();
+    if (*s_word != (step + 1u) * G) continue;
+    if (step == 3) return true;
+    for (int b = threadIdx.x; b < kWideBins; b += kWide) s_hist[b] = b < (1 << bits) ? ld_agent(&gh[b]) : 0u;
+    const uint32_t want[1] = {step ? ld_agent(&st->krem) : J.k};
+    __syncthreads();
+    RankHit h[1];
+    wide_find_rank<1>(s_hist, want, s_scan, (int)(step & 1u), h);
+    if (threadIdx.x == 0) {
+      st_agent(&st->prefix, (prefix << bits) | h[0].bin);
+      st_agent(&st->krem, want[0] - h[0].above);
+      st_agent(&st->n_eq, h[0].count);
+    }
+    wait_landed();
+    if (threadIdx.x == 0) st_agent(&st->redo_step, step + 1u);
+  }
+}
+
 template <class Src>
 __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs) {
   __shared__ __align__(16) uint32_t s_hist[kBinsBig];
   __shared__ __align__(16) uint32_t s_tile[kSmallTiles];          // above | ties << 16, at most 1024 each
   __shared__ __align__(16) uint32_t s_key[kWideList];
   __shared__ uint32_t s_idx[kWideList];
-  __shared__ uint32_t s_seg[kWideWaves], s_cnt, s_out[3];
+  __shared__ uint32_t s_seg[kWideWaves], s_cnt, s_out[3], s_word;
   __shared__ WideScratch s_scan;
   const ChainJob& J = jobs.j[blockIdx.y];
-  SelState* __restrict__ st = J.st;
+  SelState* st = J.st;
   const int64_t n = J.n;
   const int nt = (int)J.n_tiles;
   const uint32_t k = J.k, T_LO = st->t_lo, T_HI = st->t_hi;
@@ -193,13 +273,30 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
   if (threadIdx.x < kWideWaves)
     s_seg[threadIdx.x] = threadIdx.x < geo.segs ? J.seg_cnt[threadIdx.x * kSmallSegStride] : 0u;
-  if (threadIdx.x == 0) s_cnt = 0u;
+  if (threadIdx.x == 0) {
+    s_cnt = 0u;
+    s_word = gridDim.x > 1 ? atomicAdd(&st->finish_ticket, 1u) : 0u;
+  }
+  // The first workgroup to begin judges the bracket and usually does all the rest; the others wait for its
+  // word (it is running, so they need not fit the chip beside it) and go.
+  __syncthreads();
+  const bool judge = s_word == 0u;
+  if (!judge) {
+    if (threadIdx.x == 0) {
+      uint32_t v;
+      while ((v = ld_agent(&st->verdict)) == 0u) __builtin_amdgcn_s_sleep(8);
+      s_cnt = v;
+    }
+    __syncthreads();
+    if (s_cnt == 1u) return;
+  }
   uint32_t n_hi, n_low, n_list = 0;
   wide_prefix(hi, s_scan, 0, n_hi);
   wide_prefix(eqs, s_scan, 1, n_low);
   list.counted(s_seg[wave_id()]);
   for (int w = 0; w < kWideWaves; ++w) n_list += s_seg[w];
-  const bool ok = n_hi < k && k <= n_hi + n_list + n_low;
+  const bool ok = judge && n_hi < k && k <= n_hi + n_list + n_low;
+  if (judge && gridDim.x > 1 && ok && threadIdx.x == 0) st_agent(&st->verdict, 1u);
   const bool low = ok && k > n_hi + n_list;           // the lower end is the threshold
   uint32_t T = T_LO, need = k - n_hi - n_list, n_eq = n_low;
   int turn = 0;
@@ -273,48 +370,18 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     }
   }
   if (!ok) {
-    // the bracket missed: the same three levels over the data's own keys, by this workgroup alone
+    if (judge) {
+      for (int b = threadIdx.x; b < kHistEntries; b += kWide) st_agent(&J.hist[b], 0u);
+      wait_landed();
+      if (threadIdx.x == 0) st_agent(&st->verdict, 2u);
+    }
     Src src = srcs.s[blockIdx.y];
-    uint32_t prefix = 0, rank = k;
-    const int64_t trips = cdiv64(n, (int64_t)kWide * kVec);
-    for (int level = 0; level < 3; ++level) {
-      const int shift = level == 0 ? kL0Shift : level == 1 ? kL1Shift : 0;
-      const int above = level == 0 ? 31 : level == 1 ? kL0Shift : kL1Shift;
-      reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
-      __syncthreads();
-      for (int64_t t = 0; t < trips; ++t) {
-        const int64_t i = (t * kWide + threadIdx.x) * kVec;
-        uint32_t key[4] = {0u, 0u, 0u, 0u};
-        if (i < n) src.template load<false>(i, n, key);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          wide_hist_add(s_hist, (key[e] >> shift) & ((1u << (above - shift)) - 1u),
-                        i + e < n && (key[e] >> above) == prefix);
-      }
-      __syncthreads();
-      const uint32_t want[1] = {rank};
-      RankHit h[1];
-      wide_find_rank<1>(s_hist, want, s_scan, turn, h);
-      turn ^= 1;
-      prefix = (prefix << (above - shift)) | h[0].bin;
-      rank -= h[0].above;
-      n_eq = h[0].count;
-      __syncthreads();
-    }
-    T = prefix;
-    need = rank;
-    for (int t = threadIdx.x; t < nt; t += kWide) s_tile[t] = 0u;
-    __syncthreads();
-    for (int64_t t = 0; t < trips; ++t) {
-      const int64_t i = (t * kWide + threadIdx.x) * kVec;
-      uint32_t key[4] = {0u, 0u, 0u, 0u};
-      if (i < n) src.template load<false>(i, n, key);
-      uint32_t add = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (i + e < n) add += key[e] > T ? 1u : key[e] == T ? 1u << 16 : 0u;
-      if (add) atomicAdd(&s_tile[i >> 10], add);
-    }
+    if (!small_redo(src, J, s_hist, s_scan, &s_word)) return;
+    T = ld_agent(&st->prefix);
+    need = ld_agent(&st->krem);
+    n_eq = ld_agent(&st->n_eq);
+    for (int t = threadIdx.x; t < kSmallTiles; t += kWide)
+      s_tile[t] = t < nt ? ld_agent(&J.tile_gt[t]) | (ld_agent(&J.tile_eq[t]) << 16) : 0u;
     __syncthreads();
   }
   // chunk prefixes: ties granted in index order until `need` is used up (all of them: tie_all)
@@ -374,7 +441,9 @@ static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B,
   hipLaunchKernelGGL((k_pick_coarse<false>), B.grid(1), dim3(kWide), 0, s, B.jobs, kBracketSigmas);
   hipLaunchKernelGGL((k_small_sweep<Src>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)), dim3(kBlock),
                      0, s, srcs, B.jobs);
-  hipLaunchKernelGGL((k_small_finish<Src>), B.grid(1), dim3(kWide), 0, s, srcs, B.jobs);
+  const int64_t wgs = cdiv64(B.max_tiles, kRedoTiles);
+  hipLaunchKernelGGL((k_small_finish<Src>), B.grid((unsigned)(wgs < kRedoGroups ? wgs : kRedoGroups)), dim3(kWide), 0,
+                     s, srcs, B.jobs);
 }
 
 #endif  // __HIPCC__

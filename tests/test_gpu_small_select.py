@@ -122,3 +122,67 @@ def test_a_missed_bracket_is_redone_over_the_data(dev, n, side):
     sc[pos] = sc[pos] * (1e-9 if side == "low" else 1e9)
     for k in (n // 100, n // 2):
         _check(dev, sc, k, (side, n, k), path=0 if side == "low" else None)
+
+
+def _planted(n, side):
+    """Scores whose sample of the small buckets lies far below (above) all others."""
+    n_vec = n // 4
+    n_sv = min(n_vec, min(max(n // 512, 2048), 4096))
+    j = np.arange(n_sv, dtype=np.int64)
+    w0, w1 = j * n_vec // n_sv, (j + 1) * n_vec // n_sv
+    vec = w0 + _mix32(j.astype(np.uint32)).astype(np.int64) % (w1 - w0)
+    sc = student_t(n, 3).abs() + 1.0
+    sc[torch.from_numpy((vec[:, None] * 4 + np.arange(4)).reshape(-1))] *= 1e-9 if side == "low" else 1e9
+    return sc
+
+
+# one workgroup, two, one short of all 64, and all: the passes over the data are shared out between them
+@pytest.mark.parametrize("n", [32 * 1024, 32 * 1024 + 1, 63 * 32 * 1024 + 5, 64 * 32 * 1024 + 7, LIMIT])
+@pytest.mark.parametrize("grid", [False, True])
+def test_a_missed_bracket_takes_the_whole_launch(dev, n, grid):
+    sc = _planted(n, "low")
+    if grid:                                        # ties across chunks and workgroups
+        sc = sc.to(torch.bfloat16).float()
+    for k in (n // 100, n // 2, n - n // 64):
+        _check(dev, sc, k, (grid, n, k))
+
+
+def test_a_missed_bracket_costs_passes_over_the_data(dev):
+    """Four passes of the whole launch: a few ordinary selects.  One workgroup alone takes a
+    hundred of them."""
+    from sga_amd import _lib as L
+    from sga_amd.selection import read_result, select_exact_device
+    k = LIMIT // 100
+    took = {}
+    for name, sc in (("held", student_t(LIMIT, 3).abs() + 1.0), ("missed", _planted(LIMIT, "low"))):
+        sd = [sc.to(dev)]
+        assert read_result(select_exact_device(sd, k, L.TIE_LOWEST_INDEX)[0]).path == (name == "held")
+        times = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            select_exact_device(sd, k, L.TIE_LOWEST_INDEX)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        took[name] = sorted(times)[2]
+    assert took["missed"] <= 15.0 * took["held"], took
+
+
+def test_missed_and_held_brackets_in_one_batch(dev):
+    """Buckets of different sizes share the launch: only those whose bracket misses go over their data."""
+    from sga_amd.fused_step import FusedSparseStep, fused_step_multi
+    from sga_amd.shapes import segments_for
+    sizes, fs, state = [300_001, 5_000_003, 70_001], [], []
+    for b, n in enumerate(sizes):
+        g = student_t(n, b) if b == 0 else _planted(n, "low" if b == 1 else "high")
+        fs.append(FusedSparseStep(n, segments_for([("a", n)])[0], dev, values_dtype=torch.float32,
+                                  max_k=n // 50, want_mask=True))
+        state.append([g.to(dev)] + [torch.zeros(n, device=dev) for _ in range(4)])
+    ks = [n // 50 for n in sizes]
+    fused_step_multi(fs, *zip(*state), 3, ks=ks)
+    for f, n, k, b in zip(fs, sizes, ks, range(3)):
+        g = (student_t(n, b) if b == 0 else _planted(n, "low" if b == 1 else "high")).abs()
+        m_ref, _ = SEL.select_topk_flat(g, k)
+        assert torch.equal(f.mask.cpu(), m_ref.to(torch.uint8)), n
+        assert torch.equal(f.idx[:k].cpu().long(), m_ref.nonzero()[:, 0]), n
