@@ -1004,8 +1004,11 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // one each; what is left in a bin then is ranked by counting (or split by the last 7 bits, on plateaus).
 //
 // The small buckets bracket the k-th key of the data this way (sigmas: kBracketSigmas).  The large ones
-// (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with four
-// sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.
+// (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with eight
+// sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.  Sigma
+// is that of independent keys; scores that the four neighbours of a quad share halve it.  Such scores
+// missed in 32 of 1000 draws of 40 M coordinates at 10 % with four sigma, and in 12 with eight (the fine
+// sample's own five, halved); a wider coarse bracket costs the fine one a few keys of resolution.
 template <bool COARSE>
 __global__ __launch_bounds__(kWide) void k_pick_coarse(ChainJobs jobs, double sigmas) {
   const ChainJob& J = jobs.j[blockIdx.y];
@@ -1031,8 +1034,9 @@ __global__ __launch_bounds__(kWide) void k_pick_coarse(ChainJobs jobs, double si
     const double nf = (double)(J.n_sv * 4), to = (double)ns / nf;
     const RankEnds f = bracket_ranks((double)J.k, (double)n, nf, sigmas);
     const double ah = f.hi * to, al = f.lo * to;
-    rh = floor(ah - (4.0 * sqrt(fmax(ah, 0.0) + 1.0) + 4.0));
-    rl = ceil(al + (4.0 * sqrt(al + 1.0) + 4.0));
+    const double m = (double)ns;
+    rh = floor(ah - (8.0 * sqrt(fmax(ah * (1.0 - ah / m), 0.0) + 1.0) + 4.0));
+    rl = ceil(al + (8.0 * sqrt(fmax(al * (1.0 - al / m), 0.0) + 1.0) + 4.0));
   } else {
     const RankEnds f = bracket_ranks((double)J.k, (double)n, (double)ns, sigmas);
     rh = f.hi;
