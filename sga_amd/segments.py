@@ -54,7 +54,7 @@ class SegmentTable:
                       None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
                       self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
         self._hyper = list(map(_HYPER, rows))
-        self._betas = None
+        self._betas = self._last_lr = None
         self.follow_betas(rows)
 
     def follow_betas(self, rows):
@@ -83,8 +83,10 @@ class SegmentTable:
     def refresh(self, lr, count, bias_correction=True):
         """Learning rates (one number, or one per row) and the bias corrections of
         step ``count``, on the current stream."""
-        self._lr[:] = list(map(float, lr)) if isinstance(lr, list) else float(lr)
+        lr = list(map(float, lr)) if isinstance(lr, list) else float(lr)   # the caller may change its list
+        if lr != self._last_lr:
+            self._lr[:] = self._last_lr = lr
         for (b1, b2), at in self._groups:
-            self._bc1[at] = L.f32(1.0 - b1 ** count) if bias_correction else 1.0
-            self._bc2[at] = L.f32(1.0 - b2 ** count) if bias_correction else 1.0
+            self._bc1[at] = float(1.0 - b1 ** count) if bias_correction else 1.0
+            self._bc2[at] = float(1.0 - b2 ** count) if bias_correction else 1.0
         L.call("sga_segments_refresh", *self._args, L.stream())
