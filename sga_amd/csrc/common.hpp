@@ -77,7 +77,8 @@ __host__ __device__ static inline bool aligned4(const void* p, int elem) {
 }
 
 // True when the elements at p lie on multiples of their size: quads of them then go as one access each
-// (ld4 and the like take quads at any element's address).
+// (ld4 and the like take quads at any element's address).  Bytes always do, and so does whatever a tensor
+// library hands out; only a caller of the C interface can pass anything else, and takes scalar accesses.
 __host__ __device__ static inline bool quads_ok(const void* p, int elem) {
   return p == nullptr || (reinterpret_cast<uintptr_t>(p) % (size_t)elem) == 0;
 }

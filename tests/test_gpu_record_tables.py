@@ -31,7 +31,7 @@ def _records(dev, sizes, seed, with_mask):
 
 
 # 63 / 64 / 65 records: one and two rounds of the search; odd sizes shift every later record off
-# 16-byte alignment, so both the vector and the scalar forms run
+# 16-byte alignment and leave remainders, which go element by element
 @pytest.mark.parametrize("count", [1, 7, 63, 64, 65, 200])
 @pytest.mark.parametrize("with_mask", [True, False])
 def test_clip_tables(dev, count, with_mask):
@@ -47,6 +47,30 @@ def test_clip_tables(dev, count, with_mask):
     if with_mask:                                # dump steps scale in place
         c32 = torch.tensor(0.5 * exact / (norm + 1e-6), device=dev)
         assert coeff == 1.0 and torch.equal(t["g"], torch.where(mask > 0, before * c32, before))
+
+
+# the last element of every record carries the norm: a remainder that was left out would show
+@pytest.mark.parametrize("count", [1, 7, 63, 64, 65, 200])
+@pytest.mark.parametrize("was_full", [True, False])
+def test_clip_reaches_every_record_end(dev, count, was_full):
+    from sga_amd import _lib as L
+    from sga_amd.clip import masked_clip_grad_norm
+    sizes = [EDGES[i % len(EDGES)] for i in range(count)]
+    recs, t, mask = _records(dev, sizes, 300 + count, not was_full)
+    ends = torch.tensor(sizes).cumsum(0).to(dev) - 1
+    t["g"][ends] = 10.0 + torch.arange(count, device=dev) % 3
+    if mask is not None:
+        mask[ends] = 1
+    before = t["g"].clone()
+    exact = float((before if mask is None else before * mask).double().square().sum().sqrt())
+    assert len(L.host().norm_table(recs, was_full)) == 4          # the launches over the table, no other route
+    norm, coeff = masked_clip_grad_norm(recs, 0.5 * exact, was_full=was_full, trace_dumps=not was_full)
+    # a square is rounded, then added at most 16 + 6 + 2 times in fp32 (lane, wave, workgroup), then in double;
+    # the sum, its root and the result are rounded once each
+    assert abs(norm - exact) <= (25 / 2 + 2) * 2.0 ** -24 * exact
+    c32 = torch.tensor(0.5 * exact / (norm + 1e-6), device=dev)
+    want = before * c32 if mask is None else torch.where(mask > 0, before * c32, before)
+    assert coeff == 1.0 and torch.equal(t["g"], want)
 
 
 @pytest.mark.parametrize("count", [1, 7, 64, 65, 200])

@@ -58,3 +58,27 @@ def test_select_and_compaction(dev, n, off):
     assert torch.equal(m0, m1) and float(t0) == float(t1)
     mv, _ = _shifted(m0.view(torch.uint8), off)
     assert torch.equal(compact_mask_u8(mv), m0.nonzero()[:, 0].to(torch.int32))
+
+
+# the large buckets' sweeps: bit planes and settlement (a score that reads every array), and the single
+# sweep that writes the new state beside the old
+@pytest.mark.parametrize("single_sweep", [False, True])
+@pytest.mark.parametrize("off,grad", [(1, torch.bfloat16), (3, torch.float32)])
+def test_large_fused_step(dev, off, grad, single_sweep):
+    from sga_amd.fused_step import FusedSparseStep
+    from sga_amd.shapes import segments_for
+    n = 8192 * 1024 + 1027
+    segs, _ = segments_for([("a", n // 3), ("b", n - n // 3)])
+    k = n // 50
+    outs = []
+    for shift in (0, off):
+        st = [_shifted(t, shift) for t in _state(n, dev, grad)]
+        new = [_shifted(torch.zeros(n, device=dev), shift) for _ in range(4)] if single_sweep else st[1:]
+        fs = FusedSparseStep(n, segs, dev, values_dtype=torch.bfloat16, max_k=k, want_mask=True)
+        knobs = dict(single_sweep=True, seed=5, out=[t for t, _ in new]) if single_sweep else {}
+        idx, val = fs.step(*(t for t, _ in st), 7, k=k, score="update", **knobs)
+        outs.append([idx.clone(), val.clone(), fs.mask.clone()] + [t.clone() for t, _ in new])
+        for (view, buf) in st + new:                 # nothing beside the view is written
+            assert not buf[:shift].any() and not buf[shift + n:].any()
+    for a, b in zip(*outs):
+        assert torch.equal(a, b) if not a.is_floating_point() else same_bits(a.float(), b.float())
