@@ -77,9 +77,10 @@ typedef struct sga_select_result {
   uint32_t nonfinite;   /* NaN/Inf lanes seen (selection is undefined > 0) */
   uint32_t status;      /* 0 ok; 1 k out of range; 2 fast path fell back;
                            3 single-sweep bracket missed (step invalid)    */
-  uint32_t path;        /* low byte: 0 no sampled bracket decided (buckets below
-                           2^20, plateaus, radix passes), 1 sampled bracket, 2 single
-                           sweep; bit 8: an fp32 score array held a value < 0;
+  uint32_t path;        /* low byte: 1 a sampled bracket decided (reported for
+                           buckets of 2^20 coordinates and more), 2 a single sweep
+                           did, 0 everything else: plateaus, passes over the data
+                           after a miss, and all smaller buckets whatever decided; bit 8: an fp32 score array held a value < 0;
                            bit 9: an out-of-place single-sweep step was redone */
 } sga_select_result;
 

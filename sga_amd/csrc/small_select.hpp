@@ -425,8 +425,8 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
       out->n_selected = selected;
       out->nonfinite = st->nonfinite;
       out->status = 0u;
-      // reported as the bracket path where the large buckets' bracket begins, as the radix path below
-      // it and where no list decided
+      // 1 where the bracket decided, but for buckets below 2^20: they report 0 whatever decided (callers
+      // know the path of those sizes as 0)
       out->path = (ok && !single && n >= kFastMinN ? 1u : 0u) | (st->negative ? 0x100u : 0u);
     }
   }
