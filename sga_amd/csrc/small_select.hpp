@@ -169,6 +169,8 @@ static_assert(kSmallHead * kWave * kVec <= kBlockSpan, "the head never reaches p
 // coordinates, the launch takes 0.21 (a bracket that holds: 0.10).
 constexpr int kRedoGroups = 64;                       // at most; one per kRedoTiles chunks
 constexpr int kRedoTiles = 32;
+constexpr uint32_t kCrowdedList = 1 << 15;            // shorter lists are walked in less time than the passes take
+                                                      // (1.3 us a thousand equal keys, 50 to 190 us the passes)
 template <class Src>
 __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t* s_hist, WideScratch& s_scan,
                                            uint32_t* s_word) {
@@ -295,7 +297,17 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   wide_prefix(eqs, s_scan, 1, n_low);
   list.counted(s_seg[wave_id()]);
   for (int w = 0; w < kWideWaves; ++w) n_list += s_seg[w];
-  const bool ok = judge && n_hi < k && k <= n_hi + n_list + n_low;
+  // A list far longer than its margin says holds a plateau that one workgroup should not walk (keys equal
+  // to the upper end are listed): two values, k near where they change, 8.4 M coordinates: half of them
+  // on the upper one 5.7 ms, a tenth 1.06; by passes over the data 0.29 and 0.32.  Independent scores list
+  // 1.0 times what the margin says.
+  bool crowded = false;
+  if (n_list > kCrowdedList) {
+    const double ns = (double)(small_sample_vecs(n) * 4);
+    const RankEnds f = bracket_ranks((double)k, (double)n, ns, kBracketSigmas);
+    crowded = (double)n_list * ns > 2.0 * (f.lo - f.hi) * (double)n;
+  }
+  const bool ok = judge && !crowded && n_hi < k && k <= n_hi + n_list + n_low;
   if (judge && gridDim.x > 1 && ok && threadIdx.x == 0) st_agent(&st->verdict, 1u);
   const bool low = ok && k > n_hi + n_list;           // the lower end is the threshold
   uint32_t T = T_LO, need = k - n_hi - n_list, n_eq = n_low;

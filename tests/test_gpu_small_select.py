@@ -199,3 +199,33 @@ def test_shared_scores_of_large_buckets_keep_their_bracket(dev):
         sc = torch.rand(n // 4, generator=gen, device=dev).repeat_interleave(4)
         missed += read_result(select_exact_device([sc], n // 10, L.TIE_LOWEST_INDEX)[0]).path == 0
     assert missed <= 20, missed                     # 12 with this seed; 32 with half the coarse margin
+
+
+# two values, k at, before and past the place where they change: the upper one would all be listed
+@pytest.mark.parametrize("n", [600_011, 1_500_001, LIMIT])
+@pytest.mark.parametrize("frac", [0.05, 0.1, 0.5])
+def test_plateau_at_the_upper_end(dev, n, frac):
+    on = torch.rand(n, generator=torch.Generator().manual_seed(n % 83)) < frac
+    few = int(on.sum())
+    for k in (few - 1, few, few + 1):
+        _check(dev, torch.where(on, 2.0, 1.0), k, (n, frac, k))
+
+
+def test_a_plateau_at_the_upper_end_costs_passes_over_the_data(dev):
+    from sga_amd import _lib as L
+    from sga_amd.selection import select_exact_device
+    r = torch.rand(LIMIT, generator=torch.Generator(device=dev).manual_seed(3), device=dev)
+    on = r < 0.5
+    k = int(on.sum())
+    took = []
+    for sc in (r, on.float()):
+        times = []
+        for _ in range(5):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            select_exact_device([sc], k, L.TIE_LOWEST_INDEX)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        took.append(sorted(times)[2])
+    assert took[1] <= 8.0 * took[0], took            # one workgroup over the list: 32 times
