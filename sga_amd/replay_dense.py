@@ -29,8 +29,9 @@ def lr_max_abs_diff(gmeta):
 
 def lr_by_group(gmeta, entries):
     """``lr_for_step`` of every entry, each group looked up once."""
-    of = {g: float(lr_for_step(gmeta, g)) for g in {e.get("group") for e in entries}}
-    return [of[e.get("group")] for e in entries]
+    groups = [e.get("group") for e in entries]
+    of = {g: float(lr_for_step(gmeta, g)) for g in set(groups)}
+    return [of[g] for g in groups]
 
 
 class DenseReplay:
