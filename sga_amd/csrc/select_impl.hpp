@@ -38,9 +38,7 @@ struct SelState {
   uint32_t t_hi;
   uint32_t n_hi;        // keys >= t_hi
   uint32_t cand_count;  // keys in the bracket (may exceed capacity)
-  uint32_t cand_cap;
   uint32_t bracket_ok;  // 1: the sampled bracket holds the k-th key; radix passes skip
-  uint32_t sample_n;
   uint32_t overflow;    // a candidate segment ran out of room
   uint32_t skip;        // 1: kernels driven by this state do nothing
   uint32_t done[3];     // per-level "workgroups finished" tickets (last one scans)
@@ -58,13 +56,13 @@ struct SelState {
   uint32_t finish_ticket; // k_small_finish: workgroups that have begun; the first one judges the bracket ...
   uint32_t verdict;     // ... 1: it holds the k-th key, 2: all of them go over the data again
   uint32_t redo_step;   // passes of that which are done
-  uint32_t pad_[26];
+  uint32_t pad_[28];
 };
 static_assert(sizeof(SelState) == 256, "SelState layout");
 
 struct SelWorkspace {
   SelState* st;        // main state (result, bracket)
-  SelState* aux;       // aux[0], aux[1]: states of the sample / candidate descents
+  SelState* aux;       // aux[0]: state of the descent over dense records (single-sweep step)
   uint32_t* hist;      // 2 sets of 3 levels: [0,4096) [4096,8192) [8192,8320)
   uint32_t* tile_gt;   // n_tiles -> selected-count prefix
   uint32_t* tile_eq;   // n_tiles -> tie-count prefix
@@ -449,7 +447,7 @@ __device__ __forceinline__ void level_hist_body(Src& src, int64_t n, uint32_t pr
   constexpr int NB = LEVEL == 2 ? kBinsSmall : kBinsBig;
   for (int b = threadIdx.x; b < NB; b += kBlock) s_h[b] = 0u;
   __syncthreads();
-  // Raw key buffers (sample, candidates) are short and sit in L2: what their passes cost is load
+  // Raw key buffers (dense records) are short and sit in L2: what their passes cost is load
   // latency, so each lane keeps kQuads 16-byte loads in flight per trip; the passes over the data
   // itself run on a small grid and need them too.
   constexpr int kQuads = 4;
@@ -818,10 +816,9 @@ __device__ __forceinline__ void write_result(const ChainJob& J) {
 static __global__ void k_sel_result(ChainJobs jobs) { write_result(jobs.j[blockIdx.y]); }
 
 // -------------------------------------------------------------- host drivers
-// Grid of the histogram passes over raw key buffers (<= 1M sample keys, ~1e6 candidates whose
-// count lives on the device).  What a workgroup costs there is fixed (zeroing and flushing its
-// LDS bins, the device-scope fence and ticket of the merged scan): measured, 256 or 1024
-// workgroups are 5 and 40 us slower per pass than 64.
+// Grid unit of the histogram passes over dense records (the single-sweep step launches three of them;
+// the count of the records lives on the device).  What a workgroup costs there is fixed: zeroing and
+// flushing its LDS bins, and its ticket.
 constexpr unsigned kRawKeyBlocks = 64;
 static inline dim3 hist_grid(int64_t n) {
   return dim3(stream_grid(n, (int64_t)kBlock * kVec * 4, 256 * 8));
