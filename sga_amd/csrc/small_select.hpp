@@ -169,7 +169,7 @@ static_assert(kSmallHead * kWave * kVec <= kBlockSpan, "the head never reaches p
 // coordinates, the launch takes 0.21 (a bracket that holds: 0.10).
 constexpr int kRedoGroups = 64;                       // at most; one per kRedoTiles chunks
 constexpr int kRedoTiles = 32;
-constexpr uint32_t kCrowdedList = 1 << 15;            // shorter lists are walked in less time than the passes take
+constexpr uint32_t kCrowdedList = 1 << 16;            // shorter lists are walked in less time than the passes take
                                                       // (1.3 us a thousand equal keys, 50 to 190 us the passes)
 template <class Src>
 __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t* s_hist, WideScratch& s_scan,
