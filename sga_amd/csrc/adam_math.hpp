@@ -131,6 +131,24 @@ struct SegCursor {
     }
     take_uniform(a);
   }
+  // The same by all 64 lanes, each with an entry of its own: one round of loads for up to 64 tensors, two for
+  // up to 4096, where the directory and the walk behind it are two to six dependent ones (the small tensors of
+  // a layer lie side by side).  For waves that own a slab or a chunk of a small bucket and have nothing else
+  // to do meanwhile; a long sweep's scalar loads hit the scalar cache instead.
+  __device__ __forceinline__ void seek_wave(int64_t i) {
+    if (i >= lo && i < hi) return;
+    int a = 0, len = n_segs;
+    while (len > 1) {
+      const int step = (len + kWave - 1) / kWave;
+      const int e = a + lane_id() * step;
+      const bool below = e < a + len && segs[e].start <= i;
+      const int hit = __popcll(ballot64(below)) - 1;       // the table starts at 0: entry a is always below
+      const int end = a + len;
+      a += (hit < 0 ? 0 : hit) * step;
+      len = end - a < step ? end - a : step;
+    }
+    take_uniform(uniform_i32(a));
+  }
   // Steps to the segment that holds i, a little past the cached one (the
   // next tensor of a slab that straddles a boundary).
   __device__ __forceinline__ void advance_uniform(int64_t i) {

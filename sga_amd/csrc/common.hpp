@@ -164,14 +164,16 @@ __device__ __forceinline__ T wave_sum(T v) {
   return v;
 }
 
-// Inclusive scan across the 64 lanes of a wave.
+// Inclusive scan across the 64 lanes of a wave: shifts inside the rows of 16 lanes, then the rows' last
+// lanes broadcast to the rows behind (six data-parallel-primitive adds; six LDS permutes are ten times
+// their latency).
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
-  const int l = lane_id();
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    uint32_t t = __shfl_up(v, o, kWave);
-    if (l >= o) v += t;
-  }
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);      // row_shr:1
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);      // row_shr:2
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);      // row_shr:4
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);      // row_shr:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);     // row_bcast:15
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);     // row_bcast:31
   return v;
 }
 
@@ -208,6 +210,10 @@ __device__ __forceinline__ F4 ld4_nt(const float* p) {
   return F4{t.x, t.y, t.z, t.w};
 }
 typedef unsigned short h4v __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ H4 ldh4(const uint16_t* p) {
+  const h4v t = *reinterpret_cast<const h4v*>(p);
+  return H4{t.x, t.y, t.z, t.w};
+}
 __device__ __forceinline__ H4 ldh4_nt(const uint16_t* p) {
   const h4v t = __builtin_nontemporal_load(reinterpret_cast<const h4v*>(p));
   return H4{t.x, t.y, t.z, t.w};
@@ -303,9 +309,11 @@ __device__ __forceinline__ void ld_bf16(const uint16_t* base, int64_t i, int64_t
 // Loads kept as the raw vectors that arrive from memory: nothing depends on
 // them until they are unpacked, so a sweep can issue the loads of several
 // slabs before it waits for the first.
-template <bool FULL>
+// KEEP: an ordinary access, which leaves the data in the memory-side cache for a pass that reads it again
+// soon; a non-temporal one does not.
+template <bool FULL, bool KEEP = false>
 __device__ __forceinline__ F4 ldraw_f32(const float* base, int64_t i, int64_t n, bool vec) {
-  if (FULL) return ld4_nt(base + i);
+  if (FULL) return KEEP ? ld4(base + i) : ld4_nt(base + i);
   float t[4];
   load4_f32(base, i, n, t, vec);
   return F4{t[0], t[1], t[2], t[3]};
@@ -314,16 +322,16 @@ __device__ __forceinline__ void unpack_f32(const F4& r, float out[4]) {
   out[0] = r.x; out[1] = r.y; out[2] = r.z; out[3] = r.w;
 }
 struct RawG { H4 h; F4 f; };      // a gradient quad: bf16 bits (full vector path) or fp32
-template <bool BF16G, bool FULL>
+template <bool BF16G, bool FULL, bool KEEP = false>
 __device__ __forceinline__ void fetch_g(const void* g, int64_t i, int64_t n, bool vec, RawG& r) {
   if (BF16G && FULL) {
-    r.h = ldh4_nt(reinterpret_cast<const uint16_t*>(g) + i);
+    r.h = KEEP ? ldh4(reinterpret_cast<const uint16_t*>(g) + i) : ldh4_nt(reinterpret_cast<const uint16_t*>(g) + i);
   } else if (BF16G) {
     float t[4];
     load4_bf16(reinterpret_cast<const uint16_t*>(g), i, n, t, vec);
     r.f = F4{t[0], t[1], t[2], t[3]};
   } else {
-    r.f = ldraw_f32<FULL>(reinterpret_cast<const float*>(g), i, n, vec);
+    r.f = ldraw_f32<FULL, KEEP>(reinterpret_cast<const float*>(g), i, n, vec);
   }
 }
 template <bool BF16G, bool FULL>

@@ -58,13 +58,16 @@ struct SrcFused {
   __device__ __forceinline__ void chunk_hyper(int64_t c) {
     if (kHyper) sc.seek_uniform(uniform_i64(c) * kChunk);
   }
-  template <bool FULL>
+  __device__ __forceinline__ void slab_hyper(int64_t i0) {
+    if (kHyper) sc.seek_wave(i0);
+  }
+  template <bool FULL, bool KEEP = false>
   __device__ __forceinline__ void fetch(const Chunk& ck, int64_t i, int64_t n, Raw& w) {
-    if (kNeedG && has_g()) fetch_g<BF16G, FULL>(g, i, n, vec, w.g);
-    if (kNeedR) w.r = ldraw_f32<FULL>(r + ck.sh, i, n, vec);
-    if (need_m()) w.m = ldraw_f32<FULL>(m + ck.sh, i, n, vec);
-    if (kNeedP) w.p = ldraw_f32<FULL>(p + ck.sh, i, n, vec);
-    if (kNeedV && !adams) w.v = ldraw_f32<FULL>(v + ck.sh, i, n, vec);
+    if (kNeedG && has_g()) fetch_g<BF16G, FULL, KEEP>(g, i, n, vec, w.g);
+    if (kNeedR) w.r = ldraw_f32<FULL, KEEP>(r + ck.sh, i, n, vec);
+    if (need_m()) w.m = ldraw_f32<FULL, KEEP>(m + ck.sh, i, n, vec);
+    if (kNeedP) w.p = ldraw_f32<FULL, KEEP>(p + ck.sh, i, n, vec);
+    if (kNeedV && !adams) w.v = ldraw_f32<FULL, KEEP>(v + ck.sh, i, n, vec);
   }
   template <bool FULL>
   __device__ __forceinline__ void keys(const Chunk& ck, int64_t i, int64_t n, const Raw& w,
@@ -150,250 +153,220 @@ struct FinalArgs {
   const uint32_t* planes;   // the settled selection as bit planes (PLANES mode), else unused
 };
 
-// One 1024-element chunk of the final sweep, owned by one wave.  FULL: the
-// chunk is entirely in range and every array is element-aligned, so all 20
-// loads are unconditional and issued before the first use.
-// IT0 / NIT: the slabs [IT0, IT0+NIT) of the chunk are handled by this call;
-// `cur` carries the running selected / tie counts across calls.  slab: added to the slab numbers.
-// PLANES: the selection was already settled as bit planes (bracket sweep +
-// candidates): the slab's four 64-bit ballots are read on the scalar unit and
-// the keys are not formed again; SCORE is then irrelevant.
-template <bool BF16G, bool BF16V, int SCORE, bool FULL, int IT0, int NIT, bool PLANES>
-__device__ __forceinline__ void final_chunk(const FinalArgs& a, int64_t c, ChunkCursor& cur,
-                                            SegCursor& sc, int slab = 0) {
+// One 256-element slab of the final sweep, owned by one wave; the four waves of the workgroup hold the four
+// slabs of chunk c.  FULL: the chunk is entirely in range and every array is element-aligned, so all loads
+// are unconditional and issued before the first use.
+// cur: selected and tied coordinates before the chunk; what the earlier slabs hold goes through s_cnt.
+// PLANES: the selection was already settled as bit planes (bracket sweep + candidates): the slab's four
+// 64-bit ballots are read on the scalar unit and the keys are not formed again.
+template <bool BF16G, bool BF16V, int SCORE, bool FULL, bool PLANES>
+__device__ __forceinline__ void final_slab(const FinalArgs& a, int64_t c, int slab, ChunkCursor cur, SegCursor& sc,
+                                           uint32_t* s_cnt) {
   const int64_t n = a.n;
   const int64_t sh = pack_shift<true>(c << 10, a.pack_extra);     // c is wave-uniform
-  const float* const R = a.r + sh;
-  const float* const P = a.p + sh;
-  const float* const M = a.m + sh;
-  const float* const V = a.v + sh;
-  float* const RO = a.ro + sh;
-  float* const PO = a.po + sh;
-  float* const MO = a.mo + sh;
-  float* const VO = a.vo + sh;
-  float gg[kChunkIters][4], rr[kChunkIters][4], pp[kChunkIters][4], mm[kChunkIters][4],
-      vv[kChunkIters][4];
+  const int64_t s0 = uniform_i64(c) * kChunk + slab * (kWave * kVec), i = s0 + lane_id() * kVec;
+  float gg[4], rr[4], pp[4], mm[4], vv[4];
   const bool has_g = BF16G || a.g != nullptr;     // no g: the buffer `r` already holds g + r
   if (FULL) {
-    // raw loads first (bf16 kept packed), a scheduling fence, then unpacking:
-    // the wave has all 20 loads of its chunk in flight before the first wait
-    H4 graw_h[kChunkIters];
-    F4 graw_f[kChunkIters], rraw[kChunkIters], praw[kChunkIters], mraw[kChunkIters],
-        vraw[kChunkIters];
-#pragma unroll
-    for (int it = IT0; it < IT0 + NIT; ++it) {
-      const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
-      if (BF16G) graw_h[it] = ldh4_nt(reinterpret_cast<const uint16_t*>(a.g) + i);
-      else if (has_g) graw_f[it] = ld4_nt(reinterpret_cast<const float*>(a.g) + i);
-      else graw_f[it] = F4{0.0f, 0.0f, 0.0f, 0.0f};
-      rraw[it] = ld4_nt(R + i);
-      praw[it] = ld4_nt(P + i);
-      mraw[it] = ld4_nt(M + i);
-      vraw[it] = ld4_nt(V + i);
-    }
+    // raw loads first (bf16 kept packed), a scheduling fence, then unpacking: the wave has all its loads in
+    // flight before the first wait, and the chain of loads to the tensor's hyper-parameters beside them
+    H4 gh;
+    F4 gf{0.0f, 0.0f, 0.0f, 0.0f};
+    if (BF16G) gh = ldh4_nt(reinterpret_cast<const uint16_t*>(a.g) + i);
+    else if (has_g) gf = ld4_nt(reinterpret_cast<const float*>(a.g) + i);
+    const F4 r4 = ld4_nt(a.r + sh + i), p4 = ld4_nt(a.p + sh + i), m4 = ld4_nt(a.m + sh + i), v4 = ld4_nt(a.v + sh + i);
     __builtin_amdgcn_sched_barrier(0);
-    if (NIT > 1) sc.seek_uniform(uniform_i64(c) * kChunk);   // its chain of scalar loads runs beside the data's
-#pragma unroll
-    for (int it = IT0; it < IT0 + NIT; ++it) {
-      if (BF16G) {
-        gg[it][0] = bf16_to_f32(graw_h[it].x); gg[it][1] = bf16_to_f32(graw_h[it].y);
-        gg[it][2] = bf16_to_f32(graw_h[it].z); gg[it][3] = bf16_to_f32(graw_h[it].w);
-      } else {
-        gg[it][0] = graw_f[it].x; gg[it][1] = graw_f[it].y; gg[it][2] = graw_f[it].z; gg[it][3] = graw_f[it].w;
-      }
-      rr[it][0] = rraw[it].x; rr[it][1] = rraw[it].y; rr[it][2] = rraw[it].z; rr[it][3] = rraw[it].w;
-      pp[it][0] = praw[it].x; pp[it][1] = praw[it].y; pp[it][2] = praw[it].z; pp[it][3] = praw[it].w;
-      mm[it][0] = mraw[it].x; mm[it][1] = mraw[it].y; mm[it][2] = mraw[it].z; mm[it][3] = mraw[it].w;
-      vv[it][0] = vraw[it].x; vv[it][1] = vraw[it].y; vv[it][2] = vraw[it].z; vv[it][3] = vraw[it].w;
+    sc.seek_wave(s0);
+    if (BF16G) {
+      gg[0] = bf16_to_f32(gh.x); gg[1] = bf16_to_f32(gh.y); gg[2] = bf16_to_f32(gh.z); gg[3] = bf16_to_f32(gh.w);
+    } else {
+      unpack_f32(gf, gg);
     }
+    unpack_f32(r4, rr); unpack_f32(p4, pp); unpack_f32(m4, mm); unpack_f32(v4, vv);
   } else {
 #pragma unroll
-    for (int it = IT0; it < IT0 + NIT; ++it) {
-      const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) gg[it][e] = rr[it][e] = pp[it][e] = mm[it][e] = vv[it][e] = 0.0f;
-      if (i < n) {
-        if (has_g) load_g<BF16G, false>(a.g, i, n, gg[it], a.vec);
-        load4_f32(R, i, n, rr[it], a.vec);
-        load4_f32(P, i, n, pp[it], a.vec);
-        load4_f32(M, i, n, mm[it], a.vec);
-        load4_f32(V, i, n, vv[it], a.vec);
-      }
+    for (int e = 0; e < 4; ++e) gg[e] = rr[e] = pp[e] = mm[e] = vv[e] = 0.0f;
+    if (i < n) {
+      if (has_g) load_g<BF16G, false>(a.g, i, n, gg, a.vec);
+      load4_f32(a.r + sh, i, n, rr, a.vec);
+      load4_f32(a.p + sh, i, n, pp, a.vec);
+      load4_f32(a.m + sh, i, n, mm, a.vec);
+      load4_f32(a.v + sh, i, n, vv, a.vec);
     }
+    if (s0 < n) sc.seek_wave(s0);
   }
+  float q[4];
+  bool valid[4], sel[4];
+  uint32_t pos;
 #pragma unroll
-  for (int it = IT0; it < IT0 + NIT; ++it) {
-    const int64_t i = c * kChunk + (it + slab) * (kWave * kVec) + lane_id() * kVec;
-    float q[4];
-    bool valid[4], sel[4];
-    uint32_t pos;
-    if (PLANES) {
-      // words 2e, 2e + 1 of the slab are the ballot of element e over the 64 lanes; lanes are in
-      // index order, so the selected coordinates before (lane, e) are the mask bits below the
-      // lane over all four ballots plus the lane's own earlier elements
-      const uint64_t* pw = reinterpret_cast<const uint64_t*>(a.planes) + (uniform_i64(c) * kChunkIters + it + slab) * 4;
-      uint32_t below = 0, total = 0;
+  for (int e = 0; e < 4; ++e) {
+    valid[e] = FULL || i + e < n;
+    q[e] = has_g ? rr[e] + gg[e] : rr[e];
+  }
+  if (PLANES) {
+    // words 2e, 2e + 1 of the slab are the ballot of element e over the 64 lanes; lanes are in
+    // index order, so the selected coordinates before (lane, e) are the mask bits below the
+    // lane over all four ballots plus the lane's own earlier elements
+    const uint64_t* pw = reinterpret_cast<const uint64_t*>(a.planes) + uniform_i64(c) * (kChunkIters * 4);
+    for (int w = 0; w < slab * 4; ++w) cur.sel_run += (uint32_t)__popcll(pw[w]);
+    uint32_t below = 0;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint64_t mk = pw[e];
-        valid[e] = FULL || i + e < n;
-        q[e] = has_g ? rr[it][e] + gg[it][e] : rr[it][e];
-        sel[e] = __builtin_amdgcn_inverse_ballot_w64(mk);
-        below += lanes_below(mk);
-        total += (uint32_t)__popcll(mk);
+    for (int e = 0; e < 4; ++e) {
+      const uint64_t mk = pw[slab * 4 + e];
+      sel[e] = __builtin_amdgcn_inverse_ballot_w64(mk);
+      below += lanes_below(mk);
+    }
+    pos = cur.sel_run + below;
+  } else {
+    uint32_t key[4] = {0u, 0u, 0u, 0u};
+    if (SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI || SCORE == SGA_SCORE_GR_OVER_SQRT_V) {
+      if (FULL || s0 < n) {
+        float vk[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vk[e] = a.adams ? mm[e] * mm[e] : vv[e];
+        slab_score_keys<SCORE, FULL>(sc, a.adams ? 1 : 0, i, n, q, pp, mm, vk, key);
       }
-      pos = cur.sel_run + below;
-      cur.sel_run += total;
     } else {
-      uint32_t key[4] = {0u, 0u, 0u, 0u};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        valid[e] = FULL || i + e < n;
-        q[e] = has_g ? rr[it][e] + gg[it][e] : rr[it][e];
-        if (SCORE == SGA_SCORE_ABS_G) key[e] = abs_key(q[e]);
-        else if (SCORE == SGA_SCORE_ABS_G_BLIND) key[e] = abs_key(gg[it][e]);
-        else if (SCORE == SGA_SCORE_ABS_M) key[e] = abs_key(mm[it][e]);
-      }
-      if (SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI || SCORE == SGA_SCORE_GR_OVER_SQRT_V) {
-        const int64_t s0 = uniform_i64(c) * kChunk + (it + slab) * (kWave * kVec);
-        if (FULL || s0 < n) {
-          float vk[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) vk[e] = a.adams ? mm[it][e] * mm[it][e] : vv[it][e];
-          if (s0 < sc.lo || s0 >= sc.hi) sc.seek_uniform(s0);
-          slab_score_keys<SCORE, FULL>(sc, a.adams ? 1 : 0, i, n, q, pp[it], mm[it], vk, key);
-        }
-      }
-      slab_select(key, valid, a.T, a.need, cur, sel, pos);
+      for (int e = 0; e < 4; ++e)
+        key[e] = abs_key(SCORE == SGA_SCORE_ABS_M ? mm[e] : SCORE == SGA_SCORE_ABS_G_BLIND ? gg[e] : q[e]);
     }
-    if (FULL || i < n) {
-      uint32_t mk[4];
-      float ge[4];
+    uint32_t gt = 0, eq = 0;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        mk[e] = sel[e];
-        ge[e] = 0.0f;
-        if (!valid[e] || !sel[e]) continue;
-        float val = q[e];
-        if (a.scale) val = val * a.factor;
-        if (BF16V) {
-          const uint16_t hb = f32_to_bf16(val);
-          if ((int64_t)pos < a.k) {
-            a.idx_out[pos] = (int32_t)(i + e);
-            reinterpret_cast<uint16_t*>(a.values_out)[pos] = hb;
-          }
-          ge[e] = bf16_to_f32(hb);
-        } else {
-          if ((int64_t)pos < a.k) {
-            a.idx_out[pos] = (int32_t)(i + e);
-            reinterpret_cast<float*>(a.values_out)[pos] = val;
-          }
-          ge[e] = val;
-        }
-        ++pos;
-        if (a.apply_coeff) ge[e] = ge[e] * a.coeff;
-      }
-      // The commit takes its hyper-parameters from the scalar unit: the slab lies inside one
-      // tensor but for the few that hold a boundary, which are committed once per tensor piece.
-      const int64_t s0 = uniform_i64(c) * kChunk + (it + slab) * (kWave * kVec);
-      int64_t s1 = s0 + kWave * kVec;
-      if (!FULL && s1 > n) s1 = n;
-      if (s0 < sc.lo || s0 >= sc.hi) sc.seek_uniform(s0);
-      // a coordinate no tensor of the table covers keeps its p / m / v
-      float pn[4] = {pp[it][0], pp[it][1], pp[it][2], pp[it][3]};
-      float mn[4] = {mm[it][0], mm[it][1], mm[it][2], mm[it][3]};
-      float vn[4] = {vv[it][0], vv[it][1], vv[it][2], vv[it][3]};
-      for (;;) {
-        const bool whole = sc.lo <= s0 && sc.hi >= s1;
-        Hyper h = sc.h;
-        if (a.adams) { h.bc1 = 1.0f; h.bc2 = 1.0f; }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float ve = a.adams ? mm[it][e] * mm[it][e] : vv[it][e];
-          const Commit cm = adamw_commit(pp[it][e], ge[e], mm[it][e], ve, h);
-          const float pe = pp[it][e] - h.lr * cm.upd;
-          if (whole || (i + e >= sc.lo && i + e < sc.hi)) { pn[e] = pe; mn[e] = cm.m_new; vn[e] = cm.v_new; }
-        }
-        const int64_t nxt = sc.hi;
-        if (whole || nxt >= s1) break;
-        sc.advance_uniform(nxt);
-        if (sc.hi <= nxt) break;              // the table does not tile [0, n): stop
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (!valid[e]) continue;
-        pp[it][e] = pn[e]; mm[it][e] = mn[e]; vv[it][e] = vn[e];
-        rr[it][e] = sel[e] ? 0.0f : q[e];
-        if (a.fold) rr[it][e] = __fdiv_rn(rr[it][e], a.interval);
-      }
-      st_f32<FULL>(RO, i, n, rr[it], a.vec);
-      st_f32<FULL>(MO, i, n, mm[it], a.vec);
-      st_f32<FULL>(VO, i, n, vv[it], a.vec);
-      st_f32<FULL>(PO, i, n, pp[it], a.vec);
-      if (a.mask_out) st_u8<FULL>(a.mask_out, i, n, mk, a.mvec);
+    for (int e = 0; e < 4; ++e) {
+      gt += (uint32_t)__popcll(ballot64(valid[e] && key[e] > a.T));
+      eq += (uint32_t)__popcll(ballot64(valid[e] && key[e] == a.T));
     }
+    if (lane_id() == 0) { s_cnt[slab] = gt; s_cnt[kChunkIters + slab] = eq; }
+    __syncthreads();
+    for (int w = 0; w < slab; ++w) {
+      const uint32_t ties = s_cnt[kChunkIters + w];
+      cur.sel_run += s_cnt[w] + ties_taken(a.need, cur.eq_run, ties);
+      cur.eq_run += ties;
+    }
+    slab_select(key, valid, a.T, a.need, cur, sel, pos);
   }
+  if (!FULL && i >= n) return;
+  uint32_t mk[4];
+  float ge[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    mk[e] = sel[e];
+    ge[e] = 0.0f;
+    if (!valid[e] || !sel[e]) continue;
+    float val = q[e];
+    if (a.scale) val = val * a.factor;
+    if (BF16V) {
+      const uint16_t hb = f32_to_bf16(val);
+      if ((int64_t)pos < a.k) {
+        a.idx_out[pos] = (int32_t)(i + e);
+        reinterpret_cast<uint16_t*>(a.values_out)[pos] = hb;
+      }
+      ge[e] = bf16_to_f32(hb);
+    } else {
+      if ((int64_t)pos < a.k) {
+        a.idx_out[pos] = (int32_t)(i + e);
+        reinterpret_cast<float*>(a.values_out)[pos] = val;
+      }
+      ge[e] = val;
+    }
+    ++pos;
+    if (a.apply_coeff) ge[e] = ge[e] * a.coeff;
+  }
+  // The commit takes its hyper-parameters from the scalar unit: the slab lies inside one
+  // tensor but for the few that hold a boundary, which are committed once per tensor piece.
+  int64_t s1 = s0 + kWave * kVec;
+  if (!FULL && s1 > n) s1 = n;
+  if (s0 < sc.lo || s0 >= sc.hi) sc.seek_uniform(s0);             // the keys' walk has left the first tensor
+  // a coordinate no tensor of the table covers keeps its p / m / v
+  float pn[4] = {pp[0], pp[1], pp[2], pp[3]}, mn[4] = {mm[0], mm[1], mm[2], mm[3]},
+        vn[4] = {vv[0], vv[1], vv[2], vv[3]};
+  for (;;) {
+    const bool whole = sc.lo <= s0 && sc.hi >= s1;
+    Hyper h = sc.h;
+    if (a.adams) { h.bc1 = 1.0f; h.bc2 = 1.0f; }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float ve = a.adams ? mm[e] * mm[e] : vv[e];
+      const Commit cm = adamw_commit(pp[e], ge[e], mm[e], ve, h);
+      const float pe = pp[e] - h.lr * cm.upd;
+      if (whole || (i + e >= sc.lo && i + e < sc.hi)) { pn[e] = pe; mn[e] = cm.m_new; vn[e] = cm.v_new; }
+    }
+    const int64_t nxt = sc.hi;
+    if (whole || nxt >= s1) break;
+    sc.advance_uniform(nxt);
+    if (sc.hi <= nxt) break;              // the table does not tile [0, n): stop
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    if (!valid[e]) continue;
+    pp[e] = pn[e]; mm[e] = mn[e]; vv[e] = vn[e];
+    rr[e] = sel[e] ? 0.0f : q[e];
+    if (a.fold) rr[e] = __fdiv_rn(rr[e], a.interval);
+  }
+  st_f32<FULL>(a.ro + sh, i, n, rr, a.vec);
+  st_f32<FULL>(a.mo + sh, i, n, mm, a.vec);
+  st_f32<FULL>(a.vo + sh, i, n, vv, a.vec);
+  st_f32<FULL>(a.po + sh, i, n, pp, a.vec);
+  if (a.mask_out) st_u8<FULL>(a.mask_out, i, n, mk, a.mvec);
 }
 
-// Final sweep: select flags in index order, pack, residual, commit.
-// `when`: 0 run always; 1 only if the sampled bracket held (the planes are
-// settled); 2 only if it failed (the radix passes fixed the threshold and the
-// keys are formed again here); 3 like 2, and only if the single-sweep step
-// stood back before it touched anything.
-// (five waves per SIMD wherever the key is not an Adam-normalised chain formed in this kernel)
-// AHEAD: slabs of a chunk whose loads are issued together.
-template <bool BF16G, bool BF16V, int SCORE, bool PLANES, int AHEAD = 1>
-__global__ __launch_bounds__(kBlock, AHEAD > 1 ? 1 : (PLANES || SCORE == SGA_SCORE_ABS_G || SCORE == SGA_SCORE_ABS_M ||
-                                      SCORE == SGA_SCORE_ABS_G_BLIND) ? 5 : 1)
-void k_fused_final(
-    FinalArgs a, const sga_segment* __restrict__ segs, int n_segs,
-    const SelState* __restrict__ st, const uint32_t* __restrict__ tile_sel,
-    const uint32_t* __restrict__ tile_eq, int when, const int32_t* __restrict__ seg_dir) {
-  if (when == 3) { if (st->bracket_ok != 0 || st->spec != 0) return; }
-  else if (when != 0 && (st->bracket_ok != 0) != (when == 1)) return;
+// Final sweep: select flags in index order, pack, residual, commit.  Bound by memory from about 8 M
+// coordinates up (nine streams, 5.5 to 6.4 TB/s), by one wave's chain of loads and arithmetic below.  A
+// workgroup per chunk and a wave per slab: with a wave per chunk, its slabs one after the other, a bucket of
+// 261 K coordinates reached one SIMD in four and the last waves of a larger one ran alone.
+// Step, wave per chunk -> wave per slab: 261 K coordinates 45.0 -> 39.4 us, 4 M 90.9 -> 88.4, 10 M 153 -> 143,
+// 20 M 227 -> 215, 63 M 512 -> 512, packed 507 -> 488, 200 M with a mask 1607 -> 1562, without 1470 -> 1476;
+// `update` 1 M 73 -> 62.5, 40 M 463 -> 456.  (Each XCD on a contiguous eighth of packed records, which the
+// wave per chunk liked, costs this one 3 to 5 %.)
+// PLANES: the selection is settled as bit planes where the sampled bracket held; where it failed the radix
+// passes have fixed the threshold and the keys are formed again.
+template <bool BF16G, bool BF16V, int SCORE, bool PLANES>
+__device__ __forceinline__ void final_body(FinalArgs& a, int64_t c, const sga_segment* __restrict__ segs, int n_segs,
+                                           const SelState* __restrict__ st, const uint32_t* __restrict__ tile_sel,
+                                           const uint32_t* __restrict__ tile_eq, const int32_t* __restrict__ seg_dir,
+                                           uint32_t* s_cnt) {
   a.T = st->thresh_bits;
   a.need = st->need;
-  const int64_t n_chunks = cdiv64(a.n, kChunk);
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
   SegCursor sc;                  // wave-uniform (scalar unit)
   sc.init(segs, n_segs, seg_dir);
-  const bool can_full = a.vec && (a.mask_out == nullptr || a.mvec);
-  const unsigned blk = a.pack_extra != 0 ? xcd_contiguous_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  for (int64_t c = (int64_t)blk * kChunksPerBlock + wave_id(); c < n_chunks;
-       c += wstride) {
-    ChunkCursor cur;
-    cur.sel_run = tile_sel[c];
-    cur.eq_run = PLANES ? 0u : tile_eq[c];
-    if (can_full && (c + 1) * kChunk <= a.n) {
-      if (AHEAD == kChunkIters) {
-        final_chunk<BF16G, BF16V, SCORE, true, 0, kChunkIters, PLANES>(a, c, cur, sc);
-        continue;
-      }
-      // one 256-element slab at a time (5 loads in flight per lane): measured
-      // as fast as batching all four slabs, at twice the occupancy
-      final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, true, 1, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, true, 2, 1, PLANES>(a, c, cur, sc);
-      final_chunk<BF16G, BF16V, SCORE, true, 3, 1, PLANES>(a, c, cur, sc);
-    } else {
-      // A ragged chunk slab by slab (four at once would set the register count, and so the occupancy, of
-      // the whole kernel), its whole slabs by the unconditional accesses: the wave that owns it is the last
-      // to finish, which a small bucket waits for.
+  const int slab = uniform_i32(wave_id());
+  const ChunkCursor cur{tile_sel[c], tile_eq[c]};
+  if (a.vec && (a.mask_out == nullptr || a.mvec) && (c + 1) * kChunk <= a.n)
+    final_slab<BF16G, BF16V, SCORE, true, PLANES>(a, c, slab, cur, sc, s_cnt);
+  else
+    final_slab<BF16G, BF16V, SCORE, false, PLANES>(a, c, slab, cur, sc, s_cnt);
+}
+template <bool BF16G, bool BF16V, int SCORE, bool PLANES>
+__global__ __launch_bounds__(kBlock) void k_fused_final(FinalArgs a, const sga_segment* __restrict__ segs, int n_segs,
+                                                        const SelState* __restrict__ st,
+                                                        const uint32_t* __restrict__ tile_sel,
+                                                        const uint32_t* __restrict__ tile_eq,
+                                                        const int32_t* __restrict__ seg_dir) {
+  __shared__ uint32_t s_cnt[2 * kChunkIters];
+  static_assert(kChunkIters == kChunksPerBlock, "a wave per slab");
+  if (PLANES && st->bracket_ok != 0)
+    final_body<BF16G, BF16V, SCORE, true>(a, blockIdx.x, segs, n_segs, st, tile_sel, tile_eq, seg_dir, s_cnt);
+  else
+    final_body<BF16G, BF16V, SCORE, false>(a, blockIdx.x, segs, n_segs, st, tile_sel, tile_eq, seg_dir, s_cnt);
+}
+// The same behind a single-sweep step that stood back before it touched anything (or missed, out of place);
+// otherwise it returns at once, so the grid is a small one that strides over the chunks.
+template <bool BF16G, bool BF16V, int SCORE>
+__global__ __launch_bounds__(kBlock) void k_fused_final_redo(FinalArgs a, const sga_segment* __restrict__ segs, int n_segs,
+                                                        const SelState* __restrict__ st,
+                                                        const uint32_t* __restrict__ tile_sel,
+                                                        const uint32_t* __restrict__ tile_eq,
+                                                        const int32_t* __restrict__ seg_dir) {
+  __shared__ uint32_t s_cnt[2 * kChunkIters];
+  if (st->bracket_ok != 0 || st->spec != 0) return;
+  const int64_t n_chunks = cdiv64(a.n, kChunk);
 #pragma unroll 1
-      for (int sl = 0; sl < kChunkIters; ++sl) {
-        const int64_t s0 = c * kChunk + sl * (kWave * kVec);
-        if (can_full && s0 + kWave * kVec <= a.n) final_chunk<BF16G, BF16V, SCORE, true, 0, 1, PLANES>(a, c, cur, sc, sl);
-        else if (s0 < a.n) final_chunk<BF16G, BF16V, SCORE, false, 0, 1, PLANES>(a, c, cur, sc, sl);
-      }
-    }
+  for (int64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+    final_body<BF16G, BF16V, SCORE, false>(a, c, segs, n_segs, st, tile_sel, tile_eq, seg_dir, s_cnt);
+    __syncthreads();                                               // s_cnt is written again
   }
 }
-
-// Up to this many chunks (four waves per SIMD) every wave of the final sweep is resident at once, so that
-// nothing hides the latency of its four slabs but having all their loads in flight.  Step, one slab at a
-// time -> four, with the same in k_small_sweep: 2 M coordinates 64.8 -> 61.3 us, 4 M 88.3 -> 84.1, eight
-// buckets of 1 M 199 -> 183.  Large buckets have waves enough to hide it (k_fused_final).
-constexpr int64_t kBatchedTiles = 4096;
 
 // One bucket of a (possibly batched) fused step.
 struct FusedJob {
@@ -470,21 +443,13 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     fa.pack_extra = pack_extra;
     fa.adams = adams != 0; fa.fold = (flags & SGA_GC_FOLD) != 0; fa.interval = interval;
     fa.planes = w.pbits;
-    const dim3 one_shot(stream_grid(n_tiles, kChunksPerBlock, 1 << 20));
-    if (planes) {
-      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SGA_SCORE_ABS_G, true>), one_shot, dim3(kBlock), 0, s,
-                         fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 1, w.seg_dir);
-      // the rare other outcome: a small grid that strides over the chunks (returns at once otherwise)
-      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>),
-                         dim3(stream_grid(n_tiles, kChunksPerBlock, 2048)), dim3(kBlock), 0, s, fa,
-                         f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 2, w.seg_dir);
-    } else if (n_tiles <= kBatchedTiles && !Src::kHyper) {
-      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, Src::kHyper ? SGA_SCORE_ABS_G : SCORE, false, kChunkIters>),
-                         one_shot, dim3(kBlock), 0, s, fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 0, w.seg_dir);
-    } else {
-      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>), one_shot, dim3(kBlock), 0, s, fa,
-                         f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, 0, w.seg_dir);
-    }
+    // Adam-normalised scores of large buckets: the settled planes instead of a second evaluation of the chain
+    if (planes)
+      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, Src::kHyper>), dim3((unsigned)n_tiles), dim3(kBlock), 0, s,
+                         fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, w.seg_dir);
+    else
+      hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>), dim3((unsigned)n_tiles), dim3(kBlock), 0, s,
+                         fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, w.seg_dir);
     prof_end(pp, s);
   }
   return check_launch(who);
@@ -1250,9 +1215,9 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
                        0, s, w.st, x.dplane, n, mask_out, (reinterpret_cast<uintptr_t>(mask_out) & 15) == 0);
   // the sweep stood back: the key-forming final sweep does the step (a small grid that strides
   // over the chunks; it returns at once otherwise)
-  hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>),
-                     dim3(stream_grid(n_tiles, kChunksPerBlock, 2048)), dim3(kBlock), 0, s, fa,
-                     segs, n_segs, w.st, w.tile_gt, w.tile_eq, 3, w.seg_dir);
+  hipLaunchKernelGGL((k_fused_final_redo<BF16G, BF16V, SCORE>),
+                     dim3(stream_grid(n_tiles, 1, 2048)), dim3(kBlock), 0, s, fa,
+                     segs, n_segs, w.st, w.tile_gt, w.tile_eq, w.seg_dir);
   return check_launch("sga_fused_sparse_step_single_sweep");
 }
 

@@ -441,13 +441,16 @@ struct SrcReplay {
   __device__ __forceinline__ void chunk_hyper(int64_t c) {
     if (kHyper) sc.seek_uniform(uniform_i64(c) * kChunk);
   }
-  template <bool FULL>
+  __device__ __forceinline__ void slab_hyper(int64_t i0) {
+    if (kHyper) sc.seek_wave(i0);
+  }
+  template <bool FULL, bool KEEP = false>
   __device__ __forceinline__ void fetch(const Chunk& ck, int64_t i, int64_t n, Raw& t) {
-    if (kNeedG) fetch_g<BF16G, FULL>(g, i, n, vec, t.g);
-    if (need_r()) t.r = ldraw_f32<FULL>(res + ck.sh, i, n, vec);
-    if (need_m()) t.m = ldraw_f32<FULL>(m + ck.sh, i, n, vec);
-    if (kNeedW) t.w = ldraw_f32<FULL>(w + ck.sh, i, n, vec);
-    if (kNeedV && !adams) t.v = ldraw_f32<FULL>(v + ck.sh, i, n, vec);
+    if (kNeedG) fetch_g<BF16G, FULL, KEEP>(g, i, n, vec, t.g);
+    if (need_r()) t.r = ldraw_f32<FULL, KEEP>(res + ck.sh, i, n, vec);
+    if (need_m()) t.m = ldraw_f32<FULL, KEEP>(m + ck.sh, i, n, vec);
+    if (kNeedW) t.w = ldraw_f32<FULL, KEEP>(w + ck.sh, i, n, vec);
+    if (kNeedV && !adams) t.v = ldraw_f32<FULL, KEEP>(v + ck.sh, i, n, vec);
   }
   // q of the four coordinates from the raw gradient quad and residual
   __device__ __forceinline__ void form_q(float gd[4], const float rr[4], float coef, float q[4]) const {

@@ -278,12 +278,14 @@ struct SrcF32 {                 // |x| of an fp32 score array
                                 // non-negative scores are told, without a pass of their own)
   using Raw = F4;
   using Chunk = NoChunk;
+  static constexpr bool kHyper = false;
   static constexpr int kAhead = kChunkIters;
   __device__ __forceinline__ Chunk chunk_begin(int64_t) { return Chunk{}; }
   __device__ __forceinline__ void chunk_hyper(int64_t) {}
-  template <bool FULL>
+  __device__ __forceinline__ void slab_hyper(int64_t) {}
+  template <bool FULL, bool KEEP = false>
   __device__ __forceinline__ void fetch(const Chunk&, int64_t i, int64_t n, Raw& r) {
-    r = ldraw_f32<FULL>(x, i, n, vec);
+    r = ldraw_f32<FULL, KEEP>(x, i, n, vec);
   }
   template <bool FULL>
   __device__ __forceinline__ void keys(const Chunk&, int64_t, int64_t, const Raw& r, uint32_t key[4]) {
@@ -724,34 +726,34 @@ struct ChunkCursor {
   uint32_t eq_run;    // ties before the current slab
 };
 
+// Everything a slab's order needs is on the scalar unit: four ballots each for the ties and the selected
+// (a cross-lane scan is six dependent LDS permutes, 0.3 us a slab where nothing hides them).
 __device__ __forceinline__ void slab_select(const uint32_t key[4], const bool valid[4],
                                             uint32_t T, uint32_t need, ChunkCursor& cur,
                                             bool sel[4], uint32_t& pos) {
-  uint32_t my_eq = 0;
-  bool eq[4];
+  uint64_t eq[4], any_eq = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    eq[e] = valid[e] && key[e] == T;
-    my_eq += eq[e];
+    eq[e] = ballot64(valid[e] && key[e] == T);
+    any_eq |= eq[e];
+    sel[e] = valid[e] && key[e] > T;
   }
-  uint32_t eq_rank = cur.eq_run;
-  const uint64_t any_eq = ballot64(my_eq != 0);
-  if (any_eq) {
-    const uint32_t incl = wave_incl_scan(my_eq);
-    eq_rank += incl - my_eq;
-    cur.eq_run += __shfl(incl, kWave - 1, kWave);
+  if (any_eq) {                                  // scalar branch
+    uint32_t rank = cur.eq_run + lanes_below(eq[0]) + lanes_below(eq[1]) + lanes_below(eq[2]) + lanes_below(eq[3]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (valid[e] && key[e] == T) sel[e] = rank++ < need;
+    cur.eq_run += (uint32_t)(__popcll(eq[0]) + __popcll(eq[1]) + __popcll(eq[2]) + __popcll(eq[3]));
   }
-  uint32_t my_sel = 0;
+  uint32_t below = 0, total = 0;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    bool s = valid[e] && key[e] > T;
-    if (eq[e]) { s = eq_rank < need; ++eq_rank; }
-    sel[e] = s;
-    my_sel += s;
+    const uint64_t m = ballot64(sel[e]);
+    below += lanes_below(m);
+    total += (uint32_t)__popcll(m);
   }
-  const uint32_t incl = wave_incl_scan(my_sel);
-  pos = cur.sel_run + incl - my_sel;
-  cur.sel_run += __shfl(incl, kWave - 1, kWave);
+  pos = cur.sel_run + below;
+  cur.sel_run += total;
 }
 
 template <class Src>
@@ -1246,22 +1248,20 @@ __device__ __forceinline__ void plane_put(const Ballot4& a, int it, uint32_t* ld
 // PM: 0 counts only; 1 the provisional selection (keys above the bracket) also goes out as bit
 // planes; 2 as mask bytes, straight into the caller's mask (a mask-only select then needs no
 // expansion pass: the candidates are settled in the bytes).
-// BELOW: `below` also counts the keys right below the range, T_LO - 1.
-template <class Src, bool FULL, int PM, int AHEAD = Src::kAhead, bool BELOW = false>
+template <class Src, bool FULL, int PM>
 __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chunk& ck, int64_t n,
                                               int64_t c, uint32_t T_LO,
                                               uint32_t T_HI, uint32_t& chi, uint32_t& tot_nf,
                                               uint32_t& mycnt, SweepLds& lds,
                                               uint32_t* __restrict__ pbits,
                                               uint8_t* __restrict__ mask_bytes = nullptr,
-                                              bool mvec = false, bool m16 = false,
-                                              uint32_t* below = nullptr) {
+                                              bool mvec = false, bool m16 = false) {
   // The loads of kAhead slabs (256 elements each) are issued together, then
   // their keys are formed slab by slab: expensive key sources (Adam-normalised
   // scores) look fewer slabs ahead to stay within their register budget.  The
   // ragged path (the last chunk) goes one slab at a time through
   // a rolled loop: it only has to be small.
-  constexpr int kAhead = FULL ? AHEAD : 1;
+  constexpr int kAhead = FULL ? Src::kAhead : 1;
   static_assert(kChunkIters % kAhead == 0, "look-ahead divides the slabs of a chunk");
   constexpr int kGroupUnroll = kAhead == kChunkIters ? kChunkIters : 1;
   src.chunk_hyper(c);        // measured: looking the tensor up behind the first loads instead is slower
@@ -1287,7 +1287,6 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
         above.m[e] = ballot64(key[e] >= T_HI) & valid;
         cand.m[e] = ballot64(key[e] >= T_LO) & valid & ~above.m[e];
         nf |= ballot64(key[e] >= 0x7F800000u) & valid;
-        if (BELOW) *below += (uint32_t)__popcll(ballot64(key[e] == T_LO - 1u) & valid);
       }
       chi += above.count();
       if (nf) {                                  // rare: count them properly

@@ -27,55 +27,88 @@ namespace sga {
 
 #ifdef __HIPCC__
 
-// Candidate lists of the small path: WGs of the sweep share kSmallSegs counters (the segments of
-// the list); a segment has room for every coordinate of its workgroups, so it never overflows.
+// Candidate lists of the small path: the chunks of the sweep share kSmallSegs counters (the segments of
+// the list); a segment has room for every coordinate of its chunks, so it never overflows.
 // The counters lie 256 bytes apart: atomics on one cache line queue like those on one address (11 ns
 // each; 1024 workgroups on 16 adjacent words: the sweep of 4 M elements took 19 us, 8.6 with this).
-struct SmallGeom { uint32_t n_wg, segs, cap; };    // cap: list entries per segment
-__host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles) {
+struct SmallGeom { uint32_t segs, cap; };          // cap: list entries per segment
+__host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles, int cpw) {
   SmallGeom s;
-  s.n_wg = (uint32_t)cdiv64(n_tiles, kChunksPerBlock);
-  const uint32_t per = (uint32_t)cdiv64(s.n_wg, kSmallSegs);
-  s.segs = (uint32_t)cdiv64(s.n_wg, per);
-  s.cap = per * (uint32_t)kBlockSpan;
+  const uint32_t n_wg = (uint32_t)cdiv64(n_tiles, cpw), per = (uint32_t)cdiv64(n_wg, kSmallSegs);
+  s.segs = (uint32_t)cdiv64(n_wg, per);
+  s.cap = (per * cpw < 2 ? 2 : per * cpw) * (uint32_t)kChunk;      // two chunks hold the head that is read unseen
   return s;
 }
 
-// The sweep: one chunk per wave, counts above the bracket, keys inside it to the list (one
-// reservation per workgroup).  Keys equal to the bracket's lower end are counted per chunk and not
+// The sweep: a workgroup per chunk and a wave per slab, so that a bucket of a few hundred chunks still
+// reaches every SIMD; counts above the bracket, keys inside it to the list (one reservation per chunk).
+// Keys equal to the bracket's lower end are counted per chunk and not
 // listed: a plateau of equal keys (zeros, momenta that have decayed to the last denormal) puts the
 // lower end on itself, and the one workgroup behind the sweep would walk a list as long as the bucket
 // (|m| after a thousand sparse steps, 1.7 M coordinates: 889 us, 86 like this).
-template <class Src>
+// Chunks per workgroup (CPW): one up to kSweepTiles chunks and for the scores that are a chain of arithmetic;
+// beyond, four, whose loads are in flight together (a reservation per 4096 coordinates, half the waves).
+// Step of 261 K coordinates with one / four 36.1 / 38.8 us, 2 M 59.2 / 62.3, 8.3 M 145 / 140; `update`
+// 261 K 50.5 / 57.4, 8.3 M 159 / 166; select of 3 M scores 70.4 / 67.4.
+constexpr int64_t kSweepTiles = 2048;
+template <class Src, int CPW>
 __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, ChainJobs jobs) {
   const ChainJob& J = jobs.j[blockIdx.y];
-  const int64_t n = J.n, n_chunks = J.n_tiles;
-  if ((int64_t)blockIdx.x * kChunksPerBlock >= n_chunks) return;      // a smaller job of the batch
-  __shared__ SweepLds s_lds[kChunksPerBlock];
-  __shared__ uint32_t s_cnt[kChunksPerBlock], s_nf[kChunksPerBlock], s_base;
+  const int64_t n = J.n, n_chunks = J.n_tiles, c0 = (int64_t)blockIdx.x * CPW;
+  if (c0 >= n_chunks) return;                         // a smaller job of the batch
+  __shared__ uint32_t s_hi[CPW][kChunkIters], s_eq[CPW][kChunkIters], s_cnt[kChunkIters], s_nf[kChunkIters], s_base;
+  static_assert(kChunkIters == kChunksPerBlock && CPW <= kWave, "a wave per slab");
   SelState* __restrict__ st = J.st;
   Src src = srcs.s[blockIdx.y];
+  const int64_t i0 = c0 * kChunk + uniform_i32(wave_id()) * (kWave * kVec);
+  typename Src::Raw raw[CPW];
+#pragma unroll
+  for (int u = 0; u < CPW; ++u) {
+    const typename Src::Chunk ck = src.chunk_begin(c0 + u);
+    const int64_t i = i0 + u * kChunk + lane_id() * kVec;
+    if (src.vec && (c0 + u + 1) * kChunk <= n) src.template fetch<true, true>(ck, i, n, raw[u]);  // read again soon
+    else if (i < n) src.template fetch<false>(ck, i, n, raw[u]);
+  }
+  src.slab_hyper(i0);
   const uint32_t T_LO = st->t_lo, T_HI = st->t_hi;
-  const int64_t c = (int64_t)blockIdx.x * kChunksPerBlock + wave_id();
-  const bool full = src.vec && (c + 1) * kChunk <= n;
-  SweepLds& lds = s_lds[wave_id()];
-  uint32_t chi = 0, nf = 0, cnt = 0, eq = 0;
-  if (c < n_chunks) {
-    const typename Src::Chunk ck = src.chunk_begin(c);
-    // small grids: the latency of a chunk's four slabs counts, not how many waves are resident
-    if (full)
-      bracket_chunk<Src, true, 0, kChunkIters, true>(src, ck, n, c, T_LO + 1u, T_HI, chi, nf, cnt, lds, nullptr,
-                                                     nullptr, false, false, &eq);
-    else
-      bracket_chunk<Src, false, 0, 1, true>(src, ck, n, c, T_LO + 1u, T_HI, chi, nf, cnt, lds, nullptr, nullptr, false,
-                                            false, &eq);
-    if (lane_id() == 0) { J.tile_gt[c] = chi; J.tile_eq[c] = eq; }
+  uint32_t key[CPW][4], cnt = 0, nf = 0;
+  Ballot4 cand[CPW];
+#pragma unroll
+  for (int u = 0; u < CPW; ++u) {
+    const typename Src::Chunk ck = src.chunk_begin(c0 + u);
+    const int64_t i = i0 + u * kChunk + lane_id() * kVec;
+    const bool full = src.vec && (c0 + u + 1) * kChunk <= n;
+    if (u > 0) src.slab_hyper(i0 + u * kChunk);
+    key[u][0] = key[u][1] = key[u][2] = key[u][3] = 0u;
+    if (full) src.template keys<true>(ck, i, n, raw[u], key[u]);
+    else if (i < n) src.template keys<false>(ck, i, n, raw[u], key[u]);
+    uint32_t hi = 0, eq = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint64_t valid = full ? ~0ull : ballot64(i + e < n);
+      const uint64_t above = ballot64(key[u][e] >= T_HI) & valid;
+      cand[u].m[e] = ballot64(key[u][e] > T_LO) & valid & ~above;
+      hi += (uint32_t)__popcll(above);
+      eq += (uint32_t)__popcll(ballot64(key[u][e] == T_LO) & valid);
+      nf += (uint32_t)__popcll(ballot64(key[u][e] >= 0x7F800000u) & valid);
+    }
+    cnt += cand[u].count();
+    if (lane_id() == 0) { s_hi[u][wave_id()] = hi; s_eq[u][wave_id()] = eq; }
   }
   const bool neg = ballot64(src_negative(src) != 0u) != 0ull;
-  if (lane_id() == 0) { s_cnt[wave_id()] = cnt; s_nf[wave_id()] = nf | (neg ? 0x80000000u : 0u); }
+  if (lane_id() == 0) {
+    s_cnt[wave_id()] = cnt;
+    s_nf[wave_id()] = nf | (neg ? 0x80000000u : 0u);
+  }
   __syncthreads();
-  const SmallGeom geo = small_geom(n_chunks);
+  const SmallGeom geo = small_geom(n_chunks, CPW);
   const uint32_t seg = blockIdx.x % geo.segs;
+  if (threadIdx.x < CPW && c0 + (int)threadIdx.x < n_chunks) {
+    const uint32_t* h = s_hi[threadIdx.x];
+    const uint32_t* q = s_eq[threadIdx.x];
+    J.tile_gt[c0 + threadIdx.x] = h[0] + h[1] + h[2] + h[3];
+    J.tile_eq[c0 + threadIdx.x] = q[0] + q[1] + q[2] + q[3];
+  }
   if (threadIdx.x == 0) {
     const uint32_t all = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     const uint32_t f = (s_nf[0] + s_nf[1] + s_nf[2] + s_nf[3]) & 0x7FFFFFFFu;
@@ -84,21 +117,14 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
     if ((s_nf[0] | s_nf[1] | s_nf[2] | s_nf[3]) & 0x80000000u) raise_negative(st);
   }
   __syncthreads();
-  if (cnt == 0) return;
-  uint32_t base = seg * geo.cap + s_base;
-  for (int w = 0; w < wave_id(); ++w) base += s_cnt[w];
-  if (cnt <= (uint32_t)kWaveCandCap) {
-    for (uint32_t j = lane_id(); j < cnt; j += kWave) {
-      J.small_idx[base + j] = lds.idx[j];
-      J.small_key[base + j] = lds.key[j];
-    }
-    return;
-  }
-  // more keys than the wave's LDS holds: the bracket's keys crowd into few chunks
-  recollect(src, n, c, T_LO + 1u, T_HI, [&](uint32_t pos, uint32_t idx, uint32_t key) {
-    J.small_idx[base + pos] = idx;
-    J.small_key[base + pos] = key;
-  });
+  uint32_t run = seg * geo.cap + s_base;
+  for (int w = 0; w < wave_id(); ++w) run += s_cnt[w];
+#pragma unroll
+  for (int u = 0; u < CPW; ++u)
+    ballot_append(cand[u], run, [&](uint32_t pos, int e) {
+      J.small_idx[pos] = (uint32_t)(i0 + u * kChunk + lane_id() * kVec + e);
+      J.small_key[pos] = key[u][e];
+    });
 }
 
 // The candidate list as the finishing workgroup sees it: wave w owns segment w (kSmallSegs ==
@@ -117,7 +143,7 @@ struct SmallList {
     static_assert(kSmallSegs == kWideWaves, "one list segment per wave");
     keys = reinterpret_cast<const U4*>(J.small_key + (int64_t)wave_id() * geo.cap);
     idxs = reinterpret_cast<const U4*>(J.small_idx + (int64_t)wave_id() * geo.cap);
-    const bool mine = (uint32_t)wave_id() < geo.segs;   // a segment has room for 4096 entries at least
+    const bool mine = (uint32_t)wave_id() < geo.segs;   // a segment has room for 2048 entries at least
 #pragma unroll
     for (int u = 0; u < kSmallHead; ++u)
       if (mine) { key[u] = keys[u * kWave + lane_id()]; idx[u] = idxs[u * kWave + lane_id()]; }
@@ -157,7 +183,7 @@ struct SmallList {
     }
   }
 };
-static_assert(kSmallHead * kWave * kVec <= kBlockSpan, "the head never reaches past a segment");
+static_assert(kSmallHead * kWave * kVec <= 2 * kChunk, "the head never reaches past a segment");
 
 // A bracket that missed: the radix descent and the chunk counts over the data itself, as items of one
 // queue that every workgroup of the launch works on (the way of k_tail: whoever waits holds a later
@@ -242,7 +268,7 @@ __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t
 }
 
 template <class Src>
-__global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs) {
+__global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs, int cpw) {
   __shared__ __align__(16) uint32_t s_hist[kBinsBig];
   __shared__ __align__(16) uint32_t s_tile[kSmallTiles];          // above | ties << 16, at most 1024 each
   __shared__ __align__(16) uint32_t s_key[kWideList];
@@ -255,7 +281,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   const int nt = (int)J.n_tiles;
   const uint32_t k = J.k, T_LO = st->t_lo, T_HI = st->t_hi;
   const bool single = T_HI - T_LO == 1u;
-  const SmallGeom geo = small_geom(nt);
+  const SmallGeom geo = small_geom(nt, cpw);
   SmallList list;
   list.request(J, geo);
   constexpr int PER = kSmallTiles / kWide;            // 8
@@ -451,11 +477,15 @@ static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B,
                                     hipStream_t s) {
   launch_sample_coarse(srcs, B, dirs, false, s);
   hipLaunchKernelGGL((k_pick_coarse<false>), B.grid(1), dim3(kWide), 0, s, B.jobs, kBracketSigmas);
-  hipLaunchKernelGGL((k_small_sweep<Src>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)), dim3(kBlock),
-                     0, s, srcs, B.jobs);
+  const int cpw = Src::kHyper || B.max_tiles <= kSweepTiles ? 1 : 4;
+  if (cpw == 1)
+    hipLaunchKernelGGL((k_small_sweep<Src, 1>), B.grid((unsigned)B.max_tiles), dim3(kBlock), 0, s, srcs, B.jobs);
+  else
+    hipLaunchKernelGGL((k_small_sweep<Src, Src::kHyper ? 1 : 4>), B.grid((unsigned)cdiv64(B.max_tiles, 4)), dim3(kBlock), 0,
+                       s, srcs, B.jobs);
   const int64_t wgs = cdiv64(B.max_tiles, kRedoTiles);
   hipLaunchKernelGGL((k_small_finish<Src>), B.grid((unsigned)(wgs < kRedoGroups ? wgs : kRedoGroups)), dim3(kWide), 0,
-                     s, srcs, B.jobs);
+                     s, srcs, B.jobs, cpw);
 }
 
 #endif  // __HIPCC__

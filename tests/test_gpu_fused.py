@@ -336,3 +336,17 @@ def test_multi_bucket_step_refusals(dev):
     fs[1] = FusedSparseStep(n, segs, dev, values_dtype=torch.bfloat16)
     with pytest.raises(ValueError, match="share the gradient and value dtypes"):
         fused_step_multi(fs, t, t, t, t, t, 1, ratio_percent=1.0)
+
+
+# a wave owns a slab of 256 coordinates, a workgroup a chunk of 1024 (the select's sweep four of them above
+# 2048 chunks): lengths at those edges, tensors that end inside a slab, more tensors than a wave has lanes
+@pytest.mark.parametrize("score", ["abs_g", "update"])
+@pytest.mark.parametrize("n", [255, 257, 1023, 1025, 4097, 2048 * 1024, 2048 * 1024 + 1025, 9_000_001])
+def test_lengths_at_slab_and_chunk_edges(dev, n, score):
+    sizes, left = [], n
+    while left > 0 and len(sizes) < 150:
+        sizes.append(min(left, (3, 130, 700, 61)[len(sizes) % 4]))
+        left -= sizes[-1]
+    if left:
+        sizes.append(left)
+    _run(dev, sizes, 1, 1.0, torch.bfloat16, torch.bfloat16, score=score, vary=True)
