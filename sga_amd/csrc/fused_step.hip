@@ -34,6 +34,11 @@ struct SrcFused {
   // Stepwise interface of the one-sweep select.
   struct Raw { RawG g; F4 r, p, m, v; };
   struct Chunk { int64_t sh; };
+  static constexpr bool kReadAgain = true;                     // by the final sweep
+  int bytes() const {                                          // what a sweep reads of a coordinate
+    return (kNeedG && (BF16G || g) ? (BF16G ? 2 : 4) : 0) +
+           4 * ((kNeedR ? 1 : 0) + (need_m() ? 1 : 0) + (kNeedP ? 1 : 0) + (kNeedV && !adams ? 1 : 0));
+  }
   // scores that need the tensor's hyper-parameters
   static constexpr bool kHyper = SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI ||
                                  SCORE == SGA_SCORE_GR_OVER_SQRT_V;
@@ -44,7 +49,7 @@ struct SrcFused {
   static constexpr bool kNeedR = kNeedG && SCORE != SGA_SCORE_ABS_G_BLIND;
   static constexpr bool kNeedP = SCORE == SGA_SCORE_UPDATE;
   static constexpr bool kNeedV = kHyper;                       // v, or m in its place under AdamS
-  __device__ __forceinline__ bool need_m() const {
+  __host__ __device__ __forceinline__ bool need_m() const {
     return SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI || SCORE == SGA_SCORE_ABS_M ||
            (kNeedV && adams);
   }
@@ -368,6 +373,13 @@ __global__ __launch_bounds__(kBlock) void k_fused_final_redo(FinalArgs a, const 
   }
 }
 
+// Up to this many bytes the select's sweep loads by ordinary accesses, which leave its inputs in the 256 MB
+// memory-side cache for the final sweep to find; non-temporal ones do not, but a longer sweep runs faster by
+// them and little of it would survive.  Step, without -> with: |g + r| 10 M coordinates (60 MB) 141 -> 137 us,
+// 40 M 349 -> 328, 63 M (378 MB) 516 -> 491, 150 M (900 MB) 1158 -> 1145; `update` 20 M (360 MB) 276 -> 274,
+// 40 M (720 MB) 453 -> 459, 63 M 660 -> 683, 100 M 992 -> 1036.
+constexpr int64_t kKeepBytes = 512ll << 20;
+
 // One bucket of a (possibly batched) fused step.
 struct FusedJob {
   const void* g;
@@ -425,7 +437,9 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   if (small) {
     run_small_select(srcs, B, dj, s);
   } else {
-    run_select_batch<0>(srcs, B, dj, use_fast, planes ? 1 : 0, s);
+    int64_t swept = 0;
+    for (int b = 0; b < count; ++b) swept += fj[b].n * srcs.s[b].bytes();
+    run_select_batch<0>(srcs, B, dj, use_fast, planes ? 1 : 0, s, swept <= kKeepBytes);
   }
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];

@@ -420,6 +420,7 @@ struct SrcReplay {
   // Stepwise interface of the one-sweep select.
   struct Raw { RawG g; F4 r, w, m, v; };
   struct Chunk { int64_t sh; float coef; };
+  static constexpr bool kReadAgain = false;
   static constexpr bool kHyper = SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI ||
                                  SCORE == SGA_SCORE_GR_OVER_SQRT_V;
   static constexpr bool kNeedG = SCORE != SGA_SCORE_ABS_M;

@@ -278,7 +278,7 @@ struct SrcF32 {                 // |x| of an fp32 score array
                                 // non-negative scores are told, without a pass of their own)
   using Raw = F4;
   using Chunk = NoChunk;
-  static constexpr bool kHyper = false;
+  static constexpr bool kHyper = false, kReadAgain = false;
   static constexpr int kAhead = kChunkIters;
   __device__ __forceinline__ Chunk chunk_begin(int64_t) { return Chunk{}; }
   __device__ __forceinline__ void chunk_hyper(int64_t) {}
@@ -1248,7 +1248,8 @@ __device__ __forceinline__ void plane_put(const Ballot4& a, int it, uint32_t* ld
 // PM: 0 counts only; 1 the provisional selection (keys above the bracket) also goes out as bit
 // planes; 2 as mask bytes, straight into the caller's mask (a mask-only select then needs no
 // expansion pass: the candidates are settled in the bytes).
-template <class Src, bool FULL, int PM>
+// KEEP: a pass behind the select reads the same data again and finds it in the memory-side cache.
+template <class Src, bool FULL, int PM, bool KEEP>
 __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chunk& ck, int64_t n,
                                               int64_t c, uint32_t T_LO,
                                               uint32_t T_HI, uint32_t& chi, uint32_t& tot_nf,
@@ -1271,7 +1272,7 @@ __device__ __forceinline__ void bracket_chunk(Src& src, const typename Src::Chun
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
       const int64_t i = c * kChunk + (g0 + u) * (kWave * kVec) + lane_id() * kVec;
-      if (FULL || i < n) src.template fetch<FULL>(ck, i, n, raw[u]);
+      if (FULL || i < n) src.template fetch<FULL, KEEP>(ck, i, n, raw[u]);
     }
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
@@ -1340,7 +1341,7 @@ __device__ __forceinline__ void recollect(Src& src, int64_t n, int64_t c, uint32
 
 // A bracket of a single key (a plateau of equal keys holds the k-th one) collects nothing: its members
 // are ties, counted per chunk (tile_eq) and in bin 0 of the relative histogram.
-template <class Src, int PM>
+template <class Src, int PM, bool KEEP = false>
 __global__ __launch_bounds__(kBlock) void k_bracket_sweep(
     Src src, int64_t n, SelState* __restrict__ st, uint32_t* __restrict__ rel,
     uint32_t* __restrict__ tile_gt, uint32_t* __restrict__ tile_eq, uint32_t* __restrict__ seg_idx,
@@ -1361,9 +1362,9 @@ __global__ __launch_bounds__(kBlock) void k_bracket_sweep(
     SweepLds& lds = s_lds[wave_id()];
     const typename Src::Chunk ck = src.chunk_begin(c);
     if (src.vec && (c + 1) * kChunk <= n)
-      bracket_chunk<Src, true, PM>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec, m16);
+      bracket_chunk<Src, true, PM, KEEP>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec, m16);
     else
-      bracket_chunk<Src, false, PM>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec);
+      bracket_chunk<Src, false, PM, KEEP>(src, ck, n, c, T_LO, T_HI, chi, tot_nf, mycnt, lds, pbits, mask_bytes, mvec);
     if (single) { ties = mycnt; mycnt = 0; }
     if (lane_id() == 0) { tile_gt[c] = chi; tile_eq[c] = ties; }   // chi / tot_nf are wave totals
     if (mycnt) {                                        // wave-uniform
@@ -2126,8 +2127,9 @@ static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, co
   launch_sample_fine(srcs, B, s);
   chain_pick_fine(B, sigmas, s);
 }
+// keep (sources that a writing pass reads again): see bracket_chunk
 template <class Src>
-static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int pm, hipStream_t s) {
+static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int pm, hipStream_t s, bool keep = false) {
   for (int b = 0; b < B.count; ++b) {
     const ChainJob& J = B.jobs.j[b];
     const SelWorkspace& w = B.w[b];
@@ -2135,19 +2137,18 @@ static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int
     ProfPair* pp = prof_begin(SGA_PROF_SELECT_SWEEP, s);
     // the sweep's two totals go through 256 partial counters (blk_gt / blk_eq are free until
     // the tile scan, which runs after the settlement has read them)
-    if (pm == 2)
-      hipLaunchKernelGGL((k_bracket_sweep<Src, 2>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
-                         w.seg_cnt, (uint32_t)w.seg_cap, (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
-                         J.mask, true);
-    else if (pm == 1)
-      hipLaunchKernelGGL((k_bracket_sweep<Src, 1>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
-                         w.seg_cnt, (uint32_t)w.seg_cap, J.planes, w.blk_gt, w.blk_eq);
-    else
-      hipLaunchKernelGGL((k_bracket_sweep<Src, 0>), dim3(sweep_blocks), dim3(kBlock), 0, s,
-                         srcs.s[b], J.n, w.st, w.rel, w.tile_gt, w.tile_eq, w.seg_idx, w.seg_key,
-                         w.seg_cnt, (uint32_t)w.seg_cap, (uint32_t*)nullptr, w.blk_gt, w.blk_eq);
+    auto sweep = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(sweep_blocks), dim3(kBlock), 0, s, srcs.s[b], J.n, w.st, w.rel, w.tile_gt,
+                         w.tile_eq, w.seg_idx, w.seg_key, w.seg_cnt, (uint32_t)w.seg_cap,
+                         pm == 1 ? J.planes : (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
+                         pm == 2 ? J.mask : (uint8_t*)nullptr, true);
+    };
+    constexpr bool again = Src::kReadAgain;
+    if (pm == 2) sweep(k_bracket_sweep<Src, 2>);
+    else if (pm == 1 && keep) sweep(k_bracket_sweep<Src, 1, again>);
+    else if (pm == 1) sweep(k_bracket_sweep<Src, 1>);
+    else if (keep) sweep(k_bracket_sweep<Src, 0, again>);
+    else sweep(k_bracket_sweep<Src, 0>);
     prof_end(pp, s);
   }
 }
@@ -2167,10 +2168,10 @@ static inline void chain_tail(const SrcPack<Src>& srcs, const SelBatch& B, hipSt
 
 template <int OUT, class Src>
 static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, bool fast,
-                                    int pm, hipStream_t s) {
+                                    int pm, hipStream_t s, bool keep = false) {
   if (fast) {
     chain_bracket(srcs, B, dirs, kBracketSigmas, s);
-    chain_sweeps(srcs, B, pm, s);
+    chain_sweeps(srcs, B, pm, s, keep);
     chain_settle(B, s);
   } else {
     chain_begin(B, dirs, false, s);
