@@ -167,11 +167,15 @@ __device__ __forceinline__ T wave_sum(T v) {
 // Inclusive scan across the 64 lanes of a wave: shifts inside the rows of 16 lanes, then the rows' last
 // lanes broadcast to the rows behind (six data-parallel-primitive adds; six LDS permutes are ten times
 // their latency).
-__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+__device__ __forceinline__ uint32_t row_incl_scan(uint32_t v) {                      // of every row of 16 lanes
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xf, 0xf, true);      // row_shr:1
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xf, 0xf, true);      // row_shr:2
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xf, 0xf, true);      // row_shr:4
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xf, 0xf, true);      // row_shr:8
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v) {
+  v = row_incl_scan(v);
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xa, 0xf, false);     // row_bcast:15
   v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xc, 0xf, false);     // row_bcast:31
   return v;

@@ -816,24 +816,30 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
       });
     }
   };
+  auto dirs_of = [&](auto& srcs, const SelBatch& sub) {
+    using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
+    SegDirJobs dirs = {};                // only the Adam-normalised scores ever look a tensor up
+    for (int b = 0; Src::kHyper && b < sub.count; ++b) {
+      dirs.j[b].segs = segs; dirs.j[b].dir = sub.w[b].seg_dir; dirs.j[b].n = n; dirs.j[b].n_segs = n_segs;
+    }
+    return dirs;
+  };
   if (small) {
     per_score([&](auto& srcs, const SelBatch& sub) {
       using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
-      SegDirJobs dirs = {};
-      for (int b = 0; Src::kHyper && b < sub.count; ++b) {
-        dirs.j[b].segs = segs; dirs.j[b].dir = sub.w[b].seg_dir; dirs.j[b].n = n; dirs.j[b].n_segs = n_segs;
-      }
-      run_small_select(srcs, sub, dirs, s);
+      run_small_select(srcs, sub, dirs_of(srcs, sub), s);
       hipLaunchKernelGGL((k_write_bits<Src>), sub.grid((unsigned)cdiv64(sub.max_tiles, kChunksPerBlock)),
                          dim3(kBlock), 0, s, srcs, sub.jobs);
     });
     return check_launch(who);
   }
-  if (!any_hyper) dj = {};               // only the Adam-normalised scores ever look a tensor up
-  chain_begin(B, dj, fast, s);
-  if (fast) {
-    per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_coarse(srcs, sub, SegDirJobs{}, true, s); });
-    chain_pick_coarse(B, kBracketSigmas, s);
+  if (!fast) {
+    if (!any_hyper) dj = {};             // only the Adam-normalised scores ever look a tensor up
+    chain_begin(B, dj, s);
+  } else {
+    per_score([&](auto& srcs, const SelBatch& sub) {
+      launch_sample_pick<true>(srcs, sub, dirs_of(srcs, sub), kBracketSigmas, s);
+    });
     per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, s); });
     chain_pick_fine(B, kBracketSigmas, s);
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, 1, s); });

@@ -253,7 +253,7 @@ extern "C" int sga_sel_begin(int64_t k, void* ws, size_t ws_bytes, void* stream)
   }
   SelBatch B;
   B.add(w, 1, k, 0);
-  chain_begin(B, SegDirJobs{}, false, (hipStream_t)stream);
+  chain_begin(B, SegDirJobs{}, (hipStream_t)stream);
   return check_launch("sga_sel_begin");
 }
 

@@ -56,8 +56,10 @@ struct SelState {
   uint32_t finish_ticket; // k_small_finish: workgroups that have begun; the first one judges the bracket ...
   uint32_t verdict;     // ... 1: it holds the k-th key, 2: all of them go over the data again
   uint32_t redo_step;   // passes of that which are done
-  uint32_t pad_[28];
+  uint32_t sampled[16]; // k_sample_pick: the launch that a workgroup of the sample has finished in
+  uint32_t pad_[12];
 };
+static_assert(sizeof(SelState) == 256, "whole cache lines");
 static_assert(sizeof(SelState) == 256, "SelState layout");
 
 struct SelWorkspace {
@@ -928,24 +930,30 @@ __device__ __forceinline__ int rel_shift(uint32_t lo, uint32_t hi, int bins) {
   return w > b ? w - b : 0;
 }
 
-// First kernel of a select of the large buckets: clears the histograms and counters, resets the state to
-// rank k, builds the directories of the segment tables (dirs.j[job].dir null: none wanted).
-static __global__ __launch_bounds__(kBlock) void k_chain_begin(ChainJobs jobs, SegDirJobs dirs, int fast) {
+// What the kernels of a large bucket's select count in.
+__device__ __forceinline__ void clear_large(const ChainJob& J, int t0, int step, bool fast) {
+  for (int i = t0; i < kHistStride * 2; i += step) J.hist[i] = 0u;
+  if (!fast) return;
+  for (int i = t0; i <= kSegWaves + 1; i += step) J.seg_cnt[i] = 0u;     // + overflow count
+  for (int i = t0; i < kSweepParts; i += step) { J.blk_gt[i] = 0u; J.blk_eq[i] = 0u; }
+  for (int i = t0; i < kRelWords; i += step) J.rel[i] = 0u;
+  if (J.seg_fail)
+    for (int i = t0; i < kSegWaves; i += step) J.seg_fail[i] = 0u;
+}
+// The directory of a job's segment table (dirs.j[job].dir null: none wanted).
+__device__ __forceinline__ void seg_dirs(const SegDirJobs& dirs, int job, int t0, int step) {
+  const auto& D = dirs.j[job];
+  if (!D.dir) return;
+  const int nb = (int)((D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog);
+  for (int b = t0; b < nb; b += step) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
+}
+
+// First kernel of a select of the large buckets that goes by radix passes alone.
+static __global__ __launch_bounds__(kBlock) void k_chain_begin(ChainJobs jobs, SegDirJobs dirs) {
   const ChainJob& J = jobs.j[blockIdx.y];
   const int t0 = blockIdx.x * kBlock + threadIdx.x, step = gridDim.x * kBlock;
-  for (int i = t0; i < kHistStride * 2; i += step) J.hist[i] = 0u;
-  if (fast) {
-    for (int i = t0; i <= kSegWaves + 1; i += step) J.seg_cnt[i] = 0u;   // + overflow count
-    for (int i = t0; i < kSweepParts; i += step) { J.blk_gt[i] = 0u; J.blk_eq[i] = 0u; }
-    for (int i = t0; i < kRelWords; i += step) J.rel[i] = 0u;
-    if (J.seg_fail)
-      for (int i = t0; i < kSegWaves; i += step) J.seg_fail[i] = 0u;
-  }
-  const auto& D = dirs.j[blockIdx.y];
-  if (D.dir) {
-    const int nb = (int)((D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog);
-    for (int b = t0; b < nb; b += step) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
-  }
+  clear_large(J, t0, step, false);
+  seg_dirs(dirs, blockIdx.y, t0, step);
   if (t0 != 0) return;
   SelState z = {};
   z.k = J.k;
@@ -961,35 +969,6 @@ __device__ __forceinline__ auto drop_dir(S& s, int) -> decltype(s.sc.dir, void()
 template <class S>
 __device__ __forceinline__ void drop_dir(S&, long) {}
 
-// Sample keys (one quad per window at a hashed offset; the windows tile all quads, see quad_of_window),
-// the list counters, and, in a job's last workgroup, the directory of its segment table
-// (dirs.j[job].dir null: none wanted).  Gathering from one workgroup would be bound by one CU's
-// translation misses (4096 quads of two arrays: 25 us; 64 workgroups: 4).
-template <class Src>
-__global__ __launch_bounds__(kBlock) void k_sample_coarse(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
-                                                          int of_fine) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  if (blockIdx.x == gridDim.x - 1) {
-    if (threadIdx.x < kSmallSegs) J.seg_cnt[threadIdx.x * kSmallSegStride] = 0u;
-    const auto& D = dirs.j[blockIdx.y];
-    if (D.dir) {
-      const int64_t nb = (D.n + (1ll << kSegDirLog) - 1) >> kSegDirLog;
-      for (int64_t b = threadIdx.x; b < nb; b += kBlock) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
-    }
-    return;
-  }
-  Src src = srcs.s[blockIdx.y];
-  drop_dir(src, 0);
-  const int64_t n_sv = small_sample_vecs(J.n);
-  const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (j >= n_sv) return;
-  // of_fine: a subset of the windows of the large buckets' fine sample, which it then agrees with
-  const int64_t all = of_fine ? J.n_sv : n_sv;
-  uint32_t key[4];
-  src.template load<false>(quad_of_window(j * all / n_sv, J.n / 4, all, J.seed) * 4, J.n, key);
-  reinterpret_cast<U4*>(J.sample)[j] = U4{key[0], key[1], key[2], key[3]};
-}
-
 // Ranks in a sample of ns keys (1-based from the top) between which the k-th of n lies.
 struct RankEnds { double hi, lo; };
 __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns, double sigmas) {
@@ -998,35 +977,92 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
   return RankEnds{floor(r - d), ceil(r + d)};
 }
 
-// One workgroup per job: state reset, the two ends of the bracket from the sample.  The top 12 bits of
-// all keys go into one LDS histogram, the next 12 of the keys in the two bins the ends fall into into
-// one each; what is left in a bin then is ranked by counting (or split by the last 7 bits, on plateaus).
+// First kernel of a select by a sampled bracket: the sample, the two ends of the bracket from it, the state.
 //
-// The small buckets bracket the k-th key of the data this way (sigmas: kBracketSigmas).  The large ones
+// kSampleGroups workgroups take the sample (one quad per window at a hashed offset, see quad_of_window): one
+// alone would be bound by its CU's translation misses (4096 quads of two arrays: 25 us).  A workgroup that has
+// left its keys leaves the launch's number beside them and looks at the others': whoever sees all of them picks.
+// Nobody waits for anybody, and two that see all numbers at once do the same and write the same.  (Numbers of an
+// earlier launch are gone: the pick writes the whole state.  Memory that happens to hold the number could only
+// spoil the sample, and the select is exact for any.)  As two launches (three with the clearing kernel of the large
+// buckets) before -> after, us: step of 261 K 36.0 -> 34.4, 4 M 77.5 -> 74.3, 40 M 429 -> 419; select of 3 M 68.5 -> 60.8.
+//
+// The pick: one LDS histogram of the top 13 bits of all keys.  The ends of the bins that the two ends of the
+// bracket fall into will do, rounded outwards, as long as that takes in no more than a quarter of the bracket's
+// own ranks in addition; otherwise (narrow distributions, plateaus) the next 12 bits of the keys in the two bins
+// go into a histogram each, and what is left in a bin then is ranked by counting, or split by the last 6 bits.
+// kBracketSigmas etc.: the small buckets bracket the k-th key of the data this way.  The large ones
 // (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with eight
 // sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.  Sigma
 // is that of independent keys; scores that the four neighbours of a quad share halve it.  Such scores
 // missed in 32 of 1000 draws of 40 M coordinates at 10 % with four sigma, and in 12 with eight (the fine
 // sample's own five, halved); a wider coarse bracket costs the fine one a few keys of resolution.
-template <bool COARSE>
-__global__ __launch_bounds__(kWide) void k_pick_coarse(ChainJobs jobs, double sigmas) {
+//
+// The workgroups behind those of the sample keep house: counters and histograms of the kernels behind this one,
+// the directories of the segment tables (dirs.j[job].dir null: none wanted).
+constexpr int kSampleGroups = 16;
+constexpr int kPickBits = 13, kPickShift = 31 - kPickBits;
+template <class Src, bool COARSE>
+__global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
+                                                       uint32_t launch, double sigmas) {
   const ChainJob& J = jobs.j[blockIdx.y];
+  if (blockIdx.x >= kSampleGroups) {
+    const int t0 = (blockIdx.x - kSampleGroups) * kWide + threadIdx.x, step = (gridDim.x - kSampleGroups) * kWide;
+    if (COARSE) clear_large(J, t0, step, true);
+    else if (t0 < kSmallSegs) J.seg_cnt[t0 * kSmallSegStride] = 0u;
+    seg_dirs(dirs, blockIdx.y, t0, step);
+    return;
+  }
   __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
   __shared__ __align__(16) uint32_t s_list[2][kWideList];
-  __shared__ uint32_t s_cnt[2], s_out[2][3];
+  __shared__ uint32_t s_cnt[2], s_out[2][3], s_all;
   __shared__ WideScratch s_scan;
+  static_assert(1 << kPickBits == 2 * kBinsBig, "the two small histograms are the first one");
+  SelState* st = J.st;
   const int64_t n = J.n;
-  const int64_t n_sv = small_sample_vecs(n);
-  U4 key[kSmallPick];
+  const int n_sv = (int)small_sample_vecs(n);
+  unsigned long long* __restrict__ sample = reinterpret_cast<unsigned long long*>(J.sample);
+  {
+    const int per = (n_sv + kSampleGroups - 1) / kSampleGroups, j = (int)blockIdx.x * per + (int)threadIdx.x;
+    if ((int)threadIdx.x < per && j < n_sv) {
+      Src src = srcs.s[blockIdx.y];
+      drop_dir(src, 0);
+      // coarse: a subset of the windows of the fine sample, which it then agrees with
+      const int64_t all = COARSE ? J.n_sv : n_sv;
+      uint32_t key[4];
+      src.template load<false>(quad_of_window(j * all / n_sv, n / 4, all, J.seed) * 4, n, key);
 #pragma unroll
-  for (int u = 0; u < kSmallPick; ++u) {
-    const int64_t j = (int64_t)u * kWide + threadIdx.x;
-    if (u * (int64_t)kWide < n_sv && j < n_sv) key[u] = reinterpret_cast<const U4*>(J.sample)[j];
+      for (int h = 0; h < 2; ++h)
+        __hip_atomic_store(&sample[2 * j + h], (unsigned long long)key[2 * h + 1] << 32 | key[2 * h], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
   const U4 zero{0u, 0u, 0u, 0u};
   reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
+  reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
   if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
+  wait_landed();
+  if (wave_id() == 0) {
+    if (lane_id() == 0) st_agent(&st->sampled[blockIdx.x], launch);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                  // it has landed before the others' are read
+    const bool there = lane_id() >= kSampleGroups || ld_agent(&st->sampled[lane_id() % kSampleGroups]) == launch;
+    const uint32_t all = ballot64(there) == ~0ull;
+    if (lane_id() == 0) s_all = all;
+  }
   __syncthreads();
+  if (!s_all) return;
+  uint32_t key[kSmallPick][4];
+#pragma unroll
+  for (int u = 0; u < kSmallPick; ++u) {
+    const int j = u * kWide + (int)threadIdx.x;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned long long q =
+          j < n_sv ? __hip_atomic_load(&sample[2 * j + h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+      key[u][2 * h] = (uint32_t)q;
+      key[u][2 * h + 1] = (uint32_t)(q >> 32);
+    }
+  }
   const uint32_t ns = (uint32_t)(n_sv * 4);
   double rh, rl;
   if (COARSE) {
@@ -1042,72 +1078,79 @@ __global__ __launch_bounds__(kWide) void k_pick_coarse(ChainJobs jobs, double si
     rl = f.lo;
   }
   const bool open_hi = rh < 1.0 || ns == 0, open_lo = rl > (double)ns || ns == 0;
-  const uint32_t rank[2] = {open_hi ? 1u : (uint32_t)rh, open_lo ? 1u : (uint32_t)rl};
+  const uint32_t rank[2] = {open_hi ? 1u : (uint32_t)rh, open_lo ? ns : (uint32_t)rl};
   uint32_t t_hi = 0x80000000u, t_lo = 0u;
   if (ns) {
     auto each = [&](auto&& f) {
 #pragma unroll
       for (int u = 0; u < kSmallPick; ++u) {
-        if (u * (int64_t)kWide >= n_sv) break;                  // uniform
-        const bool live = (int64_t)u * kWide + threadIdx.x < n_sv;
-        f(key[u].x, live); f(key[u].y, live); f(key[u].z, live); f(key[u].w, live);
+        if (u * kWide >= n_sv) break;                           // uniform
+        const bool live = u * kWide + (int)threadIdx.x < n_sv;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f(key[u][e], live);
       }
     };
-    each([&](uint32_t kk, bool live) { if (live) atomicAdd(&s_h[0][kk >> kL0Shift], 1u); });
+    each([&](uint32_t kk, bool live) { if (live) atomicAdd(&s_h[0][kk >> kPickShift], 1u); });
     __syncthreads();
     RankHit hit[2];
-    wide_find_rank<2>(s_h[0], rank, s_scan, 0, hit);
+    wide_find_rank<2, 2 * kBinsBig>(s_h[0], rank, s_scan, 0, hit);
     uint32_t bin[2] = {hit[0].bin, hit[1].bin};
     uint32_t rk[2] = {rank[0] - hit[0].above, rank[1] - hit[1].above};
     uint32_t cnt[2] = {hit[0].count, hit[1].count};
-    int w = kL0Shift, turn = 1;                        // bits of a key below the bins found so far
-    while (w > 0 && (cnt[0] > (uint32_t)kWideList || cnt[1] > (uint32_t)kWideList)) {
-      const int sh = w > 12 ? w - 12 : 0, bits = w - sh;
-      reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
-      reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
-      __syncthreads();
-      each([&](uint32_t kk, bool live) {
-        const uint32_t top = kk >> w;
-        if (!live || (top != bin[0] && top != bin[1])) return;
-        const uint32_t low = (kk >> sh) & ((1u << bits) - 1u);
-        if (top == bin[0]) atomicAdd(&s_h[0][low], 1u);
-        if (top == bin[1]) atomicAdd(&s_h[1][low], 1u);
-      });
-      __syncthreads();
+    int w = kPickShift, turn = 1;                      // bits of a key below the bins found so far
+    const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]);
+    if (4u * more <= rank[1] - rank[0]) {
+      if (!open_hi) t_hi = (bin[0] + 1u) << w;
+      if (!open_lo) t_lo = bin[1] << w;
+    } else {
+      while (w > 0 && (cnt[0] > (uint32_t)kWideList || cnt[1] > (uint32_t)kWideList)) {
+        const int sh = w > 12 ? w - 12 : 0, bits = w - sh;
+        reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
+        reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
+        __syncthreads();
+        each([&](uint32_t kk, bool live) {
+          const uint32_t top = kk >> w;
+          if (!live || (top != bin[0] && top != bin[1])) return;
+          const uint32_t low = (kk >> sh) & ((1u << bits) - 1u);
+          if (top == bin[0]) atomicAdd(&s_h[0][low], 1u);
+          if (top == bin[1]) atomicAdd(&s_h[1][low], 1u);
+        });
+        __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const uint32_t want[1] = {rk[q]};
-        RankHit h[1];
-        wide_find_rank<1>(s_h[q], want, s_scan, turn, h);
-        turn ^= 1;
-        bin[q] = (bin[q] << bits) | h[0].bin;
-        rk[q] -= h[0].above;
-        cnt[q] = h[0].count;
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t want[1] = {rk[q]};
+          RankHit h[1];
+          wide_find_rank<1>(s_h[q], want, s_scan, turn, h);
+          turn ^= 1;
+          bin[q] = (bin[q] << bits) | h[0].bin;
+          rk[q] -= h[0].above;
+          cnt[q] = h[0].count;
+        }
+        w = sh;
       }
-      w = sh;
-    }
-    if (w > 0) {
-      each([&](uint32_t kk, bool live) {
-        const uint32_t top = kk >> w;
-        if (!live || (top != bin[0] && top != bin[1])) return;
-        if (top == bin[0]) s_list[0][atomicAdd(&s_cnt[0], 1u)] = kk;
-        if (top == bin[1]) s_list[1][atomicAdd(&s_cnt[1], 1u)] = kk;
-      });
-      __syncthreads();
+      if (w > 0) {
+        each([&](uint32_t kk, bool live) {
+          const uint32_t top = kk >> w;
+          if (!live || (top != bin[0] && top != bin[1])) return;
+          if (top == bin[0]) s_list[0][atomicAdd(&s_cnt[0], 1u)] = kk;
+          if (top == bin[1]) s_list[1][atomicAdd(&s_cnt[1], 1u)] = kk;
+        });
+        __syncthreads();
 #pragma unroll
-      for (int q = 0; q < 2; ++q) wide_list_rank(s_list[q], cnt[q], rk[q], s_out[q]);
-      __syncthreads();
+        for (int q = 0; q < 2; ++q) wide_list_rank(s_list[q], cnt[q], rk[q], s_out[q]);
+        __syncthreads();
+      }
+      // keys equal to the upper sample key stay inside the bracket
+      if (!open_hi) t_hi = (w > 0 ? s_out[0][0] : bin[0]) + 1u;
+      if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
     }
-    // keys equal to the upper sample key stay inside the bracket
-    if (!open_hi) t_hi = (w > 0 ? s_out[0][0] : bin[0]) + 1u;
-    if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
   }
   if (threadIdx.x == 0) {
     SelState z = {};
     z.k = J.k;
     z.t_hi = t_hi;
     z.t_lo = t_lo;
-    *J.st = z;
+    *st = z;
   }
 }
 
@@ -2092,27 +2135,27 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 // not form keys: chain_begin, chain_pick_* and chain_settle take the whole batch; chain_sample_*,
 // chain_sweeps and chain_tail are templates of the key source and take the jobs of one kind (a sub-batch
 // over the same workspaces).
-static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, bool fast, hipStream_t s) {
+static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStream_t s) {
   static_assert(sizeof(ChainJobs) + sizeof(SegDirJobs) + 64 <= 4096, "operands travel in the kernel arguments");
-  hipLaunchKernelGGL(k_chain_begin, B.grid(fast ? 32 : 4), dim3(kBlock), 0, s, B.jobs, dirs, fast ? 1 : 0);
+  hipLaunchKernelGGL(k_chain_begin, B.grid(4), dim3(kBlock), 0, s, B.jobs, dirs);
 }
-template <class Src>
-static inline void launch_sample_coarse(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
-                                        bool of_fine, hipStream_t s) {
+// Numbers of the launches that take a sample (never zero, as a cleared state is).
+static inline uint32_t next_launch() {
+  static std::atomic<uint32_t> count{0};
+  return count.fetch_add(2u, std::memory_order_relaxed) | 1u;
+}
+template <bool COARSE, class Src>
+static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
+                                      hipStream_t s) {
   static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + 64 <= 4096,
                 "the operands of a batched chain kernel travel in its 4 KiB of kernel arguments");
-  int64_t n_sv = 0;
-  for (int b = 0; b < B.count; ++b) n_sv = n_sv > small_sample_vecs(B.jobs.j[b].n) ? n_sv : small_sample_vecs(B.jobs.j[b].n);
-  hipLaunchKernelGGL((k_sample_coarse<Src>), B.grid((unsigned)cdiv64(n_sv, kBlock) + 1), dim3(kBlock), 0, s, srcs,
-                     B.jobs, dirs, of_fine ? 1 : 0);
+  hipLaunchKernelGGL((k_sample_pick<Src, COARSE>), B.grid(kSampleGroups + (COARSE ? 16 : 1)), dim3(kWide), 0, s, srcs,
+                     B.jobs, dirs, next_launch(), sigmas);
 }
 template <class Src>
 static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
   hipLaunchKernelGGL((k_sample_fine<Src>), B.grid((unsigned)cdiv64(B.max_nsv, kBlock)), dim3(kBlock), 0, s, srcs,
                      B.jobs);
-}
-static inline void chain_pick_coarse(const SelBatch& B, double sigmas, hipStream_t s) {
-  hipLaunchKernelGGL((k_pick_coarse<true>), B.grid(1), dim3(kWide), 0, s, B.jobs, sigmas);
 }
 static inline void chain_pick_fine(const SelBatch& B, double sigmas, hipStream_t s) {
   hipLaunchKernelGGL(k_pick_fine, B.grid(1), dim3(kWide), 0, s, B.jobs, sigmas);
@@ -2121,9 +2164,7 @@ static inline void chain_pick_fine(const SelBatch& B, double sigmas, hipStream_t
 template <class Src>
 static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
                                  hipStream_t s) {
-  chain_begin(B, dirs, true, s);
-  launch_sample_coarse(srcs, B, SegDirJobs{}, true, s);
-  chain_pick_coarse(B, sigmas, s);
+  launch_sample_pick<true>(srcs, B, dirs, sigmas, s);
   launch_sample_fine(srcs, B, s);
   chain_pick_fine(B, sigmas, s);
 }
@@ -2174,7 +2215,7 @@ static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B,
     chain_sweeps(srcs, B, pm, s, keep);
     chain_settle(B, s);
   } else {
-    chain_begin(B, dirs, false, s);
+    chain_begin(B, dirs, s);
   }
   chain_tail<OUT>(srcs, B, s);
 }

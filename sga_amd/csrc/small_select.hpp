@@ -1,6 +1,6 @@
-// Exact top-k of a bucket of up to kSmallTiles chunks (8.4 M coordinates) in four launches:
-//   k_sample_coarse   8 K to 16 K sample keys (and the directory of the segment table)
-//   k_pick_coarse     one workgroup brackets the k-th key between two sample keys
+// Exact top-k of a bucket of up to kSmallTiles chunks (8.4 M coordinates) in three launches:
+//   k_sample_pick     8 K to 16 K sample keys, and the bracket of the k-th key from them (and the
+//                     directory of the segment table)
 //   k_small_sweep     the one sweep over the data: per-chunk counts above the bracket, and a list
 //                     of the few keys inside it
 //   k_small_finish    one workgroup: exact threshold from the list, ties to grant, and the
@@ -16,7 +16,7 @@
 // Measured through the public entry points, us per call, before -> with this path:
 //   fused step, |g + r|, 1 %, 261 K elements bf16   84 -> 55       4.2 M elements fp32   184 -> 91
 //   select_topk_flat, 3 M scores, 1 %              168 -> 69
-// (4.2 M: sample 2.5, pick 8, sweep 6, finish 19, final sweep 30 us).
+// (4.2 M: sample and pick 8, sweep 6, finish 15, final sweep 28 us).
 //
 // The result is exact for any sample: where the bracket misses the k-th key the finishing launch goes
 // over the data itself, with all of its workgroups (small_redo).
@@ -159,26 +159,40 @@ struct SmallList {
 #pragma unroll
     for (int u = 0; u < kSmallHead; ++u) trim(key[u], (uint32_t)(u * kWave + lane_id()) * kVec, c);
   }
-  // head(key, idx) over the entries in registers, tail(key, idx) over the rest (whole waves)
-  template <class H, class T>
+  // head(key, idx) over the entries in registers, tail(key, idx) over the rest (whole waves).  IDX: the index is
+  // wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a microsecond
+  // a round of loads, so the next round is on its way while one is worked off.
+  template <bool IDX, class H, class T>
   __device__ __forceinline__ void visit(H&& head, T&& tail) const {
 #pragma unroll
     for (int u = 0; u < kSmallHead; ++u) {
       if ((uint32_t)(u * kWave * kVec) >= cnt) return;  // wave-uniform
       head(key[u].x, idx[u].x); head(key[u].y, idx[u].y); head(key[u].z, idx[u].z); head(key[u].w, idx[u].w);
     }
-    for (uint32_t q0 = kSmallHead * kWave; q0 * kVec < cnt; q0 += 2 * kWave) {
-      U4 k2[2], i2[2];
+    constexpr int U = IDX ? 2 : 4;
+    U4 k2[U], i2[U];
+    auto request_from = [&](uint32_t q0) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < U; ++u) {
         const uint32_t q = q0 + u * kWave + lane_id();
-        k2[u] = i2[u] = U4{0u, 0u, 0u, 0u};
-        if (q * kVec < cnt) { k2[u] = keys[q]; i2[u] = idxs[q]; }
+        k2[u] = U4{~0u, ~0u, ~0u, ~0u};
+        if (q * kVec < cnt) { k2[u] = keys[q]; if (IDX) i2[u] = idxs[q]; }
       }
+    };
+    constexpr uint32_t q_first = kSmallHead * kWave;
+    if (q_first * kVec < cnt) request_from(q_first);
+    for (uint32_t q0 = q_first; q0 * kVec < cnt; q0 += U * kWave) {
+      U4 k[U], i[U];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        trim(k2[u], (q0 + u * kWave + lane_id()) * kVec, cnt);
-        tail(k2[u].x, i2[u].x); tail(k2[u].y, i2[u].y); tail(k2[u].z, i2[u].z); tail(k2[u].w, i2[u].w);
+      for (int u = 0; u < U; ++u) {
+        k[u] = k2[u];
+        i[u] = IDX ? i2[u] : U4{0u, 0u, 0u, 0u};
+        trim(k[u], (q0 + u * kWave + lane_id()) * kVec, cnt);
+      }
+      if ((q0 + U * kWave) * kVec < cnt) request_from(q0 + U * kWave);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        tail(k[u].x, i[u].x); tail(k[u].y, i[u].y); tail(k[u].z, i[u].z); tail(k[u].w, i[u].w);
       }
     }
   }
@@ -289,8 +303,8 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = j * kWide + threadIdx.x;
-    g8[j] = t < nt ? J.tile_gt[t] : 0u;
-    e8[j] = t < nt ? J.tile_eq[t] : 0u;
+    g8[j] = e8[j] = 0u;
+    if (j * kWide < nt && t < nt) { g8[j] = J.tile_gt[t]; e8[j] = J.tile_eq[t]; }
   }
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
@@ -318,11 +332,10 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     __syncthreads();
     if (s_cnt == 1u) return;
   }
-  uint32_t n_hi, n_low, n_list = 0;
-  wide_prefix(hi, s_scan, 0, n_hi);
-  wide_prefix(eqs, s_scan, 1, n_low);
+  uint32_t n_hi, n_low, n_list;
+  wide_totals(hi, eqs, s_scan, n_hi, n_low);
+  wide_waves_before(s_seg, n_list);
   list.counted(s_seg[wave_id()]);
-  for (int w = 0; w < kWideWaves; ++w) n_list += s_seg[w];
   // A list far longer than its margin says holds a plateau that one workgroup should not walk (keys equal
   // to the upper end are listed): two values, k near where they change, 8.4 M coordinates: half of them
   // on the upper one 5.7 ms, a tenth 1.06; by passes over the data 0.29 and 0.32.  Independent scores list
@@ -342,7 +355,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     auto above = [&](uint32_t key, uint32_t idx) {
       if (key != ~0u) atomicAdd(&s_tile[idx >> 10], 1u);
     };
-    list.visit(above, above);
+    list.visit<true>(above, above);
     __syncthreads();
   } else if (ok) {
     // the lower end is below the threshold: its members are no ties
@@ -354,15 +367,12 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     int w = 32 - __clz((int)(T_HI - 1u - lo));         // bits of the offset (the list is not empty)
     for (;;) {
       const int sh = w > 12 ? w - 12 : 0;
-      list.visit(
-          [&](uint32_t key, uint32_t) {
-            const uint32_t off = key - lo;
-            if (off >> w == 0u) atomicAdd(&s_hist[off >> sh], 1u);
-          },
-          [&](uint32_t key, uint32_t) {
-            const uint32_t off = key - lo;
-            wide_hist_add(s_hist, off >> sh, off >> w == 0u);
-          });
+      // (plain adds: 64 lanes on one bin cost no more than asking whether they are)
+      auto count = [&](uint32_t key, uint32_t) {
+        const uint32_t off = key - lo;
+        if (off >> w == 0u) atomicAdd(&s_hist[off >> sh], 1u);
+      };
+      list.visit<false>(count, count);
       __syncthreads();
       const uint32_t want[1] = {rank};
       RankHit h[1];
@@ -379,19 +389,25 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     // one pass with the indices: keys above the bin are selected, the bin's own go to the short list
     // (a bin of one key value, of any size, are the ties)
     const bool ties_only = w == 0;
-    auto place = [&](uint32_t key, uint32_t idx) {
-      const uint32_t off = key - lo;
-      if ((int32_t)off < 0) return;
-      const bool in_bin = off >> w == 0u;
-      if (!in_bin || ties_only) {
-        atomicAdd(&s_tile[idx >> 10], in_bin ? 1u << 16 : 1u);
-      } else {
-        const uint32_t at = atomicAdd(&s_cnt, 1u);
-        s_key[at] = key;
-        s_idx[at] = idx;
-      }
-    };
-    list.visit(place, place);
+    const uint32_t width = 1u << w;
+    if (ties_only) {
+      auto place = [&](uint32_t key, uint32_t idx) {
+        const uint32_t off = key - lo;
+        if ((int32_t)off >= 0) atomicAdd(&s_tile[idx >> 10], off < width ? 1u << 16 : 1u);
+      };
+      list.visit<true>(place, place);
+    } else {
+      auto place = [&](uint32_t key, uint32_t idx) {
+        const uint32_t off = key - lo;
+        if (off - width < 0x80000000u - width) atomicAdd(&s_tile[idx >> 10], 1u);
+        if (off < width) {
+          const uint32_t at = atomicAdd(&s_cnt, 1u);
+          s_key[at] = key;
+          s_idx[at] = idx;
+        }
+      };
+      list.visit<true>(place, place);
+    }
     T = lo;
     need = rank;
     __syncthreads();
@@ -422,32 +438,37 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
       s_tile[t] = t < nt ? ld_agent(&J.tile_gt[t]) | (ld_agent(&J.tile_eq[t]) << 16) : 0u;
     __syncthreads();
   }
-  // chunk prefixes: ties granted in index order until `need` is used up (all of them: tie_all)
-  const uint32_t quota = J.tie_all ? 0xFFFFFFFFu : need;
-  uint32_t tv[PER], my_e = 0, total;                  // eight consecutive chunks per thread
+  // chunk prefixes: ties granted in index order until `need` is used up (all of them: tie_all); where all are,
+  // the writing pass need not know how many lie before a chunk
+  const uint32_t quota = J.tie_all || need == n_eq ? 0xFFFFFFFFu : need;
+  uint32_t tv[PER], my_e = 0, er = 0, total;          // eight consecutive chunks per thread
 #pragma unroll
   for (int j = 0; j < PER; j += 4) {
     const U4 q = *reinterpret_cast<const U4*>(s_tile + threadIdx.x * PER + j);
     tv[j] = q.x; tv[j + 1] = q.y; tv[j + 2] = q.z; tv[j + 3] = q.w;
   }
+  if (quota != 0xFFFFFFFFu) {
 #pragma unroll
-  for (int j = 0; j < PER; ++j) my_e += tv[j] >> 16;
-  uint32_t er = wide_prefix(my_e, s_scan, turn, total);
+    for (int j = 0; j < PER; ++j) my_e += tv[j] >> 16;
+    er = wide_prefix(my_e, s_scan, turn, total);
+  }
   uint32_t my_s = 0, eb[PER], sc[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     eb[j] = er;
     sc[j] = (tv[j] & 0xFFFFu) + ties_taken(quota, er, tv[j] >> 16);
     my_s += sc[j];
-    er += tv[j] >> 16;
+    if (quota != 0xFFFFFFFFu) er += tv[j] >> 16;
   }
   uint32_t selected;
   uint32_t sr = wide_prefix(my_s, s_scan, turn ^ 1, selected);
+  if ((int)threadIdx.x * PER < nt) {
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int t = threadIdx.x * PER + j;
-    if (t < nt) { J.tile_gt[t] = sr; J.tile_eq[t] = eb[j]; }
-    sr += sc[j];
+    for (int j = 0; j < PER; ++j) {
+      const int t = threadIdx.x * PER + j;
+      if (t < nt) { J.tile_gt[t] = sr; J.tile_eq[t] = eb[j]; }
+      sr += sc[j];
+    }
   }
   if (threadIdx.x == 0) {
     st->thresh_bits = T;
@@ -470,13 +491,12 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   }
 }
 
-// The three launches for every job of a batch (all of them SelBatch::small_ok).  dirs: segment
+// The launches for every job of a batch (all of them SelBatch::small_ok).  dirs: segment
 // directories to build on the way (the finishing and writing passes read them).
 template <class Src>
 static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
                                     hipStream_t s) {
-  launch_sample_coarse(srcs, B, dirs, false, s);
-  hipLaunchKernelGGL((k_pick_coarse<false>), B.grid(1), dim3(kWide), 0, s, B.jobs, kBracketSigmas);
+  launch_sample_pick<false>(srcs, B, dirs, kBracketSigmas, s);
   const int cpw = Src::kHyper || B.max_tiles <= kSweepTiles ? 1 : 4;
   if (cpw == 1)
     hipLaunchKernelGGL((k_small_sweep<Src, 1>), B.grid((unsigned)B.max_tiles), dim3(kBlock), 0, s, srcs, B.jobs);

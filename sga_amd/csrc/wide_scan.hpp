@@ -18,32 +18,48 @@ struct WideScratch {
   uint32_t hit[2][2][3];
 };
 
+// The sixteen waves' totals as every wave sees them: what lies before the calling wave, and all of it.  By
+// lanes: sixteen reads and adds a wave are 0.4 us where four waves share a SIMD's issue.
+__device__ __forceinline__ uint32_t wide_waves_before(const uint32_t* tot, uint32_t& all) {
+  const uint32_t incl = row_incl_scan(tot[lane_id() % kWideWaves]);
+  all = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWideWaves - 1);
+  const int w = uniform_i32(wave_id());
+  return w ? (uint32_t)__builtin_amdgcn_readlane((int)incl, w - 1) : 0u;
+}
+
 // Exclusive prefix sum over the workgroup, and the total.  One barrier.
 __device__ __forceinline__ uint32_t wide_prefix(uint32_t mine, WideScratch& s, int turn, uint32_t& total) {
   const uint32_t incl = wave_incl_scan(mine);
   if (lane_id() == kWave - 1) s.tot[turn][wave_id()] = incl;
   __syncthreads();
-  uint32_t before = incl - mine, all = 0;
-#pragma unroll
-  for (int w = 0; w < kWideWaves; ++w) {
-    const uint32_t t = s.tot[turn][w];
-    before += w < wave_id() ? t : 0u;
-    all += t;
-  }
-  total = all;
-  return before;
+  return incl - mine + wide_waves_before(s.tot[turn], total);
+}
+
+// The workgroup's totals of two numbers.  One barrier; takes both halves of the scratch.
+__device__ __forceinline__ void wide_totals(uint32_t a, uint32_t b, WideScratch& s, uint32_t& all_a, uint32_t& all_b) {
+  a = wave_incl_scan(a);
+  b = wave_incl_scan(b);
+  if (lane_id() == kWave - 1) { s.tot[0][wave_id()] = a; s.tot[1][wave_id()] = b; }
+  __syncthreads();
+  wide_waves_before(s.tot[0], all_a);
+  wide_waves_before(s.tot[1], all_b);
 }
 
 struct RankHit { uint32_t bin, above, count; };
-// The bins of a 4096-bin LDS histogram where the count from the top reaches each of NR ranks
+// The bins of an LDS histogram where the count from the top reaches each of NR ranks
 // (1-based).  All threads get the answers.  Two barriers, after the one that completes the histogram.
-template <int NR>
+template <int NR, int BINS = kWideBins>
 __device__ __forceinline__ void wide_find_rank(const uint32_t* s_hist, const uint32_t (&rank)[NR],
                                                WideScratch& s, int turn, RankHit (&hit)[NR]) {
-  constexpr int PER = kWideBins / kWide;           // 4
-  const U4 q = reinterpret_cast<const U4*>(s_hist)[threadIdx.x];
-  const uint32_t h[PER] = {q.x, q.y, q.z, q.w};
-  const uint32_t mine = h[0] + h[1] + h[2] + h[3];
+  constexpr int PER = BINS / kWide;                // 4 or 8
+  static_assert(PER % 4 == 0, "whole quads of bins per thread");
+  uint32_t h[PER], mine = 0;
+#pragma unroll
+  for (int j = 0; j < PER; j += 4) {
+    const U4 q = reinterpret_cast<const U4*>(s_hist)[threadIdx.x * (PER / 4) + j / 4];
+    h[j] = q.x; h[j + 1] = q.y; h[j + 2] = q.z; h[j + 3] = q.w;
+    mine += (q.x + q.y) + (q.z + q.w);
+  }
   uint32_t total;
   const uint32_t before = wide_prefix(mine, s, turn, total);
 #pragma unroll
