@@ -186,6 +186,10 @@ int sga_expand_blocks(const uint8_t* bmask, int x, int64_t n, uint8_t* out,
 int64_t sga_mask_chunks(int64_t n);
 int sga_mask_count(const uint8_t* mask, int64_t n, uint32_t* chunk_counts,
                    int64_t* total, void* stream);
+/* The same, and the set bytes before j * step in totals[j], j = 1 .. cuts
+ * (totals: cuts + 1 device int64). */
+int sga_mask_count_cuts(const uint8_t* mask, int64_t n, uint32_t* chunk_counts,
+                        int64_t step, int cuts, int64_t* totals, void* stream);
 /* Phase 2: idx_out[..k) = ascending positions of the non-zero bytes. */
 int sga_mask_fill(const uint8_t* mask, int64_t n, const uint32_t* chunk_offsets,
                   int32_t* idx_out, int64_t idx_capacity, void* stream);

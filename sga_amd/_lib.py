@@ -64,6 +64,7 @@ SIGNATURES = {
     "sga_expand_blocks": (I32, [P, I32, I64, P, P]),
     "sga_mask_chunks": (I64, [I64]),
     "sga_mask_count": (I32, [P, I64, P, P, P]),
+    "sga_mask_count_cuts": (I32, [P, I64, P, I64, I32, P, P]),
     "sga_mask_fill": (I32, [P, I64, P, P, I64, P]),
     "sga_adamw_grad_correct": (I32, [P, P, P, P, P, I64] + [F] * 12 + [I32, I32, P]),
     "sga_adamw_grad_correct_multi": (I32, [P, I32, I64, F, F, I32, P]),

@@ -16,7 +16,7 @@ def index_layout_bounds(idx, n, slices=2):
     splits the selected set evenly (``torch_pipelined_index.py:314-325``)."""
     k = idx.numel()
     if slices == 2:
-        mid = torch.tensor([n // 2], dtype=idx.dtype, device=idx.device)
+        mid = torch.full((1,), n // 2, dtype=idx.dtype, device=idx.device)   # an upload would wait for the stream
         n0 = int(torch.searchsorted(idx, mid).item())
         return [(0, n0), (n0, k)]
     return [(i * k // slices, (i + 1) * k // slices) for i in range(slices)]
@@ -46,11 +46,15 @@ def mask_layout_pack(grad, mask_u8, factor=1.0, slices=2):
     read of ``grad``.  Returns (payload list, idx) -- idx is kept so unpack
     does not recompute the compaction."""
     n = grad.numel()
-    idx = compact_mask_u8(mask_u8)
-    base = n // slices if slices > 1 else n
-    cuts = [i * base for i in range(slices)] + [n]
-    pos = torch.searchsorted(idx, torch.tensor(cuts, dtype=torch.int32, device=idx.device))
-    pos = pos.tolist()
+    if slices > 1 and mask_u8.numel() == n:
+        # the slices' ends come with the count: no search of its own and one wait for the device
+        idx, ends = compact_mask_u8(mask_u8, step=n // slices, cuts=slices - 1)
+        pos = [0] + ends + [idx.numel()]
+    else:
+        idx = compact_mask_u8(mask_u8)
+        base = n // slices if slices > 1 else n
+        cuts = [i * base for i in range(slices)] + [n]
+        pos = torch.searchsorted(idx, torch.tensor(cuts, dtype=torch.int32, device=idx.device)).tolist()
     payloads = []
     for lo, hi in zip(pos[:-1], pos[1:]):
         sel = torch.empty(hi - lo, dtype=torch.float32, device=grad.device)

@@ -295,59 +295,94 @@ __global__ __launch_bounds__(kBlock) void k_expand_blocks(const uint8_t* __restr
 }
 
 // ------------------------------------------------------- mask compaction
-// Chunk = 1024 consecutive bytes owned by one wave (4 x 4 bytes per lane).
-// Phase 1 counts the non-zero bytes of each chunk; a two-level exclusive scan
-// turns counts into offsets; phase 2 rewrites positions in ascending order
-// using wave ballots -- the output equals nonzero() for any launch geometry.
-__global__ __launch_bounds__(kBlock) void k_mask_count(
-    const uint8_t* __restrict__ mask, int64_t n, uint32_t* __restrict__ counts,
-    int64_t n_chunks, bool vec) {
-  const int64_t wave0 = (int64_t)blockIdx.x * kChunksPerBlock + wave_id();
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  for (int64_t c = wave0; c < n_chunks; c += wstride) {
-    const int64_t base = c * kChunk;
-    uint32_t cnt = 0;
+// Chunk = 1024 consecutive bytes owned by one wave, 16 bytes per lane in one load; four chunks per wave, whose
+// loads are in flight together.  Phase 1 counts the non-zero bytes of each chunk; a two-level exclusive scan
+// turns counts into offsets; phase 2 rewrites positions in ascending order from the lanes' prefix -- the output
+// equals nonzero() for any launch geometry.  With four
+// bytes per lane and load, 63 M bytes: count 20.0 -> 10.7 us, fill 24.1 -> 14.2 (5.9 and 4.6 TB/s of the mask and list).
+constexpr int kMaskChunks = 4;                  // per wave
+// Bit j: byte j of the lane's 16 bytes at i is not zero (past n: zero).
+__device__ __forceinline__ uint32_t nonzero_bits(const U4& w) {
+  const uint32_t x[4] = {w.x, w.y, w.z, w.w};
+  uint32_t bits = 0;
 #pragma unroll
-    for (int it = 0; it < kChunkIters; ++it) {
-      uint32_t mk[4];
-      load4_u8(mask, base + it * (kWave * kVec) + lane_id() * kVec, n, mk, vec);
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t nz = (((x[j] & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x[j]) & 0x80808080u;     // top bit of every such byte
+    bits |= ((nz >> 7) * 0x10204080u >> 28) << (4 * j);                                 // ... side by side
+  }
+  return bits;
+}
+// The lane's bits of the wave's chunks c0 .. c0 + kMaskChunks - 1.
+__device__ __forceinline__ void mask_bits(const uint8_t* __restrict__ mask, int64_t n, int64_t c0,
+                                          uint32_t (&bits)[kMaskChunks]) {
+  typedef uint32_t u4v __attribute__((ext_vector_type(4), aligned(1)));      // a view may begin at any byte
+  U4 w[kMaskChunks];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) cnt += (mk[e] != 0);
+  for (int u = 0; u < kMaskChunks; ++u) {
+    const int64_t i = (c0 + u) * kChunk + lane_id() * 16;
+    w[u] = U4{0u, 0u, 0u, 0u};
+    if (i + 16 <= n) {
+      const u4v t = *reinterpret_cast<const u4v*>(mask + i);
+      w[u] = U4{t.x, t.y, t.z, t.w};
+    } else if (i < n) {
+      uint32_t x[4] = {0u, 0u, 0u, 0u};
+      for (int e = 0; e < 16 && i + e < n; ++e) {
+        const uint32_t by = (uint32_t)mask[i + e] << (8 * (e & 3));
+        if (e < 4) x[0] |= by; else if (e < 8) x[1] |= by; else if (e < 12) x[2] |= by; else x[3] |= by;
+      }
+      w[u] = U4{x[0], x[1], x[2], x[3]};
     }
-    cnt = wave_sum(cnt);
-    if (lane_id() == 0) counts[c] = cnt;
+  }
+#pragma unroll
+  for (int u = 0; u < kMaskChunks; ++u) bits[u] = nonzero_bits(w[u]);
+}
+
+__global__ __launch_bounds__(kBlock) void k_mask_count(const uint8_t* __restrict__ mask, int64_t n,
+                                                       uint32_t* __restrict__ counts, int64_t n_chunks) {
+  const int64_t c0 = ((int64_t)blockIdx.x * kChunksPerBlock + wave_id()) * kMaskChunks;
+  if (c0 >= n_chunks) return;
+  uint32_t bits[kMaskChunks];
+  mask_bits(mask, n, c0, bits);
+#pragma unroll
+  for (int u = 0; u < kMaskChunks; ++u) {
+    const uint32_t cnt = wave_incl_scan((uint32_t)__popc(bits[u]));
+    if (lane_id() == kWave - 1 && c0 + u < n_chunks) counts[c0 + u] = cnt;
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_mask_fill(
-    const uint8_t* __restrict__ mask, int64_t n,
-    const uint32_t* __restrict__ offsets, int32_t* __restrict__ idx_out,
-    int64_t cap, int64_t n_chunks, bool vec) {
-  const int64_t wave0 = (int64_t)blockIdx.x * kChunksPerBlock + wave_id();
-  const int64_t wstride = (int64_t)gridDim.x * kChunksPerBlock;
-  for (int64_t c = wave0; c < n_chunks; c += wstride) {
-    const int64_t base = c * kChunk;
-    uint32_t run = offsets[c];
+__global__ __launch_bounds__(kBlock) void k_mask_fill(const uint8_t* __restrict__ mask, int64_t n,
+                                                      const uint32_t* __restrict__ offsets, int32_t* __restrict__ idx_out,
+                                                      int64_t cap, int64_t n_chunks) {
+  const int64_t c0 = ((int64_t)blockIdx.x * kChunksPerBlock + wave_id()) * kMaskChunks;
+  if (c0 >= n_chunks) return;
+  uint32_t bits[kMaskChunks];
+  mask_bits(mask, n, c0, bits);
 #pragma unroll
-    for (int it = 0; it < kChunkIters; ++it) {
-      const int64_t i0 = base + it * (kWave * kVec) + lane_id() * kVec;
-      uint32_t mk[4];
-      load4_u8(mask, i0, n, mk, vec);
-      uint32_t mine = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) mine += (mk[e] != 0);
-      const uint32_t incl = wave_incl_scan(mine);
-      uint32_t pos = run + incl - mine;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        if (mk[e] != 0) {
-          if ((int64_t)pos < cap) idx_out[pos] = (int32_t)(i0 + e);
-          ++pos;
-        }
-      }
-      run += __shfl(incl, kWave - 1, kWave);
-    }
+  for (int u = 0; u < kMaskChunks; ++u) {
+    if (c0 + u >= n_chunks) return;
+    const uint32_t mine = (uint32_t)__popc(bits[u]);
+    int64_t pos = (int64_t)(offsets[c0 + u] + wave_incl_scan(mine) - mine);
+    const int32_t i0 = (int32_t)((c0 + u) * kChunk + lane_id() * 16);
+    for (uint32_t left = bits[u]; left; left &= left - 1u, ++pos)
+      if (pos < cap) idx_out[pos] = i0 + __ffs((int)left) - 1;
   }
+}
+
+// out[0] = all set bytes, out[j] = those before j * step (j = 1 .. cuts): a wave per cut, from the offsets.
+__global__ __launch_bounds__(kBlock) void k_mask_cuts(const uint8_t* __restrict__ mask, int64_t n,
+                                                      const uint32_t* __restrict__ offsets, int64_t step, int cuts,
+                                                      int64_t* __restrict__ out) {
+  const int j = (int)blockIdx.x * kChunksPerBlock + wave_id() + 1;
+  if (j > cuts) return;
+  const int64_t at = (int64_t)j * step, c = at / kChunk;
+  if (at >= n) {
+    if (lane_id() == 0) out[j] = out[0];
+    return;
+  }
+  uint32_t cnt = 0;
+  for (int64_t i = c * kChunk + lane_id(); i < at; i += kWave) cnt += mask[i] != 0;
+  cnt = wave_sum(cnt);
+  if (lane_id() == 0) out[j] = (int64_t)offsets[c] + cnt;
 }
 
 }  // namespace sga
@@ -654,22 +689,33 @@ extern "C" int64_t sga_mask_chunks(int64_t n) {
 }
 static inline int64_t n_chunks_of(int64_t n) { return cdiv64(n, kChunk); }
 
-extern "C" int sga_mask_count(const uint8_t* mask, int64_t n,
-                              uint32_t* chunk_counts, int64_t* total,
-                              void* stream) {
-  if (!total || n < 0 || n >= (1ll << 31) || (n > 0 && (!mask || !chunk_counts))) {
-    set_error("sga_mask_count: bad argument (n=%lld, int32 indices need n < 2^31)", (long long)n);
+// total[0], and with cuts > 0 total[j] = set bytes before j * step
+static int mask_count(const char* who, const uint8_t* mask, int64_t n, uint32_t* chunk_counts, int64_t* total,
+                      int64_t step, int cuts, void* stream) {
+  if (!total || n < 0 || n >= (1ll << 31) || (n > 0 && (!mask || !chunk_counts)) || step < 0 || cuts < 0) {
+    set_error("%s: bad argument (n=%lld, int32 indices need n < 2^31)", who, (long long)n);
     return SGA_ERR_ARG;
   }
   hipStream_t st = (hipStream_t)stream;
   const int64_t nc = n_chunks_of(n);
   if (nc > 0)
-    hipLaunchKernelGGL(k_mask_count, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)),
-                       dim3(kBlock), 0, st, mask, n, chunk_counts, nc,
-                       quads_ok(mask, 1));
+    hipLaunchKernelGGL(k_mask_count, dim3((unsigned)cdiv64(nc, kChunksPerBlock * kMaskChunks)), dim3(kBlock), 0, st, mask,
+                       n, chunk_counts, nc);
   int rc = exclusive_scan_u32(chunk_counts, nc, total, st);
   if (rc) return rc;
-  return check_launch("sga_mask_count");
+  if (cuts > 0)
+    hipLaunchKernelGGL(k_mask_cuts, dim3((unsigned)cdiv64(cuts, kChunksPerBlock)), dim3(kBlock), 0, st, mask, n,
+                       chunk_counts, step, cuts, total);
+  return check_launch(who);
+}
+
+extern "C" int sga_mask_count(const uint8_t* mask, int64_t n, uint32_t* chunk_counts, int64_t* total, void* stream) {
+  return mask_count("sga_mask_count", mask, n, chunk_counts, total, 0, 0, stream);
+}
+
+extern "C" int sga_mask_count_cuts(const uint8_t* mask, int64_t n, uint32_t* chunk_counts, int64_t step, int cuts,
+                                   int64_t* totals, void* stream) {
+  return mask_count("sga_mask_count_cuts", mask, n, chunk_counts, totals, step, cuts, stream);
 }
 
 extern "C" int sga_mask_fill(const uint8_t* mask, int64_t n,
@@ -682,9 +728,7 @@ extern "C" int sga_mask_fill(const uint8_t* mask, int64_t n,
     return SGA_ERR_ARG;
   }
   const int64_t nc = n_chunks_of(n);
-  hipLaunchKernelGGL(k_mask_fill, dim3(stream_grid(nc, kChunksPerBlock, 1 << 22)),
-                     dim3(kBlock), 0, (hipStream_t)stream, mask, n,
-                     chunk_offsets, idx_out, idx_capacity, nc,
-                     quads_ok(mask, 1));
+  hipLaunchKernelGGL(k_mask_fill, dim3((unsigned)cdiv64(nc, kChunksPerBlock * kMaskChunks)), dim3(kBlock), 0,
+                     (hipStream_t)stream, mask, n, chunk_offsets, idx_out, idx_capacity, nc);
   return check_launch("sga_mask_fill");
 }

@@ -71,7 +71,8 @@ int exclusive_scan_u32(uint32_t* data, int64_t n, int64_t* total,
   }
   const unsigned nb = (unsigned)cdiv64(n, kScanSpan);
   uint32_t* sums = data + n;
-  hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(kBlock), 0, st, data, n, sums);
+  // one workgroup has nothing before it (counts of up to 4.2 M bytes: a launch of 5 us less)
+  if (nb > 1) hipLaunchKernelGGL(k_scan_sums, dim3(nb), dim3(kBlock), 0, st, data, n, sums);
   hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(kBlock), 0, st, data, n, sums, total);
   return SGA_OK;
 }

@@ -23,10 +23,12 @@ class IndexPool:
         return self.buf
 
 
-def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None):
+def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None, step=0, cuts=0):
     """Ascending int32 positions of the non-zero bytes of ``mask_u8``
     (``sga/support.py:57-99``): one counting sweep, one host read of k (the
-    reference syncs on the count too), one ordered fill sweep."""
+    reference syncs on the count too), one ordered fill sweep.  With ``cuts`` the
+    same read also brings how many positions lie before ``step``, ``2 * step``, ...:
+    returns ``(idx, [that many ints])``."""
     n = mask_u8.numel()
     assert n < 2 ** 31, f"int32 support indices assume < 2^31 elements, got {n}"
     L.require_dev(mask_u8)
@@ -38,17 +40,21 @@ def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None):
         raise TypeError("compact_mask_u8: uint8/bool mask")
     dev = mk.device
     if n == 0:
-        return torch.empty(0, dtype=torch.int32, device=dev)
+        idx = torch.empty(0, dtype=torch.int32, device=dev)
+        return (idx, [0] * cuts) if cuts else idx
     counts = torch.empty(int(L.raw("sga_mask_chunks", n)), dtype=torch.int32, device=dev)
-    total = torch.empty(1, dtype=torch.int64, device=dev)
-    L.call("sga_mask_count", L.ptr(mk), n, L.ptr(counts), L.ptr(total), L.stream())
-    k = int(total.item())
+    total = torch.empty(1 + cuts, dtype=torch.int64, device=dev)
+    if cuts:
+        L.call("sga_mask_count_cuts", L.ptr(mk), n, L.ptr(counts), step, cuts, L.ptr(total), L.stream())
+    else:
+        L.call("sga_mask_count", L.ptr(mk), n, L.ptr(counts), L.ptr(total), L.stream())
+    k, *before = total.tolist()
     buf = pool.get(k, dev) if pool is not None else torch.empty(
         k, dtype=torch.int32, device=dev)
     if k:
         L.call("sga_mask_fill", L.ptr(mk), n, L.ptr(counts), L.ptr(buf), buf.numel(),
                L.stream())
-    return buf[:k]
+    return (buf[:k], before) if cuts else buf[:k]
 
 
 def block_idx_from_mask(mask_u8, spans, x):

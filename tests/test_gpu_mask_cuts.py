@@ -1,0 +1,40 @@
+"""Mask compaction by 16-byte loads and the slice ends that come with its count, at the edges of
+a lane's bytes, a chunk, a workgroup's chunks and the scan's one workgroup, against torch on the CPU."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 1023, 1025, 16_385, 100_003, 4096 * 1024, 4096 * 1024 + 1])
+@pytest.mark.parametrize("at", [0, 3])
+def test_positions_and_slice_ends(dev, n, at):
+    from sga_amd.support import compact_mask_u8
+    gen = torch.Generator().manual_seed(n)
+    buf = torch.zeros(n + at, dtype=torch.uint8)
+    buf[at:] = torch.where(torch.rand(n, generator=gen) < 0.05, torch.randint(1, 256, (n,), generator=gen), 0)
+    buf[-1] = 255
+    on = buf[at:].nonzero().view(-1).to(torch.int32)
+    for cuts in (0, 1, 2, 6):
+        step = n // (cuts + 1)
+        out = compact_mask_u8(buf.to(dev)[at:], step=step, cuts=cuts)
+        idx, before = out if cuts else (out, [])
+        assert torch.equal(idx.cpu(), on)
+        assert before == [int((on < (j + 1) * step).sum()) for j in range(cuts)]
+
+
+@pytest.mark.parametrize("n", [3, 50_001])
+@pytest.mark.parametrize("slices", [1, 2, 5])
+def test_mask_layout_slices(dev, n, slices):
+    from sga_amd.backends import mask_layout_pack
+    gen = torch.Generator().manual_seed(n)
+    mask = (torch.rand(n, generator=gen) < 0.1).to(torch.uint8)
+    mask[n // 2] = 1
+    grad = torch.randn(n, generator=gen)
+    payloads, idx = mask_layout_pack(grad.to(dev), mask.to(dev), factor=0.5, slices=slices)
+    base = n // slices if slices > 1 else n
+    ends = [i * base for i in range(slices)] + [n]
+    assert torch.equal(idx.cpu(), mask.nonzero().view(-1).to(torch.int32))
+    assert len(payloads) == slices
+    for p, a, b in zip(payloads, ends[:-1], ends[1:]):
+        assert torch.equal(p.cpu(), grad[a:b][mask[a:b].bool()] * 0.5)
