@@ -10,6 +10,7 @@ the clip coefficient is run-to-run reproducible.
 import torch
 
 from . import _lib as L
+from .adamw import ParamRecord
 from .kernels import compact_norm_sq_contribution, masked_norm_sq_contribution
 
 
@@ -75,9 +76,13 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
     total = torch.zeros(1, dtype=torch.float32, device=live[0].grad.device)
     seen = set()
     for rec in live:
-        mask = None if was_full else rec.mask_u8()
         if compact is not None:
-            if mask is None:
+            if type(rec) is ParamRecord:         # without the slice of the mask: 1 us a record
+                bs = rec.bucket_state
+                no_mask = bs is None or bs.active_mask_u8 is None
+            else:
+                no_mask = rec.mask_u8() is None
+            if no_mask:
                 raise RuntimeError("compact clip: record without an active mask")
             key = id(rec.bucket_state)
             if key not in compact:
@@ -87,6 +92,7 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
                 if compact[key].numel():
                     compact_norm_sq_contribution(compact[key], total)
             continue
+        mask = None if was_full else rec.mask_u8()
         g = rec.grad.data.reshape(-1)
         if mask is None:
             compact_norm_sq_contribution(g, total)
