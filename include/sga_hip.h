@@ -572,6 +572,15 @@ int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coef_dense,
                      double* partials, double* qn2, double* coef_d,
                      float* coef_f, void* stream);
 
+/* sga_segments_refresh followed by sga_replay_pass1, with the tables written by
+ * pass 1 itself where the rows hold few distinct values (no launch of its own). */
+int sga_replay_begin(const void* g, int g_dtype, int64_t n, float coef_dense,
+                     double clip, const sga_replay_cfg* cfgs, int G,
+                     double* partials, double* qn2, double* coef_d,
+                     float* coef_f, sga_segment* segs,
+                     sga_replay_segment* rsegs, int n_segs, const double* lr,
+                     const float* bc1, const float* bc2, void* stream);
+
 /* pass 2 (replay_fused.py:1752-1825) for ONE boundary configuration:
  * score = |formula(w,m,v,(g/coef_dense + res)*coef)|, exact top-k with
  * lowest-index ties, written as a byte mask into sel_out.  The score is
@@ -657,6 +666,15 @@ int sga_dense_replay_step(const void* g, int g_dtype, float* w, float* m, float*
                           float* lab, int64_t n, const sga_replay_segment* segs,
                           int n_segs, int adams, double coef_dense, double* partials,
                           double* recon2, void* stream);
+
+/* sga_segments_refresh on segs followed by sga_dense_replay_step, likewise
+ * without a launch of its own; recon2 may be pinned host memory. */
+int sga_dense_replay_step_at(const void* g, int g_dtype, float* w, float* m,
+                             float* v, float* lab, int64_t n,
+                             sga_replay_segment* segs, int n_segs,
+                             const double* lr, const float* bc1,
+                             const float* bc2, int adams, double coef_dense,
+                             double* partials, double* recon2, void* stream);
 
 /* Bit-plane masks (layout above). */
 int64_t sga_plane_words(int64_t n);

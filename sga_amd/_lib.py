@@ -95,6 +95,7 @@ SIGNATURES = {
     "sga_segments_refresh": (I32, [P, P, I32, P, P, P, P]),
     "sga_replay_partials": (I64, []),
     "sga_replay_pass1": (I32, [P, I32, I64, F, C.c_double, P, I32, P, P, P, P, P]),
+    "sga_replay_begin": (I32, [P, I32, I64, F, C.c_double, P, I32, P, P, P, P, P, P, I32, P, P, P, P]),
     "sga_replay_reselect": (I32, [P, I32, P, P, P, P, I64, I64, P, I32, I32, P, F, I32, I32, I32,
                                   P, P, P, SZ, P]),
     "sga_replay_reselect_multi": (I32, [P, I32, I64, P, I32, F, I32, P, I32, P]),
@@ -104,6 +105,7 @@ SIGNATURES = {
     "sga_replay_pass3": (I32, [P, I32, I64, F, P, I32, P, P, I32, P]),
     "sga_branch_score_f64": (I32, [I32, P, P, P, P, P, I64] + [C.c_double] * 6 + [I32, I32, P]),
     "sga_dense_replay_step": (I32, [P, I32, P, P, P, P, I64, P, I32, I32, C.c_double, P, P, P]),
+    "sga_dense_replay_step_at": (I32, [P, I32, P, P, P, P, I64, P, I32, P, P, P, I32, C.c_double, P, P, P]),
     "sga_plane_words": (I64, [I64]),
     "sga_mask_to_planes": (I32, [P, I64, P, P]),
     "sga_planes_to_mask": (I32, [P, I64, P, P]),

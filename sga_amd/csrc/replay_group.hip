@@ -16,6 +16,8 @@
 #include "adam_math.hpp"
 #include "small_select.hpp"
 
+#include <cstring>
+
 namespace sga {
 
 constexpr int kMaxCfg = 16;
@@ -53,6 +55,52 @@ __device__ __forceinline__ void load_gd(const void* g, int64_t i, int64_t n, flo
   }
 }
 
+// The changing columns of a segment table (learning rates, bias corrections) on their way into a step's first
+// kernel, which writes them into the device tables as a side job: a launch of its own for that was 4.7 us of a
+// step, and nothing in the kernel reads the tables.  Tensors share their values (parameter groups), so a row
+// holds the number of one of up to 16 triples: 0.7 KB of kernel arguments instead of 16 bytes a row.  More
+// tensors or triples than fit take sga_segments_refresh.  Sixteen steps of 1.5 M coordinates, dense pass and two
+// configs, before -> after: 2014 -> 1992 us, 2030 -> 1978 on a new state (with the sum of the dense step written to
+// host memory by its fold, instead of copied there).
+constexpr int kNowRows = 384, kNowSets = 16;
+struct SegNow {
+  sga_segment* segs;
+  sga_replay_segment* rsegs;
+  int count;                     // 0: nothing to write
+  double lr[kNowSets];
+  float bc1[kNowSets], bc2[kNowSets];
+  uint8_t of[kNowRows];
+};
+static bool seg_now_fill(SegNow* t, sga_segment* segs, sga_replay_segment* rsegs, int n, const double* lr,
+                         const float* bc1, const float* bc2) {
+  t->segs = segs; t->rsegs = rsegs; t->count = 0;
+  if (n > kNowRows) return false;
+  int sets = 0, j = 0;
+  // compared as bits: a NaN is a value like any other
+  const auto same = [&](int s, int i) {
+    return !memcmp(&t->lr[s], lr + i, 8) && !memcmp(&t->bc1[s], bc1 + i, 4) && !memcmp(&t->bc2[s], bc2 + i, 4);
+  };
+  for (int i = 0; i < n; ++i) {
+    if (i == 0 || !same(j, i))
+      for (j = 0; j < sets && !same(j, i);) ++j;
+    if (j == sets) {
+      if (sets == kNowSets) return false;
+      t->lr[j] = lr[i]; t->bc1[j] = bc1[i]; t->bc2[j] = bc2[i];
+      ++sets;
+    }
+    t->of[i] = (uint8_t)j;
+  }
+  t->count = n;
+  return true;
+}
+__device__ __forceinline__ void seg_now_write(const SegNow& t) {
+  for (int i = threadIdx.x; i < t.count; i += blockDim.x) {
+    const int j = t.of[i];
+    if (t.segs) { t.segs[i].lr = (float)t.lr[j]; t.segs[i].bc1 = t.bc1[j]; t.segs[i].bc2 = t.bc2[j]; }
+    if (t.rsegs) { t.rsegs[i].lr = t.lr[j]; t.rsegs[i].bc1 = t.bc1[j]; t.rsegs[i].bc2 = t.bc2[j]; }
+  }
+}
+
 // ------------------------------------------------------------------ pass 1
 // One launch per step: the gradient is read once for all configurations.
 // The configs at a cycle boundary with a live residual (q = gd + res) load
@@ -80,7 +128,8 @@ template <bool BF16G, int NB>
 __global__ __launch_bounds__(kBlock) void k_replay_pass1(const void* __restrict__ g, int64_t n,
                                                          float coef_dense, P1List lst,
                                                          double* __restrict__ partials, bool vec,
-                                                         int64_t pack_extra) {
+                                                         int64_t pack_extra, SegNow now) {
+  if (blockIdx.x == gridDim.x - 1) seg_now_write(now);     // the workgroup with the least to do
   constexpr int NBA = NB > 0 ? NB : 1;
   __shared__ double s_w[kChunksPerBlock][2 * kMaxCfg];
   double accb[NBA], accm[kMaxCfg];
@@ -229,11 +278,14 @@ struct RSeg {          // sga_replay_segment, see the header
 
 struct RSegCursor {
   const RSeg* segs;
+  const SegNow* now;             // with rows: learning rates and bias corrections come from here
   int n_segs;
   int64_t lo, hi;
   RSeg s;
   float omlwd, neglr, lrf;
-  __device__ __forceinline__ void init(const RSeg* p, int ns) { segs = p; n_segs = ns; lo = 1; hi = 0; }
+  __device__ __forceinline__ void init(const RSeg* p, int ns, const SegNow* nw = nullptr) {
+    segs = p; now = nw; n_segs = ns; lo = 1; hi = 0;
+  }
   __device__ __forceinline__ void seek(int64_t i) {
     if (i >= lo && i < hi) return;
     int a = 0, b = n_segs - 1;
@@ -242,6 +294,10 @@ struct RSegCursor {
       if (segs[mid].start <= i) a = mid; else b = mid - 1;
     }
     s = segs[a];
+    if (now && now->count) {
+      const int j = now->of[a];
+      s.lr = now->lr[j]; s.bc1 = now->bc1[j]; s.bc2 = now->bc2[j];
+    }
     lo = s.start;
     hi = lo + s.n;
     omlwd = (float)(1.0 - s.lr * s.wd);
@@ -379,10 +435,10 @@ __global__ __launch_bounds__(kBlock) void k_dense_step(const void* __restrict__ 
                                                        float* w, float* m, float* v, float* lab,
                                                        int adams,
                                                        const RSeg* __restrict__ segs, int n_segs,
-                                                       double* __restrict__ partials, bool vec) {
+                                                       double* __restrict__ partials, bool vec, SegNow now) {
   __shared__ double s_w[kChunksPerBlock];
   RSegCursor sc;
-  sc.init(segs, n_segs);
+  sc.init(segs, n_segs, &now);
   double acc = 0.0;
   const int64_t stride = (int64_t)gridDim.x * kBlock * kVec;
   for (int64_t base = (int64_t)blockIdx.x * kBlock * kVec; base < n; base += stride) {
@@ -562,7 +618,8 @@ __global__ __launch_bounds__(kBlock) void k_sqdist_stage1(const float* __restric
 constexpr int kFoldThreads = 1024;
 __global__ __launch_bounds__(kFoldThreads) void k_fold_partials(const double* __restrict__ partials,
                                                                 int nb, double divisor,
-                                                                double* __restrict__ out) {
+                                                                double* __restrict__ out, SegNow now) {
+  seg_now_write(now);            // the table for whoever reads it next: the step had the values by argument
   __shared__ double s_p[kFoldThreads];
   double a = 0.0;
   for (int b = threadIdx.x; b < nb; b += kFoldThreads) a += partials[b];
@@ -623,11 +680,11 @@ static_assert(sizeof(RSeg) == sizeof(sga_replay_segment), "replay segment layout
 template <bool BF16G>
 static void launch_pass1(int n_b, unsigned nb, hipStream_t s, const void* g, int64_t n,
                          float coef_dense, const P1List& lst, double* partials, bool vec,
-                         int64_t pack_extra) {
+                         int64_t pack_extra, const SegNow& now) {
 #define SGA_P1(NB)                                                                              \
   case NB:                                                                                      \
     hipLaunchKernelGGL((k_replay_pass1<BF16G, NB>), dim3(nb), dim3(kBlock), 0, s, g, n,         \
-                       coef_dense, lst, partials, vec, pack_extra);                             \
+                       coef_dense, lst, partials, vec, pack_extra, now);                        \
     break;
   switch (n_b) {
     SGA_P1(0) SGA_P1(1) SGA_P1(2) SGA_P1(3) SGA_P1(4) SGA_P1(5) SGA_P1(6) SGA_P1(7) SGA_P1(8)
@@ -679,9 +736,9 @@ extern "C" int sga_segments_refresh(sga_segment* segs, sga_replay_segment* rsegs
 
 extern "C" int64_t sga_replay_partials(void) { return (int64_t)kReplayBlocks * kMaxCfg; }
 
-extern "C" int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coef_dense, double clip,
-                                const sga_replay_cfg* cfgs, int G, double* partials, double* qn2,
-                                double* coef_d, float* coef_f, void* stream) {
+static int replay_pass1(const void* g, int g_dtype, int64_t n, float coef_dense, double clip,
+                        const sga_replay_cfg* cfgs, int G, double* partials, double* qn2, double* coef_d,
+                        float* coef_f, const SegNow& now, void* stream) {
   RGroup grp;
   if (!g || n < 1 || !partials || !qn2 || !coef_d || !coef_f || !fill_group(&grp, cfgs, G) ||
       (g_dtype != SGA_F32 && g_dtype != SGA_BF16)) {
@@ -710,11 +767,36 @@ extern "C" int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coe
   lst.n_sel = n_m;
   for (int c = G; c < kMaxCfg; ++c) al.src[c] = 0;
   ProfPair* pp = prof_begin(SGA_PROF_REPLAY_PASS1, s);
-  if (bg) launch_pass1<true>(n_b, nb, s, g, n, coef_dense, lst, partials, vec, grp.pack_extra);
-  else launch_pass1<false>(n_b, nb, s, g, n, coef_dense, lst, partials, vec, grp.pack_extra);
+  if (bg) launch_pass1<true>(n_b, nb, s, g, n, coef_dense, lst, partials, vec, grp.pack_extra, now);
+  else launch_pass1<false>(n_b, nb, s, g, n, coef_dense, lst, partials, vec, grp.pack_extra, now);
   prof_end(pp, s);
   hipLaunchKernelGGL(k_replay_coef, dim3((unsigned)G), dim3(kBlock), 0, s, partials, (int)nb, G, clip, qn2, coef_d, coef_f, al);
   return check_launch("sga_replay_pass1");
+}
+
+extern "C" int sga_replay_pass1(const void* g, int g_dtype, int64_t n, float coef_dense, double clip,
+                                const sga_replay_cfg* cfgs, int G, double* partials, double* qn2,
+                                double* coef_d, float* coef_f, void* stream) {
+  SegNow now;
+  now.segs = nullptr; now.rsegs = nullptr; now.count = 0;
+  return replay_pass1(g, g_dtype, n, coef_dense, clip, cfgs, G, partials, qn2, coef_d, coef_f, now, stream);
+}
+
+extern "C" int sga_replay_begin(const void* g, int g_dtype, int64_t n, float coef_dense, double clip,
+                                const sga_replay_cfg* cfgs, int G, double* partials, double* qn2,
+                                double* coef_d, float* coef_f, sga_segment* segs, sga_replay_segment* rsegs,
+                                int n_segs, const double* lr, const float* bc1, const float* bc2,
+                                void* stream) {
+  if ((!segs && !rsegs) || n_segs < 1 || !lr || !bc1 || !bc2) {
+    set_error("sga_replay_begin: bad argument (n_segs=%d)", n_segs);
+    return SGA_ERR_ARG;
+  }
+  SegNow now;
+  if (!seg_now_fill(&now, segs, rsegs, n_segs, lr, bc1, bc2)) {
+    const int rc = sga_segments_refresh(segs, rsegs, n_segs, lr, bc1, bc2, stream);
+    if (rc != SGA_OK) return rc;
+  }
+  return replay_pass1(g, g_dtype, n, coef_dense, clip, cfgs, G, partials, qn2, coef_d, coef_f, now, stream);
 }
 
 extern "C" int sga_replay_pass3(const void* g, int g_dtype, int64_t n, float coef_dense,
@@ -1160,10 +1242,9 @@ extern "C" int sga_replay_reselect_balanced(const void* g, int g_dtype, const fl
 #undef SGA_RB
 }
 
-extern "C" int sga_dense_replay_step(const void* g, int g_dtype, float* w, float* m, float* v,
-                                     float* lab, int64_t n, const sga_replay_segment* segs,
-                                     int n_segs, int adams, double coef_dense, double* partials,
-                                     double* recon2, void* stream) {
+static int dense_replay_step(const void* g, int g_dtype, float* w, float* m, float* v, float* lab, int64_t n,
+                             const sga_replay_segment* segs, int n_segs, int adams, double coef_dense,
+                             double* partials, double* recon2, const SegNow& now, void* stream) {
   if (!g || !w || !m || !v || !segs || !partials || !recon2 || n < 1 || n_segs < 1 ||
       !(coef_dense > 0.0) || (g_dtype != SGA_F32 && g_dtype != SGA_BF16)) {
     set_error("sga_dense_replay_step: bad argument");
@@ -1177,11 +1258,38 @@ extern "C" int sga_dense_replay_step(const void* g, int g_dtype, float* w, float
   const unsigned nb = stream_grid(n, (int64_t)kBlock * kVec, kReplayBlocks * kMaxCfg);
   hipStream_t s = (hipStream_t)stream;
   const RSeg* rs = reinterpret_cast<const RSeg*>(segs);
-  if (bg) hipLaunchKernelGGL((k_dense_step<true>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec);
-  else hipLaunchKernelGGL((k_dense_step<false>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec);
+  if (bg) hipLaunchKernelGGL((k_dense_step<true>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec, now);
+  else hipLaunchKernelGGL((k_dense_step<false>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec, now);
   hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(kFoldThreads), 0, s, partials, (int)nb,
-                     coef_dense * coef_dense, recon2);
+                     coef_dense * coef_dense, recon2, now);
   return check_launch("sga_dense_replay_step");
+}
+
+extern "C" int sga_dense_replay_step(const void* g, int g_dtype, float* w, float* m, float* v,
+                                     float* lab, int64_t n, const sga_replay_segment* segs,
+                                     int n_segs, int adams, double coef_dense, double* partials,
+                                     double* recon2, void* stream) {
+  SegNow now;
+  now.segs = nullptr; now.rsegs = nullptr; now.count = 0;
+  return dense_replay_step(g, g_dtype, w, m, v, lab, n, segs, n_segs, adams, coef_dense, partials, recon2, now,
+                           stream);
+}
+
+extern "C" int sga_dense_replay_step_at(const void* g, int g_dtype, float* w, float* m, float* v, float* lab,
+                                        int64_t n, sga_replay_segment* segs, int n_segs, const double* lr,
+                                        const float* bc1, const float* bc2, int adams, double coef_dense,
+                                        double* partials, double* recon2, void* stream) {
+  if (!segs || n_segs < 1 || !lr || !bc1 || !bc2) {
+    set_error("sga_dense_replay_step_at: bad argument (n_segs=%d)", n_segs);
+    return SGA_ERR_ARG;
+  }
+  SegNow now;
+  if (!seg_now_fill(&now, nullptr, segs, n_segs, lr, bc1, bc2)) {
+    const int rc = sga_segments_refresh(nullptr, segs, n_segs, lr, bc1, bc2, stream);
+    if (rc != SGA_OK) return rc;
+  }
+  return dense_replay_step(g, g_dtype, w, m, v, lab, n, segs, n_segs, adams, coef_dense, partials, recon2, now,
+                           stream);
 }
 
 extern "C" int64_t sga_plane_words(int64_t n) {

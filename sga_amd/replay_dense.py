@@ -50,10 +50,11 @@ class DenseReplay:
         self.label = torch.zeros(self.N, dtype=torch.float32, device=dev)
         self._partials = torch.empty(int(L.raw("sga_replay_partials")), dtype=torch.float64,
                                      device=dev)
-        self._recon2 = torch.zeros(1, dtype=torch.float64, device=dev)
+        # the fold writes its sum straight into host memory: a step waits for it, and a copy would be
+        # one more thing to wait for
+        self._recon2 = torch.zeros(1, dtype=torch.float64, pin_memory=True)
         self._dist = torch.zeros(1, dtype=torch.float64, device=dev)
         self._seg_table = SegmentTable(entries, dev, start="a", segs=False, rsegs=True)
-        self._seg_dev = self._seg_table.rsegs
         self.si = 0
         self.den_at, self.snapshots, self.recon_steps = {}, {}, []
 
@@ -67,12 +68,13 @@ class DenseReplay:
         coef_dense, flag = coef_dense_for(gmeta)
         count = self.t0 + self.si + 1
         self._seg_table.follow(self.entries)          # callers may change them between steps
-        self._seg_table.refresh(lr_by_group(gmeta, self.entries), count, self.optimizer == "adamw")
+        self._seg_table.take(lr_by_group(gmeta, self.entries), count, self.optimizer == "adamw")
         st = L.stream()
-        L.call("sga_dense_replay_step", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),
-               L.ptr(self.v), L.ptr(self.label), self.N, L.ptr(self._seg_dev),
-               len(self.entries), int(self.optimizer == "adams"), float(coef_dense),
-               L.ptr(self._partials), L.ptr(self._recon2), st)
+        L.call("sga_dense_replay_step_at", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),
+               L.ptr(self.v), L.ptr(self.label), self.N, *self._seg_table.args[1:],
+               int(self.optimizer == "adams"), float(coef_dense), L.ptr(self._partials),
+               L.ptr(self._recon2), st)
+        torch.cuda.current_stream().synchronize()
         recon = math.sqrt(float(self._recon2.item()))
         norm = float(gmeta.get("grad_norm", float("nan")))
         self.recon_steps.append({

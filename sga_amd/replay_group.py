@@ -191,11 +191,12 @@ class ReplayGroup:
                     L.call("sga_div_inplace", C.c_void_p(self.state[ci].base("res")), N,
                            L.f32(float(c.T)), 1, st)
         self._seg_table.follow(self.entries)         # callers may change them between steps
-        self._seg_table.refresh([float(lr(e)) for e in self.entries] if callable(lr) else float(lr), count)
+        self._seg_table.take([float(lr(e)) for e in self.entries] if callable(lr) else float(lr), count)
         self._fill_cfgs(bnd, {})
         gd = L.dtype_code(g)
-        L.call("sga_replay_pass1", L.ptr(g), gd, N, L.f32(coef_dense), clip, self._cfg_host, G,
-               L.ptr(self.partials), L.ptr(self.qn2), L.ptr(self.coef_d), L.ptr(self.coef_f), st)
+        L.call("sga_replay_begin", L.ptr(g), gd, N, L.f32(coef_dense), clip, self._cfg_host, G,
+               L.ptr(self.partials), L.ptr(self.qn2), L.ptr(self.coef_d), L.ptr(self.coef_f),
+               *self._seg_table.args, st)
         out_sel = {}
         # boundary re-selections of this step: under the exact-k semantics they go out as ONE
         # call (configs that rank by the same score share the short kernels of the select)

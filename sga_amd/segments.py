@@ -50,9 +50,10 @@ class SegmentTable:
         self.segs = _host_table(_SEGMENT, rows, start).to(device) if segs else None
         self.rsegs = _host_table(_REPLAY_SEGMENT, rows, start).to(device) if rsegs else None
         self._lr, self._bc1, self._bc2 = (np.zeros(self.count, dtype=d) for d in ("f8", "f4", "f4"))
-        self._args = (None if self.segs is None else self.segs.data_ptr(),
-                      None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
-                      self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
+        # (segs, rsegs, rows, lr, bc1, bc2): what sga_segments_refresh and sga_replay_begin take
+        self.args = (None if self.segs is None else self.segs.data_ptr(),
+                     None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
+                     self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
         self._hyper = list(map(_HYPER, rows))
         self._betas = self._last_lr = None
         self.follow_betas(rows)
@@ -80,13 +81,17 @@ class SegmentTable:
         self._hyper = hyper
         self.follow_betas(rows)
 
-    def refresh(self, lr, count, bias_correction=True):
+    def take(self, lr, count, bias_correction=True):
         """Learning rates (one number, or one per row) and the bias corrections of
-        step ``count``, on the current stream."""
+        step ``count`` into the host columns, for a call that carries ``args``."""
         lr = list(map(float, lr)) if isinstance(lr, list) else float(lr)   # the caller may change its list
         if lr != self._last_lr:
             self._lr[:] = self._last_lr = lr
         for (b1, b2), at in self._groups:
             self._bc1[at] = float(1.0 - b1 ** count) if bias_correction else 1.0
             self._bc2[at] = float(1.0 - b2 ** count) if bias_correction else 1.0
-        L.call("sga_segments_refresh", *self._args, L.stream())
+
+    def refresh(self, lr, count, bias_correction=True):
+        """The same into the device tables, on the current stream."""
+        self.take(lr, count, bias_correction)
+        L.call("sga_segments_refresh", *self.args, L.stream())
