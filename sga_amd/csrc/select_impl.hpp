@@ -2132,7 +2132,7 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 //
 // The chain comes in phases so that a batch whose jobs form their keys differently (the
 // re-selections of a replay step rank by different scores) still shares every kernel that does
-// not form keys: chain_begin, chain_pick_* and chain_settle take the whole batch; chain_sample_*,
+// not form keys: chain_begin, chain_pick_fine and chain_settle take the whole batch; launch_sample_*,
 // chain_sweeps and chain_tail are templates of the key source and take the jobs of one kind (a sub-batch
 // over the same workspaces).
 static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStream_t s) {
