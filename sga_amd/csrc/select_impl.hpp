@@ -9,6 +9,7 @@
 #include <atomic>
 #include <type_traits>
 #include "adam_math.hpp"
+#include "sel_state.hpp"
 #include "wide_scan.hpp"
 
 namespace sga {
@@ -19,48 +20,6 @@ constexpr int kBinsBig = 4096, kBinsSmall = 128;
 constexpr int kTileScanPer = 16;
 constexpr int kTileScanSpan = kBlock * kTileScanPer;  // 4096 tiles / workgroup
 constexpr int kMaxTileBlocks = 1024;                  // covers n < 2^32
-
-struct SelState {
-  uint32_t k;
-  uint32_t prefix;
-  uint32_t krem;
-  uint32_t thresh_bits;
-  uint32_t need;
-  uint32_t n_gt;
-  uint32_t n_eq;
-  uint32_t nonfinite;
-  uint32_t status;
-  uint32_t total;
-  uint32_t n_selected;
-  uint32_t path;
-  // sampled-bracket path
-  uint32_t t_lo;        // candidates are keys in [t_lo, t_hi)
-  uint32_t t_hi;
-  uint32_t n_hi;        // keys >= t_hi
-  uint32_t cand_count;  // keys in the bracket (may exceed capacity)
-  uint32_t bracket_ok;  // 1: the sampled bracket holds the k-th key; radix passes skip
-  uint32_t overflow;    // a candidate segment ran out of room
-  uint32_t skip;        // 1: kernels driven by this state do nothing
-  uint32_t done[3];     // per-level "workgroups finished" tickets (last one scans)
-  uint32_t spec;        // 1: the single-sweep step committed on the sampled bracket (no way back)
-  uint32_t negative;    // 1: an fp32 score array held a value below zero (magnitudes were ranked)
-  uint32_t redone;      // 1: an out-of-place single-sweep step missed its bracket and was redone
-  uint32_t in_sample;   // sample keys inside the bracket (~0: open below, nothing bounds them)
-  uint32_t ticket;      // k_settle: workgroups that are done
-  uint32_t edge_cnt;    // k_settle: entries of the edge list
-  uint32_t edge_inv;    // k_settle: ~(smallest key of the edge list), and ...
-  uint32_t edge_max;    // ... the largest, by atomic maxima (0: none)
-  uint32_t ties_left;   // the settlement has left the ties to k_tail
-  uint32_t tail_ticket; // k_tail: items handed out, and ...
-  uint32_t tail_done;   // ... finished
-  uint32_t finish_ticket; // k_small_finish: workgroups that have begun; the first one judges the bracket ...
-  uint32_t verdict;     // ... 1: it holds the k-th key, 2: all of them go over the data again
-  uint32_t redo_step;   // passes of that which are done
-  uint32_t sampled[16]; // k_sample_pick: the launch that a workgroup of the sample has finished in
-  uint32_t pad_[12];
-};
-static_assert(sizeof(SelState) == 256, "whole cache lines");
-static_assert(sizeof(SelState) == 256, "SelState layout");
 
 struct SelWorkspace {
   SelState* st;        // main state (result, bracket)
@@ -983,8 +942,8 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // alone would be bound by its CU's translation misses (4096 quads of two arrays: 25 us).  A workgroup that has
 // left its keys leaves the launch's number beside them and looks at the others': whoever sees all of them picks.
 // Nobody waits for anybody, and two that see all numbers at once do the same and write the same.  (Numbers of an
-// earlier launch are gone: the pick writes the whole state.  Memory that happens to hold the number could only
-// spoil the sample, and the select is exact for any.)  As two launches (three with the clearing kernel of the large
+// earlier launch are gone: the pick writes the whole state.  Memory that happens to hold the number spoils the
+// sample and no more, see sampled_key.)  As two launches (three with the clearing kernel of the large
 // buckets) before -> after, us: step of 261 K 36.0 -> 34.4, 4 M 77.5 -> 74.3, 40 M 429 -> 419; select of 3 M 68.5 -> 60.8.
 //
 // The pick: one LDS histogram of the top 13 bits of all keys.  The ends of the bins that the two ends of the
@@ -1059,8 +1018,8 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
     for (int h = 0; h < 2; ++h) {
       const unsigned long long q =
           j < n_sv ? __hip_atomic_load(&sample[2 * j + h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-      key[u][2 * h] = (uint32_t)q;
-      key[u][2 * h + 1] = (uint32_t)(q >> 32);
+      key[u][2 * h] = sampled_key(q, 0);
+      key[u][2 * h + 1] = sampled_key(q, 1);
     }
   }
   const uint32_t ns = (uint32_t)(n_sv * 4);
@@ -1145,13 +1104,9 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
       if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
     }
   }
-  if (threadIdx.x == 0) {
-    SelState z = {};
-    z.k = J.k;
-    z.t_hi = t_hi;
-    z.t_lo = t_lo;
-    *st = z;
-  }
+  if (threadIdx.x < kStateWords)
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(st) + threadIdx.x, picked_word(threadIdx.x, J.k, t_lo, t_hi),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // The fine sample of a large bucket: only how its keys fall relative to the coarse bracket is kept --
