@@ -61,6 +61,12 @@ static_assert(sizeof(SelState) == 256, "whole cache lines");
 SGA_HOST_DEVICE static inline uint32_t sampled_key(unsigned long long word, int half) {
   return (uint32_t)(word >> (32 * half)) & 0x7FFFFFFFu;
 }
+// Number of the count-th launch of the library that takes a sample: different for 2^31 launches, odd and so never
+// zero as a cleared mark is, and spread over all 32 bits (consecutive small numbers are what index lists, counts
+// and flags in recycled memory look like).  A recorded graph repeats its numbers: its marks are zero again at
+// every start because the pick clears them and so does the kernel behind it (an early pick's clearing may come
+// before the last mark).
+SGA_HOST_DEVICE static inline uint32_t launch_number(uint32_t count) { return (2u * count + 1u) * 0x9E3779B1u; }
 constexpr int kStateWords = sizeof(SelState) / 8;
 constexpr int kBracketWord = offsetof(SelState, t_lo) / 8;
 static_assert(offsetof(SelState, t_lo) % 8 == 0 && offsetof(SelState, t_hi) == offsetof(SelState, t_lo) + 4,

@@ -1,8 +1,14 @@
 // Exact top-k selection entry points over fp32 score arrays, plus the
 // histogram / candidate / compare building blocks of the replay select.
+#include <atomic>
+
 #include "small_select.hpp"
 
 namespace sga {
+uint32_t next_launch() {
+  static std::atomic<uint32_t> count{0};
+  return launch_number(count.fetch_add(1u, std::memory_order_relaxed));
+}
 int exclusive_scan_u32(uint32_t* data, int64_t n, int64_t* total, hipStream_t st);
 int64_t scan_scratch_entries(int64_t n);
 

@@ -6,7 +6,6 @@
 // per-chunk count so that ties at the threshold can be granted in ascending
 // index order without any float compare ambiguity.
 #pragma once
-#include <atomic>
 #include <type_traits>
 #include "adam_math.hpp"
 #include "sel_state.hpp"
@@ -2094,11 +2093,8 @@ static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStr
   static_assert(sizeof(ChainJobs) + sizeof(SegDirJobs) + 64 <= 4096, "operands travel in the kernel arguments");
   hipLaunchKernelGGL(k_chain_begin, B.grid(4), dim3(kBlock), 0, s, B.jobs, dirs);
 }
-// Numbers of the launches that take a sample (never zero, as a cleared state is).
-static inline uint32_t next_launch() {
-  static std::atomic<uint32_t> count{0};
-  return count.fetch_add(2u, std::memory_order_relaxed) | 1u;
-}
+// Number of the next launch that takes a sample: one count for the whole library (select.hip).
+uint32_t next_launch();
 template <bool COARSE, class Src>
 static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
                                       hipStream_t s) {

@@ -59,6 +59,7 @@ __global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, Chain
   __shared__ uint32_t s_hi[CPW][kChunkIters], s_eq[CPW][kChunkIters], s_cnt[kChunkIters], s_nf[kChunkIters], s_base;
   static_assert(kChunkIters == kChunksPerBlock && CPW <= kWave, "a wave per slab");
   SelState* __restrict__ st = J.st;
+  if (blockIdx.x == 0 && threadIdx.x < kSampleGroups) st->sampled[threadIdx.x] = 0u;      // see launch_number
   Src src = srcs.s[blockIdx.y];
   const int64_t i0 = c0 * kChunk + uniform_i32(wave_id()) * (kWave * kVec);
   typename Src::Raw raw[CPW];

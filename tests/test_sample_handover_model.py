@@ -23,7 +23,7 @@ STALE = 0xF0000005                                     # what the memory held, b
 
 
 def _runs(marks, masked, one_word):
-    """All ends of one launch: ``(bracket, brackets picked, worst bin)``."""
+    """All ends of one launch: ``(bracket, brackets picked, worst bin, marks left)``."""
     ends, seen = set(), set()
     # per workgroup: 0 store keys, 1 store mark, 2 look, 3 read and pick, 4 (and 5) write the state, None done
     start = ((0,) * GROUPS, (STALE,) * GROUPS, tuple(marks), (None, None), ((),) * GROUPS, -1)
@@ -35,7 +35,7 @@ def _runs(marks, masked, one_word):
         seen.add(state)
         pcs, words, marks_, bracket, picks, worst = state
         if all(pc is None for pc in pcs):
-            ends.add((bracket, tuple(p for p in picks if p), worst))
+            ends.add((bracket, tuple(p for p in picks if p), worst, marks_))
             continue
         for g, pc in enumerate(pcs):
             if pc is None:
@@ -67,19 +67,31 @@ _MEMORIES = [[NUMBER * (bits >> g & 1) for g in range(GROUPS)] for bits in range
 
 @pytest.mark.parametrize("marks", _MEMORIES)
 def test_any_memory_leaves_a_bracket_of_one_pick(marks):
-    for bracket, picks, worst in _runs(marks, masked=True, one_word=True):
+    for bracket, picks, worst, left in _runs(marks, masked=True, one_word=True):
         assert picks and bracket in picks and bracket[0] < bracket[1]
         assert worst < BINS
         if not any(marks):                                # marks cleared before: the launch's own keys
-            assert set(picks) == {(min(OWN), max(OWN) + 1)}
+            assert set(picks) == {(min(OWN), max(OWN) + 1)} and not any(left)
 
 
 def test_the_replaced_protocol_does_neither():
     ends = [e for m in _MEMORIES for e in _runs(m, masked=False, one_word=False)]
-    assert any(worst >= BINS for _, _, worst in ends)
-    assert any(bracket not in picks for bracket, picks, _ in ends)
+    assert any(worst >= BINS for _, _, worst, _ in ends)
+    assert any(bracket not in picks for bracket, picks, _, _ in ends)
     # on cleared marks it was sound
-    assert all(b in p and w < BINS for b, p, w in _runs([0] * GROUPS, masked=False, one_word=False))
+    assert all(b in p and w < BINS for b, p, w, _ in _runs([0] * GROUPS, masked=False, one_word=False))
+
+
+def test_a_mark_can_come_after_the_clearing():
+    """Which is why the next kernel clears the marks again: a recorded graph starts every
+    replay with the same number."""
+    assert any(any(left) for m in _MEMORIES for *_, left in _runs(m, masked=True, one_word=True))
+
+
+def test_one_count_of_launches_in_the_library():
+    lib = os.path.join(ROOT, "sga_amd", "libsga_hip.so")
+    names = subprocess.run(["nm", "-C", lib], capture_output=True, text=True, check=True).stdout
+    assert names.count("next_launch()::count") == 1
 
 
 _PROGRAM = r"""
@@ -103,6 +115,13 @@ int main() {
   std::memcpy(&got, words, sizeof(got));
   want.k = 123456789u; want.t_lo = 0x3F000001u; want.t_hi = 0x80000000u;
   bad += std::memcmp(&got, &want, sizeof(got)) != 0;
+  // numbers of launches: never the cleared mark, none twice
+  static unsigned char seen[1 << 29];
+  for (uint32_t c = 0; c < 3000000u; ++c) {
+    const uint32_t x = launch_number(c);
+    bad += x == 0u || (seen[x >> 3] >> (x & 7) & 1);
+    seen[x >> 3] |= (unsigned char)(1u << (x & 7));
+  }
   std::printf("%d\n", bad);
   return bad != 0;
 }
