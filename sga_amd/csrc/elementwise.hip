@@ -703,6 +703,7 @@ static int mask_count(const char* who, const uint8_t* mask, int64_t n, uint32_t*
                        n, chunk_counts, nc);
   int rc = exclusive_scan_u32(chunk_counts, nc, total, st);
   if (rc) return rc;
+  if (step > n) step = n;                // the same answers, and j * step cannot wrap around
   if (cuts > 0)
     hipLaunchKernelGGL(k_mask_cuts, dim3((unsigned)cdiv64(cuts, kChunksPerBlock)), dim3(kBlock), 0, st, mask, n,
                        chunk_counts, step, cuts, total);

@@ -38,3 +38,15 @@ def test_mask_layout_slices(dev, n, slices):
     assert len(payloads) == slices
     for p, a, b in zip(payloads, ends[:-1], ends[1:]):
         assert torch.equal(p.cpu(), grad[a:b][mask[a:b].bool()] * 0.5)
+
+
+# cuts far past the end: j * step must not wrap around into the list (2 * 2^62 would)
+@pytest.mark.parametrize("n", [0, 1, 5000])
+@pytest.mark.parametrize("step", [2 ** 31, 2 ** 62, 2 ** 63 - 1])
+def test_steps_past_the_end(dev, n, step):
+    from sga_amd import _lib as L
+    mask = torch.ones(n, dtype=torch.uint8, device=dev)
+    counts = torch.empty(int(L.raw("sga_mask_chunks", n)) + 8, dtype=torch.int32, device=dev)
+    totals = torch.full((6,), -1, dtype=torch.int64, device=dev)
+    L.call("sga_mask_count_cuts", L.ptr(mask), n, L.ptr(counts), step, 5, L.ptr(totals), L.stream())
+    assert totals.tolist() == [n] * 6
