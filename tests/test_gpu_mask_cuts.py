@@ -50,3 +50,28 @@ def test_steps_past_the_end(dev, n, step):
     totals = torch.full((6,), -1, dtype=torch.int64, device=dev)
     L.call("sga_mask_count_cuts", L.ptr(mask), n, L.ptr(counts), step, 5, L.ptr(totals), L.stream())
     assert totals.tolist() == [n] * 6
+
+
+# chunks just below, at and above the density from which their positions are staged, all set, and lists shorter
+# than the mask has bytes
+@pytest.mark.parametrize("at", [0, 3])
+@pytest.mark.parametrize("counts", [[159, 160, 161, 0, 1024], [1024] * 9, [1, 1023, 1024, 17, 500, 160]])
+def test_dense_chunks_and_short_lists(dev, counts, at):
+    from sga_amd import _lib as L
+    gen = torch.Generator().manual_seed(sum(counts))
+    n = 1024 * len(counts) - 5 * (counts[-1] < 1000)
+    mask = torch.zeros(1024 * len(counts) + at, dtype=torch.uint8)
+    for c, k in enumerate(counts):
+        mask[at + 1024 * c:at + 1024 * (c + 1)][torch.randperm(1019 if k < 1000 else 1024, generator=gen)[:k]] = 1 + c
+    on = mask[at:at + n].nonzero().view(-1).to(torch.int32)
+    md = mask.to(dev)[at:at + n]
+    work = torch.empty(int(L.raw("sga_mask_chunks", n)), dtype=torch.int32, device=dev)
+    total = torch.empty(1, dtype=torch.int64, device=dev)
+    L.call("sga_mask_count", L.ptr(md), n, L.ptr(work), L.ptr(total), L.stream())
+    k = on.numel()
+    assert total.item() == k
+    for cap in sorted({1, 3, 159, 160, 163, k // 2, k - 1, k, k + 7}):
+        idx = torch.full((max(cap, k) + 8,), -7, dtype=torch.int32, device=dev)
+        L.call("sga_mask_fill", L.ptr(md), n, L.ptr(work), L.ptr(idx), cap, L.stream())
+        got, put = idx.cpu(), min(cap, k)
+        assert torch.equal(got[:put], on[:put]) and bool((got[put:] == -7).all()), cap
