@@ -947,8 +947,12 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 //
 // The pick: one LDS histogram of the top 13 bits of all keys.  The ends of the bins that the two ends of the
 // bracket fall into will do, rounded outwards, as long as that takes in no more than a quarter of the bracket's
-// own ranks in addition; otherwise (narrow distributions, plateaus) the next 12 bits of the keys in the two bins
-// go into a histogram each, and what is left in a bin then is ranked by counting, or split by the last 6 bits.
+// own ranks in addition and no bin between them holds a third of those ranks; otherwise (narrow distributions,
+// plateaus) the next 12 bits of the keys in the two bins go into a histogram each, and what is left in a bin then is
+// ranked by counting, or split by the last 6 bits.  A plateau that holds both ends shrinks the bracket to its one key
+// that way, whose members nobody lists.  Selects with a plateau of f times k keys around the k-th (1 %), bin edges
+// without a look at the bins between / with: 8.4 M f = 0.9 226 / 81 us, 20 M f = 1.6 315 / 156, 100 M f = 0.6
+// 980 / 518; without plateaus both alike, and key ends everywhere cost 3 us more (8 at 10 % of a large bucket).
 // kBracketSigmas etc.: the small buckets bracket the k-th key of the data this way.  The large ones
 // (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with eight
 // sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.  Sigma
@@ -960,6 +964,7 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // the directories of the segment tables (dirs.j[job].dir null: none wanted).
 constexpr int kSampleGroups = 16;
 constexpr int kPickBits = 13, kPickShift = 31 - kPickBits;
+constexpr uint32_t kHeavyBin = 3;                    // a half misses the 100 M case above, a quarter measured the same
 template <class Src, bool COARSE>
 __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
                                                        uint32_t launch, double sigmas) {
@@ -1056,8 +1061,14 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
     uint32_t rk[2] = {rank[0] - hit[0].above, rank[1] - hit[1].above};
     uint32_t cnt[2] = {hit[0].count, hit[1].count};
     int w = kPickShift, turn = 1;                      // bits of a key below the bins found so far
-    const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]);
-    if (4u * more <= rank[1] - rank[0]) {
+    const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]), held = rank[1] - rank[0];
+    bool heavy = false;
+#pragma unroll
+    for (int j = 0; j < 2 * kBinsBig / kWide; ++j) {
+      const uint32_t b = (uint32_t)j * kWide + threadIdx.x;
+      heavy = heavy || (b >= bin[1] && b <= bin[0] && kHeavyBin * s_h[0][b] > held);
+    }
+    if (!__syncthreads_or(heavy) && 4u * more <= held) {
       if (!open_hi) t_hi = (bin[0] + 1u) << w;
       if (!open_lo) t_lo = bin[1] << w;
     } else {
