@@ -160,8 +160,8 @@ struct SmallList {
 #pragma unroll
     for (int u = 0; u < kSmallHead; ++u) trim(key[u], (uint32_t)(u * kWave + lane_id()) * kVec, c);
   }
-  // head(key, idx) over the entries in registers, tail(key, idx) over the rest (whole waves).  IDX: the index is
-  // wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a microsecond
+  // head(key, idx) over the entries in registers, tail(keys, idxs) over rounds of quads of the rest (whole waves).
+  // IDX: the index is wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a microsecond
   // a round of loads, so the next round is on its way while one is worked off.
   template <bool IDX, class H, class T>
   __device__ __forceinline__ void visit(H&& head, T&& tail) const {
@@ -191,11 +191,17 @@ struct SmallList {
         trim(k[u], (q0 + u * kWave + lane_id()) * kVec, cnt);
       }
       if ((q0 + U * kWave) * kVec < cnt) request_from(q0 + U * kWave);
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        tail(k[u].x, i[u].x); tail(k[u].y, i[u].y); tail(k[u].z, i[u].z); tail(k[u].w, i[u].w);
-      }
+      tail(k, i);
     }
+  }
+  template <int U, class F>
+  static __device__ __forceinline__ void each(const U4 (&k)[U], const U4 (&i)[U], F&& f) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) { f(k[u].x, i[u].x); f(k[u].y, i[u].y); f(k[u].z, i[u].z); f(k[u].w, i[u].w); }
+  }
+  template <class F>
+  __device__ __forceinline__ void visit_all(F&& f) const {
+    visit<true>(f, [&](const auto& k, const auto& i) { each(k, i, f); });
   }
 };
 static_assert(kSmallHead * kWave * kVec <= 2 * kChunk, "the head never reaches past a segment");
@@ -211,7 +217,7 @@ static_assert(kSmallHead * kWave * kVec <= 2 * kChunk, "the head never reaches p
 constexpr int kRedoGroups = 64;                       // at most; one per kRedoTiles chunks
 constexpr int kRedoTiles = 32;
 constexpr uint32_t kCrowdedList = 1 << 16;            // shorter lists are walked in less time than the passes take
-                                                      // (1.3 us a thousand equal keys, 50 to 190 us the passes)
+                                                      // (0.9 us a thousand keys of a plateau, 50 to 190 us the passes)
 template <class Src>
 __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t* s_hist, WideScratch& s_scan,
                                            uint32_t* s_word) {
@@ -356,7 +362,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     auto above = [&](uint32_t key, uint32_t idx) {
       if (key != ~0u) atomicAdd(&s_tile[idx >> 10], 1u);
     };
-    list.visit<true>(above, above);
+    list.visit_all(above);
     __syncthreads();
   } else if (ok) {
     // the lower end is below the threshold: its members are no ties
@@ -368,12 +374,28 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     int w = 32 - __clz((int)(T_HI - 1u - lo));         // bits of the offset (the list is not empty)
     for (;;) {
       const int sh = w > 12 ? w - 12 : 0;
-      // (plain adds: 64 lanes on one bin cost no more than asking whether they are)
       auto count = [&](uint32_t key, uint32_t) {
         const uint32_t off = key - lo;
         if (off >> w == 0u) atomicAdd(&s_hist[off >> sh], 1u);
       };
-      list.visit<false>(count, count);
+      // A plateau in a long list queues on its bin: where sixteen lanes' first keys of a round share one, the lanes
+      // of that bin add together.  8.4 M coordinates, plateaus inside the bracket, plain adds / this: at 1 % 256 / 180
+      // and 295 / 181 us, at 10 % 564 / 272; without plateaus 96.7 / 96.5 and 132.6 / 133.1 (to ask for every key: 146).
+      auto count_round = [&](const auto& k, const auto& i) {
+        const uint32_t first = k[0].x - lo, lead = (uint32_t)uniform_i32((int)(first >> sh));
+        if (__popcll(ballot64(first >> w == 0u && first >> sh == lead)) < 16) {
+          SmallList::each(k, i, count);
+        } else {
+          SmallList::each(k, i, [&](uint32_t key, uint32_t) {
+            const uint32_t off = key - lo;
+            const bool in = off >> w == 0u, with = in && off >> sh == lead;
+            const uint32_t same = (uint32_t)__popcll(ballot64(with));
+            if (same && lane_id() == 0) atomicAdd(&s_hist[lead], same);
+            if (in && !with) atomicAdd(&s_hist[off >> sh], 1u);
+          });
+        }
+      };
+      list.visit<false>(count, count_round);
       __syncthreads();
       const uint32_t want[1] = {rank};
       RankHit h[1];
@@ -396,7 +418,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
         const uint32_t off = key - lo;
         if ((int32_t)off >= 0) atomicAdd(&s_tile[idx >> 10], off < width ? 1u << 16 : 1u);
       };
-      list.visit<true>(place, place);
+      list.visit_all(place);
     } else {
       auto place = [&](uint32_t key, uint32_t idx) {
         const uint32_t off = key - lo;
@@ -407,7 +429,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
           s_idx[at] = idx;
         }
       };
-      list.visit<true>(place, place);
+      list.visit_all(place);
     }
     T = lo;
     need = rank;
