@@ -137,17 +137,7 @@ struct SegCursor {
   // to do meanwhile; a long sweep's scalar loads hit the scalar cache instead.
   __device__ __forceinline__ void seek_wave(int64_t i) {
     if (i >= lo && i < hi) return;
-    int a = 0, len = n_segs;
-    while (len > 1) {
-      const int step = (len + kWave - 1) / kWave;
-      const int e = a + lane_id() * step;
-      const bool below = e < a + len && segs[e].start <= i;
-      const int hit = __popcll(ballot64(below)) - 1;       // the table starts at 0: entry a is always below
-      const int end = a + len;
-      a += (hit < 0 ? 0 : hit) * step;
-      len = end - a < step ? end - a : step;
-    }
-    take_uniform(uniform_i32(a));
+    take_uniform(wave_last(n_segs, [&](int e) { return segs[e].start <= i; }));
   }
   // Steps to the segment that holds i, a little past the cached one (the
   // next tensor of a slab that straddles a boundary).
@@ -194,7 +184,7 @@ static inline void launch_seg_dir(const sga_segment* segs, int n_segs, int64_t n
 // change only at tensor boundaries, so the slab is scored once per segment
 // that intersects it (one, but for the few slabs that hold a boundary) with
 // that segment's hyper-parameters as scalar operands.  `sc` was placed on the
-// slab's chunk with seek_uniform and is only ever moved by the uniform seeks.
+// slab's chunk or the slab (seek_uniform, seek_wave) and is only ever moved by uniform seeks.
 // key[] comes in zeroed; quads past n stay zero.
 template <int SCORE, bool FULL>
 __device__ __forceinline__ void slab_score_keys(SegCursor& sc, int adams, int64_t i, int64_t n,
@@ -204,7 +194,7 @@ __device__ __forceinline__ void slab_score_keys(SegCursor& sc, int adams, int64_
   const int64_t s0 = uniform_i64(i);
   int64_t s1 = s0 + kWave * kVec;
   if (!FULL && s1 > n) s1 = n;
-  if (s0 >= sc.hi) sc.advance_uniform(s0);   // slabs of a chunk ascend from its seek_uniform
+  if (s0 >= sc.hi) sc.advance_uniform(s0);   // slabs of a chunk ascend from where it began
   for (;;) {
     Hyper h = sc.h;
     if (adams) { h.bc1 = 1.0f; h.bc2 = 1.0f; }

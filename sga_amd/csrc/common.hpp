@@ -404,23 +404,28 @@ __device__ __forceinline__ void plane_collect(const uint32_t flag[4], int it, ui
   }
 }
 
-// The record that owns span `span` of a table ordered by first_span: the last one whose first
-// span is <= it.  Every lane of the wave looks at an entry of its own, so a table of up to 64
-// records takes one round of loads (a bisection is a chain of them: 6 for 45 records, which a
-// workgroup of a 4096-element span spends before its first data load) and one of up to 4096 two.
-template <class R>
-__device__ __forceinline__ int find_record(const R* __restrict__ recs, int n_recs, int64_t span) {
-  int lo = 0, len = n_recs;
+// The last entry of an ascending table of n for which below(entry) holds, or 0.  Every lane of the
+// wave looks at an entry of its own, so a table of up to 64 takes one round of loads (a bisection is a
+// chain of them: 6 for 45 records, which a workgroup of a 4096-element span spends before its first
+// data load) and one of up to 4096 two.
+template <class B>
+__device__ __forceinline__ int wave_last(int n, B&& below) {
+  int lo = 0, len = n;
   while (len > 1) {
     const int step = (len + kWave - 1) / kWave;
     const int at = lo + lane_id() * step;
-    const bool below = at < lo + len && recs[at].first_span <= span;
-    const int hit = __popcll(ballot64(below)) - 1;       // entry 0 of the range is always below
+    const int hit = __popcll(ballot64(at < lo + len && below(at))) - 1;      // the range's first entry holds, or none does
     const int end = lo + len;
     lo += (hit < 0 ? 0 : hit) * step;
     len = end - lo < step ? end - lo : step;
   }
   return uniform_i32(lo);
+}
+// The record that owns span `span` of a table ordered by first_span: the last one whose first
+// span is <= it.
+template <class R>
+__device__ __forceinline__ int find_record(const R* __restrict__ recs, int n_recs, int64_t span) {
+  return wave_last(n_recs, [&](int e) { return recs[e].first_span <= span; });
 }
 
 #endif  // __HIPCC__

@@ -42,6 +42,7 @@ struct SrcFused {
   // scores that need the tensor's hyper-parameters
   static constexpr bool kHyper = SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI ||
                                  SCORE == SGA_SCORE_GR_OVER_SQRT_V;
+  static constexpr int kSweep = kHyper ? 1 : 0;                // bit planes instead of the chain a second time
   static constexpr bool kNeedG = SCORE != SGA_SCORE_ABS_M;
   // g == nullptr (fp32 instantiations only): the caller's buffer `r` already holds g + r, the
   // reference's own contract (backward accumulates into the buffer that keeps the residual)
@@ -439,7 +440,7 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
   } else {
     int64_t swept = 0;
     for (int b = 0; b < count; ++b) swept += fj[b].n * srcs.s[b].bytes();
-    run_select_batch<0>(srcs, B, dj, use_fast, planes ? 1 : 0, s, swept <= kKeepBytes);
+    run_select_batch<0>(srcs, B, dj, use_fast, s, swept <= kKeepBytes);
   }
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];

@@ -477,6 +477,7 @@ struct SrcReplay {
   struct Raw { RawG g; F4 r, w, m, v; };
   struct Chunk { int64_t sh; float coef; };
   static constexpr bool kReadAgain = false;
+  static constexpr int kSweep = 1;
   static constexpr bool kHyper = SCORE == SGA_SCORE_UPDATE || SCORE == SGA_SCORE_COI ||
                                  SCORE == SGA_SCORE_GR_OVER_SQRT_V;
   static constexpr bool kNeedG = SCORE != SGA_SCORE_ABS_M;
@@ -924,7 +925,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     });
     per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, s); });
     chain_pick_fine(B, kBracketSigmas, s);
-    per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, 1, s); });
+    per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, s); });
     chain_settle(B, s);
   }
   per_score([&](auto& srcs, const SelBatch& sub) { chain_tail<1>(srcs, sub, s); });

@@ -370,7 +370,7 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   const bool fast = SelBatch::fast_ok(w, n);
   // the select sweep writes the keys above the bracket straight into mask_out
   J.mask_only = 1;
-  run_select_batch<2>(srcs, B, SegDirJobs{}, fast, 2, s);
+  run_select_batch<2>(srcs, B, SegDirJobs{}, fast, s);
   return check_launch("sga_select_topk");
 }
 

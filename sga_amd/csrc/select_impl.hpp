@@ -239,6 +239,7 @@ struct SrcF32 {                 // |x| of an fp32 score array
   using Raw = F4;
   using Chunk = NoChunk;
   static constexpr bool kHyper = false, kReadAgain = false;
+  static constexpr int kSweep = 2;                       // see chain_sweeps
   static constexpr int kAhead = kChunkIters;
   __device__ __forceinline__ Chunk chunk_begin(int64_t) { return Chunk{}; }
   __device__ __forceinline__ void chunk_hyper(int64_t) {}
@@ -2090,9 +2091,9 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 // The select of every job of a batch: begin -> (sampled-bracket path: coarse sample and pick, fine sample
 // and pick, ONE data sweep per job, settlement) -> k_tail.  The short kernels run once for the whole
 // batch; only the data sweeps are launched per job.
-// PM: what the sweep leaves behind for a mask-only caller -- 0 nothing, 1 the keys above the
-// bracket as bit planes (job.planes), 2 as mask bytes (job.mask) -- where the settlement adds the
-// candidates; the tail's writing pass over the data then has nothing to do.
+// Src::kSweep: what the sweep leaves behind -- 0 nothing, 1 the keys above the bracket as bit planes
+// (job.planes), 2 as mask bytes (job.mask) -- where the settlement adds the candidates; the tail's
+// writing pass over the data then has nothing to do.
 // All jobs of a batch take the same path (`fast`: SelBatch::fast_ok for every one of them).
 //
 // The chain comes in phases so that a batch whose jobs form their keys differently (the
@@ -2132,7 +2133,8 @@ static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, co
 }
 // keep (sources that a writing pass reads again): see bracket_chunk
 template <class Src>
-static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int pm, hipStream_t s, bool keep = false) {
+static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s, bool keep = false) {
+  constexpr int PM = Src::kSweep;
   for (int b = 0; b < B.count; ++b) {
     const ChainJob& J = B.jobs.j[b];
     const SelWorkspace& w = B.w[b];
@@ -2143,15 +2145,11 @@ static inline void chain_sweeps(const SrcPack<Src>& srcs, const SelBatch& B, int
     auto sweep = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(sweep_blocks), dim3(kBlock), 0, s, srcs.s[b], J.n, w.st, w.rel, w.tile_gt,
                          w.tile_eq, w.seg_idx, w.seg_key, w.seg_cnt, (uint32_t)w.seg_cap,
-                         pm == 1 ? J.planes : (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
-                         pm == 2 ? J.mask : (uint8_t*)nullptr, true);
+                         PM == 1 ? J.planes : (uint32_t*)nullptr, w.blk_gt, w.blk_eq,
+                         PM == 2 ? J.mask : (uint8_t*)nullptr, true);
     };
-    constexpr bool again = Src::kReadAgain;
-    if (pm == 2) sweep(k_bracket_sweep<Src, 2>);
-    else if (pm == 1 && keep) sweep(k_bracket_sweep<Src, 1, again>);
-    else if (pm == 1) sweep(k_bracket_sweep<Src, 1>);
-    else if (keep) sweep(k_bracket_sweep<Src, 0, again>);
-    else sweep(k_bracket_sweep<Src, 0>);
+    if (Src::kReadAgain && keep) sweep(k_bracket_sweep<Src, PM, Src::kReadAgain>);
+    else sweep(k_bracket_sweep<Src, PM>);
     prof_end(pp, s);
   }
 }
@@ -2171,10 +2169,10 @@ static inline void chain_tail(const SrcPack<Src>& srcs, const SelBatch& B, hipSt
 
 template <int OUT, class Src>
 static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, bool fast,
-                                    int pm, hipStream_t s, bool keep = false) {
+                                    hipStream_t s, bool keep = false) {
   if (fast) {
     chain_bracket(srcs, B, dirs, kBracketSigmas, s);
-    chain_sweeps(srcs, B, pm, s, keep);
+    chain_sweeps(srcs, B, s, keep);
     chain_settle(B, s);
   } else {
     chain_begin(B, dirs, s);
