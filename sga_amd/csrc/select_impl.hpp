@@ -943,17 +943,19 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // left its keys leaves the launch's number beside them and looks at the others': whoever sees all of them picks.
 // Nobody waits for anybody, and two that see all numbers at once do the same and write the same.  (Numbers of an
 // earlier launch are gone: the pick writes the whole state.  Memory that happens to hold the number spoils the
-// sample and no more, see sampled_key.)  As two launches (three with the clearing kernel of the large
-// buckets) before -> after, us: step of 261 K 36.0 -> 34.4, 4 M 77.5 -> 74.3, 40 M 429 -> 419; select of 3 M 68.5 -> 60.8.
+// sample and no more, see sampled_key.)  As two launches (three with the clearing kernel of the large buckets)
+// before -> after, with the bin edges below, selects in a row at 1 %, us: 261 K 28.1 -> 26.1, 3 M 41.0 -> 36.3, 20 M
+// 60.4 -> 51.8, 100 M 122 -> 114.
 //
 // The pick: one LDS histogram of the top 13 bits of all keys.  The ends of the bins that the two ends of the
 // bracket fall into will do, rounded outwards, as long as that takes in no more than a quarter of the bracket's
-// own ranks in addition and no bin between them holds a third of those ranks; otherwise (narrow distributions,
-// plateaus) the next 12 bits of the keys in the two bins go into a histogram each, and what is left in a bin then is
-// ranked by counting, or split by the last 6 bits.  A plateau that holds both ends shrinks the bracket to its one key
-// that way, whose members nobody lists.  Selects with a plateau of f times k keys around the k-th (1 %), bin edges
-// without a look at the bins between / with: 8.4 M f = 0.9 226 / 81 us, 20 M f = 1.6 315 / 156, 100 M f = 0.6
-// 980 / 518; without plateaus both alike, and key ends everywhere cost 3 us more (8 at 10 % of a large bucket).
+// own ranks in addition and no bin between them stands out: a third of those ranks, and more than both its
+// neighbours.  Otherwise (narrow distributions, plateaus) the next 12 bits of the keys in the two bins go into a
+// histogram each, and what is left in a bin then is ranked by counting, or split by the last 6 bits.  A plateau that
+// holds both ends shrinks the bracket to its one key that way, whose members nobody lists.  Selects at 1 % with a
+// plateau of f times k keys around the k-th, bin edges without a look at the bins between / with: 8.4 M f = 0.9
+// 226 / 81 us, 20 M f = 1.6 315 / 156, 100 M f = 0.6 980 / 518; without plateaus the look costs 0.3, and key ends
+// everywhere cost 3 more (8 at 10 % of a large bucket).
 // kBracketSigmas etc.: the small buckets bracket the k-th key of the data this way.  The large ones
 // (coarse) bracket the ends of the bracket that their fine sample (J.n_sv quads) will give, with eight
 // sigma of the coarse sample to either side: k_sample_fine then only looks at the keys in between.  Sigma
@@ -965,7 +967,7 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // the directories of the segment tables (dirs.j[job].dir null: none wanted).
 constexpr int kSampleGroups = 16;
 constexpr int kPickBits = 13, kPickShift = 31 - kPickBits;
-constexpr uint32_t kHeavyBin = 3;                    // a half misses the 100 M case above, a quarter measured the same
+constexpr uint32_t kHeavyBin = 3;                    // a half misses the 100 M case above
 template <class Src, bool COARSE>
 __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
                                                        uint32_t launch, double sigmas) {
@@ -979,7 +981,7 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
   }
   __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
   __shared__ __align__(16) uint32_t s_list[2][kWideList];
-  __shared__ uint32_t s_cnt[2], s_out[2][3], s_all;
+  __shared__ uint32_t s_cnt[2], s_out[2][3], s_all, s_heavy;
   __shared__ WideScratch s_scan;
   static_assert(1 << kPickBits == 2 * kBinsBig, "the two small histograms are the first one");
   SelState* st = J.st;
@@ -1005,6 +1007,7 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
   reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
   reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
   if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) s_heavy = 0u;
   wait_landed();
   if (wave_id() == 0) {
     if (lane_id() == 0) st_agent(&st->sampled[blockIdx.x], launch);
@@ -1057,19 +1060,25 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
     each([&](uint32_t kk, bool live) { if (live) atomicAdd(&s_h[0][kk >> kPickShift], 1u); });
     __syncthreads();
     RankHit hit[2];
-    wide_find_rank<2, 2 * kBinsBig>(s_h[0], rank, s_scan, 0, hit);
+    const uint32_t held = rank[1] - rank[0];
+    wide_find_rank<2, 2 * kBinsBig>(s_h[0], rank, s_scan, 0, hit, [&](uint32_t above, uint32_t mine, const auto& h) {
+      if (kHeavyBin * mine <= held || above >= rank[1] || above + mine < rank[0]) return;
+      constexpr int PER = 2 * kBinsBig / kWide, LAST = 2 * kBinsBig - 1;
+#pragma unroll
+      for (int j = PER - 1; j >= 0; --j) {
+        if (kHeavyBin * h[j] > held && above < rank[1] && above + h[j] >= rank[0]) {
+          const int b = threadIdx.x * PER + j;
+          if (h[j] > (b > 0 ? s_h[0][b - 1] : 0u) + (b < LAST ? s_h[0][b + 1] : 0u)) s_heavy = 1u;
+        }
+        above += h[j];
+      }
+    });
     uint32_t bin[2] = {hit[0].bin, hit[1].bin};
     uint32_t rk[2] = {rank[0] - hit[0].above, rank[1] - hit[1].above};
     uint32_t cnt[2] = {hit[0].count, hit[1].count};
     int w = kPickShift, turn = 1;                      // bits of a key below the bins found so far
-    const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]), held = rank[1] - rank[0];
-    bool heavy = false;
-#pragma unroll
-    for (int j = 0; j < 2 * kBinsBig / kWide; ++j) {
-      const uint32_t b = (uint32_t)j * kWide + threadIdx.x;
-      heavy = heavy || (b >= bin[1] && b <= bin[0] && kHeavyBin * s_h[0][b] > held);
-    }
-    if (!__syncthreads_or(heavy) && 4u * more <= held) {
+    const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]);
+    if (!s_heavy && 4u * more <= held) {
       if (!open_hi) t_hi = (bin[0] + 1u) << w;
       if (!open_lo) t_lo = bin[1] << w;
     } else {

@@ -47,10 +47,11 @@ __device__ __forceinline__ void wide_totals(uint32_t a, uint32_t b, WideScratch&
 
 struct RankHit { uint32_t bin, above, count; };
 // The bins of an LDS histogram where the count from the top reaches each of NR ranks
-// (1-based).  All threads get the answers.  Two barriers, after the one that completes the histogram.
-template <int NR, int BINS = kWideBins>
+// (1-based).  All threads get the answers.  Two barriers, after the one that completes the histogram; look(keys
+// above, keys in, counts of the calling thread's bins) runs before the second.
+template <int NR, int BINS = kWideBins, class L>
 __device__ __forceinline__ void wide_find_rank(const uint32_t* s_hist, const uint32_t (&rank)[NR],
-                                               WideScratch& s, int turn, RankHit (&hit)[NR]) {
+                                               WideScratch& s, int turn, RankHit (&hit)[NR], L&& look) {
   constexpr int PER = BINS / kWide;                // 4 or 8
   static_assert(PER % 4 == 0, "whole quads of bins per thread");
   uint32_t h[PER], mine = 0;
@@ -77,9 +78,15 @@ __device__ __forceinline__ void wide_find_rank(const uint32_t* s_hist, const uin
       }
     }
   }
+  look(total - before - mine, mine, h);
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < NR; ++r) hit[r] = RankHit{s.hit[turn][r][0], s.hit[turn][r][1], s.hit[turn][r][2]};
+}
+template <int NR>
+__device__ __forceinline__ void wide_find_rank(const uint32_t* s_hist, const uint32_t (&rank)[NR],
+                                               WideScratch& s, int turn, RankHit (&hit)[NR]) {
+  wide_find_rank<NR, kWideBins>(s_hist, rank, s, turn, hit, [](uint32_t, uint32_t, const auto&) {});
 }
 
 // Short list of keys in LDS (what one histogram bin holds): `rank` (1-based, from the top) by counting.
