@@ -58,11 +58,11 @@ __device__ __forceinline__ void load_gd(const void* g, int64_t i, int64_t n, flo
 // The changing columns of a segment table (learning rates, bias corrections) on their way into a step's first
 // kernel, which writes them into the device tables as a side job: a launch of its own for that was 4.7 us of a
 // step, and nothing in the kernel reads the tables.  Tensors share their values (parameter groups), so a row
-// holds the number of one of up to 16 triples: 0.7 KB of kernel arguments instead of 16 bytes a row.  More
-// tensors or triples than fit take sga_segments_refresh.  Sixteen steps of 1.5 M coordinates, dense pass and two
-// configs, before -> after: 2014 -> 1992 us, 2030 -> 1978 on a new state (with the sum of the dense step written to
-// host memory by its fold, instead of copied there).
-constexpr int kNowRows = 384, kNowSets = 16;
+// holds the number of one of up to 16 triples: a byte of kernel arguments instead of 16.  2048 rows are half of the
+// 4 KB that arguments may have, with room for the kernels' own; more tensors or triples take sga_segments_refresh.
+// Sixteen steps of 1.5 M coordinates, refresh / arguments: two configs' steps on 385 tensors 709 / 576 us, on 1500
+// 1607 / 1146, dense steps 1134 / 1064 and 3193 / 2563; on 10 and 300 tensors 2 KB of rows run like 0.4.
+constexpr int kNowRows = 2048, kNowSets = 16;
 struct SegNow {
   sga_segment* segs;
   sga_replay_segment* rsegs;
@@ -71,6 +71,7 @@ struct SegNow {
   float bc1[kNowSets], bc2[kNowSets];
   uint8_t of[kNowRows];
 };
+static_assert(sizeof(SegNow) <= 2048 + 512, "travels beside a kernel's own arguments in 4 KB");
 static bool seg_now_fill(SegNow* t, sga_segment* segs, sga_replay_segment* rsegs, int n, const double* lr,
                          const float* bc1, const float* bc2) {
   t->segs = segs; t->rsegs = rsegs; t->count = 0;

@@ -28,7 +28,7 @@ def _state(n, dev=None):
 # one tensor; boundaries at, before and behind the ends of quads, slabs and workgroups; more tensors
 # than a wave has lanes; more than travel in a step's arguments
 _SIZES = [[1], [255], [256, 1], [1, 2, 3, 250, 256, 511, 1, 1], [1023, 1025, 3], [7] * 65 + [4000],
-          [3] * 384, [3] * 385 + [5000]]
+          [3] * 384, [3] * 385 + [5000], [1] * 2048, [2] * 2049]
 
 
 @pytest.mark.parametrize("groups", [1, 3, 17])
@@ -61,10 +61,11 @@ def test_dense_steps_bit_for_bit(dev, sizes, optimizer, bf16, groups):
         assert same_bits(got, want)
 
 
-@pytest.mark.parametrize("rows,sets", [(1, 1), (2, 2), (64, 16), (300, 3), (384, 16), (384, 17), (385, 1), (700, 700)])
+@pytest.mark.parametrize("rows,sets", [(1, 1), (2, 2), (64, 16), (300, 3), (384, 16), (384, 17), (385, 1), (700, 700),
+                                       (2048, 16), (2048, 17), (2049, 16)])
 def test_first_kernel_writes_the_tables(dev, rows, sets):
     """Every row gets what the launch of its own gave it, on either side of what travels
-    in a step's arguments (384 rows, 16 different triples)."""
+    in a step's arguments (2048 rows, 16 different triples)."""
     from sga_amd import _lib as L
     from sga_amd.replay_dense import DenseReplay
     from sga_amd.replay_group import Config, ReplayGroup
