@@ -82,3 +82,47 @@ def test_fused_steps_on_dirty_workspaces(dev, n, score, how):
     for end in ends[1:]:
         for a, b in zip(ends[0], end):
             assert torch.equal(a, b) if a.dtype != torch.float32 else same_bits(a, b)
+
+
+@pytest.mark.parametrize("n", _SIZES[2:])
+def test_recorded_selects_and_steps(dev, n):
+    """A graph repeats its launches' numbers on the same workspace; eager calls and anything
+    else may write there between two replays."""
+    from sga_amd import _lib as L
+    from sga_amd.fused_step import FusedSparseStep
+    k = n // 100
+    segs = [dict(start=0, n=n, lr=1e-4, b1=0.9, b2=0.95, eps=1e-8, wd=0.1)]
+    ws = torch.zeros(int(L.raw("sga_select_workspace_bytes", n)), dtype=torch.uint8, device=dev)
+    score, mask = torch.zeros(n, device=dev), torch.empty(n, dtype=torch.uint8, device=dev)
+    res = torch.empty(8, dtype=torch.int32, device=dev)
+    fs, ref = (FusedSparseStep(n, segs, dev, values_dtype=torch.float32, max_k=k) for _ in range(2))
+    g = torch.zeros(n, device=dev)
+    p = (torch.randn(n, generator=torch.Generator().manual_seed(n)) * 0.02).to(dev)
+    cur, want = ([torch.zeros_like(p), p.clone(), torch.zeros_like(p), torch.zeros_like(p)] for _ in range(2))
+
+    def work(steps, state):
+        L.call("sga_select_topk", L.ptr(score), n, k, L.TIE_LOWEST_INDEX, L.ptr(mask), L.ptr(res), L.ptr(ws), ws.numel(),
+               L.stream())
+        return steps.step(g, *state, 1, k=k)
+    score.copy_(student_t(n, 1).abs())
+    g.copy_(student_t(n, 2))
+    work(fs, [t.clone() for t in cur])                    # every kernel is loaded once
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        idx, values = work(fs, cur)
+    for turn in range(4):
+        sc = student_t(n, 10 + turn).abs()
+        score.copy_(sc)
+        g.copy_(student_t(n, 20 + turn))
+        if turn >= 2:
+            _dirty(ws, _FILLS[turn], turn)
+            _dirty(fs.ws, _FILLS[turn], turn)
+        graph.replay()
+        torch.cuda.synchronize()
+        expect, _ = SEL.select_topk_flat(sc, k)
+        assert torch.equal(mask.cpu().bool(), expect), turn
+        mask.zero_()
+        i2, v2 = work(ref, want)                          # eager, on the same select workspace
+        assert torch.equal(mask.cpu().bool(), expect) and torch.equal(idx, i2) and same_bits(values, v2), turn
+        assert all(same_bits(a, b) for a, b in zip(cur, want)), turn

@@ -350,3 +350,26 @@ def test_lengths_at_slab_and_chunk_edges(dev, n, score):
     if left:
         sizes.append(left)
     _run(dev, sizes, 1, 1.0, torch.bfloat16, torch.bfloat16, score=score, vary=True)
+
+
+# small buckets in a batch whose largest has more than 2048 chunks: their sweeps take its four chunks a workgroup
+@pytest.mark.parametrize("score", ["abs_g", "update"])
+def test_small_buckets_beside_a_four_chunk_sweep(dev, score):
+    from sga_amd.fused_step import FusedSparseStep, fused_step_multi
+    bk = []
+    for b, sizes in enumerate([[999], [3000, 1097], [1_200_000, 7, 1_000_001], [17], [5119]]):
+        segs, n = _segments(sizes, vary=True)
+        p = torch.randn(n, generator=torch.Generator().manual_seed(b)) * 0.02
+        bk.append((segs, n, [torch.zeros(n), p, torch.zeros(n), torch.zeros(n)], student_t(n, b),
+                   FusedSparseStep(n, segs, dev, values_dtype=torch.float32, want_mask=True)))
+    state = [[t.to(dev) for t in host] for _, _, host, _, _ in bk]
+    ks = [max(1, n // 20) for _, n, *_ in bk]
+    outs = fused_step_multi([x[4] for x in bk], [x[3].to(dev) for x in bk], *map(list, zip(*state)), 1, ks=ks, score=score)
+    for (segs, n, host, g, fs), devs, k, (idx, vals) in zip(bk, state, ks, outs):
+        idx_ref, val_ref, mask_ref, th_ref = OF.fused_sparse_step(g, *host, segs, 1, k=k, score=score,
+                                                                  values_dtype=torch.float32)
+        res = fs.read_result()
+        assert res.status == 0 and res.n_selected == k and res.thresh == th_ref, n
+        assert torch.equal(idx.cpu(), idx_ref) and same_bits(vals, val_ref), n
+        assert torch.equal(fs.mask.cpu().bool(), mask_ref), n
+        assert all(same_bits(d, h) for d, h in zip(devs, host)), n
