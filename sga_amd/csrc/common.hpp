@@ -63,9 +63,10 @@ static inline unsigned stream_grid(int64_t n_items, int64_t items_per_block,
 
 // Workgroup ids are dealt round-robin over the 8 XCDs.  For a grid that walks
 // library-owned packed records this permutation of [0, nb) hands every XCD one
-// contiguous eighth of the range instead (measured: 2.4 % faster on the final
-// sweep's stream mix over 64 KiB records, 3 % slower on four flat arrays, so
-// only the packed layouts use it).  The tail beyond a multiple of 8 keeps its id.
+// contiguous eighth of the range instead.  k_fused_spec and replay pass 3, with a wave
+// per chunk, take it on packed records (measured: 2.4 % faster over 64 KiB records, 3 %
+// slower on four flat arrays); k_fused_final, with a wave per slab, takes plain ids
+// (3 to 5 % faster).  The tail beyond a multiple of 8 keeps its id.
 __device__ __forceinline__ unsigned xcd_contiguous_block(unsigned b, unsigned nb) {
   const unsigned per = nb >> 3;
   return b < (per << 3) ? (b & 7u) * per + (b >> 3) : b;

@@ -375,10 +375,11 @@ __global__ __launch_bounds__(kBlock) void k_fused_final_redo(FinalArgs a, const 
 }
 
 // Up to this many bytes the select's sweep loads by ordinary accesses, which leave its inputs in the 256 MB
-// memory-side cache for the final sweep to find; non-temporal ones do not, but a longer sweep runs faster by
-// them and little of it would survive.  Step, without -> with: |g + r| 10 M coordinates (60 MB) 141 -> 137 us,
-// 40 M 349 -> 328, 63 M (378 MB) 516 -> 491, 150 M (900 MB) 1158 -> 1145; `update` 20 M (360 MB) 276 -> 274,
-// 40 M (720 MB) 453 -> 459, 63 M 660 -> 683, 100 M 992 -> 1036.
+// memory-side cache for the final sweep to find; non-temporal ones do not, but little of a longer sweep survives.
+// The line lies where `update` begins to lose by ordinary ones; |g + r| still gains a percent at 900 MB.  Step,
+// without -> with: |g + r| 10 M coordinates (60 MB) 141 -> 137 us, 40 M 349 -> 328, 63 M (378 MB) 516 -> 491,
+// 150 M (900 MB) 1158 -> 1145; `update` 20 M (360 MB) 276 -> 274, 40 M (720 MB) 453 -> 459, 63 M 660 -> 683,
+// 100 M 992 -> 1036.
 constexpr int64_t kKeepBytes = 512ll << 20;
 
 // One bucket of a (possibly batched) fused step.

@@ -8,15 +8,16 @@
 // followed by the caller's writing pass (final sweep, k_write_mask, k_write_bits), which forms the
 // keys again: the whole bucket sits in L2 / Infinity Cache then.
 //
-// Why not the chain of the large buckets (select_impl.hpp): that is seven dependent
-// launches beside the sweeps (twenty, 150 us, when this path was written) and half-empty grids,
+// Why not the chain of the large buckets (select_impl.hpp): that is five dependent
+// launches beside the sweep (twenty, 150 us, when this path was written) and half-empty grids,
 // where the data of a 4 M-element bucket takes 24 us.  One workgroup is enough for what lies
 // between the sweeps as long as the chunk counts fit its LDS, which draws the line at kSmallTiles
 // (8 M coordinates at 1 %: 30 us in k_small_finish, as much as the sweep and a half).
 // Measured through the public entry points, us per call, before -> with this path:
 //   fused step, |g + r|, 1 %, 261 K elements bf16   84 -> 55       4.2 M elements fp32   184 -> 91
 //   select_topk_flat, 3 M scores, 1 %              168 -> 69
-// (4.2 M: sample and pick 8, sweep 6, finish 15, final sweep 28 us).
+// (Kernels of the 4.2 M step, fp32 gradients, each pass after a wait: sample and pick 12.5 us, sweep 11.4, finish
+// 20.6, final sweep 27.2.)
 //
 // The result is exact for any sample: where the bracket misses the k-th key the finishing launch goes
 // over the data itself, with all of its workgroups (small_redo).
@@ -346,7 +347,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   // A list far longer than its margin says holds a plateau that one workgroup should not walk (keys equal
   // to the upper end are listed): two values, k near where they change, 8.4 M coordinates: half of them
   // on the upper one 5.7 ms, a tenth 1.06; by passes over the data 0.29 and 0.32.  Independent scores list
-  // 1.0 times what the margin says.
+  // 1.0 to 1.25 times what the margin says (the bracket ends at bin edges).
   bool crowded = false;
   if (n_list > kCrowdedList) {
     const double ns = (double)(small_sample_vecs(n) * 4);
