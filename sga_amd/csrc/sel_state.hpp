@@ -57,7 +57,8 @@ static_assert(sizeof(SelState) == 256, "whole cache lines");
 // to hold the launch's number let a workgroup pick from keys that have not arrived, or several workgroups from
 // different ones.  So the pick is made for any words: what is read as a key is one (31 bits: it indexes a
 // histogram in LDS), and the two ends of the bracket are written as one word, so that they are always one
-// picking workgroup's own.  The select is exact for any bracket.
+// picking workgroup's own.  The select is exact for any bracket; a single-sweep step in place, which commits on
+// it, reports a miss like any other (status 3).
 SGA_HOST_DEVICE static inline uint32_t sampled_key(unsigned long long word, int half) {
   return (uint32_t)(word >> (32 * half)) & 0x7FFFFFFFu;
 }
