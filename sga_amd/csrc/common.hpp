@@ -202,6 +202,10 @@ __device__ __forceinline__ F4 ld4(const float* p) {
 __device__ __forceinline__ void st4(float* p, const F4& v) {
   *reinterpret_cast<f4v*>(p) = f4v{v.x, v.y, v.z, v.w};
 }
+typedef unsigned int u4v __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void st4_u32(uint32_t* p, const U4& v) {
+  *reinterpret_cast<u4v*>(p) = u4v{v.x, v.y, v.z, v.w};
+}
 __device__ __forceinline__ B4 ldb4(const uint8_t* p) {
   const b4v t = *reinterpret_cast<const b4v*>(p);
   return B4{t.x, t.y, t.z, t.w};

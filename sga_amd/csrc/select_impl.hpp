@@ -950,8 +950,11 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // The pick: one LDS histogram of the top 13 bits of all keys.  The ends of the bins that the two ends of the
 // bracket fall into will do, rounded outwards, as long as that takes in no more than a quarter of the bracket's
 // own ranks in addition and no bin between them stands out: a third of those ranks, and more than both its
-// neighbours.  Otherwise (narrow distributions, plateaus) the next 12 bits of the keys in the two bins go into a
-// histogram each, and what is left in a bin then is ranked by counting, or split by the last 6 bits.  A plateau that
+// neighbours.  Where they take in more (about 10 % of heavy-tailed scores, where a bin is a fifth of the bracket), the
+// two bins are split in 64 by their next six bits, a wave each, and the ends of those parts will do by the same rule
+// (selects at 10 %, key ends / ends of parts, us: 1 M scores 40.5 / 36.4, 3 M 55.4 / 48.8, 8 M 96.3 / 90.1).
+// Otherwise (plateaus) the next 12 bits of the keys in the two bins go into a histogram each, and what is left in a
+// bin then is ranked by counting, or split by the last 6 bits.  A plateau that
 // holds both ends shrinks the bracket to its one key that way, whose members nobody lists.  Selects at 1 % with a
 // plateau of f times k keys around the k-th, bin edges without a look at the bins between / with: 8.4 M f = 0.9
 // 226 / 81 us, 20 M f = 1.6 315 / 156, 100 M f = 0.6 980 / 518; without plateaus the look costs 0.3, and key ends
@@ -981,7 +984,7 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
   }
   __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
   __shared__ __align__(16) uint32_t s_list[2][kWideList];
-  __shared__ uint32_t s_cnt[2], s_out[2][3], s_all, s_heavy;
+  __shared__ uint32_t s_cnt[2], s_out[2][3], s_all, s_heavy, s_rank[2], s_open[2], s_sub[2][kWave];
   __shared__ WideScratch s_scan;
   static_assert(1 << kPickBits == 2 * kBinsBig, "the two small histograms are the first one");
   SelState* st = J.st;
@@ -1003,9 +1006,33 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
                            __HIP_MEMORY_SCOPE_AGENT);
     }
   }
+  const uint32_t ns = (uint32_t)(n_sv * 4);
+  if (wave_id() == kWideWaves - 1) {                 // takes no sample; double precision, 0.7 us that nobody waits for
+    double rh, rl;
+    if (COARSE) {
+      const double nf = (double)(J.n_sv * 4), to = (double)ns / nf;
+      const RankEnds f = bracket_ranks((double)J.k, (double)n, nf, sigmas);
+      const double ah = f.hi * to, al = f.lo * to;
+      const double m = (double)ns;
+      rh = floor(ah - (8.0 * sqrt(fmax(ah * (1.0 - ah / m), 0.0) + 1.0) + 4.0));
+      rl = ceil(al + (8.0 * sqrt(fmax(al * (1.0 - al / m), 0.0) + 1.0) + 4.0));
+    } else {
+      const RankEnds f = bracket_ranks((double)J.k, (double)n, (double)ns, sigmas);
+      rh = f.hi;
+      rl = f.lo;
+    }
+    const bool up = rh < 1.0 || ns == 0, down = rl > (double)ns || ns == 0;
+    if (lane_id() == 0) {
+      s_open[0] = up;
+      s_open[1] = down;
+      s_rank[0] = up ? 1u : (uint32_t)rh;
+      s_rank[1] = down ? ns : (uint32_t)rl;
+    }
+  }
   const U4 zero{0u, 0u, 0u, 0u};
   reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
   reinterpret_cast<U4*>(s_h[1])[threadIdx.x] = zero;
+  if (threadIdx.x < 2 * kWave) s_sub[threadIdx.x / kWave][threadIdx.x % kWave] = 0u;
   if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0u;
   if (threadIdx.x == 0) s_heavy = 0u;
   wait_landed();
@@ -1030,22 +1057,8 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
       key[u][2 * h + 1] = sampled_key(q, 1);
     }
   }
-  const uint32_t ns = (uint32_t)(n_sv * 4);
-  double rh, rl;
-  if (COARSE) {
-    const double nf = (double)(J.n_sv * 4), to = (double)ns / nf;
-    const RankEnds f = bracket_ranks((double)J.k, (double)n, nf, sigmas);
-    const double ah = f.hi * to, al = f.lo * to;
-    const double m = (double)ns;
-    rh = floor(ah - (8.0 * sqrt(fmax(ah * (1.0 - ah / m), 0.0) + 1.0) + 4.0));
-    rl = ceil(al + (8.0 * sqrt(fmax(al * (1.0 - al / m), 0.0) + 1.0) + 4.0));
-  } else {
-    const RankEnds f = bracket_ranks((double)J.k, (double)n, (double)ns, sigmas);
-    rh = f.hi;
-    rl = f.lo;
-  }
-  const bool open_hi = rh < 1.0 || ns == 0, open_lo = rl > (double)ns || ns == 0;
-  const uint32_t rank[2] = {open_hi ? 1u : (uint32_t)rh, open_lo ? ns : (uint32_t)rl};
+  const bool open_hi = s_open[0] != 0u, open_lo = s_open[1] != 0u;
+  const uint32_t rank[2] = {s_rank[0], s_rank[1]};
   uint32_t t_hi = 0x80000000u, t_lo = 0u;
   if (ns) {
     auto each = [&](auto&& f) {
@@ -1078,10 +1091,37 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
     uint32_t cnt[2] = {hit[0].count, hit[1].count};
     int w = kPickShift, turn = 1;                      // bits of a key below the bins found so far
     const uint32_t more = (open_hi ? 0u : rk[0] - 1u) + (open_lo ? 0u : cnt[1] - rk[1]);
+    bool ends = false;
     if (!s_heavy && 4u * more <= held) {
+      ends = true;
       if (!open_hi) t_hi = (bin[0] + 1u) << w;
       if (!open_lo) t_lo = bin[1] << w;
-    } else {
+    } else if (!s_heavy) {
+      constexpr int kSub = 6, SH = kPickShift - kSub;
+      static_assert(1 << kSub == kWave, "a bin's part per lane");
+      each([&](uint32_t kk, bool live) {
+        const uint32_t top = kk >> kPickShift, part = (kk >> SH) & (kWave - 1);
+        if (live && top == bin[0]) atomicAdd(&s_sub[0][part], 1u);
+        if (live && top == bin[1]) atomicAdd(&s_sub[1][part], 1u);
+      });
+      __syncthreads();
+      if (wave_id() < 2) {
+        const int q = wave_id(), l = lane_id();
+        const uint32_t c = s_sub[q][kWave - 1 - l], incl = wave_incl_scan(c);              // from the top
+        const uint32_t near = (l > 0 ? s_sub[q][kWave - l] : 0u) + (l < kWave - 1 ? s_sub[q][kWave - 2 - l] : 0u);
+        const bool one_bin = bin[0] == bin[1];
+        const bool between = (q == 1 && !one_bin ? true : incl >= rk[0]) && (q == 0 && !one_bin ? true : incl - c < rk[1]);
+        if (between && kHeavyBin * c > held && c > near) s_heavy = 1u;
+        const int at = __ffsll((unsigned long long)ballot64(incl >= rk[q])) - 1;
+        if (l == at) { s_out[q][0] = (uint32_t)(kWave - 1 - l); s_out[q][1] = incl - c; s_out[q][2] = c; }
+      }
+      __syncthreads();
+      const uint32_t beyond = (open_hi ? 0u : rk[0] - s_out[0][1] - 1u) + (open_lo ? 0u : s_out[1][2] - (rk[1] - s_out[1][1]));
+      ends = !s_heavy && 4u * beyond <= held;
+      if (ends && !open_hi) t_hi = ((bin[0] << kSub | s_out[0][0]) + 1u) << SH;
+      if (ends && !open_lo) t_lo = (bin[1] << kSub | s_out[1][0]) << SH;
+    }
+    if (!ends) {
       while (w > 0 && (cnt[0] > (uint32_t)kWideList || cnt[1] > (uint32_t)kWideList)) {
         const int sh = w > 12 ? w - 12 : 0, bits = w - sh;
         reinterpret_cast<U4*>(s_h[0])[threadIdx.x] = zero;
@@ -1952,9 +1992,9 @@ __global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJ
 // The items of the scan wait for one another's totals the same way (in ticket order), through 64-bit
 // words that carry the totals themselves.  All else that crosses workgroups goes by device-scope accesses,
 // waited for before an item counts as finished: a cache-wide fence costs 240 ns an item, one after the other
-// (the 256 tie items behind a scan, with a fence each: this launch took 59 to 72 us, 32 without, on 74.5 M coordinates of bf16
-// gradients without a residual, where 10 to 20 thousand keys equal the threshold).  The waiting ones look at a word
-// of its own, away from the counter that they add to.
+// (the 256 tie items behind a scan, with a fence each: this launch took 59 to 72 us, 32 without, on 74.5 M
+// coordinates of bf16 gradients without a residual, where 10 to 20 thousand keys equal the threshold).  The waiting
+// ones look at a word of its own, away from the counter that they add to.
 constexpr int kTailBlocks = 512;
 constexpr int kTailStep = kHistStride + 2 * kMaxTileBlocks + 256;    // that word, in the second histogram set
 struct TailLds {
