@@ -924,8 +924,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     per_score([&](auto& srcs, const SelBatch& sub) {
       launch_sample_pick<true>(srcs, sub, dirs_of(srcs, sub), kBracketSigmas, s);
     });
-    per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, s); });
-    chain_pick_fine(B, kBracketSigmas, s);
+    per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, kBracketSigmas, s); });
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, s); });
     chain_settle(B, s);
   }

@@ -1170,10 +1170,17 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
 }
 
 // The fine sample of a large bucket: only how its keys fall relative to the coarse bracket is kept --
-// counts above it, and a histogram of the few inside.
+// counts above it, and a histogram of the few inside.  The last workgroup to finish takes the bracket from it, at the
+// edges of the histogram's bins (rounded outwards: a few sample keys wide); an end the coarse bracket missed is left
+// open.  The tickets go by sixteen words and one: on one word they queue, 11 ns each (1024 workgroups: 8 us of a select
+// of 300 M scores), and four quads a thread by a quarter of the workgroups made the sample of `update` 12 us longer.  The pick as a launch of its own -> here, selects
+// in a row at 1 %, us: 9 M scores 43.0 -> 41.1, 20 M 53.9 -> 52.5, 40 M 69.7 -> 68.7, 100 M and more the same.
+// What the pick reads of the others' are device-scope atomics, which every wave waits for before its workgroup
+// takes its ticket; the ticket is a word of the state that the kernel before has written.
+constexpr int kFineSpread = kRelSpread;                // tickets: a word for every sixteenth workgroup, then one for those
 template <class Src>
-__global__ __launch_bounds__(kBlock) void k_sample_fine(SrcPack<Src> srcs, ChainJobs jobs) {
-  __shared__ uint32_t s_w[kChunksPerBlock];
+__global__ __launch_bounds__(kBlock) void k_sample_fine(SrcPack<Src> srcs, ChainJobs jobs, double sigmas) {
+  __shared__ uint32_t s_w[kChunksPerBlock], s_last, s_hit[2][3], s_bins[kWideBins + kBlock];
   const ChainJob& J = jobs.j[blockIdx.y];
   const int64_t j = (int64_t)blockIdx.x * kBlock + threadIdx.x;
   if ((int64_t)blockIdx.x * kBlock >= J.n_sv) return;                 // a smaller job of the batch
@@ -1205,37 +1212,64 @@ __global__ __launch_bounds__(kBlock) void k_sample_fine(SrcPack<Src> srcs, Chain
     const uint32_t all = s_w[0] + s_w[1] + s_w[2] + s_w[3];
     if (all) atomicAdd(&J.rel[kRelAbove + (blockIdx.x % kRelSpread) * 64], all);
   }
-}
-
-// The bracket from the fine sample, at the edges of its histogram's bins (rounded outwards: a few sample
-// keys wide).  An end the coarse bracket missed is left open.
-static __global__ __launch_bounds__(kWide) void k_pick_fine(ChainJobs jobs, double sigmas) {
-  __shared__ WideScratch s_scan;
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const uint32_t c_lo = J.st->t_lo, c_hi = J.st->t_hi;
-  const int sh = rel_shift(c_lo, c_hi, kWideBins);
-  const uint32_t* bins = J.rel + kRelSample;
-  uint32_t above = 0;
-  for (int i = 0; i < kRelSpread; ++i) above += J.rel[kRelAbove + i * 64];
-  const U4 q = reinterpret_cast<const U4*>(bins)[threadIdx.x];
-  uint32_t inside;
-  wide_prefix(q.x + q.y + q.z + q.w, s_scan, 1, inside);
+  wait_landed();
+  if (threadIdx.x == 0) {
+    const uint32_t groups = (uint32_t)cdiv64(J.n_sv, kBlock), w = blockIdx.x % kFineSpread;
+    const uint32_t words = groups < (uint32_t)kFineSpread ? groups : (uint32_t)kFineSpread;
+    const bool filled = atomicAdd(&J.rel[kRelAbove + w * 64 + 32], 1u) == (groups - w + kFineSpread - 1) / kFineSpread - 1;
+    s_last = filled && atomicAdd(&J.st->ticket, 1u) == words - 1u;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  constexpr int PER = kWideBins / kBlock;
+  const uint32_t part = threadIdx.x < kRelSpread ? ld_agent(&J.rel[kRelAbove + threadIdx.x * 64]) : 0u;
+  uint32_t h[PER], mine = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) h[i] = ld_agent(&bins[i * kBlock + threadIdx.x]);
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int at = i * kBlock + (int)threadIdx.x;
+    s_bins[at + at / PER] = h[i];                                     // a word between the threads' runs
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i) { h[i] = s_bins[threadIdx.x * (PER + 1) + i]; mine += h[i]; }
+  uint32_t total, inside;
+  const uint32_t before = block_excl_scan(mine, s_w, inside);
+  __syncthreads();
+  block_excl_scan(part, s_w, total);
   const double ns = (double)(J.n_sv * 4);
   const RankEnds f = bracket_ranks((double)J.k, (double)J.n, ns, sigmas);
-  const bool in_hi = f.hi >= 1.0 && f.hi > (double)above && f.hi <= (double)above + (double)inside;
-  const bool in_lo = f.lo <= ns && f.lo > (double)above && f.lo <= (double)above + (double)inside;
-  const uint32_t rank[2] = {in_hi ? (uint32_t)f.hi - above : 1u, in_lo ? (uint32_t)f.lo - above : 1u};
-  RankHit hit[2] = {};
-  if (inside) wide_find_rank<2>(bins, rank, s_scan, 0, hit);
+  const bool in_hi = f.hi >= 1.0 && f.hi > (double)total && f.hi <= (double)total + (double)inside;
+  const bool in_lo = f.lo <= ns && f.lo > (double)total && f.lo <= (double)total + (double)inside;
+  const uint32_t rank[2] = {in_hi ? (uint32_t)f.hi - total : 1u, in_lo ? (uint32_t)f.lo - total : 1u};
+  if (threadIdx.x < 2) s_hit[threadIdx.x][0] = s_hit[threadIdx.x][1] = s_hit[threadIdx.x][2] = 0u;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    uint32_t run = inside - before - mine;                            // keys in the bins above the thread's
+    if (run < rank[q] && rank[q] <= run + mine) {
+#pragma unroll
+      for (int i = PER - 1; i >= 0; --i) {
+        if (run < rank[q] && rank[q] <= run + h[i]) {
+          s_hit[q][0] = (uint32_t)(threadIdx.x * PER + i);
+          s_hit[q][1] = run;
+          s_hit[q][2] = h[i];
+        }
+        run += h[i];
+      }
+    }
+  }
+  __syncthreads();
   if (threadIdx.x != 0) return;
   uint32_t t_hi = 0x80000000u, t_lo = 0u, in_sample = ~0u;
   if (in_hi) {
-    t_hi = c_lo + ((hit[0].bin + 1u) << sh);
+    t_hi = c_lo + ((s_hit[0][0] + 1u) << sh);
     if (t_hi > c_hi) t_hi = c_hi;
   }
   if (in_lo) {
-    t_lo = c_lo + (hit[1].bin << sh);
-    in_sample = above + hit[1].above + hit[1].count - (in_hi ? above + hit[0].above : 0u);
+    t_lo = c_lo + (s_hit[1][0] << sh);
+    in_sample = total + s_hit[1][1] + s_hit[1][2] - (in_hi ? total + s_hit[0][1] : 0u);
   }
   SelState z = {};
   z.k = J.k;
@@ -1997,8 +2031,9 @@ __global__ __launch_bounds__(kBlock) void k_write_bits(SrcPack<Src> srcs, ChainJ
 // ones look at a word of its own, away from the counter that they add to.
 constexpr int kTailBlocks = 512;
 constexpr int kTailStep = kHistStride + 2 * kMaxTileBlocks + 256;    // that word, in the second histogram set
+constexpr int kTailRuns = kTileScanSpan + kBlock;     // a word between the threads' runs: no bank conflicts
 struct TailLds {
-  uint32_t h[kBinsBig];
+  uint32_t h[kTailRuns];                              // a level's bins, or a scan's counters on their way
   uint32_t suf[kBlock + 1], w4[kChunksPerBlock], last, ticket;
 };
 // armed: the chunk counts come from this launch; read_on: items behind the scan read the prefixes in it.
@@ -2008,16 +2043,45 @@ __device__ __forceinline__ void tail_scan(const ChainJob& J, uint32_t b, uint32_
   unsigned long long* words = reinterpret_cast<unsigned long long*>(J.hist + kHistStride);
   static_assert(kTailStep < 2 * kHistStride && kHistStride % 2 == 0, "a word per workgroup of the scan");
   static_assert((int64_t)kTileScanSpan * kChunk < (1 << 23), "two totals and a flag in 64 bits");
-  const int64_t base = (int64_t)b * kTileScanSpan + (int64_t)threadIdx.x * kTileScanPer;
+  // counters come and go a line a wave and instruction, by LDS; a thread scans a run of sixteen.  (By runs straight
+  // from and to memory the scan of 18,190 chunks spent 4.5 us on its loads and 7.8 on its stores.)
+  const int64_t base = (int64_t)b * kTileScanSpan;
+  auto runs = [](int i) { return i + i / kTileScanPer; };
+  const int mine = (int)threadIdx.x * (kTileScanPer + 1);
   uint32_t g[kTileScanPer], e[kTileScanPer], my_g = 0, my_e = 0;
 #pragma unroll
   for (int j = 0; j < kTileScanPer; ++j) {
-    const bool ok = base + j < n_tiles;
-    g[j] = ok ? (armed ? ld_agent(&J.tile_gt[base + j]) : J.tile_gt[base + j]) : 0u;
-    e[j] = ok ? (armed ? ld_agent(&J.tile_eq[base + j]) : J.tile_eq[base + j]) : 0u;
-    my_g += g[j];
-    my_e += e[j];
+    const int64_t at = base + j * kBlock + threadIdx.x;
+    const bool ok = at < n_tiles;
+    g[j] = ok ? (armed ? ld_agent(&J.tile_gt[at]) : J.tile_gt[at]) : 0u;
+    e[j] = ok ? (armed ? ld_agent(&J.tile_eq[at]) : J.tile_eq[at]) : 0u;
   }
+  auto turn = [&](uint32_t (&v)[kTileScanPer]) {      // from a word of every line to a run
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kTileScanPer; ++j) s.h[runs(j * kBlock + (int)threadIdx.x)] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kTileScanPer; ++j) v[j] = s.h[mine + j];
+  };
+  auto put = [&](const uint32_t (&v)[kTileScanPer], uint32_t* to) {
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kTileScanPer; ++j) s.h[mine + j] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kTileScanPer; ++j) {
+      const int64_t at = base + j * kBlock + threadIdx.x;
+      const uint32_t w = s.h[runs(j * kBlock + (int)threadIdx.x)];
+      if (at >= n_tiles) continue;
+      if (read_on) st_agent(&to[at], w);
+      else to[at] = w;
+    }
+  };
+  turn(g);
+  turn(e);
+#pragma unroll
+  for (int j = 0; j < kTileScanPer; ++j) { my_g += g[j]; my_e += e[j]; }
   uint32_t tot_g, tot_e;
   uint32_t gr = block_excl_scan(my_g, s.w4, tot_g);
   uint32_t er = block_excl_scan(my_e, s.w4, tot_e);
@@ -2041,19 +2105,14 @@ __device__ __forceinline__ void tail_scan(const ChainJob& J, uint32_t b, uint32_
   const uint32_t need = J.tie_all ? 0xFFFFFFFFu : ld_agent(&J.st->need);
 #pragma unroll
   for (int j = 0; j < kTileScanPer; ++j) {
-    if (base + j < n_tiles) {
-      const uint32_t sel = gr + (er < need ? er : need);
-      if (read_on) {
-        st_agent(&J.tile_gt[base + j], sel);
-        st_agent(&J.tile_eq[base + j], er);
-      } else {
-        J.tile_gt[base + j] = sel;
-        J.tile_eq[base + j] = er;
-      }
-    }
-    gr += g[j];
-    er += e[j];
+    const uint32_t here_g = g[j], here_e = e[j];
+    g[j] = gr + (er < need ? er : need);
+    e[j] = er;
+    gr += here_g;
+    er += here_e;
   }
+  put(g, J.tile_gt);
+  put(e, J.tile_eq);
   // (a settlement that placed a mask has stored the number and kept no selected counts)
   if (b == n_blk - 1 && threadIdx.x == 0 && !(J.mask_only && J.st->bracket_ok)) {
     const uint32_t E = E0 + tot_e;
@@ -2084,7 +2143,8 @@ __global__ __launch_bounds__(kBlock) void k_tail(SrcPack<Src> srcs, ChainJobs jo
     if (blockIdx.x == 0 && threadIdx.x == 0) write_result(J);
     return;
   }
-  if (!armed && !write && !ties && blockIdx.x >= n_scan) return;      // a workgroup per item is enough
+  const bool once = !armed && !write && total <= G;                   // a workgroup per item is enough
+  if (once && blockIdx.x >= total) return;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) s.ticket = atomicAdd(&st->tail_ticket, 1u);
@@ -2094,7 +2154,7 @@ __global__ __launch_bounds__(kBlock) void k_tail(SrcPack<Src> srcs, ChainJobs jo
     const uint32_t first = t >= at_ties ? at_ties : t >= at_scan ? at_scan : t / G * G;
     if (first) {
       if (threadIdx.x == 0)
-        while (ld_agent(&J.hist[kTailStep]) < first) __builtin_amdgcn_s_sleep(16);
+        while (ld_agent(&J.hist[kTailStep]) < first) __builtin_amdgcn_s_sleep(4);
       __syncthreads();
     }
     Src src = srcs.s[blockIdx.y];
@@ -2114,13 +2174,17 @@ __global__ __launch_bounds__(kBlock) void k_tail(SrcPack<Src> srcs, ChainJobs jo
       if (OUT == 1) write_bits_body(src, J, T, need, t - first, n_write);
       else write_mask_body(src, J, T, need, 0, J.mask, t - first, n_write);
     }
-    if (t >= at_ties) continue;                                       // nothing in this launch reads what these wrote
+    if (t >= at_ties) {                                               // nothing in this launch reads what these wrote
+      if (once) return;
+      continue;
+    }
     wait_landed();
     if (threadIdx.x == 0) {
       const uint32_t done = atomicAdd(&st->tail_done, 1u) + 1u;
       if (done == at_ties) write_result(J);                           // settled with the scan's last item
       if (done == at_ties || (done <= at_scan && done % G == 0)) st_agent(&J.hist[kTailStep], done);
     }
+    if (once) return;
   }
 }
 
@@ -2154,7 +2218,7 @@ static __global__ __launch_bounds__(kBlock) void k_mask_to_planes(const uint8_t*
 //
 // The chain comes in phases so that a batch whose jobs form their keys differently (the
 // re-selections of a replay step rank by different scores) still shares every kernel that does
-// not form keys: chain_begin, chain_pick_fine and chain_settle take the whole batch; launch_sample_*,
+// not form keys: chain_begin and chain_settle take the whole batch; launch_sample_*,
 // chain_sweeps and chain_tail are templates of the key source and take the jobs of one kind (a sub-batch
 // over the same workspaces).
 static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStream_t s) {
@@ -2172,20 +2236,16 @@ static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& 
                      B.jobs, dirs, next_launch(), sigmas);
 }
 template <class Src>
-static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, hipStream_t s) {
+static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, double sigmas, hipStream_t s) {
   hipLaunchKernelGGL((k_sample_fine<Src>), B.grid((unsigned)cdiv64(B.max_nsv, kBlock)), dim3(kBlock), 0, s, srcs,
-                     B.jobs);
-}
-static inline void chain_pick_fine(const SelBatch& B, double sigmas, hipStream_t s) {
-  hipLaunchKernelGGL(k_pick_fine, B.grid(1), dim3(kWide), 0, s, B.jobs, sigmas);
+                     B.jobs, sigmas);
 }
 // begin ... bracket, for a batch of one key source
 template <class Src>
 static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
                                  hipStream_t s) {
   launch_sample_pick<true>(srcs, B, dirs, sigmas, s);
-  launch_sample_fine(srcs, B, s);
-  chain_pick_fine(B, sigmas, s);
+  launch_sample_fine(srcs, B, sigmas, s);
 }
 // keep (sources that a writing pass reads again): see bracket_chunk
 template <class Src>
