@@ -429,6 +429,37 @@ int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int n_buckets,
                                 float factor, float coeff, int fast, int flags,
                                 float interval, void* stream);
 
+/* The same steps, which first bring the changing columns of the segment tables
+ * up to date: learning rates and bias corrections, HOST arrays of n_segs rows
+ * read before the call returns (what sga_segments_refresh writes by a launch of
+ * its own).  multi: one entry per bucket, lr NULL where the table stands. */
+typedef struct sga_segment_cols {
+  const double* lr;
+  const float* bc1;
+  const float* bc2;
+} sga_segment_cols;
+int sga_fused_sparse_step_cols(const sga_segment_cols* cols, const void* g,
+                               int g_dtype, float* resid, float* p, float* m,
+                               float* v, int64_t n, int64_t k,
+                               sga_segment* segs, int n_segs, int score_id,
+                               int32_t* idx_out, void* values_out,
+                               int values_dtype, uint8_t* mask_out,
+                               float factor, float coeff, int fast, int flags,
+                               float interval, sga_select_result* result,
+                               void* ws, size_t ws_bytes, void* stream);
+int sga_fused_sparse_step_multi_cols(const sga_fused_bucket* buckets,
+                                     const sga_segment_cols* cols,
+                                     int n_buckets, int g_dtype, int score_id,
+                                     int values_dtype, float factor,
+                                     float coeff, int fast, int flags,
+                                     float interval, void* stream);
+int sga_fused_sparse_step_packed_cols(
+    const sga_segment_cols* cols, const void* g, int g_dtype, float* state,
+    int64_t n, int64_t k, sga_segment* segs, int n_segs, int score_id,
+    int32_t* idx_out, void* values_out, int values_dtype, uint8_t* mask_out,
+    float factor, float coeff, int fast, int flags, float interval,
+    sga_select_result* result, void* ws, size_t ws_bytes, void* stream);
+
 /* Single-sweep variant of the fused step (no counterpart in the reference,
  * whose engine runs score, select, pack and commit as separate passes,
  * engine.py:416-604): g, resid, p, m, v are read ONCE.  The sampled bracket

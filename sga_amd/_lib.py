@@ -38,6 +38,11 @@ class FusedBucket(C.Structure):
                 ("ws", C.c_void_p), ("ws_bytes", C.c_size_t)]
 
 
+class SegmentCols(C.Structure):
+    """struct sga_segment_cols"""
+    _fields_ = [("lr", C.c_void_p), ("bc1", C.c_void_p), ("bc2", C.c_void_p)]
+
+
 class ReselectJob(C.Structure):
     """struct sga_reselect_job"""
     _fields_ = [("res", C.c_void_p), ("w", C.c_void_p), ("m", C.c_void_p), ("v", C.c_void_p),
@@ -115,6 +120,11 @@ SIGNATURES = {
     "sga_fused_sparse_step": (I32, [P, I32, P, P, P, P, I64, I64, P, I32, I32, P, P,
                                     I32, P, F, F, I32, I32, F, P, P, SZ, P]),
     "sga_fused_sparse_step_multi": (I32, [P, I32, I32, I32, I32, F, F, I32, I32, F, P]),
+    "sga_fused_sparse_step_cols": (I32, [P, P, I32, P, P, P, P, I64, I64, P, I32, I32, P, P,
+                                         I32, P, F, F, I32, I32, F, P, P, SZ, P]),
+    "sga_fused_sparse_step_multi_cols": (I32, [P, P, I32, I32, I32, I32, F, F, I32, I32, F, P]),
+    "sga_fused_sparse_step_packed_cols": (I32, [P, P, I32, P, I64, I64, P, I32, I32, P, P,
+                                                I32, P, F, F, I32, I32, F, P, P, SZ, P]),
     "sga_packed_state_elems": (I64, [I64]),
     "sga_fused_sparse_step_packed": (I32, [P, I32, P, I64, I64, P, I32, I32, P, P,
                                            I32, P, F, F, I32, I32, F, P, P, SZ, P]),

@@ -2,6 +2,8 @@
 // op (translation units are built with -ffp-contract=off); FMAs appear only
 // where written explicitly.
 #pragma once
+#include <string.h>
+
 #include "common.hpp"
 
 namespace sga {
@@ -77,7 +79,7 @@ struct SegCursor {
   const int32_t* dir;
   int n_segs;
   int64_t lo, hi;
-  int at;                               // index of the cached segment (uniform seeks only)
+  int at;                               // index of the cached segment
   Hyper h;
   __host__ __device__ __forceinline__ void init(const sga_segment* s, int ns,
                                                 const int32_t* d = nullptr) {
@@ -99,10 +101,10 @@ struct SegCursor {
   }
   __device__ __forceinline__ void seek(int64_t i) {
     if (i >= lo && i < hi) return;
-    const int a = find(i);
-    lo = segs[a].start;
-    hi = lo + segs[a].n;
-    h = hyper_of(segs[a]);
+    at = find(i);
+    lo = segs[at].start;
+    hi = lo + segs[at].n;
+    h = hyper_of(segs[at]);
   }
   // The same for an index every lane of the wave holds alike: the cursor and
   // the hyper-parameters it caches live on the scalar unit.
@@ -172,6 +174,70 @@ static __global__ __launch_bounds__(kBlock) void k_seg_dir(const sga_segment* __
 // The tables of up to 8 jobs whose directories a batched kernel builds on the way.
 struct SegDirJobs {
   struct { const sga_segment* segs; int32_t* dir; int64_t n; int n_segs; } j[8];
+};
+// The changing columns (learning rates, bias corrections) of the tables of up to 8 jobs, on their way into the first
+// kernel of a select, which writes them into the device tables (a launch of its own: step of 261 K coordinates 31.5 us,
+// 29.6 so).
+// Tensors share their values (parameter groups): a row is the number of one of 8 triples, a byte.  480 rows fill what
+// the select's own arguments leave of 4 KB; more rows or triples take sga_segments_refresh.
+constexpr int kColRows = 480, kColSets = 8;
+struct NowCols {
+  double lr[kColSets];
+  float bc1[kColSets], bc2[kColSets];
+  uint16_t first[9];             // job j's rows are [first[j], first[j + 1]); none: its table stands
+  uint8_t of[kColRows];
+  // Adds the rows of job j (called for the jobs in order); false where they do not fit.
+  bool add(int j, int n, const double* lr_, const float* b1, const float* b2) {
+    const int base = j == 0 ? 0 : first[j];
+    first[0] = 0;
+    first[j + 1] = (uint16_t)base;
+    if (!lr_) return true;
+    if (base + n > kColRows) return false;
+    int s = 0;
+    for (int i = 0; i < n; ++i) {
+      // compared as bits: a NaN is a value like any other
+      const auto same = [&](int t) {
+        return !memcmp(&lr[t], lr_ + i, 8) && !memcmp(&bc1[t], b1 + i, 4) && !memcmp(&bc2[t], b2 + i, 4);
+      };
+      if (s >= sets || !same(s))
+        for (s = 0; s < sets && !same(s);) ++s;
+      if (s == sets) {
+        if (sets == kColSets) return false;
+        lr[s] = lr_[i]; bc1[s] = b1[i]; bc2[s] = b2[i];
+        ++sets;
+      }
+      of[base + i] = (uint8_t)s;
+    }
+    first[j + 1] = (uint16_t)(base + n);
+    return true;
+  }
+  uint16_t sets;
+};
+__device__ __forceinline__ void now_cols_write(const NowCols& c, int job, sga_segment* __restrict__ segs, int t0,
+                                               int step) {
+  const int lo = c.first[job], n = c.first[job + 1] - lo;
+  for (int i = t0; i < n; i += step) {
+    const int s = c.of[lo + i];
+    segs[i].lr = (float)c.lr[s];
+    segs[i].bc1 = c.bc1[s];
+    segs[i].bc2 = c.bc2[s];
+  }
+}
+// What a sample's key is formed with, while the table is being written.
+struct ColsOf {
+  const NowCols* cols;
+  int job;
+  __device__ __forceinline__ void into(Hyper& h, int at) const {
+    const int lo = cols->first[job];
+    if (cols->first[job + 1] == lo) return;
+    const int s = cols->of[lo + at];
+    h.lr = (float)cols->lr[s];
+    h.bc1 = cols->bc1[s];
+    h.bc2 = cols->bc2[s];
+  }
+};
+struct NoCols {
+  __device__ __forceinline__ void into(Hyper&, int) const {}
 };
 static inline void launch_seg_dir(const sga_segment* segs, int n_segs, int64_t n, int32_t* dir,
                                   hipStream_t s) {

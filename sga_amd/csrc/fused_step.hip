@@ -33,6 +33,7 @@ struct SrcFused {
   int adams;           // AdamS: the second moment is rebuilt from m (v := m*m), no bias corrections
   // Stepwise interface of the one-sweep select.
   struct Raw { RawG g; F4 r, p, m, v; };
+  using Cols = NowCols;                                        // see k_sample_pick
   struct Chunk { int64_t sh; };
   static constexpr bool kReadAgain = true;                     // by the final sweep
   int bytes() const {                                          // what a sweep reads of a coordinate
@@ -101,8 +102,8 @@ struct SrcFused {
     }
     slab_score_keys<SCORE, FULL>(sc, adams, i, n, q, pp, mm, vv, key);
   }
-  template <bool FULL = false>
-  __device__ __forceinline__ void load(int64_t i, int64_t n, uint32_t key[4]) {
+  template <bool FULL = false, class Cols = NoCols>
+  __device__ __forceinline__ void load(int64_t i, int64_t n, uint32_t key[4], const Cols& cols = Cols()) {
     const int64_t sh = pack_shift<FULL>(i, pack_extra);
     float q[4] = {0, 0, 0, 0}, rr[4] = {0, 0, 0, 0};
     float pp[4] = {0, 0, 0, 0}, mm[4] = {0, 0, 0, 0}, vv[4] = {0, 0, 0, 0};
@@ -125,6 +126,7 @@ struct SrcFused {
       if (FULL || i + e < n) {
         sc.seek(i + e);
         Hyper h = sc.h;
+        cols.into(h, sc.at);
         float ve = vv[e];
         if (adams) { ve = mm[e] * mm[e]; h.bc1 = 1.0f; h.bc2 = 1.0f; }
         key[e] = score_key<SCORE>(q[e], pp[e], mm[e], ve, h);
@@ -374,6 +376,34 @@ __global__ __launch_bounds__(kBlock) void k_fused_final_redo(FinalArgs a, const 
   }
 }
 
+// The final sweeps of a batch of small buckets, one launch: a bucket's own is mostly the launch.  With the tables'
+// columns by argument as well (NowCols), a launch each before, steps of several buckets, |g + r|, us: 1 M coordinates
+// in eight 137 -> 78, 3 M in twelve (`update`) 207 -> 126, 20 M in twelve 312 -> 231.
+struct FinalJobs {
+  struct {
+    FinalArgs a;
+    const sga_segment* segs;
+    const SelState* st;
+    const uint32_t* tile_sel;
+    const uint32_t* tile_eq;
+    const int32_t* seg_dir;
+    int n_segs;
+    uint32_t first;              // workgroup of the bucket's first chunk
+  } j[kMaxJobs];
+  int count;
+};
+static_assert(sizeof(FinalJobs) <= 4000, "travels in the kernel arguments");
+template <bool BF16G, bool BF16V, int SCORE>
+__global__ __launch_bounds__(kBlock) void k_fused_final_batch(FinalJobs jobs) {
+  __shared__ uint32_t s_cnt[2 * kChunkIters];
+  int b = 0;
+  for (int i = 1; i < jobs.count; ++i) b = blockIdx.x >= jobs.j[i].first ? i : b;
+  const auto& J = jobs.j[b];
+  FinalArgs a = J.a;
+  final_body<BF16G, BF16V, SCORE, false>(a, blockIdx.x - J.first, J.segs, J.n_segs, J.st, J.tile_sel, J.tile_eq,
+                                         J.seg_dir, s_cnt);
+}
+
 // Up to this many bytes the select's sweep loads by ordinary accesses, which leave its inputs in the 256 MB
 // memory-side cache for the final sweep to find; non-temporal ones do not, but little of a longer sweep survives.
 // The line lies where `update` begins to lose by ordinary ones; |g + r| still gains a percent at 900 MB.  Step,
@@ -398,7 +428,17 @@ struct FusedJob {
   sga_select_result* result;
   SelWorkspace w;
   float* out[4];            // resid / p / m / v of the new state; all null: in place
+  const sga_segment_cols* cols;   // the table's changing columns for this step; null: it stands
 };
+// The columns of jobs whose select cannot take them along, by launches of their own.
+static int refresh_tables(const FusedJob* fj, int count, hipStream_t s) {
+  for (int b = 0; b < count; ++b)
+    if (const sga_segment_cols* c = fj[b].cols)
+      if (const int rc = sga_segments_refresh(const_cast<sga_segment*>(fj[b].segs), nullptr, fj[b].n_segs, c->lr, c->bc1,
+                                              c->bc2, (void*)s))
+        return rc;
+  return SGA_OK;
+}
 
 // The two-sweep step for up to kMaxJobs buckets that share dtypes, score and knobs: the short
 // kernels of the buckets' selects run as one batched chain, the sweeps are launched per bucket.
@@ -423,6 +463,16 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     use_fast = use_fast && SelBatch::fast_ok(fj[b].w, fj[b].n);
   }
   if (small) use_fast = false;       // three launches do the whole select (small_select.hpp)
+  NowCols cols = {};
+  bool carried = small || use_fast;
+  for (int b = 0; b < count && carried; ++b) {
+    const sga_segment_cols* c = fj[b].cols;
+    carried = c ? cols.add(b, fj[b].n_segs, c->lr, c->bc1, c->bc2) : cols.add(b, 0, nullptr, nullptr, nullptr);
+  }
+  if (!carried) {
+    cols = NowCols{};
+    if (const int rc = refresh_tables(fj, count, s)) return rc;
+  }
   const bool planes = Src::kHyper && use_fast;
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
@@ -437,17 +487,19 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     J.result = f.result;
   }
   if (small) {
-    run_small_select(srcs, B, dj, s);
+    run_small_select(srcs, B, dj, cols, s);
   } else {
     int64_t swept = 0;
     for (int b = 0; b < count; ++b) swept += fj[b].n * srcs.s[b].bytes();
-    run_select_batch<0>(srcs, B, dj, use_fast, s, swept <= kKeepBytes);
+    run_select_batch<0>(srcs, B, dj, cols, use_fast, s, swept <= kKeepBytes);
   }
+  FinalJobs fj_final;
+  uint32_t at = 0;
+  fj_final.count = count;
   for (int b = 0; b < count; ++b) {
     const FusedJob& f = fj[b];
     const SelWorkspace& w = f.w;
     const int64_t n_tiles = cdiv64(f.n, kChunk);
-    ProfPair* pp = prof_begin(SGA_PROF_FUSED_FINAL, s);
     FinalArgs fa;
     fa.g = f.g; fa.r = f.resid; fa.p = f.p; fa.m = f.m; fa.v = f.v; fa.n = f.n; fa.k = f.k;
     fa.ro = f.out[0] ? f.out[0] : f.resid; fa.po = f.out[0] ? f.out[1] : f.p;
@@ -459,6 +511,14 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     fa.pack_extra = pack_extra;
     fa.adams = adams != 0; fa.fold = (flags & SGA_GC_FOLD) != 0; fa.interval = interval;
     fa.planes = w.pbits;
+    if (small && count > 1) {
+      auto& f1 = fj_final.j[b];
+      f1.a = fa; f1.segs = f.segs; f1.n_segs = f.n_segs; f1.st = w.st; f1.tile_sel = w.tile_gt; f1.tile_eq = w.tile_eq;
+      f1.seg_dir = w.seg_dir; f1.first = at;
+      at += (uint32_t)n_tiles;
+      continue;
+    }
+    ProfPair* pp = prof_begin(SGA_PROF_FUSED_FINAL, s);
     // Adam-normalised scores of large buckets: the settled planes instead of a second evaluation of the chain
     if (planes)
       hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, Src::kHyper>), dim3((unsigned)n_tiles), dim3(kBlock), 0, s,
@@ -466,6 +526,11 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     else
       hipLaunchKernelGGL((k_fused_final<BF16G, BF16V, SCORE, false>), dim3((unsigned)n_tiles), dim3(kBlock), 0, s,
                          fa, f.segs, f.n_segs, w.st, w.tile_gt, w.tile_eq, w.seg_dir);
+    prof_end(pp, s);
+  }
+  if (small && count > 1) {
+    ProfPair* pp = prof_begin(SGA_PROF_FUSED_FINAL, s);
+    hipLaunchKernelGGL((k_fused_final_batch<BF16G, BF16V, SCORE>), dim3(at), dim3(kBlock), 0, s, fj_final);
     prof_end(pp, s);
   }
   return check_launch(who);
@@ -1186,7 +1251,7 @@ static int run_fused_spec(const void* g, float* resid, float* p, float* m, float
   J.seed = seed; J.spec = out ? 2 : 1; J.ovf_cap = (uint32_t)x.ovf_cap; J.seg_fail = x.seg_fail;
   J.seg_rec = x.seg_rec; J.cand_rec = x.cand_rec; J.result = result;
   const int64_t ns = J.n_sv * 4;
-  chain_bracket(srcs, B, dirs, out ? kSpecSigmasOut : kSpecSigmas, s);
+  chain_bracket(srcs, B, dirs, {}, out ? kSpecSigmasOut : kSpecSigmas, s);
   // the sweep
   SpecArgs sa;
   sa.splane = w.pbits; sa.fplane = x.dplane; sa.stage = x.stage;
@@ -1250,7 +1315,7 @@ static int fused_entry(const char* who, const void* g, int g_dtype, float* resid
                        float coeff, int fast, int flags, float interval, sga_select_result* result,
                        void* ws, size_t ws_bytes, void* stream, bool single = false,
                        void* ws2 = nullptr, size_t ws2_bytes = 0, uint32_t seed = 0u,
-                       float* const* out = nullptr) {
+                       float* const* out = nullptr, const sga_segment_cols* cols = nullptr) {
   if ((flags & ~(SGA_GC_ADAMS | SGA_GC_FOLD)) != 0) {
     // the dual-lr split belongs to full steps (adamw.py:570-580); HAS_MASK / CLEAR / APPLY_COEFF
     // are what this step does anyway (coeff != 1 applies the coefficient)
@@ -1310,7 +1375,7 @@ static int fused_entry(const char* who, const void* g, int g_dtype, float* resid
   }
   const FusedJob job{g, resid, p, m, v, n, k, segs, n_segs, idx_out, values_out, mask_out, result, w,
                      {out ? out[0] : nullptr, out ? out[1] : nullptr, out ? out[2] : nullptr,
-                      out ? out[3] : nullptr}};
+                      out ? out[3] : nullptr}, cols};
 #define SGA_RUN(BG, BV, SC)                                                                   \
   if (single)                                                                                 \
     return run_fused_spec<BG, BV, SC>(g, resid, p, m, v, n, k, segs, n_segs, idx_out,        \
@@ -1334,6 +1399,13 @@ static int fused_entry(const char* who, const void* g, int g_dtype, float* resid
 #undef SGA_RUN
 }
 
+// The three host columns are there.
+static bool cols_ok(const sga_segment_cols* cols, const char* who) {
+  if (cols && cols->lr && cols->bc1 && cols->bc2) return true;
+  set_error("%s: the columns lr, bc1 and bc2 are required", who);
+  return false;
+}
+
 extern "C" int sga_fused_sparse_step(const void* g, int g_dtype, float* resid, float* p, float* m,
                                      float* v, int64_t n, int64_t k, const sga_segment* segs,
                                      int n_segs, int score_id, int32_t* idx_out, void* values_out,
@@ -1346,11 +1418,22 @@ extern "C" int sga_fused_sparse_step(const void* g, int g_dtype, float* resid, f
                      flags, interval, result, ws, ws_bytes, stream);
 }
 
-extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int n_buckets,
-                                           int g_dtype, int score_id, int values_dtype,
-                                           float factor, float coeff, int fast, int flags,
-                                           float interval, void* stream) {
-  const char* who = "sga_fused_sparse_step_multi";
+extern "C" int sga_fused_sparse_step_cols(const sga_segment_cols* cols, const void* g, int g_dtype, float* resid,
+                                          float* p, float* m, float* v, int64_t n, int64_t k, sga_segment* segs,
+                                          int n_segs, int score_id, int32_t* idx_out, void* values_out,
+                                          int values_dtype, uint8_t* mask_out, float factor, float coeff, int fast,
+                                          int flags, float interval, sga_select_result* result, void* ws,
+                                          size_t ws_bytes, void* stream) {
+  const char* who = "sga_fused_sparse_step_cols";
+  if (!cols_ok(cols, who)) return SGA_ERR_ARG;
+  return fused_entry(who, g, g_dtype, resid, p, m, v, 0, n, k, segs, n_segs, score_id, idx_out, values_out,
+                     values_dtype, mask_out, factor, coeff, fast, flags, interval, result, ws, ws_bytes, stream, false,
+                     nullptr, 0, 0u, nullptr, cols);
+}
+
+static int fused_multi(const char* who, const sga_fused_bucket* buckets, const sga_segment_cols* cols, int n_buckets,
+                       int g_dtype, int score_id, int values_dtype, float factor, float coeff, int fast, int flags,
+                       float interval, void* stream) {
   if ((flags & ~(SGA_GC_ADAMS | SGA_GC_FOLD)) != 0) {
     set_error("%s: flags may carry SGA_GC_ADAMS and SGA_GC_FOLD only (got %d)", who, flags);
     return SGA_ERR_ARG;
@@ -1390,7 +1473,8 @@ extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int 
         const int path = fast != 0 && SelBatch::small_ok(u.n) ? 1 : fast != 0 && SelBatch::fast_ok(w, u.n) ? 0 : 2;
         if (path != pass) continue;
         jobs[cnt++] = FusedJob{u.g, u.resid, u.p, u.m, u.v, u.n, u.k, u.segs, u.n_segs, u.idx_out,
-                               u.values_out, u.mask_out, u.result, w, {nullptr, nullptr, nullptr, nullptr}};
+                               u.values_out, u.mask_out, u.result, w, {nullptr, nullptr, nullptr, nullptr},
+                               cols && cols[b].lr ? cols + b : nullptr};
       }
       if (cnt == kMaxJobs || (b == n_buckets && cnt > 0)) {
         int rc;
@@ -1416,6 +1500,26 @@ extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int 
     }
   }
   return SGA_OK;
+}
+
+extern "C" int sga_fused_sparse_step_multi(const sga_fused_bucket* buckets, int n_buckets,
+                                           int g_dtype, int score_id, int values_dtype,
+                                           float factor, float coeff, int fast, int flags,
+                                           float interval, void* stream) {
+  return fused_multi("sga_fused_sparse_step_multi", buckets, nullptr, n_buckets, g_dtype, score_id, values_dtype,
+                     factor, coeff, fast, flags, interval, stream);
+}
+
+extern "C" int sga_fused_sparse_step_multi_cols(const sga_fused_bucket* buckets, const sga_segment_cols* cols,
+                                                int n_buckets, int g_dtype, int score_id, int values_dtype,
+                                                float factor, float coeff, int fast, int flags, float interval,
+                                                void* stream) {
+  const char* who = "sga_fused_sparse_step_multi_cols";
+  if (!cols) { set_error("%s: cols is required", who); return SGA_ERR_ARG; }
+  for (int b = 0; b < n_buckets; ++b)
+    if (cols[b].lr && !cols_ok(cols + b, who)) return SGA_ERR_ARG;
+  return fused_multi(who, buckets, cols, n_buckets, g_dtype, score_id, values_dtype, factor, coeff, fast, flags,
+                     interval, stream);
 }
 
 extern "C" size_t sga_fused_single_sweep_workspace_bytes(int64_t n, int values_dtype) {
@@ -1538,6 +1642,24 @@ extern "C" int sga_fused_sparse_step_packed(const void* g, int g_dtype, float* s
                      state ? state + 3 * kPackRun : nullptr, kPackExtra, n, k, segs, n_segs,
                      score_id, idx_out, values_out, values_dtype, mask_out, factor, coeff, fast,
                      flags, interval, result, ws, ws_bytes, stream);
+}
+
+extern "C" int sga_fused_sparse_step_packed_cols(const sga_segment_cols* cols, const void* g, int g_dtype, float* state,
+                                                 int64_t n, int64_t k, sga_segment* segs, int n_segs, int score_id,
+                                                 int32_t* idx_out, void* values_out, int values_dtype,
+                                                 uint8_t* mask_out, float factor, float coeff, int fast, int flags,
+                                                 float interval, sga_select_result* result, void* ws, size_t ws_bytes,
+                                                 void* stream) {
+  const char* who = "sga_fused_sparse_step_packed_cols";
+  if (!cols_ok(cols, who)) return SGA_ERR_ARG;
+  if (state && (reinterpret_cast<uintptr_t>(state) & 15)) {
+    set_error("%s: state must be 16-byte aligned", who);
+    return SGA_ERR_ARG;
+  }
+  return fused_entry(who, g, g_dtype, state, state ? state + kPackRun : nullptr, state ? state + 2 * kPackRun : nullptr,
+                     state ? state + 3 * kPackRun : nullptr, kPackExtra, n, k, segs, n_segs, score_id, idx_out,
+                     values_out, values_dtype, mask_out, factor, coeff, fast, flags, interval, result, ws, ws_bytes,
+                     stream, false, nullptr, 0, 0u, nullptr, cols);
 }
 
 // resid/p/m/v <-> packed state (dir 0: pack, 1: unpack); a null array is skipped.

@@ -476,6 +476,7 @@ struct SrcReplay {
   int res_zero;              // res is known to be all zeros: not read
   // Stepwise interface of the one-sweep select.
   struct Raw { RawG g; F4 r, w, m, v; };
+  using Cols = NoCols;                                   // pass 1 has written the table
   struct Chunk { int64_t sh; float coef; };
   static constexpr bool kReadAgain = false;
   static constexpr int kSweep = 1;
@@ -911,7 +912,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
   if (small) {
     per_score([&](auto& srcs, const SelBatch& sub) {
       using Src = typename std::remove_reference<decltype(srcs.s[0])>::type;
-      run_small_select(srcs, sub, dirs_of(srcs, sub), s);
+      run_small_select(srcs, sub, dirs_of(srcs, sub), {}, s);
       hipLaunchKernelGGL((k_write_bits<Src>), sub.grid((unsigned)cdiv64(sub.max_tiles, kChunksPerBlock)),
                          dim3(kBlock), 0, s, srcs, sub.jobs);
     });
@@ -922,7 +923,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     chain_begin(B, dj, s);
   } else {
     per_score([&](auto& srcs, const SelBatch& sub) {
-      launch_sample_pick<true>(srcs, sub, dirs_of(srcs, sub), kBracketSigmas, s);
+      launch_sample_pick<true>(srcs, sub, dirs_of(srcs, sub), {}, kBracketSigmas, s);
     });
     per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, kBracketSigmas, s); });
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, s); });

@@ -362,7 +362,7 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   J.mask = mask_out;
   J.result = result;
   if (SelBatch::small_ok(n)) {
-    run_small_select(srcs, B, SegDirJobs{}, s);
+    run_small_select(srcs, B, SegDirJobs{}, {}, s);
     hipLaunchKernelGGL((k_write_mask<SrcF32>), B.grid((unsigned)cdiv64(B.max_tiles, kChunksPerBlock)),
                        dim3(kBlock), 0, s, srcs, B.jobs, (int64_t)0);
     return check_launch("sga_select_topk");
@@ -370,7 +370,7 @@ extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie
   const bool fast = SelBatch::fast_ok(w, n);
   // the select sweep writes the keys above the bracket straight into mask_out
   J.mask_only = 1;
-  run_select_batch<2>(srcs, B, SegDirJobs{}, fast, s);
+  run_select_batch<2>(srcs, B, SegDirJobs{}, {}, fast, s);
   return check_launch("sga_select_topk");
 }
 

@@ -238,6 +238,7 @@ struct SrcF32 {                 // |x| of an fp32 score array
                                 // non-negative scores are told, without a pass of their own)
   using Raw = F4;
   using Chunk = NoChunk;
+  using Cols = NoCols;                                   // see k_sample_pick
   static constexpr bool kHyper = false, kReadAgain = false;
   static constexpr int kSweep = 2;                       // see chain_sweeps
   static constexpr int kAhead = kChunkIters;
@@ -967,19 +968,23 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // sample's own five, halved); a wider coarse bracket costs the fine one a few keys of resolution.
 //
 // The workgroups behind those of the sample keep house: counters and histograms of the kernels behind this one,
-// the directories of the segment tables (dirs.j[job].dir null: none wanted).
+// the directories of the segment tables (dirs.j[job].dir null: none wanted), the tables' changing columns (cols; the
+// sample forms its keys with those that it was handed, whatever the tables hold by then).
 constexpr int kSampleGroups = 16;
 constexpr int kPickBits = 13, kPickShift = 31 - kPickBits;
 constexpr uint32_t kHeavyBin = 3;                    // a half misses the 100 M case above
 template <class Src, bool COARSE>
 __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
-                                                       uint32_t launch, double sigmas) {
+                                                       typename Src::Cols cols, uint32_t launch,
+                                                       double sigmas) {
   const ChainJob& J = jobs.j[blockIdx.y];
   if (blockIdx.x >= kSampleGroups) {
     const int t0 = (blockIdx.x - kSampleGroups) * kWide + threadIdx.x, step = (gridDim.x - kSampleGroups) * kWide;
     if (COARSE) clear_large(J, t0, step, true);
     else if (t0 < kSmallSegs) J.seg_cnt[t0 * kSmallSegStride] = 0u;
     seg_dirs(dirs, blockIdx.y, t0, step);
+    if constexpr (std::is_same<typename Src::Cols, NowCols>::value)
+      now_cols_write(cols, blockIdx.y, const_cast<sga_segment*>(dirs.j[blockIdx.y].segs), t0, step);
     return;
   }
   __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
@@ -999,7 +1004,11 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
       // coarse: a subset of the windows of the fine sample, which it then agrees with
       const int64_t all = COARSE ? J.n_sv : n_sv;
       uint32_t key[4];
-      src.template load<false>(quad_of_window(j * all / n_sv, n / 4, all, J.seed) * 4, n, key);
+      const int64_t i = quad_of_window(j * all / n_sv, n / 4, all, J.seed) * 4;
+      if constexpr (std::is_same<typename Src::Cols, NowCols>::value)
+        src.template load<false>(i, n, key, ColsOf{&cols, (int)blockIdx.y});
+      else
+        src.template load<false>(i, n, key);
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         __hip_atomic_store(&sample[2 * j + h], (unsigned long long)key[2 * h + 1] << 32 | key[2 * h], __ATOMIC_RELAXED,
@@ -2228,12 +2237,12 @@ static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStr
 // Number of the next launch that takes a sample: one count for the whole library (select.hip).
 uint32_t next_launch();
 template <bool COARSE, class Src>
-static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
-                                      hipStream_t s) {
-  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + 64 <= 4096,
+static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
+                                      const typename Src::Cols& cols, double sigmas, hipStream_t s) {
+  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + sizeof(typename Src::Cols) + 64 <= 4096,
                 "the operands of a batched chain kernel travel in its 4 KiB of kernel arguments");
   hipLaunchKernelGGL((k_sample_pick<Src, COARSE>), B.grid(kSampleGroups + (COARSE ? 16 : 1)), dim3(kWide), 0, s, srcs,
-                     B.jobs, dirs, next_launch(), sigmas);
+                     B.jobs, dirs, cols, next_launch(), sigmas);
 }
 template <class Src>
 static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, double sigmas, hipStream_t s) {
@@ -2242,9 +2251,9 @@ static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& 
 }
 // begin ... bracket, for a batch of one key source
 template <class Src>
-static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, double sigmas,
-                                 hipStream_t s) {
-  launch_sample_pick<true>(srcs, B, dirs, sigmas, s);
+static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
+                                 const typename Src::Cols& cols, double sigmas, hipStream_t s) {
+  launch_sample_pick<true>(srcs, B, dirs, cols, sigmas, s);
   launch_sample_fine(srcs, B, sigmas, s);
 }
 // keep (sources that a writing pass reads again): see bracket_chunk
@@ -2284,10 +2293,10 @@ static inline void chain_tail(const SrcPack<Src>& srcs, const SelBatch& B, hipSt
 }
 
 template <int OUT, class Src>
-static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs, bool fast,
-                                    hipStream_t s, bool keep = false) {
+static inline void run_select_batch(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
+                                    const typename Src::Cols& cols, bool fast, hipStream_t s, bool keep = false) {
   if (fast) {
-    chain_bracket(srcs, B, dirs, kBracketSigmas, s);
+    chain_bracket(srcs, B, dirs, cols, kBracketSigmas, s);
     chain_sweeps(srcs, B, s, keep);
     chain_settle(B, s);
   } else {

@@ -560,8 +560,8 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
 // directories to build on the way (the finishing and writing passes read them).
 template <class Src>
 static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
-                                    hipStream_t s) {
-  launch_sample_pick<false>(srcs, B, dirs, kBracketSigmas, s);
+                                    const typename Src::Cols& cols, hipStream_t s) {
+  launch_sample_pick<false>(srcs, B, dirs, cols, kBracketSigmas, s);
   const int cpw = Src::kHyper || B.max_tiles <= kSweepTiles ? 1 : 4;
   if (cpw == 1)
     hipLaunchKernelGGL((k_small_sweep<Src, 1>), B.grid((unsigned)B.max_tiles), dim3(kBlock), 0, s, srcs, B.jobs);

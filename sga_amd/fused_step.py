@@ -1,6 +1,8 @@
 """Fused per-rank sparse step over a flat bucket (engine order of
 ``sga/engine.py:416-604``): score -> exact top-k -> index pack -> residual
 update -> residual-aware AdamW, as two kinds of sweeps over HBM."""
+import ctypes as C
+
 import torch
 
 from . import _lib as L
@@ -62,13 +64,21 @@ class FusedSparseStep:
             self._ws2 = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         return self._ws2
 
-    def _upload_segments(self, step):
+    def _take_segments(self, step):
+        """The table's changing columns for ``step``, for a call that writes them on its way; None
+        when the table holds them.  The caller sets ``_seg_step`` once that call has been made."""
         if self._seg_step == step:
-            return
+            return None
         # callers may retune lr between steps; of the betas only the bias corrections follow
         self._seg_table.follow_betas(self.segments)
-        self._seg_table.refresh([s["lr"] for s in self.segments], step)
-        self._seg_step = step
+        self._seg_table.take([s["lr"] for s in self.segments], step)
+        self._seg_step = None
+        return self._seg_table.cols
+
+    def _upload_segments(self, step):
+        if self._take_segments(step) is not None:
+            L.call("sga_segments_refresh", *self._seg_table.args, L.stream())
+            self._seg_step = step
 
     @staticmethod
     def _flags(optimizer, fold, interval, inactive_lr_scale):
@@ -95,7 +105,6 @@ class FusedSparseStep:
             raise ValueError(f"k={k} out of range (n={n}, max_k={self.max_k})")
         if score not in SCORE_MAP:
             raise ValueError(f"Unknown SGA score '{score}'. Registered: {sorted(SCORE_MAP)}")
-        self._upload_segments(step)
         if g is None and score == "abs_g_blind":
             raise ValueError("score 'abs_g_blind' ranks the step's own gradient: pass g")
         head = [L.ptr(g), L.SGA_F32 if g is None else L.dtype_code(g), *state_args, n, k,
@@ -108,6 +117,7 @@ class FusedSparseStep:
               or not result.is_contiguous()):
             raise ValueError("result: a contiguous int32[8] device tensor")
         if single_sweep:
+            self._upload_segments(step)
             ws2 = self._single_sweep_ws()
             self._calls += 1
             L.call(name, *head, flags, L.f32(interval),
@@ -122,8 +132,12 @@ class FusedSparseStep:
                         "the state of this step is not the exact top-k step's -- restore it "
                         "from the caller's copy, or use the two-sweep step")
         else:
+            cols = self._take_segments(step)
+            if cols is not None:
+                name, head = name + "_cols", [C.addressof(cols), *head]
             L.call(name, *head, 1 if fast else 0, flags, L.f32(interval), L.ptr(result),
                    L.ptr(self.ws), self.ws_bytes, L.stream())
+            self._seg_step = step
         return self.idx[:k], self.values[:k]
 
     def step(self, g, resid, p, m, v, step, k=None, ratio_percent=None,
@@ -232,7 +246,7 @@ def fused_step_multi(steppers, grads, resids, ps, ms, vs, step, ks=None, ratio_p
         raise ValueError(f"Unknown SGA score '{score}'. Registered: {sorted(SCORE_MAP)}")
     if ks is None:
         ks = [k_for(fs.n, ratio_percent) for fs in steppers]
-    table = (L.FusedBucket * nb)()
+    table, cols = (L.FusedBucket * nb)(), (L.SegmentCols * nb)()
     some_g = next((g for g in grads if g is not None), None)
     gd = L.SGA_F32 if some_g is None else L.dtype_code(some_g)
     vd = L.dtype_code(steppers[0].values)
@@ -250,7 +264,9 @@ def fused_step_multi(steppers, grads, resids, ps, ms, vs, step, ks=None, ratio_p
             raise ValueError("the buckets of one call share the gradient and value dtypes")
         if not (1 <= ks[b] <= min(fs.n, fs.max_k)):
             raise ValueError(f"bucket {b}: k={ks[b]} out of range (n={fs.n}, max_k={fs.max_k})")
-        fs._upload_segments(step)
+        c = fs._take_segments(step)
+        if c is not None:
+            cols[b] = c
         e = table[b]
         e.g = None if g is None else g.data_ptr()
         e.resid, e.p, e.m, e.v = (t.data_ptr() for t in (r, p, m, v))
@@ -260,8 +276,10 @@ def fused_step_multi(steppers, grads, resids, ps, ms, vs, step, ks=None, ratio_p
         e.mask_out = fs.mask.data_ptr() if fs.mask is not None else None
         e.result = fs.result.data_ptr()
         e.ws, e.ws_bytes = fs.ws.data_ptr(), fs.ws_bytes
-    L.call("sga_fused_sparse_step_multi", table, nb, gd, SCORE_MAP[score], vd, L.f32(factor),
+    L.call("sga_fused_sparse_step_multi_cols", table, cols, nb, gd, SCORE_MAP[score], vd, L.f32(factor),
            L.f32(coeff), 1 if fast else 0, flags, L.f32(interval), L.stream())
+    for fs in steppers:
+        fs._seg_step = step
     return [(fs.idx[:k], fs.values[:k]) for fs, k in zip(steppers, ks)]
 
 

@@ -54,6 +54,7 @@ class SegmentTable:
         self.args = (None if self.segs is None else self.segs.data_ptr(),
                      None if self.rsegs is None else self.rsegs.data_ptr(), self.count,
                      self._lr.ctypes.data, self._bc1.ctypes.data, self._bc2.ctypes.data)
+        self.cols = L.SegmentCols(*self.args[3:])       # what the fused steps take along
         self._hyper = list(map(_HYPER, rows))
         self._betas = self._last_lr = None
         self.follow_betas(rows)
