@@ -96,6 +96,19 @@ int sga_scatter_selected(float* dst, const int32_t* idx, const float* src,
 int sga_pack_selected(float* grad, const int32_t* idx, void* values,
                       int values_dtype, float factor, int64_t k,
                       int64_t n_grad, void* stream);
+/* The same, and below[0] = number of entries of idx (ascending, k >= 1) that
+ * are under `split`: the bound of the bucket's two slices (support.py:345-351). */
+int sga_pack_selected_split(float* grad, const int32_t* idx, void* values,
+                            int values_dtype, float factor, int64_t k,
+                            int64_t n_grad, int64_t split, int64_t* below,
+                            void* stream);
+/* dst[idx[i]] = src[i] where the source list lies in up to SGA_MAX_PARTS
+ * arrays of counts[j] entries, one behind the other (HOST arrays, read before
+ * the call returns). */
+#define SGA_MAX_PARTS 8
+int sga_scatter_selected_parts(float* dst, const int32_t* idx,
+                               const float* const* src, const int64_t* counts,
+                               int n_parts, int64_t n_dst, void* stream);
 
 /* total[0] += sum(values^2), two-stage, fixed order
  *                 -- compact_norm_sq_contribution, kernels.py:252-268.
@@ -193,6 +206,22 @@ int sga_mask_count_cuts(const uint8_t* mask, int64_t n, uint32_t* chunk_counts,
 /* Phase 2: idx_out[..k) = ascending positions of the non-zero bytes. */
 int sga_mask_fill(const uint8_t* mask, int64_t n, const uint32_t* chunk_offsets,
                   int32_t* idx_out, int64_t idx_capacity, void* stream);
+
+/* The same in two launches before the read of the totals and one behind it.
+ * sga_mask_totals: totals as sga_mask_count_cuts gives them (n >= 1); scratch
+ * has sga_mask_list_words(n) uint32 entries and is what sga_mask_list, on the
+ * same mask, starts from.
+ * sga_mask_list: idx_out[..capacity) = ascending positions of the non-zero
+ * bytes; with grad also their values, grad[idx] * factor, into up to
+ * SGA_MAX_PARTS arrays of counts[j] entries, one behind the other (HOST
+ * arrays; torch_pipelined_mask.py:91-116). */
+int64_t sga_mask_list_words(int64_t n);
+int sga_mask_totals(const uint8_t* mask, int64_t n, uint32_t* scratch,
+                    int64_t step, int cuts, int64_t* totals, void* stream);
+int sga_mask_list(const uint8_t* mask, int64_t n, const uint32_t* scratch,
+                  int32_t* idx_out, int64_t capacity, const float* grad,
+                  float factor, float* const* values, const int64_t* counts,
+                  int n_parts, void* stream);
 
 /* ---- residual-aware AdamW (sga/plugins/optimizer/adamw.py) -------------- */
 

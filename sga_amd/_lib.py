@@ -58,6 +58,8 @@ SIGNATURES = {
     "sga_last_error": (C.c_char_p, []),
     "sga_scatter_selected": (I32, [P, P, P, I64, I64, P]),
     "sga_pack_selected": (I32, [P, P, P, I32, F, I64, I64, P]),
+    "sga_pack_selected_split": (I32, [P, P, P, I32, F, I64, I64, I64, P, P]),
+    "sga_scatter_selected_parts": (I32, [P, P, P, P, I32, I64, P]),
     "sga_norm_partials": (I64, [I64]),
     "sga_compact_norm_sq": (I32, [P, I64, P, P, P]),
     "sga_compact_norm_sq_noalloc": (I32, [P, I64, P, P]),
@@ -71,6 +73,9 @@ SIGNATURES = {
     "sga_mask_count": (I32, [P, I64, P, P, P]),
     "sga_mask_count_cuts": (I32, [P, I64, P, I64, I32, P, P]),
     "sga_mask_fill": (I32, [P, I64, P, P, I64, P]),
+    "sga_mask_list_words": (I64, [I64]),
+    "sga_mask_totals": (I32, [P, I64, P, I64, I32, P, P]),
+    "sga_mask_list": (I32, [P, I64, P, P, I64, P, F, P, P, I32, P]),
     "sga_adamw_grad_correct": (I32, [P, P, P, P, P, I64] + [F] * 12 + [I32, I32, P]),
     "sga_adamw_grad_correct_multi": (I32, [P, I32, I64, F, F, I32, P]),
     "sga_adamw_grad_correct_compact_multi": (I32, [P, I32, I64, I32, F, F, P]),
@@ -292,6 +297,15 @@ def dtype_code(t):
     if t.dtype == torch.bfloat16:
         return SGA_BF16
     raise TypeError(f"unsupported dtype {t.dtype} (fp32 or bf16)")
+
+
+MAX_PARTS = 8                    # SGA_MAX_PARTS
+
+
+def parts(tensors, counts):
+    """(addresses, counts, number) of a list in several arrays, as host arrays."""
+    m = len(tensors)
+    return (P * m)(*map(ptr, tensors)), (I64 * m)(*counts), m
 
 
 class TableUploader:

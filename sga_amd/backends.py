@@ -6,7 +6,7 @@ import torch
 
 from . import _lib as L
 from . import kernels as K
-from .support import compact_mask_u8
+from .support import compact_mask_u8, mask_totals
 
 
 def index_layout_bounds(idx, n, slices=2):
@@ -27,11 +27,15 @@ def index_layout_pack(grad, idx, values, factor=1.0, slices=2):
     ``idx``, packed slice by slice as the reference pipelines it
     (``torch_pipelined_index.py:508-520``); the packed positions of ``grad``
     are zeroed.  Returns the per-slice (lo, hi) ranges of ``values``."""
-    out = index_layout_bounds(idx, grad.numel(), slices)
-    for lo, hi in out:
-        if hi > lo:
-            K.pack_selected(grad, idx[lo:hi], values[lo:hi], factor)
-    return out
+    k = idx.numel()
+    if slices != 2 or k == 0:
+        out = index_layout_bounds(idx, grad.numel(), slices)
+        K.pack_selected(grad, idx, values, factor)     # the slices follow one another: one launch
+        return out
+    below = torch.empty(1, dtype=torch.int64, device=idx.device)
+    K.pack_selected(grad, idx, values, factor, below)  # ... and the bound comes with it
+    n0 = int(below.item())
+    return [(0, n0), (n0, k)]
 
 
 def index_layout_writeback(grad, idx, values):
@@ -46,6 +50,18 @@ def mask_layout_pack(grad, mask_u8, factor=1.0, slices=2):
     read of ``grad``.  Returns (payload list, idx) -- idx is kept so unpack
     does not recompute the compaction."""
     n = grad.numel()
+    if (1 < slices <= L.MAX_PARTS and mask_u8.numel() == n and grad.is_cuda and grad.is_contiguous()
+            and grad.dtype == torch.float32):
+        # the slices' ends come with the count, the values with the positions
+        mk, scratch, k, ends = mask_totals(mask_u8, step=n // slices, cuts=slices - 1)
+        pos = [0] + ends + [k]
+        counts = [hi - lo for lo, hi in zip(pos[:-1], pos[1:])]
+        idx = torch.empty(k, dtype=torch.int32, device=grad.device)
+        payloads = [torch.empty(c, dtype=torch.float32, device=grad.device) for c in counts]
+        if k:
+            L.call("sga_mask_list", L.ptr(mk), n, L.ptr(scratch), L.ptr(idx), k, L.ptr(grad),
+                   L.f32(factor), *L.parts(payloads, counts), L.stream())
+        return payloads, idx
     if slices > 1 and mask_u8.numel() == n:
         # the slices' ends come with the count: no search of its own and one wait for the device
         idx, ends = compact_mask_u8(mask_u8, step=n // slices, cuts=slices - 1)
@@ -68,8 +84,4 @@ def mask_layout_pack(grad, mask_u8, factor=1.0, slices=2):
 
 def mask_layout_unpack(grad, idx, payloads):
     """``grad[s:e][mask] = payload`` per slice (``torch_pipelined_mask.py:117-138``)."""
-    off = 0
-    for p in payloads:
-        if p.numel():
-            K.scatter_selected(grad, idx[off:off + p.numel()], p)
-        off += p.numel()
+    K.scatter_parts(grad, idx, payloads)

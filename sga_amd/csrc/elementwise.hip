@@ -19,15 +19,62 @@ __global__ __launch_bounds__(kBlock) void k_scatter(float* __restrict__ dst,
   }
 }
 
+// Up to kParts arrays that hold consecutive ranges of one list: part j is entries [end[j - 1], end[j]).
+constexpr int kParts = SGA_MAX_PARTS;
+struct Parts {
+  float* base[kParts];           // of entry 0, were the part that long
+  int64_t end[kParts];
+  int count;
+  __host__ __device__ __forceinline__ float* at(int64_t i) const {
+    float* p = base[0];
+    for (int j = 1; j < count; ++j)
+      if (i >= end[j - 1]) p = base[j];
+    return p + i;
+  }
+};
+// One launch for the slices of a list (two of them: 4.8 us less a step, and a call from the host).
+__global__ __launch_bounds__(kBlock) void k_scatter_parts(float* __restrict__ dst, const int32_t* __restrict__ idx,
+                                                          Parts src, int64_t k, int64_t n_dst) {
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < k; i += (int64_t)gridDim.x * kBlock) {
+    const int64_t j = idx[i];
+    if (j >= 0 && j < n_dst) dst[j] = *src.at(i);
+  }
+}
+
 // ------------------------------------------------------------------- pack
+// The calling wave's number of entries of the ascending idx[0, k) below `split`: 64 entries a round of loads.
+__device__ __forceinline__ int64_t wave_lower_bound(const int32_t* __restrict__ idx, int64_t k, int64_t split) {
+  int64_t lo = 0, hi = k;                            // entries before lo are below, those from hi on are not
+  while (lo < hi) {
+    const int64_t step = (hi - lo + kWave - 1) / kWave, at = lo + lane_id() * step;
+    const uint64_t below = ballot64(at < hi && idx[at] < split);
+    const int c = __popcll(below);                   // lanes 0 .. c - 1
+    const int64_t from = lo;
+    lo = c ? from + (c - 1) * step + 1 : from;
+    if (from + c * step < hi) hi = from + c * step;
+    if (c == 0) break;
+  }
+  return uniform_i64(lo);
+}
+// With `below`, the last workgroup of the grid counts the entries under `split` instead: the slices' bound is there
+// with the pack, where a search of its own and the wait for it came first (index layout, 63 M coordinates: kernels of
+// 27 us with a wait between them, 19.9 so; a step 370 -> 366 us).
 template <bool BF16, bool SCALE>
 __global__ __launch_bounds__(kBlock) void k_pack(float* __restrict__ grad,
                                                  const int32_t* __restrict__ idx,
                                                  void* __restrict__ values,
                                                  float factor, int64_t k,
-                                                 int64_t n_grad) {
+                                                 int64_t n_grad, int64_t split = 0, int64_t* __restrict__ below = nullptr) {
+  unsigned groups = gridDim.x;
+  if (below && blockIdx.x == --groups) {
+    if (wave_id() == 0) {
+      const int64_t c = wave_lower_bound(idx, k, split);
+      if (lane_id() == 0) *below = c;
+    }
+    return;
+  }
   for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < k;
-       i += (int64_t)gridDim.x * kBlock) {
+       i += (int64_t)groups * kBlock) {
     const int64_t j = idx[i];
     if (j < 0 || j >= n_grad) continue;
     float x = grad[j];
@@ -396,6 +443,128 @@ __global__ __launch_bounds__(kBlock) void k_mask_fill(const uint8_t* __restrict_
   }
 }
 
+// The compaction around one wait of the host, which needs the count to allocate: before it, the chunks' counts with
+// their sums by workgroup (a group of 16 chunks), and one workgroup that turns the sums into offsets and takes the
+// totals; behind it, the positions, and with GATHER the values at them.  (Counts, two launches of a scan, a launch for
+// the slices' ends, the positions, and a gather for each slice were eight: mask layout, step on 1.15 M coordinates in
+// 45 tensors 125 to 139 us, 119 so.)
+__global__ __launch_bounds__(kBlock) void k_mask_groups(const uint8_t* __restrict__ mask, int64_t n,
+                                                        uint32_t* __restrict__ counts, uint32_t* __restrict__ sums,
+                                                        int64_t n_chunks) {
+  __shared__ uint32_t s_w[kChunksPerBlock];
+  const int64_t c0 = ((int64_t)blockIdx.x * kChunksPerBlock + wave_id()) * kMaskChunks;
+  uint32_t bits[kMaskChunks], all = 0;
+  mask_bits(mask, n, c0, bits);                       // chunks past the end: zero
+#pragma unroll
+  for (int u = 0; u < kMaskChunks; ++u) {
+    const uint32_t cnt = (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan((uint32_t)__popc(bits[u])), kWave - 1);
+    if (lane_id() == 0 && c0 + u < n_chunks) counts[c0 + u] = cnt;
+    all += cnt;
+  }
+  if (lane_id() == 0) s_w[wave_id()] = all;
+  __syncthreads();
+  if (threadIdx.x == 0) sums[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+}
+
+constexpr int kGroupChunks = kChunksPerBlock * kMaskChunks;
+constexpr int kTotalsBlock = 1024, kTotalsWaves = kTotalsBlock / kWave;
+// out[0] = all set bytes, out[j] = those before j * step (j = 1 .. cuts).  sums become the groups' offsets.
+__global__ __launch_bounds__(kTotalsBlock) void k_mask_totals(const uint8_t* __restrict__ mask, int64_t n,
+                                                              const uint32_t* __restrict__ counts,
+                                                              uint32_t* __restrict__ sums, int64_t n_groups, int64_t step,
+                                                              int cuts, int64_t* __restrict__ out) {
+  __shared__ uint32_t s_w[2][kTotalsWaves];
+  uint32_t run = 0;                                   // set bytes before the round
+  int turn = 0;
+  for (int64_t g0 = 0; g0 < n_groups; g0 += kTotalsBlock, turn ^= 1) {
+    const int64_t g = g0 + threadIdx.x;
+    const uint32_t v = g < n_groups ? sums[g] : 0u, incl = wave_incl_scan(v);
+    if (lane_id() == kWave - 1) s_w[turn][wave_id()] = incl;
+    __syncthreads();
+    const uint32_t waves = row_incl_scan(s_w[turn][lane_id() % kTotalsWaves]);
+    const int w = uniform_i32(wave_id());
+    const uint32_t before = w ? (uint32_t)__builtin_amdgcn_readlane((int)waves, w - 1) : 0u;
+    if (g < n_groups) sums[g] = run + before + incl - v;
+    run += (uint32_t)__builtin_amdgcn_readlane((int)waves, kTotalsWaves - 1);
+  }
+  if (threadIdx.x == 0) out[0] = (int64_t)run;
+  __syncthreads();                                    // the offsets, which the same workgroup wrote
+  for (int j = 1 + wave_id(); j <= cuts; j += kTotalsWaves) {
+    const int64_t at = (int64_t)j * step, c = at / kChunk;
+    if (at >= n) {
+      if (lane_id() == 0) out[j] = (int64_t)run;
+      continue;
+    }
+    const int64_t c0 = c / kGroupChunks * kGroupChunks;
+    uint32_t cnt = lane_id() < c - c0 ? counts[c0 + lane_id()] : 0u;
+    for (int64_t i = c * kChunk + lane_id(); i < at; i += kWave) cnt += mask[i] != 0;
+    cnt = wave_sum(cnt);
+    if (lane_id() == 0) out[j] = (int64_t)sums[c / kGroupChunks] + cnt;
+  }
+}
+
+// Positions (and values) of a wave's four chunks.  They go through LDS and leave in order, as whole lines: with few
+// set (a hundredth: 41 of 4096) in one piece, whose values are one round of loads in flight together.
+template <bool GATHER, bool SCALE>
+__global__ __launch_bounds__(kBlock) void k_mask_list(const uint8_t* __restrict__ mask, int64_t n,
+                                                      const uint32_t* __restrict__ counts,
+                                                      const uint32_t* __restrict__ offsets, int32_t* __restrict__ idx_out,
+                                                      int64_t cap, int64_t n_chunks, const float* __restrict__ grad,
+                                                      float factor, Parts values) {
+  __shared__ int32_t s_idx[kChunksPerBlock][kChunk + kChunk / 16];
+  const int64_t g0 = (int64_t)blockIdx.x * kGroupChunks, c0 = g0 + wave_id() * kMaskChunks;
+  if (c0 >= n_chunks) return;
+  uint32_t bits[kMaskChunks];
+  mask_bits(mask, n, c0, bits);
+  const uint32_t in_group = lane_id() < kGroupChunks && g0 + lane_id() < n_chunks ? counts[g0 + lane_id()] : 0u;
+  const uint32_t upto = row_incl_scan(in_group);      // lane l < 16: set bytes of the group's chunks 0 .. l
+  const int first = uniform_i32(wave_id()) * kMaskChunks;
+  const uint32_t lead = first ? (uint32_t)__builtin_amdgcn_readlane((int)upto, first - 1) : 0u;
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)upto, first + kMaskChunks - 1) - lead;
+  int64_t base = (int64_t)offsets[blockIdx.x] + lead;
+  int32_t* own = s_idx[wave_id()];
+  auto leave = [&](uint32_t have) {                   // the staged positions, in order
+    __builtin_amdgcn_wave_barrier();                  // the wave's own LDS: its accesses stay in order
+    const int64_t room = cap - base;
+    const uint32_t put = room < (int64_t)have ? (uint32_t)(room < 0 ? 0 : room) : have;
+    if (GATHER) {
+      for (uint32_t j = lane_id(); j < put; j += kWave) {
+        const int32_t i = own[j + j / 16];
+        idx_out[base + j] = i;
+        float v = grad[i];
+        if (SCALE) v = v * factor;
+        *values.at(base + j) = v;
+      }
+    } else {
+      typedef int32_t i4v __attribute__((ext_vector_type(4), aligned(4)));
+      for (uint32_t j = lane_id() * kVec; j < put; j += kWave * kVec) {
+        const int32_t* q = own + j + j / 16;          // the quad lies in one group of 16
+        const int32_t v[4] = {q[0], q[1], q[2], q[3]};
+        if (j + kVec <= put) {
+          *reinterpret_cast<i4v*>(idx_out + base + j) = i4v{v[0], v[1], v[2], v[3]};
+        } else {
+          for (uint32_t e = 0; j + e < put; ++e) idx_out[base + j + e] = v[e];
+        }
+      }
+    }
+    base += have;
+    __builtin_amdgcn_wave_barrier();
+  };
+  const bool together = total <= (uint32_t)kChunk;
+  uint32_t at0 = 0;
+#pragma unroll
+  for (int u = 0; u < kMaskChunks; ++u) {
+    const uint32_t mine = (uint32_t)__popc(bits[u]), incl = wave_incl_scan(mine);
+    const uint32_t count = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    const int32_t i0 = (int32_t)((c0 + u) * kChunk + lane_id() * 16);
+    uint32_t at = at0 + incl - mine;
+    for (uint32_t left = bits[u]; left; left &= left - 1u, ++at) own[at + at / 16] = i0 + __ffs((int)left) - 1;
+    if (together) at0 += count;
+    else leave(count);
+  }
+  if (together) leave(at0);
+}
+
 // out[0] = all set bytes, out[j] = those before j * step (j = 1 .. cuts): a wave per cut, from the offsets.
 __global__ __launch_bounds__(kBlock) void k_mask_cuts(const uint8_t* __restrict__ mask, int64_t n,
                                                       const uint32_t* __restrict__ offsets, int64_t step, int cuts,
@@ -439,27 +608,73 @@ extern "C" int sga_scatter_selected(float* dst, const int32_t* idx,
   return check_launch("sga_scatter_selected");
 }
 
+static int pack_selected(const char* who, float* grad, const int32_t* idx, void* values, int values_dtype, float factor,
+                         int64_t k, int64_t n_grad, int64_t split, int64_t* below, void* stream) {
+  if (!grad || !idx || !values || k < 0 || n_grad >= (1ll << 31) ||
+      (values_dtype != SGA_F32 && values_dtype != SGA_BF16)) {
+    set_error("%s: bad argument (k=%lld n_grad=%lld dtype=%d, needs < 2^31)", who, (long long)k, (long long)n_grad,
+              values_dtype);
+    return SGA_ERR_ARG;
+  }
+  dim3 grid(stream_grid(k, kBlock) + (below ? 1u : 0u)), block(kBlock);
+  hipStream_t st = (hipStream_t)stream;
+  const bool scale = factor != 1.0f;
+  if (values_dtype == SGA_BF16) {
+    if (scale) hipLaunchKernelGGL((k_pack<true, true>), grid, block, 0, st, grad, idx, values, factor, k, n_grad, split, below);
+    else hipLaunchKernelGGL((k_pack<true, false>), grid, block, 0, st, grad, idx, values, factor, k, n_grad, split, below);
+  } else {
+    if (scale) hipLaunchKernelGGL((k_pack<false, true>), grid, block, 0, st, grad, idx, values, factor, k, n_grad, split, below);
+    else hipLaunchKernelGGL((k_pack<false, false>), grid, block, 0, st, grad, idx, values, factor, k, n_grad, split, below);
+  }
+  return check_launch(who);
+}
+
 extern "C" int sga_pack_selected(float* grad, const int32_t* idx, void* values,
                                  int values_dtype, float factor, int64_t k,
                                  int64_t n_grad, void* stream) {
   if (k == 0) return SGA_OK;
-  if (!grad || !idx || !values || k < 0 || n_grad >= (1ll << 31) ||
-      (values_dtype != SGA_F32 && values_dtype != SGA_BF16)) {
-    set_error("sga_pack_selected: bad argument (k=%lld n_grad=%lld dtype=%d, needs < 2^31)",
-              (long long)k, (long long)n_grad, values_dtype);
+  return pack_selected("sga_pack_selected", grad, idx, values, values_dtype, factor, k, n_grad, 0, nullptr, stream);
+}
+
+extern "C" int sga_pack_selected_split(float* grad, const int32_t* idx, void* values, int values_dtype, float factor,
+                                       int64_t k, int64_t n_grad, int64_t split, int64_t* below, void* stream) {
+  if (!below || k < 1) {
+    set_error("sga_pack_selected_split: bad argument (k=%lld, below is required)", (long long)k);
     return SGA_ERR_ARG;
   }
-  dim3 grid(stream_grid(k, kBlock)), block(kBlock);
-  hipStream_t st = (hipStream_t)stream;
-  const bool scale = factor != 1.0f;
-  if (values_dtype == SGA_BF16) {
-    if (scale) hipLaunchKernelGGL((k_pack<true, true>), grid, block, 0, st, grad, idx, values, factor, k, n_grad);
-    else hipLaunchKernelGGL((k_pack<true, false>), grid, block, 0, st, grad, idx, values, factor, k, n_grad);
-  } else {
-    if (scale) hipLaunchKernelGGL((k_pack<false, true>), grid, block, 0, st, grad, idx, values, factor, k, n_grad);
-    else hipLaunchKernelGGL((k_pack<false, false>), grid, block, 0, st, grad, idx, values, factor, k, n_grad);
+  return pack_selected("sga_pack_selected_split", grad, idx, values, values_dtype, factor, k, n_grad, split, below,
+                       stream);
+}
+
+// The parts' arrays as Parts; false (with the error text) where they do not fit together.
+static bool parts_of(const char* who, float* const* base, const int64_t* counts, int n_parts, Parts* p, int64_t* total) {
+  bool ok = base && counts && n_parts >= 1 && n_parts <= kParts;
+  *total = 0;
+  p->count = n_parts;
+  for (int j = 0; ok && j < n_parts; ++j) {
+    ok = counts[j] >= 0 && (base[j] || counts[j] == 0);
+    p->base[j] = reinterpret_cast<float*>(reinterpret_cast<uintptr_t>(base[j]) - (uintptr_t)*total * sizeof(float));
+    *total += counts[j];
+    p->end[j] = *total;
   }
-  return check_launch("sga_pack_selected");
+  if (!ok) set_error("%s: bad parts (1 <= n_parts=%d <= %d, counts >= 0)", who, n_parts, kParts);
+  return ok;
+}
+
+extern "C" int sga_scatter_selected_parts(float* dst, const int32_t* idx, const float* const* src, const int64_t* counts,
+                                          int n_parts, int64_t n_dst, void* stream) {
+  const char* who = "sga_scatter_selected_parts";
+  Parts p = {};
+  int64_t k = 0;
+  if (!parts_of(who, const_cast<float* const*>(src), counts, n_parts, &p, &k)) return SGA_ERR_ARG;
+  if (k == 0) return SGA_OK;
+  if (!dst || !idx || n_dst >= (1ll << 31)) {
+    set_error("%s: bad argument (n_dst=%lld, needs < 2^31)", who, (long long)n_dst);
+    return SGA_ERR_ARG;
+  }
+  hipLaunchKernelGGL(k_scatter_parts, dim3(stream_grid(k, kBlock)), dim3(kBlock), 0, (hipStream_t)stream, dst, idx, p, k,
+                     n_dst);
+  return check_launch(who);
 }
 
 static const int64_t kNormMaxBlocks = 2048;
@@ -760,4 +975,56 @@ extern "C" int sga_mask_fill(const uint8_t* mask, int64_t n,
   hipLaunchKernelGGL(k_mask_fill, dim3((unsigned)cdiv64(nc, kChunksPerBlock * kMaskChunks)), dim3(kBlock), 0,
                      (hipStream_t)stream, mask, n, chunk_offsets, idx_out, idx_capacity, nc);
   return check_launch("sga_mask_fill");
+}
+
+static inline int64_t n_groups_of(int64_t n) { return cdiv64(n_chunks_of(n), kGroupChunks); }
+// Words of the scratch of sga_mask_totals / sga_mask_list: a count per chunk, an offset per group of 16.
+extern "C" int64_t sga_mask_list_words(int64_t n) { return n_chunks_of(n) + n_groups_of(n); }
+
+extern "C" int sga_mask_totals(const uint8_t* mask, int64_t n, uint32_t* scratch, int64_t step, int cuts, int64_t* totals,
+                               void* stream) {
+  if (!mask || !scratch || !totals || n < 1 || n >= (1ll << 31) || step < 0 || cuts < 0) {
+    set_error("sga_mask_totals: bad argument (n=%lld, int32 indices need n < 2^31)", (long long)n);
+    return SGA_ERR_ARG;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t nc = n_chunks_of(n), ng = n_groups_of(n);
+  if (step > n) step = n;                // the same answers, and j * step cannot wrap around
+  hipLaunchKernelGGL(k_mask_groups, dim3((unsigned)ng), dim3(kBlock), 0, st, mask, n, scratch, scratch + nc, nc);
+  hipLaunchKernelGGL(k_mask_totals, dim3(1), dim3(kTotalsBlock), 0, st, mask, n, scratch, scratch + nc, ng, step, cuts,
+                     totals);
+  return check_launch("sga_mask_totals");
+}
+
+extern "C" int sga_mask_list(const uint8_t* mask, int64_t n, const uint32_t* scratch, int32_t* idx_out, int64_t capacity,
+                             const float* grad, float factor, float* const* values, const int64_t* counts, int n_parts,
+                             void* stream) {
+  const char* who = "sga_mask_list";
+  if (!mask || !scratch || (!idx_out && capacity > 0) || n < 1 || n >= (1ll << 31) || capacity < 0) {
+    set_error("%s: bad argument (n=%lld capacity=%lld)", who, (long long)n, (long long)capacity);
+    return SGA_ERR_ARG;
+  }
+  Parts p = {};
+  int64_t room = 0;
+  if (grad) {
+    if (!parts_of(who, values, counts, n_parts, &p, &room)) return SGA_ERR_ARG;
+    if (capacity > room) {
+      set_error("%s: the parts hold %lld values, the list %lld", who, (long long)room, (long long)capacity);
+      return SGA_ERR_ARG;
+    }
+  }
+  hipStream_t st = (hipStream_t)stream;
+  const int64_t nc = n_chunks_of(n);
+  const dim3 grid((unsigned)n_groups_of(n)), block(kBlock);
+  const uint32_t* off = scratch + nc;
+  if (!grad)
+    hipLaunchKernelGGL((k_mask_list<false, false>), grid, block, 0, st, mask, n, scratch, off, idx_out, capacity, nc, grad,
+                       factor, p);
+  else if (factor != 1.0f)
+    hipLaunchKernelGGL((k_mask_list<true, true>), grid, block, 0, st, mask, n, scratch, off, idx_out, capacity, nc, grad,
+                       factor, p);
+  else
+    hipLaunchKernelGGL((k_mask_list<true, false>), grid, block, 0, st, mask, n, scratch, off, idx_out, capacity, nc, grad,
+                       factor, p);
+  return check_launch(who);
 }

@@ -22,9 +22,11 @@ def scatter_selected(dst, indices, src):
            dst.numel(), L.stream())
 
 
-def pack_selected(grad, indices, values, factor):
+def pack_selected(grad, indices, values, factor, below=None):
     """``values[i] = grad[idx[i]]*factor; grad[idx[i]] = 0`` in one pass
-    (``sga/kernels.py:166-187``).  ``values`` may be fp32 or bf16."""
+    (``sga/kernels.py:166-187``).  ``values`` may be fp32 or bf16.  ``below``
+    (one int64 on the device): also the number of ascending indices under
+    ``grad.numel() // 2``."""
     k = indices.numel()
     if k == 0:
         return
@@ -37,8 +39,30 @@ def pack_selected(grad, indices, values, factor):
     if grad.dtype != torch.float32:
         raise TypeError("pack_selected: fp32 grad buffer")
     assert values.numel() >= k
-    L.call("sga_pack_selected", L.ptr(grad), L.ptr(indices), L.ptr(values),
-           L.dtype_code(values), L.f32(factor), k, grad.numel(), L.stream())
+    args = (L.ptr(grad), L.ptr(indices), L.ptr(values), L.dtype_code(values), L.f32(factor), k,
+            grad.numel())
+    if below is None:
+        L.call("sga_pack_selected", *args, L.stream())
+    else:
+        L.call("sga_pack_selected_split", *args, grad.numel() // 2, L.ptr(below), L.stream())
+
+
+def scatter_parts(dst, indices, parts):
+    """``scatter_selected`` of a list that lies in several arrays, one behind
+    the other: one launch for up to eight of them."""
+    counts = [p.numel() for p in parts]
+    if (not 1 < len(parts) <= L.MAX_PARTS or sum(counts) != indices.numel() or indices.dtype != torch.int32
+            or not all(t.is_cuda and t.is_contiguous() for t in (dst, indices, *parts))
+            or not all(t.dtype == torch.float32 for t in (dst, *parts)) or dst.numel() >= 2 ** 31):
+        off = 0
+        for p, c in zip(parts, counts):
+            if c:
+                scatter_selected(dst, indices[off:off + c], p)
+            off += c
+        return
+    if indices.numel():
+        L.call("sga_scatter_selected_parts", L.ptr(dst), L.ptr(indices), *L.parts(parts, counts),
+               dst.numel(), L.stream())
 
 
 def _check_x(x):

@@ -23,12 +23,9 @@ class IndexPool:
         return self.buf
 
 
-def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None, step=0, cuts=0):
-    """Ascending int32 positions of the non-zero bytes of ``mask_u8``
-    (``sga/support.py:57-99``): one counting sweep, one host read of k (the
-    reference syncs on the count too), one ordered fill sweep.  With ``cuts`` the
-    same read also brings how many positions lie before ``step``, ``2 * step``, ...:
-    returns ``(idx, [that many ints])``."""
+def mask_totals(mask_u8, step=0, cuts=0):
+    """First half of a compaction: ``(flat uint8 mask, scratch, k, [set bytes before step,
+    2 * step, ...])``, with one host read.  The second half is ``sga_mask_list``."""
     n = mask_u8.numel()
     assert n < 2 ** 31, f"int32 support indices assume < 2^31 elements, got {n}"
     L.require_dev(mask_u8)
@@ -38,22 +35,28 @@ def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None, step=0, cuts=0):
         mk = mk.view(torch.uint8)
     if mk.dtype != torch.uint8:
         raise TypeError("compact_mask_u8: uint8/bool mask")
-    dev = mk.device
     if n == 0:
-        idx = torch.empty(0, dtype=torch.int32, device=dev)
-        return (idx, [0] * cuts) if cuts else idx
-    counts = torch.empty(int(L.raw("sga_mask_chunks", n)), dtype=torch.int32, device=dev)
-    total = torch.empty(1 + cuts, dtype=torch.int64, device=dev)
-    if cuts:
-        L.call("sga_mask_count_cuts", L.ptr(mk), n, L.ptr(counts), step, cuts, L.ptr(total), L.stream())
-    else:
-        L.call("sga_mask_count", L.ptr(mk), n, L.ptr(counts), L.ptr(total), L.stream())
-    k, *before = total.tolist()
-    buf = pool.get(k, dev) if pool is not None else torch.empty(
+        return mk, None, 0, [0] * cuts
+    scratch = torch.empty(int(L.raw("sga_mask_list_words", n)), dtype=torch.int32, device=mk.device)
+    totals = torch.empty(1 + cuts, dtype=torch.int64, device=mk.device)
+    L.call("sga_mask_totals", L.ptr(mk), n, L.ptr(scratch), step, cuts, L.ptr(totals), L.stream())
+    k, *before = totals.tolist()
+    return mk, scratch, k, before
+
+
+def compact_mask_u8(mask_u8, pool: Optional[IndexPool] = None, step=0, cuts=0):
+    """Ascending int32 positions of the non-zero bytes of ``mask_u8``
+    (``sga/support.py:57-99``): one counting sweep, one host read of k (the
+    reference syncs on the count too), one ordered fill sweep.  With ``cuts`` the
+    same read also brings how many positions lie before ``step``, ``2 * step``, ...:
+    returns ``(idx, [that many ints])``."""
+    mk, scratch, k, before = mask_totals(mask_u8, step, cuts)
+    dev, n = mk.device, mk.numel()
+    buf = pool.get(k, dev) if pool is not None and n else torch.empty(
         k, dtype=torch.int32, device=dev)
     if k:
-        L.call("sga_mask_fill", L.ptr(mk), n, L.ptr(counts), L.ptr(buf), buf.numel(),
-               L.stream())
+        L.call("sga_mask_list", L.ptr(mk), n, L.ptr(scratch), L.ptr(buf), buf.numel(), None, 1.0,
+               None, None, 0, L.stream())
     return (buf[:k], before) if cuts else buf[:k]
 
 
