@@ -223,7 +223,7 @@ __device__ __forceinline__ void now_cols_write(const NowCols& c, int job, sga_se
     segs[i].bc2 = c.bc2[s];
   }
 }
-// What a sample's key is formed with, while the table is being written.
+// What the keys are formed with that a launch forms while it writes the table.
 struct ColsOf {
   const NowCols* cols;
   int job;
@@ -251,16 +251,19 @@ static inline void launch_seg_dir(const sga_segment* segs, int n_segs, int64_t n
 // that intersects it (one, but for the few slabs that hold a boundary) with
 // that segment's hyper-parameters as scalar operands.  `sc` was placed on the
 // slab's chunk or the slab (seek_uniform, seek_wave) and is only ever moved by uniform seeks.
-// key[] comes in zeroed; quads past n stay zero.
-template <int SCORE, bool FULL>
+// key[] comes in zeroed; quads past n stay zero.  now: see ColsOf; `sc` was placed with it as well.
+template <int SCORE, bool FULL, class Now = NoCols>
 __device__ __forceinline__ void slab_score_keys(SegCursor& sc, int adams, int64_t i, int64_t n,
                                                 const float q[4], const float p[4],
                                                 const float m[4], const float v[4],
-                                                uint32_t key[4]) {
+                                                uint32_t key[4], const Now& now = Now()) {
   const int64_t s0 = uniform_i64(i);
   int64_t s1 = s0 + kWave * kVec;
   if (!FULL && s1 > n) s1 = n;
-  if (s0 >= sc.hi) sc.advance_uniform(s0);   // slabs of a chunk ascend from where it began
+  if (s0 >= sc.hi) {                         // slabs of a chunk ascend from where it began
+    sc.advance_uniform(s0);
+    now.into(sc.h, sc.at);
+  }
   for (;;) {
     Hyper h = sc.h;
     if (adams) { h.bc1 = 1.0f; h.bc2 = 1.0f; }
@@ -278,6 +281,7 @@ __device__ __forceinline__ void slab_score_keys(SegCursor& sc, int adams, int64_
     const int64_t pos = sc.hi;
     if (pos >= s1) break;
     sc.advance_uniform(pos);
+    now.into(sc.h, sc.at);
     if (sc.hi <= pos) break;              // the table does not tile [0, n): stop
   }
 }

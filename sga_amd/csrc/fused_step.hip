@@ -76,9 +76,9 @@ struct SrcFused {
     if (kNeedP) w.p = ldraw_f32<FULL, KEEP>(p + ck.sh, i, n, vec);
     if (kNeedV && !adams) w.v = ldraw_f32<FULL, KEEP>(v + ck.sh, i, n, vec);
   }
-  template <bool FULL>
+  template <bool FULL, class Now = NoCols>
   __device__ __forceinline__ void keys(const Chunk& ck, int64_t i, int64_t n, const Raw& w,
-                                       uint32_t key[4]) {
+                                       uint32_t key[4], const Now& now = Now()) {
     float q[4] = {0, 0, 0, 0}, rr[4] = {0, 0, 0, 0};
     float pp[4] = {0, 0, 0, 0}, mm[4] = {0, 0, 0, 0}, vv[4] = {0, 0, 0, 0};
     if (kNeedG && has_g()) unpack_g<BF16G, FULL>(w.g, q);
@@ -100,7 +100,7 @@ struct SrcFused {
     } else {
       unpack_f32(w.v, vv);
     }
-    slab_score_keys<SCORE, FULL>(sc, adams, i, n, q, pp, mm, vv, key);
+    slab_score_keys<SCORE, FULL>(sc, adams, i, n, q, pp, mm, vv, key, now);
   }
   template <bool FULL = false, class Cols = NoCols>
   __device__ __forceinline__ void load(int64_t i, int64_t n, uint32_t key[4], const Cols& cols = Cols()) {

@@ -521,9 +521,9 @@ struct SrcReplay {
 #pragma unroll
     for (int e = 0; e < 4; ++e) q[e] = (gd[e] + rr[e]) * coef;
   }
-  template <bool FULL>
+  template <bool FULL, class Now = NoCols>
   __device__ __forceinline__ void keys(const Chunk& ck, int64_t i, int64_t n, const Raw& t,
-                                       uint32_t key[4]) {
+                                       uint32_t key[4], const Now& = Now()) {
     float gd[4] = {0, 0, 0, 0}, rr[4] = {0, 0, 0, 0}, q[4] = {0, 0, 0, 0};
     float ww[4] = {0, 0, 0, 0}, mm[4] = {0, 0, 0, 0}, vv[4] = {0, 0, 0, 0};
     if (kNeedG) {
@@ -923,7 +923,7 @@ static int run_reselect(const void* g, int64_t n, const sga_segment* segs, int n
     chain_begin(B, dj, s);
   } else {
     per_score([&](auto& srcs, const SelBatch& sub) {
-      launch_sample_pick<true>(srcs, sub, dirs_of(srcs, sub), {}, kBracketSigmas, s);
+      launch_sample_pick(srcs, sub, dirs_of(srcs, sub), {}, kBracketSigmas, s);
     });
     per_score([&](auto& srcs, const SelBatch& sub) { launch_sample_fine(srcs, sub, kBracketSigmas, s); });
     per_score([&](auto& srcs, const SelBatch& sub) { chain_sweeps(srcs, sub, s); });

@@ -48,7 +48,7 @@ struct SelState {
   uint32_t finish_ticket; // k_small_finish: workgroups that have begun; the first one judges the bracket ...
   uint32_t verdict;     // ... 1: it holds the k-th key, 2: all of them go over the data again
   uint32_t redo_step;   // passes of that which are done
-  uint32_t sampled[16]; // k_sample_pick: the launch that a workgroup of the sample has finished in
+  uint32_t sampled[16]; // sample_pick_body: the launch that a workgroup of the sample has finished in
   uint32_t pad_[12];
 };
 static_assert(sizeof(SelState) == 256, "whole cache lines");
@@ -66,7 +66,7 @@ SGA_HOST_DEVICE static inline uint32_t sampled_key(unsigned long long word, int 
 // zero as a cleared mark is, and spread over all 32 bits (consecutive small numbers are what index lists, counts
 // and flags in recycled memory look like).  A recorded graph repeats its numbers: its marks are zero again at
 // every start because the pick clears them and so does the kernel behind it (an early pick's clearing may come
-// before the last mark).
+// before the last mark); those of the small buckets' front are cleared by the kernel behind it alone.
 SGA_HOST_DEVICE static inline uint32_t launch_number(uint32_t count) { return (2u * count + 1u) * 0x9E3779B1u; }
 constexpr int kStateWords = sizeof(SelState) / 8;
 constexpr int kBracketWord = offsetof(SelState, t_lo) / 8;

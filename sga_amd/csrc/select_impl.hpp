@@ -249,8 +249,9 @@ struct SrcF32 {                 // |x| of an fp32 score array
   __device__ __forceinline__ void fetch(const Chunk&, int64_t i, int64_t n, Raw& r) {
     r = ldraw_f32<FULL, KEEP>(x, i, n, vec);
   }
-  template <bool FULL>
-  __device__ __forceinline__ void keys(const Chunk&, int64_t, int64_t, const Raw& r, uint32_t key[4]) {
+  template <bool FULL, class Now = NoCols>
+  __device__ __forceinline__ void keys(const Chunk&, int64_t, int64_t, const Raw& r, uint32_t key[4],
+                                       const Now& = Now()) {
     key[0] = abs_key(r.x); key[1] = abs_key(r.y); key[2] = abs_key(r.z); key[3] = abs_key(r.w);
     neg |= (uint32_t)((r.x < 0.0f) | (r.y < 0.0f) | (r.z < 0.0f) | (r.w < 0.0f));
   }
@@ -325,6 +326,12 @@ __device__ __forceinline__ uint32_t ld_agent(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void st_agent(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ unsigned long long ld_agent64(const unsigned long long* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_agent64(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 // Every such store and atomic of the workgroup has landed when this returns.
@@ -502,8 +509,8 @@ __global__ __launch_bounds__(kBlock) void k_level_scan(ChainJobs jobs) {
 }
 
 // Per-chunk (1024 elements, one wave) counts of keys above / equal to the
-// threshold, by wave `wave` of `wstride`.
-template <class Src>
+// threshold, by wave `wave` of `wstride`.  ROLL: a slab at a time, for kernels with few registers to spare.
+template <class Src, bool ROLL = false>
 __device__ __forceinline__ void tile_count_body(Src& src, const ChainJob& J, uint32_t T, int64_t tile_base,
                                                 int64_t wave, int64_t wstride) {
   const int64_t n = J.n;
@@ -512,7 +519,8 @@ __device__ __forceinline__ void tile_count_body(Src& src, const ChainJob& J, uin
   const int64_t n_chunks = cdiv64(n, kChunk);
   for (int64_t c = wave; c < n_chunks; c += wstride) {
     uint32_t cg = 0, ce = 0;
-    if (src.vec && (c + 1) * kChunk <= n) {
+    const bool full = src.vec && (c + 1) * kChunk <= n;
+    if (!ROLL && full) {
       uint32_t key[kChunkIters][4];
 #pragma unroll
       for (int it = 0; it < kChunkIters; ++it)
@@ -522,11 +530,13 @@ __device__ __forceinline__ void tile_count_body(Src& src, const ChainJob& J, uin
 #pragma unroll
         for (int e = 0; e < 4; ++e) { cg += key[it][e] > T; ce += key[it][e] == T; }
     } else {
-#pragma unroll
+      constexpr int kUnroll = ROLL ? 1 : kChunkIters;
+#pragma unroll kUnroll
       for (int it = 0; it < kChunkIters; ++it) {
         const int64_t i = c * kChunk + it * (kWave * kVec) + lane_id() * kVec;
         uint32_t key[4] = {0, 0, 0, 0};
-        if (i < n) src.template load<false>(i, n, key);
+        if (ROLL && full) src.template load<true>(i, n, key);
+        else if (i < n) src.template load<false>(i, n, key);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const bool valid = i + e < n;
@@ -807,7 +817,7 @@ struct SelBatch {
     J = ChainJob{};
     J.st = ws.st; J.aux = ws.aux; J.hist = ws.hist;
     J.tile_gt = ws.tile_gt; J.tile_eq = ws.tile_eq; J.blk_gt = ws.blk_gt; J.blk_eq = ws.blk_eq;
-    J.sample = ws.sample ? ws.sample : ws.small_idx; J.rel = ws.rel; J.seg_cnt = ws.seg_cnt; J.seg_idx = ws.seg_idx; J.seg_key = ws.seg_key;
+    J.sample = ws.sample; J.rel = ws.rel; J.seg_cnt = ws.seg_cnt; J.seg_idx = ws.seg_idx; J.seg_key = ws.seg_key;
     J.cand_idx = ws.cand_idx; J.cand_key = ws.cand_key;
     J.small_idx = ws.small_idx; J.small_key = ws.small_key;
     J.n = n; J.n_tiles = cdiv64(n, kChunk);
@@ -908,6 +918,19 @@ __device__ __forceinline__ void seg_dirs(const SegDirJobs& dirs, int job, int t0
   for (int b = t0; b < nb; b += step) D.dir[b] = seg_dir_entry(D.segs, D.n_segs, b);
 }
 
+// ... and what a select's first kernel carries for the tables' changing columns.
+template <class Cols>
+__device__ __forceinline__ void keep_tables(const SegDirJobs& dirs, const Cols& cols, int t0, int step) {
+  seg_dirs(dirs, blockIdx.y, t0, step);
+  if constexpr (std::is_same<Cols, NowCols>::value)
+    now_cols_write(cols, blockIdx.y, const_cast<sga_segment*>(dirs.j[blockIdx.y].segs), t0, step);
+}
+// Small buckets: the bracket on its way from the pick to the sweep, a copy beside each segment counter (on a line of
+// its own), either end with the launch's number above it.
+__device__ __forceinline__ unsigned long long* small_bracket_copy(const ChainJob& J, int c) {
+  return reinterpret_cast<unsigned long long*>(J.seg_cnt + c * kSmallSegStride + kSmallSegStride / 2);
+}
+
 // First kernel of a select of the large buckets that goes by radix passes alone.
 static __global__ __launch_bounds__(kBlock) void k_chain_begin(ChainJobs jobs, SegDirJobs dirs) {
   const ChainJob& J = jobs.j[blockIdx.y];
@@ -967,6 +990,11 @@ __device__ __forceinline__ RankEnds bracket_ranks(double k, double n, double ns,
 // missed in 32 of 1000 draws of 40 M coordinates at 10 % with four sigma, and in 12 with eight (the fine
 // sample's own five, halved); a wider coarse bracket costs the fine one a few keys of resolution.
 //
+// COARSE: the large buckets' launch, k_sample_pick; the other one is k_small_front (small_select.hpp), in which others
+// wait for the bracket: there the first workgroup clears the state and the segment counters before it leaves its mark,
+// so that no pick comes before that, and a pick writes the bracket and its copies alone (a second pick writes the
+// same; what others have counted meanwhile stays).
+//
 // The workgroups behind those of the sample keep house: counters and histograms of the kernels behind this one,
 // the directories of the segment tables (dirs.j[job].dir null: none wanted), the tables' changing columns (cols; the
 // sample forms its keys with those that it was handed, whatever the tables hold by then).
@@ -974,19 +1002,8 @@ constexpr int kSampleGroups = 16;
 constexpr int kPickBits = 13, kPickShift = 31 - kPickBits;
 constexpr uint32_t kHeavyBin = 3;                    // a half misses the 100 M case above
 template <class Src, bool COARSE>
-__global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
-                                                       typename Src::Cols cols, uint32_t launch,
-                                                       double sigmas) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  if (blockIdx.x >= kSampleGroups) {
-    const int t0 = (blockIdx.x - kSampleGroups) * kWide + threadIdx.x, step = (gridDim.x - kSampleGroups) * kWide;
-    if (COARSE) clear_large(J, t0, step, true);
-    else if (t0 < kSmallSegs) J.seg_cnt[t0 * kSmallSegStride] = 0u;
-    seg_dirs(dirs, blockIdx.y, t0, step);
-    if constexpr (std::is_same<typename Src::Cols, NowCols>::value)
-      now_cols_write(cols, blockIdx.y, const_cast<sga_segment*>(dirs.j[blockIdx.y].segs), t0, step);
-    return;
-  }
+__device__ __forceinline__ void sample_pick_body(const SrcPack<Src>& srcs, const ChainJob& J,
+                                                 const typename Src::Cols& cols, uint32_t launch, double sigmas) {
   __shared__ __align__(16) uint32_t s_h[2][kBinsBig];
   __shared__ __align__(16) uint32_t s_list[2][kWideList];
   __shared__ uint32_t s_cnt[2], s_out[2][3], s_all, s_heavy, s_rank[2], s_open[2], s_sub[2][kWave];
@@ -995,7 +1012,15 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
   SelState* st = J.st;
   const int64_t n = J.n;
   const int n_sv = (int)small_sample_vecs(n);
-  unsigned long long* __restrict__ sample = reinterpret_cast<unsigned long long*>(J.sample);
+  // small: the histograms, which only a missed bracket needs (the list may be written while a second picks)
+  unsigned long long* __restrict__ sample = reinterpret_cast<unsigned long long*>(COARSE ? J.sample : J.hist);
+  static_assert(kHistStride * 2 >= kSmallSampleMax * 4, "two keys a word");
+  if (!COARSE && blockIdx.x == 0) {
+    constexpr uint32_t MARKS = offsetof(SelState, sampled) / 4;
+    const uint32_t t = threadIdx.x;
+    if (t < kSmallSegs) st_agent(&J.seg_cnt[t * kSmallSegStride], 0u);
+    if (t < sizeof(SelState) / 4 && t - MARKS >= kSampleGroups) st_agent(reinterpret_cast<uint32_t*>(st) + t, t == 0 ? J.k : 0u);
+  }
   {
     const int per = (n_sv + kSampleGroups - 1) / kSampleGroups, j = (int)blockIdx.x * per + (int)threadIdx.x;
     if ((int)threadIdx.x < per && j < n_sv) {
@@ -1011,8 +1036,7 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
         src.template load<false>(i, n, key);
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        __hip_atomic_store(&sample[2 * j + h], (unsigned long long)key[2 * h + 1] << 32 | key[2 * h], __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+        st_agent64(&sample[2 * j + h], (unsigned long long)key[2 * h + 1] << 32 | key[2 * h]);
     }
   }
   const uint32_t ns = (uint32_t)(n_sv * 4);
@@ -1061,7 +1085,7 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const unsigned long long q =
-          j < n_sv ? __hip_atomic_load(&sample[2 * j + h], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+          j < n_sv ? ld_agent64(&sample[2 * j + h]) : 0ull;
       key[u][2 * h] = sampled_key(q, 0);
       key[u][2 * h + 1] = sampled_key(q, 1);
     }
@@ -1173,9 +1197,30 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
       if (!open_lo) t_lo = w > 0 ? s_out[1][0] : bin[1];
     }
   }
-  if (threadIdx.x < kStateWords)
-    __hip_atomic_store(reinterpret_cast<unsigned long long*>(st) + threadIdx.x, picked_word(threadIdx.x, J.k, t_lo, t_hi),
-                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (COARSE) {
+    if (threadIdx.x < kStateWords)
+      st_agent64(reinterpret_cast<unsigned long long*>(st) + threadIdx.x, picked_word(threadIdx.x, J.k, t_lo, t_hi));
+  } else {
+    if (threadIdx.x < kSmallSegs) {
+      unsigned long long* w = small_bracket_copy(J, (int)threadIdx.x);
+      st_agent64(w, (unsigned long long)launch << 32 | t_lo);
+      st_agent64(w + 1, (unsigned long long)launch << 32 | t_hi);
+    }
+    if (threadIdx.x == 0)
+      st_agent64(reinterpret_cast<unsigned long long*>(st) + kBracketWord, picked_word(kBracketWord, J.k, t_lo, t_hi));
+  }
+}
+template <class Src>
+__global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
+                                                       typename Src::Cols cols, uint32_t launch, double sigmas) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  if (blockIdx.x < kSampleGroups) {
+    sample_pick_body<Src, true>(srcs, J, cols, launch, sigmas);
+    return;
+  }
+  const int t0 = (blockIdx.x - kSampleGroups) * kWide + threadIdx.x, step = (gridDim.x - kSampleGroups) * kWide;
+  clear_large(J, t0, step, true);
+  keep_tables(dirs, cols, t0, step);
 }
 
 // The fine sample of a large bucket: only how its keys fall relative to the coarse bracket is kept --
@@ -2236,13 +2281,13 @@ static inline void chain_begin(const SelBatch& B, const SegDirJobs& dirs, hipStr
 }
 // Number of the next launch that takes a sample: one count for the whole library (select.hip).
 uint32_t next_launch();
-template <bool COARSE, class Src>
+template <class Src>
 static inline void launch_sample_pick(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
                                       const typename Src::Cols& cols, double sigmas, hipStream_t s) {
   static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + sizeof(typename Src::Cols) + 64 <= 4096,
                 "the operands of a batched chain kernel travel in its 4 KiB of kernel arguments");
-  hipLaunchKernelGGL((k_sample_pick<Src, COARSE>), B.grid(kSampleGroups + (COARSE ? 16 : 1)), dim3(kWide), 0, s, srcs,
-                     B.jobs, dirs, cols, next_launch(), sigmas);
+  hipLaunchKernelGGL((k_sample_pick<Src>), B.grid(kSampleGroups + 16), dim3(kWide), 0, s, srcs, B.jobs, dirs, cols,
+                     next_launch(), sigmas);
 }
 template <class Src>
 static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& B, double sigmas, hipStream_t s) {
@@ -2253,7 +2298,7 @@ static inline void launch_sample_fine(const SrcPack<Src>& srcs, const SelBatch& 
 template <class Src>
 static inline void chain_bracket(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
                                  const typename Src::Cols& cols, double sigmas, hipStream_t s) {
-  launch_sample_pick<true>(srcs, B, dirs, cols, sigmas, s);
+  launch_sample_pick(srcs, B, dirs, cols, sigmas, s);
   launch_sample_fine(srcs, B, sigmas, s);
 }
 // keep (sources that a writing pass reads again): see bracket_chunk

@@ -1,8 +1,9 @@
-// Exact top-k of a bucket of up to kSmallTiles chunks (8.4 M coordinates) in three launches:
-//   k_sample_pick     8 K to 16 K sample keys, and the bracket of the k-th key from them (and the
-//                     directory of the segment table)
-//   k_small_sweep     the one sweep over the data: per-chunk counts above the bracket, and a list
-//                     of the few keys inside it
+// Exact top-k of a bucket of up to kSmallTiles chunks (8.4 M coordinates) in two or three launches:
+//   k_small_front     8 K to 16 K sample keys, the bracket of the k-th key from them (and the
+//                     directory of the segment table), and in the same launch, where its workgroups are all
+//                     resident at once, the one sweep over the data: per-chunk counts above the bracket, and a
+//                     list of the few keys inside it
+//   k_small_sweep     that sweep where they are not
 //   k_small_finish    one workgroup: exact threshold from the list, ties to grant, and the
 //                     per-chunk (selected, ties) prefixes the writing pass starts from
 // followed by the caller's writing pass (final sweep, k_write_mask, k_write_bits), which forms the
@@ -16,8 +17,11 @@
 // Measured through the public entry points, us per call, before -> with this path:
 //   fused step, |g + r|, 1 %, 261 K elements bf16   84 -> 55       4.2 M elements fp32   184 -> 91
 //   select_topk_flat, 3 M scores, 1 %              168 -> 69
-// (Kernels of the 4.2 M step, fp32 gradients, each pass after a wait: sample and pick 12.5 us, sweep 11.4, finish
-// 20.6, final sweep 27.2.)
+// (Kernels of the 4.2 M step, fp32 gradients: front 18, finish 16, final sweep 27.  In the front, us after its start:
+// sample loaded 4 to 5, bracket 10, seen by the sweep 10.5, its list reserved 13.5, launch over 17; the finish is
+// bound by one workgroup's instruction issue and LDS atomics: loads 3, totals 1, histogram of 35 K entries 4, chunk
+// counts 6, edge and prefixes 2.  Adding the list to a histogram in the sweep instead moves its 4 us to 5 of
+// device-wide atomics there; counting by a bit per entry is no faster below 8 M.)
 //
 // The result is exact for any sample: where the bracket misses the k-th key the finishing launch goes
 // over the data itself, with all of its workgroups (small_redo).
@@ -41,92 +45,187 @@ __host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles, int cpw)
   return s;
 }
 
-// The sweep: a workgroup per chunk and a wave per slab, so that a bucket of a few hundred chunks still
-// reaches every SIMD; counts above the bracket, keys inside it to the list (one reservation per chunk).
-// Keys equal to the bracket's lower end are counted per chunk and not
+// What a chunk's two words carry from the sweep to the finish, numbers up to 1024 in halves whose sums over the eight
+// chunks of a thread fit (an instruction per chunk is 0.07 us of the finish at 8 M coordinates):
+//   a   keys above the bracket | ten bits of the bracket's tag | listed keys
+//   b   keys equal to the lower end | a value was negative | no bracket, or no room | eight more of the tag | non-finite keys
+struct SmallChunk {
+  static constexpr uint32_t kNumbers = 0x07FF07FFu, kNegative = 1u << 11, kLost = 1u << 12;
+  uint32_t a, b;
+  // the words of a chunk without a key in it, under the bracket [lo, hi)
+  static __device__ __forceinline__ SmallChunk none(uint32_t lo, uint32_t hi) {
+    uint32_t x = lo * 0x9E3779B1u ^ hi * 0x85EBCA6Bu;
+    x = (x ^ (x >> 15)) * 0x2C1B3C6Du;
+    return SmallChunk{(x & 0xF800F800u), ((x << 8) & 0xF8000000u) | ((x >> 3) & 0xE000u)};
+  }
+};
+
+// Sample, bracket and the one sweep over the data, one launch: the first kSampleGroups workgroups of a job take the
+// sample and one of them the bracket (sample_pick_body), one keeps house (directory and columns of the segment
+// table), the others sweep.  These request their data and form its keys while the bracket is on its way, and then
+// look for it in one of kSmallSegs copies.  Counts above the bracket, keys inside it to the list (one reservation per
+// workgroup).  Keys equal to the bracket's lower end are counted per chunk and not
 // listed: a plateau of equal keys (zeros, momenta that have decayed to the last denormal) puts the
 // lower end on itself, and the one workgroup behind the sweep would walk a list as long as the bucket
 // (|m| after a thousand sparse steps, 1.7 M coordinates: 889 us, 86 like this).
-// Chunks per workgroup (CPW): one up to kSweepTiles chunks and for the scores that are a chain of arithmetic;
-// beyond, four, whose loads are in flight together (a reservation per 4096 coordinates, half the waves).
-// Step of 261 K coordinates with one / four 36.1 / 38.8 us, 2 M 59.2 / 62.3, 8.3 M 145 / 140; `update`
-// 261 K 50.5 / 57.4, 8.3 M 159 / 166; select of 3 M scores 70.4 / 67.4.
-constexpr int64_t kSweepTiles = 2048;
-template <class Src, int CPW>
-__global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, ChainJobs jobs) {
-  const ChainJob& J = jobs.j[blockIdx.y];
-  const int64_t n = J.n, n_chunks = J.n_tiles, c0 = (int64_t)blockIdx.x * CPW;
+//
+// One launch or two: the waiting workgroups hold their registers and LDS, one on a CU, so they go along where they are
+// no more than the CUs (kFrontSweeps: 4.2 M coordinates, 1 M of a score that is a chain of arithmetic).  With twice
+// as many the ones behind begin when the first are done, which two launches are faster than (`update` 8.4 M one launch
+// 155 us, two 136; twelve buckets of 20 M 493 / 291).  Two launches -> one, us: step of 261 K 28.8 -> 27.6, `update`
+// 43.6 -> 39.9, 3 M 60.1 -> 56.3, 4.2 M fp32 65.9 -> 62.9; selects of 1 M at 10 % 59.1 -> 54.6, of 3 M 56.6 -> 55.1.
+// Slabs per wave (SPW): one up to kFrontTiles chunks (kSweepTiles for a sweep of its own) and for the scores that are a
+// chain of arithmetic; beyond, four, whose loads are in flight together.
+// In the front a workgroup's entries leave by LDS, whole lines at a time (few lanes of a store hold one: 5 us of the
+// front at 4.2 M, 3.5 so); a sweep of its own has other workgroups to fill that time.
+//
+// Nobody waits for long: a sweeping workgroup looks kBracketLooks times (some milliseconds; those that it waits for
+// wait for nobody and come before it in the grid, so that it does not happen) and then says in its chunks' words that
+// it had none.  The launch's number makes a copy this launch's; k_small_finish clears copies and marks for recorded
+// graphs, which repeat their numbers.  Memory that happens to hold the number may give a workgroup a bracket that is
+// not the one in the state, or clear a segment's counter after somebody has added to it: tags and counts then do not
+// agree, or a reservation does not fit, and the finish goes over the data itself.
+constexpr int64_t kSweepTiles = 2048, kFrontTiles = 1024, kFrontSweeps = 256;
+constexpr int kBracketLooks = 4096;
+constexpr int kSweepList = 2048;                     // entries of a workgroup that are gathered in LDS
+template <class Src, int WAVES, int SPW, bool WAIT, class Now>
+__device__ __forceinline__ void small_sweep_body(Src src, const ChainJob& J, const Now& now, uint32_t launch, int64_t blk) {
+  constexpr int ROUND = WAVES / kChunkIters, CPW = ROUND * SPW, SLABS = WAVES * SPW;
+  static_assert(SLABS <= kWave, "a lane per slab");
+  __shared__ uint32_t s_hi[SLABS], s_eq[SLABS], s_cnt[SLABS], s_nf[SLABS], s_got[3], s_base, s_fit;
+  __shared__ uint32_t s_lkey[WAIT ? kSweepList : 1], s_lidx[WAIT ? kSweepList : 1];
+  const int64_t n = J.n, n_chunks = J.n_tiles, c0 = blk * CPW;
   if (c0 >= n_chunks) return;                         // a smaller job of the batch
-  __shared__ uint32_t s_hi[CPW][kChunkIters], s_eq[CPW][kChunkIters], s_cnt[kChunkIters], s_nf[kChunkIters], s_base;
-  static_assert(kChunkIters == kChunksPerBlock && CPW <= kWave, "a wave per slab");
-  SelState* __restrict__ st = J.st;
-  if (blockIdx.x == 0 && threadIdx.x < kSampleGroups) st->sampled[threadIdx.x] = 0u;      // see launch_number
-  Src src = srcs.s[blockIdx.y];
-  const int64_t i0 = c0 * kChunk + uniform_i32(wave_id()) * (kWave * kVec);
-  typename Src::Raw raw[CPW];
+  const int w = uniform_i32(wave_id());
+  const int64_t c1 = c0 + w / kChunkIters, i1 = c1 * kChunk + (w % kChunkIters) * (kWave * kVec);
+  uint32_t left_lo = 0, left_hi = 0;                  // by the launch before
+  if (!WAIT) { left_lo = J.st->t_lo; left_hi = J.st->t_hi; }
+  typename Src::Raw raw[SPW];
 #pragma unroll
-  for (int u = 0; u < CPW; ++u) {
-    const typename Src::Chunk ck = src.chunk_begin(c0 + u);
-    const int64_t i = i0 + u * kChunk + lane_id() * kVec;
-    if (src.vec && (c0 + u + 1) * kChunk <= n) src.template fetch<true, true>(ck, i, n, raw[u]);  // read again soon
+  for (int u = 0; u < SPW; ++u) {
+    const int64_t c = c1 + u * ROUND, i = i1 + u * ROUND * kChunk + lane_id() * kVec;
+    const typename Src::Chunk ck = src.chunk_begin(c);
+    if (src.vec && (c + 1) * kChunk <= n) src.template fetch<true, true>(ck, i, n, raw[u]);       // read again soon
     else if (i < n) src.template fetch<false>(ck, i, n, raw[u]);
   }
-  src.slab_hyper(i0);
-  const uint32_t T_LO = st->t_lo, T_HI = st->t_hi;
-  uint32_t key[CPW][4], cnt = 0, nf = 0;
-  Ballot4 cand[CPW];
+  uint32_t key[SPW][4], nf[SPW];
 #pragma unroll
-  for (int u = 0; u < CPW; ++u) {
-    const typename Src::Chunk ck = src.chunk_begin(c0 + u);
-    const int64_t i = i0 + u * kChunk + lane_id() * kVec;
-    const bool full = src.vec && (c0 + u + 1) * kChunk <= n;
-    if (u > 0) src.slab_hyper(i0 + u * kChunk);
+  for (int u = 0; u < SPW; ++u) {
+    const int64_t c = c1 + u * ROUND, i0 = i1 + u * ROUND * kChunk, i = i0 + lane_id() * kVec;
+    const typename Src::Chunk ck = src.chunk_begin(c);
     key[u][0] = key[u][1] = key[u][2] = key[u][3] = 0u;
-    if (full) src.template keys<true>(ck, i, n, raw[u], key[u]);
-    else if (i < n) src.template keys<false>(ck, i, n, raw[u], key[u]);
+    const bool full = (c + 1) * kChunk <= n;
+    src.slab_hyper(i0);
+    if constexpr (Src::kHyper) now.into(src.sc.h, src.sc.at);
+    if (src.vec && full) src.template keys<true>(ck, i, n, raw[u], key[u], now);
+    else if (i < n) src.template keys<false>(ck, i, n, raw[u], key[u], now);
+    nf[u] = 0u;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if (!full && i + e >= n) key[u][e] = ~0u;       // below every bound, as the signed number it is compared as
+      nf[u] += (uint32_t)__popcll(ballot64((int32_t)key[u][e] >= 0x7F800000));
+    }
+  }
+  const uint32_t neg = ballot64(src_negative(src) != 0u) != 0ull ? 0x80000000u : 0u;
+  if (WAIT && threadIdx.x == 0) {
+    const unsigned long long* from = small_bracket_copy(J, (int)(blk % kSmallSegs));
+    unsigned long long lo = 0, hi = 0;
+    bool there = false;
+    for (int t = 0; t < kBracketLooks && !there; ++t) {
+      if (t) __builtin_amdgcn_s_sleep(4);
+      lo = ld_agent64(from);
+      hi = ld_agent64(from + 1);
+      there = (uint32_t)(lo >> 32) == launch && (uint32_t)(hi >> 32) == launch;
+    }
+    s_got[0] = there ? (uint32_t)lo : 0x7FFFFFFFu;    // without a bracket no key is listed
+    s_got[1] = there ? (uint32_t)hi : 0x80000000u;
+    s_got[2] = there;
+  }
+  if (WAIT) __syncthreads();
+  const uint32_t T_LO = WAIT ? s_got[0] : left_lo, T_HI = WAIT ? s_got[1] : left_hi;
+  const int32_t below = (int32_t)T_LO, top = (int32_t)(T_HI - 1u);
+  Ballot4 cand[SPW];
+#pragma unroll
+  for (int u = 0; u < SPW; ++u) {
     uint32_t hi = 0, eq = 0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const uint64_t valid = full ? ~0ull : ballot64(i + e < n);
-      const uint64_t above = ballot64(key[u][e] >= T_HI) & valid;
-      cand[u].m[e] = ballot64(key[u][e] > T_LO) & valid & ~above;
+      const uint64_t above = ballot64((int32_t)key[u][e] > top);
+      cand[u].m[e] = ballot64((int32_t)key[u][e] > below) & ~above;
       hi += (uint32_t)__popcll(above);
-      eq += (uint32_t)__popcll(ballot64(key[u][e] == T_LO) & valid);
-      nf += (uint32_t)__popcll(ballot64(key[u][e] >= 0x7F800000u) & valid);
+      eq += (uint32_t)__popcll(ballot64(key[u][e] == T_LO));
     }
-    cnt += cand[u].count();
-    if (lane_id() == 0) { s_hi[u][wave_id()] = hi; s_eq[u][wave_id()] = eq; }
-  }
-  const bool neg = ballot64(src_negative(src) != 0u) != 0ull;
-  if (lane_id() == 0) {
-    s_cnt[wave_id()] = cnt;
-    s_nf[wave_id()] = nf | (neg ? 0x80000000u : 0u);
+    if (lane_id() == 0) {
+      const int q = u * WAVES + w;
+      s_hi[q] = hi; s_eq[q] = eq; s_cnt[q] = cand[u].count(); s_nf[q] = nf[u] | neg;
+    }
   }
   __syncthreads();
-  const SmallGeom geo = small_geom(n_chunks, CPW);
-  const uint32_t seg = blockIdx.x % geo.segs;
-  if (threadIdx.x < CPW && c0 + (int)threadIdx.x < n_chunks) {
-    const uint32_t* h = s_hi[threadIdx.x];
-    const uint32_t* q = s_eq[threadIdx.x];
-    J.tile_gt[c0 + threadIdx.x] = h[0] + h[1] + h[2] + h[3];
-    J.tile_eq[c0 + threadIdx.x] = q[0] + q[1] + q[2] + q[3];
-  }
-  if (threadIdx.x == 0) {
-    const uint32_t all = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-    const uint32_t f = (s_nf[0] + s_nf[1] + s_nf[2] + s_nf[3]) & 0x7FFFFFFFu;
-    if (all) s_base = atomicAdd(&J.seg_cnt[seg * kSmallSegStride], all);
-    if (f) atomicAdd(&st->nonfinite, f);
-    if ((s_nf[0] | s_nf[1] | s_nf[2] | s_nf[3]) & 0x80000000u) raise_negative(st);
-  }
-  __syncthreads();
-  uint32_t run = seg * geo.cap + s_base;
-  for (int w = 0; w < wave_id(); ++w) run += s_cnt[w];
+  // every wave sums the slabs' counts for itself; the first one reserves and writes the chunks' words meanwhile
+  const uint32_t mine = lane_id() < SLABS ? s_cnt[lane_id()] : 0u, incl = wave_incl_scan(mine);
+  const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+  if (w == 0) {
+    const SmallGeom geo = small_geom(n_chunks, CPW);
+    const uint32_t seg = (uint32_t)(blk % geo.segs);
+    uint32_t base = 0;
+    if (lane_id() == 0 && all) base = atomicAdd(&J.seg_cnt[seg * kSmallSegStride], all);
+    base = (uint32_t)uniform_i32((int)base);
+    const bool fit = base <= geo.cap && all <= geo.cap - base;
+    if (lane_id() == 0) { s_base = seg * geo.cap + base; s_fit = fit; }
+    if (lane_id() < CPW && c0 + lane_id() < n_chunks) {
+      uint32_t hi = 0, eq = 0, cnt = 0, bad = 0, minus = 0;
 #pragma unroll
-  for (int u = 0; u < CPW; ++u)
-    ballot_append(cand[u], run, [&](uint32_t pos, int e) {
-      J.small_idx[pos] = (uint32_t)(i0 + u * kChunk + lane_id() * kVec + e);
-      J.small_key[pos] = key[u][e];
-    });
+      for (int j = 0; j < kChunkIters; ++j) {
+        const int q = lane_id() * kChunkIters + j;
+        hi += s_hi[q]; eq += s_eq[q]; cnt += s_cnt[q];
+        bad += s_nf[q] & 0x7FFFFFFFu; minus |= s_nf[q] >> 31;
+      }
+      SmallChunk ch = SmallChunk::none(T_LO, T_HI);
+      ch.a |= hi | cnt << 16;
+      ch.b |= eq | bad << 16 | (minus ? SmallChunk::kNegative : 0u) | (!fit || (WAIT && s_got[2] == 0u) ? SmallChunk::kLost : 0u);
+      J.tile_gt[c0 + lane_id()] = ch.a;
+      J.tile_eq[c0 + lane_id()] = ch.b;
+    }
+  }
+  const bool via_lds = WAIT && all <= (uint32_t)kSweepList;
+  if (!via_lds) __syncthreads();                      // uniform; the list goes straight to its place then
+  if (!via_lds && !s_fit) return;
+#pragma unroll
+  for (int u = 0; u < SPW; ++u) {
+    const int q = u * WAVES + w;
+    uint32_t run = (uint32_t)__builtin_amdgcn_readlane((int)(incl - mine), q);
+    const uint32_t i = (uint32_t)(i1 + u * ROUND * kChunk + lane_id() * kVec);
+    if (via_lds) {
+      ballot_append(cand[u], run, [&](uint32_t pos, int e) { s_lidx[pos] = i + e; s_lkey[pos] = key[u][e]; });
+    } else {
+      run += s_base;
+      ballot_append(cand[u], run, [&](uint32_t pos, int e) { J.small_idx[pos] = i + e; J.small_key[pos] = key[u][e]; });
+    }
+  }
+  if (!via_lds) return;
+  __syncthreads();
+  if (!s_fit) return;
+  for (uint32_t t = threadIdx.x; t < all; t += WAVES * kWave) {
+    J.small_idx[s_base + t] = s_lidx[t];
+    J.small_key[s_base + t] = s_lkey[t];
+  }
+}
+template <class Src, int SPW>
+__global__ __launch_bounds__(kWide) void k_small_front(SrcPack<Src> srcs, ChainJobs jobs, SegDirJobs dirs,
+                                                       typename Src::Cols cols, uint32_t launch, double sigmas) {
+  const ChainJob& J = jobs.j[blockIdx.y];
+  const int64_t sweep = (int64_t)blockIdx.x - kSampleGroups - 1;
+  if (blockIdx.x < kSampleGroups) sample_pick_body<Src, false>(srcs, J, cols, launch, sigmas);
+  else if (sweep < 0) keep_tables(dirs, cols, threadIdx.x, kWide);
+  else if constexpr (std::is_same<typename Src::Cols, NowCols>::value)
+    small_sweep_body<Src, kWideWaves, SPW, true>(srcs.s[blockIdx.y], J, ColsOf{&cols, (int)blockIdx.y}, launch, sweep);
+  else
+    small_sweep_body<Src, kWideWaves, SPW, true>(srcs.s[blockIdx.y], J, NoCols{}, launch, sweep);
+}
+// The sweep behind a launch that took the sample and the bracket alone.
+template <class Src, int SPW>
+__global__ __launch_bounds__(kBlock) void k_small_sweep(SrcPack<Src> srcs, ChainJobs jobs) {
+  small_sweep_body<Src, kChunksPerBlock, SPW, false>(srcs.s[blockIdx.y], jobs.j[blockIdx.y], NoCols{}, 0u, blockIdx.x);
 }
 
 // The candidate list as the finishing workgroup sees it: wave w owns segment w (kSmallSegs ==
@@ -159,7 +258,8 @@ struct SmallList {
   __device__ __forceinline__ void counted(uint32_t c) {
     cnt = c;
 #pragma unroll
-    for (int u = 0; u < kSmallHead; ++u) trim(key[u], (uint32_t)(u * kWave + lane_id()) * kVec, c);
+    for (int u = 0; u < kSmallHead; ++u)
+      if (c < (uint32_t)(u + 1) * kWave * kVec) trim(key[u], (uint32_t)(u * kWave + lane_id()) * kVec, c);   // uniform
   }
   // head(key, idx) over the entries in registers, tail(keys, idxs) over rounds of quads of the rest (whole waves).
   // IDX: the index is wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a microsecond
@@ -225,13 +325,19 @@ struct SmallList {
 // no index to speak of.
 __device__ __forceinline__ void quad_add(uint32_t* s_tile, const U4& idx, const U4& num) {
   const uint32_t c0 = idx.x >> 10, c1 = idx.y >> 10, c2 = idx.z >> 10, c3 = idx.w >> 10;
-  const bool a1 = c1 == c0, a2 = c2 == c0, a3 = c3 == c0, b1 = !a1 && c1 == c3, b2 = !a2 && c2 == c3;
+  const bool a1 = c1 == c0, a2 = c2 == c0, a3 = c3 == c0;
   const uint32_t first = num.x + (a1 ? num.y : 0u) + (a2 ? num.z : 0u) + (a3 ? num.w : 0u);
-  const uint32_t last = (a3 ? 0u : num.w) + (b1 ? num.y : 0u) + (b2 ? num.z : 0u);
+  const uint32_t behind = num.x + num.y + num.z + num.w - first;
   if (first) atomicAdd(&s_tile[c0], first);
-  if (last) atomicAdd(&s_tile[c3], last);
-  if (!a1 && !b1 && num.y) atomicAdd(&s_tile[c1], num.y);
-  if (!a2 && !b2 && num.z) atomicAdd(&s_tile[c2], num.z);
+  if (behind) {
+    const bool b1 = c1 == c3, b2 = c2 == c3;          // of c3's chunk, which is not c0's
+    const uint32_t last = a3 ? 0u : num.w + (b1 ? num.y : 0u) + (b2 ? num.z : 0u);
+    if (last) atomicAdd(&s_tile[c3], last);
+    if (behind != last) {
+      if (!a1 && (a3 || !b1) && num.y) atomicAdd(&s_tile[c1], num.y);
+      if (!a2 && (a3 || !b2) && num.z) atomicAdd(&s_tile[c2], num.z);
+    }
+  }
 }
 static_assert(kSmallHead * kWave * kVec <= 2 * kChunk, "the head never reaches past a segment");
 
@@ -269,11 +375,11 @@ __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t
     const int above = step == 0 ? 31 : step == 1 ? kL0Shift : kL1Shift, bits = above - shift;
     uint32_t* gh = J.hist + (step == 0 ? 0 : step == 1 ? kBinsBig : 2 * kBinsBig);
     if (step == 3) {
-      tile_count_body(src, J, prefix, 0, (int64_t)blk * kWideWaves + wave_id(), (int64_t)G * kWideWaves);
+      tile_count_body<Src, Src::kHyper>(src, J, prefix, 0, (int64_t)blk * kWideWaves + wave_id(), (int64_t)G * kWideWaves);
     } else {
       reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
       __syncthreads();
-      constexpr int U = 4;                            // quads in flight per thread
+      constexpr int U = Src::kHyper ? 1 : 4;          // quads in flight per thread (the chains: four of them spill)
       constexpr int64_t kSlab = (int64_t)kWide * kVec;
       for (int64_t base = (int64_t)blk * kSlab * U; base < n; base += (int64_t)G * kSlab * U) {
         uint32_t key[U][4];
@@ -319,11 +425,11 @@ __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t
 
 template <class Src>
 __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs, int cpw) {
-  __shared__ __align__(16) uint32_t s_hist[kBinsBig];
+  __shared__ __align__(16) uint32_t s_hist[kBinsBig + kWave];     // behind the bins, a word per lane for what is in none
   __shared__ __align__(16) uint32_t s_tile[kSmallTiles];          // above | ties << 16, at most 1024 each
   __shared__ __align__(16) uint32_t s_key[kWideList];
   __shared__ uint32_t s_idx[kWideList];
-  __shared__ uint32_t s_seg[kWideWaves], s_cnt, s_out[3], s_word;
+  __shared__ uint32_t s_seg[kWideWaves], s_cnt, s_out[3], s_word, s_listed, s_nf, s_flags;
   __shared__ WideScratch s_scan;
   const ChainJob& J = jobs.j[blockIdx.y];
   SelState* st = J.st;
@@ -335,23 +441,35 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   SmallList list;
   list.request(J, geo);
   constexpr int PER = kSmallTiles / kWide;            // 8
-  uint32_t g8[PER], e8[PER], hi = 0, eqs = 0;
+  const SmallChunk none = SmallChunk::none(T_LO, T_HI);
+  SmallChunk ch[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = j * kWide + threadIdx.x;
-    g8[j] = e8[j] = 0u;
-    if (j * kWide < nt && t < nt) { g8[j] = J.tile_gt[t]; e8[j] = J.tile_eq[t]; }
+    ch[j] = none;
+    if (j * kWide < nt && t < nt) { ch[j].a = J.tile_gt[t]; ch[j].b = J.tile_eq[t]; }
   }
+  uint32_t sum_a = 0, sum_b = 0, off_a = 0, off_b = 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    s_tile[j * kWide + threadIdx.x] = g8[j] | (e8[j] << 16);
-    hi += g8[j];
-    eqs += e8[j];
+    sum_a += ch[j].a & SmallChunk::kNumbers;
+    sum_b += ch[j].b & SmallChunk::kNumbers;
+    off_a |= ch[j].a ^ none.a;
+    off_b |= ch[j].b ^ none.b;
   }
+  const uint32_t hi = sum_a & 0xFFFFu, eqs = sum_b & 0xFFFFu, nonfinite = sum_b >> 16;
+  uint32_t listed = sum_a >> 16;
+  const bool minus = (off_b & SmallChunk::kNegative) != 0u;
+  const bool wrong = ((off_a | (off_b & ~SmallChunk::kNegative)) & ~SmallChunk::kNumbers) != 0u;
   reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
   if (threadIdx.x < kWideWaves)
     s_seg[threadIdx.x] = threadIdx.x < geo.segs ? J.seg_cnt[threadIdx.x * kSmallSegStride] : 0u;
+  if (blockIdx.x == 0 && threadIdx.x < 4 * kSmallSegs) {             // behind the launch that used them
+    reinterpret_cast<uint32_t*>(small_bracket_copy(J, (int)threadIdx.x / 4))[threadIdx.x % 4] = 0u;
+    if (threadIdx.x < kSampleGroups) st->sampled[threadIdx.x] = 0u;
+  }
   if (threadIdx.x == 0) {
+    s_listed = s_nf = s_flags = 0u;
     s_cnt = 0u;
     s_word = gridDim.x > 1 ? atomicAdd(&st->finish_ticket, 1u) : 0u;
   }
@@ -369,6 +487,10 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     if (s_cnt == 1u) return;
   }
   uint32_t n_hi, n_low, n_list;
+  listed = wave_sum(listed);
+  if (lane_id() == 0 && listed) atomicAdd(&s_listed, listed);
+  if (nonfinite) atomicAdd(&s_nf, nonfinite);
+  if (minus | wrong) atomicOr(&s_flags, (minus ? 1u : 0u) | (wrong ? 2u : 0u));
   wide_totals(hi, eqs, s_scan, n_hi, n_low);
   wide_waves_before(s_seg, n_list);
   list.counted(s_seg[wave_id()]);
@@ -382,29 +504,34 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     const RankEnds f = bracket_ranks((double)k, (double)n, ns, kBracketSigmas);
     crowded = (double)n_list * ns > 2.0 * (f.lo - f.hi) * (double)n;
   }
-  const bool ok = judge && !crowded && n_hi < k && k <= n_hi + n_list + n_low;
+  const bool whole = s_listed == n_list && (s_flags & 2u) == 0u;     // of one bracket, and nothing lost
+  const bool ok = judge && whole && !crowded && n_hi < k && k <= n_hi + n_list + n_low;
   if (judge && gridDim.x > 1 && ok && threadIdx.x == 0) st_agent(&st->verdict, 1u);
   const bool low = ok && k > n_hi + n_list;           // the lower end is the threshold
   uint32_t T = T_LO, need = k - n_hi - n_list, n_eq = n_low;
   int turn = 0;
+  if (ok) {
+#pragma unroll
+    for (int j = 0; j < PER; ++j)                     // the lower end below the threshold: its members are no ties
+      s_tile[j * kWide + threadIdx.x] = (ch[j].a & 0x7FFu) | (low ? (ch[j].b & 0x7FFu) << 16 : 0u);
+  }
   if (low) {
+    __syncthreads();
     list.visit_quads([&](const U4& key, const U4& idx) {
       quad_add(s_tile, idx, U4{key.x != ~0u, key.y != ~0u, key.z != ~0u, key.w != ~0u});
     });
     __syncthreads();
   } else if (ok) {
-    // the lower end is below the threshold: its members are no ties
-#pragma unroll
-    for (int j = 0; j < PER; ++j) s_tile[j * kWide + threadIdx.x] = g8[j];
     // descent over the list inside (T_LO, T_HI): 4096 bins per level, until one bin is left whose
     // keys fit the short list (nearly always after the first level) or are all equal
     uint32_t lo = T_LO + 1u, rank = k - n_hi;
     int w = 32 - __clz((int)(T_HI - 1u - lo));         // bits of the offset (the list is not empty)
     for (;;) {
       const int sh = w > 12 ? w - 12 : 0;
+      const uint32_t bins = 1u << (w - sh), none = kBinsBig + (uint32_t)lane_id();
       auto count = [&](uint32_t key, uint32_t) {
-        const uint32_t off = key - lo;
-        if (off >> w == 0u) atomicAdd(&s_hist[off >> sh], 1u);
+        const uint32_t bin = (key - lo) >> sh;
+        atomicAdd(&s_hist[bin < bins ? bin : none], 1u);
       };
       // A plateau in a long list queues on its bin: where sixteen lanes' first keys of a round share one, the lanes
       // of that bin add together.  8.4 M coordinates, plateaus inside the bracket, plain adds / this: at 1 % 256 / 180
@@ -450,15 +577,18 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
         quad_add(s_tile, idx, U4{num(key.x), num(key.y), num(key.z), num(key.w)});
       });
     } else {
-      auto num = [&](uint32_t key) { return (uint32_t)(key - lo - width < 0x80000000u - width); };
+      const int32_t last = (int32_t)(lo + width - 1u), first = (int32_t)lo;     // of the bin; keys past the list are -1
+      auto num = [&](uint32_t key) { return (uint32_t)((int32_t)key > last); };
+      auto in = [&](uint32_t key) { return (int32_t)key >= first && (int32_t)key <= last; };
       auto keep = [&](uint32_t key, uint32_t idx) {
-        if (key - lo >= width) return;
+        if (!in(key)) return;
         const uint32_t at = atomicAdd(&s_cnt, 1u);
         s_key[at] = key;
         s_idx[at] = idx;
       };
       list.visit_quads([&](const U4& key, const U4& idx) {
         quad_add(s_tile, idx, U4{num(key.x), num(key.y), num(key.z), num(key.w)});
+        if (ballot64(in(key.x) | in(key.y) | in(key.z) | in(key.w)) == 0ull) return;
         keep(key.x, idx.x); keep(key.y, idx.y); keep(key.z, idx.z); keep(key.w, idx.w);
       });
     }
@@ -480,6 +610,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   if (!ok) {
     if (judge) {
       for (int b = threadIdx.x; b < kHistEntries; b += kWide) st_agent(&J.hist[b], 0u);
+      if (threadIdx.x == 0) { st_agent(&st->nonfinite, s_nf); st_agent(&st->negative, s_flags & 1u); }
       wait_landed();
       if (threadIdx.x == 0) st_agent(&st->verdict, 2u);
     }
@@ -488,6 +619,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     T = ld_agent(&st->prefix);
     need = ld_agent(&st->krem);
     n_eq = ld_agent(&st->n_eq);
+    if (threadIdx.x == 0) { s_nf = ld_agent(&st->nonfinite); s_flags = ld_agent(&st->negative); }
     for (int t = threadIdx.x; t < kSmallTiles; t += kWide)
       s_tile[t] = t < nt ? ld_agent(&J.tile_gt[t]) | (ld_agent(&J.tile_eq[t]) << 16) : 0u;
     __syncthreads();
@@ -547,11 +679,11 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
       out->n_gt = k - need;
       out->n_eq = n_eq;
       out->n_selected = selected;
-      out->nonfinite = st->nonfinite;
+      out->nonfinite = s_nf;
       out->status = 0u;
       // 1 where the bracket decided, but for buckets below 2^20: they report 0 whatever decided (callers
       // know the path of those sizes as 0)
-      out->path = (ok && !single && n >= kFastMinN ? 1u : 0u) | (st->negative ? 0x100u : 0u);
+      out->path = (ok && !single && n >= kFastMinN ? 1u : 0u) | (s_flags & 1u ? 0x100u : 0u);
     }
   }
 }
@@ -561,13 +693,28 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
 template <class Src>
 static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B, const SegDirJobs& dirs,
                                     const typename Src::Cols& cols, hipStream_t s) {
-  launch_sample_pick<false>(srcs, B, dirs, cols, kBracketSigmas, s);
-  const int cpw = Src::kHyper || B.max_tiles <= kSweepTiles ? 1 : 4;
-  if (cpw == 1)
-    hipLaunchKernelGGL((k_small_sweep<Src, 1>), B.grid((unsigned)B.max_tiles), dim3(kBlock), 0, s, srcs, B.jobs);
-  else
-    hipLaunchKernelGGL((k_small_sweep<Src, Src::kHyper ? 1 : 4>), B.grid((unsigned)cdiv64(B.max_tiles, 4)), dim3(kBlock), 0,
-                       s, srcs, B.jobs);
+  static_assert(sizeof(ChainJobs) + sizeof(SrcPack<Src>) + sizeof(SegDirJobs) + sizeof(typename Src::Cols) + 64 <= 4096,
+                "the operands travel in the kernel arguments");
+  constexpr int MANY = Src::kHyper ? 1 : 4, ROUND = kWideWaves / kChunkIters;
+  const int64_t t = B.max_tiles;
+  int cpw = MANY == 1 || t <= kFrontTiles ? ROUND : ROUND * MANY;
+  const bool together = cdiv64(t, cpw) * B.count <= kFrontSweeps;
+  const auto front = [&](auto kernel, unsigned sweeps) {
+    hipLaunchKernelGGL(kernel, B.grid(kSampleGroups + 1 + sweeps), dim3(kWide), 0, s, srcs, B.jobs, dirs, cols,
+                       next_launch(), kBracketSigmas);
+  };
+  const auto sweep = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, B.grid((unsigned)cdiv64(t, cpw)), dim3(kBlock), 0, s, srcs, B.jobs);
+  };
+  if (together) {
+    if (cpw == ROUND) front(k_small_front<Src, 1>, (unsigned)cdiv64(t, cpw));
+    else front(k_small_front<Src, MANY>, (unsigned)cdiv64(t, cpw));
+  } else {
+    front(k_small_front<Src, 1>, 0u);
+    cpw = t <= kSweepTiles ? 1 : MANY;
+    if (cpw == 1) sweep(k_small_sweep<Src, 1>);
+    else sweep(k_small_sweep<Src, MANY>);
+  }
   const int64_t wgs = cdiv64(B.max_tiles, kRedoTiles);
   hipLaunchKernelGGL((k_small_finish<Src>), B.grid((unsigned)(wgs < kRedoGroups ? wgs : kRedoGroups)), dim3(kWide), 0,
                      s, srcs, B.jobs, cpw);
