@@ -117,6 +117,14 @@ int64_t sga_norm_partials(int64_t n);
 int sga_compact_norm_sq(const float* values, int64_t k, float* partials,
                         float* total, void* stream);
 
+/* total[0] = before[0] + the same sum (before NULL: the sum alone); the two
+ * may be the same.  Like the totals of sga_norm_sq_multi and sga_mask_totals,
+ * the bound of sga_pack_selected_split, the result of sga_select_topk and the
+ * sum of a dense replay step, total may lie in pinned host memory: its words
+ * arrive while the stream goes on, and none of them has all bits set. */
+int sga_compact_norm_sq_from(const float* values, int64_t k, float* partials,
+                             const float* before, float* total, void* stream);
+
 /* Allocation-free variant of sga_compact_norm_sq.  It has no counterpart in
  * the reference (whose compact_norm_sq_contribution allocates its partials on
  * every call, kernels.py:264); it is for callers that cannot allocate device

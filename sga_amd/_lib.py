@@ -62,6 +62,7 @@ SIGNATURES = {
     "sga_scatter_selected_parts": (I32, [P, P, P, P, I32, I64, P]),
     "sga_norm_partials": (I64, [I64]),
     "sga_compact_norm_sq": (I32, [P, I64, P, P, P]),
+    "sga_compact_norm_sq_from": (I32, [P, I64, P, P, P, P]),
     "sga_compact_norm_sq_noalloc": (I32, [P, I64, P, P]),
     "sga_masked_norm_sq": (I32, [P, P, I64, P, P, P]),
     "sga_gather_selected_blocks": (I32, [P, P, P, P, I64, I32, F, I64, P]),
@@ -284,6 +285,24 @@ def stream():
     """The current stream's handle, straight from torch's C layer (building a
     ``torch.cuda.Stream`` object to ask for its handle takes 3 us per call)."""
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def words(n):
+    """``n`` 32-bit words of pinned host memory, none of which has arrived: for
+    results that a kernel hands to the host while it waits (``arrived``)."""
+    return host().words(n)
+
+
+def arrived(t):
+    """The words of ``t`` as ints, waited for; the launch that writes them is on
+    the current stream."""
+    got = host().arrived(t)
+    if got is None:                      # a long kernel ahead of it, or an error: the stream tells
+        torch.cuda.current_stream().synchronize()
+        got = host().arrived(t)
+        if got is None:
+            raise RuntimeError("a result that its kernel should have written has not arrived")
+    return got
 
 
 def capturing():

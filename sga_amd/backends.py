@@ -32,9 +32,9 @@ def index_layout_pack(grad, idx, values, factor=1.0, slices=2):
         out = index_layout_bounds(idx, grad.numel(), slices)
         K.pack_selected(grad, idx, values, factor)     # the slices follow one another: one launch
         return out
-    below = torch.empty(1, dtype=torch.int64, device=idx.device)
-    K.pack_selected(grad, idx, values, factor, below)  # ... and the bound comes with it
-    n0 = int(below.item())
+    below = L.words(2)                                 # an int64
+    K.pack_selected(grad, idx, values, factor, below)  # ... and the bound comes with it, ahead of its end
+    n0 = L.arrived(below)[0]
     return [(0, n0), (n0, k)]
 
 

@@ -11,7 +11,7 @@ import torch
 
 from . import _lib as L
 from .adamw import ParamRecord
-from .kernels import compact_norm_sq_contribution, masked_norm_sq_contribution
+from .kernels import compact_norm, compact_norm_sq_contribution, masked_norm_sq_contribution
 
 
 def scale_masked_(grad, mask, coeff):
@@ -73,8 +73,8 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
     if not live:
         return 0.0, 1.0
     compact = compact_values if (not was_full and compact_values) else None
-    total = torch.zeros(1, dtype=torch.float32, device=live[0].grad.device)
-    seen = set()
+    total = None if compact is not None else torch.zeros(1, dtype=torch.float32, device=live[0].grad.device)
+    seen = {}
     for rec in live:
         if compact is not None:
             if type(rec) is ParamRecord:         # without the slice of the mask: 1 us a record
@@ -87,10 +87,7 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
             key = id(rec.bucket_state)
             if key not in compact:
                 raise RuntimeError("compact clip: bucket state without a values entry")
-            if key not in seen:
-                seen.add(key)
-                if compact[key].numel():
-                    compact_norm_sq_contribution(compact[key], total)
+            seen[key] = compact[key]
             continue
         mask = None if was_full else rec.mask_u8()
         g = rec.grad.data.reshape(-1)
@@ -98,7 +95,7 @@ def masked_clip_grad_norm(records, clip_grad, was_full, compact_values=None,
             compact_norm_sq_contribution(g, total)
         else:
             masked_norm_sq_contribution(g, mask, total)
-    grad_norm = total.sqrt().item()
+    grad_norm = total.sqrt().item() if compact is None else compact_norm(list(seen.values()))
     sparse_coeff = 1.0
     if clip_grad > 0.0:
         coeff = clip_grad / (grad_norm + 1.0e-6)

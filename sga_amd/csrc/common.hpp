@@ -199,6 +199,20 @@ __device__ __forceinline__ F4 ld4(const float* p) {
   const f4v t = *reinterpret_cast<const f4v*>(p);
   return F4{t.x, t.y, t.z, t.w};
 }
+// What the host may be waiting for in memory of its own, word by word, while the kernel still runs.  All bits set is
+// the word that has not arrived: no count, threshold or sum is (of the NaNs another one is stored).
+__device__ __forceinline__ void st_host(uint32_t* p, uint32_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void st_host(int64_t* p, int64_t v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+__device__ __forceinline__ void st_host(double* p, double v) {
+  st_host(reinterpret_cast<int64_t*>(p), __double_as_longlong(v != v ? __longlong_as_double(0x7FF8000000000000ll) : v));
+}
+__device__ __forceinline__ void st_host(float* p, float v) {
+  st_host(reinterpret_cast<uint32_t*>(p), v != v ? 0x7FC00000u : __float_as_uint(v));
+}
 __device__ __forceinline__ void st4(float* p, const F4& v) {
   *reinterpret_cast<f4v*>(p) = f4v{v.x, v.y, v.z, v.w};
 }

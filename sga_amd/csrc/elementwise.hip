@@ -56,24 +56,25 @@ __device__ __forceinline__ int64_t wave_lower_bound(const int32_t* __restrict__ 
   }
   return uniform_i64(lo);
 }
-// With `below`, the last workgroup of the grid counts the entries under `split` instead: the slices' bound is there
-// with the pack, where a search of its own and the wait for it came first (index layout, 63 M coordinates: kernels of
-// 27 us with a wait between them, 19.9 so; a step 370 -> 366 us).
+// With `below`, the first workgroup counts the entries under `split` instead: a host that waits for the slices' bound
+// in its own memory goes on while the pack runs, where a search of its own and the wait for it came first.
+// Index layout, a step on 63 M coordinates, bound with the pack's last workgroup and a copy of it -> so: 360 -> 338 us
+// (with the clip's sum in host memory as well), 92 M 579 -> 533, 290 K 97 -> 70.
 template <bool BF16, bool SCALE>
 __global__ __launch_bounds__(kBlock) void k_pack(float* __restrict__ grad,
                                                  const int32_t* __restrict__ idx,
                                                  void* __restrict__ values,
                                                  float factor, int64_t k,
                                                  int64_t n_grad, int64_t split = 0, int64_t* __restrict__ below = nullptr) {
-  unsigned groups = gridDim.x;
-  if (below && blockIdx.x == --groups) {
+  const unsigned extra = below ? 1u : 0u, groups = gridDim.x - extra;
+  if (blockIdx.x < extra) {
     if (wave_id() == 0) {
       const int64_t c = wave_lower_bound(idx, k, split);
-      if (lane_id() == 0) *below = c;
+      if (lane_id() == 0) st_host(below, c);
     }
     return;
   }
-  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < k;
+  for (int64_t i = (int64_t)(blockIdx.x - extra) * kBlock + threadIdx.x; i < k;
        i += (int64_t)groups * kBlock) {
     const int64_t j = idx[i];
     if (j < 0 || j >= n_grad) continue;
@@ -122,7 +123,7 @@ __global__ __launch_bounds__(kBlock) void k_norm_stage1(
 
 // Stage 2: single workgroup folds the partials in index order.
 __global__ __launch_bounds__(kBlock) void k_norm_stage2(
-    const float* __restrict__ partials, int64_t np, float* __restrict__ total) {
+    const float* __restrict__ partials, int64_t np, const float* before, float* total) {
   __shared__ float s_w[kChunksPerBlock];
   float acc = 0.0f;
   for (int64_t i = threadIdx.x; i < np; i += kBlock) acc += partials[i];
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(kBlock) void k_norm_stage2(
   if (threadIdx.x == 0) {
     float t = 0.0f;
     for (int w = 0; w < kChunksPerBlock; ++w) t += s_w[w];
-    total[0] += t;
+    st_host(total, before ? before[0] + t : t);
   }
 }
 
@@ -227,7 +228,7 @@ __global__ __launch_bounds__(kFoldBlock) void k_norm_multi_fold(const float* __r
   if (threadIdx.x == 0) {
     double t = 0.0;
     for (int w = 0; w < kFoldBlock / kWave; ++w) t += s_w[w];
-    total[0] = (float)t;
+    st_host(total, (float)t);
   }
 }
 
@@ -487,19 +488,19 @@ __global__ __launch_bounds__(kTotalsBlock) void k_mask_totals(const uint8_t* __r
     if (g < n_groups) sums[g] = run + before + incl - v;
     run += (uint32_t)__builtin_amdgcn_readlane((int)waves, kTotalsWaves - 1);
   }
-  if (threadIdx.x == 0) out[0] = (int64_t)run;
+  if (threadIdx.x == 0) st_host(out, (int64_t)run);
   __syncthreads();                                    // the offsets, which the same workgroup wrote
   for (int j = 1 + wave_id(); j <= cuts; j += kTotalsWaves) {
     const int64_t at = (int64_t)j * step, c = at / kChunk;
     if (at >= n) {
-      if (lane_id() == 0) out[j] = (int64_t)run;
+      if (lane_id() == 0) st_host(out + j, (int64_t)run);
       continue;
     }
     const int64_t c0 = c / kGroupChunks * kGroupChunks;
     uint32_t cnt = lane_id() < c - c0 ? counts[c0 + lane_id()] : 0u;
     for (int64_t i = c * kChunk + lane_id(); i < at; i += kWave) cnt += mask[i] != 0;
     cnt = wave_sum(cnt);
-    if (lane_id() == 0) out[j] = (int64_t)sums[c / kGroupChunks] + cnt;
+    if (lane_id() == 0) st_host(out + j, (int64_t)sums[c / kGroupChunks] + cnt);
   }
 }
 
@@ -740,8 +741,22 @@ extern "C" int sga_compact_norm_sq(const float* values, int64_t k,
                      values, (const uint8_t*)nullptr, k, partials,
                      quads_ok(values, 4));
   hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials,
-                     (int64_t)nb, total);
+                     (int64_t)nb, total, total);
   return check_launch("sga_compact_norm_sq");
+}
+
+extern "C" int sga_compact_norm_sq_from(const float* values, int64_t k, float* partials, const float* before,
+                                        float* total, void* stream) {
+  if (!values || !partials || !total || k < 1) {
+    set_error("sga_compact_norm_sq_from: bad argument (k=%lld)", (long long)k);
+    return SGA_ERR_ARG;
+  }
+  const unsigned nb = (unsigned)sga_norm_partials(k);
+  hipStream_t st = (hipStream_t)stream;
+  hipLaunchKernelGGL((k_norm_stage1<false>), dim3(nb), dim3(kBlock), 0, st, values, (const uint8_t*)nullptr, k,
+                     partials, quads_ok(values, 4));
+  hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials, (int64_t)nb, before, total);
+  return check_launch("sga_compact_norm_sq_from");
 }
 
 // The stage-1 partials of the allocation-free norm: one array per device,
@@ -799,7 +814,7 @@ extern "C" int sga_compact_norm_sq_noalloc(const float* values, int64_t k, float
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL((k_norm_stage1<false>), dim3(nb), dim3(kBlock), 0, st, values,
                      (const uint8_t*)nullptr, k, partials, quads_ok(values, 4));
-  hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials, (int64_t)nb, total);
+  hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials, (int64_t)nb, total, total);
   return check_launch("sga_compact_norm_sq_noalloc");
 }
 
@@ -816,7 +831,7 @@ extern "C" int sga_masked_norm_sq(const float* grad, const uint8_t* mask,
   hipLaunchKernelGGL((k_norm_stage1<true>), dim3(nb), dim3(kBlock), 0, st, grad,
                      mask, n, partials, quads_ok(grad, 4) && quads_ok(mask, 1));
   hipLaunchKernelGGL(k_norm_stage2, dim3(1), dim3(kBlock), 0, st, partials,
-                     (int64_t)nb, total);
+                     (int64_t)nb, total, total);
   return check_launch("sga_masked_norm_sq");
 }
 

@@ -23,6 +23,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <chrono>
 #include <cmath>
 #include <vector>
 
@@ -334,6 +335,68 @@ PyObject* norm_table(PyObject*, PyObject* args) {
   END_HANDLE_TH_ERRORS
 }
 
+// Results that the host waits for come into words of its own, which the kernel writes one by one (st_host): a copy and
+// the stream's end behind it were 5 to 15 us of every wait, and what follows the kernel on the stream runs on.  With a
+// copy -> so, us: select of 3 M scores 56.6 -> 42, mask layout step on 1.15 M coordinates 122 -> 106, dense replay step
+// and two configurations of 1.5 M 1,930 -> 1,783, full step on 63 M 854 -> 835.  A block is one call's, from torch's
+// pool; it goes back when all of its words have been written.
+// words(n): n 32-bit words of pinned host memory, all bits set: none of them has arrived.
+at::Tensor blank_words(int64_t n) {
+  at::Tensor t = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+  memset(t.data_ptr(), 0xFF, (size_t)n * 4);
+  return t;
+}
+PyObject* words(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  long long n;
+  if (!PyArg_ParseTuple(args, "L", &n)) return nullptr;
+  return THPVariable_Wrap(blank_words(n));
+  END_HANDLE_TH_ERRORS
+}
+// True when all of them have been written; looks for kLook at most.
+constexpr std::chrono::milliseconds kLook(20);
+bool all_arrived(const uint32_t* w, int64_t n) {
+  const auto written = [&] {
+    for (int64_t i = 0; i < n; ++i)
+      if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == ~0u) return false;
+    return true;
+  };
+  const auto end = std::chrono::steady_clock::now() + kLook;
+  for (;;) {
+    for (int i = 0; i < 64; ++i) {
+      if (written()) return true;
+      __builtin_ia32_pause();
+    }
+    if (std::chrono::steady_clock::now() > end) return written();
+  }
+}
+// arrived(words) -> their values, or None where they have not come for some time
+PyObject* arrived(PyObject*, PyObject* args) {
+  HANDLE_TH_ERRORS
+  PyObject* t;
+  if (!PyArg_ParseTuple(args, "O", &t)) return nullptr;
+  if (!THPVariable_Check(t)) {
+    PyErr_SetString(PyExc_TypeError, "arrived: a tensor of words");
+    return nullptr;
+  }
+  const at::Tensor held = THPVariable_Unpack(t);
+  if (held.is_cuda() || held.scalar_type() != at::kInt || !held.is_contiguous()) {
+    PyErr_SetString(PyExc_TypeError, "arrived: 32-bit words in host memory");
+    return nullptr;
+  }
+  const uint32_t* w = static_cast<const uint32_t*>(held.data_ptr());
+  const int64_t n = held.numel();
+  const bool there = [&] {
+    Unlocked released;
+    return all_arrived(w, n);
+  }();
+  if (!there) Py_RETURN_NONE;
+  PyObject* out = PyTuple_New(n);
+  for (int64_t i = 0; out && i < n; ++i) PyTuple_SET_ITEM(out, i, PyLong_FromUnsignedLong(w[i]));
+  return out;
+  END_HANDLE_TH_ERRORS
+}
+
 // norm(table, n_rows, spans, stream) -> sqrt of the sum of squares (waits for the stream)
 PyObject* norm(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
@@ -343,15 +406,18 @@ PyObject* norm(PyObject*, PyObject* args) {
   unsigned long long stream;
   if (!PyArg_ParseTuple(args, "OiLK", &t, &n_rows, &spans, &stream)) return nullptr;
   const at::Tensor& table = THPVariable_Unpack(t);
-  // [partials | total], fp32; every slot that is read is written first
-  at::Tensor buf = at::empty({spans + 1}, at::TensorOptions().dtype(at::kFloat).device(table.device()));
-  float* partials = static_cast<float*>(buf.data_ptr());
-  const int rc = f_norm_multi(static_cast<const sga_span_record*>(table.data_ptr()), n_rows, spans, partials,
-                              partials + spans, (void*)stream);
+  // the partials, fp32; every slot that is read is written first.  The total comes into host memory (a copy of it is
+  // a launch, and 3 us of the wait).
+  at::Tensor buf = at::empty({spans}, at::TensorOptions().dtype(at::kFloat).device(table.device()));
+  const at::Tensor word = table.is_cuda() ? blank_words(1) : at::empty({1}, at::kInt);
+  const int rc = f_norm_multi(static_cast<const sga_span_record*>(table.data_ptr()), n_rows, spans,
+                              static_cast<float*>(buf.data_ptr()), static_cast<float*>(word.data_ptr()), (void*)stream);
   if (rc != 0) return PyLong_FromLong(rc);
   const double total = [&] {
     Unlocked released;
-    return buf[spans].item<float>();
+    // not there in time: a read from the device waits for the stream, and raises its errors
+    if (!table.is_cuda() || !all_arrived(static_cast<const uint32_t*>(word.data_ptr()), 1)) (void)buf[0].item<float>();
+    return *static_cast<const volatile float*>(word.data_ptr());
   }();
   return PyFloat_FromDouble((double)(float)std::sqrt(total));
   END_HANDLE_TH_ERRORS
@@ -386,7 +452,9 @@ PyObject* bind(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"bind", bind, METH_VARARGS, nullptr},
+PyMethodDef methods[] = {{"words", words, METH_VARARGS, nullptr},
+                         {"arrived", arrived, METH_VARARGS, nullptr},
+                         {"bind", bind, METH_VARARGS, nullptr},
                          {"commit", commit, METH_VARARGS, nullptr},
                          {"commit_compact", commit_compact, METH_VARARGS, nullptr},
                          {"norm_table", norm_table, METH_VARARGS, nullptr},

@@ -632,7 +632,7 @@ __global__ __launch_bounds__(kFoldThreads) void k_fold_partials(const double* __
     if ((int)threadIdx.x < o) s_p[threadIdx.x] += s_p[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = s_p[0] / divisor;
+  if (threadIdx.x == 0) st_host(out, s_p[0] / divisor);
 }
 __global__ __launch_bounds__(kWave) void k_sqdist_stage2(const double* __restrict__ partials, int nb,
                                                          double* __restrict__ out) {

@@ -778,14 +778,14 @@ __device__ __forceinline__ void write_result(const ChainJob& J) {
   const SelState* st = J.st;
   sga_select_result* out = J.result;
   if (!out) return;
-  out->thresh_bits = ld_agent(&st->thresh_bits);
-  out->need = ld_agent(&st->need);
-  out->n_gt = ld_agent(&st->n_gt);
-  out->n_eq = ld_agent(&st->n_eq);
-  out->n_selected = ld_agent(&st->n_selected);
-  out->nonfinite = ld_agent(&st->nonfinite);
-  out->status = ld_agent(&st->status);
-  out->path = st->path | (ld_agent(&st->negative) ? 0x100u : 0u) | (st->redone ? 0x200u : 0u);
+  st_host(&out->thresh_bits, ld_agent(&st->thresh_bits));
+  st_host(&out->need, ld_agent(&st->need));
+  st_host(&out->n_gt, ld_agent(&st->n_gt));
+  st_host(&out->n_eq, ld_agent(&st->n_eq));
+  st_host(&out->n_selected, ld_agent(&st->n_selected));
+  st_host(&out->nonfinite, ld_agent(&st->nonfinite));
+  st_host(&out->status, ld_agent(&st->status));
+  st_host(&out->path, st->path | (ld_agent(&st->negative) ? 0x100u : 0u) | (st->redone ? 0x200u : 0u));
 }
 static __global__ void k_sel_result(ChainJobs jobs) { write_result(jobs.j[blockIdx.y]); }
 

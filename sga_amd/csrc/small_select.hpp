@@ -674,16 +674,16 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
     st->n_gt = k - need;
     st->n_selected = selected;
     if (sga_select_result* out = J.result) {
-      out->thresh_bits = T;
-      out->need = need;
-      out->n_gt = k - need;
-      out->n_eq = n_eq;
-      out->n_selected = selected;
-      out->nonfinite = s_nf;
-      out->status = 0u;
+      st_host(&out->thresh_bits, T);
+      st_host(&out->need, need);
+      st_host(&out->n_gt, k - need);
+      st_host(&out->n_eq, n_eq);
+      st_host(&out->n_selected, selected);
+      st_host(&out->nonfinite, s_nf);
+      st_host(&out->status, 0u);
       // 1 where the bracket decided, but for buckets below 2^20: they report 0 whatever decided (callers
       // know the path of those sizes as 0)
-      out->path = (ok && !single && n >= kFastMinN ? 1u : 0u) | (s_flags & 1u ? 0x100u : 0u);
+      st_host(&out->path, (ok && !single && n >= kFastMinN ? 1u : 0u) | (s_flags & 1u ? 0x100u : 0u));
     }
   }
 }

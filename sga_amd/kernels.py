@@ -25,7 +25,7 @@ def scatter_selected(dst, indices, src):
 def pack_selected(grad, indices, values, factor, below=None):
     """``values[i] = grad[idx[i]]*factor; grad[idx[i]] = 0`` in one pass
     (``sga/kernels.py:166-187``).  ``values`` may be fp32 or bf16.  ``below``
-    (one int64 on the device): also the number of ascending indices under
+    (one int64 on the device, or two words of the host's): also the number of ascending indices under
     ``grad.numel() // 2``."""
     k = indices.numel()
     if k == 0:
@@ -119,6 +119,27 @@ def compact_norm_sq_contribution(values, total_norm_sq):
         raise TypeError("compact_norm_sq_contribution: fp32 values and total")
     L.call("sga_compact_norm_sq", L.ptr(v), k, L.ptr(_partials(k, v.device)),
            L.ptr(total_norm_sq), L.stream())
+
+
+def compact_norm(values):
+    """The 2-norm of fp32 arrays taken together, as ``compact_norm_sq_contribution``
+    of one after the other and a square root give it, on the host: the last sum
+    comes into host memory."""
+    flat = [v.reshape(-1) for v in values if v.numel()]
+    if not flat:
+        return 0.0
+    L.require_dev(*flat)
+    L.require_contig(**{f"values{i}": v for i, v in enumerate(flat)})
+    if any(v.dtype != torch.float32 for v in flat):
+        raise TypeError("compact_norm: fp32 values")
+    before = None
+    for i, v in enumerate(flat):
+        total = L.words(1) if i + 1 == len(flat) else torch.empty(1, dtype=torch.float32, device=v.device)
+        L.call("sga_compact_norm_sq_from", L.ptr(v), v.numel(), L.ptr(_partials(v.numel(), v.device)), L.ptr(before),
+               L.ptr(total), L.stream())
+        before = total
+    L.arrived(total)
+    return total.view(torch.float32).sqrt().item()
 
 
 def use_fused_masked_op(grad, mask):

@@ -58,7 +58,8 @@ def select_topk_flat(t, k, check=True):
     """Exact top-k of a non-negative finite fp32 device vector; boundary ties
     go to the lowest flat indices (``sga/replay.py:538-572``).  Returns
     (bool mask, threshold).  The whole select runs on the device; the single
-    host read fetches the threshold and the rejection counters."""
+    host wait is for the threshold and the rejection counters; the mask follows
+    on the current stream."""
     L.require_dev(t)
     flat = t.reshape(-1)
     n = flat.numel()
@@ -66,7 +67,7 @@ def select_topk_flat(t, k, check=True):
         raise ValueError(f"k={k} > N={n}")
     mask = torch.empty(n, dtype=torch.bool, device=flat.device)
     res, _ = select_exact_device([flat], k, L.TIE_LOWEST_INDEX,
-                                 masks=[mask.view(torch.uint8)])
+                                 masks=[mask.view(torch.uint8)], res=L.words(8))
     r = read_result(res)
     if check:
         if r.nonfinite:

@@ -50,9 +50,6 @@ class DenseReplay:
         self.label = torch.zeros(self.N, dtype=torch.float32, device=dev)
         self._partials = torch.empty(int(L.raw("sga_replay_partials")), dtype=torch.float64,
                                      device=dev)
-        # the fold writes its sum straight into host memory: a step waits for it, and a copy would be
-        # one more thing to wait for
-        self._recon2 = torch.zeros(1, dtype=torch.float64, pin_memory=True)
         self._dist = torch.zeros(1, dtype=torch.float64, device=dev)
         self._seg_table = SegmentTable(entries, dev, start="a", segs=False, rsegs=True)
         self.si = 0
@@ -70,19 +67,25 @@ class DenseReplay:
         self._seg_table.follow(self.entries)          # callers may change them between steps
         self._seg_table.take(lr_by_group(gmeta, self.entries), count, self.optimizer == "adamw")
         st = L.stream()
+        # the fold writes its sum straight into host memory: a step waits for it, and a copy would be
+        # one more thing to wait for
+        recon2 = L.words(2)
         L.call("sga_dense_replay_step_at", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),
                L.ptr(self.v), L.ptr(self.label), self.N, *self._seg_table.args[1:],
                int(self.optimizer == "adams"), float(coef_dense), L.ptr(self._partials),
-               L.ptr(self._recon2), st)
-        torch.cuda.current_stream().synchronize()
-        recon = math.sqrt(float(self._recon2.item()))
+               L.ptr(recon2), st)
         norm = float(gmeta.get("grad_norm", float("nan")))
-        self.recon_steps.append({
-            "step": gstep, "lr": lr_for_step(gmeta), "lr_max_abs_diff": lr_max_abs_diff(gmeta),
-            "grad_norm": norm, "clip_grad": float(gmeta.get("clip_grad", 0.0)),
-            "coef_dense": coef_dense, "reconstruct_flag": flag, "recon_grad_norm": recon,
-            "recon_rel_err": ((recon - norm) / norm
-                              if math.isfinite(norm) and norm > 0.0 else None)})
+        try:
+            record = {
+                "step": gstep, "lr": lr_for_step(gmeta), "lr_max_abs_diff": lr_max_abs_diff(gmeta),
+                "grad_norm": norm, "clip_grad": float(gmeta.get("clip_grad", 0.0)),
+                "coef_dense": coef_dense, "reconstruct_flag": flag}
+        finally:
+            L.arrived(recon2)                         # before the words can be anyone else's
+        recon = math.sqrt(float(recon2.view(torch.float64).item()))
+        record.update(recon_grad_norm=recon, recon_rel_err=((recon - norm) / norm
+                                                            if math.isfinite(norm) and norm > 0.0 else None))
+        self.recon_steps.append(record)
         self.si += 1
         if self.si in horizons:
             L.call("sga_sq_dist", L.ptr(self.w), 0, L.ptr(self.w0), self.N, L.ptr(self._partials),

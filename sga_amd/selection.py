@@ -34,8 +34,9 @@ def _f32_of(bits):
 
 
 def read_result(res_t):
-    """Decode a device uint32[8] result block (one host sync)."""
-    r = res_t.cpu().tolist()
+    """Decode a device uint32[8] result block (one host sync), or one in words of
+    the host's (``_lib.words``), which is there before the mask is written."""
+    r = res_t.cpu().tolist() if res_t.is_cuda else L.arrived(res_t)
     out = SimpleNamespace(thresh_bits=r[0], need=r[1], n_gt=r[2], n_eq=r[3],
                           n_selected=r[4], nonfinite=r[5], status=r[6], path=r[7] & 0xFF,
                           negative=bool(r[7] & 0x100), redone=bool(r[7] & 0x200))
@@ -78,11 +79,11 @@ def _flat_span(views):
         store, first.storage_offset(), (total,), (1,))
 
 
-def select_exact_device(views, k, tie_mode, masks=None):
+def select_exact_device(views, k, tie_mode, masks=None, res=None):
     """Exact top-k over a list of flat fp32 views; returns (result, masks).
     Views are laid out back to back in chunk space, each on a fresh
     1024-element chunk, so flat-index order == view order then in-view order
-    (the reference's catalog order)."""
+    (the reference's catalog order).  ``res``: where the result goes."""
     views = _flat_views(views)
     dev = views[0].device
     bases, nt = [], 0
@@ -94,7 +95,8 @@ def select_exact_device(views, k, tie_mode, masks=None):
         raise ValueError(f"k={k} > N={n_total}" if k > n_total else f"k={k} < 1")
     ws_bytes = int(L.raw("sga_select_workspace_bytes", nt * _CHUNK))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    res = torch.empty(8, dtype=torch.int32, device=dev)
+    if res is None:
+        res = torch.empty(8, dtype=torch.int32, device=dev)
     st = L.stream()
     flat = None
     if masks is None and len(views) > 1:
@@ -147,7 +149,7 @@ def select_masks_histogram(grads, k, comm_group=None, mode="exact",
     except KeyError:
         raise ValueError(f"unknown histogram_mode: {mode!r}") from None
     if mode == "exact":
-        res, masks = select_exact_device(grads, k, L.TIE_ALL)
+        res, masks = select_exact_device(grads, k, L.TIE_ALL, res=L.words(8))
         return read_result(res).thresh, masks
     views = _flat_views(grads)
     dev = views[0].device

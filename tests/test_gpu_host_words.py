@@ -1,0 +1,56 @@
+"""Results that kernels write into words of the host's while it waits: every
+value arrives, also those that look like a word that has not."""
+import math
+import struct
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("bits", [0xFFFFFFFF, 0x7FC00000, 0xFF800000, 0x7F7FFFFF, 0x00000001])
+def test_norms_of_any_value_arrive(dev, bits):
+    from sga_amd.kernels import compact_norm, compact_norm_sq_contribution
+    x = torch.full((5000,), 0.5)
+    x.view(torch.int32)[1234] = bits - (1 << 32) if bits >= 1 << 31 else bits
+    total = torch.zeros(1, device=dev)
+    compact_norm_sq_contribution(x.to(dev), total)
+    want, got = total.cpu().sqrt().item(), compact_norm([x.to(dev)])
+    assert math.isnan(got) if math.isnan(want) else got == want
+
+
+@pytest.mark.parametrize("sizes", [(1,), (0, 3), (1024, 0, 1025), (4099, 70_001, 1_000_003)])
+def test_norms_of_several_arrays(dev, sizes):
+    """Bit for bit the sum that one contribution after the other gives; its root is rounded once."""
+    from sga_amd.kernels import compact_norm, compact_norm_sq_contribution
+    gen = torch.Generator().manual_seed(sum(sizes))
+    arrays = [torch.randn(s, generator=gen).to(dev) for s in sizes]
+    total = torch.zeros(1, device=dev)
+    for a in arrays:
+        compact_norm_sq_contribution(a, total)
+    assert struct.pack("<f", compact_norm(arrays)) == struct.pack("<f", total.cpu().sqrt().item())
+    assert compact_norm([torch.empty(0, device=dev)]) == 0.0
+
+
+def test_words_behind_a_long_queue(dev):
+    """Nothing arrives for longer than the host looks: it waits for the stream then."""
+    from sga_amd.replay import select_topk_flat
+    score = torch.rand(300_001, generator=torch.Generator().manual_seed(1)).to(dev)
+    big = torch.empty(1 << 28, device=dev)
+    torch.cuda.synchronize()
+    for _ in range(150):                          # some 40 ms of fills
+        big.zero_()
+    mask, thresh = select_topk_flat(score, 3000)
+    assert int(mask.sum()) == 3000 and thresh == score.topk(3000).values[-1].item()
+
+
+def test_selects_in_a_row_keep_their_masks(dev):
+    """The result is there before the mask is written; the mask follows on the stream."""
+    from sga_amd.replay import select_topk_flat
+    scores = [torch.rand(n, generator=torch.Generator().manual_seed(n)).to(dev) for n in (5, 70_001, 3_000_017, 12_000_001)]
+    got = [select_topk_flat(s, max(1, s.numel() // 50)) for s in scores for _ in range(3)]
+    for i, (mask, thresh) in enumerate(got):
+        s = scores[i // 3]
+        assert torch.equal(mask, s >= thresh) or int(mask.sum()) == max(1, s.numel() // 50)
+        assert not bool((mask & (s < thresh)).any()) and not bool((~mask & (s > thresh)).any())

@@ -89,3 +89,22 @@ def test_segment_tables_take_and_refuse_what_struct_fields_do(monkeypatch, repla
     for key, value in (("start", 0.5), ("n", 7.0)):
         with pytest.raises(TypeError):
             SegmentTable([dict(rows[1], **{key: value})], "cpu", **kw)
+
+
+def test_words_that_have_not_arrived():
+    """The wait ends by itself, and says which it was."""
+    _run("""
+        t = torch.full((3,), -1, dtype=torch.int32)
+        assert host.arrived(t) is None
+        t[0], t[1] = 7, -2
+        assert host.arrived(t) is None
+        t[2] = 0
+        assert host.arrived(t) == (7, 2 ** 32 - 2, 0)
+        for bad in (torch.zeros(2), torch.zeros(4, dtype=torch.int32)[::2], 3):
+            try:
+                host.arrived(bad)
+                raise SystemExit("no error")
+            except TypeError:
+                pass
+        print("done")
+        """)
