@@ -17,7 +17,7 @@ namespace sga {
 // EMIT: -1 sparse step; 0 update, 1 |g|, 2 |m|, 3 coi -> written into g.
 // FULL: the whole workgroup span is in range and every array element-aligned,
 // so all loads are unconditional and in flight together.
-template <int EMIT, bool FULL>
+template <int EMIT, bool FULL, bool KEEP = false>
 __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict__ g,
                                        float* __restrict__ m, float* __restrict__ v,
                                        const uint8_t* __restrict__ mask, int64_t i, int64_t n,
@@ -71,7 +71,8 @@ __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict_
   }
   st_f32<FULL>(m, i, n, mm, vec);
   st_f32<FULL>(v, i, n, vv, vec);
-  if (EMIT >= 0 || fold || (clear && touch_g)) st_f32<FULL>(g, i, n, gout, vec);
+  if (EMIT >= 0 && FULL && KEEP) st4(g + i, F4{gout[0], gout[1], gout[2], gout[3]});
+  else if (EMIT >= 0 || fold || (clear && touch_g)) st_f32<FULL>(g, i, n, gout, vec);
   st_f32<FULL>(p, i, n, pp, vec);
 }
 
@@ -101,7 +102,13 @@ struct GcRecord {           // sga_gc_record, see the header
   int flags, pad_;
 };
 
-template <int EMIT>
+// KEEP, up to this many spans (288 MB of scores): the emitted score leaves by ordinary stores and stays in the 256 MB
+// memory-side cache, where the select behind the commit reads it; the other streams are non-temporal and pass it by.
+// Full step, non-temporal -> ordinary, us: 20 M coordinates 354 -> 339, 40 M 588 -> 560, 63 M (252 MB) 821 -> 798, 67 M
+// (268 MB) 910 -> 876, 80 M (320 MB) the same, 100 M 1,341 -> 1,369, 200 M 2,781 -> 2,876.  (An instantiation of its
+// own: as a branch in one kernel the non-temporal side lost as much.)
+constexpr int64_t kKeepSpans = (288ll << 20) / (kBlockSpan * 4);
+template <int EMIT, bool KEEP>
 __global__ __launch_bounds__(kBlock) void k_grad_correct_multi(const GcRecord* __restrict__ recs,
                                                                int n_recs, float coeff,
                                                                float interval) {
@@ -118,8 +125,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_correct_multi(const GcRecord* _
   for (int it = 0; it < kBlockSpan / (kBlock * kVec); ++it) {
     const int64_t i = base + ((int64_t)it * kBlock + threadIdx.x) * kVec;
     if (full)
-      gc_vec<EMIT, true>(r.p, r.g, r.m, r.v, r.mask, i, r.n, h, coeff, interval, r.lr_inactive,
-                         r.flags, true);
+      gc_vec<EMIT, true, KEEP>(r.p, r.g, r.m, r.v, r.mask, i, r.n, h, coeff, interval, r.lr_inactive,
+                               r.flags, true);
     else if (i < r.n)
       gc_vec<EMIT, false>(r.p, r.g, r.m, r.v, r.mask, i, r.n, h, coeff, interval, r.lr_inactive,
                           r.flags, vec);
@@ -385,8 +392,10 @@ extern "C" int sga_adamw_grad_correct_multi(const sga_gc_record* recs, int n_rec
   const GcRecord* r = reinterpret_cast<const GcRecord*>(recs);
   dim3 grid((unsigned)total_spans), block(kBlock);
   hipStream_t st = (hipStream_t)stream;
+  const bool keep = total_spans <= kKeepSpans;
 #define SGA_GCM_LAUNCH(E) \
-  hipLaunchKernelGGL((k_grad_correct_multi<E>), grid, block, 0, st, r, n_recs, coeff, interval)
+  if (E >= 0 && keep) hipLaunchKernelGGL((k_grad_correct_multi<E, (E >= 0)>), grid, block, 0, st, r, n_recs, coeff, interval); \
+  else hipLaunchKernelGGL((k_grad_correct_multi<E, false>), grid, block, 0, st, r, n_recs, coeff, interval)
   switch (emit_mode) {
     case -1: SGA_GCM_LAUNCH(-1); break;
     case 0: SGA_GCM_LAUNCH(0); break;
