@@ -71,8 +71,7 @@ __device__ __forceinline__ void gc_vec(float* __restrict__ p, float* __restrict_
   }
   st_f32<FULL>(m, i, n, mm, vec);
   st_f32<FULL>(v, i, n, vv, vec);
-  if (EMIT >= 0 && FULL && KEEP) st4(g + i, F4{gout[0], gout[1], gout[2], gout[3]});
-  else if (EMIT >= 0 || fold || (clear && touch_g)) st_f32<FULL>(g, i, n, gout, vec);
+  if (EMIT >= 0 || fold || (clear && touch_g)) st_f32<FULL, KEEP>(g, i, n, gout, vec);
   st_f32<FULL>(p, i, n, pp, vec);
 }
 

@@ -375,11 +375,12 @@ __device__ __forceinline__ void ld_u8(const uint8_t* base, int64_t i, int64_t n,
     load4_u8(base, i, n, out, vec);
   }
 }
-template <bool FULL>
+template <bool FULL, bool KEEP = false>
 __device__ __forceinline__ void st_f32(float* base, int64_t i, int64_t n, const float v[4], bool vec) {
   if (FULL) {
     F4 t{v[0], v[1], v[2], v[3]};
-    st4_nt(base + i, t);
+    if (KEEP) st4(base + i, t);
+    else st4_nt(base + i, t);
   } else {
     store4_f32(base, i, n, v, vec);
   }

@@ -307,7 +307,13 @@ struct RSegCursor {
   }
 };
 
-template <bool BF16G, bool FULL>
+// KEEP, where a step writes up to this many coordinates (times configurations; 16 bytes each, 240 MB): the state leaves by
+// ordinary stores and stays in the 256 MB memory-side cache for the next recorded step, whose first reads it is.
+// Replay of 16 steps, non-temporal -> ordinary stores, us: 1 M coordinates by eight configurations 2,362 -> 2,310, 2 M by
+// six 2,393 -> 2,284, 4 M by three 2,518 -> 2,400, 8 M by two 3,086 -> 3,051; dense pass and one configuration of 15 M
+// 4,240 -> 4,095; 16.5 M (264 MB) 2,430 -> 2,472.
+constexpr int64_t kKeepState = 15ll << 20;
+template <bool BF16G, bool FULL, bool KEEP>
 __device__ __forceinline__ void pass3_vec(const void* g, int64_t i, int64_t n, float is_one,
                                           float coef_dense, const RGroup& grp,
                                           const float* __restrict__ coef_f, RSegCursor& sc,
@@ -363,14 +369,14 @@ __device__ __forceinline__ void pass3_vec(const void* g, int64_t i, int64_t n, f
       mm[e] = mn;
       vv[e] = vn;
     }
-    if (!(cf.boundary && cf.res_zero)) st_f32<FULL>(RES, i, n, rr, vec);   // zero stays zero
-    st_f32<FULL>(MM, i, n, mm, vec);
-    st_f32<FULL>(VV, i, n, vv, vec);
-    st_f32<FULL>(WW, i, n, ww, vec);
+    if (!(cf.boundary && cf.res_zero)) st_f32<FULL, KEEP>(RES, i, n, rr, vec);   // zero stays zero
+    st_f32<FULL, KEEP>(MM, i, n, mm, vec);
+    st_f32<FULL, KEEP>(VV, i, n, vv, vec);
+    st_f32<FULL, KEEP>(WW, i, n, ww, vec);
   }
 }
 
-template <bool BF16G>
+template <bool BF16G, bool KEEP>
 __global__ __launch_bounds__(kBlock) void k_replay_pass3(const void* __restrict__ g, int64_t n,
                                                          float coef_dense, RGroup grp,
                                                          const float* __restrict__ coef_f,
@@ -384,9 +390,9 @@ __global__ __launch_bounds__(kBlock) void k_replay_pass3(const void* __restrict_
   for (int64_t base = (int64_t)blk * kBlock * kVec; base < n; base += stride) {
     const int64_t i = base + (int64_t)threadIdx.x * kVec;
     if (vec && base + kBlock * kVec <= n)
-      pass3_vec<BF16G, true>(g, i, n, is_one, coef_dense, grp, coef_f, sc, true);
+      pass3_vec<BF16G, true, KEEP>(g, i, n, is_one, coef_dense, grp, coef_f, sc, true);
     else if (i < n)
-      pass3_vec<BF16G, false>(g, i, n, is_one, coef_dense, grp, coef_f, sc, vec);
+      pass3_vec<BF16G, false, KEEP>(g, i, n, is_one, coef_dense, grp, coef_f, sc, vec);
   }
 }
 
@@ -394,7 +400,7 @@ __global__ __launch_bounds__(kBlock) void k_replay_pass3(const void* __restrict_
 // One commit of the recorded (post-clip) gradient on the dense trajectory,
 // with the per-coordinate label lab += (lr*upd)^2 and sum(q^2) in double for
 // the pre-clip reconstruction (the launcher divides the sum by coef_dense^2).
-template <bool BF16G, bool FULL>
+template <bool BF16G, bool FULL, bool KEEP>
 __device__ __forceinline__ double dense_vec(const void* g, int64_t i, int64_t n, float* w,
                                             float* m, float* v, float* lab, int adams,
                                             RSegCursor& sc, bool vec) {
@@ -424,14 +430,14 @@ __device__ __forceinline__ double dense_vec(const void* g, int64_t i, int64_t n,
     const double qd = (double)q[e];
     acc += qd * qd;                       // exact product; the divisor is applied once, to the sum
   }
-  st_f32<FULL>(m, i, n, mm, vec);
-  st_f32<FULL>(v, i, n, vv, vec);
-  st_f32<FULL>(w, i, n, ww, vec);
-  if (lab) st_f32<FULL>(lab, i, n, ll, vec);
+  st_f32<FULL, KEEP>(m, i, n, mm, vec);
+  st_f32<FULL, KEEP>(v, i, n, vv, vec);
+  st_f32<FULL, KEEP>(w, i, n, ww, vec);
+  if (lab) st_f32<FULL, KEEP>(lab, i, n, ll, vec);
   return acc;
 }
 
-template <bool BF16G>
+template <bool BF16G, bool KEEP>
 __global__ __launch_bounds__(kBlock) void k_dense_step(const void* __restrict__ g, int64_t n,
                                                        float* w, float* m, float* v, float* lab,
                                                        int adams,
@@ -445,9 +451,9 @@ __global__ __launch_bounds__(kBlock) void k_dense_step(const void* __restrict__ 
   for (int64_t base = (int64_t)blockIdx.x * kBlock * kVec; base < n; base += stride) {
     const int64_t i = base + (int64_t)threadIdx.x * kVec;
     if (vec && base + kBlock * kVec <= n)
-      acc += dense_vec<BF16G, true>(g, i, n, w, m, v, lab, adams, sc, true);
+      acc += dense_vec<BF16G, true, KEEP>(g, i, n, w, m, v, lab, adams, sc, true);
     else if (i < n)
-      acc += dense_vec<BF16G, false>(g, i, n, w, m, v, lab, adams, sc, vec);
+      acc += dense_vec<BF16G, false, KEEP>(g, i, n, w, m, v, lab, adams, sc, vec);
   }
   acc = wave_sum(acc);
   if (lane_id() == 0) s_w[wave_id()] = acc;
@@ -817,8 +823,11 @@ extern "C" int sga_replay_pass3(const void* g, int g_dtype, int64_t n, float coe
   hipStream_t s = (hipStream_t)stream;
   const RSeg* rs = reinterpret_cast<const RSeg*>(segs);
   ProfPair* pp = prof_begin(SGA_PROF_REPLAY_PASS3, s);
-  if (bg) hipLaunchKernelGGL((k_replay_pass3<true>), dim3(nb), dim3(kBlock), 0, s, g, n, coef_dense, grp, coef_f, rs, n_segs, vec);
-  else hipLaunchKernelGGL((k_replay_pass3<false>), dim3(nb), dim3(kBlock), 0, s, g, n, coef_dense, grp, coef_f, rs, n_segs, vec);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, s, g, n, coef_dense, grp, coef_f, rs, n_segs, vec);
+  };
+  if ((int64_t)G * n <= kKeepState) bg ? launch(k_replay_pass3<true, true>) : launch(k_replay_pass3<false, true>);
+  else bg ? launch(k_replay_pass3<true, false>) : launch(k_replay_pass3<false, false>);
   prof_end(pp, s);
   return check_launch("sga_replay_pass3");
 }
@@ -1260,8 +1269,11 @@ static int dense_replay_step(const void* g, int g_dtype, float* w, float* m, flo
   const unsigned nb = stream_grid(n, (int64_t)kBlock * kVec, kReplayBlocks * kMaxCfg);
   hipStream_t s = (hipStream_t)stream;
   const RSeg* rs = reinterpret_cast<const RSeg*>(segs);
-  if (bg) hipLaunchKernelGGL((k_dense_step<true>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec, now);
-  else hipLaunchKernelGGL((k_dense_step<false>), dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec, now);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nb), dim3(kBlock), 0, s, g, n, w, m, v, lab, adams, rs, n_segs, partials, vec, now);
+  };
+  if (n <= kKeepState) bg ? launch(k_dense_step<true, true>) : launch(k_dense_step<false, true>);
+  else bg ? launch(k_dense_step<true, false>) : launch(k_dense_step<false, false>);
   hipLaunchKernelGGL(k_fold_partials, dim3(1), dim3(kFoldThreads), 0, s, partials, (int)nb,
                      coef_dense * coef_dense, recon2, now);
   return check_launch("sga_dense_replay_step");

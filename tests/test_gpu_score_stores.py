@@ -64,3 +64,41 @@ def test_scores_around_the_line(dev, n):
         SgaAdamW().full_step(OptContext(recs, "full", bucket_states=[]))
         assert torch.equal(state[1], want)
         del recs, state, want
+
+
+@pytest.mark.parametrize("n,configs", [(5_000_000, 2), (15 << 20, 1), ((15 << 20) + 1, 1)])
+def test_replay_steps_around_their_line(dev, n, configs):
+    """Steps of several configurations against each of them alone (fewer bytes a step), dense steps against
+    the commit in torch."""
+    from sga_amd.replay_dense import DenseReplay
+    from sga_amd.replay_group import Config, ReplayGroup
+    gen = torch.Generator(device=dev).manual_seed(n)
+    w, m = (torch.randn(n, generator=gen, device=dev) * s for s in (0.02, 1e-4))
+    v = torch.rand(n, generator=gen, device=dev) * 1e-6 + 1e-8
+    entries = [{"a": 0, "n": n - 1000, "b1": 0.9, "b2": 0.95, "eps": 1e-8, "wd": 0.1, "group": 0},
+               {"a": n - 1000, "n": 1000, "b1": 0.8, "b2": 0.99, "eps": 1e-6, "wd": 0.0, "group": 0}]
+    steps = [(torch.randn(n, generator=gen, device=dev) * 1e-3).to(torch.bfloat16) for _ in range(3)]
+    meta = {"clip_grad": 1.0, "grad_norm": 1.5, "lr": 1e-4}
+    arms = [Config("abs_g", 1.0, 2), Config("abs_g_blind", 2.0, 4)][:configs]
+    sel = [torch.rand(n, generator=gen, device=dev) < 0.01 for _ in arms]
+
+    def run(which):
+        group = ReplayGroup(entries, w, m, v, [sel[j] for j in which], [arms[j] for j in which], t0=5, window=1 << 10)
+        for g in steps:
+            group.step(g, meta)
+        return [(st.data.clone(), st.sel.clone()) for st in group.state]
+    together = run(range(configs))
+    for j in range(configs):
+        (data, picked), = run([j])
+        assert same_bits(together[j][0], data) and torch.equal(together[j][1], picked)
+    dense = DenseReplay(entries, w, m, v, 5, "adamw")
+    for t, g in enumerate(steps):
+        dense.step(t, g, dict(meta, lr=[1e-4]))
+    pm, pv = m.clone(), v.clone()
+    for g in steps:
+        q = g.float()
+        pm[:n - 1000] = pm[:n - 1000] * 0.9 + q[:n - 1000] * 0.1
+        pv[:n - 1000] = pv[:n - 1000] * 0.95 + q[:n - 1000] ** 2 * 0.05
+    # three roundings a step of each moment
+    assert torch.allclose(dense.m[:n - 1000], pm[:n - 1000], rtol=1e-6, atol=1e-10)
+    assert torch.allclose(dense.v[:n - 1000], pv[:n - 1000], rtol=1e-6, atol=1e-16)
