@@ -100,8 +100,10 @@ struct SegCursor {
     return a;
   }
   __device__ __forceinline__ void seek(int64_t i) {
-    if (i >= lo && i < hi) return;
-    at = find(i);
+    if (i < lo || i >= hi) place(find(i));
+  }
+  __device__ __forceinline__ void place(int a) {
+    at = a;
     lo = segs[at].start;
     hi = lo + segs[at].n;
     h = hyper_of(segs[at]);

@@ -95,3 +95,24 @@ def test_steps_agree_with_the_radix_passes(dev, sizes, score):
         ends.append(out + [x for v in views for x in v])
     for a, b in zip(*ends):
         assert torch.equal(a, b) if a.dtype != torch.float32 else same_bits(a, b)
+
+
+@pytest.mark.parametrize("tensors", [1, 2, 8192, 8193])
+@pytest.mark.parametrize("n", [300_001, 9_000_003])
+def test_tables_of_many_tensors(dev, n, tensors):
+    """The sample looks tensors up among their starts in LDS, up to 8192 of them; the hyper-parameters decide
+    what is selected.  Against the select without a sample."""
+    from sga_amd.fused_step import FusedSparseStep
+    each = n // tensors
+    ends = []
+    for fast in (True, False):
+        segs = [dict(start=t * each, n=each if t + 1 < tensors else n - t * each, lr=1e-4, b1=0.9, b2=0.95,
+                     eps=1e-8 * (1 + 50 * (t % 3)), wd=0.1 * (t % 2)) for t in range(tensors)]
+        gen = torch.Generator().manual_seed(tensors)
+        state = [torch.zeros(n, device=dev), (torch.randn(n, generator=gen) * 0.02).to(dev),
+                 (torch.randn(n, generator=gen) * 1e-4).to(dev), torch.full((n,), 1e-8, device=dev)]
+        fs = FusedSparseStep(n, segs, dev, values_dtype=torch.float32, max_k=n // 100)
+        idx, val = fs.step(student_t(n, 7).to(dev), *state, 3, k=n // 100, score="update", fast=fast)
+        ends.append([idx, val, *state])
+    for a, b in zip(*ends):
+        assert torch.equal(a, b) if a.dtype != torch.float32 else same_bits(a, b)
