@@ -120,8 +120,9 @@ int sga_compact_norm_sq(const float* values, int64_t k, float* partials,
 /* total[0] = before[0] + the same sum (before NULL: the sum alone); the two
  * may be the same.  Like the totals of sga_norm_sq_multi and sga_mask_totals,
  * the bound of sga_pack_selected_split, the result of sga_select_topk and the
- * sum of a dense replay step, total may lie in pinned host memory: its words
- * arrive while the stream goes on, and none of them has all bits set. */
+ * sum of a dense replay step, total may lie in pinned host memory: a result
+ * of 32 or 64 bits arrives in one piece while the stream goes on, and never
+ * has all of its bits set (half of one that has 64 may). */
 int sga_compact_norm_sq_from(const float* values, int64_t k, float* partials,
                              const float* before, float* total, void* stream);
 

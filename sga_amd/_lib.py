@@ -287,14 +287,14 @@ def stream():
     return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
-def words(n):
-    """``n`` 32-bit words of pinned host memory, none of which has arrived: for
-    results that a kernel hands to the host while it waits (``arrived``)."""
-    return host().words(n)
+def words(n, wide=False):
+    """``n`` words of 32 bits (``wide``: of 64) in pinned host memory, none of which has arrived:
+    for results of that size that a kernel hands to the host while it waits (``arrived``)."""
+    return host().words(n, wide)
 
 
 def arrived(t):
-    """The words of ``t`` as ints, waited for; the launch that writes them is on
+    """The words of ``t`` as unsigned ints, waited for; the launch that writes them is on
     the current stream."""
     got = host().arrived(t)
     if got is None:                      # a long kernel ahead of it, or an error: the stream tells

@@ -32,7 +32,7 @@ def index_layout_pack(grad, idx, values, factor=1.0, slices=2):
         out = index_layout_bounds(idx, grad.numel(), slices)
         K.pack_selected(grad, idx, values, factor)     # the slices follow one another: one launch
         return out
-    below = L.words(2)                                 # an int64
+    below = L.words(1, wide=True)
     K.pack_selected(grad, idx, values, factor, below)  # ... and the bound comes with it, ahead of its end
     n0 = L.arrived(below)[0]
     return [(0, n0), (n0, k)]

@@ -199,8 +199,9 @@ __device__ __forceinline__ F4 ld4(const float* p) {
   const f4v t = *reinterpret_cast<const f4v*>(p);
   return F4{t.x, t.y, t.z, t.w};
 }
-// What the host may be waiting for in memory of its own, word by word, while the kernel still runs.  All bits set is
-// the word that has not arrived: no count, threshold or sum is (of the NaNs another one is stored).
+// What the host may be waiting for in memory of its own while the kernel still runs: a result of 32 or 64 bits, stored
+// in one piece.  All of its bits set is the result that has not arrived: no count, threshold or sum is that (of the NaNs
+// another one is stored).
 __device__ __forceinline__ void st_host(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }

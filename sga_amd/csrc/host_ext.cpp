@@ -340,25 +340,29 @@ PyObject* norm_table(PyObject*, PyObject* args) {
 // copy -> so, us: select of 3 M scores 56.6 -> 42, mask layout step on 1.15 M coordinates 122 -> 106, dense replay step
 // and two configurations of 1.5 M 1,930 -> 1,783, full step on 63 M 854 -> 835.  A block is one call's, from torch's
 // pool; it goes back when all of its words have been written.
-// words(n): n 32-bit words of pinned host memory, all bits set: none of them has arrived.
-at::Tensor blank_words(int64_t n) {
-  at::Tensor t = at::empty({n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-  memset(t.data_ptr(), 0xFF, (size_t)n * 4);
+// words(n, wide): n results of 32 bits, or of 64, in pinned host memory, all bits set: none of them has arrived.
+// A result of 64 bits is stored and looked at in one piece: its halves may well have all bits set (2^53 - 1 as a
+// double), the whole of it never has.
+at::Tensor blank_words(int64_t n, bool wide = false) {
+  at::Tensor t = at::empty({n}, at::TensorOptions().dtype(wide ? at::kLong : at::kInt).pinned_memory(true));
+  memset(t.data_ptr(), 0xFF, (size_t)n * (wide ? 8 : 4));
   return t;
 }
 PyObject* words(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
   long long n;
-  if (!PyArg_ParseTuple(args, "L", &n)) return nullptr;
-  return THPVariable_Wrap(blank_words(n));
+  int wide = 0;
+  if (!PyArg_ParseTuple(args, "L|p", &n, &wide)) return nullptr;
+  return THPVariable_Wrap(blank_words(n, wide != 0));
   END_HANDLE_TH_ERRORS
 }
 // True when all of them have been written; looks for kLook at most.
 constexpr std::chrono::milliseconds kLook(20);
-bool all_arrived(const uint32_t* w, int64_t n) {
+template <class W>
+bool all_arrived(const W* w, int64_t n) {
   const auto written = [&] {
     for (int64_t i = 0; i < n; ++i)
-      if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == ~0u) return false;
+      if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == (W)~(W)0) return false;
     return true;
   };
   const auto end = std::chrono::steady_clock::now() + kLook;
@@ -380,19 +384,21 @@ PyObject* arrived(PyObject*, PyObject* args) {
     return nullptr;
   }
   const at::Tensor held = THPVariable_Unpack(t);
-  if (held.is_cuda() || held.scalar_type() != at::kInt || !held.is_contiguous()) {
-    PyErr_SetString(PyExc_TypeError, "arrived: 32-bit words in host memory");
+  const bool wide = held.scalar_type() == at::kLong;
+  if (held.is_cuda() || (!wide && held.scalar_type() != at::kInt) || !held.is_contiguous()) {
+    PyErr_SetString(PyExc_TypeError, "arrived: words of 32 or 64 bits in host memory");
     return nullptr;
   }
   const uint32_t* w = static_cast<const uint32_t*>(held.data_ptr());
+  const uint64_t* w64 = static_cast<const uint64_t*>(held.data_ptr());
   const int64_t n = held.numel();
   const bool there = [&] {
     Unlocked released;
-    return all_arrived(w, n);
+    return wide ? all_arrived(w64, n) : all_arrived(w, n);
   }();
   if (!there) Py_RETURN_NONE;
   PyObject* out = PyTuple_New(n);
-  for (int64_t i = 0; out && i < n; ++i) PyTuple_SET_ITEM(out, i, PyLong_FromUnsignedLong(w[i]));
+  for (int64_t i = 0; out && i < n; ++i) PyTuple_SET_ITEM(out, i, PyLong_FromUnsignedLongLong(wide ? w64[i] : w[i]));
   return out;
   END_HANDLE_TH_ERRORS
 }

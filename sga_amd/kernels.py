@@ -25,7 +25,7 @@ def scatter_selected(dst, indices, src):
 def pack_selected(grad, indices, values, factor, below=None):
     """``values[i] = grad[idx[i]]*factor; grad[idx[i]] = 0`` in one pass
     (``sga/kernels.py:166-187``).  ``values`` may be fp32 or bf16.  ``below``
-    (one int64 on the device, or two words of the host's): also the number of ascending indices under
+    (one int64, on the device or a wide word of the host's): also the number of ascending indices under
     ``grad.numel() // 2``."""
     k = indices.numel()
     if k == 0:

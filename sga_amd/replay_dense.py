@@ -69,7 +69,7 @@ class DenseReplay:
         st = L.stream()
         # the fold writes its sum straight into host memory: a step waits for it, and a copy would be
         # one more thing to wait for
-        recon2 = L.words(2)
+        recon2 = L.words(1, wide=True)
         L.call("sga_dense_replay_step_at", L.ptr(g), L.dtype_code(g), L.ptr(self.w), L.ptr(self.m),
                L.ptr(self.v), L.ptr(self.label), self.N, *self._seg_table.args[1:],
                int(self.optimizer == "adams"), float(coef_dense), L.ptr(self._partials),

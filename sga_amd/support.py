@@ -38,9 +38,9 @@ def mask_totals(mask_u8, step=0, cuts=0):
     if n == 0:
         return mk, None, 0, [0] * cuts
     scratch = torch.empty(int(L.raw("sga_mask_list_words", n)), dtype=torch.int32, device=mk.device)
-    totals = L.words(2 * (1 + cuts))
+    totals = L.words(1 + cuts, wide=True)
     L.call("sga_mask_totals", L.ptr(mk), n, L.ptr(scratch), step, cuts, L.ptr(totals), L.stream())
-    k, *before = L.arrived(totals)[::2]
+    k, *before = L.arrived(totals)
     return mk, scratch, k, before
 
 

@@ -54,3 +54,24 @@ def test_selects_in_a_row_keep_their_masks(dev):
         s = scores[i // 3]
         assert torch.equal(mask, s >= thresh) or int(mask.sum()) == max(1, s.numel() // 50)
         assert not bool((mask & (s < thresh)).any()) and not bool((~mask & (s > thresh)).any())
+
+
+@pytest.mark.parametrize("adams", [False, True])
+def test_sums_whose_low_half_has_all_bits_set(dev, adams):
+    """Squares of whole numbers that add up to 2^53 - 1, the double 0x433FFFFFFFFFFFFF: every partial sum is
+    exact, in any order."""
+    from sga_amd.replay_dense import DenseReplay
+    left, values = 2 ** 53 - 1, []
+    while left:
+        values.append(min(math.isqrt(left), 2 ** 24))
+        left -= values[-1] ** 2
+    assert struct.pack(">d", float(sum(x * x for x in values))).hex() == "433fffffffffffff"
+    n = 3 * len(values) + 1000
+    g = torch.zeros(n)
+    g[torch.arange(len(values)) * 3] = torch.tensor(values, dtype=torch.float32)
+    w, m, v = torch.zeros(n, device=dev), torch.zeros(n, device=dev), torch.full((n,), 1.0, device=dev)
+    rep = DenseReplay([dict(a=0, n=n, b1=0.9, b2=0.95, eps=1e-8, wd=0.0, group=0)], w, m, v, 3,
+                      "adams" if adams else "adamw")
+    for t in range(2):
+        rep.step(t, g.to(dev), {"lr": [1e-3], "clip_grad": 0.0})
+    assert [r["recon_grad_norm"] for r in rep.recon_steps] == [math.sqrt(2.0 ** 53 - 1)] * 2

@@ -108,3 +108,19 @@ def test_words_that_have_not_arrived():
                 pass
         print("done")
         """)
+
+
+def test_results_of_64_bits_arrive_in_one_piece():
+    """Either half may have all bits set (the low one of the double 2^53 - 1); the whole is looked at."""
+    _run("""
+        import struct
+        t = torch.full((3,), -1, dtype=torch.int64)
+        assert host.arrived(t) is None
+        low = struct.unpack("<q", struct.pack("<d", 2.0 ** 53 - 1))[0]
+        t[0], t[1] = low, 7
+        assert low & 0xFFFFFFFF == 0xFFFFFFFF and host.arrived(t) is None
+        t[2] = -(1 << 32)
+        assert host.arrived(t) == (low, 7, 2 ** 64 - 2 ** 32)
+        assert host.arrived(t[:1]) == (low,)
+        print("done")
+        """)
