@@ -337,8 +337,8 @@ PyObject* norm_table(PyObject*, PyObject* args) {
 
 // Results that the host waits for come into words of its own, which the kernel writes one by one (st_host): a copy and
 // the stream's end behind it were 5 to 15 us of every wait, and what follows the kernel on the stream runs on.  With a
-// copy -> so, us: select of 3 M scores 56.6 -> 42, mask layout step on 1.15 M coordinates 122 -> 106, dense replay step
-// and two configurations of 1.5 M 1,930 -> 1,783, full step on 63 M 854 -> 835.  A block is one call's, from torch's
+// copy -> so, us: mask layout step on 1.15 M coordinates 122 -> 106, dense replay step and two configurations of 1.5 M
+// 1,930 -> 1,783, full step on 63 M 854 -> 835.  A block is one call's, from torch's
 // pool; it goes back when all of its words have been written.
 // words(n, wide): n results of 32 bits, or of 64, in pinned host memory, all bits set: none of them has arrived.
 // A result of 64 bits is stored and looked at in one piece: its halves may well have all bits set (2^53 - 1 as a

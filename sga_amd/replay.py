@@ -6,7 +6,7 @@ import torch
 
 from . import _lib as L
 from . import replay_kernels as K
-from .selection import read_result, select_exact_device
+from .selection import select_exact
 
 OPTIMIZERS = ("adamw", "adams")
 ADAMS_BIAS_CORRECTION = 1.0
@@ -58,17 +58,15 @@ def select_topk_flat(t, k, check=True):
     """Exact top-k of a non-negative finite fp32 device vector; boundary ties
     go to the lowest flat indices (``sga/replay.py:538-572``).  Returns
     (bool mask, threshold).  The whole select runs on the device; the single
-    host wait is for the threshold and the rejection counters; the mask follows
-    on the current stream."""
+    host wait is for its end: threshold, rejection counters and mask are there
+    when this returns."""
     L.require_dev(t)
     flat = t.reshape(-1)
     n = flat.numel()
     if k > n:
         raise ValueError(f"k={k} > N={n}")
     mask = torch.empty(n, dtype=torch.bool, device=flat.device)
-    res, _ = select_exact_device([flat], k, L.TIE_LOWEST_INDEX,
-                                 masks=[mask.view(torch.uint8)], res=L.words(8))
-    r = read_result(res)
+    r, _ = select_exact([flat], k, L.TIE_LOWEST_INDEX, masks=[mask.view(torch.uint8)])
     if check:
         if r.nonfinite:
             raise ValueError("select_topk_flat requires finite scores (NaN/Inf would "

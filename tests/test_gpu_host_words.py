@@ -46,7 +46,7 @@ def test_words_behind_a_long_queue(dev):
 
 
 def test_selects_in_a_row_keep_their_masks(dev):
-    """The result is there before the mask is written; the mask follows on the stream."""
+    """Each call's mask and threshold belong together, however many calls follow."""
     from sga_amd.replay import select_topk_flat
     scores = [torch.rand(n, generator=torch.Generator().manual_seed(n)).to(dev) for n in (5, 70_001, 3_000_017, 12_000_001)]
     got = [select_topk_flat(s, max(1, s.numel() // 50)) for s in scores for _ in range(3)]
@@ -75,3 +75,26 @@ def test_sums_whose_low_half_has_all_bits_set(dev, adams):
     for t in range(2):
         rep.step(t, g.to(dev), {"lr": [1e-3], "clip_grad": 0.0})
     assert [r["recon_grad_norm"] for r in rep.recon_steps] == [math.sqrt(2.0 ** 53 - 1)] * 2
+
+
+@pytest.mark.parametrize("n", [5000, 3_000_017, 12_000_001, 200_000_003])
+def test_a_select_returns_behind_its_mask(dev, n, monkeypatch):
+    """Mask and threshold are there when the call returns: on any stream, without an event."""
+    from types import SimpleNamespace
+    from sga_amd import config
+    from sga_amd.replay import select_topk_flat
+    from sga_amd.selection import TopkSelection, select_masks_histogram
+    monkeypatch.setattr(config, "_ARGS", SimpleNamespace(sga_selection_method="histogram",
+                                                         sga_selection_ratio_percent=2.0))
+    score = torch.rand(n, generator=torch.Generator(device=dev).manual_seed(n), device=dev)
+    views, k = [score[:n // 2], score[n // 2:]], int(round(n * 0.02))
+    plugin, other, main = TopkSelection(), torch.cuda.Stream(), torch.cuda.current_stream()
+    ties = int((score >= score.topk(k).values[-1]).sum())
+    for call in (lambda: [select_topk_flat(score, k)[0]], lambda: select_masks_histogram(views, k)[1],
+                 lambda: plugin.select(SimpleNamespace(grad_views=[score]))):
+        main.synchronize()
+        masks = call()
+        assert main.query()
+        with torch.cuda.stream(other):
+            on = sum(int(m.sum(dtype=torch.int64)) for m in masks)
+        assert on in (k, ties)                    # of the scores at the threshold as many as make k, or all
