@@ -289,7 +289,8 @@ def stream():
 
 def words(n, wide=False):
     """``n`` words of 32 bits (``wide``: of 64) in pinned host memory, none of which has arrived:
-    for results of that size that a kernel hands to the host while it waits (``arrived``)."""
+    for results of that size that a kernel, launched next on the current stream, hands to the
+    host while it waits (``arrived``).  Nobody else gets their memory before that kernel has ended."""
     return host().words(n, wide)
 
 

@@ -20,6 +20,8 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/core/CachingHostAllocator.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -339,14 +341,33 @@ PyObject* norm_table(PyObject*, PyObject* args) {
 // the stream's end behind it were 5 to 15 us of every wait, and what follows the kernel on the stream runs on.  With a
 // copy -> so, us: mask layout step on 1.15 M coordinates 122 -> 106, dense replay step and two configurations of 1.5 M
 // 1,930 -> 1,783, full step on 63 M 854 -> 835.  A block is one call's, from torch's
-// pool; it goes back when all of its words have been written.
+// pool.  It goes back with the tensor once all of its words have been written; a tensor that dies before (an error or
+// an interrupt between the launch and the wait) leaves it with an event of the stream, behind which nothing writes there.
 // words(n, wide): n results of 32 bits, or of 64, in pinned host memory, all bits set: none of them has arrived.
 // A result of 64 bits is stored and looked at in one piece: its halves may well have all bits set (2^53 - 1 as a
 // double), the whole of it never has.
+template <class W>
+bool written(const W* w, int64_t n) {
+  for (int64_t i = 0; i < n; ++i)
+    if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == (W)~(W)0) return false;
+  return true;
+}
 at::Tensor blank_words(int64_t n, bool wide = false) {
-  at::Tensor t = at::empty({n}, at::TensorOptions().dtype(wide ? at::kLong : at::kInt).pinned_memory(true));
-  memset(t.data_ptr(), 0xFF, (size_t)n * (wide ? 8 : 4));
-  return t;
+  const auto options = at::TensorOptions().dtype(wide ? at::kLong : at::kInt);
+  const at::Tensor block = at::empty({n}, options.pinned_memory(true));
+  memset(block.data_ptr(), 0xFF, (size_t)n * (wide ? 8 : 4));
+  const c10::impl::VirtualGuardImpl gpu(c10::DeviceType::CUDA);
+  const auto done = [block, n, wide, stream = gpu.getStream(gpu.getDevice())](void* p) {
+    if (wide ? written(static_cast<uint64_t*>(p), n) : written(static_cast<uint32_t*>(p), n)) return;
+    bool kept = false;
+    try {
+      const at::DataPtr& mem = block.storage().data_ptr();
+      kept = at::getHostAllocator(at::kCUDA)->record_event(mem.get(), mem.get_context(), stream);
+    } catch (...) {
+    }
+    if (!kept) (void)new at::Tensor(block);          // not the pool's, or no events any more: nobody else gets it
+  };
+  return at::from_blob(block.data_ptr(), {n}, done, options);
 }
 PyObject* words(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
@@ -360,18 +381,13 @@ PyObject* words(PyObject*, PyObject* args) {
 constexpr std::chrono::milliseconds kLook(20);
 template <class W>
 bool all_arrived(const W* w, int64_t n) {
-  const auto written = [&] {
-    for (int64_t i = 0; i < n; ++i)
-      if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == (W)~(W)0) return false;
-    return true;
-  };
   const auto end = std::chrono::steady_clock::now() + kLook;
   for (;;) {
     for (int i = 0; i < 64; ++i) {
-      if (written()) return true;
+      if (written(w, n)) return true;
       __builtin_ia32_pause();
     }
-    if (std::chrono::steady_clock::now() > end) return written();
+    if (std::chrono::steady_clock::now() > end) return written(w, n);
   }
 }
 // arrived(words) -> their values, or None where they have not come for some time

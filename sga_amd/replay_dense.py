@@ -75,13 +75,11 @@ class DenseReplay:
                int(self.optimizer == "adams"), float(coef_dense), L.ptr(self._partials),
                L.ptr(recon2), st)
         norm = float(gmeta.get("grad_norm", float("nan")))
-        try:
-            record = {
-                "step": gstep, "lr": lr_for_step(gmeta), "lr_max_abs_diff": lr_max_abs_diff(gmeta),
-                "grad_norm": norm, "clip_grad": float(gmeta.get("clip_grad", 0.0)),
-                "coef_dense": coef_dense, "reconstruct_flag": flag}
-        finally:
-            L.arrived(recon2)                         # before the words can be anyone else's
+        record = {
+            "step": gstep, "lr": lr_for_step(gmeta), "lr_max_abs_diff": lr_max_abs_diff(gmeta),
+            "grad_norm": norm, "clip_grad": float(gmeta.get("clip_grad", 0.0)),
+            "coef_dense": coef_dense, "reconstruct_flag": flag}
+        L.arrived(recon2)
         recon = math.sqrt(float(recon2.view(torch.float64).item()))
         record.update(recon_grad_norm=recon, recon_rel_err=((recon - norm) / norm
                                                             if math.isfinite(norm) and norm > 0.0 else None))

@@ -98,3 +98,76 @@ def test_a_select_returns_behind_its_mask(dev, n, monkeypatch):
         with torch.cuda.stream(other):
             on = sum(int(m.sum(dtype=torch.int64)) for m in masks)
         assert on in (k, ties)                    # of the scores at the threshold as many as make k, or all
+
+
+@pytest.mark.parametrize("wide", [False, True])
+def test_words_given_up_early_stay_out_of_the_pool(dev, wide):
+    """Whoever stops waiting (an interrupt, an error) leaves a kernel behind that has yet to write: nobody
+    else's words lie there before it has; afterwards the memory is used again."""
+    from sga_amd import _lib as L
+    big = torch.empty(1 << 28, device=dev)
+    x, partials = torch.ones(5000, device=dev), torch.empty(2048, device=dev)
+    grad, idx, values = torch.ones(9, device=dev), torch.arange(5, dtype=torch.int32, device=dev), torch.empty(5, device=dev)
+
+    def launch():
+        w = L.words(1, wide)
+        if wide:
+            L.call("sga_pack_selected_split", L.ptr(grad), L.ptr(idx), L.ptr(values), L.SGA_F32, 1.0, 5, 9, 3, L.ptr(w),
+                   L.stream())
+        else:
+            L.call("sga_compact_norm_sq_from", L.ptr(x), 5000, L.ptr(partials), None, L.ptr(w), L.stream())
+        return w
+    assert L.arrived(launch()) == ((3,) if wide else (0x459C4000,))
+    torch.cuda.synchronize()
+    for _ in range(150):                          # some 40 ms of fills
+        big.zero_()
+    given_up = [launch() for _ in range(4)]
+    there = {w.data_ptr() for w in given_up}
+    del given_up
+    assert not torch.cuda.current_stream().query()
+    later = [L.words(1, wide) for _ in range(40)]
+    assert not there & {w.data_ptr() for w in later}
+    torch.cuda.synchronize()
+    assert all(w.item() == -1 for w in later)
+    del later
+    torch.cuda.synchronize()
+    seen = set()
+    for _ in range(300):
+        w = launch()
+        L.arrived(w)
+        seen.add(w.data_ptr())
+        del w
+    assert len(seen) < 100
+
+
+@pytest.mark.parametrize("call", ["index", "mask", "norm"])
+def test_an_interrupted_wait(dev, call, monkeypatch):
+    """The next call has its own words, whatever the one before has left on the stream."""
+    from sga_amd import _lib as L
+    from sga_amd.backends import index_layout_pack, mask_layout_pack
+    from sga_amd.kernels import compact_norm
+    n = 100_000
+    mask = torch.zeros(n, dtype=torch.uint8, device=dev)
+    mask[1::7] = 1
+    idx, grad = mask.nonzero().view(-1).to(torch.int32), torch.ones(n, device=dev)
+    values, big = torch.empty(idx.numel(), device=dev), torch.empty(1 << 28, device=dev)
+    run = {"index": lambda m: index_layout_pack(grad, idx[:m], values)[0][1], "mask": lambda m: mask_layout_pack(
+        grad, mask * (m > 0))[1].numel(), "norm": lambda m: compact_norm([grad[:m]])}[call]
+    want = {"index": lambda m: min(m, int((idx < n // 2).sum())), "mask": lambda m: idx.numel(),
+            "norm": lambda m: float(torch.tensor(float(m)).sqrt())}[call]
+    run(10)
+    torch.cuda.synchronize()
+    arrived = L.arrived
+
+    def interrupted(t):
+        raise KeyboardInterrupt
+    for _ in range(150):
+        big.zero_()
+    monkeypatch.setattr(L, "arrived", interrupted)
+    for _ in range(4):
+        with pytest.raises(KeyboardInterrupt):
+            run(77)
+    monkeypatch.setattr(L, "arrived", arrived)
+    grad.fill_(1.0)
+    for m in (500, 9000, 3):
+        assert run(m) == want(m)
