@@ -431,16 +431,22 @@ PyObject* norm(PyObject*, PyObject* args) {
   // the partials, fp32; every slot that is read is written first.  The total comes into host memory (a copy of it is
   // a launch, and 3 us of the wait).
   at::Tensor buf = at::empty({spans}, at::TensorOptions().dtype(at::kFloat).device(table.device()));
-  const at::Tensor word = table.is_cuda() ? blank_words(1) : at::empty({1}, at::kInt);
+  const at::Tensor word = table.is_cuda() ? blank_words(1) : at::full({1}, -1, at::kInt);
   const int rc = f_norm_multi(static_cast<const sga_span_record*>(table.data_ptr()), n_rows, spans,
                               static_cast<float*>(buf.data_ptr()), static_cast<float*>(word.data_ptr()), (void*)stream);
   if (rc != 0) return PyLong_FromLong(rc);
-  const double total = [&] {
+  const uint32_t* w = static_cast<const uint32_t*>(word.data_ptr());
+  const bool there = [&] {
     Unlocked released;
     // not there in time: a read from the device waits for the stream, and raises its errors
-    if (!table.is_cuda() || !all_arrived(static_cast<const uint32_t*>(word.data_ptr()), 1)) (void)buf[0].item<float>();
-    return *static_cast<const volatile float*>(word.data_ptr());
+    if (!table.is_cuda() || !all_arrived(w, 1)) (void)buf[0].item<float>();
+    return written(w, 1);
   }();
+  if (!there) {
+    PyErr_SetString(PyExc_RuntimeError, "norm: a result that its kernel should have written has not arrived");
+    return nullptr;
+  }
+  const double total = *static_cast<const float*>(word.data_ptr());
   return PyFloat_FromDouble((double)(float)std::sqrt(total));
   END_HANDLE_TH_ERRORS
 }

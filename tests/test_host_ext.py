@@ -124,3 +124,15 @@ def test_results_of_64_bits_arrive_in_one_piece():
         assert host.arrived(t[:1]) == (low,)
         print("done")
         """)
+
+
+def test_a_norm_that_no_kernel_has_written_raises():
+    """The bound function here writes nothing: its word is no norm (read as a float it is NaN)."""
+    _run("""
+        host.bind(object, addr, addr, addr, addr)
+        try:
+            print(host.norm(torch.zeros(64, dtype=torch.uint8), 1, 1, 0))
+        except RuntimeError as e:
+            assert "not arrived" in str(e), e
+            print("done")
+        """)
