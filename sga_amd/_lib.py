@@ -211,7 +211,18 @@ def load():
     return lib
 
 
-_host = None
+_host = _host_loads = None
+
+
+def host_loads():
+    """Whether the native host side is there; without it results come by a copy (``words``)."""
+    global _host_loads
+    if _host_loads is None:
+        try:
+            _host_loads = host() is not None
+        except RuntimeError:
+            _host_loads = False
+    return _host_loads
 
 
 def host():
@@ -290,13 +301,18 @@ def stream():
 def words(n, wide=False):
     """``n`` words of 32 bits (``wide``: of 64) in pinned host memory, none of which has arrived:
     for results of that size that a kernel, launched next on the current stream, hands to the
-    host while it waits (``arrived``).  Nobody else gets their memory before that kernel has ended."""
+    host while it waits (``arrived``).  Nobody else gets their memory before that kernel has ended.
+    Without the native host side they lie on the device, and ``arrived`` copies them."""
+    if not host_loads():
+        return torch.empty(n, dtype=torch.int64 if wide else torch.int32, device="cuda")
     return host().words(n, wide)
 
 
 def arrived(t):
     """The words of ``t`` as unsigned ints, waited for; the launch that writes them is on
     the current stream."""
+    if t.is_cuda:
+        return t.tolist()
     got = host().arrived(t)
     if got is None:                      # a long kernel ahead of it, or an error: the stream tells
         torch.cuda.current_stream().synchronize()

@@ -171,3 +171,40 @@ def test_an_interrupted_wait(dev, call, monkeypatch):
     grad.fill_(1.0)
     for m in (500, 9000, 3):
         assert run(m) == want(m)
+
+
+def test_results_without_the_native_host_side(dev, monkeypatch):
+    """Selects, compaction, the layouts, the compact norm and the dense replay need libsga_hip.so alone."""
+    from sga_amd import _lib as L
+    from sga_amd.backends import index_layout_pack, mask_layout_pack
+    from sga_amd.kernels import compact_norm
+    from sga_amd.replay import select_topk_flat
+    from sga_amd.replay_dense import DenseReplay
+    from sga_amd.selection import select_masks_histogram
+    from sga_amd.support import compact_mask_u8
+    n = 70_001
+    score = torch.rand(n, generator=torch.Generator().manual_seed(3)).to(dev)
+
+    def results():
+        mask, thresh = select_topk_flat(score, 700)
+        views = [score[:30_000], score[30_000:]]
+        t2, masks = select_masks_histogram(views, 700)
+        idx, before = compact_mask_u8(mask.view(torch.uint8), step=n // 3, cuts=2)
+        grad, values = score.clone(), torch.empty(700, device=dev)
+        bounds = index_layout_pack(grad, idx, values)
+        payloads, _ = mask_layout_pack(score, mask.view(torch.uint8))
+        rep = DenseReplay([dict(a=0, n=n, b1=0.9, b2=0.95, eps=1e-8, wd=0.0, group=0)], score, score * 0.1,
+                          score * score, 3)
+        rep.step(0, score, {"lr": [1e-3], "clip_grad": 0.0})
+        return ([mask, idx, grad, values, rep.w, *masks, *payloads],
+                [thresh, t2, before, bounds, compact_norm([score, values]), rep.recon_steps[0]["recon_grad_norm"]])
+    tensors, numbers = results()
+
+    def missing():
+        raise RuntimeError("sga_amd/_host.so is missing")
+    monkeypatch.setattr(L, "host", missing)
+    monkeypatch.setattr(L, "_host_loads", None)
+    t2, n2 = results()
+    assert all(torch.equal(a, b) for a, b in zip(tensors, t2)) and numbers[:4] == n2[:4]
+    # the root of the norm is the host's or the device's
+    assert numbers[5] == n2[5] and abs(numbers[4] - n2[4]) <= 2.0 ** -22 * numbers[4]
