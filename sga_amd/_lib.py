@@ -302,8 +302,10 @@ def words(n, wide=False):
     """``n`` words of 32 bits (``wide``: of 64) in pinned host memory, none of which has arrived:
     for results of that size that a kernel, launched next on the current stream, hands to the
     host while it waits (``arrived``).  Nobody else gets their memory before that kernel has ended.
-    Without the native host side they lie on the device, and ``arrived`` copies them."""
-    if not host_loads():
+    Without the native host side they lie on the device, and ``arrived`` copies them; so they do
+    while a graph is recorded, which must not write into the host's memory at its replays (the copy
+    refuses: nothing arrives during a recording)."""
+    if torch._C._cuda_isCurrentStreamCapturing() or not host_loads():
         return torch.empty(n, dtype=torch.int64 if wide else torch.int32, device="cuda")
     return host().words(n, wide)
 

@@ -208,3 +208,21 @@ def test_results_without_the_native_host_side(dev, monkeypatch):
     assert all(torch.equal(a, b) for a, b in zip(tensors, t2)) and numbers[:4] == n2[:4]
     # the root of the norm is the host's or the device's
     assert numbers[5] == n2[5] and abs(numbers[4] - n2[4]) <= 2.0 ** -22 * numbers[4]
+
+
+def test_a_recorded_graph_keeps_no_words_of_the_host(dev):
+    from sga_amd import _lib as L
+    grad, idx, values = torch.ones(9, device=dev), torch.arange(5, dtype=torch.int32, device=dev), torch.empty(5, device=dev)
+    L.arrived(L.words(0, True))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        below = L.words(1, wide=True)
+        L.call("sga_pack_selected_split", L.ptr(grad), L.ptr(idx), L.ptr(values), L.SGA_F32, 1.0, 5, 9, 3, L.ptr(below),
+               L.stream())
+    assert below.is_cuda
+    for _ in range(3):
+        below.fill_(-1)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert L.arrived(below) == [3]
+    assert not L.words(1).is_cuda
