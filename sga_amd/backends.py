@@ -30,7 +30,8 @@ def index_layout_pack(grad, idx, values, factor=1.0, slices=2):
     k = idx.numel()
     if slices != 2 or k == 0:
         out = index_layout_bounds(idx, grad.numel(), slices)
-        K.pack_selected(grad, idx, values, factor)     # the slices follow one another: one launch
+        if out:
+            K.pack_selected(grad, idx, values, factor)     # the slices follow one another: one launch
         return out
     below = L.words(1, wide=True)
     K.pack_selected(grad, idx, values, factor, below)  # ... and the bound comes with it, ahead of its end

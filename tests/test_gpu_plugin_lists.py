@@ -63,3 +63,11 @@ def test_mask_lists_on_views(dev):
         payloads, idx = mask_layout_pack(grad[off:], mask[off:], slices=2)
         assert torch.equal(torch.cat(payloads), grad[off:][mask[off:] != 0])
         assert torch.equal(idx.long(), mask[off:].nonzero().reshape(-1))
+
+
+@pytest.mark.parametrize("slices", [0, -1])
+def test_no_slices_pack_nothing(dev, slices):
+    from sga_amd.backends import index_layout_pack
+    grad, values = torch.ones(9, device=dev), torch.zeros(5, device=dev)
+    assert index_layout_pack(grad, torch.arange(5, dtype=torch.int32, device=dev), values, slices=slices) == []
+    assert grad.sum().item() == 9 and values.sum().item() == 0
