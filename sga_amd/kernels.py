@@ -47,11 +47,18 @@ def pack_selected(grad, indices, values, factor, below=None):
         L.call("sga_pack_selected_split", *args, grad.numel() // 2, L.ptr(below), L.stream())
 
 
+# Entries up to which a list in parts is one launch.  The look for an entry's part costs more than the launches it saves
+# beyond: two and five parts, a launch each -> one, us: 6.3 M entries of 63 M coordinates 65 -> 62 and 75 -> 64, 10 M of
+# 200 M 306 -> 309 and 305 -> 312, 20 M of 200 M 409 -> 415 and 402 -> 417, all of 63 M 194 -> 198 and 203 -> 216.
+_ONE_SCATTER = 8 << 20
+
+
 def scatter_parts(dst, indices, parts):
     """``scatter_selected`` of a list that lies in several arrays, one behind
     the other: one launch for up to eight of them."""
     counts = [p.numel() for p in parts]
     if (not 1 < len(parts) <= L.MAX_PARTS or sum(counts) != indices.numel() or indices.dtype != torch.int32
+            or indices.numel() > _ONE_SCATTER
             or not all(t.is_cuda and t.is_contiguous() for t in (dst, indices, *parts))
             or not all(t.dtype == torch.float32 for t in (dst, *parts)) or dst.numel() >= 2 ** 31):
         off = 0

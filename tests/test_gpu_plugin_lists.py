@@ -71,3 +71,15 @@ def test_no_slices_pack_nothing(dev, slices):
     grad, values = torch.ones(9, device=dev), torch.zeros(5, device=dev)
     assert index_layout_pack(grad, torch.arange(5, dtype=torch.int32, device=dev), values, slices=slices) == []
     assert grad.sum().item() == 9 and values.sum().item() == 0
+
+
+@pytest.mark.parametrize("k", [(8 << 20) - 1, 8 << 20, (8 << 20) + 1])
+def test_long_lists_in_parts(dev, k):
+    """Around the number of entries from which the parts are launches of their own."""
+    from sga_amd.kernels import scatter_parts
+    gen = torch.Generator(device=dev).manual_seed(k)
+    idx = torch.arange(k, dtype=torch.int32, device=dev) * 2
+    values = torch.randn(k, generator=gen, device=dev)
+    dst = torch.zeros(2 * k, device=dev)
+    scatter_parts(dst, idx, [values[:5].clone(), values[5:k // 2 + 3].clone(), values[k // 2 + 3:].clone()])
+    assert torch.equal(dst[::2], values) and not bool(dst[1::2].any())
