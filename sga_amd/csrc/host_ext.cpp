@@ -27,6 +27,7 @@
 
 #include <chrono>
 #include <cmath>
+#include <utility>
 #include <vector>
 
 #include "../../include/sga_hip.h"
@@ -352,22 +353,36 @@ bool written(const W* w, int64_t n) {
     if (__atomic_load_n(w + i, __ATOMIC_ACQUIRE) == (W)~(W)0) return false;
   return true;
 }
-at::Tensor blank_words(int64_t n, bool wide = false) {
-  const auto options = at::TensorOptions().dtype(wide ? at::kLong : at::kInt);
-  const at::Tensor block = at::empty({n}, options.pinned_memory(true));
-  memset(block.data_ptr(), 0xFF, (size_t)n * (wide ? 8 : 4));
-  const c10::impl::VirtualGuardImpl gpu(c10::DeviceType::CUDA);
-  const auto done = [block, n, wide, stream = gpu.getStream(gpu.getDevice())](void* p) {
-    if (wide ? written(static_cast<uint64_t*>(p), n) : written(static_cast<uint32_t*>(p), n)) return;
-    bool kept = false;
+struct Words {
+  at::DataPtr block;
+  int64_t n;
+  bool wide;
+  c10::Stream stream;
+  bool all_written() const {
+    return wide ? written(static_cast<uint64_t*>(block.get()), n) : written(static_cast<uint32_t*>(block.get()), n);
+  }
+  // of the tensor, on whichever thread drops it
+  static void release(void* ctx) {
+    auto* w = static_cast<Words*>(ctx);
+    bool ours = w->all_written();
     try {
-      const at::DataPtr& mem = block.storage().data_ptr();
-      kept = at::getHostAllocator(at::kCUDA)->record_event(mem.get(), mem.get_context(), stream);
+      if (!ours) ours = at::getHostAllocator(at::kCUDA)->record_event(w->block.get(), w->block.get_context(), w->stream);
     } catch (...) {
     }
-    if (!kept) (void)new at::Tensor(block);          // not the pool's, or no events any more: nobody else gets it
-  };
-  return at::from_blob(block.data_ptr(), {n}, done, options);
+    if (ours) delete w;                                // otherwise (a lost device) nobody gets the block any more
+  }
+};
+at::Tensor blank_words(int64_t n, bool wide = false) {
+  const size_t bytes = (size_t)n * (wide ? 8 : 4);
+  const c10::impl::VirtualGuardImpl gpu(c10::DeviceType::CUDA);
+  auto* w = new Words{at::getHostAllocator(at::kCUDA)->allocate(bytes), n, wide, gpu.getStream(gpu.getDevice())};
+  void* at = w->block.get();
+  if (bytes) memset(at, 0xFF, bytes);
+  c10::Storage mem(c10::Storage::use_byte_size_t(), bytes, at::DataPtr(at, w, &Words::release, at::kCPU), nullptr, false);
+  at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(std::move(mem), c10::DispatchKeySet(c10::DispatchKey::CPU),
+                                                          caffe2::TypeMeta::fromScalarType(wide ? at::kLong : at::kInt));
+  t.unsafeGetTensorImpl()->set_sizes_contiguous({n});
+  return t;
 }
 PyObject* words(PyObject*, PyObject* args) {
   HANDLE_TH_ERRORS
