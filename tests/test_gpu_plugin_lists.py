@@ -83,3 +83,17 @@ def test_long_lists_in_parts(dev, k):
     dst = torch.zeros(2 * k, device=dev)
     scatter_parts(dst, idx, [values[:5].clone(), values[5:k // 2 + 3].clone(), values[k // 2 + 3:].clone()])
     assert torch.equal(dst[::2], values) and not bool(dst[1::2].any())
+
+
+# rounds of the workgroup that adds up: of 1024 groups of 16 K bytes a thread each, of 16 K by runs of sixteen
+@pytest.mark.parametrize("n", [2 ** 24, 2 ** 24 + 1, 1040 * 2 ** 14 - 3, 1041 * 2 ** 14, 2 ** 28, 2 ** 28 + 1,
+                               3 * 2 ** 28 + 123_457])
+def test_long_masks(dev, n):
+    from sga_amd.support import compact_mask_u8
+    mask = torch.zeros(n, dtype=torch.uint8, device=dev)
+    on = torch.cat([torch.randint(0, n, (50_000,), generator=torch.Generator().manual_seed(n % 1009)),
+                    torch.arange(n - 40_000, n), torch.arange(0, n, 2 ** 14)]).unique().to(dev)
+    mask[on] = 2
+    idx, before = compact_mask_u8(mask, step=n // 3, cuts=3)
+    assert torch.equal(idx, on.to(torch.int32))
+    assert before == [int((on < (j + 1) * (n // 3)).sum()) for j in range(3)]
