@@ -2121,12 +2121,19 @@ __device__ __forceinline__ void tail_scan(const ChainJob& J, uint32_t b, uint32_
   // counters come and go a line a wave and instruction, by LDS; a thread scans a run of sixteen.  (By runs straight
   // from and to memory the scan of 18,190 chunks spent 4.5 us on its loads and 7.8 on its stores.)
   const int64_t base = (int64_t)b * kTileScanSpan;
-  auto runs = [](int i) { return i + i / kTileScanPer; };
-  const int mine = (int)threadIdx.x * (kTileScanPer + 1);
+  // Places in LDS by offsets from two numbers that the compiler does not know ahead of the queue's loop: held in registers
+  // throughout, the places cost the radix passes of scores that are chains of arithmetic half of their waves (a step by
+  // `coi` on 20 M coordinates whose k-th score 0.9 M share: 1,298 us, 997 so).
+  int tid = (int)threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  constexpr int kTurn = kBlock + kBlock / kTileScanPer;
+  static_assert(kBlock % kTileScanPer == 0, "word j * kBlock + i lies at j * kTurn + i + i / kTileScanPer");
+  uint32_t* const line = s.h + tid + tid / kTileScanPer;
+  uint32_t* const mine = s.h + tid * (kTileScanPer + 1);
   uint32_t g[kTileScanPer], e[kTileScanPer], my_g = 0, my_e = 0;
 #pragma unroll
   for (int j = 0; j < kTileScanPer; ++j) {
-    const int64_t at = base + j * kBlock + threadIdx.x;
+    const int64_t at = base + j * kBlock + tid;
     const bool ok = at < n_tiles;
     g[j] = ok ? (armed ? ld_agent(&J.tile_gt[at]) : J.tile_gt[at]) : 0u;
     e[j] = ok ? (armed ? ld_agent(&J.tile_eq[at]) : J.tile_eq[at]) : 0u;
@@ -2134,20 +2141,20 @@ __device__ __forceinline__ void tail_scan(const ChainJob& J, uint32_t b, uint32_
   auto turn = [&](uint32_t (&v)[kTileScanPer]) {      // from a word of every line to a run
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kTileScanPer; ++j) s.h[runs(j * kBlock + (int)threadIdx.x)] = v[j];
+    for (int j = 0; j < kTileScanPer; ++j) line[j * kTurn] = v[j];
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kTileScanPer; ++j) v[j] = s.h[mine + j];
+    for (int j = 0; j < kTileScanPer; ++j) v[j] = mine[j];
   };
   auto put = [&](const uint32_t (&v)[kTileScanPer], uint32_t* to) {
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kTileScanPer; ++j) s.h[mine + j] = v[j];
+    for (int j = 0; j < kTileScanPer; ++j) mine[j] = v[j];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kTileScanPer; ++j) {
-      const int64_t at = base + j * kBlock + threadIdx.x;
-      const uint32_t w = s.h[runs(j * kBlock + (int)threadIdx.x)];
+      const int64_t at = base + j * kBlock + tid;
+      const uint32_t w = line[j * kTurn];
       if (at >= n_tiles) continue;
       if (read_on) st_agent(&to[at], w);
       else to[at] = w;
