@@ -33,15 +33,16 @@ namespace sga {
 #ifdef __HIPCC__
 
 // Candidate lists of the small path: the chunks of the sweep share kSmallSegs counters (the segments of
-// the list); a segment has room for every coordinate of its chunks, so it never overflows.
+// the list), by units of a few chunks that reserve together and go round the segments; a segment has room for every
+// coordinate of its chunks, so it never overflows.
 // The counters lie 256 bytes apart: atomics on one cache line queue like those on one address (11 ns
 // each; 1024 workgroups on 16 adjacent words: the sweep of 4 M elements took 19 us, 8.6 with this).
 struct SmallGeom { uint32_t segs, cap; };          // cap: list entries per segment
-__host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles, int cpw) {
+__host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles, int unit) {
   SmallGeom s;
-  const uint32_t n_wg = (uint32_t)cdiv64(n_tiles, cpw), per = (uint32_t)cdiv64(n_wg, kSmallSegs);
-  s.segs = (uint32_t)cdiv64(n_wg, per);
-  s.cap = (per * cpw < 2 ? 2 : per * cpw) * (uint32_t)kChunk;      // two chunks hold the head that is read unseen
+  const uint32_t units = (uint32_t)cdiv64(n_tiles, unit), per = (uint32_t)cdiv64(units, kSmallSegs);
+  s.segs = (uint32_t)cdiv64(units, per);
+  s.cap = (per * unit < 2 ? 2 : per * unit) * (uint32_t)kChunk;      // two chunks hold the head that is read unseen
   return s;
 }
 
@@ -63,8 +64,12 @@ struct SmallChunk {
 // Sample, bracket and the one sweep over the data, one launch: the first kSampleGroups workgroups of a job take the
 // sample and one of them the bracket (sample_pick_body), one keeps house (directory and columns of the segment
 // table), the others sweep.  These request their data and form its keys while the bracket is on its way, and then
-// look for it in one of kSmallSegs copies.  Counts above the bracket, keys inside it to the list (one reservation per
-// workgroup).  Keys equal to the bracket's lower end are counted per chunk and not
+// look for it in one of kSmallSegs copies.  Counts above the bracket, keys inside it to the list.  A workgroup reserves
+// its entries together; in the front four chunks' entries, so that a workgroup that has all of the list spreads it over
+// the segments, each of which is one wave's work in the finish.  Selects at 1 %, a reservation per workgroup / per four
+// chunks, us: ascending scores 1.3 M 64 / 46, 3 M 75 / 54, 4.2 M 77 / 59; a fiftieth of the scores high, in one piece
+// 49 / 35, 47 / 41, 50 / 44; independent ones the same.
+// Keys equal to the bracket's lower end are counted per chunk and not
 // listed: a plateau of equal keys (zeros, momenta that have decayed to the last denormal) puts the
 // lower end on itself, and the one workgroup behind the sweep would walk a list as long as the bucket
 // (|m| after a thousand sparse steps, 1.7 M coordinates: 889 us, 86 like this).
@@ -91,8 +96,9 @@ constexpr int kSweepList = 2048;                     // entries of a workgroup t
 template <class Src, int WAVES, int SPW, bool WAIT, class Now>
 __device__ __forceinline__ void small_sweep_body(Src src, const ChainJob& J, const Now& now, uint32_t launch, int64_t blk) {
   constexpr int ROUND = WAVES / kChunkIters, CPW = ROUND * SPW, SLABS = WAVES * SPW;
+  constexpr int PARTS = WAIT ? SPW : 1, UNIT = CPW / PARTS;         // chunks of a reservation; slabs u * WAVES + w
   static_assert(SLABS <= kWave, "a lane per slab");
-  __shared__ uint32_t s_hi[SLABS], s_eq[SLABS], s_cnt[SLABS], s_nf[SLABS], s_got[3], s_base, s_fit;
+  __shared__ uint32_t s_hi[SLABS], s_eq[SLABS], s_cnt[SLABS], s_nf[SLABS], s_got[3], s_base[PARTS], s_off[PARTS], s_fit;
   __shared__ uint32_t s_lkey[WAIT ? kSweepList : 1], s_lidx[WAIT ? kSweepList : 1];
   const int64_t n = J.n, n_chunks = J.n_tiles, c0 = blk * CPW;
   if (c0 >= n_chunks) return;                         // a smaller job of the batch
@@ -164,15 +170,23 @@ __device__ __forceinline__ void small_sweep_body(Src src, const ChainJob& J, con
   // every wave sums the slabs' counts for itself; the first one reserves and writes the chunks' words meanwhile
   const uint32_t mine = lane_id() < SLABS ? s_cnt[lane_id()] : 0u, incl = wave_incl_scan(mine);
   const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+  // of the part that slab q lies in: where it begins in the workgroup's list (uniform q)
+  auto part_off = [&](int p) { return p ? (uint32_t)__builtin_amdgcn_readlane((int)incl, p * (SLABS / PARTS) - 1) : 0u; };
   if (w == 0) {
-    const SmallGeom geo = small_geom(n_chunks, CPW);
-    const uint32_t seg = (uint32_t)(blk % geo.segs);
-    uint32_t base = 0;
-    if (lane_id() == 0 && all) base = atomicAdd(&J.seg_cnt[seg * kSmallSegStride], all);
-    base = (uint32_t)uniform_i32((int)base);
-    const bool fit = base <= geo.cap && all <= geo.cap - base;
-    if (lane_id() == 0) { s_base = seg * geo.cap + base; s_fit = fit; }
+    const SmallGeom geo = small_geom(n_chunks, UNIT);
+    uint32_t base = 0, off = 0, cnt_p = all, seg = (uint32_t)(blk % geo.segs);      // of the lane's part
+#pragma unroll
+    for (int p = 0; PARTS > 1 && p < PARTS; ++p) {
+      const uint32_t from = part_off(p), to = p + 1 < PARTS ? part_off(p + 1) : all;
+      if (lane_id() == p) { off = from; cnt_p = to - from; seg = (uint32_t)((blk * PARTS + p) % geo.segs); }
+    }
+    const bool reserves = lane_id() < PARTS && cnt_p != 0u;
+    if (reserves) base = atomicAdd(&J.seg_cnt[seg * kSmallSegStride], cnt_p);
+    const uint32_t fits = (uint32_t)ballot64(!reserves || (base <= geo.cap && cnt_p <= geo.cap - base));      // a bit a part
+    if (lane_id() < PARTS) { s_base[lane_id()] = seg * geo.cap + base; s_off[lane_id()] = off; }
+    if (lane_id() == 0) s_fit = fits;
     if (lane_id() < CPW && c0 + lane_id() < n_chunks) {
+      const bool fit = (fits >> (lane_id() / UNIT) & 1u) != 0u;
       uint32_t hi = 0, eq = 0, cnt = 0, bad = 0, minus = 0;
 #pragma unroll
       for (int j = 0; j < kChunkIters; ++j) {
@@ -189,25 +203,28 @@ __device__ __forceinline__ void small_sweep_body(Src src, const ChainJob& J, con
   }
   const bool via_lds = WAIT && all <= (uint32_t)kSweepList;
   if (!via_lds) __syncthreads();                      // uniform; the list goes straight to its place then
-  if (!via_lds && !s_fit) return;
 #pragma unroll
   for (int u = 0; u < SPW; ++u) {
-    const int q = u * WAVES + w;
+    const int q = u * WAVES + w, p = PARTS > 1 ? u : 0;
     uint32_t run = (uint32_t)__builtin_amdgcn_readlane((int)(incl - mine), q);
     const uint32_t i = (uint32_t)(i1 + u * ROUND * kChunk + lane_id() * kVec);
     if (via_lds) {
       ballot_append(cand[u], run, [&](uint32_t pos, int e) { s_lidx[pos] = i + e; s_lkey[pos] = key[u][e]; });
-    } else {
-      run += s_base;
+    } else if (s_fit >> p & 1u) {
+      run += s_base[p] - s_off[p];
       ballot_append(cand[u], run, [&](uint32_t pos, int e) { J.small_idx[pos] = i + e; J.small_key[pos] = key[u][e]; });
     }
   }
   if (!via_lds) return;
   __syncthreads();
-  if (!s_fit) return;
   for (uint32_t t = threadIdx.x; t < all; t += WAVES * kWave) {
-    J.small_idx[s_base + t] = s_lidx[t];
-    J.small_key[s_base + t] = s_lkey[t];
+    int p = 0;
+#pragma unroll
+    for (int j = 1; j < PARTS; ++j) p += t >= s_off[j];
+    if (!(s_fit >> p & 1u)) continue;
+    const uint32_t at = s_base[p] + (t - s_off[p]);
+    J.small_idx[at] = s_lidx[t];
+    J.small_key[at] = s_lkey[t];
   }
 }
 template <class Src, int SPW>
@@ -424,7 +441,7 @@ __device__ __forceinline__ bool small_redo(Src& src, const ChainJob& J, uint32_t
 }
 
 template <class Src>
-__global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs, int cpw) {
+__global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, ChainJobs jobs, int unit) {
   __shared__ __align__(16) uint32_t s_hist[kBinsBig + kWave];     // behind the bins, a word per lane for what is in none
   __shared__ __align__(16) uint32_t s_tile[kSmallTiles];          // above | ties << 16, at most 1024 each
   __shared__ __align__(16) uint32_t s_key[kWideList];
@@ -437,7 +454,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   const int nt = (int)J.n_tiles;
   const uint32_t k = J.k, T_LO = st->t_lo, T_HI = st->t_hi;
   const bool single = T_HI - T_LO == 1u;
-  const SmallGeom geo = small_geom(nt, cpw);
+  const SmallGeom geo = small_geom(nt, unit);
   SmallList list;
   list.request(J, geo);
   constexpr int PER = kSmallTiles / kWide;            // 8
@@ -717,7 +734,7 @@ static inline void run_small_select(const SrcPack<Src>& srcs, const SelBatch& B,
   }
   const int64_t wgs = cdiv64(B.max_tiles, kRedoTiles);
   hipLaunchKernelGGL((k_small_finish<Src>), B.grid((unsigned)(wgs < kRedoGroups ? wgs : kRedoGroups)), dim3(kWide), 0,
-                     s, srcs, B.jobs, cpw);
+                     s, srcs, B.jobs, together ? ROUND : cpw);
 }
 
 #endif  // __HIPCC__

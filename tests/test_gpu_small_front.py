@@ -116,3 +116,18 @@ def test_tables_of_many_tensors(dev, n, tensors):
         ends.append([idx, val, *state])
     for a, b in zip(*ends):
         assert torch.equal(a, b) if a.dtype != torch.float32 else same_bits(a, b)
+
+
+# a workgroup's sixteen chunks reserve by fours: the whole list in one of them, over its parts and those of its neighbour
+@pytest.mark.parametrize("chunks", [1025, 1031, 2500, 4096])
+@pytest.mark.parametrize("how", ["ascending", "descending", "piece"])
+def test_lists_of_one_workgroup(dev, chunks, how):
+    n = CHUNK * chunks - 3
+    sc = torch.rand(n, generator=torch.Generator().manual_seed(chunks)).sort(descending=how == "descending").values
+    if how == "piece":
+        sc = sc[torch.randperm(n, generator=torch.Generator().manual_seed(1))]
+        sc[n // 3:n // 3 + n // 60] += 8
+    for k in (200, n // 100, n // 10):
+        want, thresh = SEL.select_topk_flat(sc, k)
+        r, mask = _select(dev, sc, k)
+        assert (r.n_selected, r.thresh, r.path) == (k, thresh, 1) and torch.equal(mask, want), k
