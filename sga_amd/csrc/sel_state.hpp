@@ -1,5 +1,5 @@
-// State of a select in its workspace, and the hand-over of a sample's keys between the workgroups of one
-// launch (k_sample_pick).  No HIP in here: the host compiles it too.
+// State of a select in its workspace, the hand-over of a sample's keys between the workgroups of one
+// launch (sample_pick_body), and of the small buckets' counts to the finish.  No HIP in here: the host compiles it too.
 #pragma once
 #include <stddef.h>
 #include <stdint.h>
@@ -77,5 +77,30 @@ static_assert(offsetof(SelState, k) == 0, "word 0 is the rank");
 SGA_HOST_DEVICE static inline unsigned long long picked_word(int w, uint32_t k, uint32_t t_lo, uint32_t t_hi) {
   return w == 0 ? k : w == kBracketWord ? (unsigned long long)t_hi << 32 | t_lo : 0ull;
 }
+
+// What a chunk's two words carry from the sweep to the finish, numbers up to 1024 in halves whose sums over the eight
+// chunks of a thread fit (an instruction per chunk is 0.07 us of the finish at 8 M coordinates):
+//   a   keys above the bracket | ten bits of the bracket's tag | listed keys
+//   b   keys equal to the lower end | a value was negative | no bracket, or no room | eight more of the tag | non-finite keys
+struct SmallChunk {
+  static constexpr uint32_t kNumbers = 0x07FF07FFu, kNegative = 1u << 11, kLost = 1u << 12;
+  uint32_t a, b;
+  // the words of a chunk without a key in it, under the bracket [lo, hi)
+  SGA_HOST_DEVICE static inline SmallChunk none(uint32_t lo, uint32_t hi) {
+    uint32_t x = lo * 0x9E3779B1u ^ hi * 0x85EBCA6Bu;
+    x = (x ^ (x >> 15)) * 0x2C1B3C6Du;
+    return SmallChunk{(x & 0xF800F800u), ((x << 8) & 0xF8000000u) | ((x >> 3) & 0xE000u)};
+  }
+  SGA_HOST_DEVICE static inline SmallChunk of(uint32_t lo, uint32_t hi, uint32_t above, uint32_t listed, uint32_t equal,
+                                              uint32_t nonfinite, bool negative, bool lost) {
+    const SmallChunk z = none(lo, hi);
+    return SmallChunk{z.a | above | listed << 16,
+                      z.b | equal | nonfinite << 16 | (negative ? kNegative : 0u) | (lost ? kLost : 0u)};
+  }
+  // off_a, off_b: where words differ from none() of the state's bracket.  True: a chunk of another bracket, or a lost one.
+  SGA_HOST_DEVICE static inline bool wrong(uint32_t off_a, uint32_t off_b) {
+    return ((off_a | (off_b & ~kNegative)) & ~kNumbers) != 0u;
+  }
+};
 
 }  // namespace sga

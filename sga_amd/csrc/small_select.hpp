@@ -46,21 +46,6 @@ __host__ __device__ static inline SmallGeom small_geom(int64_t n_tiles, int unit
   return s;
 }
 
-// What a chunk's two words carry from the sweep to the finish, numbers up to 1024 in halves whose sums over the eight
-// chunks of a thread fit (an instruction per chunk is 0.07 us of the finish at 8 M coordinates):
-//   a   keys above the bracket | ten bits of the bracket's tag | listed keys
-//   b   keys equal to the lower end | a value was negative | no bracket, or no room | eight more of the tag | non-finite keys
-struct SmallChunk {
-  static constexpr uint32_t kNumbers = 0x07FF07FFu, kNegative = 1u << 11, kLost = 1u << 12;
-  uint32_t a, b;
-  // the words of a chunk without a key in it, under the bracket [lo, hi)
-  static __device__ __forceinline__ SmallChunk none(uint32_t lo, uint32_t hi) {
-    uint32_t x = lo * 0x9E3779B1u ^ hi * 0x85EBCA6Bu;
-    x = (x ^ (x >> 15)) * 0x2C1B3C6Du;
-    return SmallChunk{(x & 0xF800F800u), ((x << 8) & 0xF8000000u) | ((x >> 3) & 0xE000u)};
-  }
-};
-
 // Sample, bracket and the one sweep over the data, one launch: the first kSampleGroups workgroups of a job take the
 // sample and one of them the bracket (sample_pick_body), one keeps house (directory and columns of the segment
 // table), the others sweep.  These request their data and form its keys while the bracket is on its way, and then
@@ -194,9 +179,7 @@ __device__ __forceinline__ void small_sweep_body(Src src, const ChainJob& J, con
         hi += s_hi[q]; eq += s_eq[q]; cnt += s_cnt[q];
         bad += s_nf[q] & 0x7FFFFFFFu; minus |= s_nf[q] >> 31;
       }
-      SmallChunk ch = SmallChunk::none(T_LO, T_HI);
-      ch.a |= hi | cnt << 16;
-      ch.b |= eq | bad << 16 | (minus ? SmallChunk::kNegative : 0u) | (!fit || (WAIT && s_got[2] == 0u) ? SmallChunk::kLost : 0u);
+      const SmallChunk ch = SmallChunk::of(T_LO, T_HI, hi, cnt, eq, bad, minus != 0u, !fit || (WAIT && s_got[2] == 0u));
       J.tile_gt[c0 + lane_id()] = ch.a;
       J.tile_eq[c0 + lane_id()] = ch.b;
     }
@@ -477,7 +460,7 @@ __global__ __launch_bounds__(kWide) void k_small_finish(SrcPack<Src> srcs, Chain
   const uint32_t hi = sum_a & 0xFFFFu, eqs = sum_b & 0xFFFFu, nonfinite = sum_b >> 16;
   uint32_t listed = sum_a >> 16;
   const bool minus = (off_b & SmallChunk::kNegative) != 0u;
-  const bool wrong = ((off_a | (off_b & ~SmallChunk::kNegative)) & ~SmallChunk::kNumbers) != 0u;
+  const bool wrong = SmallChunk::wrong(off_a, off_b);
   reinterpret_cast<U4*>(s_hist)[threadIdx.x] = U4{0u, 0u, 0u, 0u};
   if (threadIdx.x < kWideWaves)
     s_seg[threadIdx.x] = threadIdx.x < geo.segs ? J.seg_cnt[threadIdx.x * kSmallSegStride] : 0u;

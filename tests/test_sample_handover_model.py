@@ -1,6 +1,7 @@
-"""Host-side model of how the workgroups of ``k_sample_pick``
-(csrc/select_impl.hpp) hand their sample keys over inside one launch, and the
-pieces of it that the host can compile (csrc/sel_state.hpp).
+"""Host-side models of how the workgroups of ``k_sample_pick`` and
+``k_small_front`` (csrc/select_impl.hpp, csrc/small_select.hpp) hand their
+sample keys and the bracket over inside one launch, and the pieces of it that
+the host can compile (csrc/sel_state.hpp).
 
 A workgroup stores its keys, then the launch's number as its mark, then looks
 at all marks; whoever sees every mark reads all keys, picks a bracket and
@@ -10,7 +11,15 @@ pick from keys that are not there yet.  The model runs every order of the
 steps of three workgroups over every such memory and checks what the select
 needs: a key indexes the pick's histogram in range, and the bracket left
 behind is one picking workgroup's own.  The protocol that this one replaced
-(keys as they come, the two ends as two stores) gives neither."""
+(keys as they come, the two ends as two stores) gives neither.
+
+In the small buckets' front others wait for the bracket.  There the first
+workgroup clears the state and the list's counters before its mark, a pick
+writes the bracket and its copies alone, and the finish, a kernel behind it,
+clears marks and copies.  The second model adds a sweeping workgroup and the
+finish's judgement: whatever the memory held and in whatever order things
+happen, a select that the finish accepts has counted all of its keys by the
+state's own bracket, and everything else is done again over the data."""
 import os
 import subprocess
 
@@ -88,6 +97,92 @@ def test_a_mark_can_come_after_the_clearing():
     assert any(any(left) for m in _MEMORIES for *_, left in _runs(m, masked=True, one_word=True))
 
 
+# The front: two workgroups of the sample, two that sweep, and the finish.  A sweeping workgroup has two keys; one of
+# them lies in either bracket that a pick can leave here, so that each reserves one entry of the list's counter.
+PAIR = (0x10000000, 0x20000000)
+
+
+def _front(marks, copy_held, counter_held, state_held, clears=True, tags=True):
+    """All ends of one launch of the front: ``(accepted, brackets the sweeps used, bracket in the state, listed,
+    counter)``."""
+    ends, seen = set(), set()
+    # sample: 0 clear (the first alone), 1 store keys, 2 store mark, 3 look, 4 read and pick, 5 copies, 6 state, None
+    # sweep:  0 look for the bracket (or give up), 1 reserve and write the chunk's words, None
+    start = ((0, 1), (0, 0), (STALE, STALE), tuple(marks), (None, None), copy_held, counter_held, state_held,
+             (None, None), 0)
+    todo = [start]
+    while todo:
+        at = todo.pop()
+        if at in seen:
+            continue
+        seen.add(at)
+        pcs, spcs, words, marks_, picks, copy, counter, bracket, used, listed = at
+        if all(pc is None for pc in pcs + spcs):
+            # the finish: of one bracket, the state's, nobody lost, and as many listed as the counter says
+            ok = listed == counter and (not tags or all(u == bracket for u in used))
+            ends.add((ok, used, bracket, listed, counter))
+            continue
+        for g, pc in enumerate(pcs):
+            if pc is None:
+                continue
+            w, m, p, cp, cn, b, nxt = list(words), list(marks_), list(picks), copy, counter, bracket, pc + 1
+            if pc == 0:
+                if clears:
+                    cn, b = 0, None
+            elif pc == 1:
+                w[g] = PAIR[g]
+            elif pc == 2:
+                m[g] = NUMBER
+            elif pc == 3:
+                nxt = 4 if all(x == NUMBER for x in m) else None
+            elif pc == 4:
+                keys = [x & 0x7FFFFFFF for x in w]
+                p[g] = (min(keys), max(keys) + 1)
+            elif pc == 5:
+                cp = (NUMBER, p[g])
+            else:
+                b, nxt = p[g], None
+            todo.append((pcs[:g] + (nxt,) + pcs[g + 1:], spcs, tuple(w), tuple(m), tuple(p), cp, cn, b, used, listed))
+        for g, pc in enumerate(spcs):
+            if pc is None:
+                continue
+            if pc == 0:
+                looks = [None]                                     # gives up, without a bracket
+                if copy[0] == NUMBER:
+                    looks.append(copy[1])
+                for got in looks:
+                    todo.append((pcs, spcs[:g] + (1,) + spcs[g + 1:], words, marks_, picks, copy, counter, bracket,
+                                 used[:g] + (got if got else "lost",) + used[g + 1:], listed))
+            else:
+                here = used[g] != "lost"
+                todo.append((pcs, spcs[:g] + (None,) + spcs[g + 1:], words, marks_, picks, copy, counter + here, bracket,
+                             used, listed + here))
+    return ends
+
+
+_OTHER = (0x30000000, 0x30000001)
+_FRONTS = [(m, c, n, s) for m in ((0, 0), (NUMBER, 0), (0, NUMBER), (NUMBER, NUMBER))
+           for c in ((0, None), (NUMBER, _OTHER)) for n in (0, 5, -1) for s in (None, _OTHER)]
+
+
+@pytest.mark.parametrize("marks,copy,counter,state", _FRONTS)
+def test_what_the_finish_accepts_is_one_bracket_and_all_keys(marks, copy, counter, state):
+    ends = _front(marks, copy, counter, state)
+    assert any(ok for ok, *_ in ends)
+    for ok, used, bracket, listed, held in ends:
+        if ok:
+            assert used == (bracket, bracket) and listed == held == 2
+    if not any(marks) and copy[0] != NUMBER:                       # cleared before: only a lost one is not accepted
+        assert all(ok or "lost" in used for ok, used, *_ in ends)
+
+
+def test_neither_the_clearing_nor_the_tags_can_be_left_out():
+    """Stale counters alone: entries that the finish would read, and nobody wrote.  Another bracket alone: counts
+    that add up, by two brackets."""
+    assert all(not ok for ok, *_ in _front((0, 0), (0, None), 5, None, clears=False))
+    assert any(ok and len(set(used)) == 2 for ok, used, *_ in _front((0, 0), (NUMBER, _OTHER), 0, None, tags=False))
+
+
 def test_one_count_of_launches_in_the_library():
     lib = os.path.join(ROOT, "sga_amd", "libsga_hip.so")
     names = subprocess.run(["nm", "-C", lib], capture_output=True, text=True, check=True).stdout
@@ -122,6 +217,32 @@ int main() {
     bad += x == 0u || (seen[x >> 3] >> (x & 7) & 1);
     seen[x >> 3] |= (unsigned char)(1u << (x & 7));
   }
+  // a chunk's words: numbers come back from the sums of eight chunks, a foreign bracket and a lost one do not pass
+  const uint32_t nums[] = {0u, 1u, 511u, 1023u, 1024u};
+  for (uint32_t lo : {0u, 1u, 0x3F000001u, 0x7F7FFFFFu, 0x7FFFFFFFu})
+    for (uint32_t hi : {lo + 1u, lo + 0x1000u, 0x80000000u})
+      for (uint32_t above : nums)
+        for (uint32_t listed : nums)
+          for (uint32_t equal : nums)
+            for (int flags = 0; flags < 4; ++flags) {
+              const uint32_t nf = (above * 7u + equal) % 1025u;
+              const bool neg = flags & 1, lost = flags & 2;
+              const SmallChunk c = SmallChunk::of(lo, hi, above, listed, equal, nf, neg, lost), z = SmallChunk::none(lo, hi);
+              uint32_t sa = 0, sb = 0;
+              for (int j = 0; j < 8; ++j) { sa += c.a & SmallChunk::kNumbers; sb += c.b & SmallChunk::kNumbers; }
+              bad += (sa & 0xFFFFu) != 8u * above || sa >> 16 != 8u * listed || (sb & 0xFFFFu) != 8u * equal || sb >> 16 != 8u * nf;
+              bad += (((c.b ^ z.b) & SmallChunk::kNegative) != 0u) != neg || SmallChunk::wrong(c.a ^ z.a, c.b ^ z.b) != lost;
+            }
+  // another bracket: 18 bits of a tag, so that a few in 2^18 pass
+  uint32_t x = 1u;
+  int missed = 0;
+  for (int i = 0; i < 1 << 18; ++i) {
+    x = x * 1664525u + 1013904223u;
+    const uint32_t lo = x >> 1, lo2 = lo ^ (1u << (i % 31)), hi = lo + 1u + (x & 0xFFFFu);
+    const SmallChunk c = SmallChunk::of(lo2, hi, 3u, 5u, 7u, 0u, false, false), z = SmallChunk::none(lo, hi);
+    missed += !SmallChunk::wrong(c.a ^ z.a, c.b ^ z.b);
+  }
+  bad += missed > 16;
   std::printf("%d\n", bad);
   return bad != 0;
 }
