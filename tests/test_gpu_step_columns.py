@@ -1,5 +1,6 @@
 """Learning rates and bias corrections that a step takes along: the same bits as with the tables brought up
-to date by a launch of their own, whatever path the bucket's select takes."""
+to date by a launch of their own, whatever path the bucket's select takes: small or large, or by radix passes
+(``fast=False``), whose steps bring the table up to date by that launch themselves."""
 import pytest
 import torch
 
@@ -18,7 +19,7 @@ def _bucket(dev, n, tensors, seed):
     return FusedSparseStep(n, segs, dev, max_k=k_for(n, 1.0), want_mask=True), state, grads
 
 
-def _run(dev, ahead, n, tensors, rates, score, buckets):
+def _run(dev, ahead, n, tensors, rates, score, buckets, fast=True):
     from sga_amd.fused_step import fused_step_multi, k_for
     sets = [_bucket(dev, m, t, 7 + i) for i, (m, t) in enumerate(zip(n, tensors))]
     out = []
@@ -31,10 +32,10 @@ def _run(dev, ahead, n, tensors, rates, score, buckets):
         gs = [grads[step - 1] for _fs, _state, grads in sets]
         if buckets:
             packs = fused_step_multi([s[0] for s in sets], gs, *zip(*[s[1] for s in sets]), step,
-                                     ratio_percent=1.0, score=score)
+                                     ratio_percent=1.0, score=score, fast=fast)
         else:
             fs, state, _grads = sets[0]
-            packs = [fs.step(gs[0], *state, step, k=k_for(n[0], 1.0), score=score, fast=ahead != "radix")]
+            packs = [fs.step(gs[0], *state, step, k=k_for(n[0], 1.0), score=score, fast=fast)]
         out += [t.clone() for p in packs for t in p]
         out += [t.clone() for fs, state, _grads in sets for t in (*state, fs.mask)]
     return out
@@ -45,17 +46,16 @@ def _run(dev, ahead, n, tensors, rates, score, buckets):
 @pytest.mark.parametrize("n,tensors,rates", [(5000, 3, 3), (1_200_001, 480, 4), (1_200_001, 481, 4), (300_000, 40, 11),
                                              (9_000_001, 100, 2)])
 def test_columns_by_argument(dev, n, tensors, rates, score):
-    a = _run(dev, False, [n], [tensors], rates, score, False)
-    b = _run(dev, True, [n], [tensors], rates, score, False)
-    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    ends = [_run(dev, ahead, [n], [tensors], rates, score, False, fast) for fast in (True, False) for ahead in (False, True)]
+    assert all(torch.equal(x, y) for end in ends[1:] for x, y in zip(ends[0], end))
 
 
 @pytest.mark.parametrize("n,tensors", [((4097, 70_001, 1, 1_500_000), (5, 60, 1, 200)),
                                        ((200_001,) * 10, (50,) * 10), ((300_000, 9_000_001, 8_500_000), (7, 9, 400))])
 def test_columns_of_several_buckets(dev, n, tensors):
     a = _run(dev, False, n, tensors, 2, "update", True)
-    b = _run(dev, True, n, tensors, 2, "update", True)
-    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    for ahead, fast in ((True, True), (False, False), (True, False)):
+        assert all(torch.equal(x, y) for x, y in zip(a, _run(dev, ahead, n, tensors, 2, "update", True, fast)))
     single = [t for i in range(len(n)) for t in _run_one(dev, n, tensors, i)]
     assert all(torch.equal(x, y) for x, y in zip(a[-5 * len(n):], single))
 
