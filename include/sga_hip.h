@@ -216,7 +216,10 @@ int sga_mask_count_cuts(const uint8_t* mask, int64_t n, uint32_t* chunk_counts,
 int sga_mask_fill(const uint8_t* mask, int64_t n, const uint32_t* chunk_offsets,
                   int32_t* idx_out, int64_t idx_capacity, void* stream);
 
-/* The same in two launches before the read of the totals and one behind it.
+/* The same in two launches before the read of the totals and one behind it,
+ * which is the way of the Python calls; sga_mask_count_cuts and sga_mask_fill
+ * stay for callers of the C interface, whose scratch and order of calls are
+ * theirs.
  * sga_mask_totals: totals as sga_mask_count_cuts gives them (n >= 1); scratch
  * has sga_mask_list_words(n) uint32 entries and is what sga_mask_list, on the
  * same mask, starts from.

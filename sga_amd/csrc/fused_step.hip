@@ -462,7 +462,7 @@ static int run_fused(const FusedJob* fj, int count, float factor, float coeff, i
     small = small && SelBatch::small_ok(fj[b].n);
     use_fast = use_fast && SelBatch::fast_ok(fj[b].w, fj[b].n);
   }
-  if (small) use_fast = false;       // three launches do the whole select (small_select.hpp)
+  if (small) use_fast = false;       // two or three launches do the whole select (small_select.hpp)
   NowCols cols = {};
   bool carried = small || use_fast;
   for (int b = 0; b < count && carried; ++b) {

@@ -81,7 +81,8 @@ SGA_HOST_DEVICE static inline unsigned long long picked_word(int w, uint32_t k, 
 // What a chunk's two words carry from the sweep to the finish, numbers up to 1024 in halves whose sums over the eight
 // chunks of a thread fit (an instruction per chunk is 0.07 us of the finish at 8 M coordinates):
 //   a   keys above the bracket | ten bits of the bracket's tag | listed keys
-//   b   keys equal to the lower end | a value was negative | no bracket, or no room | eight more of the tag | non-finite keys
+//   b   keys equal to the lower end | a value was negative | no bracket, or no room | eight more of the tag |
+//       non-finite keys
 struct SmallChunk {
   static constexpr uint32_t kNumbers = 0x07FF07FFu, kNegative = 1u << 11, kLost = 1u << 12;
   uint32_t a, b;

@@ -1248,8 +1248,9 @@ __global__ __launch_bounds__(kWide) void k_sample_pick(SrcPack<Src> srcs, ChainJ
 // counts above it, and a histogram of the few inside.  The last workgroup to finish takes the bracket from it, at the
 // edges of the histogram's bins (rounded outwards: a few sample keys wide); an end the coarse bracket missed is left
 // open.  The tickets go by sixteen words and one: on one word they queue, 11 ns each (1024 workgroups: 8 us of a select
-// of 300 M scores), and four quads a thread by a quarter of the workgroups made the sample of `update` 12 us longer.  The pick as a launch of its own -> here, selects
-// in a row at 1 %, us: 9 M scores 43.0 -> 41.1, 20 M 53.9 -> 52.5, 40 M 69.7 -> 68.7, 100 M and more the same.
+// of 300 M scores), and four quads a thread by a quarter of the workgroups made the sample of `update` 12 us longer.
+// The pick as a launch of its own -> here, selects in a row at 1 %, us: 9 M scores 43.0 -> 41.1, 20 M 53.9 -> 52.5,
+// 40 M 69.7 -> 68.7, 100 M and more the same.
 // What the pick reads of the others' are device-scope atomics, which every wave waits for before its workgroup
 // takes its ticket; the ticket is a word of the state that the kernel before has written.
 constexpr int kFineSpread = kRelSpread;                // tickets: a word for every sixteenth workgroup, then one for those

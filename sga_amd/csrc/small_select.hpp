@@ -262,8 +262,8 @@ struct SmallList {
       if (c < (uint32_t)(u + 1) * kWave * kVec) trim(key[u], (uint32_t)(u * kWave + lane_id()) * kVec, c);   // uniform
   }
   // head(key, idx) over the entries in registers, tail(keys, idxs) over rounds of quads of the rest (whole waves).
-  // IDX: the index is wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a microsecond
-  // a round of loads, so the next round is on its way while one is worked off.
+  // IDX: the index is wanted; without it twice as many keys are in flight.  The rest comes from other XCDs' stores, a
+  // microsecond a round of loads, so the next round is on its way while one is worked off.
   template <bool IDX, class H, class T>
   __device__ __forceinline__ void visit(H&& head, T&& tail) const {
 #pragma unroll
