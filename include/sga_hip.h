@@ -326,6 +326,11 @@ size_t sga_select_workspace_bytes(int64_t n);
 int sga_select_topk(const float* score, int64_t n, int64_t k, int tie_mode,
                     uint8_t* mask_out, sga_select_result* result, void* ws,
                     size_t ws_bytes, void* stream);
+/* dst[0..n) = src[0..n), n <= 64 words of 32 bits from the device to pinned
+ * host memory, when everything before on the stream has ended: a host that
+ * sees them (none of src has all bits set) may use all of that, also by other
+ * streams. */
+int sga_words_to_host(const uint32_t* src, int n, uint32_t* dst, void* stream);
 
 /* The same select over several disjoint runs (the online plugin's per-param
  * views, _histogram.py:97-112): begin, then per radix level one hist call per

@@ -92,6 +92,7 @@ SIGNATURES = {
     "sga_sel_tile_scan": (I32, [I64, I32, P, SZ, P]),
     "sga_sel_mask": (I32, [P, I64, I64, I32, P, P, SZ, P]),
     "sga_sel_result": (I32, [P, P, SZ, P]),
+    "sga_words_to_host": (I32, [P, I32, P, P]),
     "sga_hist_topbits": (I32, [P, I64, I32, I32, I32, P, I32, P, P]),
     "sga_mask_topbits_ge": (I32, [P, I64, I32, I32, P, P]),
     "sga_scale_masked": (I32, [P, P, I64, F, P]),

@@ -344,6 +344,25 @@ extern "C" int sga_sel_result(sga_select_result* result, void* ws, size_t ws_byt
   return check_launch("sga_sel_result");
 }
 
+// A launch of its own: it begins when everything before it on the stream has ended, and its fence makes that, too,
+// come before the words.
+static __global__ __launch_bounds__(kWave) void k_words_to_host(const uint32_t* __restrict__ src, int n,
+                                                                uint32_t* __restrict__ dst) {
+  const int i = (int)threadIdx.x;
+  const uint32_t v = i < n ? src[i] : 0u;
+  __threadfence_system();
+  if (i < n) st_host(dst + i, v);
+}
+
+extern "C" int sga_words_to_host(const uint32_t* src, int n, uint32_t* dst, void* stream) {
+  if (!src || !dst || n < 1 || n > kWave) {
+    set_error("sga_words_to_host: bad argument (1 <= n=%d <= %d)", n, kWave);
+    return SGA_ERR_ARG;
+  }
+  hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(kWave), 0, (hipStream_t)stream, src, n, dst);
+  return check_launch("sga_words_to_host");
+}
+
 extern "C" int sga_select_topk(const float* score, int64_t n, int64_t k, int tie_mode,
                                uint8_t* mask_out, sga_select_result* result, void* ws,
                                size_t ws_bytes, void* stream) {

@@ -88,13 +88,14 @@ def test_a_select_returns_behind_its_mask(dev, n, monkeypatch):
                                                          sga_selection_ratio_percent=2.0))
     score = torch.rand(n, generator=torch.Generator(device=dev).manual_seed(n), device=dev)
     views, k = [score[:n // 2], score[n // 2:]], int(round(n * 0.02))
-    plugin, other, main = TopkSelection(), torch.cuda.Stream(), torch.cuda.current_stream()
+    plugin, other = TopkSelection(), torch.cuda.Stream()
     ties = int((score >= score.topk(k).values[-1]).sum())
     for call in (lambda: [select_topk_flat(score, k)[0]], lambda: select_masks_histogram(views, k)[1],
                  lambda: plugin.select(SimpleNamespace(grad_views=[score]))):
-        main.synchronize()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(other):
+            torch.zeros(1, device=dev)                # the other stream is there
         masks = call()
-        assert main.query()
         with torch.cuda.stream(other):
             on = sum(int(m.sum(dtype=torch.int64)) for m in masks)
         assert on in (k, ties)                    # of the scores at the threshold as many as make k, or all
@@ -226,3 +227,17 @@ def test_a_recorded_graph_keeps_no_words_of_the_host(dev):
         torch.cuda.synchronize()
         assert L.arrived(below) == [3]
     assert not L.words(1).is_cuda
+
+
+@pytest.mark.parametrize("n", [1, 8, 63, 64])
+def test_words_to_host(dev, n):
+    from sga_amd import _lib as L
+    src = torch.randint(-2 ** 31, 2 ** 31 - 1, (n + 1,), dtype=torch.int32, device=dev)
+    src[src == -1] = 0
+    for at in (0, 1):
+        words = L.words(n)
+        L.call("sga_words_to_host", L.ptr(src[at:]), n, L.ptr(words), L.stream())
+        assert [w & 0xFFFFFFFF for w in src[at:at + n].tolist()] == list(L.arrived(words))
+    for bad in (0, 65, -1):
+        with pytest.raises(RuntimeError, match="bad argument"):
+            L.call("sga_words_to_host", L.ptr(src), bad, L.ptr(words), L.stream())
