@@ -638,7 +638,10 @@ __global__ __launch_bounds__(kFoldThreads) void k_fold_partials(const double* __
     if ((int)threadIdx.x < o) s_p[threadIdx.x] += s_p[threadIdx.x + o];
     __syncthreads();
   }
-  if (threadIdx.x == 0) st_host(out, s_p[0] / divisor);
+  if (threadIdx.x == 0) {
+    __threadfence_system();                           // the step's state, written by the launch before, comes first
+    st_host(out, s_p[0] / divisor);
+  }
 }
 __global__ __launch_bounds__(kWave) void k_sqdist_stage2(const double* __restrict__ partials, int nb,
                                                          double* __restrict__ out) {
